@@ -45,7 +45,7 @@ enum {
  * (it builds a HYBRID plan, which may consist of a single family). */
 enum {
     SDDMM_KERNEL_AUTO = 0,
-    SDDMM_KERNEL_ROW_GATHER = 1, /* W row in VGPRs, H rows gathered from L2/HBM (as a plan: the unpadded stream kernel;
+    SDDMM_KERNEL_ROW_GATHER = 1, /* W row in VGPRs, H rows gathered from L2/HBM (as a plan: the unpadded gather kernel;
                                     as the short-row launch of a HYBRID plan: the padded, pipelined gather, over
                                     column slabs when H is far larger than the caches) */
     SDDMM_KERNEL_LDS_TILE = 2,   /* column tiles of H staged in LDS, W row (re)loaded per row run */
@@ -382,7 +382,7 @@ int sddmm_execute_ws(const sddmm_plan *plan, const float *d_val, const float *d_
  * before any entry can be normalised): every row of up to 16,376 entries is
  * taken into registers whole -- by a lane, a group of lanes, a wave or a
  * workgroup, by its length -- so it is read once and written once; a longer row
- * is cut into pieces of 4096 entries whose (max, sum) records are merged by a
+ * is cut into pieces of up to 4096 entries whose (max, sum) records are merged by a
  * last kernel.  The layout of the work and those records are kept in fixed
  * device arrays of the library (18 MiB per GPU), so softmax calls that overlap
  * in time on one GPU (different streams or threads) race unless they bring a
@@ -391,9 +391,9 @@ int sddmm_execute_ws(const sddmm_plan *plan, const float *d_val, const float *d_
  * memory (d_out may be d_x; n_rows < 2^31 - 1, row_ptr[n_rows] entries).
  * sddmm_spmm_csr: Y[r, 0:K] = sum over row r's entries p of x[p] * H[col_p, 0:K]
  * (d_Y: n_rows*K fp32, overwritten; rows without entries become 0), the product
- * that consumes the attention weights.  Rows that straddle the 256-entry chunks
- * the waves work in are completed with fp32 atomic adds, so their last bits can
- * differ from run to run.
+ * that consumes the attention weights.  Rows that straddle the pieces of 4 to 32
+ * entries in which the work is dealt out are completed with fp32 atomic adds, so
+ * their last bits can differ from run to run.
  *
  * sddmm_plan_spmm: the same product behind the plan of its SDDMM.  A plan made
  * with spmm_stream = 1 walks the rows of its LDS_TILE launch once more, as
@@ -440,25 +440,23 @@ int sddmm_execute_profiled(const sddmm_plan *plan, const float *d_val, const flo
 int sddmm_gpu(const sddmm_plan *plan, const float *h_W, const float *h_H, float *h_out,
               float *kernel_ms);
 
-/* Plan-free SDDMM over a CSR pattern in device memory that allocates nothing:
- * no hipMalloc / hipFree and no allocating library routine in the call.  The
- * first call of a process on a device looks up the address of the library's
- * fixed array and is the first launch of its kernels, which is when the runtime
- * may load the code object and materialise that array: make one warm-up call per
- * device outside any graph capture; after it, no call allocates.  It has
+/* Plan-free SDDMM over a CSR pattern in device memory that allocates nothing and
+ * keeps nothing: no hipMalloc / hipFree, no allocating library routine, no scratch
+ * memory.  The first call of a process on a device is the first launch of its
+ * kernel, which is when the runtime may load the code object: make one warm-up call
+ * per device outside any graph capture; after it, no call allocates.  It has
  * no counterpart in the reference (whose sddmm_GPU allocates and frees on every
  * call, sddmm.cu:38-73, 147-150); it is for callers that cannot allocate --
  * code under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc -- and therefore cannot create a plan.  Same result as
+ * hipMalloc -- and for patterns that are new on every call, where a plan would not
+ * pay.  Same result as
  * sddmm_plan_create_device(..., SDDMM_KERNEL_ROW_GATHER) + sddmm_execute, bit
- * for bit: the row-gather kernel, whose per-batch side array (the row of every
- * 64th nonzero) is built on the device, on `stream`, into a fixed 16 MiB
- * device array of the library.  All pointers are device pointers; d_val may be
+ * for bit: the row-gather kernel in one launch, every wave finding the rows of its
+ * nonzeros from the row pointers.  All pointers are device pointers; d_val may be
  * NULL (out[p] = dot).  The pattern is not validated (that would need a copy
  * to the host): d_row_ptr must be monotone with d_row_ptr[0] = 0 and
  * d_row_ptr[n_rows] = nnz, columns inside [0, n_cols).  nnz above SDDMM_NOALLOC_MAX_NNZ is rejected with
- * SDDMM_ERR_RANGE.  Every call on a GPU uses that GPU's one array: calls that
- * overlap in time on the same GPU (different streams or threads) race.       */
+ * SDDMM_ERR_RANGE.  Calls may overlap in time (other threads, other streams).  */
 #define SDDMM_NOALLOC_MAX_NNZ (1 << 28)
 int sddmm_csr_noalloc(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *d_row_ptr,
                       const int32_t *d_col_ind, const float *d_val, int32_t K, const float *d_W,

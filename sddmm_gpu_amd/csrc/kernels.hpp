@@ -30,13 +30,9 @@ struct KArgs {
     int32_t K;
     int32_t tile_x;
     int32_t n_cols;
-    int32_t generic_perm;
     int32_t residual;          // 0: out = val * dot;  1: out = val - dot
-    // Plan-free form (batch_seg and batch_mask are null then): batch_row[b] is the row of stream
-    // position 64*b, and every lane finds its own row by a search of row_ptr between the
-    // rows of two consecutive batches.
+    // Plan-free form (batch_seg and batch_mask are null then): the rows are found from the row pointers.
     const int32_t *row_ptr;    // [n_rows+1]
-    const int32_t *batch_row;  // [ceil(nnz/64)]
     int32_t n_rows;
 };
 
@@ -197,9 +193,11 @@ struct DenseArgs {
 using DenseFn = void (*)(const DenseArgs);
 DenseFn dense_kernel();
 
-// lanes per nonzero and float4 slots per lane for a given K (K % 4 == 0); G == 0: none
-Variant pick_variant(int K, bool lds_tile);
-KernelFn stream_kernel(const Variant &v, bool lds_tile);
-KernelFn generic_kernel();
+// lanes per nonzero and float4 slots per lane for a given K; G == 0: none
+Variant pick_gather_variant(int K);  // row gather, any K from 4 to 2048
+KernelFn gather_kernel(const Variant &v);
+KernelFn generic_kernel();           // row gather, any K
+Variant pick_stream_variant(int K);  // unpadded LDS tile (K % 4 == 0)
+KernelFn stream_kernel(const Variant &v);
 
 }  // namespace sddmm

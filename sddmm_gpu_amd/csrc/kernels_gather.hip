@@ -1,0 +1,290 @@
+// Row-gather kernel of the SDDMM engine for gfx950 (MI355X): S walked in sorted order, H rows read from
+// global memory.  It serves plans of the row-gather family (rows of each batch from the plan's side arrays)
+// and the plan-free entry point (rows from the row pointers).
+//
+// A wave takes up to 8 batches of 64 consecutive nonzeros, one per lane.  In a batch a group of G lanes works
+// on its own G nonzeros, all lanes of the group on one nonzero per step: each lane keeps KPL pieces of four
+// floats of the W row, reads the same pieces of the nonzero's H row, and the G partial sums of the G nonzeros
+// are reduced together by a halving exchange that leaves nonzero i's dot product in lane i.
+//
+// What bounds it is the load path (64 bytes per clock and compute unit for everything read, cached or not) and,
+// where H and W are larger than the caches, the traffic across the fabric.  So: the W row is read again only in
+// steps in which some group's row changes (a uniform branch on a bit mask made once per batch), and the pieces
+// of step i + 1 are requested before the arithmetic of step i, across batches too; index data is requested a
+// batch ahead.  K needs no alignment (see RowPiece): the pieces behind the end of a row read its last four
+// floats again, with what they share with the piece before masked to zero in both factors.
+#include <hip/hip_runtime.h>
+#include <algorithm>
+#include <utility>
+#include "kernels.hpp"
+#include "csr_walk.hpp"
+
+using namespace sddmm;
+
+namespace {
+
+// value held by lane I of the caller's group of G lanes
+template <int G, int I>
+__device__ __forceinline__ int group_bcast(int v)
+{
+    if constexpr (G == 64) return __builtin_amdgcn_readlane(v, I);
+    else if constexpr (G == 4) return __builtin_amdgcn_mov_dpp(v, I * 0x55, 0xf, 0xf, true);  // quad_perm [I, I, I, I]
+    else return __builtin_amdgcn_ds_swizzle(v, (I << 5) | (0x1f & ~(G - 1)));                 // src = (lane & ~(G-1)) | I
+}
+
+// value of lane (lane ^ S)
+template <int S>
+__device__ __forceinline__ float xor_lane(float v)
+{
+    if constexpr (S == 1)
+        return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xf, 0xf, true));  // quad_perm [1,0,3,2]
+    else if constexpr (S == 2)
+        return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xf, 0xf, true));  // quad_perm [2,3,0,1]
+    else if constexpr (S < 32)
+        return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (S << 10) | 0x1f));
+    else
+        return __shfl_xor(v, S, 64);
+}
+
+// Running halving reduction: acc[i] is this lane's share of nonzero i; lane i of the group ends with the sum.
+template <int G, int S = G / 2>
+__device__ __forceinline__ void transpose_reduce_step(float (&acc)[G], int l)
+{
+    if constexpr (S >= 1) {
+        const bool upper = (l & S) != 0;
+#pragma unroll
+        for (int j = 0; j < S; ++j) {
+            const float keep = upper ? acc[j + S] : acc[j];
+            const float send = upper ? acc[j] : acc[j + S];
+            acc[j] = keep + xor_lane<S>(send);
+        }
+        transpose_reduce_step<G, S / 2>(acc, l);
+    }
+}
+
+// bit 0 of every group of G lanes
+template <int G> constexpr uint64_t group_bits()
+{
+    uint64_t m = 0;
+    for (int i = 0; i < 64; i += G) m |= 1ull << i;
+    return m;
+}
+
+// RAGGED: K is not 4 * G * KPL (its pieces are masked; any K > 4 * G * (KPL - 1) up to 4 * G * KPL, K >= 4).
+template <int G, int KPL, bool RAGGED>
+__global__ __launch_bounds__(kRowGatherBlock)
+void sddmm_gather_kernel(const KArgs a)
+{
+    constexpr int NW = kRowGatherBlock / 64;
+    __shared__ int row_tab[NW][64 * kRowGatherBatchesPerWave + 1];  // (plan-free form)
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l = lane & (G - 1);
+    const int K = a.K;
+    const uint64_t le = (lane == 63) ? ~0ull : ((2ull << lane) - 1ull);
+
+    int off[KPL];
+    int first[KPL];
+#pragma unroll
+    for (int j = 0; j < KPL; ++j) {
+        const RowPiece r = row_piece(j * G + l, K);
+        off[j] = RAGGED ? r.off : 4 * (j * G + l);
+        first[j] = r.first;
+    }
+
+    const int begin = blockIdx.x * a.chunk;
+    const int end = min(a.nnz, begin + a.chunk);
+    const int nb = (end - begin + 63) >> 6;
+    const int b0 = __builtin_amdgcn_readfirstlane((int)((int64_t)nb * wave / NW));
+    const int b1 = __builtin_amdgcn_readfirstlane((int)((int64_t)nb * (wave + 1) / NW));
+    if (b0 >= b1) return;
+    const int batch_base = begin >> 6;
+    const bool planned = a.batch_seg != nullptr;
+    int *tab = row_tab[wave];
+    if (!planned) {
+        const int p0 = begin + (b0 << 6);
+        rows_of_range(a.row_ptr, a.n_rows, wave_find_row(a.row_ptr, a.n_rows, p0, lane), p0, (b1 - b0) << 6, tab, lane);
+    }
+
+    struct Batch {
+        int row, p, col;
+        float v;
+    };
+    // (lanes past the end repeat the last nonzero and store nothing; beyond a wave's last batch its last one again)
+    auto load_batch = [&](int bi_in) -> Batch {
+        const int bi = min(bi_in, b1 - 1);
+        const int pos = min(begin + (bi << 6) + lane, end - 1);
+        Batch b;
+        if (planned) {
+            const int gb = batch_base + bi;
+            const int seg = a.batch_seg[gb] + __popcll(a.batch_mask[gb] & le);  // (lanes past the end: the last segment)
+            b.row = a.seg_row ? a.seg_row[seg] : seg;
+        } else {
+            b.row = tab[pos - begin - (b0 << 6)];
+        }
+        b.p = a.perm ? a.perm[pos] : pos;
+        b.col = a.col_ind[b.p];
+        b.v = a.sval ? a.sval[pos] : (a.val ? a.val[b.p] : 1.0f);
+        return b;
+    };
+
+    vec4u w[2][KPL], h[2][KPL];
+#pragma unroll
+    for (int j = 0; j < KPL; ++j) w[0][j] = w[1][j] = vec4u{0.f, 0.f, 0.f, 0.f};
+    auto mask_piece = [&](vec4u &v, int j) {
+        if constexpr (RAGGED) {
+            v.x = first[j] > 0 ? 0.f : v.x;
+            v.y = first[j] > 1 ? 0.f : v.y;
+            v.z = first[j] > 2 ? 0.f : v.z;
+            v.w = first[j] > 3 ? 0.f : v.w;
+        }
+    };
+    // requests the pieces of step I of a batch; changed: the lanes whose nonzero is in another row than the one before
+    auto issue = [&]<int I>(std::integral_constant<int, I>, const Batch &b, uint64_t changed) {
+        if (changed & (group_bits<G>() << I)) {
+            const float *wr = a.W + (size_t)group_bcast<G, I>(b.row) * K;
+#pragma unroll
+            for (int j = 0; j < KPL; ++j) w[I & 1][j] = *reinterpret_cast<const vec4u *>(wr + off[j]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < KPL; ++j) w[I & 1][j] = w[(I & 1) ^ 1][j];
+        }
+        const float *hr = a.H + (size_t)group_bcast<G, I>(b.col) * K;
+#pragma unroll
+        for (int j = 0; j < KPL; ++j) h[I & 1][j] = *reinterpret_cast<const vec4u *>(hr + off[j]);
+    };
+    // rows of a batch that differ from the row before: inside a group the lane before, for its first lane the
+    // group's row at the end of the batch before
+    auto row_changes = [&](const Batch &b, int last_row) -> uint64_t {
+        int before = __shfl_up(b.row, 1);
+        if (l == 0) before = last_row;
+        return __ballot(b.row != before);
+    };
+
+    Batch cur = load_batch(b0);
+    Batch nxt = load_batch(b0 + 1);
+    uint64_t changed = row_changes(cur, -1);
+    issue(std::integral_constant<int, 0>{}, cur, changed);
+    for (int bi = b0; bi < b1; ++bi) {
+        float acc[G];
+        const Batch after = load_batch(bi + 2);
+        const uint64_t changed_next = row_changes(nxt, group_bcast<G, G - 1>(cur.row));
+        [&]<int... I>(std::integer_sequence<int, I...>) {
+            ((void)[&] {
+                if constexpr (I + 1 < G) issue(std::integral_constant<int, I + 1>{}, cur, changed);
+                __builtin_amdgcn_sched_barrier(0);
+                float s = 0.f;
+#pragma unroll
+                for (int j = 0; j < KPL; ++j) {
+                    vec4u hv = h[I & 1][j], wv = w[I & 1][j];
+                    mask_piece(hv, j);
+                    mask_piece(wv, j);
+                    s = fmaf(wv.x, hv.x, s); s = fmaf(wv.y, hv.y, s);
+                    s = fmaf(wv.z, hv.z, s); s = fmaf(wv.w, hv.w, s);
+                }
+                asm volatile("" : "+v"(s));  // (computed here: left alone the compiler sinks it behind the branches of the later steps)
+                acc[I] = s;
+                // (the last step's: the next batch's first, requested before the reduction)
+                if constexpr (I + 1 == G) issue(std::integral_constant<int, 0>{}, nxt, changed_next);
+                __builtin_amdgcn_sched_barrier(0);
+            }(), ...);
+        }(std::make_integer_sequence<int, G>{});
+        transpose_reduce_step<G>(acc, l);
+        if (begin + (bi << 6) + lane < end) a.out[cur.p] = a.residual ? cur.v - acc[0] : acc[0] * cur.v;
+        cur = nxt;
+        nxt = after;
+        changed = changed_next;
+    }
+}
+
+// Any K >= 1 (used below 4 and beyond 2048): 8 lanes per nonzero striding over the row one float at a time,
+// W re-read through the cache.  The slow, always-correct path.
+__global__ __launch_bounds__(kRowGatherBlock)
+void sddmm_generic_kernel(const KArgs a)
+{
+    constexpr int G = 8;
+    constexpr int NW = kRowGatherBlock / 64;
+    __shared__ int row_tab[NW][64 * kRowGatherBatchesPerWave + 1];  // (plan-free form)
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l = lane & (G - 1);
+    const int begin = blockIdx.x * a.chunk;
+    const int end = min(a.nnz, begin + a.chunk);
+    const int batch_base = begin >> 6;
+    const int nb = (end - begin + 63) >> 6;
+    const int b0 = __builtin_amdgcn_readfirstlane((int)((int64_t)nb * wave / NW));
+    const int b1 = __builtin_amdgcn_readfirstlane((int)((int64_t)nb * (wave + 1) / NW));
+    if (b0 >= b1) return;
+    const bool planned = a.batch_seg != nullptr;
+    int *tab = row_tab[wave];
+    if (!planned) {
+        const int p0 = begin + (b0 << 6);
+        rows_of_range(a.row_ptr, a.n_rows, wave_find_row(a.row_ptr, a.n_rows, p0, lane), p0, (b1 - b0) << 6, tab, lane);
+    }
+    for (int bi = b0; bi < b1; ++bi) {
+        const int pos = begin + (bi << 6) + lane;
+        const bool valid = pos < end;
+        const int gb = batch_base + bi;
+        const uint64_t le = (lane == 63) ? ~0ull : ((2ull << lane) - 1ull);
+        int row = -1, col = 0, p = 0;
+        float v = 0.f;
+        if (valid) {
+            if (planned) {
+                const int seg = a.batch_seg[gb] + __popcll(a.batch_mask[gb] & le);
+                row = a.seg_row ? a.seg_row[seg] : seg;
+            } else {
+                row = tab[pos - begin - (b0 << 6)];
+            }
+            p = a.perm ? a.perm[pos] : pos;
+            col = a.col_ind[p];
+            v = a.val ? a.val[p] : 1.0f;
+        }
+        float acc[G];
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+            const int r_i = __shfl(row, i, G);
+            const int c_i = __shfl(col, i, G);
+            float s = 0.f;
+            if (r_i >= 0) {
+                const float *wr = a.W + (size_t)r_i * a.K;
+                const float *hr = a.H + (size_t)c_i * a.K;
+                for (int t = l; t < a.K; t += G) s = fmaf(wr[t], hr[t], s);
+            }
+            acc[i] = s;
+        }
+        transpose_reduce_step<G>(acc, l);
+        if (valid) a.out[p] = a.residual ? v - acc[0] : acc[0] * v;
+    }
+}
+
+}  // namespace
+
+namespace sddmm {
+
+// The smallest number of lanes whose pieces cover a row, at least 8 (128 contiguous bytes per gathered row) from
+// K = 17 on; K < 4 and K > 2048 are left to the generic kernel (G == 0).
+Variant pick_gather_variant(int K)
+{
+    const int K4 = (K + 3) / 4;
+    const int cand[][2] = {{4, 1}, {8, 1}, {8, 2}, {8, 3}, {8, 4}, {16, 3}, {16, 4}, {32, 3}, {32, 4}, {64, 3}, {64, 4}, {64, 8}};
+    if (K < 4) return {0, 0, false};
+    for (auto &c : cand)
+        if (c[0] * c[1] >= K4) return {c[0], c[1], c[0] * c[1] * 4 == K};
+    return {0, 0, false};
+}
+
+KernelFn gather_kernel(const Variant &v)
+{
+#define SDDMM_CASE(g, kpl)                                                                 \
+    if (v.G == g && v.KPL == kpl)                                                          \
+        return v.exact ? (KernelFn)sddmm_gather_kernel<g, kpl, false>                      \
+                       : (KernelFn)sddmm_gather_kernel<g, kpl, true>;
+    SDDMM_CASE(4, 1) SDDMM_CASE(8, 1) SDDMM_CASE(8, 2) SDDMM_CASE(8, 3) SDDMM_CASE(8, 4) SDDMM_CASE(16, 3) SDDMM_CASE(16, 4)
+    SDDMM_CASE(32, 3) SDDMM_CASE(32, 4) SDDMM_CASE(64, 3) SDDMM_CASE(64, 4) SDDMM_CASE(64, 8)
+#undef SDDMM_CASE
+    return nullptr;
+}
+
+KernelFn generic_kernel() { return (KernelFn)sddmm_generic_kernel; }
+
+}  // namespace sddmm

@@ -1,19 +1,16 @@
-// Stream kernels of the SDDMM engine for gfx950 (MI355X).
+// Unpadded LDS-tile kernel of the SDDMM engine for gfx950 (MI355X): explicit LDS_TILE plans at ranks that
+// the padded tile kernel has no variant for.
 //
-// Both kernel families walk a "stream" of nonzeros in batches of 64 (one per
-// lane of a wavefront):
-//   row-gather : the stream is the sorted S itself, cut into fixed chunks;
-//   LDS-tile   : the stream is S in tile order (column tile by column tile,
-//                rows ascending inside a tile) reached through the permutation
-//                the tiling pass produced; the workgroup stages the tile's H
-//                rows in LDS first.
+// The stream of nonzeros is S in tile order (column tile by column tile, rows ascending inside a tile),
+// reached through the permutation the tiling pass produced, and walked in batches of 64 (one per lane of a
+// wavefront); the workgroup stages the tile's H rows in LDS first.
 // A batch loads its 64 column indices / values / outputs coalesced.  The rows
 // of the 64 nonzeros come from two small side arrays (first segment of the
 // batch + a 64-bit mask of "a new row starts here"), so no per-nonzero row
 // index is read.  Inside a batch, groups of G lanes each take G consecutive
-// nonzeros: for each, the group reads the H row (from LDS or global) as
-// contiguous 16-byte pieces, multiplies with the W row slice it keeps in
-// VGPRs while the row lasts, and the G partial sums of G nonzeros are reduced
+// nonzeros: for each, the group reads the H row from LDS in 16-byte pieces,
+// multiplies with the W row slice it keeps in VGPRs while the row lasts, and
+// the G partial sums of G nonzeros are reduced
 // together by a butterfly of cross-lane exchanges that leaves nonzero i's dot
 // product in lane i, which scales it by S.val and stores it.
 #include <hip/hip_runtime.h>
@@ -86,37 +83,18 @@ struct Batch {
     float v;
 };
 
-// Row (segment) of stream position pos, which lies in batch gb.  With the plan's side
-// arrays: the batch's first segment plus the number of segment starts up to this lane.
-// Plan-free form: the largest row r between the rows of this batch's and the next
-// batch's first positions with row_ptr[r] <= pos (empty rows in between never qualify
-// as the largest).
-__device__ __forceinline__ int segment_of(const KArgs &a, int gb, int pos, uint64_t le)
-{
-    if (a.batch_row) {
-        int lo = a.batch_row[gb];
-        int hi = (gb + 1 < ((a.nnz + 63) >> 6)) ? a.batch_row[gb + 1] : a.n_rows - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (a.row_ptr[mid] <= pos) lo = mid; else hi = mid - 1;
-        }
-        return lo;
-    }
-    return a.batch_seg[gb] + __popcll(a.batch_mask[gb] & le);
-}
-
 // K = 4 * (number of float4 per row); each lane of a group owns KPL float4
 // slots of a row: slot j sits at float4 index (((j + rot) % KPL) * G + l).  `rot`
 // differs between the groups that share one 16-lane LDS access phase, so that
 // their 16-byte reads fall into different banks when rows are a multiple of
 // 256 bytes apart.  EXACT: K == 4*G*KPL (no slot is out of range).
 // The index data of batch b+1 is requested before batch b is computed.
-template <int G, int KPL, bool EXACT, bool LDS_TILE>
-__global__ __launch_bounds__(LDS_TILE ? kLdsBlock : kRowGatherBlock)
+template <int G, int KPL, bool EXACT>
+__global__ __launch_bounds__(kLdsBlock)
 void sddmm_stream_kernel(const KArgs a)
 {
     extern __shared__ float4 lds_tile[];
-    constexpr int NW = (LDS_TILE ? kLdsBlock : kRowGatherBlock) / 64;
+    constexpr int NW = kLdsBlock / 64;
     constexpr int PHASE_GROUPS = (16 / G) >= 1 ? (16 / G) : 1;
     constexpr int ROT_MASK = (PHASE_GROUPS < KPL ? PHASE_GROUPS : KPL) - 1;
 
@@ -134,36 +112,24 @@ void sddmm_stream_kernel(const KArgs a)
     const float4 *__restrict__ W4 = reinterpret_cast<const float4 *>(a.W);
     const float4 *__restrict__ H4 = reinterpret_cast<const float4 *>(a.H);
 
-    int item0, item1;
-    if (LDS_TILE) {  // contiguous run of items per workgroup: the tile changes rarely
-        item0 = (int)((int64_t)a.n_items * blockIdx.x / gridDim.x);
-        item1 = (int)((int64_t)a.n_items * (blockIdx.x + 1) / gridDim.x);
-    } else {
-        item0 = blockIdx.x;
-        item1 = item0 + 1;
-    }
+    // contiguous run of items per workgroup: the tile changes rarely
+    const int item0 = (int)((int64_t)a.n_items * blockIdx.x / gridDim.x);
+    const int item1 = (int)((int64_t)a.n_items * (blockIdx.x + 1) / gridDim.x);
     int cur_tile = -1;
     int tile_base = 0;
 
     for (int it = item0; it < item1; ++it) {
-        int begin, end, batch_base;
-        if (LDS_TILE) {
-            const WorkItem wi = a.items[it];
-            begin = wi.begin; end = wi.end; batch_base = wi.batch_base;
-            if (wi.tile != cur_tile) {
-                __syncthreads();  // everyone is done with the previous tile
-                cur_tile = wi.tile;
-                tile_base = cur_tile * a.tile_x;
-                int rows = min(a.tile_x, a.n_cols - tile_base);
-                const float4 *src = H4 + (size_t)tile_base * K4;
-                const int n4 = rows * K4;
-                for (int i = threadIdx.x; i < n4; i += blockDim.x) lds_tile[i] = src[i];
-                __syncthreads();
-            }
-        } else {
-            begin = it * a.chunk;
-            end = min(a.nnz, begin + a.chunk);
-            batch_base = begin >> 6;
+        const WorkItem wi = a.items[it];
+        const int begin = wi.begin, end = wi.end, batch_base = wi.batch_base;
+        if (wi.tile != cur_tile) {
+            __syncthreads();  // everyone is done with the previous tile
+            cur_tile = wi.tile;
+            tile_base = cur_tile * a.tile_x;
+            int rows = min(a.tile_x, a.n_cols - tile_base);
+            const float4 *src = H4 + (size_t)tile_base * K4;
+            const int n4 = rows * K4;
+            for (int i = threadIdx.x; i < n4; i += blockDim.x) lds_tile[i] = src[i];
+            __syncthreads();
         }
         const int nb = (end - begin + 63) >> 6;
         const int b0 = (int)((int64_t)nb * wave / NW), b1 = (int)((int64_t)nb * (wave + 1) / NW);
@@ -173,7 +139,7 @@ void sddmm_stream_kernel(const KArgs a)
             const int pos = begin + (bi << 6) + lane;
             if (bi < b1 && pos < end) {
                 const int gb = batch_base + bi;
-                const int seg = segment_of(a, gb, pos, le);
+                const int seg = a.batch_seg[gb] + __popcll(a.batch_mask[gb] & le);
                 b.row = a.seg_row ? a.seg_row[seg] : seg;
                 b.p = a.perm ? a.perm[pos] : pos;
                 b.col = a.scol ? a.scol[pos] : a.col_ind[b.p];
@@ -209,8 +175,7 @@ void sddmm_stream_kernel(const KArgs a)
                 [&]<int... I>(std::integer_sequence<int, I...>) {
                     ((void)[&] {
                         const int c_i = group_bcast<G, I>(cur.col);
-                        const float4 *hr = LDS_TILE ? (lds_tile + (size_t)(c_i - tile_base) * K4)
-                                                    : (H4 + (size_t)c_i * K4);
+                        const float4 *hr = lds_tile + (size_t)(c_i - tile_base) * K4;
 #pragma unroll
                         for (int j = 0; j < KPL; ++j)
                             if (EXACT || slot[j] < K4) acc[I] = dot4(w[j], hr[slot[j]], acc[I]);
@@ -229,8 +194,7 @@ void sddmm_stream_kernel(const KArgs a)
                                 for (int j = 0; j < KPL; ++j)
                                     w[j] = (EXACT || slot[j] < K4) ? wr[slot[j]] : make_float4(0.f, 0.f, 0.f, 0.f);
                             }
-                            const float4 *hr = LDS_TILE ? (lds_tile + (size_t)(c_i - tile_base) * K4)
-                                                        : (H4 + (size_t)c_i * K4);
+                            const float4 *hr = lds_tile + (size_t)(c_i - tile_base) * K4;
 #pragma unroll
                             for (int j = 0; j < KPL; ++j)
                                 if (EXACT || slot[j] < K4) acc[I] = dot4(w[j], hr[slot[j]], acc[I]);
@@ -244,82 +208,28 @@ void sddmm_stream_kernel(const KArgs a)
     }
 }
 
-// Any K >= 1: 8 lanes per nonzero striding over the row one float at a time,
-// W re-read through the cache.  The slow, always-correct path.
-__global__ __launch_bounds__(kRowGatherBlock)
-void sddmm_generic_kernel(const KArgs a)
-{
-    constexpr int G = 8;
-    constexpr int NW = kRowGatherBlock / 64;
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int l = lane & (G - 1);
-    const int begin = blockIdx.x * a.chunk;
-    const int end = min(a.nnz, begin + a.chunk);
-    const int batch_base = begin >> 6;
-    const int nb = (end - begin + 63) >> 6;
-    const int b0 = (int)((int64_t)nb * wave / NW), b1 = (int)((int64_t)nb * (wave + 1) / NW);
-    for (int bi = b0; bi < b1; ++bi) {
-        const int pos = begin + (bi << 6) + lane;
-        const bool valid = pos < end;
-        const int gb = batch_base + bi;
-        const uint64_t le = (lane == 63) ? ~0ull : ((2ull << lane) - 1ull);
-        int row = -1, col = 0, p = 0;
-        float v = 0.f;
-        if (valid) {
-            const int seg = segment_of(a, gb, pos, le);
-            row = a.seg_row ? a.seg_row[seg] : seg;
-            p = a.perm ? a.perm[pos] : pos;
-            col = a.col_ind[p];
-            v = a.val ? a.val[p] : 1.0f;
-        }
-        float acc[G];
-#pragma unroll
-        for (int i = 0; i < G; ++i) {
-            const int r_i = __shfl(row, i, G);
-            const int c_i = __shfl(col, i, G);
-            float s = 0.f;
-            if (r_i >= 0) {
-                const float *wr = a.W + (size_t)r_i * a.K;
-                const float *hr = a.H + (size_t)c_i * a.K;
-                for (int t = l; t < a.K; t += G) s = fmaf(wr[t], hr[t], s);
-            }
-            acc[i] = s;
-        }
-        const float sum = transpose_reduce<G>(acc, l);
-        if (valid) a.out[p] = a.residual ? v - sum : sum * v;
-    }
-}
-
 }  // namespace
 
 namespace sddmm {
 
-// With H in LDS fewer lanes per nonzero pay (less cross-lane work per FMA);
-// gathers from global memory prefer at least 8 lanes (128 contiguous bytes).
-Variant pick_variant(int K, bool lds_tile)
+// With H in LDS few lanes per nonzero pay (less cross-lane work per FMA).
+Variant pick_stream_variant(int K)
 {
     const int K4 = K / 4;
-    if (lds_tile) {
-        const int c4[][2] = {{4, 2}, {4, 4}, {4, 8}};
-        for (auto &c : c4)
-            if (c[0] * c[1] == K4) return {c[0], c[1], true};
-    }
-    const int cand[][2] = {{8, 1}, {8, 2}, {8, 3}, {8, 4}, {8, 6}, {8, 8}, {16, 6}, {16, 8}, {32, 6}, {32, 8}, {64, 6}, {64, 8}};
+    const int cand[][2] = {{4, 2}, {4, 4}, {4, 8}, {8, 1}, {8, 2}, {8, 3}, {8, 4}, {8, 6}, {8, 8}, {16, 6}, {16, 8}, {32, 6}, {32, 8}, {64, 6}, {64, 8}};
     for (auto &c : cand)
         if (c[0] * c[1] == K4) return {c[0], c[1], true};
     for (auto &c : cand)
-        if (c[0] * c[1] >= K4) return {c[0], c[1], false};
-    return {0, 0, false};  // K > 2048: generic kernel
+        if (c[0] >= 8 && c[0] * c[1] >= K4) return {c[0], c[1], false};
+    return {0, 0, false};  // K > 2048
 }
 
-template <bool LDS_TILE>
-static KernelFn lookup(const Variant &v)
+KernelFn stream_kernel(const Variant &v)
 {
 #define SDDMM_CASE(g, kpl)                                                              \
     if (v.G == g && v.KPL == kpl)                                                       \
-        return v.exact ? (KernelFn)sddmm_stream_kernel<g, kpl, true, LDS_TILE>          \
-                       : (KernelFn)sddmm_stream_kernel<g, kpl, false, LDS_TILE>;
+        return v.exact ? (KernelFn)sddmm_stream_kernel<g, kpl, true>                    \
+                       : (KernelFn)sddmm_stream_kernel<g, kpl, false>;
     SDDMM_CASE(4, 2) SDDMM_CASE(4, 4) SDDMM_CASE(4, 8)
     SDDMM_CASE(8, 1) SDDMM_CASE(8, 2) SDDMM_CASE(8, 3) SDDMM_CASE(8, 4) SDDMM_CASE(8, 6) SDDMM_CASE(8, 8)
     SDDMM_CASE(16, 6) SDDMM_CASE(16, 8) SDDMM_CASE(32, 6) SDDMM_CASE(32, 8) SDDMM_CASE(64, 6) SDDMM_CASE(64, 8)
@@ -342,8 +252,5 @@ void launch_gather_values(const int32_t *perm, const float *src, float *dst, int
     const int blocks = (int)std::min<int64_t>((n + 255) / 256, 65536);
     hipLaunchKernelGGL(gather_values_kernel, dim3(blocks), dim3(256), 0, (hipStream_t)stream, perm, src, dst, n);
 }
-
-KernelFn stream_kernel(const Variant &v, bool lds_tile) { return lds_tile ? lookup<true>(v) : lookup<false>(v); }
-KernelFn generic_kernel() { return (KernelFn)sddmm_generic_kernel; }
 
 }  // namespace sddmm

@@ -259,7 +259,7 @@ int load_plan_file(const char *path, int64_t n_rows, int64_t n_cols, int64_t nnz
             memcpy(field, &q, 8);
         }
         L.ka.col_ind = nullptr; L.ka.val = nullptr; L.ka.W = L.ka.H = nullptr; L.ka.out = nullptr; L.ka.sval = nullptr;
-        L.ka.row_ptr = nullptr; L.ka.batch_row = nullptr;
+        L.ka.row_ptr = nullptr;
         L.ta.sval = nullptr; L.ta.val = nullptr; L.ta.W = L.ta.H = nullptr; L.ta.out = nullptr;
         L.pa.row_ptr = nullptr; L.pa.col_ind = nullptr; L.pa.val = nullptr; L.pa.W = L.pa.H = nullptr; L.pa.out = nullptr;
         L.da.nz_val = nullptr; L.da.val = nullptr; L.da.W = L.da.H = nullptr; L.da.out = nullptr;

@@ -129,7 +129,7 @@ int resolve_functions(Launch &L)
     case 1:
     case 2: {
         const Variant v{L.fn_g, L.fn_kpl, L.fn_exact != 0};
-        L.fn = v.G ? stream_kernel(v, L.fn_kind == 2) : (L.fn_kind == 1 ? generic_kernel() : nullptr);
+        L.fn = L.fn_kind == 2 ? stream_kernel(v) : v.G ? gather_kernel(v) : generic_kernel();
         if (!L.fn) return fail(SDDMM_ERR_ARG, "plan: no stream kernel for lanes %d x %d", v.G, v.KPL);
         if (L.lds > 0) HIP_TRY(hipFuncSetAttribute((const void *)L.fn, hipFuncAttributeMaxDynamicSharedMemorySize, L.lds));
         return SDDMM_OK;
@@ -243,8 +243,7 @@ int add_row_gather(Ctx &c, const std::vector<int32_t> &rows, bool all_rows)
     const int64_t n = all_rows ? c.nnz : list_nnz(c, rows);
     L.nnz = n;
     if (n == 0) return SDDMM_OK;
-    const bool vec4 = c.K % 4 == 0;
-    Variant var = vec4 ? pick_variant(c.K, false) : Variant{0, 0, false};
+    const Variant var = pick_gather_variant(c.K);
     L.fn_kind = 1; L.fn_g = var.G; L.fn_kpl = var.KPL; L.fn_exact = var.exact;
     if (int rc = resolve_functions(L)) return rc;
     std::vector<int32_t> seg_end(rows.size()), perm;
@@ -282,7 +281,6 @@ int add_row_gather(Ctx &c, const std::vector<int32_t> &rows, bool all_rows)
     const int per_wave = (int)std::clamp<int64_t>(n / (64 * waves_wanted), 1, kRowGatherBatchesPerWave);
     a.chunk = 64 * per_wave * (kRowGatherBlock / 64);
     a.K = c.K; a.n_cols = (int32_t)c.n_cols; a.tile_x = (int32_t)c.n_cols;
-    a.generic_perm = var.G == 0;
     L.grid = (int32_t)((n + a.chunk - 1) / a.chunk);
     L.block = kRowGatherBlock;
     L.k_slice = c.K;
@@ -298,7 +296,7 @@ int add_lds_tile(Ctx &c, const std::vector<int32_t> &rows, bool all_rows, int32_
     Launch L;
     L.kind = SDDMM_KERNEL_LDS_TILE;
     L.rows = (int64_t)rows.size();
-    Variant var = pick_variant(c.K, true);
+    Variant var = pick_stream_variant(c.K);
     if (!var.G) return fail(SDDMM_ERR_ARG, "plan: no LDS-tile kernel for K = %d", c.K);
     L.fn_kind = 2; L.fn_g = var.G; L.fn_kpl = var.KPL; L.fn_exact = var.exact;
     sddmm_tiling T;
@@ -602,7 +600,7 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         c.dev_bytes += nnz * 4;
     }
 
-    const bool have_vec = (K % 4 == 0) && pick_variant(K, true).G != 0;
+    const bool have_vec = (K % 4 == 0) && pick_stream_variant(K).G != 0;
     const int64_t row_bytes = (int64_t)K * 4;
     const int32_t fit_x = (int32_t)std::min<int64_t>(kLdsMaxBytes / row_bytes, INT32_MAX);  // H rows per LDS tile at full K
     const int ks = (K % 128 == 0) ? 128 : (K % 64 == 0) ? 64 : (K % 32 == 0) ? 32 : 0;    // panel kernel K slice
