@@ -1,0 +1,262 @@
+// Sparse-times-dense product Y = X H over a plain CSR pattern in device memory, for gfx950 (MI355X):
+// Y[r, :] = sum over row r's entries p of x[p] * H[col_p, :].
+//
+// A wave takes n = S * 64 / G consecutive nonzeros, G lanes spanning a row of H (a slice of it beyond 256 floats)
+// in pieces of four floats, and each group of G lanes S consecutive nonzeros of its own, so that the work is the
+// same for every wave whatever the rows' lengths.  Columns, values and rows of the wave's nonzeros are put into
+// LDS once, from where a group's lanes read them by broadcast; a group adds in registers while the row lasts and
+// writes it when it changes.  The parts of a row cut between groups are added across the wave, those of a row cut
+// between waves through LDS; a row cut between workgroups is completed with fp32 atomic adds (the only place where
+// the order of additions can vary from run to run; with an add per group and cut row the atomics took half the
+// time).  The rows that need it -- those, and empty ones -- are zeroed by a kernel before this one.
+//
+// What bounds it is the load path (64 bytes per clock and compute unit) and, for an H larger than the caches, the
+// fabric; what bounded the form before (a wave per 256 nonzeros, row by row: three dependent loads for every row)
+// was latency: 429 us at 1.8 M nonzeros and K = 100, 129 us at 18 thousand and K = 16;
+// now 82 and 8 us.
+#include <hip/hip_runtime.h>
+#include <algorithm>
+#include "internal.hpp"
+#include "csr_walk.hpp"
+
+using namespace sddmm;
+
+namespace {
+
+constexpr int kSpmmMost = 512;  // nonzeros of a wave at most
+constexpr int kSpmmUnroll = 4;  // H pieces requested together
+
+// Zeroes the rows of Y that the product adds to or leaves out: empty rows, and rows cut between workgroups (of 2^shift nonzeros).
+__global__ __launch_bounds__(256)
+void sddmm_spmm_zero_rows_kernel(const int32_t *__restrict__ row_ptr, float *Y, int64_t n_rows, int K, int shift)
+{
+    __shared__ int list[4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    bool zero = false;
+    if (r < n_rows) {
+        const int s = row_ptr[r], e = row_ptr[r + 1];
+        zero = s >= e || (s >> shift) != ((e - 1) >> shift);
+    }
+    const uint64_t todo = __ballot(zero);
+    if (zero) list[wave][__builtin_popcountll(todo & (((uint64_t)1 << lane) - 1))] = (int)r;
+    __builtin_amdgcn_wave_barrier();
+    const int pieces = (K + 3) >> 2, n = __builtin_popcountll(todo) * pieces;
+    for (int t = lane; t < n; t += 64) {
+        const int i = t / pieces, q = t - i * pieces;
+        *reinterpret_cast<vec4u *>(Y + (size_t)list[wave][i] * K + row_piece(q, K).off) = vec4u{0.f, 0.f, 0.f, 0.f};
+    }
+}
+
+template <int G>
+__global__ __launch_bounds__(256)
+void sddmm_spmm_csr_kernel(const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col_ind, const float *__restrict__ x,
+                           const float *__restrict__ H, float *Y, int n_rows, int nnz, int K, int S, int slice_pieces)
+{
+    constexpr int NG = 64 / G, U = kSpmmUnroll, NW = 4;
+    __shared__ int row_tab[NW][kSpmmMost + 1];
+    __shared__ int2 entry_tab[NW][kSpmmMost];  // column, value
+    __shared__ vec4u head_sum[NW][G], tail_sum[NW][G];
+    __shared__ int head_row[NW], tail_row[NW];  // -1: none
+    __shared__ bool tail_started[NW];
+    const int lane = threadIdx.x & 63, l = lane & (G - 1), g = lane / G;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = S * NG;
+    const int slot = blockIdx.y * slice_pieces + l;
+    const RowPiece pc = row_piece(slot, K);
+    const int first = l < slice_pieces ? pc.first : 4;  // (4: nothing of this lane's piece is written)
+    auto store = [&](int row, const vec4u &v) {
+        if (row >= n_rows) return;  // (past the last nonzero)
+        float *y = Y + (size_t)row * K + pc.off;
+        if (first == 0) {
+            *reinterpret_cast<vec4u *>(y) = v;
+        } else {
+            if (first <= 1) y[1] = v.y;
+            if (first <= 2) y[2] = v.z;
+            if (first <= 3) y[3] = v.w;
+        }
+    };
+    auto add = [&](int row, const vec4u &v) {
+        if (row >= n_rows) return;
+        float *y = Y + (size_t)row * K + pc.off;
+        if (first <= 0) unsafeAtomicAdd(y + 0, v.x);
+        if (first <= 1) unsafeAtomicAdd(y + 1, v.y);
+        if (first <= 2) unsafeAtomicAdd(y + 2, v.z);
+        if (first <= 3) unsafeAtomicAdd(y + 3, v.w);
+    };
+    const vec4u zero = {0.f, 0.f, 0.f, 0.f};
+
+    const int64_t p0l = ((int64_t)blockIdx.x * NW + wave) * n;
+    if (lane == 0) { head_row[wave] = -1; tail_row[wave] = -1; tail_started[wave] = true; }
+    if (p0l < nnz) {
+        const int p0 = (int)p0l;
+        int *rows = row_tab[wave];
+        int2 *entries = entry_tab[wave];
+        for (int i = lane; i < n; i += 64) {
+            const int p = p0 + min(i, nnz - 1 - p0);
+            entries[i] = make_int2(col_ind[p], i < nnz - p0 ? __float_as_int(x[p]) : 0);
+        }
+        const int r0 = wave_find_row(row_ptr, n_rows, p0, lane);
+        rows_of_range(row_ptr, n_rows, r0, p0, n, rows, lane);
+
+        const float *Hl = H + pc.off;
+        const int gb = g * S;
+        const int row_first = rows[gb], row_last = rows[gb + S - 1];
+        // does the group's first row begin with the group, its last one end with it
+        const bool began = gb > 0 ? rows[gb - 1] != row_first : row_ptr[r0] == p0;
+        const bool ended = rows[gb + S] != row_last;
+        auto request = [&](vec4u (&h)[U], int i0) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) h[u] = *reinterpret_cast<const vec4u *>(Hl + (size_t)entries[gb + i0 + u].x * K);
+        };
+        vec4u acc = zero, head = zero;  // head: the part of a row that began before the group
+        vec4u h[U], hn[U];
+        request(h, 0);
+        int cur = row_first;
+        for (int i0 = 0; i0 < S; i0 += U) {
+            if (i0 + U < S) request(hn, i0 + U);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int r = rows[gb + i0 + u];
+                const float xs = __int_as_float(entries[gb + i0 + u].y);
+                if (r != cur) {
+                    if (cur == row_first && !began) head = acc;
+                    else store(cur, acc);
+                    acc = zero;
+                    cur = r;
+                }
+                acc.x = fmaf(xs, h[u].x, acc.x); acc.y = fmaf(xs, h[u].y, acc.y);
+                acc.z = fmaf(xs, h[u].z, acc.z); acc.w = fmaf(xs, h[u].w, acc.w);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) h[u] = hn[u];
+        }
+        // The rows cut between the groups: acc is the part of the group's last row; `started` says whether that
+        // row's beginning is in it.  A running sum over the groups carries the part on while it stays open.
+        bool has_head = !began && row_first != row_last, started = began || row_first != row_last;
+        if (ended) {
+            if (started) store(row_last, acc);
+            else { head = acc; has_head = true; }
+            acc = zero;
+            started = true;
+        }
+#pragma unroll
+        for (int d = G; d < 64; d *= 2) {
+            vec4u up;
+            up.x = __shfl_up(acc.x, d); up.y = __shfl_up(acc.y, d); up.z = __shfl_up(acc.z, d); up.w = __shfl_up(acc.w, d);
+            const bool started_up = __shfl_up((int)started, d) != 0;
+            if (lane >= d && !started) { acc += up; started = started_up; }
+        }
+        vec4u before = zero;
+        bool started_before = false;
+        if constexpr (NG > 1) {
+            before.x = __shfl_up(acc.x, G); before.y = __shfl_up(acc.y, G); before.z = __shfl_up(acc.z, G); before.w = __shfl_up(acc.w, G);
+            started_before = __shfl_up((int)started, G) != 0 && g > 0;
+            if (g == 0) before = zero;
+        }
+        if (has_head) {
+            head += before;
+            if (started_before) {
+                store(row_first, head);
+            } else {  // (one group of a wave at most: the first whose row ends)
+                head_sum[wave][l] = head;
+                if (l == 0) head_row[wave] = row_first;
+            }
+        }
+        if (g == NG - 1 && !ended) {
+            tail_sum[wave][l] = acc;
+            if (l == 0) { tail_row[wave] = row_last; tail_started[wave] = started; }
+        }
+    }
+    __syncthreads();
+    // The rows cut between the waves, the same way; only what is cut between workgroups is added atomically.
+    // (a wave whose last row ends with it has tail_started, and no sum)
+    auto with_waves_before = [&](int w, vec4u v, bool &started) -> vec4u {
+        while (!started && --w >= 0) {
+            if (tail_row[w] >= 0) v += tail_sum[w][l];
+            started = tail_started[w];
+        }
+        return v;
+    };
+    if (g > 0) return;
+    if (head_row[wave] >= 0) {
+        bool started = false;
+        const vec4u v = with_waves_before(wave, head_sum[wave][l], started);
+        if (started) store(head_row[wave], v);
+        else add(head_row[wave], v);
+    }
+    if (wave == NW - 1 && tail_row[wave] >= 0) {
+        bool started = tail_started[wave];
+        add(tail_row[wave], with_waves_before(wave, tail_sum[wave][l], started));
+    }
+}
+
+// K < 4: one lane per output column
+__global__ __launch_bounds__(256)
+void sddmm_spmm_generic_kernel(const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col_ind, const float *__restrict__ x,
+                               const float *__restrict__ H, float *Y, int64_t n_rows, int K)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t wave = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 6;
+    const int64_t n_waves = ((int64_t)gridDim.x * 256) >> 6;
+    for (int64_t r = wave; r < n_rows; r += n_waves) {
+        const int64_t b = row_ptr[r], e = row_ptr[r + 1];
+        for (int k = 0; k < K; ++k) {
+            float acc = 0.f;
+            for (int64_t p = b + lane; p < e; p += 64) acc = fmaf(x[p], H[(int64_t)col_ind[p] * K + k], acc);
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
+            if (lane == 0) Y[r * (int64_t)K + k] = acc;
+        }
+    }
+}
+
+int last_error(const char *who)
+{
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(SDDMM_ERR_HIP, "%s: %s", who, hipGetErrorString(e));
+    return SDDMM_OK;
+}
+
+}  // namespace
+
+extern "C" int sddmm_spmm_csr(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *d_row_ptr, const int32_t *d_col_ind,
+                              const float *d_x, int32_t K, const float *d_H, float *d_Y, void *stream)
+{
+    if (n_rows < 0 || n_cols < 0 || nnz < 0 || K < 1) return fail(SDDMM_ERR_ARG, "sddmm_spmm_csr: bad sizes");
+    if (n_rows == 0) return SDDMM_OK;
+    if (!d_row_ptr || !d_Y || (nnz > 0 && (!d_col_ind || !d_x || !d_H))) return fail(SDDMM_ERR_ARG, "sddmm_spmm_csr: NULL argument");
+    if (nnz >= INT32_MAX || n_rows >= INT32_MAX) return fail(SDDMM_ERR_RANGE, "sddmm_spmm_csr: sizes beyond int32 offsets");
+    hipStream_t st = (hipStream_t)stream;
+    if (K < 4) {
+        const unsigned grid = (unsigned)std::min<int64_t>((n_rows + 3) / 4, 256 * 64);
+        hipLaunchKernelGGL(sddmm_spmm_generic_kernel, dim3(grid), dim3(256), 0, st, d_row_ptr, d_col_ind, d_x, d_H, d_Y, n_rows, (int)K);
+        return last_error("sddmm_spmm_csr");
+    }
+    // slices of at most 64 pieces of a row, all of one width; the lanes of a group cover a slice
+    const int pieces = (K + 3) / 4, slices = (pieces + 63) / 64, slice_pieces = (pieces + slices - 1) / slices;
+    int G = 4;
+    while (G < slice_pieces) G *= 2;
+    // Nonzeros per wave: up to 512 (a workgroup's cut rows cost atomic adds), as many as leave 8192 waves, but not fewer
+    // than 64 until there are less than 2048 of them: too few waves leave the latency of the gathers bare.  Measured,
+    // us at 32 / 64 / 128 / 256 / 512 per wave: 253 thousand nonzeros, K = 256: 42 / 37 / 38 / 54 / -; 1.8 million, K = 100:
+    // 106 / 85 / 82 / 88 / 100; 98 million, K = 128: 5148 / 3483 / 3125 / 3029 / 2979.
+    const int groups_log2 = __builtin_ctz(64 / G);
+    int shift = 9 - groups_log2;
+    auto waves = [&] { return (nnz >> (shift + groups_log2)) * slices; };
+    while (shift > 2 && shift + groups_log2 > 6 && waves() < 8192) --shift;
+    while (shift > 2 && waves() < 2048) --shift;
+    const int S = 1 << shift;
+    hipLaunchKernelGGL(sddmm_spmm_zero_rows_kernel, dim3((unsigned)((n_rows + 255) / 256)), dim3(256), 0, st, d_row_ptr, d_Y, n_rows, (int)K,
+                       shift + groups_log2 + 2);
+    if (nnz > 0) {
+        const int64_t per_group = (int64_t)4 * S * (64 / G);
+        const dim3 grid((unsigned)((nnz + per_group - 1) / per_group), (unsigned)slices);
+#define SPMM(g) case g: hipLaunchKernelGGL((sddmm_spmm_csr_kernel<g>), grid, dim3(256), 0, st, d_row_ptr, d_col_ind, d_x, d_H, d_Y, \
+                                           (int)n_rows, (int)nnz, (int)K, S, slice_pieces); break
+        switch (G) { SPMM(4); SPMM(8); SPMM(16); SPMM(32); SPMM(64); }
+#undef SPMM
+    }
+    return last_error("sddmm_spmm_csr");
+}
