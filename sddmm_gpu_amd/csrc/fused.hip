@@ -12,14 +12,14 @@ namespace {
 // Row softmax.  Every row is worked on whole, in registers, by as many lanes as its length asks for, so
 // that an entry is read once and written once whatever the rows' lengths (a matrix may hold a few rows of
 // a million entries next to millions of rows of ten, so the work is cut by entries, not by rows):
-//   short rows (up to kSmChunk entries) are grouped into chunks of consecutive whole rows: chunk c
-//        starts with the row that holds entry c * kSmChunk and ends before the row that holds entry
-//        (c + 1) * kSmChunk.  A wave takes a chunk, 64 of its rows at a time: a lane per row of up to 8
+//   short rows (up to kSmShortMax entries) are grouped into chunks of consecutive whole rows: chunk c
+//        starts with the row that holds entry c * C and ends before the row that holds entry (c + 1) * C
+//        (C: see softmax_chunk_shift; a row of several C leaves all but its last chunk empty).  A wave takes a chunk, 64 of its rows at a time: a lane per row of up to 8
 //        entries, then groups of 8 lanes (up to 96), of 32 lanes (up to 512), the whole wave (up to 1024
 //        in registers, beyond that in two walks over the row).
 //   long rows (up to kSmLongMax entries) belong to no chunk: a workgroup each (the recommender shape
 //        keeps 56 % of its entries in rows of more than 4096).
-//   huge rows (beyond that) are cut at the multiples of kSmChunk: a workgroup takes a piece, stores it
+//   huge rows (beyond that) are cut at the multiples of C: a workgroup takes a piece, stores it
 //        as exp(x - m) with the piece's own maximum m and leaves (m, sum) in a record of the chunk; a last
 //        kernel merges the records of each huge row and scales its pieces.
 // Three kernels: the first lays the chunks out (one thread per chunk); the second takes the short rows
@@ -27,16 +27,26 @@ namespace {
 // lists that the second makes.  All read the number of entries from row_ptr[n_rows] on the device and walk
 // the chunks with a grid-sized stride.  No LDS staging: a
 // row's loads are all in flight together, and 16 waves per compute unit hide their latency.
-constexpr int kSmChunk = 4096;
+constexpr int kSmShortMax = 4096;                         // entries of a row that a wave works on
 constexpr int kSmBlock = 256;
-constexpr int64_t kSmMaxChunks = ((int64_t)1 << 31) / kSmChunk;
+constexpr int64_t kSmMaxChunks = ((int64_t)1 << 31) >> 12;  // (of 2^12 entries; fewer than 2^13 of the smaller ones)
 constexpr int kSmLongQ = 16;                             // float4 per thread of the long-row kernel
 constexpr int kSmLongMax = kSmLongQ * 4 * kSmBlock - 8;  // (less what a misaligned start costs)
 constexpr int kSmListRows = 1 << 30, kSmListHuge = 1 << 29, kSmListChunk = kSmListHuge - 1;  // an item of the last kernel's list: flags | chunk
 constexpr int kSmOwnBatches = 32;                       // batches of 64 rows that a chunk's own wave takes at least
 constexpr int kSmByLane = 8, kSmBy8 = 96, kSmBy32 = 512, kSmByWave16 = 1024;  // row lengths up to which a lane / 8 lanes / 32 lanes / the wave with 16 entries per lane work on a row
 
-__device__ __forceinline__ int softmax_row_class(int64_t len) { return len <= kSmChunk ? 0 : len <= kSmLongMax ? 1 : 2; }
+// log2 of the entries per chunk: 4096 on matrices with enough of them to give every wave of the machine a chunk
+// (4096 chunks), less below that, down to 64 -- a wave works through its chunk at memory latency, so few chunks leave
+// the machine idle: 18 thousand entries took 48 us as 5 chunks, 1.8 million 64 us as 447.
+__host__ __device__ inline int softmax_chunk_shift(int64_t nnz)
+{
+    int shift = 12;
+    while (shift > 6 && (nnz >> shift) < 4096) --shift;
+    return shift;
+}
+
+__device__ __forceinline__ int softmax_row_class(int64_t len) { return len <= kSmShortMax ? 0 : len <= kSmLongMax ? 1 : 2; }
 
 // (m, sum) of the pieces of huge rows: [2c] the row that began before chunk c, [2c + 1] the row that ends
 // after it; and the layout of each chunk: first entry, end, first row, last row.  The kernels take both
@@ -50,8 +60,8 @@ static __device__ __align__(256) int4 g_softmax_rows_store[kSmMaxChunks];
 static __device__ __align__(256) int32_t g_softmax_list_store[kSmMaxChunks + 64];
 
 // First kernel: the layout, one thread per chunk (a binary search of row_ptr whose loads the other
-// threads' searches hide).  With r the row that holds entry c * kSmChunk, chunk c begins at r's first
-// entry (r short), after r's last (r long; the chunk may come out empty) or at entry c * kSmChunk itself
+// threads' searches hide).  With r the row that holds entry c * C, chunk c begins at r's first
+// entry (r short), after r's last (r long; the chunk may come out empty) or at entry c * C itself
 // (r huge); it ends where chunk c + 1 would begin if that row were short (so a long row that starts
 // past the chunk's rows is left out) or at the multiple (huge).  The row of chunk c + 1 is the next
 // thread's search: a workgroup of 256 threads lays out 255 chunks (the kernel is bound by the number of
@@ -63,9 +73,10 @@ void sddmm_row_softmax_rows_kernel(const int32_t *__restrict__ row_ptr, int64_t 
     __shared__ int row_of[256], begin_of[256], end_of[256];  // the row that holds a chunk's first entry, and its extent
     if (blockIdx.x == 0 && threadIdx.x < 2) g_softmax_list[threadIdx.x] = 0;  // (the second kernel counts in them)
     const int64_t nnz = row_ptr[n_rows];
-    const int64_t n_chunks = (nnz + kSmChunk - 1) / kSmChunk;
+    const int shift = softmax_chunk_shift(nnz);
+    const int64_t n_chunks = (nnz + ((int64_t)1 << shift) - 1) >> shift;
     for (int64_t base = (int64_t)blockIdx.x * 255; base < n_chunks; base += (int64_t)gridDim.x * 255) {
-        const int64_t c = base + threadIdx.x, p0 = c * kSmChunk;
+        const int64_t c = base + threadIdx.x, p0 = c << shift, p1 = p0 + ((int64_t)1 << shift);
         int64_t lo0 = 0, b0 = 0, e0 = 0;
         if (c < n_chunks) {
             int64_t hi0 = n_rows - 1;  // first row whose end lies beyond p0
@@ -84,13 +95,13 @@ void sddmm_row_softmax_rows_kernel(const int32_t *__restrict__ row_ptr, int64_t 
         const int k0 = softmax_row_class(e0 - b0);
         lay.x = (int)(k0 == 0 ? b0 : k0 == 1 ? e0 : p0);
         lay.z = (int)(k0 == 1 ? lo0 + 1 : lo0);
-        if (p0 + kSmChunk >= nnz) {
+        if (p1 >= nnz) {
             lay.y = (int)nnz;
             lay.w = (int)(n_rows - 1);
-        } else {  // (chunk c + 1 exists: its first entry p0 + kSmChunk is an entry)
+        } else {  // (chunk c + 1 exists: its first entry p1 is an entry)
             const int64_t lo1 = row_of[threadIdx.x + 1], b1 = begin_of[threadIdx.x + 1], e1 = end_of[threadIdx.x + 1];
             const int k1 = softmax_row_class(e1 - b1);
-            lay.y = (int)(k1 == 2 ? p0 + kSmChunk : b1);
+            lay.y = (int)(k1 == 2 ? p1 : b1);
             lay.w = (int)(k1 == 2 ? lo1 : lo1 - 1);
         }
         g_softmax_rows[c] = lay;
@@ -204,7 +215,7 @@ __device__ __forceinline__ void softmax_row_batch(const int32_t *__restrict__ ro
             if (r <= last) {
                 rb = row_ptr[r];
                 const int64_t l = (int64_t)row_ptr[r + 1] - rb;
-                len = l <= kSmChunk ? (int)l : 0;  // (a huge row at either end of the chunk is not this kernel's)
+                len = l <= kSmShortMax ? (int)l : 0;  // (a huge row at either end of the chunk is not this kernel's)
             }
             // a lane per row
             if (__ballot(len >= 1 && len <= kSmByLane)) softmax_row_by_group<1, kSmByLane>(x + rb, out + rb, len, len <= kSmByLane);
@@ -255,7 +266,8 @@ __device__ __forceinline__ void softmax_short_rows(const int32_t *__restrict__ r
 {
     const int lane = threadIdx.x & 63;
     const int64_t nnz = row_ptr[n_rows];
-    const int64_t n_chunks = (nnz + kSmChunk - 1) / kSmChunk;
+    const int shift = softmax_chunk_shift(nnz);
+    const int64_t n_chunks = (nnz + ((int64_t)1 << shift) - 1) >> shift;
     const int64_t n_waves = n_groups * (kSmBlock / 64);
     const int64_t own = softmax_own_batches(n_rows, n_chunks);
     for (int64_t c = group * (kSmBlock / 64) + (threadIdx.x >> 6); c < n_chunks; c += n_waves) {
@@ -353,9 +365,9 @@ __device__ __forceinline__ void softmax_long_row(const float *x, float *out, int
     // (the next row writes its maxima after this row's second barrier and its sums after its own first: no barrier needed here)
 }
 
-// The long rows and the pieces of huge rows; workgroup `group` of `n_groups`.  A long row holds the multiple of kSmChunk
+// The long rows and the pieces of huge rows; workgroup `group` of `n_groups`.  A long row holds the multiple of C
 // that follows its first entry, so it is the row after the last row of the chunk whose window
-// [c * kSmChunk, (c + 1) * kSmChunk) it starts in; a huge row is the first or the last row of every chunk
+// [c C, (c + 1) C) it starts in; a huge row is the first or the last row of every chunk
 // it touches.  Workgroup b looks at the chunks b, b + n_groups, ...: first at many of them at once, a thread
 // per chunk (a few dependent loads each, which a walk chunk by chunk would pay for one after the other),
 // what it finds collected in a list; then the list item by item.
@@ -367,7 +379,8 @@ __device__ __forceinline__ void softmax_long_rows(const int32_t *__restrict__ ro
     __shared__ int4 todo[3 * kSmBlock];  // first entry, end, record (-1: a whole row)
     __shared__ int n_todo;
     const int64_t nnz = row_ptr[n_rows];
-    const int64_t n_chunks = (nnz + kSmChunk - 1) / kSmChunk;
+    const int shift = softmax_chunk_shift(nnz);
+    const int64_t n_chunks = (nnz + ((int64_t)1 << shift) - 1) >> shift;
     const bool vec_in = (reinterpret_cast<uintptr_t>(x) & 15u) == 0, vec_out = (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
     const int64_t own = softmax_own_batches(n_rows, n_chunks);
     for (int64_t base = group; base < n_chunks; base += n_groups * kSmBlock) {
@@ -381,7 +394,7 @@ __device__ __forceinline__ void softmax_long_rows(const int32_t *__restrict__ ro
             const int64_t r = (int64_t)lay.w + 1;
             if (r < n_rows) {
                 const int64_t rb = row_ptr[r], re = row_ptr[r + 1];
-                if (rb >= c * kSmChunk && rb < (c + 1) * kSmChunk && softmax_row_class(re - rb) == 1)
+                if ((rb >> shift) == c && softmax_row_class(re - rb) == 1)
                     todo[atomicAdd(&n_todo, 1)] = make_int4((int)rb, (int)re, -1, 0);
             }
             if (lay.x < lay.y) {
@@ -450,10 +463,10 @@ void sddmm_row_softmax_main_kernel(const int32_t *__restrict__ row_ptr, int64_t 
 
 // (m, sum) of the huge row [rb, re) from the records of the chunks it spans: the last-slot record of its
 // first chunk, the first-slot records of the others; every wave of the workgroup computes the same pair.
-__device__ __forceinline__ float2 merged_record(const float2 *__restrict__ g_softmax_rec, int64_t rb, int64_t re)
+__device__ __forceinline__ float2 merged_record(const float2 *__restrict__ g_softmax_rec, int64_t rb, int64_t re, int shift)
 {
     const int lane = threadIdx.x & 63;
-    const int64_t ca = rb / kSmChunk, cb = (re - 1) / kSmChunk;
+    const int64_t ca = rb >> shift, cb = (re - 1) >> shift;
     float m = -INFINITY, s = 0.f;
     for (int64_t k = ca + lane; k <= cb; k += 64) {
         const float2 rec = g_softmax_rec[2 * k + (k == ca ? 1 : 0)];
@@ -489,20 +502,20 @@ __device__ __forceinline__ void scale_range(float *out, int64_t b, int64_t e, fl
 // holds at most two of them: at its beginning (the row came from the chunk before, or fills this one and
 // goes on) and at its end.
 __device__ __forceinline__ void softmax_merge_chunk(const int32_t *__restrict__ row_ptr, float *out, const float2 *__restrict__ g_softmax_rec,
-                                                    const int4 *__restrict__ g_softmax_rows, int64_t c)
+                                                    const int4 *__restrict__ g_softmax_rows, int64_t c, int shift)
 {
     const int4 lay = g_softmax_rows[c];
     const int64_t c0 = lay.x, c1 = lay.y, r0 = lay.z, r1 = lay.w;
     const int64_t b0 = row_ptr[r0], e0 = row_ptr[r0 + 1], b1 = row_ptr[r1], e1 = row_ptr[r1 + 1];
     if (softmax_row_class(e0 - b0) == 2 && (b0 < c0 || e0 > c1)) {  // a huge row begins the chunk
-        const float2 all = merged_record(g_softmax_rec, b0, e0);
+        const float2 all = merged_record(g_softmax_rec, b0, e0, shift);
         const float2 mine = g_softmax_rec[2 * c + (b0 < c0 ? 0 : 1)];
         const float f = expf(mine.x - all.x) / all.y;
         const int64_t pb = max(b0, c0), pe = min(e0, c1);
         scale_range(out, pb, pe, f);
     }
     if (r1 != r0 && softmax_row_class(e1 - b1) == 2 && e1 > c1) {  // another one begins inside the chunk and ends after it
-        const float2 all = merged_record(g_softmax_rec, b1, e1);
+        const float2 all = merged_record(g_softmax_rec, b1, e1, shift);
         const float2 mine = g_softmax_rec[2 * c + 1];
         const float f = expf(mine.x - all.x) / all.y;
         scale_range(out, b1, c1, f);
@@ -528,7 +541,8 @@ void sddmm_row_softmax_merge_kernel(const int32_t *__restrict__ row_ptr, int64_t
     const int n_list = g_softmax_list[0], n_huge = g_softmax_list[1];
     if (n_list <= 0 && n_huge <= 0) return;
     const int64_t nnz = row_ptr[n_rows];
-    const int64_t n_chunks = (nnz + kSmChunk - 1) / kSmChunk;
+    const int shift = softmax_chunk_shift(nnz);
+    const int64_t n_chunks = (nnz + ((int64_t)1 << shift) - 1) >> shift;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t own = softmax_own_batches(n_rows, n_chunks), G = gridDim.x;
     for (int base = 0; base < n_list; base += kSmBlock) {
@@ -553,7 +567,7 @@ void sddmm_row_softmax_merge_kernel(const int32_t *__restrict__ row_ptr, int64_t
         const int n = n_todo;
         for (int q = 0; q < n; ++q) {
             if (todo_first[q] < 0) {
-                softmax_merge_chunk(row_ptr, out, g_softmax_rec, g_softmax_rows, -1 - todo_first[q]);
+                softmax_merge_chunk(row_ptr, out, g_softmax_rec, g_softmax_rows, -1 - todo_first[q], shift);
                 continue;
             }
             const int64_t last = todo_last[q];
@@ -563,7 +577,7 @@ void sddmm_row_softmax_merge_kernel(const int32_t *__restrict__ row_ptr, int64_t
         }
     }
     for (int64_t i = blockIdx.x; i < n_huge; i += G)
-        softmax_merge_chunk(row_ptr, out, g_softmax_rec, g_softmax_rows, g_softmax_list[n_chunks + 1 - i] & kSmListChunk);
+        softmax_merge_chunk(row_ptr, out, g_softmax_rec, g_softmax_rows, g_softmax_list[n_chunks + 1 - i] & kSmListChunk, shift);
 }
 
 int last_error(const char *who)
@@ -607,7 +621,8 @@ static int softmax_store(float2 **rec, int4 **rows, int32_t **list)
 
 int64_t row_softmax_workspace_bytes(int64_t nnz)
 {
-    const int64_t n_chunks = (nnz + kSmChunk - 1) / kSmChunk;
+    const int shift = softmax_chunk_shift(nnz);
+    const int64_t n_chunks = (nnz + ((int64_t)1 << shift) - 1) >> shift;
     return (((n_chunks * 36 + 8) + 255) / 256) * 256;  // two float2, one int4 and one list item per chunk, and the two lists' lengths
 }
 
@@ -618,7 +633,8 @@ int launch_row_softmax(int64_t n_rows, const int32_t *d_row_ptr, const float *d_
     int4 *rows = nullptr;
     int32_t *list = nullptr;
     if (d_ws) {  // [2 * n_chunks] records, then [n_chunks] chunk layouts, then the two lists: their lengths and [n_chunks] items
-        const int64_t n_chunks = (nnz + kSmChunk - 1) / kSmChunk;
+        const int shift = softmax_chunk_shift(nnz);
+    const int64_t n_chunks = (nnz + ((int64_t)1 << shift) - 1) >> shift;
         rec = static_cast<float2 *>(d_ws);
         rows = reinterpret_cast<int4 *>(rec + 2 * n_chunks);
         list = reinterpret_cast<int32_t *>(rows + n_chunks);
