@@ -343,37 +343,6 @@ int sddmm_execute_profiled(const sddmm_plan *plan, const float *d_val, const flo
     return SDDMM_OK;
 }
 
-int sddmm_gpu(const sddmm_plan *plan, const float *h_W, const float *h_H, float *h_out, float *kernel_ms)
-{
-    if (!plan || !h_W || !h_H || !h_out) return fail(SDDMM_ERR_ARG, "sddmm_gpu: NULL argument");
-    const sddmm_plan_info &I = plan->info;
-    float *dW = nullptr, *dH = nullptr, *dO = nullptr;
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    struct Free {
-        float *&a, *&b, *&c; hipEvent_t &e0, &e1;
-        ~Free() { if (a) (void)hipFree(a); if (b) (void)hipFree(b); if (c) (void)hipFree(c);
-                  if (e0) (void)hipEventDestroy(e0); if (e1) (void)hipEventDestroy(e1); }
-    } fr{dW, dH, dO, e0, e1};
-    const size_t wb = (size_t)std::max<int64_t>(I.n_rows * (int64_t)I.K, 1) * 4, hb = (size_t)std::max<int64_t>(I.n_cols * (int64_t)I.K, 1) * 4;
-    const size_t ob = (size_t)std::max<int64_t>(I.nnz, 1) * 4;
-    HIP_TRY(hipMalloc((void **)&dW, wb));
-    HIP_TRY(hipMalloc((void **)&dH, hb));
-    HIP_TRY(hipMalloc((void **)&dO, ob));
-    HIP_TRY(hipMemcpy(dW, h_W, (size_t)I.n_rows * I.K * 4, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(dH, h_H, (size_t)I.n_cols * I.K * 4, hipMemcpyHostToDevice));
-    HIP_TRY(hipEventCreate(&e0));
-    HIP_TRY(hipEventCreate(&e1));
-    HIP_TRY(hipEventRecord(e0, nullptr));
-    if (int rc = sddmm_execute(plan, nullptr, dW, dH, dO, nullptr)) return rc;
-    HIP_TRY(hipEventRecord(e1, nullptr));
-    HIP_TRY(hipEventSynchronize(e1));
-    float ms = 0.f;
-    HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
-    if (kernel_ms) *kernel_ms = ms;
-    HIP_TRY(hipMemcpy(h_out, dO, (size_t)I.nnz * 4, hipMemcpyDeviceToHost));
-    return SDDMM_OK;
-}
-
 int sddmm_device_info(int *n_devices, char *arch, int arch_len)
 {
     int n = 0;

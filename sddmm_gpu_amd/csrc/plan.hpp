@@ -2,6 +2,8 @@
 // and the functions that build them.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <memory>
+#include <mutex>
 #include "internal.hpp"
 #include "kernels.hpp"
 
@@ -47,6 +49,11 @@ struct Launch {
     int64_t sp_part_bytes = 0, ws_sp_part = 0;
 };
 
+namespace sddmm {
+struct HostCall;  // host_call.hip
+struct HostCallDelete { void operator()(HostCall *c) const; };
+}  // namespace sddmm
+
 struct sddmm_plan {
     sddmm_plan_info info{};
     std::vector<Launch> launches;
@@ -58,6 +65,8 @@ struct sddmm_plan {
     int32_t requested_kernel = 0;
     int64_t ws_softmax = 0, ws_bytes = 0;  // workspace layout: the launches' scratch, then the softmax pass's records
     sddmm_plan_options options{};  // what the plan was built with, environment overrides applied
+    mutable std::mutex host_mu;    // sddmm_gpu: one call at a time, with the device arrays it keeps
+    mutable std::unique_ptr<sddmm::HostCall, sddmm::HostCallDelete> host_call;
     ~sddmm_plan()
     {
         for (const Owned &o : owned) (void)hipFree(o.p);
