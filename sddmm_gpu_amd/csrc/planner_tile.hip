@@ -9,6 +9,61 @@
 
 namespace sddmm {
 
+namespace {
+
+// Deals the items of one group of workgroups out anew when their loads are uneven (a band or a window puts nearly
+// all nonzeros of a row block into a few column tiles; skewed columns do so less drastically): the items, in tile
+// order, are cut into consecutive pieces of `quantum` units and handed to the workgroups in order, each filled up to
+// the least load at which they all fit, where a piece costs its length and, for the first one of a tile, `stage`.
+// load(item) is an item's length in the units of cut(item, from, to).  Returns that least load.
+struct Piece {
+    int32_t item;
+    int64_t from, to;
+};
+int64_t deal_evenly(const std::vector<int64_t> &loads, const std::vector<int32_t> &tiles, size_t n_wgs, int64_t stage, int64_t quantum,
+                    std::vector<std::vector<Piece>> *out)
+{
+    int64_t total = 0;
+    for (int64_t l : loads) total += l;
+    auto fits = [&](int64_t most, std::vector<std::vector<Piece>> *seq) {
+        size_t w = 0;
+        int64_t used = 0;
+        int32_t held = -1;
+        for (size_t i = 0; i < loads.size(); ++i) {
+            int64_t at = 0;
+            while (at < loads[i]) {
+                const int64_t cost = held == tiles[i] ? 0 : stage;
+                const int64_t room = (most - used - cost) / quantum * quantum;
+                if (room <= 0) {
+                    if (++w >= n_wgs) return false;
+                    used = 0;
+                    held = -1;
+                    if (most <= stage) return false;
+                    continue;
+                }
+                const int64_t n = std::min(room, loads[i] - at);
+                if (seq) (*seq)[w].push_back({(int32_t)i, at, at + n});
+                at += n;
+                used += cost + n;
+                held = tiles[i];
+            }
+        }
+        return true;
+    };
+    int64_t lo = std::max<int64_t>(1, total / (int64_t)std::max<size_t>(n_wgs, 1)), hi = total + (stage + quantum) * ((int64_t)loads.size() + 1);
+    while (hi - lo > std::max<int64_t>(quantum, lo / 256)) {
+        const int64_t mid = (lo + hi) / 2;
+        if (fits(mid, nullptr)) hi = mid; else lo = mid;
+    }
+    if (out) {
+        out->assign(n_wgs, {});
+        fits(hi, out);
+    }
+    return hi;
+}
+
+}  // namespace
+
 // Tile launch: the rows' nonzeros in tile order (tiles of x columns), every
 // (row, tile) run padded to a multiple of G stream positions.
 int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t panel_rows, int want_g, int ks,
@@ -579,6 +634,64 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
             }
             // the product walks the same (row block, tile) items on the same workgroups
             if (want_spmm && !panel_local && item_keys.size() == items.size()) build_spmm(item_keys);
+            // uneven items (see deal_evenly): inside a die where the row blocks belong to dies, over all workgroups
+            // otherwise; in units of stream positions for the SDDMM and of rounds for the product
+            auto even = [&](std::vector<WorkItem> &list, int64_t stage, int64_t quantum, const std::function<int64_t(const WorkItem &)> &load,
+                            const std::function<WorkItem(const WorkItem &, int64_t, int64_t)> &cut_item) {
+                const int groups = xcd_local ? 8 : 1;
+                std::vector<std::vector<WorkItem>> seq((size_t)c.cus);
+                int64_t most_now = 0, most_new = 0, total = 0;
+                for (int b = 0; b < c.cus; ++b) {
+                    int64_t sum = 0;
+                    int32_t held = -1;
+                    for (size_t k = (size_t)b; k < list.size(); k += (size_t)c.cus) {
+                        if (list[k].end <= list[k].begin) continue;
+                        sum += load(list[k]) + (list[k].tile != held ? stage : 0);
+                        total += load(list[k]);
+                        held = list[k].tile;
+                    }
+                    most_now = std::max(most_now, sum);
+                }
+                // (what is nearly even keeps its whole tiles: here when no dealing can gain enough, below when this one does not)
+                if ((total / c.cus + stage) * 10 > most_now * 7) return;
+                for (int gr = 0; gr < groups; ++gr) {
+                    std::vector<WorkItem> mine;
+                    std::vector<int> wgs;
+                    for (int b = gr; b < c.cus; b += groups) {
+                        wgs.push_back(b);
+                        for (size_t k = (size_t)b; k < list.size(); k += (size_t)c.cus)
+                            if (list[k].end > list[k].begin) mine.push_back(list[k]);
+                    }
+                    std::stable_sort(mine.begin(), mine.end(), [](const WorkItem &u, const WorkItem &v) { return u.tile < v.tile; });
+                    std::vector<int64_t> loads;
+                    std::vector<int32_t> tiles;
+                    for (const WorkItem &w : mine) { loads.push_back(load(w)); tiles.push_back(w.tile); }
+                    std::vector<std::vector<Piece>> got;
+                    most_new = std::max(most_new, deal_evenly(loads, tiles, wgs.size(), stage, quantum, &got));
+                    for (size_t w = 0; w < wgs.size(); ++w)
+                        for (const Piece &pc : got[w]) seq[(size_t)wgs[w]].push_back(cut_item(mine[(size_t)pc.item], pc.from, pc.to));
+                }
+                if (most_new * 10 > most_now * 7) return;
+                size_t turns = 0;
+                for (auto &q : seq) turns = std::max(turns, q.size());
+                list.assign(turns * (size_t)c.cus, WorkItem{0, 0, 0, 0});
+                for (int b = 0; b < c.cus; ++b)
+                    for (size_t k = 0; k < seq[(size_t)b].size(); ++k) list[k * (size_t)c.cus + (size_t)b] = seq[(size_t)b][k];
+            };
+            // (staging a tile of x rows takes about as long as 8 x positions, at every rank)
+            if (!panel_local && mf_nwm == 0 && c.opt.tile_assign < 0) {
+                even(items, 8 * (int64_t)x, 64, [](const WorkItem &w) { return (int64_t)w.end - w.begin; },
+                     [&](const WorkItem &w, int64_t from, int64_t to) {
+                         return WorkItem{(int32_t)(w.begin + from), (int32_t)(w.begin + to), (int32_t)(w.batch_base + (shorts ? from / 64 : 0)), w.tile};
+                     });
+                if (sp.built) {
+                    auto bundle_at = [&](const WorkItem &w, int64_t round) {  // the first bundle that begins at or after a round of the item
+                        return (int32_t)(std::lower_bound(sp.b_off.begin() + w.begin, sp.b_off.begin() + w.end, sp.b_off[(size_t)w.begin] + (int32_t)round) - sp.b_off.begin());
+                    };
+                    even(sp.items, std::max<int64_t>(1, x / 8), 1, [&](const WorkItem &w) { return (int64_t)sp.b_off[(size_t)w.end] - sp.b_off[(size_t)w.begin]; },
+                         [&](const WorkItem &w, int64_t from, int64_t to) { return WorkItem{bundle_at(w, from), bundle_at(w, to), 0, w.tile}; });
+                }
+            }
         } else if (want_spmm && rb == 0 && rows.size() <= (size_t)panel_rows) {
             // (equal position ranges for the SDDMM: the product takes one item per column tile)
             std::vector<std::pair<int, int32_t>> keys;
