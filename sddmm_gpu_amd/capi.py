@@ -302,6 +302,8 @@ class Plan:
     def __init__(self, handle, keep=None):
         self.h = handle
         self._keep = keep  # device arrays the plan borrows
+        self._lib = lib()
+        self._execute = self._lib.sddmm_execute
 
     @classmethod
     def from_device_csr(cls, n_rows, n_cols, nnz, d_row_ptr, d_col_ind, K, tile_x=0, tile_y=0, kernel=KERNEL_AUTO,
@@ -338,17 +340,23 @@ class Plan:
         check(lib().sddmm_plan_get_info(self.h, byref(i)))
         return i.as_dict()
 
+    # (The calls below are what a program makes in every step: plain integers go straight through the declared
+    # argument types, 0 becomes NULL, and the functions are looked up once -- on small matrices a call costs as much as
+    # its kernels.)
     def execute(self, d_val, d_W, d_H, d_out, stream=0):
-        check(lib().sddmm_execute(self.h, c_void_p(d_val or None), c_void_p(d_W), c_void_p(d_H), c_void_p(d_out),
-                                  c_void_p(stream or None)))
+        rc = self._execute(self.h, d_val or None, d_W, d_H, d_out, stream or None)
+        if rc:
+            check(rc)
 
     def execute_epilogue(self, d_val, d_W, d_H, d_out, epilogue, stream=0):
-        check(lib().sddmm_execute_epilogue(self.h, c_void_p(d_val or None), c_void_p(d_W), c_void_p(d_H), c_void_p(d_out),
-                                           c_int32(epilogue), c_void_p(stream or None)))
+        rc = self._lib.sddmm_execute_epilogue(self.h, d_val or None, d_W, d_H, d_out, epilogue, stream or None)
+        if rc:
+            check(rc)
 
     def execute_softmax(self, d_val, d_W, d_H, d_out, stream=0):
-        check(lib().sddmm_execute_softmax(self.h, c_void_p(d_val or None), c_void_p(d_W), c_void_p(d_H), c_void_p(d_out),
-                                          c_void_p(stream or None)))
+        rc = self._lib.sddmm_execute_softmax(self.h, d_val or None, d_W, d_H, d_out, stream or None)
+        if rc:
+            check(rc)
 
     def workspace_bytes(self):
         n = c_int64()
@@ -357,12 +365,14 @@ class Plan:
 
     def execute_ws(self, d_val, d_W, d_H, d_out, d_workspace, workspace_bytes, form=0, stream=0):
         """sddmm_execute_ws: form = EPILOGUE_SCALE / EPILOGUE_RESIDUAL, ored with FORM_SOFTMAX."""
-        check(lib().sddmm_execute_ws(self.h, c_void_p(d_val or None), c_void_p(d_W), c_void_p(d_H), c_void_p(d_out), c_int32(form),
-                                     c_void_p(d_workspace or None), c_int64(workspace_bytes), c_void_p(stream or None)))
+        rc = self._lib.sddmm_execute_ws(self.h, d_val or None, d_W, d_H, d_out, form, d_workspace or None, workspace_bytes, stream or None)
+        if rc:
+            check(rc)
 
     def spmm(self, d_x, d_H, d_Y, d_workspace=0, workspace_bytes=0, stream=0):
-        check(lib().sddmm_plan_spmm(self.h, c_void_p(d_x or None), c_void_p(d_H), c_void_p(d_Y), c_void_p(d_workspace or None),
-                                    c_int64(workspace_bytes), c_void_p(stream or None)))
+        rc = self._lib.sddmm_plan_spmm(self.h, d_x or None, d_H, d_Y, d_workspace or None, workspace_bytes, stream or None)
+        if rc:
+            check(rc)
 
     def execute_profiled(self, d_val, d_W, d_H, d_out, stream=0):
         n = c_int32()
@@ -404,17 +414,21 @@ def init_reference(n, k):
 
 def csr_noalloc(n_rows, n_cols, nnz, d_row_ptr, d_col_ind, d_val, K, d_W, d_H, d_out, stream=0):
     """Plan-free SDDMM over a device CSR that allocates nothing (sddmm_csr_noalloc)."""
-    check(lib().sddmm_csr_noalloc(n_rows, n_cols, nnz, c_void_p(d_row_ptr), c_void_p(d_col_ind), c_void_p(d_val or None), K,
-                                  c_void_p(d_W), c_void_p(d_H), c_void_p(d_out), c_void_p(stream or None)))
+    rc = lib().sddmm_csr_noalloc(n_rows, n_cols, nnz, d_row_ptr, d_col_ind, d_val or None, K, d_W, d_H, d_out, stream or None)
+    if rc:
+        check(rc)
 
 
 def row_softmax(n_rows, d_row_ptr, d_x, d_out, stream=0):
-    check(lib().sddmm_row_softmax(n_rows, c_void_p(d_row_ptr), c_void_p(d_x), c_void_p(d_out), c_void_p(stream or None)))
+    rc = lib().sddmm_row_softmax(n_rows, d_row_ptr, d_x, d_out, stream or None)
+    if rc:
+        check(rc)
 
 
 def spmm_csr(n_rows, n_cols, nnz, d_row_ptr, d_col_ind, d_x, K, d_H, d_Y, stream=0):
-    check(lib().sddmm_spmm_csr(n_rows, n_cols, nnz, c_void_p(d_row_ptr), c_void_p(d_col_ind or None), c_void_p(d_x or None), K,
-                               c_void_p(d_H or None), c_void_p(d_Y), c_void_p(stream or None)))
+    rc = lib().sddmm_spmm_csr(n_rows, n_cols, nnz, d_row_ptr, d_col_ind or None, d_x or None, K, d_H or None, d_Y, stream or None)
+    if rc:
+        check(rc)
 
 
 def copy_probe(d_src, d_dst, n_bytes, stream=0):

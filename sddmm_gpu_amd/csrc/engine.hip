@@ -5,6 +5,7 @@
 #include <cstring>
 #include <new>
 #include <unistd.h>
+#include "launch.hpp"
 #include "plan.hpp"
 
 using namespace sddmm;
@@ -120,7 +121,7 @@ static int check_execute_args(const sddmm_plan *plan, const float *d_W, const fl
 
 // Issues the kernels of one launch-list entry (one per K slice) on `stream`.
 // ws: the caller's workspace (null: the plan's own scratch memory)
-static void issue_launch(const sddmm_plan *plan, const Launch &L, const float *d_val, const float *d_W,
+static hipError_t issue_launch(const sddmm_plan *plan, const Launch &L, const float *d_val, const float *d_W,
                          const float *d_H, float *d_out, hipStream_t stream, int epilogue = SDDMM_EPILOGUE_SCALE, char *ws = nullptr)
 {
     const int residual = epilogue == SDDMM_EPILOGUE_RESIDUAL;
@@ -134,15 +135,16 @@ static void issue_launch(const sddmm_plan *plan, const Launch &L, const float *d
         for (int k_off = 0; k_off < I.K; k_off += L.k_slice) {
             pa.k_off = k_off;
             pa.accumulate = k_off > 0;
-            hipLaunchKernelGGL(L.pfn, dim3((unsigned)L.grid), dim3((unsigned)L.block), (size_t)L.lds, stream, pa);
+            if (hipError_t e = launch(L.pfn, dim3((unsigned)L.grid), dim3((unsigned)L.block), (size_t)L.lds, stream, pa)) return e;
         }
+        return hipSuccess;
     } else if (L.dfn) {
         DenseArgs da = L.da;
         da.nz_val = d_val ? nullptr : L.sval;
         da.val = val;
         da.W = d_W; da.H = d_H; da.out = d_out;
         da.residual = residual;
-        hipLaunchKernelGGL(L.dfn, dim3((unsigned)L.grid), dim3((unsigned)L.block), 0, stream, da);
+        return launch(L.dfn, dim3((unsigned)L.grid), dim3((unsigned)L.block), 0, stream, da);
     } else if (L.tfn) {
         TileArgs ta = L.ta;
         ta.val = val;
@@ -164,14 +166,16 @@ static void issue_launch(const sddmm_plan *plan, const Launch &L, const float *d
         const bool sliced = L.k_slice < I.K;
         if (sliced && L.fused_slices) {
             ta.k_off = 0; ta.n_slices = I.K / L.k_slice; ta.to_part = 0;
-            hipLaunchKernelGGL(L.tfns[vm][3], dim3((unsigned)L.grid), dim3((unsigned)L.block), (size_t)L.lds, stream, ta);
-        } else
+            return launch(L.tfns[vm][3], dim3((unsigned)L.grid), dim3((unsigned)L.block), (size_t)L.lds, stream, ta);
+        }
         for (int k_off = 0; k_off < I.K; k_off += L.k_slice) {
             ta.k_off = k_off;
             ta.to_part = sliced && k_off + L.k_slice < I.K;
-            hipLaunchKernelGGL(L.tfns[vm][!sliced ? 0 : k_off == 0 ? 1 : 2], dim3((unsigned)L.grid), dim3((unsigned)L.block), (size_t)L.lds,
-                               stream, ta);
+            if (hipError_t e = launch(L.tfns[vm][!sliced ? 0 : k_off == 0 ? 1 : 2], dim3((unsigned)L.grid), dim3((unsigned)L.block), (size_t)L.lds,
+                                      stream, ta))
+                return e;
         }
+        return hipSuccess;
     } else {
         KArgs a = L.ka;
         a.col_ind = plan->d_col;
@@ -179,7 +183,7 @@ static void issue_launch(const sddmm_plan *plan, const Launch &L, const float *d
         a.sval = d_val ? nullptr : L.sval;
         a.W = d_W; a.H = d_H; a.out = d_out;
         a.residual = residual;
-        hipLaunchKernelGGL(L.fn, dim3((unsigned)L.grid), dim3((unsigned)L.block), (size_t)L.lds, stream, a);
+        return launch(L.fn, dim3((unsigned)L.grid), dim3((unsigned)L.block), (size_t)L.lds, stream, a);
     }
 }
 
@@ -188,8 +192,7 @@ int sddmm_execute(const sddmm_plan *plan, const float *d_val, const float *d_W, 
 {
     if (int rc = check_execute_args(plan, d_W, d_H, d_out, "sddmm_execute")) return rc;
     if (plan->info.nnz == 0) return SDDMM_OK;
-    for (const Launch &L : plan->launches) issue_launch(plan, L, d_val, d_W, d_H, d_out, (hipStream_t)stream);
-    HIP_TRY(hipGetLastError());
+    for (const Launch &L : plan->launches) HIP_TRY(issue_launch(plan, L, d_val, d_W, d_H, d_out, (hipStream_t)stream));
     return SDDMM_OK;
 }
 
@@ -202,8 +205,7 @@ int sddmm_execute_epilogue(const sddmm_plan *plan, const float *d_val, const flo
     if (epilogue == SDDMM_EPILOGUE_RESIDUAL && !d_val && !plan->d_val && plan->info.nnz > 0)
         return fail(SDDMM_ERR_ARG, "sddmm_execute_epilogue: the residual val - dot needs values (d_val or plan-owned)");
     if (plan->info.nnz == 0) return SDDMM_OK;
-    for (const Launch &L : plan->launches) issue_launch(plan, L, d_val, d_W, d_H, d_out, (hipStream_t)stream, epilogue);
-    HIP_TRY(hipGetLastError());
+    for (const Launch &L : plan->launches) HIP_TRY(issue_launch(plan, L, d_val, d_W, d_H, d_out, (hipStream_t)stream, epilogue));
     return SDDMM_OK;
 }
 
@@ -239,8 +241,7 @@ int sddmm_execute_ws(const sddmm_plan *plan, const float *d_val, const float *d_
                     (long long)plan->ws_bytes);
     if ((uintptr_t)d_workspace & 255u) return fail(SDDMM_ERR_ARG, "sddmm_execute_ws: the workspace must be 256-byte aligned");
     char *ws = static_cast<char *>(d_workspace);
-    for (const Launch &L : plan->launches) issue_launch(plan, L, d_val, d_W, d_H, d_out, (hipStream_t)stream, epilogue, ws);
-    HIP_TRY(hipGetLastError());
+    for (const Launch &L : plan->launches) HIP_TRY(issue_launch(plan, L, d_val, d_W, d_H, d_out, (hipStream_t)stream, epilogue, ws));
     if (!softmax) return SDDMM_OK;
     if (!plan->d_row_ptr) return fail(SDDMM_ERR_ARG, "sddmm_execute_ws: the plan holds no row pointers");
     return launch_row_softmax(plan->info.n_rows, plan->d_row_ptr, d_out, d_out, stream, ws + plan->ws_softmax, plan->info.nnz);
@@ -322,7 +323,7 @@ int sddmm_execute_profiled(const sddmm_plan *plan, const float *d_val, const flo
     for (auto &x : ev) HIP_TRY(hipEventCreate(&x));
     HIP_TRY(hipEventRecord(ev[0], (hipStream_t)stream));
     for (size_t i = 0; i < n; ++i) {
-        issue_launch(plan, plan->launches[i], d_val, d_W, d_H, d_out, (hipStream_t)stream);
+        HIP_TRY(issue_launch(plan, plan->launches[i], d_val, d_W, d_H, d_out, (hipStream_t)stream));
         HIP_TRY(hipEventRecord(ev[i + 1], (hipStream_t)stream));
     }
     HIP_TRY(hipGetLastError());

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <mutex>
 #include "internal.hpp"
+#include "launch.hpp"
 
 using namespace sddmm;
 
@@ -580,13 +581,6 @@ void sddmm_row_softmax_merge_kernel(const int32_t *__restrict__ row_ptr, int64_t
         softmax_merge_chunk(row_ptr, out, g_softmax_rec, g_softmax_rows, g_softmax_list[n_chunks + 1 - i] & kSmListChunk, shift);
 }
 
-int last_error(const char *who)
-{
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return fail(SDDMM_ERR_HIP, "%s: %s", who, hipGetErrorString(e));
-    return SDDMM_OK;
-}
-
 }  // namespace
 
 namespace sddmm {
@@ -643,12 +637,12 @@ int launch_row_softmax(int64_t n_rows, const int32_t *d_row_ptr, const float *d_
     }
     // (the entry count lives on the device: the grids are sized for the machine, the kernels stride over the chunks)
     const unsigned grid = 256 * 4;
-    hipLaunchKernelGGL(sddmm_row_softmax_rows_kernel, dim3(256), dim3(256), 0, (hipStream_t)stream, d_row_ptr, n_rows, rows, list);
-    hipLaunchKernelGGL(sddmm_row_softmax_main_kernel, dim3(6 * grid), dim3(kSmBlock), 0, (hipStream_t)stream, d_row_ptr, n_rows, d_x, d_out,
-                       rec, (const int4 *)rows, list);
-    hipLaunchKernelGGL(sddmm_row_softmax_merge_kernel, dim3(2 * grid), dim3(kSmBlock), 0, (hipStream_t)stream, d_row_ptr, n_rows, d_x,
-                       d_out, (const float2 *)rec, (const int4 *)rows, (const int32_t *)list);
-    return last_error("sddmm_row_softmax");
+    const hipStream_t st = (hipStream_t)stream;
+    hipError_t e = launch(sddmm_row_softmax_rows_kernel, dim3(256), dim3(256), 0, st, d_row_ptr, n_rows, rows, list);
+    if (e == hipSuccess) e = launch(sddmm_row_softmax_main_kernel, dim3(6 * grid), dim3(kSmBlock), 0, st, d_row_ptr, n_rows, d_x, d_out, rec, rows, list);
+    if (e == hipSuccess) e = launch(sddmm_row_softmax_merge_kernel, dim3(2 * grid), dim3(kSmBlock), 0, st, d_row_ptr, n_rows, d_x, d_out, rec, rows, list);
+    if (e != hipSuccess) return fail(SDDMM_ERR_HIP, "sddmm_row_softmax: %s", hipGetErrorString(e));
+    return SDDMM_OK;
 }
 
 }  // namespace sddmm

@@ -18,6 +18,7 @@
 #include <algorithm>
 #include "internal.hpp"
 #include "csr_walk.hpp"
+#include "launch.hpp"
 
 using namespace sddmm;
 
@@ -212,10 +213,9 @@ void sddmm_spmm_generic_kernel(const int32_t *__restrict__ row_ptr, const int32_
     }
 }
 
-int last_error(const char *who)
+int checked(hipError_t e)
 {
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return fail(SDDMM_ERR_HIP, "%s: %s", who, hipGetErrorString(e));
+    if (e != hipSuccess) return fail(SDDMM_ERR_HIP, "sddmm_spmm_csr: %s", hipGetErrorString(e));
     return SDDMM_OK;
 }
 
@@ -231,8 +231,7 @@ extern "C" int sddmm_spmm_csr(int64_t n_rows, int64_t n_cols, int64_t nnz, const
     hipStream_t st = (hipStream_t)stream;
     if (K < 4) {
         const unsigned grid = (unsigned)std::min<int64_t>((n_rows + 3) / 4, 256 * 64);
-        hipLaunchKernelGGL(sddmm_spmm_generic_kernel, dim3(grid), dim3(256), 0, st, d_row_ptr, d_col_ind, d_x, d_H, d_Y, n_rows, (int)K);
-        return last_error("sddmm_spmm_csr");
+        return checked(launch(sddmm_spmm_generic_kernel, dim3(grid), dim3(256), 0, st, d_row_ptr, d_col_ind, d_x, d_H, d_Y, n_rows, (int)K));
     }
     // slices of at most 64 pieces of a row, all of one width; the lanes of a group cover a slice
     const int pieces = (K + 3) / 4, slices = (pieces + 63) / 64, slice_pieces = (pieces + slices - 1) / slices;
@@ -248,15 +247,16 @@ extern "C" int sddmm_spmm_csr(int64_t n_rows, int64_t n_cols, int64_t nnz, const
     while (shift > 2 && shift + groups_log2 > 6 && waves() < 8192) --shift;
     while (shift > 2 && waves() < 2048) --shift;
     const int S = 1 << shift;
-    hipLaunchKernelGGL(sddmm_spmm_zero_rows_kernel, dim3((unsigned)((n_rows + 255) / 256)), dim3(256), 0, st, d_row_ptr, d_Y, n_rows, (int)K,
-                       shift + groups_log2 + 2);
+    if (int rc = checked(launch(sddmm_spmm_zero_rows_kernel, dim3((unsigned)((n_rows + 255) / 256)), dim3(256), 0, st, d_row_ptr, d_Y, n_rows,
+                                (int)K, shift + groups_log2 + 2)))
+        return rc;
     if (nnz > 0) {
         const int64_t per_group = (int64_t)4 * S * (64 / G);
         const dim3 grid((unsigned)((nnz + per_group - 1) / per_group), (unsigned)slices);
-#define SPMM(g) case g: hipLaunchKernelGGL((sddmm_spmm_csr_kernel<g>), grid, dim3(256), 0, st, d_row_ptr, d_col_ind, d_x, d_H, d_Y, \
-                                           (int)n_rows, (int)nnz, (int)K, S, slice_pieces); break
+#define SPMM(g) case g: return checked(launch(sddmm_spmm_csr_kernel<g>, grid, dim3(256), 0, st, d_row_ptr, d_col_ind, d_x, d_H, d_Y, \
+                                              (int)n_rows, (int)nnz, (int)K, S, slice_pieces))
         switch (G) { SPMM(4); SPMM(8); SPMM(16); SPMM(32); SPMM(64); }
 #undef SPMM
     }
-    return last_error("sddmm_spmm_csr");
+    return SDDMM_OK;
 }

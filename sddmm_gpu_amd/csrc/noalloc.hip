@@ -4,6 +4,7 @@
 #include <algorithm>
 #include "internal.hpp"
 #include "kernels.hpp"
+#include "launch.hpp"
 
 using namespace sddmm;
 
@@ -33,8 +34,7 @@ extern "C" int sddmm_csr_noalloc(int64_t n_rows, int64_t n_cols, int64_t nnz, co
     const int per_wave = (int)std::clamp<int64_t>(nnz / (64 * waves_wanted), 1, kRowGatherBatchesPerWave);
     a.chunk = 64 * per_wave * (kRowGatherBlock / 64);
     const int grid = (int)((nnz + a.chunk - 1) / a.chunk);
-    hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(kRowGatherBlock), 0, (hipStream_t)stream, a);
-    hipError_t e = hipGetLastError();
+    const hipError_t e = launch(fn, dim3((unsigned)grid), dim3(kRowGatherBlock), 0, (hipStream_t)stream, a);
     if (e != hipSuccess) return fail(SDDMM_ERR_HIP, "sddmm_csr_noalloc: launch failed: %s", hipGetErrorString(e));
     return SDDMM_OK;
 }
