@@ -88,7 +88,7 @@ typedef struct sddmm_plan_info {
     int64_t dense_blocks; /* its 128 x 128 blocks */
     int64_t matrix_nnz;   /* nonzeros of the LDS_TILE launch computed by its matrix-core waves (counted in class_nnz[0]) */
     int64_t matrix_rows;  /* the rows they belong to */
-    int64_t spmm_runs;    /* (row, tile) runs of the product's tile stream, one partial row of Y each (0: not built) */
+    int64_t spmm_runs;    /* (row, tile) runs of the product's tile stream (or cut rows' parts), one partial row of Y each (0: not built) */
 } sddmm_plan_info;
 
 const char *sddmm_last_error(void);
@@ -400,7 +400,9 @@ int sddmm_execute_ws(const sddmm_plan *plan, const float *d_val, const float *d_
  * (row, tile) runs: a group of 8 lanes adds x[p] * (its slice of the H row, read
  * from the column tile in LDS) over a run and writes one partial row; a second
  * kernel adds the partial rows of every row; the plan's other rows gather their
- * H rows as sddmm_spmm_csr does.  No atomics: the same bits on every call.  The
+ * H rows as sddmm_spmm_csr does.  (Runs of fewer than 12 entries on average: the
+ * whole product as sddmm_spmm_csr does it, with the parts of its cut rows written
+ * down and added up in order.)  No atomics: the same bits on every call.  The
  * partial rows (K floats per run; sddmm_plan_info.spmm_runs) live in the plan, or
  * in d_workspace (NULL, or as for sddmm_execute_ws).  Other plans (and H or Y not
  * 16-byte aligned) take the sddmm_spmm_csr path on the plan's pattern.  d_x: nnz

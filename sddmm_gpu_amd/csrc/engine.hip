@@ -257,7 +257,7 @@ int sddmm_plan_spmm(const sddmm_plan *plan, const float *d_x, const float *d_H, 
     const Launch *Ls = nullptr;
     for (const Launch &L : plan->launches)
         if (L.sp_on) Ls = &L;
-    if (!Ls || ((((uintptr_t)d_H) | ((uintptr_t)d_Y)) & 15u)) {
+    if (!Ls || (Ls->sp_on == 1 && ((((uintptr_t)d_H) | ((uintptr_t)d_Y)) & 15u))) {
         // no tile stream for the product in this plan: the CSR form, gathering H rows
         if (!plan->d_row_ptr || (I.nnz > 0 && !plan->d_col)) return fail(SDDMM_ERR_ARG, "sddmm_plan_spmm: the plan holds no pattern");
         return sddmm_spmm_csr(I.n_rows, I.n_cols, I.nnz, plan->d_row_ptr, plan->d_col, d_x, I.K, d_H, d_Y, stream);
@@ -266,6 +266,9 @@ int sddmm_plan_spmm(const sddmm_plan *plan, const float *d_x, const float *d_H, 
         if (workspace_bytes < plan->ws_bytes) return fail(SDDMM_ERR_ARG, "sddmm_plan_spmm: the plan needs a workspace of %lld bytes", (long long)plan->ws_bytes);
         if ((uintptr_t)d_workspace & 255u) return fail(SDDMM_ERR_ARG, "sddmm_plan_spmm: the workspace must be 256-byte aligned");
     }
+    if (Ls->sp_on == 2)
+        return launch_spmm_csr_records(I.n_rows, I.nnz, plan->d_row_ptr, plan->d_col, d_x, I.K, d_H, d_Y,
+                                       d_workspace ? reinterpret_cast<float *>(static_cast<char *>(d_workspace) + Ls->ws_sp_part) : Ls->sa.part, stream);
     SpmmArgs sa = Ls->sa;
     sa.x = d_x; sa.H = d_H; sa.Y = d_Y;
     sa.row_ptr = plan->d_row_ptr; sa.col_ind = plan->d_col;

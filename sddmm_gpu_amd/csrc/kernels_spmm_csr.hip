@@ -9,6 +9,8 @@
 // between waves through LDS; a row cut between workgroups is completed with fp32 atomic adds (the only place where
 // the order of additions can vary from run to run; with an add per group and cut row the atomics took half the
 // time).  The rows that need it -- those, and empty ones -- are zeroed by a kernel before this one.
+// Behind a plan (sddmm_plan_spmm) there is memory for a record per workgroup instead: the parts of rows cut between
+// workgroups go there, and a kernel after this one adds them up in order -- no atomics, the same bits on every call.
 //
 // What bounds it is the load path (64 bytes per clock and compute unit) and, for an H larger than the caches, the
 // fabric; what bounded the form before (a wave per 256 nonzeros, row by row: three dependent loads for every row)
@@ -49,10 +51,45 @@ void sddmm_spmm_zero_rows_kernel(const int32_t *__restrict__ row_ptr, float *Y, 
     }
 }
 
-template <int G>
+// The rows that the product with records leaves: empty rows become 0, rows cut between workgroups (of 2^shift
+// nonzeros) the sum of their records, workgroup by workgroup.
+__global__ __launch_bounds__(256)
+void sddmm_spmm_cut_rows_kernel(const int32_t *__restrict__ row_ptr, const float *__restrict__ part, float *Y, int64_t n_rows, int K, int shift)
+{
+    __shared__ int list[4][64];
+    __shared__ int2 range[4][64];  // first and last workgroup; (0, -1): an empty row
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    int s = 0, e = 1;
+    if (r < n_rows) { s = row_ptr[r]; e = row_ptr[r + 1]; }
+    const int w0 = s >> shift, w1 = (e - 1) >> shift;
+    const bool mine = r < n_rows && (s >= e || w0 != w1);
+    const uint64_t todo = __ballot(mine);
+    if (mine) {
+        const int i = __builtin_popcountll(todo & (((uint64_t)1 << lane) - 1));
+        list[wave][i] = (int)r;
+        range[wave][i] = s >= e ? make_int2(0, -1) : make_int2(w0, w1);
+    }
+    __builtin_amdgcn_wave_barrier();
+    const int pieces = (K + 3) >> 2, n = __builtin_popcountll(todo) * pieces;
+    for (int t = lane; t < n; t += 64) {
+        const int i = t / pieces, q = t - i * pieces;
+        const RowPiece pc = row_piece(q, K);
+        const int2 w = range[wave][i];
+        vec4u sum = {0.f, 0.f, 0.f, 0.f};
+        for (int k = w.x; k <= w.y; ++k)
+            sum += *reinterpret_cast<const vec4u *>(part + (2 * (size_t)k + (k < w.y ? 1 : 0)) * K + pc.off);
+        // (pieces at the end of a row may overlap: they hold the same sums)
+        *reinterpret_cast<vec4u *>(Y + (size_t)list[wave][i] * K + pc.off) = sum;
+    }
+}
+
+// RECORDS: part[(2 wg + 0) K ..] takes the part of a row that ends in workgroup wg and began before it, part[(2 wg + 1) K ..]
+// that of a row that goes on behind it.
+template <int G, bool RECORDS>
 __global__ __launch_bounds__(256)
 void sddmm_spmm_csr_kernel(const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col_ind, const float *__restrict__ x,
-                           const float *__restrict__ H, float *Y, int n_rows, int nnz, int K, int S, int slice_pieces)
+                           const float *__restrict__ H, float *Y, float *part, int n_rows, int nnz, int K, int S, int slice_pieces)
 {
     constexpr int NG = 64 / G, U = kSpmmUnroll, NW = 4;
     __shared__ int row_tab[NW][kSpmmMost + 1];
@@ -66,9 +103,7 @@ void sddmm_spmm_csr_kernel(const int32_t *__restrict__ row_ptr, const int32_t *_
     const int slot = blockIdx.y * slice_pieces + l;
     const RowPiece pc = row_piece(slot, K);
     const int first = l < slice_pieces ? pc.first : 4;  // (4: nothing of this lane's piece is written)
-    auto store = [&](int row, const vec4u &v) {
-        if (row >= n_rows) return;  // (past the last nonzero)
-        float *y = Y + (size_t)row * K + pc.off;
+    auto put = [&](float *y, const vec4u &v) {
         if (first == 0) {
             *reinterpret_cast<vec4u *>(y) = v;
         } else {
@@ -77,8 +112,15 @@ void sddmm_spmm_csr_kernel(const int32_t *__restrict__ row_ptr, const int32_t *_
             if (first <= 3) y[3] = v.w;
         }
     };
-    auto add = [&](int row, const vec4u &v) {
+    auto store = [&](int row, const vec4u &v) {
+        if (row < n_rows) put(Y + (size_t)row * K + pc.off, v);  // (n_rows: past the last nonzero)
+    };
+    auto add = [&](int row, const vec4u &v, int which) {
         if (row >= n_rows) return;
+        if constexpr (RECORDS) {
+            put(part + (2 * (size_t)blockIdx.x + which) * K + pc.off, v);
+            return;
+        }
         float *y = Y + (size_t)row * K + pc.off;
         if (first <= 0) unsafeAtomicAdd(y + 0, v.x);
         if (first <= 1) unsafeAtomicAdd(y + 1, v.y);
@@ -185,11 +227,11 @@ void sddmm_spmm_csr_kernel(const int32_t *__restrict__ row_ptr, const int32_t *_
         bool started = false;
         const vec4u v = with_waves_before(wave, head_sum[wave][l], started);
         if (started) store(head_row[wave], v);
-        else add(head_row[wave], v);
+        else add(head_row[wave], v, 0);
     }
     if (wave == NW - 1 && tail_row[wave] >= 0) {
         bool started = tail_started[wave];
-        add(tail_row[wave], with_waves_before(wave, tail_sum[wave][l], started));
+        add(tail_row[wave], with_waves_before(wave, tail_sum[wave][l], started), 1);
     }
 }
 
@@ -221,6 +263,66 @@ int checked(hipError_t e)
 
 }  // namespace
 
+namespace {
+
+// How the product over nnz nonzeros at rank K >= 4 is dealt out: lanes per group, log2 of the nonzeros per group and
+// of those per workgroup, slices of a row (of slice_pieces pieces each; the lanes of a group cover a slice).
+struct CsrShape {
+    int G, shift, wg_shift, slices, slice_pieces;
+    int64_t workgroups;
+};
+CsrShape csr_shape(int64_t nnz, int K)
+{
+    CsrShape c;
+    const int pieces = (K + 3) / 4;
+    c.slices = (pieces + 63) / 64;
+    c.slice_pieces = (pieces + c.slices - 1) / c.slices;
+    c.G = 4;
+    while (c.G < c.slice_pieces) c.G *= 2;
+    // Nonzeros per wave: up to 512 (a workgroup's cut rows cost atomic adds), as many as leave 8192 waves, but not fewer
+    // than 64 until there are less than 2048 of them: too few waves leave the latency of the gathers bare.  Measured,
+    // us at 32 / 64 / 128 / 256 / 512 per wave: 253 thousand nonzeros, K = 256: 42 / 37 / 38 / 54 / -; 1.8 million, K = 100:
+    // 106 / 85 / 82 / 88 / 100; 98 million, K = 128: 5148 / 3483 / 3125 / 3029 / 2979.
+    const int groups_log2 = __builtin_ctz(64 / c.G);
+    c.shift = 9 - groups_log2;
+    auto waves = [&] { return (nnz >> (c.shift + groups_log2)) * c.slices; };
+    while (c.shift > 2 && c.shift + groups_log2 > 6 && waves() < 8192) --c.shift;
+    while (c.shift > 2 && waves() < 2048) --c.shift;
+    c.wg_shift = c.shift + groups_log2 + 2;
+    c.workgroups = (nnz + ((int64_t)1 << c.wg_shift) - 1) >> c.wg_shift;
+    return c;
+}
+
+template <bool RECORDS>
+hipError_t launch_csr(const CsrShape &c, int64_t n_rows, int64_t nnz, const int32_t *row_ptr, const int32_t *col_ind, const float *x, int K,
+                      const float *H, float *Y, float *part, hipStream_t st)
+{
+    const dim3 grid((unsigned)c.workgroups, (unsigned)c.slices);
+#define SPMM(g) case g: return launch(sddmm_spmm_csr_kernel<g, RECORDS>, grid, dim3(256), 0, st, row_ptr, col_ind, x, H, Y, part, \
+                                      (int)n_rows, (int)nnz, K, 1 << c.shift, c.slice_pieces)
+    switch (c.G) { SPMM(4); SPMM(8); SPMM(16); SPMM(32); SPMM(64); }
+#undef SPMM
+    return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+namespace sddmm {
+
+int64_t spmm_csr_records(int64_t nnz, int K) { return K < 4 ? 0 : 2 * csr_shape(nnz, K).workgroups; }
+
+int launch_spmm_csr_records(int64_t n_rows, int64_t nnz, const int32_t *d_row_ptr, const int32_t *d_col_ind, const float *d_x, int32_t K,
+                            const float *d_H, float *d_Y, float *d_part, void *stream)
+{
+    const CsrShape c = csr_shape(nnz, K);
+    hipStream_t st = (hipStream_t)stream;
+    if (int rc = checked(launch_csr<true>(c, n_rows, nnz, d_row_ptr, d_col_ind, d_x, K, d_H, d_Y, d_part, st))) return rc;
+    return checked(launch(sddmm_spmm_cut_rows_kernel, dim3((unsigned)((n_rows + 255) / 256)), dim3(256), 0, st, d_row_ptr, d_part, d_Y, n_rows,
+                          (int)K, c.wg_shift));
+}
+
+}  // namespace sddmm
+
 extern "C" int sddmm_spmm_csr(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *d_row_ptr, const int32_t *d_col_ind,
                               const float *d_x, int32_t K, const float *d_H, float *d_Y, void *stream)
 {
@@ -233,30 +335,10 @@ extern "C" int sddmm_spmm_csr(int64_t n_rows, int64_t n_cols, int64_t nnz, const
         const unsigned grid = (unsigned)std::min<int64_t>((n_rows + 3) / 4, 256 * 64);
         return checked(launch(sddmm_spmm_generic_kernel, dim3(grid), dim3(256), 0, st, d_row_ptr, d_col_ind, d_x, d_H, d_Y, n_rows, (int)K));
     }
-    // slices of at most 64 pieces of a row, all of one width; the lanes of a group cover a slice
-    const int pieces = (K + 3) / 4, slices = (pieces + 63) / 64, slice_pieces = (pieces + slices - 1) / slices;
-    int G = 4;
-    while (G < slice_pieces) G *= 2;
-    // Nonzeros per wave: up to 512 (a workgroup's cut rows cost atomic adds), as many as leave 8192 waves, but not fewer
-    // than 64 until there are less than 2048 of them: too few waves leave the latency of the gathers bare.  Measured,
-    // us at 32 / 64 / 128 / 256 / 512 per wave: 253 thousand nonzeros, K = 256: 42 / 37 / 38 / 54 / -; 1.8 million, K = 100:
-    // 106 / 85 / 82 / 88 / 100; 98 million, K = 128: 5148 / 3483 / 3125 / 3029 / 2979.
-    const int groups_log2 = __builtin_ctz(64 / G);
-    int shift = 9 - groups_log2;
-    auto waves = [&] { return (nnz >> (shift + groups_log2)) * slices; };
-    while (shift > 2 && shift + groups_log2 > 6 && waves() < 8192) --shift;
-    while (shift > 2 && waves() < 2048) --shift;
-    const int S = 1 << shift;
+    const CsrShape c = csr_shape(nnz, K);
     if (int rc = checked(launch(sddmm_spmm_zero_rows_kernel, dim3((unsigned)((n_rows + 255) / 256)), dim3(256), 0, st, d_row_ptr, d_Y, n_rows,
-                                (int)K, shift + groups_log2 + 2)))
+                                (int)K, c.wg_shift)))
         return rc;
-    if (nnz > 0) {
-        const int64_t per_group = (int64_t)4 * S * (64 / G);
-        const dim3 grid((unsigned)((nnz + per_group - 1) / per_group), (unsigned)slices);
-#define SPMM(g) case g: return checked(launch(sddmm_spmm_csr_kernel<g>, grid, dim3(256), 0, st, d_row_ptr, d_col_ind, d_x, d_H, d_Y, \
-                                              (int)n_rows, (int)nnz, (int)K, S, slice_pieces))
-        switch (G) { SPMM(4); SPMM(8); SPMM(16); SPMM(32); SPMM(64); }
-#undef SPMM
-    }
-    return SDDMM_OK;
+    if (nnz == 0) return SDDMM_OK;
+    return checked(launch_csr<false>(c, n_rows, nnz, d_row_ptr, d_col_ind, d_x, K, d_H, d_Y, nullptr, st));
 }

@@ -43,7 +43,8 @@ struct Launch {
     // sizes, and where each lies in a caller's workspace (sddmm_execute_ws); the plan's own copies are in ta
     int64_t part_bytes = 0, hp_bytes = 0, wp_bytes = 0;
     int64_t ws_part = 0, ws_hp = 0, ws_wp = 0;
-    // the product Y = X H on this launch's tiles (spmm_stream = 1; sp_on == 0: not built)
+    // the product Y = X H (spmm_stream = 1): sp_on == 1 on this launch's tiles, 2 over the plan's CSR pattern with records
+    // in sa.part (see add_tile), 0 not built
     sddmm::SpmmArgs sa{};
     int32_t sp_on = 0, sp_grid = 0, sp_nwaves = 16;  // (16 waves per workgroup: 1.54 against 1.59 ms with 12 on the recommender shape)
     int64_t sp_part_bytes = 0, ws_sp_part = 0;

@@ -136,7 +136,7 @@ int resolve_functions(Launch &L)
     }
     case 3: {
         const TileVariant tv{L.fn_g, L.fn_kpl};
-        if (L.sp_on && spmm_tile_set_lds(L.k_slice, L.sp_nwaves, L.k_slice * 4 * L.ta.tile_x) != 0)
+        if (L.sp_on == 1 && spmm_tile_set_lds(L.k_slice, L.sp_nwaves, L.k_slice * 4 * L.ta.tile_x) != 0)
             return fail(SDDMM_ERR_HIP, "plan: cannot set up the tile kernel of the product Y = X H");
         if (L.fn_nwm > 0) {  // (a launch with a matrix-core share covers all of K: one form per value mode)
             for (int vm = 0; vm < 5; ++vm) {
