@@ -165,7 +165,7 @@ static hipError_t issue_launch(const sddmm_plan *plan, const Launch &L, const fl
         const int vm = residual ? (ta.sval ? 3 : 4) : ta.sval ? 0 : (val ? 1 : 2);
         const bool sliced = L.k_slice < I.K;
         if (sliced && L.fused_slices) {
-            ta.k_off = 0; ta.n_slices = I.K / L.k_slice; ta.to_part = 0;
+            ta.k_off = 0; ta.n_slices = (I.K + L.k_slice - 1) / L.k_slice; ta.to_part = 0;
             return launch(L.tfns[vm][3], dim3((unsigned)L.grid), dim3((unsigned)L.block), (size_t)L.lds, stream, ta);
         }
         for (int k_off = 0; k_off < I.K; k_off += L.k_slice) {
@@ -338,7 +338,7 @@ int sddmm_execute_profiled(const sddmm_plan *plan, const float *d_val, const flo
         prof[i].kernel = L.kind;
         prof[i].lanes_per_nnz = L.dfn ? 0 : L.kind == SDDMM_KERNEL_PANEL ? 8 : (L.tfn ? L.tile_g : L.gather_g);
         prof[i].k_slice = L.k_slice;
-        prof[i].n_kernel_launches = (L.k_slice > 0 && L.k_slice < plan->info.K && !L.fused_slices) ? plan->info.K / L.k_slice : 1;
+        prof[i].n_kernel_launches = (L.k_slice > 0 && L.k_slice < plan->info.K && !L.fused_slices) ? (plan->info.K + L.k_slice - 1) / L.k_slice : 1;
         prof[i].nnz = L.nnz;
         prof[i].rows = L.rows;
         prof[i].stream_positions = L.positions;

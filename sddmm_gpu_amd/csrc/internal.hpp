@@ -2,6 +2,10 @@
 #pragma once
 #include <cstdint>
 #include <cstdarg>
+#include <cstdlib>
+#include <new>
+#include <sys/mman.h>
+#include <utility>
 #include <vector>
 #include <thread>
 #include <algorithm>
@@ -15,6 +19,44 @@ struct sddmm_coo {
     int sorted = 0;  // 1: (row, col)-sorted.  Set by whatever creates or reorders the matrix, never lazily.
 };
 
+namespace sddmm {
+
+// Allocator of the planner's large arrays: what a container makes without a value stays as it comes from the system
+// (a plain vector writes zeros first, on one thread, and takes every page fault of the array there), and arrays of
+// several megabytes ask for huge pages.
+template <class T>
+struct big_alloc {
+    using value_type = T;
+    big_alloc() = default;
+    template <class U> big_alloc(const big_alloc<U> &) {}
+    T *allocate(size_t n) { return static_cast<T *>(big_allocate(n * sizeof(T))); }
+    void deallocate(T *p, size_t) { big_free(p); }
+    template <class U> void construct(U *) noexcept {}
+    template <class U, class A, class... R> void construct(U *p, A &&a, R &&...r) { ::new ((void *)p) U(std::forward<A>(a), std::forward<R>(r)...); }
+    template <class U> bool operator==(const big_alloc<U> &) const { return true; }
+    template <class U> bool operator!=(const big_alloc<U> &) const { return false; }
+    static void *big_allocate(size_t bytes);
+    static void big_free(void *p) { free(p); }
+};
+template <class T>
+void *big_alloc<T>::big_allocate(size_t bytes)
+{
+    constexpr size_t kHuge = (size_t)2 << 20;
+    void *p = nullptr;
+    if (bytes < 2 * kHuge) {
+        p = malloc(bytes ? bytes : 1);
+    } else if (posix_memalign(&p, kHuge, bytes) == 0) {
+        (void)madvise(p, bytes, MADV_HUGEPAGE);
+    } else {
+        p = nullptr;
+    }
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+template <class T> using big_vector = std::vector<T, big_alloc<T>>;
+
+}  // namespace sddmm
+
 // Tile-order view of a sorted matrix: tiles ascending, rows ascending inside a
 // tile, columns ascending inside a row (the order rewrite_matrix_1D produces,
 // HiPC18/src/util.h:267-343), stored compactly.
@@ -22,7 +64,7 @@ struct sddmm_tiling {
     int32_t tile_x = 0, tile_y = 0, n_tiles = 0;
     int64_t nnz = 0, n_rows = 0, n_cols = 0;
     std::vector<int32_t> tile_ptr;    // [n_tiles+1] offsets in tile order
-    std::vector<int32_t> tiled_ind;   // [nnz] original position of each tile-order nonzero
+    sddmm::big_vector<int32_t> tiled_ind;  // [nnz] original position of each tile-order nonzero
     std::vector<int64_t> active_ptr;  // [n_tiles+1] offsets into active_row/active_end
     std::vector<int32_t> active_row;  // global row id of each (tile, active row)
     std::vector<int32_t> active_end;  // tile-order end offset of that row's run

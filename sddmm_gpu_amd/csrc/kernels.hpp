@@ -54,6 +54,7 @@ struct TileArgs {
     const int32_t *scol;   // per stream position: byte offset of the column's H row inside the LDS tile;
                            // gather form: index of the H row's first float4, column * K/4
     const int32_t *grow;   // per group of G consecutive stream positions: index of the W row's first float4, row * K/4
+                           // (ragged ranks: of its first float, row * K; in the compact form row * 8)
     const float *sval;     // values in stream order or null
     // Compact form (LDS tiles of a K slice of at most 64 elements, where the kernel is bound by
     // the bytes it streams): scol16 replaces scol with the column's index inside the tile,
@@ -113,7 +114,9 @@ TileVariant pick_tile_variant(int K, int want_g);
 // vmode: 0 = values in stream order (sval), 1 = values in sorted order (val), 2 = no values
 // gather: H rows from global memory, 4 waves per workgroup (otherwise H tiles in LDS, nwaves = 16 or 12 waves)
 // slice: 0 the launch covers all of K, 1 first of several K slices, 2 a later one (see the kernel template)
-TileFn tile_kernel(const TileVariant &v, int vmode, bool gather, int slice, int nwaves);
+// ragged: the form for ranks that are no multiple of the variant's width (see the kernel template)
+TileFn tile_kernel(const TileVariant &v, int vmode, bool gather, int slice, int nwaves, bool ragged);
+int ragged_tile_width(int K);  // the width for such a rank (0: none)
 // The variant with a matrix-core share (TileArgs::mf_*): groups of 8 lanes on rows of 128 elements, all of K
 // in one launch, nw vector waves + nwm matrix-core waves per workgroup ((12, 4), (8, 8) or (8, 4)).
 TileFn tile_kernel_mf(int vmode, int nw, int nwm);

@@ -17,21 +17,25 @@ TileVariant pick_tile_variant(int K, int want_g)
     return best;
 }
 
-TileFn tile_kernel_part0(const TileVariant &v, int vmode, bool gather, int slice, int nwaves);
-TileFn tile_kernel_part1(const TileVariant &v, int vmode, bool gather, int slice, int nwaves);
-TileFn tile_kernel_part2(const TileVariant &v, int vmode, bool gather, int slice, int nwaves);
-TileFn tile_kernel_part3(const TileVariant &v, int vmode, bool gather, int slice, int nwaves);
-TileFn tile_kernel_part4(const TileVariant &v, int vmode, bool gather, int slice, int nwaves);
+// The width of the padded tile kernel that serves a rank it has no exact variant for: 32, 64 or 128 elements, beyond 128
+// slices of 128.  Below 8 most of a width of 32 would be padding.
+int ragged_tile_width(int K) { return K < 8 ? 0 : K <= 32 ? 32 : K <= 64 ? 64 : 128; }
+
+TileFn tile_kernel_part0(const TileVariant &v, int vmode, bool gather, int slice, int nwaves, bool ragged);
+TileFn tile_kernel_part1(const TileVariant &v, int vmode, bool gather, int slice, int nwaves, bool ragged);
+TileFn tile_kernel_part2(const TileVariant &v, int vmode, bool gather, int slice, int nwaves, bool ragged);
+TileFn tile_kernel_part3(const TileVariant &v, int vmode, bool gather, int slice, int nwaves, bool ragged);
+TileFn tile_kernel_part4(const TileVariant &v, int vmode, bool gather, int slice, int nwaves, bool ragged);
 
 // vmode: see the kernel template (where S.val comes from, which epilogue)
-TileFn tile_kernel(const TileVariant &v, int vmode, bool gather, int slice, int nwaves)
+TileFn tile_kernel(const TileVariant &v, int vmode, bool gather, int slice, int nwaves, bool ragged)
 {
     switch (vmode) {
-    case 0: return tile_kernel_part0(v, vmode, gather, slice, nwaves);
-    case 1: return tile_kernel_part1(v, vmode, gather, slice, nwaves);
-    case 2: return tile_kernel_part2(v, vmode, gather, slice, nwaves);
-    case 3: return tile_kernel_part3(v, vmode, gather, slice, nwaves);
-    case 4: return tile_kernel_part4(v, vmode, gather, slice, nwaves);
+    case 0: return tile_kernel_part0(v, vmode, gather, slice, nwaves, ragged);
+    case 1: return tile_kernel_part1(v, vmode, gather, slice, nwaves, ragged);
+    case 2: return tile_kernel_part2(v, vmode, gather, slice, nwaves, ragged);
+    case 3: return tile_kernel_part3(v, vmode, gather, slice, nwaves, ragged);
+    case 4: return tile_kernel_part4(v, vmode, gather, slice, nwaves, ragged);
     }
     return nullptr;
 }

@@ -27,6 +27,7 @@
 // steps one more exchange between the halves completes the dot products.
 #include <hip/hip_runtime.h>
 #include <utility>
+#include "csr_walk.hpp"
 #include "kernels.hpp"
 
 using namespace sddmm;
@@ -295,17 +296,22 @@ __device__ __forceinline__ void matrix_core_waves(const TileArgs &a, int mw, int
 // launch costs as much as its work): a wave meets the same positions in every slice, so the partial
 // results it left in a.part are its own, and a workgroup barrier between the slices is all the
 // ordering needed.
+// RAGGED: K is no multiple of the kernel's width (K <= 4 * G * KPL: one launch; else the last of several slices is cut
+// short), and K needs no alignment: H rows are staged with the tail filled up with zeros, W rows are read in pieces at
+// any 4-byte address, the one at the end of the row from its last four floats on with what it shares with the piece
+// before masked to zero (see RowPiece; the H tail is staged the same way).  4 v_cndmask per piece and batch more.
 // NWM > 0: the workgroup has NWM more waves, which run the matrix-core share of the launch
 // (matrix_core_waves) and take no part in staging or in the stream; the NW vector waves then
 // synchronise among themselves through a counter in LDS, since a hardware barrier would wait
 // for all waves.
-template <int G, int KPL, int VMODE, int NW, bool GATHER, int SLICE, int NWM = 0>
+template <int G, int KPL, int VMODE, int NW, bool GATHER, int SLICE, int NWM = 0, bool RAGGED = false>
 __global__ __launch_bounds__((NW + NWM) * 64)
 void sddmm_tile_kernel(const TileArgs a)
 {
     constexpr bool FUSED = SLICE == 3;
     constexpr bool ACC = SLICE == 2;
     constexpr bool PART = SLICE >= 1;
+    static_assert(!RAGGED || (!GATHER && NWM == 0));
     extern __shared__ float4 lds_tile[];
     constexpr int K4 = G * KPL;
     constexpr bool RESIDUAL = VMODE >= 3;
@@ -411,6 +417,22 @@ void sddmm_tile_kernel(const TileArgs a)
     const int k_off = a.k_off + sl * 4 * K4;
     const float4 *__restrict__ W4 = reinterpret_cast<const float4 *>(a.W) + (k_off >> 2);
     const float4 *__restrict__ H4 = reinterpret_cast<const float4 *>(a.H) + (k_off >> 2);
+    int w_off[RAGGED ? KPL : 1], w_first[RAGGED ? KPL : 1];  // this lane's pieces of a W row
+    if constexpr (RAGGED) {
+#pragma unroll
+        for (int j = 0; j < KPL; ++j) {
+            const RowPiece pc = row_piece(slot[j], a.K - k_off);
+            w_off[j] = pc.off;
+            w_first[j] = pc.first;
+        }
+    }
+    auto from_piece = [](vec4u v, int first) -> vec4u {
+        v.x = first > 0 ? 0.f : v.x;
+        v.y = first > 1 ? 0.f : v.y;
+        v.z = first > 2 ? 0.f : v.z;
+        v.w = first > 3 ? 0.f : v.w;
+        return v;
+    };
     if (FUSED && sl > 0) wg_sync();  // everyone is done with the slice before: its tile, and its partial results are stored
     int cur_tile = -1;
     for (int step = 0; step < n_steps; ++step) {
@@ -439,21 +461,26 @@ void sddmm_tile_kernel(const TileArgs a)
             // (eight loads in flight per lane: a workgroup with many tiles in its turn -- a wide matrix --
             // spends its time between tiles waiting for these, one memory latency per round)
             constexpr int kStageUnroll = 8, kStride = NW * 64;
+            // 16 bytes of the tile: piece q of the tile's row r
+            auto stage_piece = [&](int ii) -> float4 {
+                const int r = ii / K4, q = ii - r * K4;
+                if constexpr (RAGGED) {
+                    const RowPiece pc = row_piece(q, a.K - k_off);
+                    const vec4u v = from_piece(*reinterpret_cast<const vec4u *>(a.H + ((size_t)(tile_base + r) * a.K + k_off) + pc.off), pc.first);
+                    return make_float4(v.x, v.y, v.z, v.w);
+                } else {
+                    return src[(size_t)r * row_k4 + q];
+                }
+            };
             int i = threadIdx.x;
             for (; i + (kStageUnroll - 1) * kStride < n4; i += kStageUnroll * kStride) {
                 float4 v[kStageUnroll];
 #pragma unroll
-                for (int u = 0; u < kStageUnroll; ++u) {
-                    const int ii = i + u * kStride, r = ii / K4, q = ii - r * K4;
-                    v[u] = src[(size_t)r * row_k4 + q];
-                }
+                for (int u = 0; u < kStageUnroll; ++u) v[u] = stage_piece(i + u * kStride);
 #pragma unroll
                 for (int u = 0; u < kStageUnroll; ++u) lds_tile[i + u * kStride] = v[u];
             }
-            for (; i < n4; i += kStride) {
-                const int r = i / K4, q = i - r * K4;
-                lds_tile[i] = src[(size_t)r * row_k4 + q];
-            }
+            for (; i < n4; i += kStride) lds_tile[i] = stage_piece(i);
             wg_sync();
         }
         const int nb = (end - begin + 63) >> 6;
@@ -485,7 +512,7 @@ void sddmm_tile_kernel(const TileArgs a)
             Meta m;
             if constexpr (COMPACT) {
                 const uint32_t g = ld_meta<STREAM_HINT>(reinterpret_cast<const uint32_t *>(grow_b + og));
-                m.wrow = g & ~(uint32_t)(G - 1);
+                m.wrow = RAGGED ? (g >> 3) * (uint32_t)a.K : g & ~(uint32_t)(G - 1);
                 m.p = ld_meta<STREAM_HINT>(reinterpret_cast<const uint32_t *>(perm_b + og)) + min((uint32_t)l, g & (uint32_t)(G - 1));
                 m.col = (int)ld_meta<STREAM_HINT>(reinterpret_cast<const uint16_t *>(scol_b + (o4 >> 1))) << ROW_SHIFT;
             } else {
@@ -506,7 +533,7 @@ void sddmm_tile_kernel(const TileArgs a)
             const uint32_t tg = (t4 / (4 * G)) << 2;
             if constexpr (COMPACT) {
                 const uint32_t g = *reinterpret_cast<const uint32_t *>(grow_b + tg);
-                m.wrow = g & ~(uint32_t)(G - 1);
+                m.wrow = RAGGED ? (g >> 3) * (uint32_t)a.K : g & ~(uint32_t)(G - 1);
                 m.p = *reinterpret_cast<const uint32_t *>(perm_b + tg) + min((t4 >> 2) & (uint32_t)(G - 1), g & (uint32_t)(G - 1));
                 m.col = (int)*reinterpret_cast<const uint16_t *>(scol_b + (t4 >> 1)) << ROW_SHIFT;
             } else {
@@ -532,6 +559,15 @@ void sddmm_tile_kernel(const TileArgs a)
         };
         // wrow: float4 index of the row's first element in W
         auto issue_w = [&](float4 (&w)[KPL], uint32_t wrow) {
+            if constexpr (RAGGED) {  // (wrow: index of the row's first float)
+                const float *wr = a.W + k_off + wrow;
+#pragma unroll
+                for (int j = 0; j < KPL; ++j) {
+                    const vec4u v = *reinterpret_cast<const vec4u *>(wr + w_off[j]);
+                    w[j] = make_float4(v.x, v.y, v.z, v.w);
+                }
+                return;
+            }
             const float4 *wbase[NB];  // piece j is at wbase[j % NB] + a compile-time offset
             wbase[0] = W4 + (wrow + (uint32_t)slot[0]);
 #pragma unroll
@@ -557,9 +593,18 @@ void sddmm_tile_kernel(const TileArgs a)
         // c[I]: where the H row this lane works on in step I starts (LDS: byte address of
         // this lane's first piece; gather form: float4 index of the row); cn: the same for the next batch, requested here after the last LDS
         // read so that the latency hides behind the reduction
-        auto compute = [&]<bool SHORT>(std::bool_constant<SHORT>, const float4 (&w)[KPL], const Meta &m, const int (&c)[G],
+        auto compute = [&]<bool SHORT>(std::bool_constant<SHORT>, const float4 (&w_in)[KPL], const Meta &m, const int (&c)[G],
                                        int (&cn)[G], int next_col) {
             constexpr int STEPS = SHORT ? G / 2 : G;
+            float4 w[KPL];
+#pragma unroll
+            for (int j = 0; j < KPL; ++j) {
+                w[j] = w_in[j];
+                if constexpr (RAGGED) {
+                    const vec4u v = from_piece(vec4u{w_in[j].x, w_in[j].y, w_in[j].z, w_in[j].w}, w_first[j]);
+                    w[j] = make_float4(v.x, v.y, v.z, v.w);
+                }
+            }
             float v = m.sv;
             if (SORTED_VAL) v = a.val[GATHER ? (m.p & 0x7fffffffu) : m.p];
             float acc[STEPS];
@@ -698,6 +743,23 @@ TileFn fused_slices_kernel()
 {
     if constexpr (G == 8 && KPL == 4) return (TileFn)sddmm_tile_kernel<G, KPL, VMODE, NW, GATHER, 3>;
     else return nullptr;
+}
+
+// The ragged form exists for the widths the planner rounds other ranks up to: 32, 64 and 128 elements, and of the sliced
+// forms for slices of 128; null for everything else.
+template <int VMODE>
+TileFn ragged_tile_kernel(const TileVariant &v, bool gather, int slice, int nwaves)
+{
+    if (gather) return nullptr;
+    if (v.G == 4 && v.KPL == 2 && nwaves == 16 && slice == 0) return (TileFn)sddmm_tile_kernel<4, 2, VMODE, 16, false, 0, 0, true>;
+    if (v.G == 4 && v.KPL == 4 && nwaves == 12 && slice == 0) return (TileFn)sddmm_tile_kernel<4, 4, VMODE, 12, false, 0, 0, true>;
+    if (v.G == 8 && v.KPL == 4 && nwaves == 12) {
+        if (slice == 0) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 0, 0, true>;
+        if (slice == 1) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 1, 0, true>;
+        if (slice == 2) return (TileFn)sddmm_tile_kernel<8, 4, (VMODE == 4 ? 3 : VMODE), 12, false, 2, 0, true>;
+        if (slice == 3) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 3, 0, true>;
+    }
+    return nullptr;
 }
 
 }  // namespace

@@ -37,6 +37,7 @@ struct Launch {
     // what the function pointers above were looked up with (they are looked up again when a saved plan is loaded)
     int32_t fn_kind = 0;  // 1 stream kernel (row gather), 2 stream kernel with an LDS tile, 3 tile kernel, 4 panel, 5 dense
     int32_t fn_g = 0, fn_kpl = 0, fn_exact = 0, fn_gather = 0, fn_nwaves = 0;
+    int32_t fn_ragged = 0;  // tile kernel: the form for ranks that are no multiple of its width
     int32_t fn_nwm = 0;  // tile kernel: waves per workgroup that run the launch's matrix-core share (0: none)
     int32_t fused_slices = 0;  // sliced tile launch small enough that its K slices run inside one kernel launch
     // Scratch memory of the launch (partial results between K slices; packed operands of the matrix-core share):
@@ -85,8 +86,8 @@ __host__ __device__ inline uint64_t mix64(uint64_t x)
     return x;
 }
 
-template <class T>
-int upload(T **dst, const std::vector<T> &src, int64_t *bytes)
+template <class T, class A>
+int upload(T **dst, const std::vector<T, A> &src, int64_t *bytes)
 {
     *dst = nullptr;
     if (src.empty()) return SDDMM_OK;
@@ -113,8 +114,8 @@ struct Ctx {
     int32_t pos(int64_t p) const { return orig ? orig[p] : (int32_t)p; }
     float value(int64_t p) const { return vals[orig ? orig[p] : p]; }
 
-    template <class T>
-    int up(T **dst, const std::vector<T> &src)
+    template <class T, class A>
+    int up(T **dst, const std::vector<T, A> &src)
     {
         int rc = upload(dst, src, &dev_bytes);
         if (rc == SDDMM_OK && *dst) P->owned.push_back({(void *)*dst, src.size() * sizeof(T)});
@@ -151,6 +152,7 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
               const float *vals, const int32_t *d_row_ptr_borrowed, const int32_t *d_col_borrowed, int32_t K,
               const sddmm_plan_options &opt_in, sddmm_plan **out);
 // planner_tile.hip: the rows' nonzeros in tile order (tiles of x columns), every (row, tile) run padded
+// ks: K elements per launch, a divisor of K or (ragged ranks) the width K is rounded up to
 int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t panel_rows, int want_g, int ks,
              sddmm_plan_info *I, bool gather = false, bool x_explicit = false);
 }  // namespace sddmm

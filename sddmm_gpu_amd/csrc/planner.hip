@@ -60,7 +60,9 @@ int count_touched(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *ro
     for (int64_t r = 0; r < n_rows; ++r) rt += row_ptr[r + 1] > row_ptr[r];
     std::vector<uint8_t> seen((size_t)n_cols, 0);
     parallel_ranges(nnz, 1 << 16, [&](int64_t b, int64_t e, int) {
-        for (int64_t i = b; i < e; ++i) __atomic_store_n(&seen[col_ind[i]], (uint8_t)1, __ATOMIC_RELAXED);
+        // (looked at before it is written: the threads would pass the lines of popular columns back and forth)
+        for (int64_t i = b; i < e; ++i)
+            if (!__atomic_load_n(&seen[col_ind[i]], __ATOMIC_RELAXED)) __atomic_store_n(&seen[col_ind[i]], (uint8_t)1, __ATOMIC_RELAXED);
     });
     int64_t ct = 0;
     for (int64_t c = 0; c < n_cols; ++c) ct += seen[c];
@@ -150,8 +152,9 @@ int resolve_functions(Launch &L)
         }
         for (int vm = 0; vm < 5; ++vm)
             for (int ac = 0; ac < 4; ++ac) {
-                L.tfns[vm][ac] = tile_kernel(tv, vm, L.fn_gather != 0, ac, L.fn_nwaves);
+                L.tfns[vm][ac] = tile_kernel(tv, vm, L.fn_gather != 0, ac, L.fn_nwaves, L.fn_ragged != 0);
                 if (!L.tfns[vm][ac] && ac == 3) { L.fused_slices = 0; continue; }  // (that form exists for some variants only)
+                if (!L.tfns[vm][ac] && ac > 0 && L.fn_ragged && L.k_slice >= L.ta.K) continue;  // (one launch: no sliced forms needed)
                 if (!L.tfns[vm][ac]) return fail(SDDMM_ERR_ARG, "plan: no tile kernel for lanes %d x %d", tv.G, tv.KPL);
                 HIP_TRY(hipFuncSetAttribute((const void *)L.tfns[vm][ac], hipFuncAttributeMaxDynamicSharedMemorySize, L.lds));
             }
@@ -540,6 +543,59 @@ void assign_workspace(sddmm_plan *P)
     P->ws_bytes = at;
 }
 
+// The split of the rows over the tile kernel and the gather that a model of the two finds cheapest, from a sample of
+// the rows.  Microseconds of one launch of the tile kernel, per K slice of w elements: 5.5, plus the H tiles staged (once
+// for every row block) at the rate of the fabric, plus 2.7 / 4.8 / 6.0 ps per stream position at w = 32 / 64 / 128 (a chunk
+// of at most half a group's positions counts half where short batches exist), plus the W row of every (row, tile) run
+// at 21 TB/s, 7 where W is larger than the dies' L2s together.  Of the gather: 4.5, plus an H row per nonzero at 18
+// TB/s (14 for rows of less than 256 bytes) while H fits one die's L2, 11.5 up to 64 MB, 8 beyond.  A second launch: 3.
+// Measured over 60 matrices of 0.1 to 28 M nonzeros (power-law, word counts, R-MAT, uniform, banded; K from 11 to 512)
+// the fixed rules this replaces were more than 10 % from the best of the three on 21 of them, up to 1.7 times.
+enum class Split { all_tiled, by_length, all_gathered };
+static Split estimate_split(const Ctx &c, const std::vector<int32_t> &rows, int w, int32_t x, int g, int64_t short_max)
+{
+    const size_t n = rows.size();
+    if (n == 0) return Split::all_gathered;
+    // a sample of whole rows, evenly spaced, of about a million nonzeros at most
+    const size_t stride = std::max<size_t>({1, n / 4096, (size_t)((double)c.nnz / 1.0e6)});
+    struct Class { double nnz = 0, runs = 0, pos = 0; } lng, shrt;
+    const bool shorts = tile_variant_shorts(g, w / (4 * g), false);
+    double sampled = 0;
+    for (size_t i = stride / 2; i < n; i += stride) {
+        const int32_t b = c.row_ptr[rows[i]], e = c.row_ptr[rows[i] + 1];
+        Class &k = e - b >= short_max ? lng : shrt;
+        sampled += e - b;
+        k.nnz += e - b;
+        for (int32_t p = b; p < e;) {
+            const int64_t end = ((int64_t)c.col_ind[p] / x + 1) * x;
+            int32_t q = p + 1;
+            while (q < e && c.col_ind[q] < end) ++q;
+            const int len = q - p, r = len % g;
+            k.runs += 1;
+            k.pos += len - r + (r == 0 ? 0 : shorts && r <= g / 2 ? g / 2 + 0.5 : g);
+            p = q;
+        }
+    }
+    if (sampled <= 0) return Split::by_length;
+    const double f = (double)c.nnz / sampled;
+    const double slices = (c.K + w - 1) / w, K = c.K;
+    const double tiles = (double)((c.n_cols + x - 1) / x), h_slice = (double)c.n_cols * std::min<double>(w, K) * 4, h_all = (double)c.n_cols * K * 4;
+    const double blocks = tiles >= c.cus ? 1.0 : std::min(8.0, c.cus / tiles);
+    const double stage_us = h_slice * blocks / (h_slice <= 4.0e6 ? 20.0e6 : 5.3e6);
+    const double ps = w <= 32 ? 2.7 : w <= 64 ? 4.8 : 6.0;
+    const double w_rate = (double)c.n_rows * w * 4 <= 32.0e6 ? 21.0 : 7.0;  // bytes per ps
+    auto tile_us = [&](double runs, double pos) {
+        return slices * (5.5 + stage_us + 1e-6 * f * (pos * ps + runs * std::max(128.0, std::min<double>(w, K) * 4) / w_rate));
+    };
+    const double h_rate = h_all <= 4.2e6 ? (K * 4 >= 256 ? 18.0 : 14.0) : h_all <= 64.0e6 ? 11.5 : 8.0;
+    auto gather_us = [&](double nnz) { return 4.5 + 1e-6 * f * nnz * K * 4 / h_rate; };
+    // (the tile kernel's time is underestimated where its items are uneven: 12 % more)
+    const double t_tile = 1.12 * tile_us(lng.runs + shrt.runs, lng.pos + shrt.pos), t_gather = gather_us(lng.nnz + shrt.nnz);
+    const double t_both = lng.nnz > 0 && shrt.nnz > 0 ? 3.0 + 1.12 * tile_us(lng.runs, lng.pos) + gather_us(shrt.nnz) : 1e30;
+    if (t_both < t_tile && t_both < t_gather) return Split::by_length;
+    return t_tile < t_gather ? Split::all_tiled : Split::all_gathered;
+}
+
 // Common plan builder from host CSR arrays.  d_*_borrowed != null: the device
 // already holds that array.
 int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_ptr_all, const int32_t *col_ind_all,
@@ -612,6 +668,8 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
     else if (K > 128 && K % 64 == 0) kt = 64;
     else if (pick_tile_variant(K, 0).G) kt = K;
     if (opt.k_slice > 0 && K % opt.k_slice == 0 && pick_tile_variant(opt.k_slice, 0).G) kt = opt.k_slice;
+    const bool ragged = kt == 0;  // no exact width: the tile kernel in a width K is rounded up to
+    if (ragged) kt = ragged_tile_width(K);
     const int32_t fit_t = kt ? kLdsMaxBytes / (kt * 4) : 0;  // H rows per LDS tile of the tile kernel
 
     // row-panel height of the tile kernel's stream: the panel's W slice (y rows of kt floats)
@@ -686,7 +744,7 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
             span = acc / (double)cnt;
         }
         const double tiles = std::max(1.0, span / std::max(1, x));
-        const int g_long = pick_tile_variant(kt, opt.tile_lanes).G ? pick_tile_variant(kt, opt.tile_lanes).G : pick_tile_variant(kt, 0).G;
+        const int g_long = !ragged && pick_tile_variant(kt, opt.tile_lanes).G ? pick_tile_variant(kt, opt.tile_lanes).G : pick_tile_variant(kt, 0).G;
         // rows with at least short_max nonzeros (2 per column tile with groups of 8 lanes) go to the tile kernel
         int64_t short_max = (int64_t)std::max(4.0, (g_long == 8 ? 2.0 : 1.0 * g_long) * tiles);
         if (opt.short_row_max >= 0) short_max = opt.short_row_max;
@@ -697,34 +755,35 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
             if (d >= short_max) { rl.push_back(r); nl += d; }
             else { rs.push_back(r); nsh += d; }
         }
+        auto join = [&](std::vector<int32_t> &into, std::vector<int32_t> &from, int64_t &n_into, int64_t &n_from) {
+            if (from.empty()) return;
+            into.insert(into.end(), from.begin(), from.end());
+            n_into += n_from; n_from = 0; from.clear();
+            std::sort(into.begin(), into.end());
+        };
+        // By default the split that a model of the three kernels finds cheapest (see estimate_split): all rows tiled,
+        // the long ones tiled and the short ones gathered, or all gathered.  A caller who sets one of the thresholds,
+        // and the remainder of a dense core, get the fixed rules.
+        const bool by_model = D.n_dense == 0 && opt.short_row_max < 0 && opt.stage_factor < 0 && opt.split_min_nnz < 0;
+        if (by_model) {
+            switch (estimate_split(c, ne, kt, x, g_long, short_max)) {
+            case Split::all_tiled: join(rl, rs, nl, nsh); break;
+            case Split::all_gathered: join(rs, rl, nsh, nl); break;
+            case Split::by_length: break;
+            }
+        }
         // staging every H tile must be paid for by the nonzeros that use it
         const int64_t n_tiles_all = (n_cols + x - 1) / x;
         const int64_t stage_rows = std::max<int64_t>(n_tiles_all, c.cus) * x;
-        if (nl < (opt.stage_factor >= 0 ? opt.stage_factor : 8) * stage_rows) {
-            rs.insert(rs.end(), rl.begin(), rl.end());
-            nsh += nl; nl = 0; rl.clear();
-            std::sort(rs.begin(), rs.end());
-        }
+        if (!by_model && nl < (opt.stage_factor >= 0 ? opt.stage_factor : 8) * stage_rows) join(rs, rl, nsh, nl);
         // a small problem is one launch: splitting it only adds launch latency
-        if (nl && nnz_part < (opt.split_min_nnz >= 0 ? opt.split_min_nnz : (int64_t)4 * 1000 * 1000)) {
-            rl.insert(rl.end(), rs.begin(), rs.end());
-            nl += nsh; nsh = 0; rs.clear();
-            std::sort(rl.begin(), rl.end());
-        }
+        if (!by_model && nl && nnz_part < (opt.split_min_nnz >= 0 ? opt.split_min_nnz : (int64_t)4 * 1000 * 1000)) join(rl, rs, nl, nsh);
         // a class too small to fill the machine joins the other
-        if (!rl.empty() && !rs.empty() && nl * 50 < nnz_part) {
-            rs.insert(rs.end(), rl.begin(), rl.end());
-            nsh += nl; nl = 0; rl.clear();
-            std::sort(rs.begin(), rs.end());
-        }
+        if (!by_model && !rl.empty() && !rs.empty() && nl * 50 < nnz_part) join(rs, rl, nsh, nl);
         // (a handful of short rows -- the clipped rows at the corners of a band -- are not worth a launch
         // of their own: a single workgroup would walk them batch by batch at memory latency;
         // banded 2^20, K = 512: 711 nonzeros took 0.065 ms of a 4.14 ms step)
-        if (!rl.empty() && !rs.empty() && opt.short_row_max < 0 && nsh * 2000 < nnz_part) {
-            rl.insert(rl.end(), rs.begin(), rs.end());
-            nl += nsh; nsh = 0; rs.clear();
-            std::sort(rl.begin(), rl.end());
-        }
+        if (!rl.empty() && !rs.empty() && opt.short_row_max < 0 && nsh * 2000 < nnz_part) join(rl, rs, nl, nsh);
         if (!rl.empty())
             if (int rc = add_tile(c, rl, x, y_panel, opt.tile_lanes, kt, &I, false, tile_x > 0)) return rc;
         if (!rs.empty()) {
@@ -738,8 +797,8 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
             const bool huge_h = rl.empty() && D.n_dense == 0 && (int64_t)n_cols * K * 4 > ((int64_t)256 << 20);
             int gg = opt.gather_lanes > 0 ? opt.gather_lanes : 8;
             if (huge_h && opt.gather_lanes <= 0 && opt.gather_slab_cols != 0 && pick_tile_variant(kt, 4).G) gg = 4;
-            const bool slabs = huge_h && opt.gather_slab_cols != 0 && opt.gather_padded != 0 && pick_tile_variant(kt, gg).G != 0;
-            const bool padded = opt.gather_padded != 0 && pick_tile_variant(kt, gg).G != 0 && (!rl.empty() || D.n_dense > 0 || slabs);
+            const bool slabs = !ragged && huge_h && opt.gather_slab_cols != 0 && opt.gather_padded != 0 && pick_tile_variant(kt, gg).G != 0;
+            const bool padded = !ragged && opt.gather_padded != 0 && pick_tile_variant(kt, gg).G != 0 && (!rl.empty() || D.n_dense > 0 || slabs);
             if (padded) {
                 const int64_t keep = c.opt.gather_slab_cols;
                 if (slabs && keep < 0) c.opt.gather_slab_cols = std::max<int64_t>(1024, ((int64_t)32 << 20) / ((int64_t)K * 4));
@@ -768,7 +827,7 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         I.kernel = kernel; I.class_nnz[0] = nnz; I.class_rows[0] = (int64_t)ne.size();
     } else {
         const int gg = opt.gather_lanes > 0 ? opt.gather_lanes : 0;
-        if (opt.row_padded > 0 && kt && pick_tile_variant(kt, gg).G != 0) {
+        if (opt.row_padded > 0 && kt && !ragged && pick_tile_variant(kt, gg).G != 0) {
             if (int rc = add_tile(c, ne, 0, 0, gg, kt, &I, true)) return rc;
         } else if (int rc = add_row_gather(c, ne, true)) return rc;
         I.kernel = SDDMM_KERNEL_ROW_GATHER; I.class_nnz[2] = nnz; I.class_rows[2] = (int64_t)ne.size();
@@ -779,7 +838,7 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         if (int rc = c.need_row_ptr()) return rc;
     if (!P->launches.empty() && I.grid == 0) { I.grid = P->launches[0].grid; I.block = P->launches[0].block; I.lds_bytes = P->launches[0].lds; }
     I.n_launches = 0;
-    for (const Launch &L : P->launches) I.n_launches += (L.k_slice > 0 && L.k_slice < K && !L.fused_slices) ? K / L.k_slice : 1;
+    for (const Launch &L : P->launches) I.n_launches += (L.k_slice > 0 && L.k_slice < K && !L.fused_slices) ? (K + L.k_slice - 1) / L.k_slice : 1;
     I.device_bytes = c.dev_bytes;
     assign_workspace(P);
     I.plan_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();

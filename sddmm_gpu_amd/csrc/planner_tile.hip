@@ -81,18 +81,26 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         panel_rows = c.opt.gather_panel_rows > 0 ? (int32_t)std::min<int64_t>(c.opt.gather_panel_rows, INT32_MAX) : INT32_MAX;
     }
     L.rows = (int64_t)rows_in.size();
-    const TileVariant tv = pick_tile_variant(ks, want_g);  // ks: K elements per launch (K itself or a slice of it)
+    const bool ragged = c.K % ks != 0;  // (ks >= K: one launch of that width; ks < K: the last slice is cut short)
+    const TileVariant tv = pick_tile_variant(ks, ragged ? 0 : want_g);  // ks: K elements per launch (K itself or a slice of it)
     // 12 waves per workgroup measured 2-5 % faster than 16 on slices of 64 and 128, slower on 32
     int nwaves = gather ? 4 : (int)(c.opt.tile_waves > 0 ? c.opt.tile_waves : (ks >= 64 ? 12 : 16));
     if (!gather && nwaves != 12) nwaves = 16;
-    if (!tv.G || !tile_kernel(tv, 0, gather, 0, nwaves)) return fail(SDDMM_ERR_ARG, "plan: no tile kernel for K = %d", c.K);
-    L.fn_kind = 3; L.fn_g = tv.G; L.fn_kpl = tv.KPL; L.fn_gather = gather; L.fn_nwaves = nwaves;
+    if (ragged) nwaves = ks >= 64 ? 12 : 16;
+    if (!tv.G || !tile_kernel(tv, 0, gather, 0, nwaves, ragged)) return fail(SDDMM_ERR_ARG, "plan: no tile kernel for K = %d", c.K);
+    L.fn_kind = 3; L.fn_g = tv.G; L.fn_kpl = tv.KPL; L.fn_gather = gather; L.fn_nwaves = nwaves; L.fn_ragged = ragged;
     const int G = tv.G;
     L.nnz = list_nnz(c, rows_in);
     if (L.nnz == 0) return SDDMM_OK;
     // the kernel addresses W (and, in the gather form, H) rows by 32-bit float4 indices
+    // (ragged ranks: by 32-bit float indices, in the compact stream computed from a row number of 28 bits)
+    if (ragged && ((int64_t)c.n_rows * c.K > (int64_t)UINT32_MAX || c.n_rows >= ((int64_t)1 << 28))) return add_row_gather(c, rows_in, false);
     if ((int64_t)c.n_rows * (c.K / 4) > (int64_t)UINT32_MAX || (gather && (int64_t)c.n_cols * (c.K / 4) > (int64_t)UINT32_MAX))
         return add_row_gather(c, rows_in, false);
+    const bool compact = !gather && ks / 4 <= 16;  // the compact stream format (see TileArgs)
+    auto row_word = [&](int32_t row) {  // what grow holds for a row
+        return (int32_t)((uint32_t)row * (ragged ? (compact ? 8u : (uint32_t)c.K) : (uint32_t)(c.K / 4)));
+    };
     // Work assignment.  grid2d: every workgroup owns one column tile for good (its H
     // tile is staged once) and one of `shares` row blocks that are the same for all
     // tiles, so the workgroups of different tiles read the same W rows at about the same
@@ -210,11 +218,9 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
     // (panel, tile) pair with nonzeros is a "unit"; workgroups that work on the units of
     // one panel at the same time share its W rows in L2.
     if (panel_rows < 1) panel_rows = 1;
-    std::vector<int32_t> perm, scol, grow, unit_ptr, unit_tile;
-    std::vector<float> sval;
-    const size_t guess = (size_t)(L.nnz + L.nnz / 4);
-    perm.reserve(guess); scol.reserve(guess); grow.reserve(guess / G + 1);
-    if (c.vals) sval.reserve(guess);
+    big_vector<int32_t> perm, scol, grow;
+    std::vector<int32_t> unit_ptr, unit_tile;
+    big_vector<float> sval;
     std::vector<int64_t> poff;
     std::vector<int32_t> seg_tile;
     int64_t np = 0;
@@ -229,7 +235,9 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         // Runs of less than 12 nonzeros: a partial row of Y per run is written and read for little work, and the product
         // goes over the CSR pattern instead (attention window, 16,384 tokens, K = 64, runs of 10: 131 -> 65 us; K = 32, runs
         // of 8: 146 -> 46 us; ratings, K = 128, runs of 16: 98 against 124 us at 4.9 M nonzeros, 435 against 388 at 19 M).
-        if (want_spmm && rb == 0 && c.nnz == c.P->info.nnz && L.nnz < 12 * n_seg) { want_spmm = false; sp_csr = true; }
+        // Below 4 million nonzeros the two are level at best (0.5 M, K = 128: 27 us) or the walk is far ahead (window
+        // of 101, 8,898 tokens, K = 32, runs of 14: 110 against 25 us).
+        if (want_spmm && rb == 0 && c.nnz == c.P->info.nnz && (ragged || L.nnz < 12 * n_seg || L.nnz < 4000000)) { want_spmm = false; sp_csr = true; }
         // row-block boundaries of the 2-D assignment: equal shares of the rows' nonzeros
         std::vector<int32_t> cut;
         auto make_cuts = [&](int n_shares) {
@@ -333,11 +341,16 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
                     if (np >= INT32_MAX - 4096) return fail(SDDMM_ERR_RANGE, "plan: padded stream beyond int32 offsets");
                 }
             }
-            perm.assign((size_t)np, 0); scol.assign((size_t)np, 0); grow.assign((size_t)(np / G), 0);
-            if (c.vals) sval.assign((size_t)np, 0.f);
+            // (zeroed by all threads: the positions behind an item's last nonzero, up to a whole batch, stay so)
+            auto zeroed = [&](auto &v, int64_t n) {
+                v.reserve((size_t)n + kStreamSlack);
+                v.resize((size_t)n);
+                parallel_ranges(n, 1 << 16, [&](int64_t b, int64_t e, int) { std::fill(v.begin() + b, v.begin() + e, 0); });
+            };
+            zeroed(perm, np); zeroed(scol, np); zeroed(grow, np / G);
+            if (c.vals) zeroed(sval, np);
             std::vector<uint8_t> is_short((size_t)n_batches, 0);
             const int32_t row_bytes = ks * 4;
-            const uint32_t k4 = (uint32_t)(c.K / 4);
             parallel_ranges((int64_t)lay.size(), 1, [&](int64_t ib, int64_t ie, int) {
                 struct Chunk { int64_t sg, e0; int cnt; };
                 for (int64_t ii = ib; ii < ie; ++ii) {
@@ -366,7 +379,7 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
                             perm[(size_t)d] = perm[(size_t)d - span]; scol[(size_t)d] = scol[(size_t)d - span];
                             if (c.vals) sval[(size_t)d] = sval[(size_t)d - span];
                         }
-                        grow[(size_t)(d0 / G)] = (int32_t)((uint32_t)T.active_row[ch.sg] * k4);
+                        grow[(size_t)(d0 / G)] = row_word(T.active_row[ch.sg]);
                     };
                     auto emit = [&](const Chunk *q, int n, bool is_s) {
                         const int64_t d0 = it.begin + next * 64;
@@ -418,6 +431,10 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         }
         const int64_t np_new = shorts ? np : poff[n_seg];
         if (np_new >= INT32_MAX - 4096) return fail(SDDMM_ERR_RANGE, "plan: padded stream beyond int32 offsets");
+        if (n_panels == 0) {
+            perm.reserve((size_t)np_new + kStreamSlack); scol.reserve((size_t)np_new + kStreamSlack); grow.reserve((size_t)(np_new / G) + kStreamSlack);
+            if (c.vals) sval.reserve((size_t)np_new + kStreamSlack);
+        }
         perm.resize((size_t)np_new); scol.resize((size_t)np_new); grow.resize((size_t)(np_new / G));
         if (c.vals) sval.resize((size_t)np_new);
         parallel_ranges(shorts ? 0 : n_seg, 1 << 10, [&](int64_t sb, int64_t se, int) {
@@ -443,7 +460,7 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
                     scol[d] = scol[d - 1];
                     if (c.vals) sval[d] = sval[d - 1];
                 }
-                for (int64_t g = poff[s] / G; g < poff[s + 1] / G; ++g) grow[g] = (int32_t)((uint32_t)T.active_row[s] * k4);
+                for (int64_t g = poff[s] / G; g < poff[s + 1] / G; ++g) grow[g] = row_word(T.active_row[s]);
             }
         });
         np = np_new;
@@ -683,9 +700,9 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
                 for (int b = 0; b < c.cus; ++b)
                     for (size_t k = 0; k < seq[(size_t)b].size(); ++k) list[k * (size_t)c.cus + (size_t)b] = seq[(size_t)b][k];
             };
-            // (staging a tile of x rows takes about as long as 8 x positions, at every rank)
+            // (staging a tile of x rows takes about as long as 4 x positions of one workgroup, at every rank)
             if (!panel_local && mf_nwm == 0 && c.opt.tile_assign < 0) {
-                even(items, 8 * (int64_t)x, 64, [](const WorkItem &w) { return (int64_t)w.end - w.begin; },
+                even(items, 4 * (int64_t)x, 64, [](const WorkItem &w) { return (int64_t)w.end - w.begin; },
                      [&](const WorkItem &w, int64_t from, int64_t to) {
                          return WorkItem{(int32_t)(w.begin + from), (int32_t)(w.begin + to), (int32_t)(w.batch_base + (shorts ? from / 64 : 0)), w.tile};
                      });
@@ -693,7 +710,7 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
                     auto bundle_at = [&](const WorkItem &w, int64_t round) {  // the first bundle that begins at or after a round of the item
                         return (int32_t)(std::lower_bound(sp.b_off.begin() + w.begin, sp.b_off.begin() + w.end, sp.b_off[(size_t)w.begin] + (int32_t)round) - sp.b_off.begin());
                     };
-                    even(sp.items, std::max<int64_t>(1, x / 8), 1, [&](const WorkItem &w) { return (int64_t)sp.b_off[(size_t)w.end] - sp.b_off[(size_t)w.begin]; },
+                    even(sp.items, std::max<int64_t>(1, x / 16), 1, [&](const WorkItem &w) { return (int64_t)sp.b_off[(size_t)w.end] - sp.b_off[(size_t)w.begin]; },
                          [&](const WorkItem &w, int64_t from, int64_t to) { return WorkItem{bundle_at(w, from), bundle_at(w, to), 0, w.tile}; });
                 }
             }
@@ -722,13 +739,14 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
     // kernel is bound by the bytes it streams (K=32: 0.476 -> 0.411 ms); at 128 it is bound by
     // VALU issue and the 6 extra instructions per batch cost more than the bytes save.  perm
     // stays on the device for sddmm_plan_set_values only.
-    const bool compact = !gather && ks / 4 <= 16;
     // (the compact form needs a group's nonzeros at consecutive positions of S: not so in a remainder)
     if (compact && c.orig) return fail(SDDMM_ERR_ARG, "plan: compact tile stream over a remainder matrix");
     if (compact) {
         const int64_t ng = np / G;
-        std::vector<uint16_t> scol16((size_t)np + kStreamSlack, 0);
-        std::vector<int32_t> pbase((size_t)ng + kStreamSlack, 0);
+        big_vector<uint16_t> scol16((size_t)np + kStreamSlack);
+        big_vector<int32_t> pbase((size_t)ng + kStreamSlack);
+        std::fill(scol16.begin() + np, scol16.end(), (uint16_t)0);
+        std::fill(pbase.begin() + ng, pbase.end(), 0);
         const int32_t row_bytes = ks * 4;
         parallel_ranges(ng, 1 << 12, [&](int64_t gb, int64_t ge, int) {
             for (int64_t g = gb; g < ge; ++g) {
@@ -744,7 +762,7 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         if (int rc = c.up(&d_scol16, scol16)) return rc;
         if (int rc = c.up(&d_pbase, pbase)) return rc;
         L.ta.scol16 = d_scol16; L.ta.pbase = d_pbase;
-        std::vector<int32_t>().swap(scol);  // not used by the compact kernels
+        big_vector<int32_t>().swap(scol);  // not used by the compact kernels
     }
     if (shorts) {
         uint32_t *d_btype = nullptr;
@@ -891,13 +909,14 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         // (every workgroup's matrix-core waves take a share of their die's pairs: all workgroups must exist)
         if (L.grid != c.cus) return fail(SDDMM_ERR_ARG, "plan: matrix-core share on a launch of %d workgroups", L.grid);
     }
-    L.k_slice = ks;
-    if (gather) L.grid = (int32_t)std::max<int64_t>(1, (np + 2047) / 2048);
+    L.k_slice = std::min(ks, c.K);
+    // (gather form: 2048 positions per workgroup, fewer where that would leave less than four workgroups per compute unit)
+    if (gather) L.grid = (int32_t)std::max<int64_t>({1, (np + 2047) / 2048, std::min<int64_t>(4 * (int64_t)c.cus, (np + 255) / 256)});
     if (int rc = resolve_functions(L)) return rc;
     if (I) {
         I->tile_size_x = x; I->tile_size_y = grid2d ? (int32_t)std::min<int64_t>(block_rows_max, INT32_MAX) : panel_rows; I->n_col_tiles = n_tiles_all;
         I->n_row_panels = panel_local ? shares : n_panels; I->n_blocks = n_blocks; I->lanes_per_nnz = G; I->lds_bytes = L.lds;
-        I->grid = L.grid; I->block = L.block; I->k_slice = ks;
+        I->grid = L.grid; I->block = L.block; I->k_slice = L.k_slice;
     }
     c.P->info.padded_positions += np;
     L.positions = np; L.tile_g = G;
