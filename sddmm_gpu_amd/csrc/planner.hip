@@ -591,7 +591,8 @@ static Split estimate_split(const Ctx &c, const std::vector<int32_t> &rows, int 
     auto gather_us = [&](double nnz) { return 4.5 + 1e-6 * f * nnz * K * 4 / h_rate; };
     // (the tile kernel's time is underestimated where its items are uneven: 12 % more)
     const double t_tile = 1.12 * tile_us(lng.runs + shrt.runs, lng.pos + shrt.pos), t_gather = gather_us(lng.nnz + shrt.nnz);
-    const double t_both = lng.nnz > 0 && shrt.nnz > 0 ? 3.0 + 1.12 * tile_us(lng.runs, lng.pos) + gather_us(shrt.nnz) : 1e30;
+    // (an H too large for the caches is gathered slab by slab, which takes all rows)
+    const double t_both = lng.nnz > 0 && shrt.nnz > 0 && h_all <= 268.0e6 ? 3.0 + 1.12 * tile_us(lng.runs, lng.pos) + gather_us(shrt.nnz) : 1e30;
     if (t_both < t_tile && t_both < t_gather) return Split::by_length;
     return t_tile < t_gather ? Split::all_tiled : Split::all_gathered;
 }
@@ -779,7 +780,7 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         // a small problem is one launch: splitting it only adds launch latency
         if (!by_model && nl && nnz_part < (opt.split_min_nnz >= 0 ? opt.split_min_nnz : (int64_t)4 * 1000 * 1000)) join(rl, rs, nl, nsh);
         // a class too small to fill the machine joins the other
-        if (!by_model && !rl.empty() && !rs.empty() && nl * 50 < nnz_part) join(rs, rl, nsh, nl);
+        if (!rl.empty() && !rs.empty() && nl * 50 < nnz_part) join(rs, rl, nsh, nl);
         // (a handful of short rows -- the clipped rows at the corners of a band -- are not worth a launch
         // of their own: a single workgroup would walk them batch by batch at memory latency;
         // banded 2^20, K = 512: 711 nonzeros took 0.065 ms of a 4.14 ms step)
