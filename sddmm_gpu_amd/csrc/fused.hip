@@ -37,13 +37,15 @@ constexpr int kSmListRows = 1 << 30, kSmListHuge = 1 << 29, kSmListChunk = kSmLi
 constexpr int kSmOwnBatches = 32;                       // batches of 64 rows that a chunk's own wave takes at least
 constexpr int kSmByLane = 8, kSmBy8 = 96, kSmBy32 = 512, kSmByWave16 = 1024;  // row lengths up to which a lane / 8 lanes / 32 lanes / the wave with 16 entries per lane work on a row
 
-// log2 of the entries per chunk: 4096 on matrices with enough of them to give every wave of the machine a chunk
-// (4096 chunks), less below that, down to 64 -- a wave works through its chunk at memory latency, so few chunks leave
-// the machine idle: 18 thousand entries took 48 us as 5 chunks, 1.8 million 64 us as 447.
-__host__ __device__ inline int softmax_chunk_shift(int64_t nnz)
+// log2 of the entries per chunk, 6 to 12: as large as leaves 8192 chunks, but not below 16 average rows (n_rows = 0: without
+// that bound) while there are 1024 chunks.  A wave works through its chunk at memory latency, so few chunks leave the machine idle (18
+// thousand entries took 48 us as 5 chunks, 1.8 million 64 us as 447, 9 million of 34 a row 91 us as 2148 and 70 now);
+// chunks of a row or two make waves of too little work (5.2 million of 319 a row: 32 us in chunks of 4096, 35 of 1024,
+// 40 of 512).
+__host__ __device__ inline int softmax_chunk_shift(int64_t nnz, int64_t n_rows)
 {
     int shift = 12;
-    while (shift > 6 && (nnz >> shift) < 4096) --shift;
+    while (shift > 6 && ((nnz >> shift) < 1024 || ((nnz >> shift) < 8192 && (n_rows == 0 || n_rows << (shift - 1) >= 16 * nnz)))) --shift;
     return shift;
 }
 
@@ -74,7 +76,7 @@ void sddmm_row_softmax_rows_kernel(const int32_t *__restrict__ row_ptr, int64_t 
     __shared__ int row_of[256], begin_of[256], end_of[256];  // the row that holds a chunk's first entry, and its extent
     if (blockIdx.x == 0 && threadIdx.x < 2) g_softmax_list[threadIdx.x] = 0;  // (the second kernel counts in them)
     const int64_t nnz = row_ptr[n_rows];
-    const int shift = softmax_chunk_shift(nnz);
+    const int shift = softmax_chunk_shift(nnz, n_rows);
     const int64_t n_chunks = (nnz + ((int64_t)1 << shift) - 1) >> shift;
     for (int64_t base = (int64_t)blockIdx.x * 255; base < n_chunks; base += (int64_t)gridDim.x * 255) {
         const int64_t c = base + threadIdx.x, p0 = c << shift, p1 = p0 + ((int64_t)1 << shift);
@@ -267,7 +269,7 @@ __device__ __forceinline__ void softmax_short_rows(const int32_t *__restrict__ r
 {
     const int lane = threadIdx.x & 63;
     const int64_t nnz = row_ptr[n_rows];
-    const int shift = softmax_chunk_shift(nnz);
+    const int shift = softmax_chunk_shift(nnz, n_rows);
     const int64_t n_chunks = (nnz + ((int64_t)1 << shift) - 1) >> shift;
     const int64_t n_waves = n_groups * (kSmBlock / 64);
     const int64_t own = softmax_own_batches(n_rows, n_chunks);
@@ -380,7 +382,7 @@ __device__ __forceinline__ void softmax_long_rows(const int32_t *__restrict__ ro
     __shared__ int4 todo[3 * kSmBlock];  // first entry, end, record (-1: a whole row)
     __shared__ int n_todo;
     const int64_t nnz = row_ptr[n_rows];
-    const int shift = softmax_chunk_shift(nnz);
+    const int shift = softmax_chunk_shift(nnz, n_rows);
     const int64_t n_chunks = (nnz + ((int64_t)1 << shift) - 1) >> shift;
     const bool vec_in = (reinterpret_cast<uintptr_t>(x) & 15u) == 0, vec_out = (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
     const int64_t own = softmax_own_batches(n_rows, n_chunks);
@@ -542,7 +544,7 @@ void sddmm_row_softmax_merge_kernel(const int32_t *__restrict__ row_ptr, int64_t
     const int n_list = g_softmax_list[0], n_huge = g_softmax_list[1];
     if (n_list <= 0 && n_huge <= 0) return;
     const int64_t nnz = row_ptr[n_rows];
-    const int shift = softmax_chunk_shift(nnz);
+    const int shift = softmax_chunk_shift(nnz, n_rows);
     const int64_t n_chunks = (nnz + ((int64_t)1 << shift) - 1) >> shift;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t own = softmax_own_batches(n_rows, n_chunks), G = gridDim.x;
@@ -615,7 +617,7 @@ static int softmax_store(float2 **rec, int4 **rows, int32_t **list)
 
 int64_t row_softmax_workspace_bytes(int64_t nnz)
 {
-    const int shift = softmax_chunk_shift(nnz);
+    const int shift = softmax_chunk_shift(nnz, 0);
     const int64_t n_chunks = (nnz + ((int64_t)1 << shift) - 1) >> shift;
     return (((n_chunks * 36 + 8) + 255) / 256) * 256;  // two float2, one int4 and one list item per chunk, and the two lists' lengths
 }
@@ -627,7 +629,7 @@ int launch_row_softmax(int64_t n_rows, const int32_t *d_row_ptr, const float *d_
     int4 *rows = nullptr;
     int32_t *list = nullptr;
     if (d_ws) {  // [2 * n_chunks] records, then [n_chunks] chunk layouts, then the two lists: their lengths and [n_chunks] items
-        const int shift = softmax_chunk_shift(nnz);
+        const int shift = softmax_chunk_shift(nnz, n_rows);
     const int64_t n_chunks = (nnz + ((int64_t)1 << shift) - 1) >> shift;
         rec = static_cast<float2 *>(d_ws);
         rows = reinterpret_cast<int4 *>(rec + 2 * n_chunks);
