@@ -50,7 +50,7 @@ enum {
                                     column slabs when H is far larger than the caches) */
     SDDMM_KERNEL_LDS_TILE = 2,   /* column tiles of H staged in LDS, W row (re)loaded per row run */
     SDDMM_KERNEL_PANEL = 3,      /* row panels of W resident in VGPRs, column tiles of H swept through LDS */
-    SDDMM_KERNEL_HYBRID = 4,     /* what AUTO builds: (from K = 512 on, or when asked) the dense core as a DENSE_BLOCK
+    SDDMM_KERNEL_HYBRID = 4,     /* what AUTO builds: (from K = 384 on, or when asked) the dense core as a DENSE_BLOCK
                                     launch, the rest split by row length: rows with at least 2 nonzeros per column
                                     tile -> LDS_TILE (padded tile kernel), shorter rows -> ROW_GATHER; a class too
                                     small to pay for its launch joins the other.  Never a PANEL launch. */

@@ -2,20 +2,39 @@
 //
 // Where S has a dense core (heavy rows x popular columns of a power-law
 // matrix), the sampled products of a 128 x 128 block are cheaper as one dense
-// fp32 contraction on the matrix cores than as gathered dot products on the
+// contraction on the matrix cores than as gathered dot products on the
 // vector ALU: a block of 128 rows (any rows, given by a list) times 128 columns
-// (any columns, given by a list) is computed whole with v_mfma_f32_32x32x2_f32
-// (plain fp32 in, fp32 accumulate), left in LDS, and the block's nonzeros pick
-// their entries from there, scale them by S.val and store them at their own
-// positions of the output.  Structural zeros of the block are computed and
-// dropped; the planner only hands over blocks dense enough for that to pay.
+// (any columns, given by a list) is computed whole, left in LDS, and the block's
+// nonzeros pick their entries from there, scale them by S.val and store them at
+// their own positions of the output.  Structural zeros of the block are computed
+// and dropped; the planner only hands over blocks dense enough for that to pay.
+//
+// Arithmetic.  The fp32 matrix instruction runs at a sixteenth of the bf16 one, so
+// every operand is cut into three bf16 parts whose sum it is exactly (8 + 8 + 8
+// significant bits), and six of the nine products of parts are summed in fp32; the
+// three left out lie below 2^-24 of the product (each at most 2^-27, 2^-27 and 2^-36
+// of it).  Error against 64 bits over the blocks of a recommender matrix (relative,
+// 2-norm; fp32 instruction -> parts): K = 128 1.72e-7 -> 1.41e-7, K = 256 2.39e-7 ->
+// 2.00e-7, K = 512 3.32e-7 -> 2.80e-7, all-positive factors 2.83e-7 -> 2.16e-7, factors
+// spread over e^(+-9) 9.2e-8 -> 8.6e-8: fewer roundings of the running sum (6 per 16
+// elements, 8 before).  What parts cannot carry -- infinities, NaNs, sums beyond the
+// range, values with bits under bf16's smallest subnormal -- is found and those
+// results are computed once more in fp32 (redo_picks).
 //
 // One workgroup of 4 waves per block, each wave a 64 x 64 quarter (2 x 2 MFMA
 // tiles of 32 x 32, 64 accumulator registers).  K runs in chunks of 32: the
 // chunk's 128 x 32 slices of the W rows and of the H rows are gathered from
-// global memory into registers while the previous chunk is multiplied, then
-// written to LDS (double-buffered, rows padded to 144 bytes so that the
-// 16-byte operand reads of 16 lanes fall into 64 different banks).
+// global memory into registers while the previous chunk is multiplied, cut into
+// their parts between its last 24 matrix instructions (8 vector instructions after
+// each: 768 clocks of either) and written to LDS.  One buffer: two would leave
+// room for one workgroup per CU only, and the second workgroup is what works while
+// the first passes its barriers.  What bounds it is the matrix cores and LDS about
+// alike: 1536 clocks of matrix instructions per chunk and wave, 1150 of LDS reads and
+// writes per workgroup, two workgroups on a CU.  Recommender shape, 57.6 M
+// nonzeros in 5687 blocks, K = 512: 1.04 ms with the fp32 instruction, 0.82 with parts
+// cut after the products, 0.71 with the cutting among them and conflict-free writes
+// (6 x 95 GFLOP take 0.23 ms at the nominal bf16 rate; picking and storing 14 B per
+// nonzero about 0.2).
 #include <hip/hip_runtime.h>
 #include "kernels.hpp"
 
@@ -25,13 +44,39 @@ namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float vec4f __attribute__((ext_vector_type(4)));  // (a plain vector type: stays in registers)
+typedef float vec2f __attribute__((ext_vector_type(2)));
+typedef uint32_t vec4u __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int kT = kDenseTile;        // 128 rows and 128 columns per block
-constexpr int kKC = 32;               // K elements per chunk
-constexpr int kRowF = kKC + 4;        // floats per staged row (144 bytes)
-constexpr int kStageF = kT * kRowF;   // floats per staged operand slice
-constexpr int kCRowF = kT + 8;        // floats per row of the result block in LDS
-static_assert(4 * kStageF >= kT * kCRowF, "the result block reuses the staging buffers");
+constexpr int kT = kDenseTile;           // 128 rows and 128 columns per block
+constexpr int kKC = 32;                  // K elements per chunk
+constexpr int kPartB = kKC * 2;          // bytes of one part of a staged row
+constexpr int kRowB = 3 * kPartB + 16;   // bytes per staged row: 13 times 16, odd, so 16 rows spread over all banks
+constexpr int kStageB = kT * kRowB;      // bytes per staged operand
+constexpr int kCRowF = kT + 8;           // floats per row of the result block in LDS
+constexpr int kLdsB = 2 * kStageB > kT * kCRowF * 4 ? 2 * kStageB : kT * kCRowF * 4;
+
+// Eight floats as three bf16 parts each: part 0 is x rounded to 8 significant bits, part 1 what is
+// left rounded to 8, part 2 the rest, so x = p0 + p1 + p2 exactly.  `lost` collects the bits below
+// part 2, which are nonzero only where x is so small that they lie under bf16's smallest subnormal.
+// An infinity or a NaN leaves a NaN in part 1, a value that rounds beyond the range an infinity.
+__device__ __forceinline__ void split8(const vec4f lo4, const vec4f hi4, vec4u (&part)[3], uint32_t &lost)
+{
+    const float x[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        vec2f v = {x[2 * e], x[2 * e + 1]};
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            if (p == 2) lost |= __float_as_uint(v.x) | __float_as_uint(v.y);
+            const uint32_t b = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+            part[p][e] = b;
+            v.x -= __uint_as_float(b << 16);
+            v.y -= __uint_as_float(b & 0xffff0000u);
+        }
+    }
+}
 
 // Workgroup barrier that orders LDS traffic only.  __syncthreads() also waits for every global
 // load and store in flight (its workgroup-scope fence), which would drain the requests this kernel
@@ -45,7 +90,8 @@ __device__ __forceinline__ void lds_barrier()
 __global__ __launch_bounds__(256, 2)
 void sddmm_dense_kernel(const DenseArgs a)
 {
-    __shared__ __attribute__((aligned(16))) float lds[4 * kStageF];  // A0 B0 A1 B1 | result block
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kLdsB];  // A B | result block
+    __shared__ uint32_t inexact;  // nonzero: some operand of the block has bits below its three parts
     const int t = threadIdx.x;
     const int lane = t & 63, wave = t >> 6;
     const int wr = wave >> 1, wc = wave & 1;  // this wave's 64 x 64 quarter
@@ -54,8 +100,10 @@ void sddmm_dense_kernel(const DenseArgs a)
     const int n_chunks = a.K / kKC;
     const vec4f *__restrict__ W4 = reinterpret_cast<const vec4f *>(a.W);
     const vec4f *__restrict__ H4 = reinterpret_cast<const vec4f *>(a.H);
-    // staging: thread t carries float4 q of rows r0, r0 + 32, r0 + 64, r0 + 96 of both operands
-    const int q = t & 7, r0 = t >> 3;
+    // staging: thread t carries float4 q and q + 4 of rows r0 and r0 + 64 of both operands.  They go
+    // side by side into LDS; the order of the K elements is the same for both operands, so it does not matter.
+    //  16 neighbouring lanes write four rows that lie 4 apart: 64 different banks.
+    const int q = t & 3, r0 = 16 * wave + 4 * ((t >> 2) & 3) + ((t >> 4) & 3);
 
     // Workgroup b works on slots b, b + grid, ...; its filled slots come first.
     int slot = blockIdx.x;
@@ -63,28 +111,39 @@ void sddmm_dense_kernel(const DenseArgs a)
     int2 range = a.slot_range[slot];
     if (range.y <= range.x) return;
 
-    // float4 index of this thread's piece of each of its rows of W and H at chunk 0
-    auto load_ids = [&](int s, uint32_t (&wofs)[4], uint32_t (&hofs)[4]) {
+    // float4 index of this thread's first piece of each of its rows of W and H at chunk 0
+    auto load_ids = [&](int s, uint32_t (&wofs)[2], uint32_t (&hofs)[2]) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            wofs[i] = (uint32_t)a.slot_rows[s * kT + r0 + 32 * i] * K4 + (uint32_t)q;
-            hofs[i] = (uint32_t)a.slot_cols[s * kT + r0 + 32 * i] * K4 + (uint32_t)q;
+        for (int i = 0; i < 2; ++i) {
+            wofs[i] = (uint32_t)a.slot_rows[s * kT + r0 + 64 * i] * K4 + (uint32_t)q;
+            hofs[i] = (uint32_t)a.slot_cols[s * kT + r0 + 64 * i] * K4 + (uint32_t)q;
         }
     };
     vec4f ga[4], gb[4];
-    auto fetch = [&](const uint32_t (&wofs)[4], const uint32_t (&hofs)[4]) {
+    auto fetch = [&](const uint32_t (&wofs)[2], const uint32_t (&hofs)[2]) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ga[i] = W4[wofs[i]];
+        for (int i = 0; i < 4; ++i) ga[i] = W4[wofs[i >> 1] + 4 * (i & 1)];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) gb[i] = H4[hofs[i]];
+        for (int i = 0; i < 4; ++i) gb[i] = H4[hofs[i >> 1] + 4 * (i & 1)];
     };
-    auto stage = [&](int buf) {
-        float *A = lds + buf * 2 * kStageF, *B = A + kStageF;
+    uint32_t lost = 0;  // of the operands staged by this thread for the block in hand
+    vec4u pa[2][3], pb[2][3];
+    auto split = [&]() {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            *reinterpret_cast<vec4f *>(A + (r0 + 32 * i) * kRowF + 4 * q) = ga[i];
-            *reinterpret_cast<vec4f *>(B + (r0 + 32 * i) * kRowF + 4 * q) = gb[i];
+        for (int i = 0; i < 2; ++i) {
+            split8(ga[2 * i], ga[2 * i + 1], pa[i], lost);
+            split8(gb[2 * i], gb[2 * i + 1], pb[i], lost);
         }
+    };
+    auto stage = [&]() {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                unsigned char *at = lds + (r0 + 64 * i) * kRowB + p * kPartB + 16 * q;
+                *reinterpret_cast<vec4u *>(at) = pa[i][p];
+                *reinterpret_cast<vec4u *>(at + kStageB) = pb[i][p];
+            }
     };
     // One round of the block's nonzero list: 8 entries per thread, strided by the workgroup.
     constexpr int U = 8;
@@ -98,7 +157,28 @@ void sddmm_dense_kernel(const DenseArgs a)
             r.v[u] = a.nz_val ? a.nz_val[idx] : 1.0f;
         }
     };
-    const float *Cb = lds;
+    const float *Cb = reinterpret_cast<const float *>(lds);
+    // Picks that are not stored from the result block but once more computed in fp32: all of a block
+    // whose operands three parts do not hold, and any that come out as an infinity or a NaN (there is
+    // one among the operands, or a sum left the range).
+    bool redo = false, left = false;
+    auto redo_picks = [&](int first, int n1) {
+        for (int idx = first; idx < n1; idx += 256) {
+            const uint32_t rc = a.nz_rc[idx];
+            if (!redo && fabsf(Cb[(rc >> 8) * kCRowF + (rc & 255u)]) < INFINITY) continue;
+            const vec4f *w = W4 + (uint32_t)a.slot_rows[slot * kT + (int)(rc >> 8)] * K4;
+            const vec4f *h = H4 + (uint32_t)a.slot_cols[slot * kT + (int)(rc & 255u)] * K4;
+            float d = 0.f;
+#pragma unroll 1
+            for (uint32_t k = 0; k < K4; ++k) {
+                const vec4f x = w[k], y = h[k];
+                d = fmaf(x.x, y.x, d); d = fmaf(x.y, y.y, d); d = fmaf(x.z, y.z, d); d = fmaf(x.w, y.w, d);
+            }
+            const int p = a.nz_p[idx];
+            const float v = a.nz_val ? a.nz_val[idx] : a.val ? a.val[p] : 1.0f;
+            a.out[p] = a.residual ? v - d : v * d;
+        }
+    };
     auto store_round = [&](Round &r, int first, int n1) {
         if (!a.nz_val && a.val) {
 #pragma unroll
@@ -107,14 +187,18 @@ void sddmm_dense_kernel(const DenseArgs a)
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const float dot = Cb[(r.rc[u] >> 8) * kCRowF + (r.rc[u] & 255u)];
-            if (first + 256 * u < n1) a.out[r.p[u]] = a.residual ? r.v[u] - dot : r.v[u] * dot;
+            const bool keep = !redo && fabsf(dot) < INFINITY;
+            left |= !keep;
+            if (keep && first + 256 * u < n1) a.out[r.p[u]] = a.residual ? r.v[u] - dot : r.v[u] * dot;
         }
     };
 
-    uint32_t wofs[4], hofs[4];
+    uint32_t wofs[2], hofs[2];
     load_ids(slot, wofs, hofs);
     fetch(wofs, hofs);
-    stage(0);
+    if (t == 0) inexact = 0;
+    split();
+    stage();
     lds_barrier();
     for (;;) {
         // what the next block needs is requested while this one is computed: its row and column
@@ -123,7 +207,7 @@ void sddmm_dense_kernel(const DenseArgs a)
         int2 nrange = make_int2(0, 0);
         if (nslot < a.n_slots) nrange = a.slot_range[nslot];
         const bool has_next = nrange.y > nrange.x;
-        uint32_t nw[4], nh[4];
+        uint32_t nw[2], nh[2];
         load_ids(has_next ? nslot : slot, nw, nh);
         // the first round of this block's nonzero list is requested before the arithmetic starts
         Round r0d;
@@ -136,50 +220,61 @@ void sddmm_dense_kernel(const DenseArgs a)
             for (int j = 0; j < 2; ++j)
 #pragma unroll
                 for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-        int par = 0;
-        for (int c = 0; c < n_chunks; ++c) {
-            const bool last = c + 1 == n_chunks;
-            // the next chunk's loads (the last chunk: the next block's first) are issued before this
-            // chunk's arithmetic and waited for after it
-            uint32_t sw[4], sh[4];
+        const unsigned char *ap = lds + (wr * 64 + m) * kRowB + kh * 16;
+        const unsigned char *bp = lds + kStageB + (wc * 64 + m) * kRowB + kh * 16;
+        auto products = [&](int s) {  // 16 elements of K
+            bf16x8 av[2][3], bv[2][3];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                sw[i] = last ? nw[i] : wofs[i] + (uint32_t)((c + 1) * (kKC / 4));
-                sh[i] = last ? nh[i] : hofs[i] + (uint32_t)((c + 1) * (kKC / 4));
+            for (int p = 2; p >= 0; --p)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    av[i][2 - p] = *reinterpret_cast<const bf16x8 *>(ap + 32 * i * kRowB + (2 - p) * kPartB + 32 * s);
+                    bv[i][p] = *reinterpret_cast<const bf16x8 *>(bp + 32 * i * kRowB + p * kPartB + 32 * s);
+                }
+            // the products of parts that reach into the upper 24 bits, small ones first
+#pragma unroll
+            for (int pq = 0; pq < 6; ++pq) {
+                constexpr int pp[6] = {0, 1, 2, 0, 1, 0}, qq[6] = {2, 1, 0, 1, 0, 0};
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[i][pp[pq]], bv[j][qq[pq]], acc[i][j], 0, 0, 0);
             }
-            fetch(sw, sh);
+        };
+        for (int c = 0; c + 1 < n_chunks; ++c) {
+            // the next chunk's loads are issued before this chunk's arithmetic, and what they bring is
+            // cut into its parts between the chunk's later products
+#pragma unroll
+            for (int i = 0; i < 2; ++i) { wofs[i] += kKC / 4; hofs[i] += kKC / 4; }
+            fetch(wofs, hofs);
             __builtin_amdgcn_sched_barrier(0);
-            const float *A = lds + par * 2 * kStageF, *B = A + kStageF;
-            const float *ap = A + (wr * 64 + m) * kRowF + kh * 4;
-            const float *bp = B + (wc * 64 + m) * kRowF + kh * 4;
+            products(0);
+            __builtin_amdgcn_sched_barrier(0);  // (one step's operands in registers at a time)
+            products(1);
+            split();
 #pragma unroll
-            for (int s = 0; s < kKC / 8; ++s) {
-                // lanes 0-31 hold elements 8s .. 8s+3 of their row, lanes 32-63 elements 8s+4 .. 8s+7:
-                // instruction e of this step multiplies elements 8s+e and 8s+4+e of both operands
-                const vec4f a0 = *reinterpret_cast<const vec4f *>(ap + 8 * s);
-                const vec4f a1 = *reinterpret_cast<const vec4f *>(ap + 32 * kRowF + 8 * s);
-                const vec4f b0 = *reinterpret_cast<const vec4f *>(bp + 8 * s);
-                const vec4f b1 = *reinterpret_cast<const vec4f *>(bp + 32 * kRowF + 8 * s);
-                const float av[2][4] = {{a0.x, a0.y, a0.z, a0.w}, {a1.x, a1.y, a1.z, a1.w}};
-                const float bv[2][4] = {{b0.x, b0.y, b0.z, b0.w}, {b1.x, b1.y, b1.z, b1.w}};
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-#pragma unroll
-                    for (int i = 0; i < 2; ++i)
-#pragma unroll
-                        for (int j = 0; j < 2; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][e], bv[j][e], acc[i][j], 0, 0, 0);
+            for (int i = 0; i < 24; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a matrix instruction
+                __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);  // vector instructions
             }
             __builtin_amdgcn_sched_barrier(0);
-            if (!last) {
-                stage(par ^ 1);
-                par ^= 1;
-            }
+            lds_barrier();  // everyone has read this chunk
+            stage();
             lds_barrier();
         }
+        fetch(nw, nh);  // the last chunk: the next block's first
+        __builtin_amdgcn_sched_barrier(0);
+        products(0);
+        __builtin_amdgcn_sched_barrier(0);
+        products(1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (lost & 0xffffu) inexact = 1;  // (read after the next barriers; any writer writes the same)
+        lost = 0;
+        lds_barrier();  // everyone has read the last chunk
         // the 128 x 128 block of dot products into LDS (over the staging buffers, which everyone has
         // left): register v of lane (m, kh) of tile (i, j) holds row 8*(v/4) + 4*kh + v%4, column m
-        float *Cw = lds;
+        float *Cw = reinterpret_cast<float *>(lds);
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -201,6 +296,8 @@ void sddmm_dense_kernel(const DenseArgs a)
             load_round(r2d, first + 2 * R, n1);
             load_round(r3d, first + 3 * R, n1);
             lds_barrier();
+            redo = inexact != 0;
+            left = false;
             store_round(r0d, first, n1);
             store_round(r1d, first + R, n1);
             store_round(r2d, first + 2 * R, n1);
@@ -215,15 +312,18 @@ void sddmm_dense_kernel(const DenseArgs a)
                 store_round(r2d, f + 2 * R, n1);
                 store_round(r3d, f + 3 * R, n1);
             }
+            if (left) redo_picks(first, n1);
         }
         lds_barrier();  // the next block's staging overwrites the result block
         if (!has_next) break;
-        stage(0);  // the next block's first chunk has been in registers since this block's last chunk
+        split();  // the next block's first chunk has been in registers since this block's last chunk
+        stage();
+        if (t == 0) inexact = 0;
         lds_barrier();
         slot = nslot;
         range = nrange;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { wofs[i] = nw[i]; hofs[i] = nh[i]; }
+        for (int i = 0; i < 2; ++i) { wofs[i] = nw[i]; hofs[i] = nh[i]; }
     }
 }
 
