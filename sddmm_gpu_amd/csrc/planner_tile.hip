@@ -232,12 +232,13 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
             return rc;
         n_tiles_all = T.n_tiles;
         const int64_t n_seg = (int64_t)T.active_end.size();
-        // Runs of less than 12 nonzeros: a partial row of Y per run is written and read for little work, and the product
+        // Runs of less than 15 nonzeros: a partial row of Y per run is written and read for little work, and the product
         // goes over the CSR pattern instead (attention window, 16,384 tokens, K = 64, runs of 10: 131 -> 65 us; K = 32, runs
-        // of 8: 146 -> 46 us; ratings, K = 128, runs of 16: 98 against 124 us at 4.9 M nonzeros, 435 against 388 at 19 M).
+        // of 8: 146 -> 46 us; ratings, K = 128, runs of 12.8: 255 -> 209 us, K = 64, runs of 13.7: 242 -> 153, runs of 19: 111
+        // against 110; K = 128, runs of 16: 98 against 124 us at 4.9 M nonzeros, 435 against 388 at 19 M).
         // Below 4 million nonzeros the two are level at best (0.5 M, K = 128: 27 us) or the walk is far ahead (window
         // of 101, 8,898 tokens, K = 32, runs of 14: 110 against 25 us).
-        if (want_spmm && rb == 0 && c.nnz == c.P->info.nnz && (ragged || L.nnz < 12 * n_seg || L.nnz < 4000000)) { want_spmm = false; sp_csr = true; }
+        if (want_spmm && rb == 0 && c.nnz == c.P->info.nnz && (ragged || L.nnz < 15 * n_seg || L.nnz < 4000000)) { want_spmm = false; sp_csr = true; }
         // row-block boundaries of the 2-D assignment: equal shares of the rows' nonzeros
         std::vector<int32_t> cut;
         auto make_cuts = [&](int n_shares) {
@@ -654,10 +655,8 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
                 for (int sh = 0; sh < shares; ++sh)
                     for (int32_t j : tiles_ne) { items.push_back(item_of(sh, j)); item_keys.push_back({sh, j}); }
             }
-            // the product walks the same (row block, tile) items on the same workgroups
-            if (want_spmm && !panel_local && item_keys.size() == items.size()) build_spmm(item_keys);
             // uneven items (see deal_evenly): inside a die where the row blocks belong to dies, over all workgroups
-            // otherwise; in units of stream positions for the SDDMM and of rounds for the product
+            // otherwise, in units of stream positions.  True: dealt out anew.
             auto even = [&](std::vector<WorkItem> &list, int64_t stage, int64_t quantum, const std::function<int64_t(const WorkItem &)> &load,
                             const std::function<WorkItem(const WorkItem &, int64_t, int64_t)> &cut_item) {
                 const int groups = xcd_local ? 8 : 1;
@@ -675,7 +674,7 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
                     most_now = std::max(most_now, sum);
                 }
                 // (what is nearly even keeps its whole tiles: here when no dealing can gain enough, below when this one does not)
-                if ((total / c.cus + stage) * 10 > most_now * 7) return;
+                if ((total / c.cus + stage) * 10 > most_now * 7) return false;
                 for (int gr = 0; gr < groups; ++gr) {
                     std::vector<WorkItem> mine;
                     std::vector<int> wgs;
@@ -693,27 +692,29 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
                     for (size_t w = 0; w < wgs.size(); ++w)
                         for (const Piece &pc : got[w]) seq[(size_t)wgs[w]].push_back(cut_item(mine[(size_t)pc.item], pc.from, pc.to));
                 }
-                if (most_new * 10 > most_now * 7) return;
+                if (most_new * 10 > most_now * 7) return false;
                 size_t turns = 0;
                 for (auto &q : seq) turns = std::max(turns, q.size());
                 list.assign(turns * (size_t)c.cus, WorkItem{0, 0, 0, 0});
                 for (int b = 0; b < c.cus; ++b)
                     for (size_t k = 0; k < seq[(size_t)b].size(); ++k) list[k * (size_t)c.cus + (size_t)b] = seq[(size_t)b][k];
+                return true;
             };
+            bool uneven = false;
+            const size_t items_whole = items.size();
             // (staging a tile of x rows takes about as long as 4 x positions of one workgroup, at every rank)
-            if (!panel_local && mf_nwm == 0 && c.opt.tile_assign < 0) {
-                even(items, 4 * (int64_t)x, 64, [](const WorkItem &w) { return (int64_t)w.end - w.begin; },
-                     [&](const WorkItem &w, int64_t from, int64_t to) {
-                         return WorkItem{(int32_t)(w.begin + from), (int32_t)(w.begin + to), (int32_t)(w.batch_base + (shorts ? from / 64 : 0)), w.tile};
-                     });
-                if (sp.built) {
-                    auto bundle_at = [&](const WorkItem &w, int64_t round) {  // the first bundle that begins at or after a round of the item
-                        return (int32_t)(std::lower_bound(sp.b_off.begin() + w.begin, sp.b_off.begin() + w.end, sp.b_off[(size_t)w.begin] + (int32_t)round) - sp.b_off.begin());
-                    };
-                    even(sp.items, std::max<int64_t>(1, x / 16), 1, [&](const WorkItem &w) { return (int64_t)sp.b_off[(size_t)w.end] - sp.b_off[(size_t)w.begin]; },
-                         [&](const WorkItem &w, int64_t from, int64_t to) { return WorkItem{bundle_at(w, from), bundle_at(w, to), 0, w.tile}; });
-                }
-            }
+            if (!panel_local && mf_nwm == 0 && c.opt.tile_assign < 0)
+                uneven = even(items, 4 * (int64_t)x, 64, [](const WorkItem &w) { return (int64_t)w.end - w.begin; },
+                              [&](const WorkItem &w, int64_t from, int64_t to) {
+                                  return WorkItem{(int32_t)(w.begin + from), (int32_t)(w.begin + to), (int32_t)(w.batch_base + (shorts ? from / 64 : 0)), w.tile};
+                              });
+            // The product walks the same (row block, tile) items on the same workgroups.  Where they are uneven -- rows that
+            // lie together use columns that lie together -- the walk over the CSR pattern finds its H rows in the caches
+            // and is the faster one at any run length (windows of 400 to 600, 5 to 14 million nonzeros, items cut and
+            // dealt out anew against the walk: K = 128 451 / 279, 283 / 236 and 423 / 287 us, K = 64 283 / 150, 175 / 126
+            // and 155 / 68, K = 32 with runs of 41 220 / 84).
+            if (want_spmm && uneven && c.nnz == c.P->info.nnz) { want_spmm = false; sp_csr = true; }
+            if (want_spmm && !panel_local && item_keys.size() == items_whole) build_spmm(item_keys);
         } else if (want_spmm && rb == 0 && rows.size() <= (size_t)panel_rows) {
             // (equal position ranges for the SDDMM: the product takes one item per column tile)
             std::vector<std::pair<int, int32_t>> keys;
