@@ -3,6 +3,7 @@
 // their environment layer, kernel lookup, pattern hashes, workspace layout.
 #include <hip/hip_runtime.h>
 #include <chrono>
+#include <cmath>
 #include <cstring>
 #include <new>
 #include <unistd.h>
@@ -551,8 +552,71 @@ void assign_workspace(sddmm_plan *P)
 // TB/s (14 for rows of less than 256 bytes) while H fits one die's L2, 11.5 up to 64 MB, 8 beyond.  A second launch: 3.
 // Measured over 60 matrices of 0.1 to 28 M nonzeros (power-law, word counts, R-MAT, uniform, banded; K from 11 to 512)
 // the fixed rules this replaces were more than 10 % from the best of the three on 21 of them, up to 1.7 times.
-enum class Split { all_tiled, by_length, all_gathered };
-static Split estimate_split(const Ctx &c, const std::vector<int32_t> &rows, int w, int32_t x, int g, int64_t short_max)
+enum class Split { all_tiled, by_length, all_gathered, slabs };
+
+// The gather over column slabs (add_tile's gather form, groups of 4 lanes), for an H of which one K slice of w
+// elements does not stay in a die's 4 MB of L2: which slab width is cheapest, from the sampled rows.  Narrow slabs
+// have short runs (more padding, the W row once per run), wide ones miss the L2.  Picoseconds per padded position and
+// slice, measured with 2 / 4 / 8 / 16 / 32 MB of H slice per slab: uniform columns, w = 128: 28 / 30 / 43 / 55 / 62, w = 64:
+// 18 / 20 / 23 / 27 / 31; R-MAT, w = 128: 30 / 31 / 32 / 33 / 35 and 42 / 53 with 64 / 128 MB, w = 64: 16 to 20 up to 32 MB -- as if
+// its slabs were a twelfth as large, since few columns get most of the accesses.  So the size E counts by a power of the
+// share of the columns (in 1024 stretches) that gets 60 % of the nonzeros, and a position costs 26 + 40 E^2 / (E^2 + 70) at
+// w = 128, 17.5 + 16 E^2 / (E^2 + 110) at w = 64.  us against the best of the other three: uniform 95 M of 220,000 columns,
+// K = 128 6494 -> 3142; 20 M of 100,000, K = 64 563 -> 392, K = 256 2664 -> 1424; R-MAT 2^20, 78 M, K = 128 4094 -> 2990, 36 M, K = 512
+// 12960 -> 7154; 2^18, 13 M, K = 128 678 -> 467.  Slices of 32 gain nothing (2^20: 620 against 685), nor does a band whose
+// neighbouring rows use neighbouring columns anyway (200,000 rows, 20 of +-20,000 each: 300 against 342).
+struct SlabChoice { int64_t cols = 0; double us = 1e30; };
+static SlabChoice estimate_slabs(const Ctx &c, const std::vector<int32_t> &rows, int w)
+{
+    SlabChoice best;
+    const double slice_bytes = 4.0 * w;
+    if (w < 64 || (double)c.n_cols * slice_bytes < 8.0e6) return best;
+    const size_t n = rows.size();
+    const size_t stride = std::max<size_t>({1, n / 4096, (size_t)((double)c.nnz / 2.5e5)});
+    std::vector<int64_t> hits(1024, 0);
+    const int64_t stretch = ((int64_t)c.n_cols + 1023) / 1024;
+    constexpr int kSizes = 6;  // 2 to 64 MB
+    int first_shift = 0;
+    while (((int64_t)1 << (first_shift + 1)) * slice_bytes <= 2.1e6) ++first_shift;
+    double pos[kSizes] = {}, width = 0, shift = 0;  // columns between a row's 10th and 90th percentile; its middle from the next row's
+    int64_t sampled = 0, wide_rows = 0;
+    for (size_t i = stride / 2; i < n; i += stride) {
+        const int32_t b = c.row_ptr[rows[i]], e = c.row_ptr[rows[i] + 1];
+        sampled += e - b;
+        for (int32_t p = b; p < e; ++p) ++hits[(size_t)(c.col_ind[p] / stretch)];
+        if (e - b >= 10 && i + 1 < n) {
+            const int32_t b1 = c.row_ptr[rows[i + 1]], e1 = c.row_ptr[rows[i + 1] + 1];
+            width += c.col_ind[e - 1 - (e - b) / 10] - c.col_ind[b + (e - b) / 10];
+            shift += std::abs((double)c.col_ind[b + (e - b) / 2] - c.col_ind[b1 + (e1 - b1) / 2]);
+            ++wide_rows;
+        }
+        for (int k = 0; k < kSizes; ++k)
+            for (int32_t p = b; p < e;) {
+                const int32_t slab = c.col_ind[p] >> (first_shift + k);
+                int32_t q = p + 1;
+                while (q < e && (c.col_ind[q] >> (first_shift + k)) == slab) ++q;
+                pos[k] += (q - p + 3) & ~3;
+                p = q;
+            }
+    }
+    if (sampled <= 0 || (wide_rows > 0 && std::max(width, shift) < 0.25 * c.n_cols * wide_rows)) return best;
+    std::sort(hits.begin(), hits.end(), std::greater<int64_t>());
+    int64_t seen = 0;
+    size_t top = 0;
+    while (top < hits.size() && seen * 10 < sampled * 6) seen += hits[top++];
+    const double used = std::min(1024.0, (double)c.n_cols / stretch);  // stretches there are
+    const double spread = std::pow(std::min(1.0, (double)top / (0.6 * used)), 1.3);
+    const double slices = (c.K + w - 1) / w, f = (double)c.nnz / sampled;
+    for (int k = kSizes - 1; k >= 0; --k) {  // (about level: the wider one, which has the shorter stream)
+        const int64_t cols = (int64_t)1 << (first_shift + k);
+        const double mb = spread * std::min<double>((double)cols, c.n_cols) * slice_bytes / 1048576.0;
+        const double e2 = mb * mb, ps = w == 64 ? 17.5 + 16.0 * e2 / (e2 + 110.0) : (26.0 + 40.0 * e2 / (e2 + 70.0)) * w / 128;
+        const double us = slices * (4.5 + 1e-6 * f * pos[k] * ps);
+        if (us < 0.97 * best.us) best = {cols, us};
+    }
+    return best;
+}
+static Split estimate_split(const Ctx &c, const std::vector<int32_t> &rows, int w, int32_t x, int g, int64_t short_max, double slab_us)
 {
     const size_t n = rows.size();
     if (n == 0) return Split::all_gathered;
@@ -593,6 +657,7 @@ static Split estimate_split(const Ctx &c, const std::vector<int32_t> &rows, int 
     const double t_tile = 1.12 * tile_us(lng.runs + shrt.runs, lng.pos + shrt.pos), t_gather = gather_us(lng.nnz + shrt.nnz);
     // (an H too large for the caches is gathered slab by slab, which takes all rows)
     const double t_both = lng.nnz > 0 && shrt.nnz > 0 && h_all <= 268.0e6 ? 3.0 + 1.12 * tile_us(lng.runs, lng.pos) + gather_us(shrt.nnz) : 1e30;
+    if (slab_us < std::min({t_both, t_tile, t_gather})) return Split::slabs;
     if (t_both < t_tile && t_both < t_gather) return Split::by_length;
     return t_tile < t_gather ? Split::all_tiled : Split::all_gathered;
 }
@@ -709,6 +774,9 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         } catch (const std::bad_alloc &) {
             D = DenseBlocks{};
         }
+        // (what is left of a small core is most of S, and better off as a whole under the model below: R-MAT 2^20, K = 384,
+        // 6 % dense: 4697 us with the core, 3600 without; the ratings and word-count shapes have 50 to 60 %)
+        if (opt.dense_blocks < 0 && opt.dense_min_nnz < 0 && D.n_dense * 4 < nnz) D = DenseBlocks{};
         if (D.n_dense > 0) {
             if (int rc = add_dense(c, D, vals)) return rc;
             row_ptr = D.rem_row_ptr.data(); col_ind = D.rem_col.data(); nnz_part = nnz - D.n_dense;
@@ -771,8 +839,14 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         // the long ones tiled and the short ones gathered, or all gathered.  A caller who sets one of the thresholds,
         // and the remainder of a dense core, get the fixed rules.
         const bool by_model = D.n_dense == 0 && opt.short_row_max < 0 && opt.stage_factor < 0 && opt.split_min_nnz < 0;
+        int64_t slab_cols = 0;  // chosen by the model
         if (by_model) {
-            switch (estimate_split(c, ne, kt, x, g_long, short_max)) {
+            SlabChoice slab;
+            if (!ragged && opt.gather_lanes <= 0 && opt.gather_slab_cols < 0 && opt.gather_padded != 0 && opt.spmm_stream <= 0 &&
+                pick_tile_variant(kt, 4).G)
+                slab = estimate_slabs(c, ne, kt);
+            switch (estimate_split(c, ne, kt, x, g_long, short_max, slab.us)) {
+            case Split::slabs: join(rs, rl, nsh, nl); slab_cols = slab.cols; break;
             case Split::all_tiled: join(rl, rs, nl, nsh); break;
             case Split::all_gathered: join(rs, rl, nsh, nl); break;
             case Split::by_length: break;
@@ -800,14 +874,16 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
             // algorithmic bytes, 8.27 ms).  The padded gather then walks S in column slabs whose H rows
             // come to 32 MB, with groups of 4 lanes (runs inside a slab are short): 26.3 GB, 4.96 ms.
             // Narrower slabs lose to the W rows re-read per (row, slab) run, wider ones to H misses.
-            const bool huge_h = rl.empty() && D.n_dense == 0 && (int64_t)n_cols * K * 4 > ((int64_t)256 << 20);
+            // (where the model above has its say it chooses the slabs; this is for plans whose caller set a threshold,
+            // and for slices of less than 64 elements)
+            const bool huge_h = slab_cols > 0 || (rl.empty() && D.n_dense == 0 && (int64_t)n_cols * K * 4 > ((int64_t)256 << 20));
             int gg = opt.gather_lanes > 0 ? opt.gather_lanes : 8;
             if (huge_h && opt.gather_lanes <= 0 && opt.gather_slab_cols != 0 && pick_tile_variant(kt, 4).G) gg = 4;
             const bool slabs = !ragged && huge_h && opt.gather_slab_cols != 0 && opt.gather_padded != 0 && pick_tile_variant(kt, gg).G != 0;
             const bool padded = !ragged && opt.gather_padded != 0 && pick_tile_variant(kt, gg).G != 0 && (!rl.empty() || D.n_dense > 0 || slabs);
             if (padded) {
                 const int64_t keep = c.opt.gather_slab_cols;
-                if (slabs && keep < 0) c.opt.gather_slab_cols = std::max<int64_t>(1024, ((int64_t)32 << 20) / ((int64_t)K * 4));
+                if (slabs && keep < 0) c.opt.gather_slab_cols = slab_cols > 0 ? slab_cols : std::max<int64_t>(1024, ((int64_t)32 << 20) / ((int64_t)kt * 4));
                 const int rc = add_tile(c, rs, 0, 0, gg, kt, nullptr, true);
                 c.opt.gather_slab_cols = keep;
                 if (rc) return rc;
