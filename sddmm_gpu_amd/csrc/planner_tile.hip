@@ -232,13 +232,16 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
             return rc;
         n_tiles_all = T.n_tiles;
         const int64_t n_seg = (int64_t)T.active_end.size();
-        // Runs of less than 15 nonzeros: a partial row of Y per run is written and read for little work, and the product
+        // Runs of less than 12 nonzeros: a partial row of Y per run is written and read for little work, and the product
         // goes over the CSR pattern instead (attention window, 16,384 tokens, K = 64, runs of 10: 131 -> 65 us; K = 32, runs
-        // of 8: 146 -> 46 us; ratings, K = 128, runs of 12.8: 255 -> 209 us, K = 64, runs of 13.7: 242 -> 153, runs of 19: 111
-        // against 110; K = 128, runs of 16: 98 against 124 us at 4.9 M nonzeros, 435 against 388 at 19 M).
+        // of 8: 146 -> 46 us; ratings, K = 128, runs of 17: 81 against 110 us at 4.1 M nonzeros, 342 against 445 at 19.6 M).
         // Below 4 million nonzeros the two are level at best (0.5 M, K = 128: 27 us) or the walk is far ahead (window
-        // of 101, 8,898 tokens, K = 32, runs of 14: 110 against 25 us).
-        if (want_spmm && rb == 0 && c.nnz == c.P->info.nnz && (ragged || L.nnz < 15 * n_seg || L.nnz < 4000000)) { want_spmm = false; sp_csr = true; }
+        // of 101, 8,898 tokens, K = 32, runs of 14: 110 against 25 us).  Both hold while H is about as large as a die's L2,
+        // from where the walk then gathers; beyond, only really short runs (ratings, K = 384, 2 to 3.5 M nonzeros, H of 7 and
+        // 8 MB, runs of 10: 180 against 211 and 338 against 387 us).
+        const bool h_near = (int64_t)c.n_cols * c.K * 4 <= 6000000;
+        if (want_spmm && rb == 0 && c.nnz == c.P->info.nnz &&
+            (ragged || (h_near && (L.nnz < 12 * n_seg || c.nnz < 4000000)) || L.nnz < 8 * n_seg)) { want_spmm = false; sp_csr = true; }
         // row-block boundaries of the 2-D assignment: equal shares of the rows' nonzeros
         std::vector<int32_t> cut;
         auto make_cuts = [&](int n_shares) {
