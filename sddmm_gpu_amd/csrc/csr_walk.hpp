@@ -11,11 +11,10 @@ namespace sddmm {
 // so rows of any length take the same instructions as aligned ones (a piece may touch one cache line more).
 typedef float vec4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// The row that holds nonzero p (0 <= p < row_ptr[n_rows], uniform), by the whole wave: 64 probes a round, so three
-// rounds of one load each for a quarter of a million rows where a binary search is a chain of eighteen.
-__device__ __forceinline__ int wave_find_row(const int32_t *__restrict__ row_ptr, int n_rows, int p, int lane)
+// The row in [lo, hi) that holds nonzero p (row_ptr[lo] <= p < row_ptr[hi], all uniform), by the whole wave: 64 probes a
+// round, so three rounds of one load each for a quarter of a million rows where a binary search is a chain of eighteen.
+__device__ __forceinline__ int wave_find_row(const int32_t *__restrict__ row_ptr, int lo, int hi, int p, int lane)
 {
-    int lo = 0, hi = n_rows;  // row_ptr[lo] <= p < row_ptr[hi]
     while (hi - lo > 1) {
         const int step = (hi - lo + 63) >> 6;
         const int64_t at = (int64_t)lo + (int64_t)step * (lane + 1);
@@ -41,24 +40,56 @@ __device__ __forceinline__ int wave_max_scan(int v)
 }
 
 // tab[i] = the row of nonzero p0 + i for 0 <= i < n, tab in this wave's own LDS, n rounded up to 64, plus one entry;
-// r0 = the row of p0.  tab[n] becomes the row of nonzero p0 + n, or n_rows where the nonzeros end there.
+// nnz = row_ptr[n_rows] > p0.  Returns the row of p0.  tab[n] becomes a row other than that of nonzero p0 + n - 1 if a row ends there.
 // (Entries past the last nonzero hold n_rows.)  The row starts inside the range are marked, one coalesced read of
 // the row pointers for 64 rows, and a running maximum fills the rest; of the rows that start at one nonzero (empty
-// ones) the last counts.
-__device__ __forceinline__ void rows_of_range(const int32_t *__restrict__ row_ptr, int n_rows, int r0, int p0, int n, int *tab, int lane)
+// ones) the last counts.  Every read waits for the one before (0.34 us each), so the walk ends at the last
+// nonzero, and after as many steps as the search takes it is given up for that: each lane looks for the rows of its
+// own nonzeros among those left.  (20 thousand nonzeros, K = 16, us without / with both: 4 million empty rows behind
+// them 20700 / 8, spread over 4 million rows 59 / 14.)
+__device__ __forceinline__ int rows_of_range(const int32_t *__restrict__ row_ptr, int n_rows, int nnz, int p0, int n, int *tab, int lane)
 {
     const int n_pad = (n + 63) & ~63;
+    const int end = min(n, nnz - p0);
+    const int r0 = wave_find_row(row_ptr, 0, n_rows, p0, lane);
     for (int i = lane; i <= n_pad; i += 64) tab[i] = 0;
     __builtin_amdgcn_wave_barrier();
     if (lane == 0) tab[0] = r0;
     __builtin_amdgcn_wave_barrier();
-    for (int base = r0 + 1; base <= n_rows; base += 64) {
+    const int most = 16 + (n >> 4);
+    int base = r0 + 1, last = 0;  // the rows before base are marked; row base - 1 starts at nonzero p0 + last, or before p0
+    for (int step = 0; step < most && last < end; ++step, base += 64) {
         const int r = base + lane;
         const int rel = r <= n_rows ? row_ptr[r] - p0 : INT32_MAX;
         const int next = __shfl_down(rel, 1);
-        if (rel <= n && (rel != next || lane == 63)) tab[rel] = r;
-        if (__builtin_amdgcn_readlane(rel, 63) > n) break;
+        if (rel <= end && (rel != next || lane == 63)) tab[rel] = r;
+        last = __builtin_amdgcn_readlane(rel, 63);
     }
+    if (last < end) {  // (so base <= n_rows)
+        const int r1 = wave_find_row(row_ptr, base - 1, n_rows, p0 + end - 1, lane);
+        constexpr int U = 4;  // searches of a lane at a time
+        for (int i0 = last & ~63; i0 < end; i0 += 64 * U) {
+            int lo[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) lo[u] = base - 1;
+            for (int span = r1 - (base - 1); span > 0; span >>= 1) {  // the row lies in [lo, lo + span]
+                const int half = (span + 1) >> 1;
+                int at[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) at[u] = row_ptr[lo[u] + half];
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (at[u] - p0 <= i0 + 64 * u + lane) lo[u] += half;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int i = i0 + 64 * u + lane;
+                if (i >= last && i < end) tab[i] = lo[u];
+            }
+        }
+        if (lane == 0 && row_ptr[r1 + 1] == p0 + end) tab[end] = r1 + 1;
+    }
+    if (lane == 0 && nnz - p0 <= n) tab[nnz - p0] = n_rows;
     __builtin_amdgcn_wave_barrier();  // (LDS operations of one wave complete in order)
     int carry = 0;
     for (int i = 0; i < n_pad; i += 64) {
@@ -68,6 +99,7 @@ __device__ __forceinline__ void rows_of_range(const int32_t *__restrict__ row_pt
     }
     if (lane == 0) tab[n_pad] = max(tab[n_pad], carry);
     __builtin_amdgcn_wave_barrier();
+    return r0;
 }
 
 // Lane slot of a row of K >= 4 floats read in pieces of four, when K is no multiple of the lanes' pieces: piece

@@ -103,7 +103,7 @@ void sddmm_gather_kernel(const KArgs a)
     int *tab = row_tab[wave];
     if (!planned) {
         const int p0 = begin + (b0 << 6);
-        rows_of_range(a.row_ptr, a.n_rows, wave_find_row(a.row_ptr, a.n_rows, p0, lane), p0, (b1 - b0) << 6, tab, lane);
+        rows_of_range(a.row_ptr, a.n_rows, a.nnz, p0, (b1 - b0) << 6, tab, lane);
     }
 
     struct Batch {
@@ -219,7 +219,7 @@ void sddmm_generic_kernel(const KArgs a)
     int *tab = row_tab[wave];
     if (!planned) {
         const int p0 = begin + (b0 << 6);
-        rows_of_range(a.row_ptr, a.n_rows, wave_find_row(a.row_ptr, a.n_rows, p0, lane), p0, (b1 - b0) << 6, tab, lane);
+        rows_of_range(a.row_ptr, a.n_rows, a.nnz, p0, (b1 - b0) << 6, tab, lane);
     }
     for (int bi = b0; bi < b1; ++bi) {
         const int pos = begin + (bi << 6) + lane;

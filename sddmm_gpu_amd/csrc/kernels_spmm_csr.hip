@@ -150,8 +150,7 @@ void sddmm_spmm_csr_kernel(const int32_t *__restrict__ row_ptr, const int32_t *_
             const int p = p0 + min(i, nnz - 1 - p0);
             entries[i] = make_int2(col_ind[p], i < nnz - p0 ? __float_as_int(x[p]) : 0);
         }
-        const int r0 = wave_find_row(row_ptr, n_rows, p0, lane);
-        rows_of_range(row_ptr, n_rows, r0, p0, n, rows, lane);
+        const int r0 = rows_of_range(row_ptr, n_rows, nnz, p0, n, rows, lane);
 
         const float *Hl = H + pc.off;
         const int gb = g * S;
