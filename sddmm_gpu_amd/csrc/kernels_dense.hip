@@ -11,31 +11,41 @@
 //
 // Arithmetic.  The fp32 matrix instruction runs at a sixteenth of the bf16 one, so
 // every operand is cut into three bf16 parts whose sum it is exactly (8 + 8 + 8
-// significant bits), and six of the nine products of parts are summed in fp32; the
-// three left out lie below 2^-24 of the product (each at most 2^-27, 2^-27 and 2^-36
-// of it).  Error against 64 bits over the blocks of a recommender matrix (relative,
-// 2-norm; fp32 instruction -> parts): K = 128 1.72e-7 -> 1.41e-7, K = 256 2.39e-7 ->
-// 2.00e-7, K = 512 3.32e-7 -> 2.80e-7, all-positive factors 2.83e-7 -> 2.16e-7, factors
-// spread over e^(+-9) 9.2e-8 -> 8.6e-8: fewer roundings of the running sum (6 per 16
-// elements, 8 before).  What parts cannot carry -- infinities, NaNs, sums beyond the
-// range, values with bits under bf16's smallest subnormal -- is found and those
-// results are computed once more in fp32 (redo_picks).
+// significant bits), and eight of the nine products of parts are taken; the one left
+// out, of the two last parts, is at most 2^-34 of the product.  A part is at most 2^-8
+// of the one before it, so two of the others reach 2^-25 of the product: leaving them
+// out as well would show where a sum has few products.  The matrix instruction does
+// not round its sums to nearest either (a product alone comes out up to 2^-23 off), so
+// it adds up 16 elements of K at a time, the products of the first parts (exact for
+// one alone) apart from the seven small ones, and vector instructions, which round to
+// nearest, add the two to the running sum.  Error against 64 bits over the blocks
+// of a recommender matrix (relative, 2-norm; fp32 matrix instruction -> parts):
+// K = 128 1.72e-7 -> 0.73e-7, K = 512 3.32e-7 -> 1.06e-7, all-positive factors at 512
+// 2.83e-7 -> 0.77e-7, factors spread over e^(+-9) 9.2e-8 -> 7.2e-8; a product alone in
+// its row 2.53e-8 -> 2.53e-8 (at most 2^-24 (1 + 2^-7) of it), four in a row 4.6e-8 ->
+// 4.9e-8 (4.8e-8 for the chain of fp32 FMAs of the other kernels).  (Six products summed
+// into one accumulator, 0.70 ms where this takes 0.84: 2.8e-7 at K = 512, but 3.2e-8 and up
+// to 2.4 x 2^-24 for a product alone, 7.3e-8 for four.)  What parts cannot
+// carry -- infinities, NaNs, sums beyond the range, values with bits under bf16's
+// smallest subnormal -- is found and those results are computed once more in fp32
+// (redo_picks).
 //
 // One workgroup of 4 waves per block, each wave a 64 x 64 quarter (2 x 2 MFMA
 // tiles of 32 x 32, 64 accumulator registers).  K runs in chunks of 32: the
 // chunk's 128 x 32 slices of the W rows and of the H rows are gathered from
 // global memory into registers while the previous chunk is multiplied, cut into
-// their parts between its last 24 matrix instructions (8 vector instructions after
-// each: 768 clocks of either) and written to LDS.  One buffer: two would leave
-// room for one workgroup per CU only, and the second workgroup is what works while
-// the first passes its barriers.  What bounds it is the matrix cores and LDS about
-// alike: 1536 clocks of matrix instructions per chunk and wave, 1150 of LDS reads and
-// writes per workgroup, two workgroups on a CU.  Recommender shape, 57.6 M
-// nonzeros in 5687 blocks, K = 512: 1.04 ms with the fp32 instruction, 0.82 with parts
-// cut after the products, 0.71 with the cutting among them and conflict-free writes
-// (6 x 95 GFLOP take 0.23 ms at the nominal bf16 rate; picking and storing 14 B per
-// nonzero about 0.2).
+// their parts among its last 32 matrix instructions, and written to LDS.  One
+// buffer: two would leave room for one workgroup per CU only, and the second workgroup
+// is what works while the first passes its barriers.  What bounds it is the matrix
+// cores and the vector ALU about alike: per chunk and wave 2048 clocks of matrix
+// instructions, 1800 of cutting and adding, and per workgroup 1150 of LDS reads and
+// writes, two workgroups on a CU.  A tile's sums are added among the products of the
+// tile after it (0.88 -> 0.84 ms; all four tiles' sums at a time do not fit the
+// registers).  Recommender shape, 59.4 M nonzeros, K = 512: 1.03 ms with the fp32
+// instruction, 0.84 with parts; K = 384 0.80 and 0.66 (8 x 95 GFLOP take 0.3 ms at the
+// nominal bf16 rate; picking and storing 14 B per nonzero about 0.2).
 #include <hip/hip_runtime.h>
+#include <type_traits>
 #include "kernels.hpp"
 
 using namespace sddmm;
@@ -128,12 +138,14 @@ void sddmm_dense_kernel(const DenseArgs a)
     };
     uint32_t lost = 0;  // of the operands staged by this thread for the block in hand
     vec4u pa[2][3], pb[2][3];
+    auto split_part = [&](int k) {  // a quarter of it
+        const int i = k >> 1;
+        if (k & 1) split8(gb[2 * i], gb[2 * i + 1], pb[i], lost);
+        else split8(ga[2 * i], ga[2 * i + 1], pa[i], lost);
+    };
     auto split = [&]() {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            split8(ga[2 * i], ga[2 * i + 1], pa[i], lost);
-            split8(gb[2 * i], gb[2 * i + 1], pb[i], lost);
-        }
+        for (int k = 0; k < 4; ++k) split_part(k);
     };
     auto stage = [&]() {
 #pragma unroll
@@ -209,9 +221,6 @@ void sddmm_dense_kernel(const DenseArgs a)
         const bool has_next = nrange.y > nrange.x;
         uint32_t nw[2], nh[2];
         load_ids(has_next ? nslot : slot, nw, nh);
-        // the first round of this block's nonzero list is requested before the arithmetic starts
-        Round r0d;
-        load_round(r0d, range.x + t, range.y);
 
         floatx16 acc[2][2];
 #pragma unroll
@@ -222,7 +231,17 @@ void sddmm_dense_kernel(const DenseArgs a)
                 for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
         const unsigned char *ap = lds + (wr * 64 + m) * kRowB + kh * 16;
         const unsigned char *bp = lds + kStageB + (wc * 64 + m) * kRowB + kh * 16;
-        auto products = [&](int s) {  // 16 elements of K
+        // 16 elements of K, one 32 x 32 tile after the other, a tile's sums added to the running ones among the products
+        // of the tile after it; between(k) is further vector work to be done among the products of tile k
+        const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        floatx16 low = zero, high = zero;
+        auto add = [&](int k) {
+            floatx16 &sum = acc[k >> 1][k & 1];
+            sum += high + low;
+            asm volatile("" : "+v"(sum));  // (added here: left alone the compiler sinks it to where the sums are read)
+        };
+        auto products = [&](auto step, auto between) {
+            constexpr int s = decltype(step)::value;
             bf16x8 av[2][3], bv[2][3];
 #pragma unroll
             for (int p = 2; p >= 0; --p)
@@ -231,16 +250,21 @@ void sddmm_dense_kernel(const DenseArgs a)
                     av[i][2 - p] = *reinterpret_cast<const bf16x8 *>(ap + 32 * i * kRowB + (2 - p) * kPartB + 32 * s);
                     bv[i][p] = *reinterpret_cast<const bf16x8 *>(bp + 32 * i * kRowB + p * kPartB + 32 * s);
                 }
-            // the products of parts that reach into the upper 24 bits, small ones first
 #pragma unroll
-            for (int pq = 0; pq < 6; ++pq) {
-                constexpr int pp[6] = {0, 1, 2, 0, 1, 0}, qq[6] = {2, 1, 0, 1, 0, 0};
+            for (int k = 0; k < 4; ++k) {
+                const int i = k >> 1, j = k & 1;
+                constexpr int pp[7] = {1, 2, 0, 1, 2, 0, 1}, qq[7] = {2, 1, 2, 1, 0, 1, 0};
+                floatx16 l = zero;  // small ones first
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[i][pp[pq]], bv[j][qq[pq]], acc[i][j], 0, 0, 0);
+                for (int pq = 0; pq < 7; ++pq) l = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[i][pp[pq]], bv[j][qq[pq]], l, 0, 0, 0);
+                if (s + k > 0) add((k + 3) & 3);
+                const floatx16 h = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[i][0], bv[j][0], zero, 0, 0, 0);
+                between(k);
+                low = l;
+                high = h;
+                __builtin_amdgcn_sched_barrier(0);
             }
+            if (s == 1) add(3);
         };
         for (int c = 0; c + 1 < n_chunks; ++c) {
             // the next chunk's loads are issued before this chunk's arithmetic, and what they bring is
@@ -249,26 +273,18 @@ void sddmm_dense_kernel(const DenseArgs a)
             for (int i = 0; i < 2; ++i) { wofs[i] += kKC / 4; hofs[i] += kKC / 4; }
             fetch(wofs, hofs);
             __builtin_amdgcn_sched_barrier(0);
-            products(0);
-            __builtin_amdgcn_sched_barrier(0);  // (one step's operands in registers at a time)
-            products(1);
-            split();
-#pragma unroll
-            for (int i = 0; i < 24; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a matrix instruction
-                __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);  // vector instructions
-            }
-            __builtin_amdgcn_sched_barrier(0);
+            products(std::integral_constant<int, 0>{}, [](int) {});
+            products(std::integral_constant<int, 1>{}, split_part);
             lds_barrier();  // everyone has read this chunk
             stage();
             lds_barrier();
         }
         fetch(nw, nh);  // the last chunk: the next block's first
+        Round r0d;      // and the first round of this block's nonzero list
+        load_round(r0d, range.x + t, range.y);
         __builtin_amdgcn_sched_barrier(0);
-        products(0);
-        __builtin_amdgcn_sched_barrier(0);
-        products(1);
-        __builtin_amdgcn_sched_barrier(0);
+        products(std::integral_constant<int, 0>{}, [](int) {});
+        products(std::integral_constant<int, 1>{}, [](int) {});
         if (lost & 0xffffu) inexact = 1;  // (read after the next barriers; any writer writes the same)
         lost = 0;
         lds_barrier();  // everyone has read the last chunk

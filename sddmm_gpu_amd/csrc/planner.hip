@@ -757,13 +757,13 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
     // the non-compact tile streams, which can address a remainder): blocks of 128 ranked rows x
     // 128 ranked columns filled to the threshold go to the matrix cores.
     DenseBlocks D;
-    // Recommender shape, us per product without and with it (98 M nonzeros; 4.9 M): K = 512 3421 -> 2946
-    // (240 -> 213), K = 384 2579 -> 2234, K = 256 1715 -> 1567 (119 -> 124), K = 128 857 -> 903: below, the
-    // remainder's shorter runs cost the tile kernel what the matrix cores save.  The search makes planning
-    // 110-150 ms longer there, 300 calls' gain at K = 384 but 1000 at K = 256, so "choose" takes it from 384 on.
+    // Recommender shape, us per product without and with it (99.8 M nonzeros; 5.1 M): K = 512 3490 -> 3113
+    // (221 -> 220), K = 384 2611 -> 2367 (177 -> 172), K = 256 1729 -> 1626 (119 -> 126), K = 128 828 -> 916 (70 -> 83): below,
+    // the remainder's shorter runs cost the tile kernel what the matrix cores save.  The search makes planning
+    // 120-150 ms longer there, 600 calls' gain at K = 384 but 1300 at K = 256, so "choose" takes it from 384 on.
     // Plans that also serve the product with the dense factor keep the whole matrix on its column tiles below
     // 512: behind a dense core that product walks the CSR pattern (98 M nonzeros, K = 128: 2.98 ms against 1.46).
-    // The threshold is flat: 2953 / 2946 / 2938 / 3001 us at K = 512 for 40 / 30 / 22 / 16 % filled.
+    // The threshold is flat: 3118 / 3113 / 3166 / 3284 us at K = 512 for 40 / 30 / 22 / 16 % filled.
     const bool want_dense = opt.dense_blocks > 0 || (opt.dense_blocks < 0 && K >= (opt.spmm_stream > 0 ? 512 : 384));
     if (kernel == SDDMM_KERNEL_HYBRID && want_dense && K % 32 == 0 && kt / 4 > 16 &&
         (int64_t)n_rows * (K / 4) <= (int64_t)UINT32_MAX && (int64_t)n_cols * (K / 4) <= (int64_t)UINT32_MAX) {

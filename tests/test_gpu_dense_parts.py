@@ -67,3 +67,34 @@ def test_infinities_nans_and_sums_beyond_the_range():
     assert torch.equal(out[inf], ref32[inf]) and bool(inf.any())
     fin = torch.isfinite(ref32)
     assert bool((torch.abs(out.double() - ref)[fin] <= (K + 4) * 2.0 ** -24 * mag[fin]).all())
+
+
+@pytest.mark.parametrize("K", [96, 512])
+@pytest.mark.parametrize("kind", ["dense", "positive", "four a row", "one a row", "small"])
+def test_no_less_precise_than_fp32_sums(K, kind):
+    """The error against 64 bits beside that of fp32 sums which round once for every two products (what an fp32 matrix
+    instruction of two elements does at best), also where a row of W has one or a few elements, so that each product's
+    own rounding shows."""
+    d, plan = dense_plan(K)
+    g = torch.Generator(device=DEV); g.manual_seed(5)
+    W = torch.randn(d["n_rows"], K, generator=g, device=DEV)
+    H = torch.randn(d["n_cols"], K, generator=g, device=DEV)
+    if kind == "positive":
+        W, H = W.abs(), H.abs()
+    elif kind in ("four a row", "one a row"):
+        n = 4 if kind == "four a row" else 1
+        W *= torch.zeros_like(W).scatter_(1, torch.randint(0, K, (W.shape[0], n), generator=g, device=DEV), 1.0)
+    elif kind == "small":  # products of 2^-122, parts of them subnormal
+        W, H = torch.ldexp(W, torch.tensor(-60, device=DEV)), torch.ldexp(H, torch.tensor(-62, device=DEV))
+    out, ref, _, rows, cols = product(d, plan, W, H)
+    sums = torch.zeros(d["nnz"], device=DEV)
+    for k in range(0, K, 2):
+        sums = (sums.double() + (W[rows, k:k + 2].double() * H[cols, k:k + 2].double()).sum(1)).float()
+    scale = 2.0 ** 122 if kind == "small" else 1.0
+    err, err32 = (out.double() - ref) * scale, (sums.double() - ref) * scale
+    # A product alone is rounded once, to half a unit in the last place (2^-24 of it); next to others the sum of its 16
+    # is rounded, and then the running sum: at most a quarter more in the 2-norm than the sums of two, and less the
+    # denser the rows are.
+    if kind == "one a row":
+        assert bool((err.abs() <= 2.0 ** -24 * (1 + 2.0 ** -6) * ref.abs() * scale).all())
+    assert float(err.norm()) <= 1.25 * float(err32.norm()), (float(err.norm()), float(err32.norm()))
