@@ -412,6 +412,12 @@ int sddmm_execute_softmax(const sddmm_plan *plan, const float *d_val, const floa
                           float *d_out, void *stream);
 int sddmm_plan_spmm(const sddmm_plan *plan, const float *d_x, const float *d_H, float *d_Y, void *d_workspace,
                     int64_t workspace_bytes, void *stream);
+/* Which of them sddmm_plan_spmm takes for this plan: SDDMM_SPMM_CSR (as sddmm_spmm_csr), _TILES or _WALK (over the
+ * pattern, with the parts of cut rows kept). */
+#define SDDMM_SPMM_CSR 0
+#define SDDMM_SPMM_TILES 1
+#define SDDMM_SPMM_WALK 2
+int sddmm_plan_spmm_form(const sddmm_plan *plan, int32_t *form);
 int sddmm_row_softmax(int64_t n_rows, const int32_t *d_row_ptr, const float *d_x, float *d_out, void *stream);
 int sddmm_spmm_csr(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *d_row_ptr,
                    const int32_t *d_col_ind, const float *d_x, int32_t K, const float *d_H, float *d_Y,

@@ -19,6 +19,7 @@ OK, ERR_ARG, ERR_IO, ERR_FORMAT, ERR_RANGE, ERR_UNSORTED, ERR_HIP, ERR_NOMEM = r
 KERNEL_AUTO, KERNEL_ROW_GATHER, KERNEL_LDS_TILE, KERNEL_PANEL, KERNEL_HYBRID, KERNEL_DENSE_BLOCK = 0, 1, 2, 3, 4, 5
 EPILOGUE_SCALE, EPILOGUE_RESIDUAL = 0, 1
 FORM_SOFTMAX = 0x100
+SPMM_CSR, SPMM_TILES, SPMM_WALK = 0, 1, 2
 
 
 class SddmmError(RuntimeError):
@@ -117,6 +118,7 @@ SIGNATURES = {
     "sddmm_execute_softmax": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "sddmm_plan_workspace_bytes": (c_int, [c_void_p, POINTER(c_int64)]),
     "sddmm_execute_ws": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_void_p, c_int64, c_void_p]),
+    "sddmm_plan_spmm_form": (c_int, [c_void_p, POINTER(c_int32)]),
     "sddmm_plan_spmm": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
     "sddmm_row_softmax": (c_int, [c_int64, c_void_p, c_void_p, c_void_p, c_void_p]),
     "sddmm_spmm_csr": (c_int, [c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_void_p]),
@@ -368,6 +370,12 @@ class Plan:
         rc = self._lib.sddmm_execute_ws(self.h, d_val or None, d_W, d_H, d_out, form, d_workspace or None, workspace_bytes, stream or None)
         if rc:
             check(rc)
+
+    def spmm_form(self):
+        """SPMM_CSR, SPMM_TILES or SPMM_WALK: what spmm does behind this plan."""
+        f = c_int32()
+        check(lib().sddmm_plan_spmm_form(self.h, byref(f)))
+        return f.value
 
     def spmm(self, d_x, d_H, d_Y, d_workspace=0, workspace_bytes=0, stream=0):
         rc = self._lib.sddmm_plan_spmm(self.h, d_x or None, d_H, d_Y, d_workspace or None, workspace_bytes, stream or None)

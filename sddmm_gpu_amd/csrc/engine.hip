@@ -247,6 +247,22 @@ int sddmm_execute_ws(const sddmm_plan *plan, const float *d_val, const float *d_
     return launch_row_softmax(plan->info.n_rows, plan->d_row_ptr, d_out, d_out, stream, ws + plan->ws_softmax, plan->info.nnz);
 }
 
+static const Launch *spmm_launch(const sddmm_plan *plan)
+{
+    const Launch *found = nullptr;
+    for (const Launch &L : plan->launches)
+        if (L.sp_on) found = &L;
+    return found;
+}
+
+int sddmm_plan_spmm_form(const sddmm_plan *plan, int32_t *form)
+{
+    if (!plan || !form) return fail(SDDMM_ERR_ARG, "sddmm_plan_spmm_form: NULL argument");
+    const Launch *L = spmm_launch(plan);
+    *form = !L ? SDDMM_SPMM_CSR : L->sp_on == 1 ? SDDMM_SPMM_TILES : SDDMM_SPMM_WALK;
+    return SDDMM_OK;
+}
+
 int sddmm_plan_spmm(const sddmm_plan *plan, const float *d_x, const float *d_H, float *d_Y, void *d_workspace,
                     int64_t workspace_bytes, void *stream)
 {
@@ -254,9 +270,7 @@ int sddmm_plan_spmm(const sddmm_plan *plan, const float *d_x, const float *d_H, 
     const sddmm_plan_info &I = plan->info;
     if (I.n_rows == 0) return SDDMM_OK;
     if (!d_Y || (I.nnz > 0 && (!d_x || !d_H))) return fail(SDDMM_ERR_ARG, "sddmm_plan_spmm: NULL device pointer");
-    const Launch *Ls = nullptr;
-    for (const Launch &L : plan->launches)
-        if (L.sp_on) Ls = &L;
+    const Launch *Ls = spmm_launch(plan);
     if (!Ls || (Ls->sp_on == 1 && ((((uintptr_t)d_H) | ((uintptr_t)d_Y)) & 15u))) {
         // no tile stream for the product in this plan: the CSR form, gathering H rows
         if (!plan->d_row_ptr || (I.nnz > 0 && !plan->d_col)) return fail(SDDMM_ERR_ARG, "sddmm_plan_spmm: the plan holds no pattern");

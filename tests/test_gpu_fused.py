@@ -261,21 +261,51 @@ def spmm_ok(oracle, d, x, got, K):
     assert np.all(got[deg == 0] == 0)
 
 
-@pytest.mark.parametrize("cfg,scale,K,opts", [
-    (3, 0.05, 128, {"split_min_nnz": 0}), (3, 0.05, 128, {"split_min_nnz": 0, "tile_few_blocks": 0}),
-    (3, 0.03, 256, {"split_min_nnz": 0}), (3, 0.03, 64, {"split_min_nnz": 0, "stage_factor": 0}), (3, 0.03, 32, {"split_min_nnz": 0, "stage_factor": 0}),
-    (2, 1.0, 256, {}), (2, 1.0, 128, {"tile_size_x": 192}), (5, 2.0 ** -6, 128, {}), (5, 2.0 ** -6, 512, {"tile_runs": 1}),
-    (1, 1.0, 32, {"kernel": capi.KERNEL_LDS_TILE})])
-def test_plan_spmm_on_the_tile_stream(oracle, cfg, scale, K, opts):
-    """Y = X H on the plan's column tiles (spmm_stream = 1): against the oracle, the same bits on
+TILES, WALK = capi.SPMM_TILES, capi.SPMM_WALK
+
+
+@pytest.mark.parametrize("cfg,scale,K,opts,form", [
+    (3, 0.05, 128, {"split_min_nnz": 0}, WALK), (3, 0.05, 128, {"split_min_nnz": 0, "tile_few_blocks": 0}, WALK),
+    (3, 0.03, 256, {"split_min_nnz": 0}, WALK), (3, 0.03, 64, {"split_min_nnz": 0, "stage_factor": 0}, WALK),
+    (3, 0.03, 32, {"split_min_nnz": 0, "stage_factor": 0}, WALK),
+    (2, 1.0, 256, {}, TILES), (2, 1.0, 128, {"tile_size_x": 192}, TILES), (5, 2.0 ** -6, 128, {}, WALK), (5, 2.0 ** -6, 512, {"tile_runs": 1}, WALK),
+    (1, 1.0, 32, {"kernel": capi.KERNEL_LDS_TILE}, WALK)])
+def test_plan_spmm_on_the_tile_stream(oracle, cfg, scale, K, opts, form):
+    check_plan_spmm(oracle, synth.make(cfg, scale, K=K), K, opts, form)
+
+
+def wide(n_cols, per_row, K, short):
+    """400 rows of per_row nonzeros at uniform columns, H of more than 6 MB; short: among them rows of 1 to 6 nonzeros
+    and empty ones."""
+    from test_gpu_parity import _dict_of
+    rng = np.random.default_rng(K)
+    counts = np.full(400, per_row)
+    if short:
+        counts = np.concatenate([counts, rng.integers(0, 7, 500)])
+        rng.shuffle(counts)
+    rows = np.repeat(np.arange(len(counts)), counts)
+    cols = np.concatenate([rng.choice(n_cols, c, replace=False) for c in counts])
+    return _dict_of(len(counts), n_cols, rows, cols, K, rng)
+
+
+# every width of a K slice, two slices, and a second class of rows that gather
+@pytest.mark.parametrize("short", [False, True])
+@pytest.mark.parametrize("n_cols,per_row,K", [(50000, 1500, 32), (25000, 1200, 64), (13000, 1100, 128), (13000, 1100, 256)])
+def test_plan_spmm_tiles_at_every_slice_width(oracle, n_cols, per_row, K, short):
+    opts = dict(split_min_nnz=0, stage_factor=0, short_row_max=16 if short else 0)
+    info = check_plan_spmm(oracle, wide(n_cols, per_row, K, short), K, opts, TILES)
+    assert (info["class_nnz"][2] > 0) == short and info["k_slice"] == min(K, 128)
+
+
+def check_plan_spmm(oracle, d, K, opts, form):
+    """Y = X H behind a plan (spmm_stream = 1) in the form expected: against the oracle, the same bits on
     every call and with a caller's workspace, and the SDDMM of the same plan unchanged."""
-    d = synth.make(cfg, scale, K=K)
     dev = torch.device(DEV)
     S = capi.Coo.from_arrays(d["n_rows"], d["n_cols"], d["row_ind"].numpy(), d["col_ind"].numpy(), d["val"].numpy())
     plan = S.plan(K, options=capi.PlanOptions.defaults(ignore_env=1, spmm_stream=1, **opts))
     info = plan.info()
-    assert info["spmm_runs"] > 0, info
-    g = torch.Generator().manual_seed(K + cfg)
+    assert info["spmm_runs"] > 0 and plan.spmm_form() == form, (plan.spmm_form(), info)
+    g = torch.Generator().manual_seed(K)
     x = torch.randn(d["nnz"], generator=g)
     xd = x.to(dev); H = d["H"].to(dev).contiguous(); W = d["W"].to(dev)
     Y = torch.full((d["n_rows"], K), float("nan"), device=dev)
@@ -307,6 +337,7 @@ def test_plan_spmm_on_the_tile_stream(oracle, cfg, scale, K, opts):
     torch.cuda.synchronize()
     from test_gpu_parity import check
     check(d, out.cpu().numpy(), oracle, K)
+    return info
 
 
 def test_plan_spmm_without_a_tile_stream_takes_the_csr_path(oracle):
@@ -318,7 +349,7 @@ def test_plan_spmm_without_a_tile_stream_takes_the_csr_path(oracle):
     xd = x.to(dev); H = d["H"].to(dev).contiguous()
     for opts in ({}, {"kernel": capi.KERNEL_ROW_GATHER, "spmm_stream": 1}):
         plan = S.plan(K, options=capi.PlanOptions.defaults(ignore_env=1, **opts))
-        assert plan.info()["spmm_runs"] == 0
+        assert plan.info()["spmm_runs"] == 0 and plan.spmm_form() == capi.SPMM_CSR
         Y = torch.full((d["n_rows"], K), float("nan"), device=dev)
         plan.spmm(xd.data_ptr(), H.data_ptr(), Y.data_ptr())
         torch.cuda.synchronize()

@@ -71,6 +71,30 @@ def test_saved_plan_reproduces_the_fresh_plan(oracle, tmp_path, cfg, scale, K, o
     assert e.value.code == capi.ERR_ARG
 
 
+@pytest.mark.parametrize("K,form", [(64, capi.SPMM_WALK), (50, capi.SPMM_WALK), (205, capi.SPMM_WALK), (256, capi.SPMM_TILES)])
+def test_saved_plan_with_a_product_and_ragged_ranks(tmp_path, K, form):
+    """Plans that also serve the product with the dense factor, over the pattern and on column tiles, and ranks without a
+    tile kernel of their width: the loaded plan gives the bits of the saved one, in both operations."""
+    d = synth.make(2 if form == capi.SPMM_TILES else 3, 1.0 if form == capi.SPMM_TILES else 0.03, K=K)
+    dev = torch.device("cuda:0")
+    o = capi.PlanOptions.defaults(ignore_env=1, spmm_stream=1, kernel=capi.KERNEL_HYBRID, short_row_max=0, stage_factor=0, split_min_nnz=0)
+    S = capi.Coo.from_arrays(d["n_rows"], d["n_cols"], d["row_ind"].numpy(), d["col_ind"].numpy(), d["val"].numpy())
+    fresh = S.plan(K, options=o)
+    path = tmp_path / "product.plan"
+    fresh.save(path)
+    loaded = S.load_plan(path, K, options=o)
+    assert fresh.spmm_form() == loaded.spmm_form() == form and loaded.info()["class_nnz"][0] == d["nnz"]
+    H = d["H"].to(dev); x = d["val"].to(dev)
+    Y = [torch.full((d["n_rows"], K), float("nan"), device=dev) for _ in range(2)]
+    out = []
+    for p, y in ((fresh, Y[0]), (loaded, Y[1])):
+        out.append(run_plan(p, d, dev))
+        p.spmm(x.data_ptr(), H.data_ptr(), y.data_ptr())
+        torch.cuda.synchronize()
+        p.close()
+    assert torch.equal(out[0], out[1]) and torch.equal(Y[0], Y[1]) and bool(torch.isfinite(Y[0]).all())
+
+
 def test_mismatched_key_is_rejected(tmp_path):
     d = synth.make(3, 0.03, K=64)
     S = capi.Coo.from_arrays(d["n_rows"], d["n_cols"], d["row_ind"].numpy(), d["col_ind"].numpy(), d["val"].numpy())

@@ -43,6 +43,8 @@ def test_uneven_items(oracle, kind, K, few):
     plan.execute(t["val"].data_ptr(), t["W"].data_ptr(), t["H"].data_ptr(), out.data_ptr())
     torch.cuda.synchronize()
     check(d, out.cpu().numpy(), oracle, K=K)
+    # (cut and dealt out anew or not: the product of these goes over the pattern, as the runs are short or the matrix is small)
+    assert plan.spmm_form() == capi.SPMM_WALK
     Y = torch.full((n, K), float("nan"), device=dev)
     plan.spmm(t["val"].data_ptr(), t["H"].data_ptr(), Y.data_ptr())
     torch.cuda.synchronize()
