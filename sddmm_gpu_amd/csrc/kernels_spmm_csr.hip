@@ -52,14 +52,17 @@ void sddmm_spmm_zero_rows_kernel(const int32_t *__restrict__ row_ptr, float *Y, 
 }
 
 // The rows that the product with records leaves: empty rows become 0, rows cut between workgroups (of 2^shift
-// nonzeros) the sum of their records, workgroup by workgroup.
+// nonzeros) the sum of their records, workgroup by workgroup.  A wave looks at 64 rows, at fewer where that would leave
+// less than 2048 waves: where rows are longer than a workgroup's share all of them are cut, and a few waves taking 64 each,
+// piece after piece, are slower than the product itself.
 __global__ __launch_bounds__(256)
-void sddmm_spmm_cut_rows_kernel(const int32_t *__restrict__ row_ptr, const float *__restrict__ part, float *Y, int64_t n_rows, int K, int shift)
+void sddmm_spmm_cut_rows_kernel(const int32_t *__restrict__ row_ptr, const float *__restrict__ part, float *Y, int64_t n_rows, int K, int shift,
+                                int rows_per_wave)
 {
     __shared__ int list[4][64];
     __shared__ int2 range[4][64];  // first and last workgroup; (0, -1): an empty row
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t r = lane < rows_per_wave ? ((int64_t)blockIdx.x * 4 + wave) * rows_per_wave + lane : n_rows;
     int s = 0, e = 1;
     if (r < n_rows) { s = row_ptr[r]; e = row_ptr[r + 1]; }
     const int w0 = s >> shift, w1 = (e - 1) >> shift;
@@ -327,8 +330,10 @@ int launch_spmm_csr_records(int64_t n_rows, int64_t nnz, const int32_t *d_row_pt
     const CsrShape c = csr_shape(nnz, K);
     hipStream_t st = (hipStream_t)stream;
     if (int rc = checked(launch_csr<true>(c, n_rows, nnz, d_row_ptr, d_col_ind, d_x, K, d_H, d_Y, d_part, st))) return rc;
-    return checked(launch(sddmm_spmm_cut_rows_kernel, dim3((unsigned)((n_rows + 255) / 256)), dim3(256), 0, st, d_row_ptr, d_part, d_Y, n_rows,
-                          (int)K, c.wg_shift));
+    int per_wave = 64;
+    while (per_wave > 1 && n_rows < (int64_t)2048 * per_wave) per_wave /= 2;
+    return checked(launch(sddmm_spmm_cut_rows_kernel, dim3((unsigned)((n_rows + 4 * per_wave - 1) / (4 * per_wave))), dim3(256), 0, st, d_row_ptr,
+                          d_part, d_Y, n_rows, (int)K, c.wg_shift, per_wave));
 }
 
 }  // namespace sddmm
