@@ -13,27 +13,28 @@ namespace {
 
 // Deals the items of one group of workgroups out anew when their loads are uneven (a band or a window puts nearly
 // all nonzeros of a row block into a few column tiles; skewed columns do so less drastically): the items, in tile
-// order, are cut into consecutive pieces of `quantum` units and handed to the workgroups in order, each filled up to
-// the least load at which they all fit, where a piece costs its length and, for the first one of a tile, `stage`.
-// load(item) is an item's length in the units of cut(item, from, to).  Returns that least load.
+// order, are cut into consecutive pieces of whole batches and handed to the workgroups in order, each filled up to
+// the least load at which they all fit, where a piece costs its positions and, for the first one of a tile, `stage`.
+// Returns that least load; out[w] lists the pieces of workgroup w.
 struct Piece {
     int32_t item;
-    int64_t from, to;
+    int64_t from, to;  // stream positions from the item's first
 };
-int64_t deal_evenly(const std::vector<int64_t> &loads, const std::vector<int32_t> &tiles, size_t n_wgs, int64_t stage, int64_t quantum,
-                    std::vector<std::vector<Piece>> *out)
+int64_t deal_evenly(const std::vector<WorkItem> &items, size_t n_wgs, int64_t stage, std::vector<std::vector<Piece>> &out)
 {
+    constexpr int64_t kBatch = 64;
     int64_t total = 0;
-    for (int64_t l : loads) total += l;
+    for (const WorkItem &it : items) total += it.end - it.begin;
     auto fits = [&](int64_t most, std::vector<std::vector<Piece>> *seq) {
         size_t w = 0;
         int64_t used = 0;
         int32_t held = -1;
-        for (size_t i = 0; i < loads.size(); ++i) {
+        for (size_t i = 0; i < items.size(); ++i) {
+            const int64_t load = items[i].end - items[i].begin;
             int64_t at = 0;
-            while (at < loads[i]) {
-                const int64_t cost = held == tiles[i] ? 0 : stage;
-                const int64_t room = (most - used - cost) / quantum * quantum;
+            while (at < load) {
+                const int64_t cost = held == items[i].tile ? 0 : stage;
+                const int64_t room = (most - used - cost) / kBatch * kBatch;
                 if (room <= 0) {
                     if (++w >= n_wgs) return false;
                     used = 0;
@@ -41,24 +42,22 @@ int64_t deal_evenly(const std::vector<int64_t> &loads, const std::vector<int32_t
                     if (most <= stage) return false;
                     continue;
                 }
-                const int64_t n = std::min(room, loads[i] - at);
+                const int64_t n = std::min(room, load - at);
                 if (seq) (*seq)[w].push_back({(int32_t)i, at, at + n});
                 at += n;
                 used += cost + n;
-                held = tiles[i];
+                held = items[i].tile;
             }
         }
         return true;
     };
-    int64_t lo = std::max<int64_t>(1, total / (int64_t)std::max<size_t>(n_wgs, 1)), hi = total + (stage + quantum) * ((int64_t)loads.size() + 1);
-    while (hi - lo > std::max<int64_t>(quantum, lo / 256)) {
+    int64_t lo = std::max<int64_t>(1, total / (int64_t)std::max<size_t>(n_wgs, 1)), hi = total + (stage + kBatch) * ((int64_t)items.size() + 1);
+    while (hi - lo > std::max<int64_t>(kBatch, lo / 256)) {
         const int64_t mid = (lo + hi) / 2;
         if (fits(mid, nullptr)) hi = mid; else lo = mid;
     }
-    if (out) {
-        out->assign(n_wgs, {});
-        fits(hi, out);
-    }
+    out.assign(n_wgs, {});
+    fits(hi, &out);
     return hi;
 }
 
@@ -658,21 +657,21 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
                 for (int sh = 0; sh < shares; ++sh)
                     for (int32_t j : tiles_ne) { items.push_back(item_of(sh, j)); item_keys.push_back({sh, j}); }
             }
-            // uneven items (see deal_evenly): inside a die where the row blocks belong to dies, over all workgroups
-            // otherwise, in units of stream positions.  True: dealt out anew.
-            auto even = [&](std::vector<WorkItem> &list, int64_t stage, int64_t quantum, const std::function<int64_t(const WorkItem &)> &load,
-                            const std::function<WorkItem(const WorkItem &, int64_t, int64_t)> &cut_item) {
+            // Uneven items (see deal_evenly): inside a die where the row blocks belong to dies, over all workgroups
+            // otherwise.
+            auto even = [&]() {
+                const int64_t stage = 4 * (int64_t)x;  // (staging a tile of x rows takes about as long as 4 x positions of one workgroup, at every rank)
                 const int groups = xcd_local ? 8 : 1;
                 std::vector<std::vector<WorkItem>> seq((size_t)c.cus);
                 int64_t most_now = 0, most_new = 0, total = 0;
                 for (int b = 0; b < c.cus; ++b) {
                     int64_t sum = 0;
                     int32_t held = -1;
-                    for (size_t k = (size_t)b; k < list.size(); k += (size_t)c.cus) {
-                        if (list[k].end <= list[k].begin) continue;
-                        sum += load(list[k]) + (list[k].tile != held ? stage : 0);
-                        total += load(list[k]);
-                        held = list[k].tile;
+                    for (size_t k = (size_t)b; k < items.size(); k += (size_t)c.cus) {
+                        if (items[k].end <= items[k].begin) continue;
+                        sum += items[k].end - items[k].begin + (items[k].tile != held ? stage : 0);
+                        total += items[k].end - items[k].begin;
+                        held = items[k].tile;
                     }
                     most_now = std::max(most_now, sum);
                 }
@@ -683,34 +682,29 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
                     std::vector<int> wgs;
                     for (int b = gr; b < c.cus; b += groups) {
                         wgs.push_back(b);
-                        for (size_t k = (size_t)b; k < list.size(); k += (size_t)c.cus)
-                            if (list[k].end > list[k].begin) mine.push_back(list[k]);
+                        for (size_t k = (size_t)b; k < items.size(); k += (size_t)c.cus)
+                            if (items[k].end > items[k].begin) mine.push_back(items[k]);
                     }
                     std::stable_sort(mine.begin(), mine.end(), [](const WorkItem &u, const WorkItem &v) { return u.tile < v.tile; });
-                    std::vector<int64_t> loads;
-                    std::vector<int32_t> tiles;
-                    for (const WorkItem &w : mine) { loads.push_back(load(w)); tiles.push_back(w.tile); }
                     std::vector<std::vector<Piece>> got;
-                    most_new = std::max(most_new, deal_evenly(loads, tiles, wgs.size(), stage, quantum, &got));
+                    most_new = std::max(most_new, deal_evenly(mine, wgs.size(), stage, got));
                     for (size_t w = 0; w < wgs.size(); ++w)
-                        for (const Piece &pc : got[w]) seq[(size_t)wgs[w]].push_back(cut_item(mine[(size_t)pc.item], pc.from, pc.to));
+                        for (const Piece &pc : got[w]) {
+                            const WorkItem &it = mine[(size_t)pc.item];
+                            seq[(size_t)wgs[w]].push_back({(int32_t)(it.begin + pc.from), (int32_t)(it.begin + pc.to),
+                                                           (int32_t)(it.batch_base + (shorts ? pc.from / 64 : 0)), it.tile});
+                        }
                 }
                 if (most_new * 10 > most_now * 7) return false;
                 size_t turns = 0;
                 for (auto &q : seq) turns = std::max(turns, q.size());
-                list.assign(turns * (size_t)c.cus, WorkItem{0, 0, 0, 0});
+                items.assign(turns * (size_t)c.cus, WorkItem{0, 0, 0, 0});
                 for (int b = 0; b < c.cus; ++b)
-                    for (size_t k = 0; k < seq[(size_t)b].size(); ++k) list[k * (size_t)c.cus + (size_t)b] = seq[(size_t)b][k];
+                    for (size_t k = 0; k < seq[(size_t)b].size(); ++k) items[k * (size_t)c.cus + (size_t)b] = seq[(size_t)b][k];
                 return true;
             };
-            bool uneven = false;
             const size_t items_whole = items.size();
-            // (staging a tile of x rows takes about as long as 4 x positions of one workgroup, at every rank)
-            if (!panel_local && mf_nwm == 0 && c.opt.tile_assign < 0)
-                uneven = even(items, 4 * (int64_t)x, 64, [](const WorkItem &w) { return (int64_t)w.end - w.begin; },
-                              [&](const WorkItem &w, int64_t from, int64_t to) {
-                                  return WorkItem{(int32_t)(w.begin + from), (int32_t)(w.begin + to), (int32_t)(w.batch_base + (shorts ? from / 64 : 0)), w.tile};
-                              });
+            const bool uneven = !panel_local && mf_nwm == 0 && c.opt.tile_assign < 0 && even();
             // The product walks the same (row block, tile) items on the same workgroups.  Where they are uneven -- rows that
             // lie together use columns that lie together -- the walk over the CSR pattern finds its H rows in the caches
             // and is the faster one at any run length (windows of 400 to 600, 5 to 14 million nonzeros, items cut and
