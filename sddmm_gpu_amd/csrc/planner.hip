@@ -842,7 +842,9 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         // So do plans that also serve the product with the dense factor on column tiles: that product wants long runs, and
         // tiling the short rows as well, 10 % faster for the SDDMM alone, costs it more (ratings, SDDMM + product, us by
         // length / all tiled: 15.7 M nonzeros, K = 64 93 + 132 / 82 + 229; 5.4 M, K = 128 64 + 103 / 67 + 145; 11.8 M, K = 192
-        // 213 + 338 / 188 + 500).  Below 4 million nonzeros it walks the CSR pattern whatever the split.
+        // 213 + 338 / 188 + 500).  Below 4 million nonzeros the split is the model's: the fixed rules make one class of the rows
+        // there, and the product mostly walks the CSR pattern (3 to 4 M, K = 256, windows: 196 + 174 by the fixed rules,
+        // 113 + 169 by the model; uniform 522 + 517 and 332 + 515).
         const bool tiled_product = opt.spmm_stream > 0 && nnz >= 4000000 && !ragged && spmm_tile_supported(kt);
         const bool by_model = D.n_dense == 0 && opt.short_row_max < 0 && opt.stage_factor < 0 && opt.split_min_nnz < 0 && !tiled_product;
         int64_t slab_cols = 0;  // chosen by the model

@@ -2,6 +2,7 @@
 // work assignment across dies, the opt-in matrix-core share and the SpMM stream on the same tiles.
 #include <hip/hip_runtime.h>
 #include <chrono>
+#include <cmath>
 #include <cstring>
 #include <new>
 #include <unistd.h>
@@ -233,14 +234,16 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         const int64_t n_seg = (int64_t)T.active_end.size();
         // Runs of less than 12 nonzeros: a partial row of Y per run is written and read for little work, and the product
         // goes over the CSR pattern instead (attention window, 16,384 tokens, K = 64, runs of 10: 131 -> 65 us; K = 32, runs
-        // of 8: 146 -> 46 us; ratings, K = 128, runs of 17: 81 against 110 us at 4.1 M nonzeros, 342 against 445 at 19.6 M).
-        // Below 4 million nonzeros the two are level at best (0.5 M, K = 128: 27 us) or the walk is far ahead (window
-        // of 101, 8,898 tokens, K = 32, runs of 14: 110 against 25 us).  Both hold while H is about as large as a die's L2,
+        // of 8: 146 -> 46 us; ratings, K = 128, runs of 17, 4.9 M nonzeros: 90 against 114 us, 19.6 M 342 against 445).  So it
+        // does on small matrices (product_walks; tiles against walk, ratings of 1.5 / 2.4 / 3.6 M, K = 64 47 / 28, 55 / 40 and
+        // 64 / 55, K = 128 51 / 47, 64 / 64 and 86 / 91; word counts of 0.9 M, K = 128 35 / 31, 1.5 and 3.6 M, K = 64 31 / 30
+        // and 58 / 55; uniform, 2.3 M, K = 64 37 / 37).  Both hold while H is about as large as a die's L2,
         // from where the walk then gathers; beyond, only really short runs (ratings, K = 384, 2 to 3.5 M nonzeros, H of 7 and
-        // 8 MB, runs of 10: 180 against 211 and 338 against 387 us).
+        // 8 MB, runs of 10: 180 against 211 and 338 against 387 us; word counts of 6.9 M, K = 128, H of 27 MB, runs of 7 392
+        // against 269, but uniform, 2.3 M, K = 256, H of 17 MB, runs of 5 190 against 261).
         const bool h_near = (int64_t)c.n_cols * c.K * 4 <= 6000000;
         if (want_spmm && rb == 0 && c.nnz == c.P->info.nnz &&
-            (ragged || (h_near && (L.nnz < 12 * n_seg || c.nnz < 4000000)) || L.nnz < 8 * n_seg)) { want_spmm = false; sp_csr = true; }
+            (ragged || (h_near && (L.nnz < 12 * n_seg || product_walks(c.nnz, c.K))) || L.nnz < 8 * n_seg)) { want_spmm = false; sp_csr = true; }
         // row-block boundaries of the 2-D assignment: equal shares of the rows' nonzeros
         std::vector<int32_t> cut;
         auto make_cuts = [&](int n_shares) {
@@ -658,22 +661,25 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
                     for (int32_t j : tiles_ne) { items.push_back(item_of(sh, j)); item_keys.push_back({sh, j}); }
             }
             // Uneven items (see deal_evenly): inside a die where the row blocks belong to dies, over all workgroups
-            // otherwise.
+            // otherwise.  busiest: the positions of the workgroup that has most.
+            int64_t busiest = 0, total = 0;
             auto even = [&]() {
                 const int64_t stage = 4 * (int64_t)x;  // (staging a tile of x rows takes about as long as 4 x positions of one workgroup, at every rank)
                 const int groups = xcd_local ? 8 : 1;
                 std::vector<std::vector<WorkItem>> seq((size_t)c.cus);
-                int64_t most_now = 0, most_new = 0, total = 0;
+                int64_t most_now = 0, most_new = 0;
                 for (int b = 0; b < c.cus; ++b) {
-                    int64_t sum = 0;
+                    int64_t sum = 0, staged = 0;
                     int32_t held = -1;
                     for (size_t k = (size_t)b; k < items.size(); k += (size_t)c.cus) {
                         if (items[k].end <= items[k].begin) continue;
-                        sum += items[k].end - items[k].begin + (items[k].tile != held ? stage : 0);
-                        total += items[k].end - items[k].begin;
+                        sum += items[k].end - items[k].begin;
+                        staged += items[k].tile != held ? stage : 0;
                         held = items[k].tile;
                     }
-                    most_now = std::max(most_now, sum);
+                    most_now = std::max(most_now, sum + staged);
+                    busiest = std::max(busiest, sum);
+                    total += sum;
                 }
                 // (what is nearly even keeps its whole tiles: here when no dealing can gain enough, below when this one does not)
                 if ((total / c.cus + stage) * 10 > most_now * 7) return false;
@@ -709,8 +715,13 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
             // lie together use columns that lie together -- the walk over the CSR pattern finds its H rows in the caches
             // and is the faster one at any run length (windows of 400 to 600, 5 to 14 million nonzeros, items cut and
             // dealt out anew against the walk: K = 128 451 / 279, 283 / 236 and 423 / 287 us, K = 64 283 / 150, 175 / 126
-            // and 155 / 68, K = 32 with runs of 41 220 / 84).
-            if (want_spmm && uneven && c.nnz == c.P->info.nnz) { want_spmm = false; sp_csr = true; }
+            // and 155 / 68, K = 32 with runs of 41 220 / 84), but only so far as the caches go: where the busiest workgroup
+            // has less than 3.5 times the mean, the longer the rows of H the smaller H may be (bands of 1.4 to 4.8 M,
+            // 2 to 2.5 times the mean: K = 64, H of 12, 48 and 53 MB 68 / 57, 108 / 81 and 133 / 150; K = 128, 16, 18 and 20 MB
+            // 57 / 60, 55 / 64 and 99 / 117; K = 256, 37 and 41 MB 107 / 151 and 198 / 332; word counts of 24.5 M, K = 256 1946 / 2937; R-MAT of 4.3 M, 16 times the mean, K = 64 to 256, H of
+            // 34 to 134 MB 211 / 94, 369 / 227 and 777 / 618).
+            if (want_spmm && uneven && c.nnz == c.P->info.nnz &&
+                (busiest * c.cus * 2 >= total * 7 || (double)c.n_cols * c.K * c.K * std::sqrt((double)c.K) <= 6.4e9)) { want_spmm = false; sp_csr = true; }
             if (want_spmm && !panel_local && item_keys.size() == items_whole) build_spmm(item_keys);
         } else if (want_spmm && rb == 0 && rows.size() <= (size_t)panel_rows) {
             // (equal position ranges for the SDDMM: the product takes one item per column tile)

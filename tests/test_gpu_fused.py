@@ -297,6 +297,22 @@ def test_plan_spmm_tiles_at_every_slice_width(oracle, n_cols, per_row, K, short)
     assert (info["class_nnz"][2] > 0) == short and info["k_slice"] == min(K, 128)
 
 
+# On either side of each line between the forms: a matrix whose H is near a die's L2 in size below and above 1.8 GB of
+# gathered H rows; bands whose tiles are uneven, at a short and a long row of H.
+@pytest.mark.parametrize("kind,n_rows,K,form", [("near", 3400, 256, WALK), ("near", 3600, 256, TILES), ("band", 36000, 64, WALK), ("band", 36000, 256, TILES)])
+def test_plan_spmm_form_by_size_and_evenness(oracle, kind, n_rows, K, form):
+    from test_gpu_parity import _dict_of
+    rng = np.random.default_rng(n_rows)
+    if kind == "near":
+        rows = np.repeat(np.arange(n_rows), 500)
+        cols = np.argsort(rng.random((n_rows, 5000), dtype=np.float32), axis=1)[:, :500].ravel()
+        d = _dict_of(n_rows, 5000, rows, cols, K, rng)
+    else:
+        key = np.unique(np.repeat(np.arange(n_rows), 40) * n_rows + np.clip(np.repeat(np.arange(n_rows), 40) + rng.integers(-200, 201, n_rows * 40), 0, n_rows - 1))
+        d = _dict_of(n_rows, n_rows, key // n_rows, key % n_rows, K, rng)
+    check_plan_spmm(oracle, d, K, dict(split_min_nnz=0, stage_factor=0, short_row_max=0), form)
+
+
 # The rows cut between workgroups are added up by waves that look at 1 to 64 rows each, by how many rows there are.
 # (The SDDMM's check counts results off by more than 1e-5 sqrt(K) where the CPU's are not: it means nothing on a row or two.)
 @pytest.mark.parametrize("K", [32, 50, 300])
