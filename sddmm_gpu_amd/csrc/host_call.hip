@@ -297,9 +297,18 @@ extern "C" int sddmm_gpu(const sddmm_plan *plan, const float *h_W, const float *
         HIP_TRY(hipGetDevice(&device));
         if (device != c.device) return fail(SDDMM_ERR_ARG, "sddmm_gpu: the plan's host calls belong to device %d, the current device is %d", c.device, device);
         std::lock_guard<std::mutex> transfer(c.pipe->busy);
+        // nothing of a call that failed, by its code or by an exception, is left on the streams for the next one to meet
+        struct Drain {
+            HostPipe &pipe;
+            bool failed = true;
+            ~Drain()
+            {
+                if (failed)
+                    for (hipStream_t s : pipe.stream) (void)hipStreamSynchronize(s);
+            }
+        } drain{*c.pipe};
         const int rc = host_call(plan, c, h_W, h_H, h_out, kernel_ms);
-        if (rc != SDDMM_OK)  // nothing of a failed call is left on the streams for the next one to meet
-            for (hipStream_t s : c.pipe->stream) (void)hipStreamSynchronize(s);
+        drain.failed = rc != SDDMM_OK;
         return rc;
     } catch (const std::exception &e) {
         return fail(SDDMM_ERR_NOMEM, "sddmm_gpu: %s", e.what());
