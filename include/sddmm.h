@@ -77,7 +77,7 @@ typedef struct sddmm_plan_info {
     int32_t lds_bytes;    /* LDS per workgroup of the main kernel */
     int32_t grid, block;  /* launch shape of the main kernel */
     int64_t n_blocks;     /* (row panel, column tile) work items with at least one nonzero */
-    int64_t device_bytes; /* device memory owned by the plan */
+    int64_t device_bytes; /* device memory owned by the plan, what sddmm_gpu keeps included */
     int64_t class_nnz[3]; /* nonzeros handled by LDS_TILE, PANEL (explicit PANEL plans only), ROW_GATHER launches;
                              with dense_nnz they add up to nnz */
     int64_t class_rows[3];
@@ -448,9 +448,18 @@ int sddmm_execute_profiled(const sddmm_plan *plan, const float *d_val, const flo
  * sddmm_GPU(S, tiledS, P, W, H) (sddmm.cu:32): copies W and H to the device,
  * runs the kernels between two events, copies the result back into h_out
  * (nnz fp32, sorted order) and reports the kernel-only time in milliseconds,
- * the quantity the reference prints at sddmm.cu:109-114.                    */
+ * the quantity the reference prints at sddmm.cu:109-114.  The device copies of W,
+ * H and the result stay with the plan after its first call (counted in
+ * sddmm_plan_info.device_bytes), and with the first such call on a device 16 MiB
+ * of pinned host memory, two streams and up to seven threads, which all plans
+ * share; sddmm_plan_release_host gives the plan's arrays and its share in the
+ * rest back (the next call makes them anew), as sddmm_plan_destroy does.  Calls
+ * from several threads take turns.  The kernels of a call are an sddmm_execute of
+ * the plan: where that keeps scratch memory in the plan (k_slice < K), the two
+ * must not overlap.                                                          */
 int sddmm_gpu(const sddmm_plan *plan, const float *h_W, const float *h_H, float *h_out,
               float *kernel_ms);
+int sddmm_plan_release_host(const sddmm_plan *plan);
 
 /* Plan-free SDDMM over a CSR pattern in device memory that allocates nothing and
  * keeps nothing: no hipMalloc / hipFree, no allocating library routine, no scratch

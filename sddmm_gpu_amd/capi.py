@@ -124,6 +124,7 @@ SIGNATURES = {
     "sddmm_spmm_csr": (c_int, [c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_void_p]),
     "sddmm_plan_launch_count": (c_int, [c_void_p, POINTER(c_int32)]),
     "sddmm_execute_profiled": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, POINTER(LaunchProfile), c_int32]),
+    "sddmm_plan_release_host": (c_int, [c_void_p]),
     "sddmm_gpu": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, POINTER(c_float)]),
     "sddmm_csr_noalloc": (c_int, [c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_int32, c_void_p, c_void_p,
                                   c_void_p, c_void_p]),
@@ -389,6 +390,10 @@ class Plan:
         check(lib().sddmm_execute_profiled(self.h, c_void_p(d_val or None), c_void_p(d_W), c_void_p(d_H), c_void_p(d_out),
                                            c_void_p(stream or None), prof, n.value))
         return [{f: getattr(prof[i], f) for f, _ in LaunchProfile._fields_} for i in range(n.value)]
+
+    def release_host(self):
+        """Gives back the device arrays that gpu() keeps with the plan."""
+        check(lib().sddmm_plan_release_host(self.h))
 
     def gpu(self, W, H):
         """Host arrays in, host array out (+ kernel-only ms): the calling

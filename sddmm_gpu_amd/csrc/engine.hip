@@ -104,6 +104,7 @@ int sddmm_plan_get_info(const sddmm_plan *plan, sddmm_plan_info *info)
 {
     if (!plan || !info) return fail(SDDMM_ERR_ARG, "sddmm_plan_get_info: NULL argument");
     *info = plan->info;
+    info->device_bytes += plan->host_bytes.load();
     return SDDMM_OK;
 }
 

@@ -6,7 +6,7 @@
 // a copy kernel per piece moves the ones before over the link, on two streams so that one kernel's start hides
 // behind another's work.  27.4 MB up and 19.5 MB down: 2.20 -> 1.20 ms a call (0.83 ms of it the link).  The pieces, streams and
 // threads (HostPipe) are shared by all plans that have made such a call and go with the last of them; the device
-// arrays stay with their plan.
+// arrays stay with their plan, until it is destroyed or sddmm_plan_release_host.
 #include <hip/hip_runtime.h>
 #include <atomic>
 #include <condition_variable>
@@ -243,17 +243,20 @@ void HostCallDelete::operator()(HostCall *c) const { delete c; }
 
 namespace {
 
-int make_host_call(const sddmm_plan_info &I, std::unique_ptr<HostCall, HostCallDelete> &out)
+int make_host_call(const sddmm_plan *plan)
 {
+    const sddmm_plan_info &I = plan->info;
     std::unique_ptr<HostCall, HostCallDelete> c(new (std::nothrow) HostCall);
     if (!c) return fail(SDDMM_ERR_NOMEM, "sddmm_gpu: out of memory");
     HIP_TRY(hipGetDevice(&c->device));
     c->pipe = HostPipe::get(c->device);
     if (!c->pipe) return fail(SDDMM_ERR_HIP, "sddmm_gpu: cannot set up the host transfers: %s", hipGetErrorString(hipGetLastError()));
-    HIP_TRY(hipMalloc((void **)&c->W, (size_t)std::max<int64_t>(I.n_rows * (int64_t)I.K, 1) * 4));
-    HIP_TRY(hipMalloc((void **)&c->H, (size_t)std::max<int64_t>(I.n_cols * (int64_t)I.K, 1) * 4));
-    HIP_TRY(hipMalloc((void **)&c->out, (size_t)std::max<int64_t>(I.nnz, 1) * 4));
-    out = std::move(c);
+    const int64_t n[3] = {std::max<int64_t>(I.n_rows * (int64_t)I.K, 1), std::max<int64_t>(I.n_cols * (int64_t)I.K, 1), std::max<int64_t>(I.nnz, 1)};
+    HIP_TRY(hipMalloc((void **)&c->W, (size_t)n[0] * 4));
+    HIP_TRY(hipMalloc((void **)&c->H, (size_t)n[1] * 4));
+    HIP_TRY(hipMalloc((void **)&c->out, (size_t)n[2] * 4));
+    plan->host_call = std::move(c);
+    plan->host_bytes = 4 * (n[0] + n[1] + n[2]);
     return SDDMM_OK;
 }
 
@@ -291,7 +294,7 @@ extern "C" int sddmm_gpu(const sddmm_plan *plan, const float *h_W, const float *
     std::lock_guard<std::mutex> one(plan->host_mu);
     try {
         if (!plan->host_call)
-            if (int rc = make_host_call(plan->info, plan->host_call)) return rc;
+            if (int rc = make_host_call(plan)) return rc;
         HostCall &c = *plan->host_call;
         int device = 0;
         HIP_TRY(hipGetDevice(&device));
@@ -313,4 +316,13 @@ extern "C" int sddmm_gpu(const sddmm_plan *plan, const float *h_W, const float *
     } catch (const std::exception &e) {
         return fail(SDDMM_ERR_NOMEM, "sddmm_gpu: %s", e.what());
     }
+}
+
+extern "C" int sddmm_plan_release_host(const sddmm_plan *plan)
+{
+    if (!plan) return fail(SDDMM_ERR_ARG, "sddmm_plan_release_host: plan is NULL");
+    std::lock_guard<std::mutex> one(plan->host_mu);
+    plan->host_call.reset();
+    plan->host_bytes = 0;
+    return SDDMM_OK;
 }

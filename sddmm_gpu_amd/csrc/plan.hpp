@@ -2,6 +2,7 @@
 // and the functions that build them.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include <memory>
 #include <mutex>
 #include "internal.hpp"
@@ -69,6 +70,7 @@ struct sddmm_plan {
     sddmm_plan_options options{};  // what the plan was built with, environment overrides applied
     mutable std::mutex host_mu;    // sddmm_gpu: one call at a time, with the device arrays it keeps
     mutable std::unique_ptr<sddmm::HostCall, sddmm::HostCallDelete> host_call;
+    mutable std::atomic<int64_t> host_bytes{0};  // size of those arrays
     ~sddmm_plan()
     {
         for (const Owned &o : owned) (void)hipFree(o.p);

@@ -56,3 +56,20 @@ def test_two_threads_with_a_plan_each_and_one_plan():
     for t in th:
         t.join()
     assert not bad
+
+
+def test_what_a_call_keeps_is_counted_and_given_back():
+    plan, W, H = make(60000, 30000, 400_000, 128, 9)
+    want = expected(plan, W, H, 400_000)
+    kept = 4 * (W.size + H.size + 400_000)  # 47 MB
+    before = plan.info()["device_bytes"]
+    for _ in range(2):
+        assert np.array_equal(plan.gpu(W, H)[0], want)
+        assert plan.info()["device_bytes"] == before + kept
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        plan.release_host()
+        assert plan.info()["device_bytes"] == before
+        assert torch.cuda.mem_get_info()[0] >= free + kept // 2
+    plan.release_host()  # nothing to give back
+    plan.close()
