@@ -15,10 +15,11 @@
  * last failure on the calling thread.  "host" / "device" say where a pointer
  * must live.  Plans are immutable after creation: sddmm_execute may be called
  * from several threads on the same plan (each call on its own stream) -- with
- * one exception: a plan that works in K slices (sddmm_plan_info.k_slice < K,
- * i.e. K > 128) keeps the partial results between its slices in a buffer of
- * its own, so executes of such a plan must not overlap in time -- unless they
- * are made through sddmm_execute_ws, which takes that memory from the caller.
+ * one exception: a plan that works in K slices (sddmm_plan_info.k_slice < K:
+ * most plans of K > 128, and those made with a k_slice below K) keeps the
+ * partial results between its slices in a buffer of its own, so executes of
+ * such a plan must not overlap in time -- unless they are made through
+ * sddmm_execute_ws, which takes that memory from the caller.
  */
 #ifndef SDDMM_H
 #define SDDMM_H
@@ -407,8 +408,9 @@ int sddmm_execute_ws(const sddmm_plan *plan, const float *d_val, const float *d_
  * above) and where a few workgroups would hold most of the work, the whole product
  * goes over the CSR pattern as sddmm_spmm_csr does it, with the parts of its cut rows
  * written down and added up in order.  No atomics: the same bits on every call.  The
- * partial rows (K floats per run; sddmm_plan_info.spmm_runs) live in the plan, or
- * in d_workspace (NULL, or as for sddmm_execute_ws).  Other plans (and H or Y not
+ * partial rows (K floats per run; sddmm_plan_info.spmm_runs) live in the plan, so
+ * calls on one plan must not overlap in time, or in d_workspace (NULL, or as for
+ * sddmm_execute_ws): calls with a workspace each may.  Other plans (and H or Y not
  * 16-byte aligned) take the sddmm_spmm_csr path on the plan's pattern.  d_x: nnz
  * fp32 in sorted order, e.g. the output of sddmm_execute_softmax.            */
 int sddmm_execute_softmax(const sddmm_plan *plan, const float *d_val, const float *d_W, const float *d_H,

@@ -375,6 +375,42 @@ def check_plan_spmm(oracle, d, K, opts, form, sddmm=True):
     return info
 
 
+@pytest.mark.parametrize("K,form", [(50, WALK), (205, WALK), (128, TILES)])
+def test_plan_calls_overlap_with_workspaces_of_their_own(K, form):
+    """The product and the SDDMM of one plan on two streams at a time, a workspace for each call: a rank in one launch and
+    one in slices without a tile width of its own, and column tiles."""
+    d = wide(13000, 1100, K, True)
+    dev = torch.device(DEV)
+    S = capi.Coo.from_arrays(d["n_rows"], d["n_cols"], d["row_ind"].numpy(), d["col_ind"].numpy(), d["val"].numpy())
+    plan = S.plan(K, options=capi.PlanOptions.defaults(ignore_env=1, spmm_stream=1, split_min_nnz=0, stage_factor=0, short_row_max=16))
+    assert plan.spmm_form() == form and plan.info()["k_slice"] == min(K, 128)
+    g = torch.Generator().manual_seed(K)
+    xs = [torch.randn(d["nnz"], generator=g).to(dev) for _ in range(2)]
+    Hs = [torch.randn(d["n_cols"], K, generator=g).to(dev) for _ in range(2)]
+    W = d["W"].to(dev)
+    nbytes = plan.workspace_bytes()
+    ws = [torch.full((nbytes // 4,), float("nan"), device=dev) for _ in range(2)]
+    Y = [torch.empty(d["n_rows"], K, device=dev) for _ in range(2)]
+    out = [torch.empty(d["nnz"], device=dev) for _ in range(2)]
+    want = []
+    for i in range(2):  # one after the other, with the plan's own memory
+        plan.spmm(xs[i].data_ptr(), Hs[i].data_ptr(), Y[i].data_ptr())
+        plan.execute(0, W.data_ptr(), Hs[i].data_ptr(), out[i].data_ptr())
+        torch.cuda.synchronize()
+        want.append((Y[i].clone(), out[i].clone()))
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for t in Y + out:
+        t.fill_(float("nan"))
+    torch.cuda.synchronize()
+    for _ in range(10):
+        for i, st in enumerate(streams):
+            plan.execute_ws(0, W.data_ptr(), Hs[i].data_ptr(), out[i].data_ptr(), ws[i].data_ptr(), nbytes, capi.EPILOGUE_SCALE, st.cuda_stream)
+            plan.spmm(xs[i].data_ptr(), Hs[i].data_ptr(), Y[i].data_ptr(), ws[i].data_ptr(), nbytes, st.cuda_stream)
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert torch.equal(Y[i], want[i][0]) and torch.equal(out[i], want[i][1])
+
+
 def test_plan_spmm_without_a_tile_stream_takes_the_csr_path(oracle):
     K = 64
     d = synth.make(3, 0.02, K=K)
