@@ -48,12 +48,16 @@ enum {
     SDDMM_KERNEL_AUTO = 0,
     SDDMM_KERNEL_ROW_GATHER = 1, /* W row in VGPRs, H rows gathered from L2/HBM (as a plan: the unpadded gather kernel;
                                     as the short-row launch of a HYBRID plan: the padded, pipelined gather, over
-                                    column slabs when H is far larger than the caches) */
+                                    column slabs when H is larger than the caches) */
     SDDMM_KERNEL_LDS_TILE = 2,   /* column tiles of H staged in LDS, W row (re)loaded per row run */
     SDDMM_KERNEL_PANEL = 3,      /* row panels of W resident in VGPRs, column tiles of H swept through LDS */
     SDDMM_KERNEL_HYBRID = 4,     /* what AUTO builds: (from K = 384 on, or when asked) the dense core as a DENSE_BLOCK
-                                    launch, the rest split by row length: rows with at least 2 nonzeros per column
-                                    tile -> LDS_TILE (padded tile kernel), shorter rows -> ROW_GATHER; a class too
+                                    launch; of the rest the rows with at least 2 nonzeros per column tile to an
+                                    LDS_TILE launch (padded tile kernel) and shorter ones to a ROW_GATHER launch, or
+                                    all rows to either, whichever a model of the two finds cheapest -- ROW_GATHER over
+                                    column slabs where that is.  The split is by length alone beside a dense core, when
+                                    the caller sets short_row_max, stage_factor or split_min_nnz, and with spmm_stream
+                                    from 4 million nonzeros on (at ranks with an exact tile width); then a class too
                                     small to pay for its launch joins the other.  Never a PANEL launch. */
     SDDMM_KERNEL_DENSE_BLOCK = 5 /* blocks of 128 heavy rows x 128 popular columns computed whole on the matrix cores,
                                     their nonzeros picked from the result; never a plan of its own, only a launch of a

@@ -1,5 +1,5 @@
-// Unpadded LDS-tile kernel of the SDDMM engine for gfx950 (MI355X): explicit LDS_TILE plans at ranks that
-// the padded tile kernel has no variant for.
+// Unpadded LDS-tile kernel of the SDDMM engine for gfx950 (MI355X): explicit LDS_TILE plans with
+// unpadded_tile = 1, and at K = 4, for which the padded tile kernel has no form.
 //
 // The stream of nonzeros is S in tile order (column tile by column tile, rows ascending inside a tile),
 // reached through the permutation the tiling pass produced, and walked in batches of 64 (one per lane of a
