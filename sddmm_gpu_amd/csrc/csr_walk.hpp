@@ -65,7 +65,7 @@ __device__ __forceinline__ int rows_of_range(const int32_t *__restrict__ row_ptr
         if (rel <= end && (rel != next || lane == 63)) tab[rel] = r;
         last = __builtin_amdgcn_readlane(rel, 63);
     }
-    if (last < end) {  // (so base <= n_rows)
+    if (__builtin_expect(last < end, 0)) {  // (so base <= n_rows)
         const int r1 = wave_find_row(row_ptr, base - 1, n_rows, p0 + end - 1, lane);
         constexpr int U = 4;  // searches of a lane at a time
         for (int i0 = last & ~63; i0 < end; i0 += 64 * U) {
@@ -89,7 +89,7 @@ __device__ __forceinline__ int rows_of_range(const int32_t *__restrict__ row_ptr
         }
         if (lane == 0 && row_ptr[r1 + 1] == p0 + end) tab[end] = r1 + 1;
     }
-    if (lane == 0 && nnz - p0 <= n) tab[nnz - p0] = n_rows;
+    if (__builtin_expect(nnz - p0 <= n, 0) && lane == 0) tab[nnz - p0] = n_rows;
     __builtin_amdgcn_wave_barrier();  // (LDS operations of one wave complete in order)
     int carry = 0;
     for (int i = 0; i < n_pad; i += 64) {

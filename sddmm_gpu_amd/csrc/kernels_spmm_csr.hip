@@ -53,8 +53,9 @@ void sddmm_spmm_zero_rows_kernel(const int32_t *__restrict__ row_ptr, float *Y, 
 
 // The rows that the product with records leaves: empty rows become 0, rows cut between workgroups (of 2^shift
 // nonzeros) the sum of their records, workgroup by workgroup.  A wave looks at 64 rows, at fewer where that would leave
-// less than 2048 waves: where rows are longer than a workgroup's share all of them are cut, and a few waves taking 64 each,
-// piece after piece, are slower than the product itself.
+// less than 1024 waves, though not at fewer than fill its lanes with pieces: where rows are longer than a workgroup's share
+// all of them are cut, and a few waves taking 64 each, piece after piece, are slower than the product itself.  us for both
+// kernels with 64 rows a wave and with this: 2220 rows, K = 128 49 and 28, 1800 rows, K = 32 23 and 18.
 __global__ __launch_bounds__(256)
 void sddmm_spmm_cut_rows_kernel(const int32_t *__restrict__ row_ptr, const float *__restrict__ part, float *Y, int64_t n_rows, int K, int shift,
                                 int rows_per_wave)
@@ -331,7 +332,7 @@ int launch_spmm_csr_records(int64_t n_rows, int64_t nnz, const int32_t *d_row_pt
     hipStream_t st = (hipStream_t)stream;
     if (int rc = checked(launch_csr<true>(c, n_rows, nnz, d_row_ptr, d_col_ind, d_x, K, d_H, d_Y, d_part, st))) return rc;
     int per_wave = 64;
-    while (per_wave > 1 && n_rows < (int64_t)2048 * per_wave) per_wave /= 2;
+    while (per_wave > 1 && n_rows < (int64_t)1024 * per_wave && per_wave / 2 * ((K + 3) / 4) >= 64) per_wave /= 2;
     return checked(launch(sddmm_spmm_cut_rows_kernel, dim3((unsigned)((n_rows + 4 * per_wave - 1) / (4 * per_wave))), dim3(256), 0, st, d_row_ptr,
                           d_part, d_Y, n_rows, (int)K, c.wg_shift, per_wave));
 }

@@ -153,11 +153,12 @@ void assign_workspace(sddmm_plan *P);
 int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_ptr_all, const int32_t *col_ind_all,
               const float *vals, const int32_t *d_row_ptr_borrowed, const int32_t *d_col_borrowed, int32_t K,
               const sddmm_plan_options &opt_in, sddmm_plan **out);
-// Is the product with the dense factor, behind a plan of a matrix of this size, a walk over the CSR pattern whatever the
-// runs (see add_tile)?  From 4 million nonzeros on the rows are split by length, and tiles that hold long rows only are
-// the faster ones; so they are when the walk, at 17 TB/s, has more than 1.8 GB of H rows to read (ratings of 2.4 and
-// 3.6 M, K = 256: 123 against 139 and 167 against 190 us; 1.5 M 101 against 83).
-inline bool product_walks(int64_t nnz, int32_t K) { return nnz < 4000000 && nnz * K < 450000000; }
+// Is the product with the dense factor, behind a plan of a matrix of this size (tile slices of ks elements), a walk over
+// the CSR pattern whatever the runs (see add_tile)?  From 4 million nonzeros on the rows are split by length, and tiles that
+// hold long rows only are the faster ones; so they are when the walk, at 17 TB/s, has more than 1.8 GB of H rows to read,
+// 2.8 where the tiles take slices of 64 (tiles against walk, ratings of 1.8, 2.4 and 3.6 M, K = 256: 108 / 101, 123 / 139 and
+// 167 / 190 us; of 2.6 and 3.8 M, K = 192: 148 / 131 and 180 / 184; K = 320, 1.8 and 2.6 M: 231 / 171 and 240 / 259).
+inline bool product_walks(int64_t nnz, int32_t K, int ks) { return nnz < 4000000 && nnz * K < (ks < 128 ? 700000000 : 450000000); }
 // planner_tile.hip: the rows' nonzeros in tile order (tiles of x columns), every (row, tile) run padded
 // ks: K elements per launch, a divisor of K or (ragged ranks) the width K is rounded up to
 int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t panel_rows, int want_g, int ks,

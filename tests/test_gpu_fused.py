@@ -298,8 +298,8 @@ def test_plan_spmm_tiles_at_every_slice_width(oracle, n_cols, per_row, K, short)
 
 
 # On either side of each line between the forms: a matrix whose H is near a die's L2 in size below and above 1.8 GB of
-# gathered H rows; bands whose tiles are uneven, at a short and a long row of H.
-@pytest.mark.parametrize("kind,n_rows,K,form", [("near", 3400, 256, WALK), ("near", 3600, 256, TILES), ("band", 36000, 64, WALK), ("band", 36000, 256, TILES)])
+# gathered H rows (2.8 where the tiles take slices of 64); bands whose tiles are uneven, at a short and a long row of H.
+@pytest.mark.parametrize("kind,n_rows,K,form", [("near", 3400, 256, WALK), ("near", 3600, 256, TILES), ("near", 5000, 192, WALK), ("band", 36000, 64, WALK), ("band", 36000, 256, TILES)])
 def test_plan_spmm_form_by_size_and_evenness(oracle, kind, n_rows, K, form):
     from test_gpu_parity import _dict_of
     rng = np.random.default_rng(n_rows)
