@@ -46,7 +46,7 @@ __device__ __forceinline__ int wave_max_scan(int v)
 // ones) the last counts.  Every read waits for the one before (0.34 us each), so the walk ends at the last
 // nonzero, and after as many steps as the search takes it is given up for that: each lane looks for the rows of its
 // own nonzeros among those left.  (20 thousand nonzeros, K = 16, us without / with both: 4 million empty rows behind
-// them 20700 / 8, spread over 4 million rows 59 / 14.)
+// them 20700 / 8, spread over 4 million rows 59 / 15.)
 __device__ __forceinline__ int rows_of_range(const int32_t *__restrict__ row_ptr, int n_rows, int nnz, int p0, int n, int *tab, int lane)
 {
     const int n_pad = (n + 63) & ~63;
@@ -65,7 +65,7 @@ __device__ __forceinline__ int rows_of_range(const int32_t *__restrict__ row_ptr
         if (rel <= end && (rel != next || lane == 63)) tab[rel] = r;
         last = __builtin_amdgcn_readlane(rel, 63);
     }
-    if (__builtin_expect(last < end, 0)) {  // (so base <= n_rows)
+    if (__builtin_expect(last < end, 0)) {
         const int r1 = wave_find_row(row_ptr, base - 1, n_rows, p0 + end - 1, lane);
         constexpr int U = 4;  // searches of a lane at a time
         for (int i0 = last & ~63; i0 < end; i0 += 64 * U) {
@@ -87,7 +87,7 @@ __device__ __forceinline__ int rows_of_range(const int32_t *__restrict__ row_ptr
                 if (i >= last && i < end) tab[i] = lo[u];
             }
         }
-        if (lane == 0 && row_ptr[r1 + 1] == p0 + end) tab[end] = r1 + 1;
+        if (lane == 0 && r1 < n_rows && row_ptr[r1 + 1] == p0 + end) tab[end] = r1 + 1;
     }
     if (__builtin_expect(nnz - p0 <= n, 0) && lane == 0) tab[nnz - p0] = n_rows;
     __builtin_amdgcn_wave_barrier();  // (LDS operations of one wave complete in order)
