@@ -60,8 +60,10 @@ enum {
                                     from 4 million nonzeros on (at ranks with an exact tile width); then a class too
                                     small to pay for its launch joins the other.  Never a PANEL launch. */
     SDDMM_KERNEL_DENSE_BLOCK = 5 /* blocks of 128 heavy rows x 128 popular columns computed whole on the matrix cores,
-                                    their nonzeros picked from the result; never a plan of its own, only a launch of a
-                                    HYBRID plan (reported by sddmm_execute_profiled) */
+                                    their nonzeros picked from the result; or, where neighbouring rows have mostly the
+                                    same columns (local attention; K = 32, 48, ... 128), all of S as 32 x 32 tiles; never
+                                    a plan of its own, only a launch of a HYBRID plan (reported by
+                                    sddmm_execute_profiled) */
 };
 
 typedef struct sddmm_coo sddmm_coo;   /* host-side sparse matrix (COO, int32/int32/fp32) */
@@ -90,7 +92,7 @@ typedef struct sddmm_plan_info {
     int64_t short_batches;    /* batches of 64 of those positions that run in half the steps */
     double plan_ms;       /* host time spent in the tiling pass + upload (a loaded plan: in reading the file) */
     int64_t dense_nnz;    /* nonzeros handled by the DENSE_BLOCK launch */
-    int64_t dense_blocks; /* its 128 x 128 blocks */
+    int64_t dense_blocks; /* its 128 x 128 blocks, or 32 x 32 tiles */
     int64_t matrix_nnz;   /* nonzeros of the LDS_TILE launch computed by its matrix-core waves (counted in class_nnz[0]) */
     int64_t matrix_rows;  /* the rows they belong to */
     int64_t spmm_runs;    /* (row, tile) runs of the product's tile stream (or cut rows' parts), one partial row of Y each (0: not built) */
@@ -262,7 +264,8 @@ typedef struct sddmm_plan_options {
     int32_t row_padded;         /* 0/1 ROW_GATHER plans use the padded gather kernel [SDDMM_ROW_PADDED]    */
     int32_t unpadded_tile;      /* 0/1 LDS_TILE plans use the unpadded stream kernel [SDDMM_UNPADDED_TILE] */
     int32_t dense_blocks;       /* 0/1 dense core on the matrix cores, in bf16 parts that add up to the
-                                   fp32 operands (-1: by K; 0: every product in fp32)  [SDDMM_DENSE]      */
+                                   fp32 operands (-1: by K, and all of a locally dense pattern; 0: every product
+                                   in fp32)                                         [SDDMM_DENSE]      */
     int32_t dense_permille;     /* least fill of a dense block, in 1/1000           [SDDMM_DENSE_PERMILLE] */
     int32_t dense_rb_group;     /* row blocks swept together by one die             [SDDMM_DENSE_RB_GROUP] */
     int32_t fuse_slices;        /* 0/1 the K slices of a launch run inside one kernel
@@ -389,7 +392,8 @@ int sddmm_execute_ws(const sddmm_plan *plan, const float *d_val, const float *d_
  * taken into registers whole -- by a lane, a group of lanes, a wave or a
  * workgroup, by its length -- so it is read once and written once; a longer row
  * is cut into pieces of up to 4096 entries whose (max, sum) records are merged by a
- * last kernel.  The layout of the work and those records are kept in fixed
+ * last kernel.  A plan on row blocks (SDDMM_KERNEL_DENSE_BLOCK on a locally dense
+ * pattern) normalises the rows in the launch that computes them.  The layout of the work and those records are kept in fixed
  * device arrays of the library (18 MiB per GPU), so softmax calls that overlap
  * in time on one GPU (different streams or threads) race unless they bring a
  * workspace (sddmm_execute_ws); calls on one stream never do.
@@ -411,7 +415,8 @@ int sddmm_execute_ws(const sddmm_plan *plan, const float *d_val, const float *d_
  * width of their own, on small matrices (fewer than 4 M nonzeros and 4.5e8 or 7e8
  * nonzeros times K, H as above) and where a few workgroups would hold most of the work, the whole product
  * goes over the CSR pattern as sddmm_spmm_csr does it, with the parts of its cut rows
- * written down and added up in order.  No atomics: the same bits on every call.  The
+ * written down and added up in order; and a plan on row blocks multiplies its tiles
+ * on the matrix cores.  No atomics: the same bits on every call.  The
  * partial rows (K floats per run; sddmm_plan_info.spmm_runs) live in the plan, so
  * calls on one plan must not overlap in time, or in d_workspace (NULL, or as for
  * sddmm_execute_ws): calls with a workspace each may.  Other plans (and H or Y not
@@ -421,11 +426,12 @@ int sddmm_execute_softmax(const sddmm_plan *plan, const float *d_val, const floa
                           float *d_out, void *stream);
 int sddmm_plan_spmm(const sddmm_plan *plan, const float *d_x, const float *d_H, float *d_Y, void *d_workspace,
                     int64_t workspace_bytes, void *stream);
-/* Which of them sddmm_plan_spmm takes for this plan: SDDMM_SPMM_CSR (as sddmm_spmm_csr), _TILES or _WALK (over the
- * pattern, with the parts of cut rows kept). */
+/* Which of them sddmm_plan_spmm takes for this plan: SDDMM_SPMM_CSR (as sddmm_spmm_csr), _TILES, _WALK (over the
+ * pattern, with the parts of cut rows kept) or _BLOCKS (on the row blocks of a locally dense pattern). */
 #define SDDMM_SPMM_CSR 0
 #define SDDMM_SPMM_TILES 1
 #define SDDMM_SPMM_WALK 2
+#define SDDMM_SPMM_BLOCKS 3
 int sddmm_plan_spmm_form(const sddmm_plan *plan, int32_t *form);
 int sddmm_row_softmax(int64_t n_rows, const int32_t *d_row_ptr, const float *d_x, float *d_out, void *stream);
 int sddmm_spmm_csr(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *d_row_ptr,

@@ -19,7 +19,7 @@ OK, ERR_ARG, ERR_IO, ERR_FORMAT, ERR_RANGE, ERR_UNSORTED, ERR_HIP, ERR_NOMEM = r
 KERNEL_AUTO, KERNEL_ROW_GATHER, KERNEL_LDS_TILE, KERNEL_PANEL, KERNEL_HYBRID, KERNEL_DENSE_BLOCK = 0, 1, 2, 3, 4, 5
 EPILOGUE_SCALE, EPILOGUE_RESIDUAL = 0, 1
 FORM_SOFTMAX = 0x100
-SPMM_CSR, SPMM_TILES, SPMM_WALK = 0, 1, 2
+SPMM_CSR, SPMM_TILES, SPMM_WALK, SPMM_BLOCKS = 0, 1, 2, 3
 
 
 class SddmmError(RuntimeError):

@@ -121,9 +121,9 @@ static int check_execute_args(const sddmm_plan *plan, const float *d_W, const fl
 }
 
 // Issues the kernels of one launch-list entry (one per K slice) on `stream`.
-// ws: the caller's workspace (null: the plan's own scratch memory)
+// ws: the caller's workspace (null: the plan's own scratch memory); softmax: of the rows as well (see softmax_in_launch)
 static hipError_t issue_launch(const sddmm_plan *plan, const Launch &L, const float *d_val, const float *d_W,
-                         const float *d_H, float *d_out, hipStream_t stream, int epilogue = SDDMM_EPILOGUE_SCALE, char *ws = nullptr)
+                         const float *d_H, float *d_out, hipStream_t stream, int epilogue = SDDMM_EPILOGUE_SCALE, char *ws = nullptr, bool softmax = false)
 {
     const int residual = epilogue == SDDMM_EPILOGUE_RESIDUAL;
     const sddmm_plan_info &I = plan->info;
@@ -146,6 +146,14 @@ static hipError_t issue_launch(const sddmm_plan *plan, const Launch &L, const fl
         da.W = d_W; da.H = d_H; da.out = d_out;
         da.residual = residual;
         return launch(L.dfn, dim3((unsigned)L.grid), dim3((unsigned)L.block), 0, stream, da);
+    } else if (L.bfns[0]) {
+        BlockArgs ba = L.ba;
+        ba.val = val; ba.W = d_W; ba.H = d_H; ba.out = d_out;
+        ba.residual = residual;
+        if (!softmax) return launch(L.bfns[0], dim3((unsigned)L.grid), dim3((unsigned)L.block), std::min<size_t>((size_t)L.lds, (size_t)kRoundTiles * kBlockTileBytes), stream, ba);
+        if (ws && ba.long_records) ba.long_records = reinterpret_cast<float2 *>(ws + L.ws_part);
+        if (hipError_t e = launch(L.bfns[1], dim3((unsigned)L.grid), dim3((unsigned)(64 * L.softmax_waves)), (size_t)L.lds, stream, ba)) return e;
+        return launch_block_long_rows(ba, plan->d_row_ptr, stream);
     } else if (L.tfn) {
         TileArgs ta = L.ta;
         ta.val = val;
@@ -188,6 +196,13 @@ static hipError_t issue_launch(const sddmm_plan *plan, const Launch &L, const fl
     }
 }
 
+// Row blocks take the softmax along, without a pass over out.  (Rows whose blocks are several units get a pass of their own, a
+// workgroup per 16,384 entries: where they are many the general pass is the faster one.)
+static bool softmax_in_launch(const sddmm_plan *plan)
+{
+    return plan->launches.size() == 1 && plan->launches[0].bfns[1] && plan->launches[0].ba.n_long_pieces <= 1024;
+}
+
 int sddmm_execute(const sddmm_plan *plan, const float *d_val, const float *d_W, const float *d_H, float *d_out,
                   void *stream)
 {
@@ -213,8 +228,12 @@ int sddmm_execute_epilogue(const sddmm_plan *plan, const float *d_val, const flo
 int sddmm_execute_softmax(const sddmm_plan *plan, const float *d_val, const float *d_W, const float *d_H, float *d_out,
                           void *stream)
 {
-    if (int rc = sddmm_execute(plan, d_val, d_W, d_H, d_out, stream)) return rc;
+    if (int rc = check_execute_args(plan, d_W, d_H, d_out, "sddmm_execute_softmax")) return rc;
     if (plan->info.nnz == 0) return SDDMM_OK;
+    const bool in_launch = softmax_in_launch(plan);
+    for (const Launch &L : plan->launches)
+        HIP_TRY(issue_launch(plan, L, d_val, d_W, d_H, d_out, (hipStream_t)stream, SDDMM_EPILOGUE_SCALE, nullptr, in_launch));
+    if (in_launch) return SDDMM_OK;
     if (!plan->d_row_ptr) return fail(SDDMM_ERR_ARG, "sddmm_execute_softmax: the plan holds no row pointers");
     return launch_row_softmax(plan->info.n_rows, plan->d_row_ptr, d_out, d_out, stream, nullptr, 0);
 }
@@ -242,8 +261,9 @@ int sddmm_execute_ws(const sddmm_plan *plan, const float *d_val, const float *d_
                     (long long)plan->ws_bytes);
     if ((uintptr_t)d_workspace & 255u) return fail(SDDMM_ERR_ARG, "sddmm_execute_ws: the workspace must be 256-byte aligned");
     char *ws = static_cast<char *>(d_workspace);
-    for (const Launch &L : plan->launches) HIP_TRY(issue_launch(plan, L, d_val, d_W, d_H, d_out, (hipStream_t)stream, epilogue, ws));
-    if (!softmax) return SDDMM_OK;
+    const bool in_launch = softmax && softmax_in_launch(plan);
+    for (const Launch &L : plan->launches) HIP_TRY(issue_launch(plan, L, d_val, d_W, d_H, d_out, (hipStream_t)stream, epilogue, ws, in_launch));
+    if (!softmax || in_launch) return SDDMM_OK;
     if (!plan->d_row_ptr) return fail(SDDMM_ERR_ARG, "sddmm_execute_ws: the plan holds no row pointers");
     return launch_row_softmax(plan->info.n_rows, plan->d_row_ptr, d_out, d_out, stream, ws + plan->ws_softmax, plan->info.nnz);
 }
@@ -260,7 +280,7 @@ int sddmm_plan_spmm_form(const sddmm_plan *plan, int32_t *form)
 {
     if (!plan || !form) return fail(SDDMM_ERR_ARG, "sddmm_plan_spmm_form: NULL argument");
     const Launch *L = spmm_launch(plan);
-    *form = !L ? SDDMM_SPMM_CSR : L->sp_on == 1 ? SDDMM_SPMM_TILES : SDDMM_SPMM_WALK;
+    *form = !L ? SDDMM_SPMM_CSR : L->sp_on == 1 ? SDDMM_SPMM_TILES : L->sp_on == 2 ? SDDMM_SPMM_WALK : SDDMM_SPMM_BLOCKS;
     return SDDMM_OK;
 }
 
@@ -284,6 +304,13 @@ int sddmm_plan_spmm(const sddmm_plan *plan, const float *d_x, const float *d_H, 
     if (Ls->sp_on == 2)
         return launch_spmm_csr_records(I.n_rows, I.nnz, plan->d_row_ptr, plan->d_col, d_x, I.K, d_H, d_Y,
                                        d_workspace ? reinterpret_cast<float *>(static_cast<char *>(d_workspace) + Ls->ws_sp_part) : Ls->sa.part, stream);
+    if (Ls->sp_on == 3) {
+        BlockArgs ba = Ls->ba;
+        ba.x = d_x; ba.H = d_H; ba.Y = d_Y;
+        if (d_workspace) ba.part = reinterpret_cast<float *>(static_cast<char *>(d_workspace) + Ls->ws_sp_part);
+        HIP_TRY(launch_block_spmm(ba, Ls->fn_nwaves, stream));
+        return SDDMM_OK;
+    }
     SpmmArgs sa = Ls->sa;
     sa.x = d_x; sa.H = d_H; sa.Y = d_Y;
     sa.row_ptr = plan->d_row_ptr; sa.col_ind = plan->d_col;
@@ -351,7 +378,7 @@ int sddmm_execute_profiled(const sddmm_plan *plan, const float *d_val, const flo
         float ms = 0.f;
         HIP_TRY(hipEventElapsedTime(&ms, ev[i], ev[i + 1]));
         prof[i].kernel = L.kind;
-        prof[i].lanes_per_nnz = L.dfn ? 0 : L.kind == SDDMM_KERNEL_PANEL ? 8 : (L.tfn ? L.tile_g : L.gather_g);
+        prof[i].lanes_per_nnz = L.dfn || L.bfns[0] ? 0 : L.kind == SDDMM_KERNEL_PANEL ? 8 : (L.tfn ? L.tile_g : L.gather_g);
         prof[i].k_slice = L.k_slice;
         prof[i].n_kernel_launches = (L.k_slice > 0 && L.k_slice < plan->info.K && !L.fused_slices) ? (plan->info.K + L.k_slice - 1) / L.k_slice : 1;
         prof[i].nnz = L.nnz;

@@ -5,6 +5,7 @@
 #include <mutex>
 #include "internal.hpp"
 #include "launch.hpp"
+#include "softmax_exp.hpp"
 
 using namespace sddmm;
 
@@ -109,18 +110,6 @@ void sddmm_row_softmax_rows_kernel(const int32_t *__restrict__ row_ptr, int64_t 
         }
         g_softmax_rows[c] = lay;
     }
-}
-
-// exp(x) for x <= 0 in six instructions: 2^t with t = x log2(e) rounded, times 1 + (what the rounding of t
-// and of log2(e) left out) ln 2.  About one ulp; the library routine costs four times as much, and these
-// passes would be bound by it.
-__device__ __forceinline__ float exp_nonpositive(float x)
-{
-    const float l2e = 1.44269502e+0f, l2e_lo = 1.92596299e-8f;
-    const float t = x * l2e;
-    const float r = fmaf(x, l2e_lo, fmaf(x, l2e, -t));
-    const float e = __builtin_amdgcn_exp2f(t);
-    return fmaf(e, r * 0.693147182f, e);
 }
 
 template <int GW>

@@ -2,6 +2,7 @@
 // and the kernel translation units.
 #pragma once
 #include <cstdint>
+#include <hip/hip_runtime_api.h>
 #include <hip/hip_vector_types.h>
 
 namespace sddmm {
@@ -201,6 +202,41 @@ struct DenseArgs {
 };
 using DenseFn = void (*)(const DenseArgs);
 DenseFn dense_kernel();
+
+// Row-block kernels (kernels_block.hip): blocks of kBlockRows rows that have mostly the same columns, computed whole on the
+// matrix cores, the SDDMM and the product with the dense factor.
+constexpr int kBlockRows = 32;
+constexpr int kBlockTiles = 32;  // tiles of a unit at most that is a whole row block: their scores stay in LDS for the softmax
+constexpr int kBlockTilesFew = 16;  // ... with workgroups of four waves and the softmax: more tiles' scores fill the LDS for one workgroup of eight
+constexpr int kRoundTiles = 16;  // tiles whose dot products are in LDS at a time without a softmax
+constexpr int kLongPiece = 16384;
+constexpr int kBlockTileBytes = kBlockRows * (kBlockRows * 4 + 8);  // of LDS per tile
+struct BlockArgs {
+    const int4 *units;        // [n_units] row block, first tile, behind the last tile, record of the unit (-1: it is the whole row block)
+    const int32_t *rows;      // [n_blocks][32] the blocks' rows (a short block repeats its last row, with empty masks)
+    const int32_t *cols;      // [n_tiles][32] the tiles' columns, ascending (a short tile repeats its last one, with no bit set)
+    const uint2 *info;        // [n_tiles][32] per row: which of the tile's columns it has; sorted position of the first one
+    // the rows of blocks that are several units, in pieces of kLongPiece entries: row, its first piece, its pieces, the number
+    // of this one among them; records of the pieces for the softmax (null where every row is one piece)
+    const int4 *long_pieces;
+    float2 *long_records;
+    const int4 *sums;         // [n_sums] blocks that are several units: row block, first record, records
+    const int32_t *empty_rows;  // [n_empty] rows without nonzeros
+    const float *val;         // [nnz] or null (no scaling)
+    const float *W, *H;
+    float *out;
+    const float *x;           // the product: [nnz]
+    float *part;              // ... its records, 1024 ceil(K / 32) floats each
+    float *Y;
+    int32_t n_units, n_long_pieces, n_sums, n_empty;
+    int32_t K, nnz, residual;
+};
+using BlockFn = void (*)(const BlockArgs);
+bool block_supported(int K);
+BlockFn block_kernel(int K, bool softmax, int nwaves);  // nwaves: waves per workgroup, 4 or 8
+hipError_t block_spmm_set_lds(int K, int nwaves);
+hipError_t launch_block_long_rows(const BlockArgs &a, const int32_t *row_ptr, void *stream);  // the softmax of a.long_pieces, in place in a.out
+hipError_t launch_block_spmm(const BlockArgs &a, int nwaves, void *stream);
 
 // lanes per nonzero and float4 slots per lane for a given K; G == 0: none
 Variant pick_gather_variant(int K);  // row gather, any K from 4 to 2048

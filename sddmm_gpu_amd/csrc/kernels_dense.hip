@@ -47,17 +47,11 @@
 #include <hip/hip_runtime.h>
 #include <type_traits>
 #include "kernels.hpp"
+#include "bf16_parts.hpp"
 
 using namespace sddmm;
 
 namespace {
-
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float vec4f __attribute__((ext_vector_type(4)));  // (a plain vector type: stays in registers)
-typedef float vec2f __attribute__((ext_vector_type(2)));
-typedef uint32_t vec4u __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kT = kDenseTile;           // 128 rows and 128 columns per block
 constexpr int kKC = 32;                  // K elements per chunk
@@ -66,27 +60,6 @@ constexpr int kRowB = 3 * kPartB + 16;   // bytes per staged row: 13 times 16, o
 constexpr int kStageB = kT * kRowB;      // bytes per staged operand
 constexpr int kCRowF = kT + 8;           // floats per row of the result block in LDS
 constexpr int kLdsB = 2 * kStageB > kT * kCRowF * 4 ? 2 * kStageB : kT * kCRowF * 4;
-
-// Eight floats as three bf16 parts each: part 0 is x rounded to 8 significant bits, part 1 what is
-// left rounded to 8, part 2 the rest, so x = p0 + p1 + p2 exactly.  `lost` collects the bits below
-// part 2, which are nonzero only where x is so small that they lie under bf16's smallest subnormal.
-// An infinity or a NaN leaves a NaN in part 1, a value that rounds beyond the range an infinity.
-__device__ __forceinline__ void split8(const vec4f lo4, const vec4f hi4, vec4u (&part)[3], uint32_t &lost)
-{
-    const float x[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        vec2f v = {x[2 * e], x[2 * e + 1]};
-#pragma unroll
-        for (int p = 0; p < 3; ++p) {
-            if (p == 2) lost |= __float_as_uint(v.x) | __float_as_uint(v.y);
-            const uint32_t b = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
-            part[p][e] = b;
-            v.x -= __uint_as_float(b << 16);
-            v.y -= __uint_as_float(b & 0xffff0000u);
-        }
-    }
-}
 
 // Workgroup barrier that orders LDS traffic only.  __syncthreads() also waits for every global
 // load and store in flight (its workgroup-scope fence), which would drain the requests this kernel
@@ -137,7 +110,7 @@ void sddmm_dense_kernel(const DenseArgs a)
         for (int i = 0; i < 4; ++i) gb[i] = H4[hofs[i >> 1] + 4 * (i & 1)];
     };
     uint32_t lost = 0;  // of the operands staged by this thread for the block in hand
-    vec4u pa[2][3], pb[2][3];
+    vec4w pa[2][3], pb[2][3];
     auto split_part = [&](int k) {  // a quarter of it
         const int i = k >> 1;
         if (k & 1) split8(gb[2 * i], gb[2 * i + 1], pb[i], lost);
@@ -153,8 +126,8 @@ void sddmm_dense_kernel(const DenseArgs a)
 #pragma unroll
             for (int p = 0; p < 3; ++p) {
                 unsigned char *at = lds + (r0 + 64 * i) * kRowB + p * kPartB + 16 * q;
-                *reinterpret_cast<vec4u *>(at) = pa[i][p];
-                *reinterpret_cast<vec4u *>(at + kStageB) = pb[i][p];
+                *reinterpret_cast<vec4w *>(at) = pa[i][p];
+                *reinterpret_cast<vec4w *>(at + kStageB) = pb[i][p];
             }
     };
     // One round of the block's nonzero list: 8 entries per thread, strided by the workgroup.

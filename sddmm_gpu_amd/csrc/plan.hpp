@@ -30,13 +30,17 @@ struct Launch {
     sddmm::TileArgs ta{};
     sddmm::DenseFn dfn = nullptr;       // dense-block kernel; null: not a dense launch
     sddmm::DenseArgs da{};
+    sddmm::BlockFn bfns[2] = {};        // row-block kernel, without and with the row softmax; null: not a row-block launch
+    sddmm::BlockArgs ba{};
+    int32_t softmax_waves = 0;          // waves per workgroup of the form with the softmax
     float *sval = nullptr;        // the plan's values in stream order (launches that walk a permuted stream)
     const int32_t *perm = nullptr;  // stream position -> sorted position of that launch (null: identity)
     int32_t grid = 0, block = 0, lds = 0, k_slice = 0;
     int32_t tile_g = 0, gather_g = 8;
     int64_t nnz = 0, rows = 0, positions = 0;
     // what the function pointers above were looked up with (they are looked up again when a saved plan is loaded)
-    int32_t fn_kind = 0;  // 1 stream kernel (row gather), 2 stream kernel with an LDS tile, 3 tile kernel, 4 panel, 5 dense
+    int32_t fn_kind = 0;  // 1 stream kernel (row gather), 2 stream kernel with an LDS tile, 3 tile kernel, 4 panel, 5 dense,
+                          // 6 row blocks
     int32_t fn_g = 0, fn_kpl = 0, fn_exact = 0, fn_gather = 0, fn_nwaves = 0;
     int32_t fn_ragged = 0;  // tile kernel: the form for ranks that are no multiple of its width
     int32_t fn_nwm = 0;  // tile kernel: waves per workgroup that run the launch's matrix-core share (0: none)
@@ -46,7 +50,7 @@ struct Launch {
     int64_t part_bytes = 0, hp_bytes = 0, wp_bytes = 0;
     int64_t ws_part = 0, ws_hp = 0, ws_wp = 0;
     // the product Y = X H (spmm_stream = 1): sp_on == 1 on this launch's tiles, 2 over the plan's CSR pattern with records
-    // in sa.part (see add_tile), 0 not built
+    // in sa.part (see add_tile), 3 on the row blocks, 0 not built
     sddmm::SpmmArgs sa{};
     int32_t sp_on = 0, sp_grid = 0, sp_nwaves = 16;  // (16 waves per workgroup: 1.54 against 1.59 ms with 12 on the recommender shape)
     int64_t sp_part_bytes = 0, ws_sp_part = 0;
@@ -163,4 +167,6 @@ inline bool product_walks(int64_t nnz, int32_t K, int ks) { return nnz < 4000000
 // ks: K elements per launch, a divisor of K or (ragged ranks) the width K is rounded up to
 int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t panel_rows, int want_g, int ks,
              sddmm_plan_info *I, bool gather = false, bool x_explicit = false);
+// planner_block.hip: all of S on the row-block kernels, where that pays (*taken)
+int add_blocks(Ctx &c, const std::vector<int32_t> &rows, bool *taken);
 }  // namespace sddmm

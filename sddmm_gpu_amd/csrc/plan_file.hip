@@ -28,7 +28,7 @@ struct PlanFileHeader {
     uint64_t data_checksum;  // over the arrays, in pieces of kPlanPiece bytes per allocation (see piece_hash)
 };
 constexpr char kPlanMagic[8] = {'S', 'D', 'D', 'M', 'M', 'P', 'L', 'N'};
-constexpr uint32_t kPlanVersion = 4;
+constexpr uint32_t kPlanVersion = 5;
 constexpr size_t kPlanPiece = (size_t)16 << 20;  // arrays are read, copied and check-summed in pieces of this size
 
 // Hash of one piece of an array: four interleaved multiply-add chains over its 8-byte words (so that a
@@ -57,10 +57,11 @@ uint64_t piece_hash(const void *data, size_t n, uint64_t alloc, uint64_t piece)
 bool launch_plausible(const Launch &L, int64_t nnz)
 {
     const int64_t slack = 2 * nnz + (1 << 20);  // padded streams stay well below twice the nonzeros + per-item rounding
-    return L.fn_kind >= 1 && L.fn_kind <= 5 && L.grid > 0 && L.grid <= (1 << 24) && L.block >= 64 && L.block <= 1024 &&
+    return L.fn_kind >= 1 && L.fn_kind <= 6 && L.grid > 0 && L.grid <= (1 << 24) && L.block >= 64 && L.block <= 1024 &&
            L.block % 64 == 0 && L.lds >= 0 && L.lds <= kLdsMaxBytes && L.nnz >= 0 && L.nnz <= nnz && L.rows >= 0 &&
            L.positions >= 0 && L.positions <= slack + 62 * nnz && L.k_slice >= 0 && L.fn_nwm >= 0 && L.fn_nwm <= 8 &&
-           L.ta.n_items >= 0 && L.ta.n_units >= 0 && L.ka.n_items >= 0 && L.ta.mf_groups >= 0 && L.ta.mf_n_cb >= 0;
+           L.ta.n_items >= 0 && L.ta.n_units >= 0 && L.ka.n_items >= 0 && L.ta.mf_groups >= 0 && L.ta.mf_n_cb >= 0 &&
+           (L.fn_kind != 6 || (L.grid == L.ba.n_units && L.block == 64 * L.fn_nwaves && L.ba.nnz == nnz && (L.softmax_waves == 4 || L.softmax_waves == 8) && L.ba.n_long_pieces >= 0 && L.ba.n_sums >= 0 && L.ba.n_empty >= 0));
 }
 constexpr uint64_t kScratchBit = 1ull << 63;
 constexpr uint64_t kBorrowedRowPtr = (1ull << 63) | 1, kBorrowedCol = (1ull << 63) | 2;
@@ -75,6 +76,7 @@ void launch_pointer_fields(Launch &L, std::vector<void *> &fields)
             &L.sa.sum_rows, &L.sa.gather_rows,
             &L.pa.slot_row, &L.pa.panel_tiles,
             &L.da.slot_rows, &L.da.slot_cols, &L.da.slot_range, &L.da.nz_p, &L.da.nz_rc,
+            &L.ba.units, &L.ba.rows, &L.ba.cols, &L.ba.info, &L.ba.long_pieces, &L.ba.long_records, &L.ba.sums, &L.ba.empty_rows, &L.ba.part,
             &L.sval, &L.perm};
 }
 
@@ -262,6 +264,7 @@ int load_plan_file(const char *path, int64_t n_rows, int64_t n_cols, int64_t nnz
         L.ka.row_ptr = nullptr;
         L.ta.sval = nullptr; L.ta.val = nullptr; L.ta.W = L.ta.H = nullptr; L.ta.out = nullptr;
         L.pa.row_ptr = nullptr; L.pa.col_ind = nullptr; L.pa.val = nullptr; L.pa.W = L.pa.H = nullptr; L.pa.out = nullptr;
+        L.ba.val = nullptr; L.ba.W = L.ba.H = nullptr; L.ba.out = nullptr; L.ba.x = nullptr; L.ba.Y = nullptr;
         L.da.nz_val = nullptr; L.da.val = nullptr; L.da.W = L.da.H = nullptr; L.da.out = nullptr;
         if (int rc = resolve_functions(L)) return rc;
     }
@@ -318,7 +321,7 @@ int sddmm_plan_save(const sddmm_plan *plan, const char *path)
                 if (!encode_pointer(plan, p, &code)) return fail(SDDMM_ERR_ARG, "sddmm_plan_save: a launch refers to memory outside the plan");
                 memcpy(field, &code, 8);
             }
-            L.fn = nullptr; L.pfn = nullptr; L.tfn = nullptr; L.dfn = nullptr;
+            L.fn = nullptr; L.pfn = nullptr; L.tfn = nullptr; L.dfn = nullptr; L.bfns[0] = L.bfns[1] = nullptr;
             for (auto &row : L.tfns) for (auto &fp : row) fp = nullptr;
         }
         HIP_TRY(hipDeviceSynchronize());  // a set_values still in flight has to land first

@@ -126,7 +126,7 @@ void apply_env_overrides(sddmm_plan_options &o)
 // Looks the launch's kernels up from its descriptor (fn_kind, fn_*, k_slice) and allows them its LDS size.
 int resolve_functions(Launch &L)
 {
-    L.fn = nullptr; L.pfn = nullptr; L.tfn = nullptr; L.dfn = nullptr;
+    L.fn = nullptr; L.pfn = nullptr; L.tfn = nullptr; L.dfn = nullptr; L.bfns[0] = L.bfns[1] = nullptr;
     for (auto &row : L.tfns) for (auto &f : row) f = nullptr;
     switch (L.fn_kind) {
     case 1:
@@ -170,6 +170,15 @@ int resolve_functions(Launch &L)
     }
     case 5:
         L.dfn = dense_kernel();
+        return SDDMM_OK;
+    case 6:
+        for (int softmax = 0; softmax < 2; ++softmax) {
+            L.bfns[softmax] = block_kernel(L.ba.K, softmax != 0, softmax ? L.softmax_waves : L.fn_nwaves);
+            if (!L.bfns[softmax]) return fail(SDDMM_ERR_ARG, "plan: no row-block kernel for K = %d and %d waves", L.ba.K, L.fn_nwaves);
+        }
+        HIP_TRY(hipFuncSetAttribute((const void *)L.bfns[0], hipFuncAttributeMaxDynamicSharedMemorySize, kRoundTiles * kBlockTileBytes));
+        HIP_TRY(hipFuncSetAttribute((const void *)L.bfns[1], hipFuncAttributeMaxDynamicSharedMemorySize, L.lds));
+        HIP_TRY(block_spmm_set_lds(L.ba.K, L.fn_nwaves));
         return SDDMM_OK;
     }
     return fail(SDDMM_ERR_FORMAT, "plan: unknown kernel descriptor %d", L.fn_kind);
@@ -663,6 +672,16 @@ static Split estimate_split(const Ctx &c, const std::vector<int32_t> &rows, int 
     return t_tile < t_gather ? Split::all_tiled : Split::all_gathered;
 }
 
+// Has the caller left the choice of kernels and their layout to the planner?  (dense_blocks = 0 asks for fp32 throughout)
+static bool only_defaults(const sddmm_plan_options &o)
+{
+    return o.tile_size_x == 0 && o.tile_size_y == 0 && o.k_slice <= 0 && o.tile_lanes <= 0 && o.tile_waves < 0 && o.tile_assign < 0 &&
+           o.tile_few_blocks < 0 && o.tile_short_batches < 0 && o.tile_deal < 0 && o.tile_runs < 0 && o.gather_lanes <= 0 && o.gather_padded < 0 &&
+           o.gather_sink < 0 && o.row_padded < 0 && o.unpadded_tile < 0 && o.dense_blocks != 0 && o.dense_permille < 0 && o.dense_rb_group < 0 &&
+           o.fuse_slices < 0 && o.matrix_rows < 0 && o.gather_slab_cols < 0 && o.gather_panel_rows < 0 && o.dense_min_nnz < 0 && o.panel_bytes < 0 &&
+           o.short_row_max < 0 && o.stage_factor < 0 && o.split_min_nnz < 0;
+}
+
 // Common plan builder from host CSR arrays.  d_*_borrowed != null: the device
 // already holds that array.
 int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_ptr_all, const int32_t *col_ind_all,
@@ -791,7 +810,13 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
     for (int64_t r = 0; r < n_rows; ++r)
         if (row_ptr[r + 1] > row_ptr[r]) ne.push_back((int32_t)r);
 
-    if (kernel == SDDMM_KERNEL_HYBRID) {
+    bool blocks = false;
+    if (kernel == SDDMM_KERNEL_HYBRID && D.n_dense == 0 && only_defaults(opt))
+        if (int rc = add_blocks(c, ne, &blocks)) return rc;
+    if (blocks) {
+        I.kernel = SDDMM_KERNEL_HYBRID;
+        I.n_blocks = I.dense_blocks;
+    } else if (kernel == SDDMM_KERNEL_HYBRID) {
         // Rows are split by length into classes:
         //   long   tile kernel with the default group size
         //   medium (only with SDDMM_MED_CLASS=1) tile kernel with groups of 4 lanes: less
