@@ -174,13 +174,13 @@ static hipError_t issue_launch(const sddmm_plan *plan, const Launch &L, const fl
         const int vm = residual ? (ta.sval ? 3 : 4) : ta.sval ? 0 : (val ? 1 : 2);
         const bool sliced = L.k_slice < I.K;
         if (sliced && L.fused_slices) {
-            ta.k_off = 0; ta.n_slices = (I.K + L.k_slice - 1) / L.k_slice; ta.to_part = 0;
+            ta.k_off = 0; ta.n_slices = (I.K + L.k_slice - 1) / L.k_slice;
             return launch(L.tfns[vm][3], dim3((unsigned)L.grid), dim3((unsigned)L.block), (size_t)L.lds, stream, ta);
         }
         for (int k_off = 0; k_off < I.K; k_off += L.k_slice) {
             ta.k_off = k_off;
-            ta.to_part = sliced && k_off + L.k_slice < I.K;
-            if (hipError_t e = launch(L.tfns[vm][!sliced ? 0 : k_off == 0 ? 1 : 2], dim3((unsigned)L.grid), dim3((unsigned)L.block), (size_t)L.lds,
+            const int slice = !sliced ? 0 : k_off + L.k_slice >= I.K ? 4 : k_off == 0 ? 1 : 2;
+            if (hipError_t e = launch(L.tfns[vm][slice], dim3((unsigned)L.grid), dim3((unsigned)L.block), (size_t)L.lds,
                                       stream, ta))
                 return e;
         }

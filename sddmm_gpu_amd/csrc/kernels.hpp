@@ -62,6 +62,7 @@ struct TileArgs {
     // pbase replaces perm with one word per group of G positions -- the sorted position of
     // the group's first nonzero; its nonzeros are consecutive there -- and grow carries the
     // group's number of nonzeros minus one in its low bits (rows are K/4 >= 8 float4 long).
+    // Launches of several K slices have their columns in scol16 as well, and nothing in scol.
     const uint16_t *scol16;
     const int32_t *pbase;
     // One bit per batch of 64 positions, counted from WorkItem::batch_base inside an item: set for a
@@ -71,8 +72,7 @@ struct TileArgs {
     const float *val;      // values in sorted order or null
     const float *W, *H;
     float *out;
-    float *part;               // partial results in stream order between the K slices of a sliced launch (else null)
-    int32_t to_part;           // sliced launch: this slice stores to part (every slice but the last)
+    float *part;               // dot products so far, in stream order, between the K slices of a sliced launch (else null)
     float *sink;               // gather form: 256 x 64 floats that take the results of flagged padding positions
     const int32_t *unit_ptr;   // [n_units+1] first stream position of each (row panel, column tile) unit
     const int32_t *unit_tile;  // [n_units] the unit's column tile
@@ -114,7 +114,8 @@ constexpr bool tile_variant_shorts(int G, int KPL, bool gather)
 TileVariant pick_tile_variant(int K, int want_g);
 // vmode: 0 = values in stream order (sval), 1 = values in sorted order (val), 2 = no values
 // gather: H rows from global memory, 4 waves per workgroup (otherwise H tiles in LDS, nwaves = 16 or 12 waves)
-// slice: 0 the launch covers all of K, 1 first of several K slices, 2 a later one (see the kernel template)
+// slice: 0 the launch covers all of K, 1 first of several K slices, 2 one in between, 4 the last one, 3 all in one launch (see
+// the kernel template); 1 and 2 are the same for every vmode
 // ragged: the form for ranks that are no multiple of the variant's width (see the kernel template)
 TileFn tile_kernel(const TileVariant &v, int vmode, bool gather, int slice, int nwaves, bool ragged);
 int ragged_tile_width(int K);  // the width for such a rank (0: none)

@@ -139,27 +139,43 @@ __device__ __forceinline__ float xor_lane(float v)
     return __int_as_float(from_lane_xor<S>(__float_as_int(v)));
 }
 
+// The dot product of lane l's nonzero as the two terms of the last sum.
 // XORDER: lane distance 1 first and the largest last, when one register is left:
 // distances 1 and 2 are one v_add with a DPP operand, larger ones cost more.
+struct Halves { float x, y; };
 template <int G, bool XORDER, int S = XORDER ? 1 : G / 2>
-__device__ __forceinline__ void transpose_reduce_step(float (&acc)[G], int l)
+__device__ __forceinline__ Halves transpose_reduce(float (&acc)[G], int l)
 {
     if constexpr (XORDER) {
-        if constexpr (S < G) {
+        if constexpr (S * 2 == G) return {acc[0], xor_lane<S>(acc[S])};
+        else {
 #pragma unroll
             for (int j = 0; j < G; j += 2 * S) acc[j] += xor_lane<S>(acc[j + S]);
-            transpose_reduce_step<G, XORDER, S * 2>(acc, l);
+            return transpose_reduce<G, XORDER, S * 2>(acc, l);
         }
-    } else if constexpr (S >= 1) {
+    } else {
         const bool upper = (l & S) != 0;
+        if constexpr (S == 1) return {upper ? acc[1] : acc[0], xor_lane<1>(upper ? acc[0] : acc[1])};
+        else {
 #pragma unroll
-        for (int j = 0; j < S; ++j) {
-            float keep = upper ? acc[j + S] : acc[j];
-            float send = upper ? acc[j] : acc[j + S];
-            acc[j] = keep + xor_lane<S>(send);
+            for (int j = 0; j < S; ++j) {
+                float keep = upper ? acc[j + S] : acc[j];
+                float send = upper ? acc[j] : acc[j + S];
+                acc[j] = keep + xor_lane<S>(send);
+            }
+            return transpose_reduce<G, XORDER, S / 2>(acc, l);
         }
-        transpose_reduce_step<G, XORDER, S / 2>(acc, l);
     }
+}
+
+// old + (x + y), nearly as if rounded once.  Three sums of a few bits' difference in size lose more to rounding than their
+// number says (the bits cut off are few and often exactly a half).  second: which half's lane this is.  (A nonzero that
+// several lanes work on, with the halves exchanged, must come out the same in all of them.)
+__device__ __forceinline__ Halves add_to(float old, Halves h, bool second)
+{
+    const float x = second ? h.y : h.x, y = second ? h.x : h.y;
+    const float t = old + x, lost = x - (t - old);
+    return {t, y + (__builtin_isfinite(t) ? lost : 0.f)};
 }
 
 // The matrix-core share of a tile launch, run by the last NWM waves of every workgroup while the
@@ -280,18 +296,21 @@ __device__ __forceinline__ void matrix_core_waves(const TileArgs &a, int mw, int
 
 // VMODE: where S.val comes from -- 0: a.sval (stream order), 1: a.val (sorted
 // order, read through the position), 2: nowhere (no scaling); 3 and 4: as 0 and 1
-// with the residual epilogue, out = val - dot (K slices after the first: out -= dot,
-// no value needed).
+// with the residual epilogue, out = val - dot.
 //
 // The loop is software-pipelined by hand and free of branches around loads, so
 // that every wait is for exactly the data needed: while batch b is computed,
 // the index data of batch b+2 and the W row slice of batch b+1 are in flight.
 // GATHER: no LDS tile; scol holds the column and H rows are read from global
 // memory (the stream is then one unit in row order, for rows too short to tile).
-// SLICE: 0 = the launch covers all of K (results go to out); 1 = first of several K slices (partial
-// results go to a.part, in stream order: one coalesced store per batch); 2 = a later slice (adds to the
-// partial result read back from a.part, coalesced, and stores to a.part again or, in the last slice,
-// a.to_part == 0, to out).  Only the last slice touches out, with one scattered store per position.
+// SLICE: 0 = the launch covers all of K (results go to out); 1 = first of several K slices (the dot
+// products so far go to a.part, in stream order: one coalesced store per batch); 2 = a slice in between
+// (adds to what it reads back from a.part, coalesced); 4 = the last one, which alone reads positions and
+// values and touches out, with one scattered store per position.
+// (The slices before it are bound by the vector unit, two thirds busy, and by waits for W; the last one by its positions,
+// values and partial output lines.  Before, all of them read positions and values, columns in 32 bits, and scaled: a band of 64
+// in 4096 columns, 2^20 rows, K = 512, 4.02 -> 3.42 ms (1.46 -> 0.29 GB of stream data in each but the last); the remainder
+// of the recommender at K = 512, 1.39 -> 1.21.  Stream data four batches ahead, or with the non-temporal hint: the same.)
 // 3 = all a.n_slices K slices inside this one launch, one after the other (small matrices, where a
 // launch costs as much as its work): a wave meets the same positions in every slice, so the partial
 // results it left in a.part are its own, and a workgroup barrier between the slices is all the
@@ -309,14 +328,16 @@ __global__ __launch_bounds__((NW + NWM) * 64)
 void sddmm_tile_kernel(const TileArgs a)
 {
     constexpr bool FUSED = SLICE == 3;
-    constexpr bool ACC = SLICE == 2;
+    constexpr bool ACC = SLICE == 2 || SLICE == 4;
     constexpr bool PART = SLICE >= 1;
+    constexpr bool TO_OUT = SLICE == 0 || SLICE >= 3;  // positions and values are needed
+    static_assert(TO_OUT || VMODE == 2);
     static_assert(!RAGGED || (!GATHER && NWM == 0));
     extern __shared__ float4 lds_tile[];
     constexpr int K4 = G * KPL;
     constexpr bool RESIDUAL = VMODE >= 3;
-    constexpr bool STREAM_VAL = VMODE == 0 || (VMODE == 3 && !ACC);  // values read in stream order
-    constexpr bool SORTED_VAL = VMODE == 1 || (VMODE == 4 && !ACC);  // values read through the position
+    constexpr bool STREAM_VAL = VMODE == 0 || VMODE == 3;  // values read in stream order
+    constexpr bool SORTED_VAL = VMODE == 1 || VMODE == 4;  // values read through the position
     constexpr bool XORDER = !GATHER && (K4 % 16 == 0);
     constexpr bool COMPACT = !GATHER && K4 <= 16;  // the compact stream format (see TileArgs)
     constexpr bool STREAM_HINT = !GATHER && !COMPACT && SLICE == 0;  // (see ld_meta)
@@ -326,7 +347,9 @@ void sddmm_tile_kernel(const TileArgs a)
     // K = 32 launch measured.  Its index data is therefore requested four batches ahead (the arrays' slack
     // of 256 entries covers exactly the four batches past the end).
     constexpr bool DEEP = COMPACT;
-    constexpr int ROW_SHIFT = K4 == 16 ? 8 : K4 == 8 ? 7 : 0;  // log2 of an LDS row in bytes (COMPACT only)
+    constexpr bool COL16 = COMPACT || (!GATHER && PART);  // columns from a.scol16
+    constexpr int ROW_SHIFT = __builtin_ctz(K4 * 16);     // log2 of an LDS row in bytes
+    static_assert(!COL16 || (K4 & (K4 - 1)) == 0);
     // SHORTS: a batch may be marked "short" in a.btype: each of its groups then holds at most G/2
     // nonzeros in its first G/2 positions and the same ones again in the other G/2.  With the
     // lane-permuted order the upper half of the lanes then works on the same nonzeros as the lower
@@ -499,8 +522,8 @@ void sddmm_tile_kernel(const TileArgs a)
         struct Meta { uint32_t wrow, p, o; int col; float sv, old; };  // o: byte offset of the position's fp32 slot inside the item
         const uint32_t last = (uint32_t)(end - begin - 1);
         const char *perm_b = reinterpret_cast<const char *>(COMPACT ? a.pbase + begin / G : a.perm + begin);
-        const char *scol_b = COMPACT ? reinterpret_cast<const char *>(a.scol16 + begin)
-                                     : reinterpret_cast<const char *>(a.scol + begin);
+        const char *scol_b = COL16 ? reinterpret_cast<const char *>(a.scol16 + begin)
+                                   : reinterpret_cast<const char *>(a.scol + begin);
         const char *sval_b = reinterpret_cast<const char *>(a.sval + begin);
         const char *grow_b = reinterpret_cast<const char *>(a.grow + begin / G);
         // Steady state: batches are requested in order, two ahead of the one computed,
@@ -513,13 +536,13 @@ void sddmm_tile_kernel(const TileArgs a)
             if constexpr (COMPACT) {
                 const uint32_t g = ld_meta<STREAM_HINT>(reinterpret_cast<const uint32_t *>(grow_b + og));
                 m.wrow = RAGGED ? (g >> 3) * (uint32_t)a.K : g & ~(uint32_t)(G - 1);
-                m.p = ld_meta<STREAM_HINT>(reinterpret_cast<const uint32_t *>(perm_b + og)) + min((uint32_t)l, g & (uint32_t)(G - 1));
-                m.col = (int)ld_meta<STREAM_HINT>(reinterpret_cast<const uint16_t *>(scol_b + (o4 >> 1))) << ROW_SHIFT;
+                if constexpr (TO_OUT) m.p = ld_meta<STREAM_HINT>(reinterpret_cast<const uint32_t *>(perm_b + og)) + min((uint32_t)l, g & (uint32_t)(G - 1));
             } else {
                 m.wrow = ld_meta<STREAM_HINT>(reinterpret_cast<const uint32_t *>(grow_b + og));
-                m.p = ld_meta<STREAM_HINT>(reinterpret_cast<const uint32_t *>(perm_b + o4));
-                m.col = ld_meta<STREAM_HINT>(reinterpret_cast<const int *>(scol_b + o4));
+                if constexpr (TO_OUT) m.p = ld_meta<STREAM_HINT>(reinterpret_cast<const uint32_t *>(perm_b + o4));
             }
+            if constexpr (COL16) m.col = (int)ld_meta<STREAM_HINT>(reinterpret_cast<const uint16_t *>(scol_b + (o4 >> 1))) << ROW_SHIFT;
+            else m.col = ld_meta<STREAM_HINT>(reinterpret_cast<const int *>(scol_b + o4));
             m.sv = STREAM_VAL ? ld_meta<STREAM_HINT>(reinterpret_cast<const float *>(sval_b + o4)) : 1.0f;
             m.o = o4;
             o4 += 256;
@@ -534,13 +557,13 @@ void sddmm_tile_kernel(const TileArgs a)
             if constexpr (COMPACT) {
                 const uint32_t g = *reinterpret_cast<const uint32_t *>(grow_b + tg);
                 m.wrow = RAGGED ? (g >> 3) * (uint32_t)a.K : g & ~(uint32_t)(G - 1);
-                m.p = *reinterpret_cast<const uint32_t *>(perm_b + tg) + min((t4 >> 2) & (uint32_t)(G - 1), g & (uint32_t)(G - 1));
-                m.col = (int)*reinterpret_cast<const uint16_t *>(scol_b + (t4 >> 1)) << ROW_SHIFT;
+                if constexpr (TO_OUT) m.p = *reinterpret_cast<const uint32_t *>(perm_b + tg) + min((t4 >> 2) & (uint32_t)(G - 1), g & (uint32_t)(G - 1));
             } else {
                 m.wrow = *reinterpret_cast<const uint32_t *>(grow_b + tg);
-                m.p = *reinterpret_cast<const uint32_t *>(perm_b + t4);
-                m.col = *reinterpret_cast<const int *>(scol_b + t4);
+                if constexpr (TO_OUT) m.p = *reinterpret_cast<const uint32_t *>(perm_b + t4);
             }
+            if constexpr (COL16) m.col = (int)*reinterpret_cast<const uint16_t *>(scol_b + (t4 >> 1)) << ROW_SHIFT;
+            else m.col = *reinterpret_cast<const int *>(scol_b + t4);
             m.sv = STREAM_VAL ? *reinterpret_cast<const float *>(sval_b + t4) : 1.0f;
             m.o = t4;
             return m;
@@ -577,17 +600,16 @@ void sddmm_tile_kernel(const TileArgs a)
         };
         float pend_v;  // result of the batch before, not yet stored
         uint32_t pend_p, pend_o;
-        const bool to_part = PART && (FUSED ? !last_slice : a.to_part != 0);  // (uniform)
         // (gather form: a position whose index carries bit 31 is padding that worked on
         // another row's column; its result goes to a scratch line instead of the output)
-        // (one store whose address is selected, not a branch around two stores: a branch inside the
-        // loop body costs the later slices of a sliced launch 8 % -- 736 against 679 us on the recommender)
+        // (FUSED: one store whose address is selected, not a branch around two stores)
         auto flush = [&]() {
             float *dst;
-            if constexpr (GATHER) dst = (int32_t)pend_p < 0 ? a.sink + (((blockIdx.x & 255) << 6) + lane) : a.out + pend_p;
-            else dst = a.out + pend_p;
             // (a padding position has a slot of its own in a.part)
-            if constexpr (PART) dst = to_part ? reinterpret_cast<float *>(part_b + pend_o) : dst;
+            if constexpr (!TO_OUT) dst = reinterpret_cast<float *>(part_b + pend_o);
+            else if constexpr (GATHER) dst = (int32_t)pend_p < 0 ? a.sink + (((blockIdx.x & 255) << 6) + lane) : a.out + pend_p;
+            else dst = a.out + pend_p;
+            if constexpr (FUSED) dst = last_slice ? dst : reinterpret_cast<float *>(part_b + pend_o);
             *dst = pend_v;
         };
         // c[I]: where the H row this lane works on in step I starts (LDS: byte address of
@@ -652,19 +674,33 @@ void sddmm_tile_kernel(const TileArgs a)
                 }(std::make_integer_sequence<int, STEPS>{});
             }
             columns_of_steps<G, XORDER>(next_col, lane_base0, cn);
+            Halves h;
             if constexpr (SHORT) {
-                transpose_reduce_step<G / 2, XORDER>(acc, l);  // inside each half group
-                acc[0] += xor_lane<G / 2>(acc[0]);             // the other half's slices of the same nonzero
+                h = transpose_reduce<G / 2, XORDER>(acc, l);  // inside each half group
+                const float half = h.x + h.y;
+                h = {half, xor_lane<G / 2>(half)};            // the other half's slices of the same nonzero
             } else {
-                transpose_reduce_step<G, XORDER>(acc, l);
+                h = transpose_reduce<G, XORDER>(acc, l);
             }
             // The store is left to the start of the next batch (flush): issued here it
             // would sit, unfinished, in front of the loads that batch waits for.  In a
             // whole batch it needs no predicate: a padding position repeats a nonzero of
             // its own group and so writes that nonzero's own result a second time.
-            if constexpr (RESIDUAL) pend_v = ACC ? m.old - acc[0] : FUSED ? (first_slice ? v : m.old) - acc[0] : v - acc[0];
-            else pend_v = (ACC || FUSED) ? fmaf(acc[0], v, m.old) : acc[0] * v;
-            pend_p = m.p;
+            // (Relative error against 64 bits of a band, 4 slices, scaled / residual: 4.09e-8 / 4.43e-8 when every slice was
+            // scaled and added; 3.93e-8 / 4.10e-8 so; with plain sums 4.20e-8 / 4.28e-8.)
+            if constexpr (!PART) {
+                pend_v = RESIDUAL ? v - (h.x + h.y) : (h.x + h.y) * v;
+            } else if constexpr (SLICE == 1) {
+                pend_v = h.x + h.y;
+            } else {
+                const Halves sum = add_to(m.old, h, (l & (XORDER ? G / 2 : 1)) != 0);
+                if constexpr (SLICE == 2) pend_v = sum.x + sum.y;
+                else {
+                    pend_v = RESIDUAL ? (v - (h.x + h.y)) - m.old : VMODE == 2 ? sum.x + sum.y : fmaf(sum.x, v, sum.y * v);
+                    if constexpr (FUSED) pend_v = last_slice ? pend_v : sum.x + sum.y;
+                }
+            }
+            if constexpr (TO_OUT) pend_p = m.p;
             pend_o = m.o;
         };
 
@@ -755,9 +791,12 @@ TileFn ragged_tile_kernel(const TileVariant &v, bool gather, int slice, int nwav
     if (v.G == 4 && v.KPL == 4 && nwaves == 12 && slice == 0) return (TileFn)sddmm_tile_kernel<4, 4, VMODE, 12, false, 0, 0, true>;
     if (v.G == 8 && v.KPL == 4 && nwaves == 12) {
         if (slice == 0) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 0, 0, true>;
-        if (slice == 1) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 1, 0, true>;
-        if (slice == 2) return (TileFn)sddmm_tile_kernel<8, 4, (VMODE == 4 ? 3 : VMODE), 12, false, 2, 0, true>;
+        if constexpr (VMODE == 2) {
+            if (slice == 1) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 1, 0, true>;
+            if (slice == 2) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 2, 0, true>;
+        }
         if (slice == 3) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 3, 0, true>;
+        if (slice == 4) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 4, 0, true>;
     }
     return nullptr;
 }

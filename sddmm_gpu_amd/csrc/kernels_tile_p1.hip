@@ -10,8 +10,7 @@ TileFn tile_kernel_part1(const TileVariant &v, int vmode, bool gather, int slice
     if (ragged) return ragged_tile_kernel<1>(v, gather, slice, nwaves);
 #define SDDMM_PICK_SLICE(g, kpl, vm, nw, ga)                                                                 \
     (slice == 3 ? fused_slices_kernel<g, kpl, vm, nw, ga>()                                                 \
-     : slice == 2 ? (TileFn)sddmm_tile_kernel<g, kpl, (vm == 4 ? 3 : vm), nw, ga, 2>                        \
-     : slice == 1 ? (TileFn)sddmm_tile_kernel<g, kpl, vm, nw, ga, 1>                                        \
+     : slice == 4 ? (TileFn)sddmm_tile_kernel<g, kpl, vm, nw, ga, 4>                                        \
                   : (TileFn)sddmm_tile_kernel<g, kpl, vm, nw, ga, 0>)
 #define SDDMM_PICK(g, kpl, vm)                                                                              \
     (gather ? SDDMM_PICK_SLICE(g, kpl, vm, 4, true)                                                         \

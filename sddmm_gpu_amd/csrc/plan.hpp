@@ -22,7 +22,7 @@ struct Launch {
     sddmm::KernelFn fn = nullptr;   // stream kernels
     sddmm::PanelFn pfn = nullptr;   // panel kernel
     sddmm::TileFn tfn = nullptr;        // tile kernel (values in stream order, first K slice); null: not a tile launch
-    sddmm::TileFn tfns[5][4] = {};      // [values in stream order / in sorted order / none / residual epilogue with values
+    sddmm::TileFn tfns[5][5] = {};      // [values in stream order / in sorted order / none / residual epilogue with values
                                  //  in stream order / in sorted order][the only K slice / first of several / a later one /
                                  //  all slices inside one launch (null: no such variant)]
     sddmm::KArgs ka{};

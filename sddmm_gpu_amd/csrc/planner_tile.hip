@@ -757,26 +757,32 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
     if (compact && c.orig) return fail(SDDMM_ERR_ARG, "plan: compact tile stream over a remainder matrix");
     if (compact) {
         const int64_t ng = np / G;
-        big_vector<uint16_t> scol16((size_t)np + kStreamSlack);
         big_vector<int32_t> pbase((size_t)ng + kStreamSlack);
-        std::fill(scol16.begin() + np, scol16.end(), (uint16_t)0);
         std::fill(pbase.begin() + ng, pbase.end(), 0);
-        const int32_t row_bytes = ks * 4;
         parallel_ranges(ng, 1 << 12, [&](int64_t gb, int64_t ge, int) {
             for (int64_t g = gb; g < ge; ++g) {
                 int cnt = 1;
                 while (cnt < G && perm[(size_t)(g * G + cnt)] != perm[(size_t)(g * G + cnt - 1)]) ++cnt;
                 pbase[(size_t)g] = perm[(size_t)(g * G)];
                 grow[(size_t)g] |= cnt - 1;
-                for (int i = 0; i < G; ++i) scol16[(size_t)(g * G + i)] = (uint16_t)(scol[(size_t)(g * G + i)] / row_bytes);
             }
         });
-        uint16_t *d_scol16 = nullptr;
         int32_t *d_pbase = nullptr;
-        if (int rc = c.up(&d_scol16, scol16)) return rc;
         if (int rc = c.up(&d_pbase, pbase)) return rc;
-        L.ta.scol16 = d_scol16; L.ta.pbase = d_pbase;
-        big_vector<int32_t>().swap(scol);  // not used by the compact kernels
+        L.ta.pbase = d_pbase;
+    }
+    if (compact || (!gather && ks < c.K)) {
+        // columns inside the tile in 16 bits (K slices read them again in every slice)
+        big_vector<uint16_t> scol16((size_t)np + kStreamSlack);
+        std::fill(scol16.begin() + np, scol16.end(), (uint16_t)0);
+        const int32_t row_bytes = ks * 4;
+        parallel_ranges(np, 1 << 15, [&](int64_t b, int64_t e, int) {
+            for (int64_t i = b; i < e; ++i) scol16[(size_t)i] = (uint16_t)(scol[(size_t)i] / row_bytes);
+        });
+        uint16_t *d_scol16 = nullptr;
+        if (int rc = c.up(&d_scol16, scol16)) return rc;
+        L.ta.scol16 = d_scol16;
+        big_vector<int32_t>().swap(scol);
     }
     if (shorts) {
         uint32_t *d_btype = nullptr;
