@@ -241,7 +241,11 @@ hipError_t launch_block_spmm(const BlockArgs &a, int nwaves, void *stream);
 
 // lanes per nonzero and float4 slots per lane for a given K; G == 0: none
 Variant pick_gather_variant(int K);  // row gather, any K from 4 to 2048
-KernelFn gather_kernel(const Variant &v);
+// How the row gather over nnz nonzeros of n_rows rows is dealt out: nonzeros per workgroup, and whether a wave has one
+// batch of 64 and the kernel made for that.
+struct GatherShape { int chunk; bool once; };
+GatherShape gather_shape(int64_t nnz, int64_t n_rows, const Variant &v);
+KernelFn gather_kernel(const Variant &v, bool once);
 KernelFn generic_kernel();           // row gather, any K
 Variant pick_stream_variant(int K);  // unpadded LDS tile (K % 4 == 0)
 KernelFn stream_kernel(const Variant &v);

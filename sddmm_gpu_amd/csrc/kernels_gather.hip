@@ -197,6 +197,87 @@ void sddmm_gather_kernel(const KArgs a)
     }
 }
 
+// The same with one batch a wave, for what the chain of loads bounds rather than the load path: the pieces of up to
+// eight steps, W's and H's, are requested together instead of one step ahead, and a step's W row is read whether it is
+// another one or not (a copy of the step before would have to wait for that step's).  The sums are the same, bit for bit.
+// us per launch from a graph, the kernel above and this one: 18 thousand nonzeros, K = 16 / 32 / 64 / 128: 3.8 / 4.6 / 4.7 / 5.1
+// and 3.0 / 3.3 / 3.6 / 4.4; R-MAT, 1.86 million, K = 32 / 100 / 256: 43 / 86 / 257 and 30 / 77 / 230.  Where it is chosen: gather_shape.
+template <int G, int KPL, bool RAGGED>
+__global__ __launch_bounds__(kRowGatherBlock)
+void sddmm_gather_once_kernel(const KArgs a)
+{
+    constexpr int ROUND = KPL <= 2 ? (G < 8 ? G : 8) : KPL <= 4 ? 4 : 2;  // steps whose pieces are requested together
+    static_assert(G % ROUND == 0);
+    __shared__ int row_tab[kRowGatherBlock / 64][64 + 1];  // (plan-free form)
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l = lane & (G - 1);
+    const int K = a.K;
+    const int batch = blockIdx.x * (kRowGatherBlock / 64) + wave;
+    const int p0 = batch << 6;
+    if (p0 >= a.nnz) return;
+    int off[KPL], first[KPL];
+#pragma unroll
+    for (int j = 0; j < KPL; ++j) {
+        const RowPiece r = row_piece(j * G + l, K);
+        off[j] = RAGGED ? r.off : 4 * (j * G + l);
+        first[j] = r.first;
+    }
+    // (lanes past the end repeat the last nonzero and store nothing)
+    const int pos = min(p0 + lane, a.nnz - 1);
+    const int p = a.perm ? a.perm[pos] : pos;
+    const int col = a.col_ind[p];
+    const float v = a.sval ? a.sval[pos] : (a.val ? a.val[p] : 1.0f);
+    int row;
+    if (a.batch_seg) {
+        const uint64_t le = (lane == 63) ? ~0ull : ((2ull << lane) - 1ull);
+        const int seg = a.batch_seg[batch] + __popcll(a.batch_mask[batch] & le);
+        row = a.seg_row ? a.seg_row[seg] : seg;
+    } else {
+        int *tab = row_tab[wave];
+        rows_of_range(a.row_ptr, a.n_rows, a.nnz, p0, 64, tab, lane);
+        row = tab[pos - p0];
+    }
+    auto mask_piece = [&](vec4u &x, int j) {
+        if constexpr (RAGGED) {
+            x.x = first[j] > 0 ? 0.f : x.x;
+            x.y = first[j] > 1 ? 0.f : x.y;
+            x.z = first[j] > 2 ? 0.f : x.z;
+            x.w = first[j] > 3 ? 0.f : x.w;
+        }
+    };
+    float acc[G];
+    auto round = [&]<int BASE, int... I>(std::integer_sequence<int, BASE>, std::integer_sequence<int, I...>) {
+        vec4u h[ROUND][KPL], w[ROUND][KPL];
+        ((void)[&] {
+            const float *hr = a.H + (size_t)group_bcast<G, BASE + I>(col) * K;
+#pragma unroll
+            for (int j = 0; j < KPL; ++j) h[I][j] = *reinterpret_cast<const vec4u *>(hr + off[j]);
+            const float *wr = a.W + (size_t)group_bcast<G, BASE + I>(row) * K;
+#pragma unroll
+            for (int j = 0; j < KPL; ++j) w[I][j] = *reinterpret_cast<const vec4u *>(wr + off[j]);
+        }(), ...);
+        __builtin_amdgcn_sched_barrier(0);
+        ((void)[&] {
+            float s = 0.f;
+#pragma unroll
+            for (int j = 0; j < KPL; ++j) {
+                vec4u hv = h[I][j], wv = w[I][j];
+                mask_piece(hv, j);
+                mask_piece(wv, j);
+                s = fmaf(wv.x, hv.x, s); s = fmaf(wv.y, hv.y, s);
+                s = fmaf(wv.z, hv.z, s); s = fmaf(wv.w, hv.w, s);
+            }
+            acc[BASE + I] = s;
+        }(), ...);
+    };
+    [&]<int... R>(std::integer_sequence<int, R...>) {
+        (round(std::integer_sequence<int, R * ROUND>{}, std::make_integer_sequence<int, ROUND>{}), ...);
+    }(std::make_integer_sequence<int, G / ROUND>{});
+    transpose_reduce_step<G>(acc, l);
+    if (p0 + lane < a.nnz) a.out[p] = a.residual ? v - acc[0] : acc[0] * v;
+}
+
 // Any K >= 1 (used below 4 and beyond 2048): 8 lanes per nonzero striding over the row one float at a time,
 // W re-read through the cache.  The slow, always-correct path.
 __global__ __launch_bounds__(kRowGatherBlock)
@@ -273,12 +354,34 @@ Variant pick_gather_variant(int K)
     return {0, 0, false};
 }
 
-KernelFn gather_kernel(const Variant &v)
+// Reading every step's W row costs load path, which is what large launches wait for, the more the longer the rows (a
+// row's nonzeros are next to each other, and the kernel with several batches reads it once).  us, several batches a wave and one: 200
+// thousand nonzeros of 2000 rows, K = 32 / 64 / 128 / 256: 4.7 / 5.5 / 7.4 / 10.7 and 4.3 / 5.5 / 8.0 / 13.2, two million of 6000 rows,
+// K = 32 / 128: 19 / 46 and 25 / 74; but R-MAT of 131,072 rows, 2.7 million, K = 32 / 64 / 128 / 256: 44 / 67 / 149 / 380 and 40 / 71 /
+// 126 / 331, of a million rows, 28 million, K = 32 / 128: 458 / 2168 and 448 / 1927.  (K = 64 is level at best from 200 thousand on, K = 32 up to
+// four million.)
+// Batches a wave: up to 8, which is as many as share a search for the rows, but fewer where that would leave less than 4096 waves
+// (16 per compute unit): 0.9 million nonzeros, K = 32 / 64 / 128 with 2048 waves 27 / 30 / 49, with 4096 19 / 23 / 44; from 1.5
+// million on all take 8 (two million of 20,000 rows, K = 64: 35, and 38 with 7).
+GatherShape gather_shape(int64_t nnz, int64_t n_rows, const Variant &v)
+{
+    const bool short_rows = nnz <= 32 * n_rows;
+    const int pieces = v.G * v.KPL;
+    const bool once = v.G != 0 && (nnz <= 1 << 16 || (short_rows ? pieces >= 32 || (pieces != 16 && nnz <= 1 << 21) : pieces <= 8 && nnz <= 1 << 18));
+    const int64_t waves_wanted = 4096;
+    const int per_wave = once ? 1 : nnz >= 1500000 ? kRowGatherBatchesPerWave : (int)std::clamp<int64_t>(nnz / (64 * waves_wanted), 1, kRowGatherBatchesPerWave);
+    return {64 * per_wave * (kRowGatherBlock / 64), once};
+}
+
+KernelFn gather_kernel(const Variant &v, bool once)
 {
 #define SDDMM_CASE(g, kpl)                                                                 \
-    if (v.G == g && v.KPL == kpl)                                                          \
+    if (v.G == g && v.KPL == kpl) {                                                        \
+        if (once) return v.exact ? (KernelFn)sddmm_gather_once_kernel<g, kpl, false>       \
+                                 : (KernelFn)sddmm_gather_once_kernel<g, kpl, true>;       \
         return v.exact ? (KernelFn)sddmm_gather_kernel<g, kpl, false>                      \
-                       : (KernelFn)sddmm_gather_kernel<g, kpl, true>;
+                       : (KernelFn)sddmm_gather_kernel<g, kpl, true>;                      \
+    }
     SDDMM_CASE(4, 1) SDDMM_CASE(8, 1) SDDMM_CASE(8, 2) SDDMM_CASE(8, 3) SDDMM_CASE(8, 4) SDDMM_CASE(16, 3) SDDMM_CASE(16, 4)
     SDDMM_CASE(32, 3) SDDMM_CASE(32, 4) SDDMM_CASE(64, 3) SDDMM_CASE(64, 4) SDDMM_CASE(64, 8)
 #undef SDDMM_CASE

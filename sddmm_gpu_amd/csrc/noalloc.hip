@@ -1,7 +1,6 @@
 // Plan-free SDDMM over a device CSR that allocates no memory and keeps none: one launch of the row-gather
 // kernel, which finds the rows of its nonzeros from the row pointers.
 #include <hip/hip_runtime.h>
-#include <algorithm>
 #include "internal.hpp"
 #include "kernels.hpp"
 #include "launch.hpp"
@@ -23,16 +22,14 @@ extern "C" int sddmm_csr_noalloc(int64_t n_rows, int64_t n_cols, int64_t nnz, co
     if ((((uintptr_t)d_W | (uintptr_t)d_H) & 15u) && K % 4 == 0)
         return fail(SDDMM_ERR_ARG, "sddmm_csr_noalloc: W and H must be 16-byte aligned");
     const Variant var = pick_gather_variant(K);
-    const KernelFn fn = var.G ? gather_kernel(var) : generic_kernel();
 
     KArgs a{};
     a.col_ind = d_col_ind; a.val = d_val; a.W = d_W; a.H = d_H; a.out = d_out;
     a.row_ptr = d_row_ptr; a.n_rows = (int32_t)n_rows;
     a.nnz = (int32_t)nnz; a.K = K; a.n_cols = (int32_t)n_cols; a.tile_x = (int32_t)n_cols;
-    // nonzeros per workgroup: up to 8 batches of 64 per wave, fewer when that would leave compute units idle
-    const int64_t waves_wanted = 2 * 256 * (kRowGatherBlock / 64);
-    const int per_wave = (int)std::clamp<int64_t>(nnz / (64 * waves_wanted), 1, kRowGatherBatchesPerWave);
-    a.chunk = 64 * per_wave * (kRowGatherBlock / 64);
+    const GatherShape shape = gather_shape(nnz, n_rows, var);
+    const KernelFn fn = var.G ? gather_kernel(var, shape.once) : generic_kernel();
+    a.chunk = shape.chunk;
     const int grid = (int)((nnz + a.chunk - 1) / a.chunk);
     const hipError_t e = launch(fn, dim3((unsigned)grid), dim3(kRowGatherBlock), 0, (hipStream_t)stream, a);
     if (e != hipSuccess) return fail(SDDMM_ERR_HIP, "sddmm_csr_noalloc: launch failed: %s", hipGetErrorString(e));

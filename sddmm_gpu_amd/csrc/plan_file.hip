@@ -28,7 +28,7 @@ struct PlanFileHeader {
     uint64_t data_checksum;  // over the arrays, in pieces of kPlanPiece bytes per allocation (see piece_hash)
 };
 constexpr char kPlanMagic[8] = {'S', 'D', 'D', 'M', 'M', 'P', 'L', 'N'};
-constexpr uint32_t kPlanVersion = 6;
+constexpr uint32_t kPlanVersion = 7;
 constexpr size_t kPlanPiece = (size_t)16 << 20;  // arrays are read, copied and check-summed in pieces of this size
 
 // Hash of one piece of an array: four interleaved multiply-add chains over its 8-byte words (so that a

@@ -132,7 +132,7 @@ int resolve_functions(Launch &L)
     case 1:
     case 2: {
         const Variant v{L.fn_g, L.fn_kpl, L.fn_exact != 0};
-        L.fn = L.fn_kind == 2 ? stream_kernel(v) : v.G ? gather_kernel(v) : generic_kernel();
+        L.fn = L.fn_kind == 2 ? stream_kernel(v) : v.G ? gather_kernel(v, L.fn_once != 0) : generic_kernel();
         if (!L.fn) return fail(SDDMM_ERR_ARG, "plan: no stream kernel for lanes %d x %d", v.G, v.KPL);
         if (L.lds > 0) HIP_TRY(hipFuncSetAttribute((const void *)L.fn, hipFuncAttributeMaxDynamicSharedMemorySize, L.lds));
         return SDDMM_OK;
@@ -258,7 +258,6 @@ int add_row_gather(Ctx &c, const std::vector<int32_t> &rows, bool all_rows)
     if (n == 0) return SDDMM_OK;
     const Variant var = pick_gather_variant(c.K);
     L.fn_kind = 1; L.fn_g = var.G; L.fn_kpl = var.KPL; L.fn_exact = var.exact;
-    if (int rc = resolve_functions(L)) return rc;
     std::vector<int32_t> seg_end(rows.size()), perm;
     int64_t acc = 0;
     for (size_t i = 0; i < rows.size(); ++i) {
@@ -289,14 +288,14 @@ int add_row_gather(Ctx &c, const std::vector<int32_t> &rows, bool all_rows)
     a.seg_row = d_seg_row; a.perm = d_perm; a.batch_seg = d_bseg; a.batch_mask = d_bmask;
     L.perm = d_perm;
     a.nnz = (int32_t)n;
-    // nonzeros per workgroup: up to 8 batches of 64 per wave, fewer when that would leave compute units idle
-    const int64_t waves_wanted = 2 * (int64_t)c.cus * (kRowGatherBlock / 64);
-    const int per_wave = (int)std::clamp<int64_t>(n / (64 * waves_wanted), 1, kRowGatherBatchesPerWave);
-    a.chunk = 64 * per_wave * (kRowGatherBlock / 64);
+    const GatherShape shape = gather_shape(n, (int64_t)rows.size(), var);
+    a.chunk = shape.chunk;
+    L.fn_once = shape.once;
     a.K = c.K; a.n_cols = (int32_t)c.n_cols; a.tile_x = (int32_t)c.n_cols;
     L.grid = (int32_t)((n + a.chunk - 1) / a.chunk);
     L.block = kRowGatherBlock;
     L.k_slice = c.K;
+    if (int rc = resolve_functions(L)) return rc;
     c.P->info.lanes_per_nnz = var.G ? var.G : 8;
     L.gather_g = var.G ? var.G : 8; L.positions = n;
     c.P->launches.push_back(L);

@@ -1,0 +1,53 @@
+"""The row gather with one batch a wave: the edges of its batches, rounds of steps and rule, against 64 bits."""
+import pytest
+import torch
+
+from sddmm_gpu_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(n_rows, n_cols, nnz, K, seed):
+    g = torch.Generator().manual_seed(seed)
+    keys = torch.randperm(n_rows * n_cols, generator=g)[:nnz].sort().values
+    rows, cols = keys // n_cols, keys % n_cols
+    row_ptr = torch.zeros(n_rows + 1, dtype=torch.int64)
+    row_ptr[1:] = torch.cumsum(torch.bincount(rows, minlength=n_rows), 0)
+    W, H = torch.randn(n_rows, K, generator=g), torch.randn(n_cols, K, generator=g)
+    val = torch.rand(nnz, generator=g)
+    dot, size = torch.empty(nnz, dtype=torch.float64), torch.empty(nnz, dtype=torch.float64)
+    for b in range(0, nnz, 1 << 14):
+        w, h = W[rows[b:b + (1 << 14)]].double(), H[cols[b:b + (1 << 14)]].double()
+        dot[b:b + (1 << 14)] = (w * h).sum(1)
+        size[b:b + (1 << 14)] = (w * h).abs().sum(1)
+    dev = [t.cuda() for t in (row_ptr.int(), cols.int(), val, W, H)]
+    # a sum of K rounded products in any order, then one product with the value
+    return dev, dot * val.double(), (K + 1) * 2.0 ** -24 * size * val.double() + 1e-30
+
+
+@pytest.mark.parametrize("K", [4, 7, 16, 32, 33, 64, 72, 96, 100, 128, 180, 256, 300, 512, 700, 1024, 2048])
+@pytest.mark.parametrize("n_rows,n_cols,nnz", [(1, 1, 1), (40, 90, 63), (3, 400, 64), (700, 30, 65), (64, 64, 257), (5000, 40, 3000)])
+def test_sizes_and_ranks(n_rows, n_cols, nnz, K):
+    (rp, ci, val, W, H), ref, bound = _case(n_rows, n_cols, nnz, K, 100 * K + nnz)
+    stream = torch.cuda.current_stream().cuda_stream
+    out = torch.full((nnz + 1,), 7.0, device="cuda")
+    capi.csr_noalloc(n_rows, n_cols, nnz, rp.data_ptr(), ci.data_ptr(), val.data_ptr(), K, W.data_ptr(), H.data_ptr(), out.data_ptr(), stream)
+    planned = torch.full((nnz + 1,), 7.0, device="cuda")
+    plan = capi.Plan.from_device_csr(n_rows, n_cols, nnz, rp.data_ptr(), ci.data_ptr(), K,
+                                     options=capi.PlanOptions.defaults(kernel=capi.KERNEL_ROW_GATHER))
+    plan.execute(val.data_ptr(), W.data_ptr(), H.data_ptr(), planned.data_ptr(), stream)
+    torch.cuda.synchronize()
+    assert ((out[:nnz].cpu().double() - ref).abs() <= bound).all()
+    assert torch.equal(out, planned) and float(out[nnz]) == 7.0
+
+
+# either side of each line of the rule: 2^16 nonzeros, 32 a row, and 2^18 nonzeros at up to 32 floats a row
+@pytest.mark.parametrize("K", [32, 64, 128])
+@pytest.mark.parametrize("n_rows,nnz", [(1024, 65536), (1024, 65537), (3000, 96000), (3000, 96001), (2000, 262144), (2000, 262145)])
+def test_rule(n_rows, nnz, K):
+    (rp, ci, val, W, H), ref, bound = _case(n_rows, 500, nnz, K, nnz + K)
+    out = torch.full((nnz + 1,), 7.0, device="cuda")
+    capi.csr_noalloc(n_rows, 500, nnz, rp.data_ptr(), ci.data_ptr(), val.data_ptr(), K, W.data_ptr(), H.data_ptr(), out.data_ptr(),
+                     torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert ((out[:nnz].cpu().double() - ref).abs() <= bound).all() and float(out[nnz]) == 7.0
