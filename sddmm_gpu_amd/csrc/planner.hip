@@ -548,7 +548,7 @@ void assign_workspace(sddmm_plan *P)
         L.ws_wp = take(L.wp_bytes);
         L.ws_sp_part = take(L.sp_part_bytes);
     }
-    P->ws_softmax = take(row_softmax_workspace_bytes(P->info.nnz));
+    P->ws_softmax = take(row_softmax_workspace_bytes(P->info.nnz, P->info.n_rows));
     P->ws_bytes = at;
 }
 

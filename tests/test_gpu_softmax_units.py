@@ -1,0 +1,53 @@
+"""The row softmax where its units meet the rows: every share size, rows at the limits of each kind of work, huge rows
+that begin, cross and end units, runs of empty rows, in place; against the oracle (relative 1e-5 per entry)."""
+import numpy as np
+import pytest
+import torch
+
+from sddmm_gpu_amd import capi
+from test_gpu_fused import softmax_ok
+
+pytestmark = pytest.mark.gpu
+
+LIMITS = [8, 9, 96, 97, 512, 513, 1024, 1025, 4088, 4089, 17400, 17401, 20000, 1, 70000, 3]
+
+
+# (entries of filler rows, their length): totals from a few thousand to 20 million on the kernel's scale, so shares of 64 to 4096
+@pytest.mark.parametrize("filler,length", [(0, 1), (40000, 7), (300000, 50), (700000, 300), (2000000, 40), (4000000, 700), (16000000, 100)])
+def test_limits_among_fillers(oracle, filler, length):
+    rng = np.random.default_rng(filler + length)
+    n = filler // length
+    lens = np.concatenate([np.full(n // 2, length), np.repeat(LIMITS, 2), np.zeros(3000), np.full(n - n // 2, length), rng.permutation(LIMITS),
+                           np.zeros(500), [1025] * 9, [17401]]).astype(np.int64)
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    x = rng.normal(0, 4, rp[-1]).astype(np.float32)
+    x[rp[np.flatnonzero(lens == 70000)] + 69999] = 60.0
+    want = oracle.row_softmax(rp, x)
+    xd, rpd = torch.from_numpy(x).cuda(), torch.from_numpy(rp).cuda()
+    out = torch.full((len(x) + 1,), float("nan"), device="cuda")
+    capi.row_softmax(len(lens), rpd.data_ptr(), xd.data_ptr(), out.data_ptr())
+    capi.row_softmax(len(lens), rpd.data_ptr(), xd.data_ptr(), xd.data_ptr())
+    torch.cuda.synchronize()
+    softmax_ok(out[:-1].cpu().numpy(), want)
+    assert torch.equal(out[:-1], xd) and bool(torch.isnan(out[-1]))
+
+
+@pytest.mark.parametrize("at", [0, 5, 2000, 19999])
+@pytest.mark.parametrize("value", ["nan", "inf", "-inf"])
+def test_special_values_stay_in_their_row(oracle, at, value):
+    lens = np.array([30, 20000, 700, 0, 5, 3000], dtype=np.int64)
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    x = np.random.default_rng(3).normal(0, 2, rp[-1]).astype(np.float32)
+    want = oracle.row_softmax(rp, x)
+    x[rp[1] + at] = float(value)
+    out = torch.empty(len(x), device="cuda")
+    xd, rpd = torch.from_numpy(x).cuda(), torch.from_numpy(rp).cuda()
+    capi.row_softmax(len(lens), rpd.data_ptr(), xd.data_ptr(), out.data_ptr())
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    touched = slice(rp[1], rp[2])
+    softmax_ok(np.delete(got, np.r_[touched]), np.delete(want, np.r_[touched]))
+    if value == "-inf":
+        softmax_ok(got[touched], oracle.row_softmax(rp, x)[touched])
+    else:
+        assert np.isnan(got[touched]).sum() >= 1
