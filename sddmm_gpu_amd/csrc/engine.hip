@@ -302,7 +302,7 @@ int sddmm_plan_spmm(const sddmm_plan *plan, const float *d_x, const float *d_H, 
         if ((uintptr_t)d_workspace & 255u) return fail(SDDMM_ERR_ARG, "sddmm_plan_spmm: the workspace must be 256-byte aligned");
     }
     if (Ls->sp_on == 2)
-        return launch_spmm_csr_records(I.n_rows, I.nnz, plan->d_row_ptr, plan->d_col, d_x, I.K, d_H, d_Y,
+        return launch_spmm_csr_records(I.n_rows, I.n_cols, I.nnz, plan->d_row_ptr, plan->d_col, d_x, I.K, d_H, d_Y,
                                        d_workspace ? reinterpret_cast<float *>(static_cast<char *>(d_workspace) + Ls->ws_sp_part) : Ls->sa.part, stream);
     if (Ls->sp_on == 3) {
         BlockArgs ba = Ls->ba;

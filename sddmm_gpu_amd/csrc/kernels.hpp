@@ -155,7 +155,7 @@ void launch_spmm_slice(const SpmmArgs &a, int k_slice, int nwaves, int grid, int
 // The product over a plain CSR pattern without atomics (K >= 4, kernels_spmm_csr.hip): d_part holds spmm_csr_records(nnz, K)
 // rows of K floats.  Returns an SDDMM_* code.
 int64_t spmm_csr_records(int64_t nnz, int K);
-int launch_spmm_csr_records(int64_t n_rows, int64_t nnz, const int32_t *d_row_ptr, const int32_t *d_col_ind, const float *d_x, int32_t K,
+int launch_spmm_csr_records(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *d_row_ptr, const int32_t *d_col_ind, const float *d_x, int32_t K,
                             const float *d_H, float *d_Y, float *d_part, void *stream);
 
 // dst[i] = perm[i] >= 0 ? src[perm[i]] : 0 for i < n, on `stream` (a hipStream_t)

@@ -15,7 +15,12 @@
 // What bounds it is the load path (64 bytes per clock and compute unit) and, for an H larger than the caches, the
 // fabric; what bounded the form before (a wave per 256 nonzeros, row by row: three dependent loads for every row)
 // was latency: 429 us at 1.8 M nonzeros and K = 100, 129 us at 18 thousand and K = 16;
-// now 82 and 8 us.
+// now 81 and 8 us.  Where H stays in the caches the vector unit came next to the load path: 64-bit addresses from columns,
+// a comparison of rows and two reads of LDS for each nonzero.  So an entry holds where its row of H begins, as a 32-bit offset
+// while H has them, and a mark where a row of S begins: one read, ahead of use, and four nonzeros of every group at a time
+// without a look at their rows where no mark is among them.  us, before and so: ratings of 5 million nonzeros in 5600
+// columns, K = 16 / 50 / 128 / 200 / 256: 45 / 73 / 107 / 243 / 266 and 37 / 69 / 103 / 186 / 227 (25 TB/s of H rows at K = 128); uniform, 4 million, K = 32
+// 40 and 35; R-MAT, 1.86 million, K = 100 83 and 81.
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include "internal.hpp"
@@ -28,6 +33,7 @@ namespace {
 
 constexpr int kSpmmMost = 512;  // nonzeros of a wave at most
 constexpr int kSpmmUnroll = 4;  // H pieces requested together
+constexpr uint32_t kRowChange = 0x80000000u;
 
 // Zeroes the rows of Y that the product adds to or leaves out: empty rows, and rows cut between workgroups (of 2^shift nonzeros).
 __global__ __launch_bounds__(256)
@@ -101,14 +107,15 @@ void sddmm_spmm_cut_rows_kernel(const int32_t *__restrict__ row_ptr, const float
 
 // RECORDS: part[(2 wg + 0) K ..] takes the part of a row that ends in workgroup wg and began before it, part[(2 wg + 1) K ..]
 // that of a row that goes on behind it.
-template <int G, bool RECORDS>
+// WIDE: H is too large for 32-bit byte offsets.
+template <int G, bool RECORDS, bool WIDE>
 __global__ __launch_bounds__(256)
 void sddmm_spmm_csr_kernel(const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col_ind, const float *__restrict__ x,
                            const float *__restrict__ H, float *Y, float *part, int n_rows, int nnz, int K, int S, int slice_pieces)
 {
     constexpr int NG = 64 / G, U = kSpmmUnroll, NW = 4;
     __shared__ int row_tab[NW][kSpmmMost + 1];
-    __shared__ int2 entry_tab[NW][kSpmmMost];  // column, value
+    __shared__ uint2 entry_tab[NW][kSpmmMost];  // column (WIDE) or where its row of H begins, kRowChange set where a row does; value
     __shared__ vec4u head_sum[NW][G], tail_sum[NW][G];
     __shared__ int head_row[NW], tail_row[NW];  // -1: none
     __shared__ bool tail_started[NW];
@@ -149,45 +156,88 @@ void sddmm_spmm_csr_kernel(const int32_t *__restrict__ row_ptr, const int32_t *_
     if (p0l < nnz) {
         const int p0 = (int)p0l;
         int *rows = row_tab[wave];
-        int2 *entries = entry_tab[wave];
-        for (int i = lane; i < n; i += 64) {
-            const int p = p0 + min(i, nnz - 1 - p0);
-            entries[i] = make_int2(col_ind[p], i < nnz - p0 ? __float_as_int(x[p]) : 0);
-        }
+        uint2 *entries = entry_tab[wave];
+        uint32_t col[kSpmmMost / 64];
+        float val[kSpmmMost / 64];
+#pragma unroll
+        for (int t = 0; t < kSpmmMost / 64; ++t)
+            if (64 * t < n) {
+                const int p = p0 + min(64 * t + lane, nnz - 1 - p0);
+                col[t] = (uint32_t)col_ind[p];
+                val[t] = 64 * t + lane < nnz - p0 ? x[p] : 0.f;
+            }
         const int r0 = rows_of_range(row_ptr, n_rows, nnz, p0, n, rows, lane);
 
-        const float *Hl = H + pc.off;
+#pragma unroll
+        for (int t = 0; t < kSpmmMost / 64; ++t)
+            if (64 * t < n) {
+                const int i = 64 * t + lane;
+                const bool changes = (i & (S - 1)) && rows[i] != rows[i - 1];
+                if (i < n) entries[i] = make_uint2((WIDE ? col[t] : col[t] * (uint32_t)K) | (changes ? kRowChange : 0u), __float_as_uint(val[t]));
+            }
+        __builtin_amdgcn_wave_barrier();  // (LDS operations of one wave complete in order)
         const int gb = g * S;
         const int row_first = rows[gb], row_last = rows[gb + S - 1];
         // does the group's first row begin with the group, its last one end with it
         const bool began = gb > 0 ? rows[gb - 1] != row_first : row_ptr[r0] == p0;
         const bool ended = rows[gb + S] != row_last;
-        auto request = [&](vec4u (&h)[U], int i0) {
+        const char *Hb = reinterpret_cast<const char *>(H);
+        const uint32_t piece_at = (uint32_t)pc.off * 4u;
+        auto read = [&](uint2 (&e)[U], int i0) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) h[u] = *reinterpret_cast<const vec4u *>(Hl + (size_t)entries[gb + i0 + u].x * K);
+            for (int u = 0; u < U; ++u) e[u] = entries[gb + min(i0, S - U) + u];
         };
-        vec4u acc = zero, head = zero;  // head: the part of a row that began before the group
-        vec4u h[U], hn[U];
-        request(h, 0);
-        int cur = row_first;
-        for (int i0 = 0; i0 < S; i0 += U) {
-            if (i0 + U < S) request(hn, i0 + U);
-            __builtin_amdgcn_sched_barrier(0);
+        auto request = [&](vec4u (&h)[U], const uint2 (&e)[U]) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int r = rows[gb + i0 + u];
-                const float xs = __int_as_float(entries[gb + i0 + u].y);
-                if (r != cur) {
+                if constexpr (WIDE) h[u] = *reinterpret_cast<const vec4u *>(H + (size_t)(e[u].x & ~kRowChange) * K + pc.off);
+                else h[u] = *reinterpret_cast<const vec4u *>(Hb + ((e[u].x << 2) + piece_at));  // (the mark is shifted out)
+            }
+        };
+        vec4u acc = zero, head = zero;  // head: the part of a row that began before the group
+        int cur = row_first;
+        auto add_entry = [&](const vec4u &h, const uint2 &e) {
+            const float xs = __uint_as_float(e.y);
+            acc.x = fmaf(xs, h.x, acc.x); acc.y = fmaf(xs, h.y, acc.y);
+            acc.z = fmaf(xs, h.z, acc.z); acc.w = fmaf(xs, h.w, acc.w);
+        };
+        // h, e: the pieces and entries from i0 on; hn, en: the entries after them, whose pieces are requested here; e then
+        // takes the entries after those
+        auto step = [&](vec4u (&h)[U], uint2 (&e)[U], vec4u (&hn)[U], uint2 (&en)[U], int i0) {
+            if (i0 + U < S) request(hn, en);
+            uint2 now[U];
+            uint32_t marks = 0;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                now[u] = e[u];
+                marks |= e[u].x;
+            }
+            read(e, i0 + 2 * U);
+            __builtin_amdgcn_sched_barrier(0);
+            if (__ballot((int)marks < 0) == 0) {  // (in most steps no group's row changes)
+#pragma unroll
+                for (int u = 0; u < U; ++u) add_entry(h[u], now[u]);
+                return;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (now[u].x & kRowChange) {
                     if (cur == row_first && !began) head = acc;
                     else store(cur, acc);
                     acc = zero;
-                    cur = r;
+                    cur = rows[gb + i0 + u];
                 }
-                acc.x = fmaf(xs, h[u].x, acc.x); acc.y = fmaf(xs, h[u].y, acc.y);
-                acc.z = fmaf(xs, h[u].z, acc.z); acc.w = fmaf(xs, h[u].w, acc.w);
+                add_entry(h[u], now[u]);
             }
-#pragma unroll
-            for (int u = 0; u < U; ++u) h[u] = hn[u];
+        };
+        vec4u h0[U], h1[U];
+        uint2 e0[U], e1[U];
+        read(e0, 0);
+        read(e1, U);
+        request(h0, e0);
+        for (int i0 = 0; i0 < S; i0 += 2 * U) {
+            step(h0, e0, h1, e1, i0);
+            if (i0 + U < S) step(h1, e1, h0, e0, i0 + U);
         }
         // The rows cut between the groups: acc is the part of the group's last row; `started` says whether that
         // row's beginning is in it.  A running sum over the groups carries the part on while it stays open.
@@ -308,12 +358,15 @@ CsrShape csr_shape(int64_t nnz, int K)
 }
 
 template <bool RECORDS>
-hipError_t launch_csr(const CsrShape &c, int64_t n_rows, int64_t nnz, const int32_t *row_ptr, const int32_t *col_ind, const float *x, int K,
-                      const float *H, float *Y, float *part, hipStream_t st)
+hipError_t launch_csr(const CsrShape &c, int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_ptr, const int32_t *col_ind, const float *x,
+                      int K, const float *H, float *Y, float *part, hipStream_t st)
 {
     const dim3 grid((unsigned)c.workgroups, (unsigned)c.slices);
-#define SPMM(g) case g: return launch(sddmm_spmm_csr_kernel<g, RECORDS>, grid, dim3(256), 0, st, row_ptr, col_ind, x, H, Y, part, \
-                                      (int)n_rows, (int)nnz, K, 1 << c.shift, c.slice_pieces)
+    const bool wide = n_cols * K >= (int64_t)1 << 30;
+#define SPMM(g)                                                                                                                          \
+    case g:                                                                                                                              \
+        return launch(wide ? sddmm_spmm_csr_kernel<g, RECORDS, true> : sddmm_spmm_csr_kernel<g, RECORDS, false>, grid, dim3(256), 0, st, \
+                      row_ptr, col_ind, x, H, Y, part, (int)n_rows, (int)nnz, K, 1 << c.shift, c.slice_pieces)
     switch (c.G) { SPMM(4); SPMM(8); SPMM(16); SPMM(32); SPMM(64); }
 #undef SPMM
     return hipErrorInvalidValue;
@@ -325,12 +378,12 @@ namespace sddmm {
 
 int64_t spmm_csr_records(int64_t nnz, int K) { return K < 4 ? 0 : 2 * csr_shape(nnz, K).workgroups; }
 
-int launch_spmm_csr_records(int64_t n_rows, int64_t nnz, const int32_t *d_row_ptr, const int32_t *d_col_ind, const float *d_x, int32_t K,
+int launch_spmm_csr_records(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *d_row_ptr, const int32_t *d_col_ind, const float *d_x, int32_t K,
                             const float *d_H, float *d_Y, float *d_part, void *stream)
 {
     const CsrShape c = csr_shape(nnz, K);
     hipStream_t st = (hipStream_t)stream;
-    if (int rc = checked(launch_csr<true>(c, n_rows, nnz, d_row_ptr, d_col_ind, d_x, K, d_H, d_Y, d_part, st))) return rc;
+    if (int rc = checked(launch_csr<true>(c, n_rows, n_cols, nnz, d_row_ptr, d_col_ind, d_x, K, d_H, d_Y, d_part, st))) return rc;
     int per_wave = 64;
     while (per_wave > 1 && n_rows < (int64_t)1024 * per_wave && per_wave / 2 * ((K + 3) / 4) >= 64) per_wave /= 2;
     return checked(launch(sddmm_spmm_cut_rows_kernel, dim3((unsigned)((n_rows + 4 * per_wave - 1) / (4 * per_wave))), dim3(256), 0, st, d_row_ptr,
@@ -356,5 +409,5 @@ extern "C" int sddmm_spmm_csr(int64_t n_rows, int64_t n_cols, int64_t nnz, const
                                 (int)K, c.wg_shift)))
         return rc;
     if (nnz == 0) return SDDMM_OK;
-    return checked(launch_csr<false>(c, n_rows, nnz, d_row_ptr, d_col_ind, d_x, K, d_H, d_Y, nullptr, st));
+    return checked(launch_csr<false>(c, n_rows, n_cols, nnz, d_row_ptr, d_col_ind, d_x, K, d_H, d_Y, nullptr, st));
 }
