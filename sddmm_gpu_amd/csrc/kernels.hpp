@@ -1,6 +1,7 @@
 // Argument blocks and lookup functions shared by the plan builder (planner.hip, planner_tile.hip), the launch code (engine.hip)
 // and the kernel translation units.
 #pragma once
+#include <algorithm>
 #include <cstdint>
 #include <hip/hip_runtime_api.h>
 #include <hip/hip_vector_types.h>
@@ -245,7 +246,8 @@ Variant pick_gather_variant(int K);  // row gather, any K from 4 to 2048
 // batch of 64 and the kernel made for that.
 struct GatherShape { int chunk; bool once; };
 GatherShape gather_shape(int64_t nnz, int64_t n_rows, const Variant &v);
-KernelFn gather_kernel(const Variant &v, bool once);
+inline bool gather_wide(int64_t n_rows, int64_t n_cols, int K) { return std::max(n_rows, n_cols) * K >= (int64_t)1 << 30; }  // byte offsets of 32 bits do not do
+KernelFn gather_kernel(const Variant &v, bool once, bool wide);
 KernelFn generic_kernel();           // row gather, any K
 Variant pick_stream_variant(int K);  // unpadded LDS tile (K % 4 == 0)
 KernelFn stream_kernel(const Variant &v);

@@ -70,8 +70,23 @@ template <int G> constexpr uint64_t group_bits()
     return m;
 }
 
+// Pieces that lie inside every row a variant is picked for (see pick_gather_variant): they need no mask.
+constexpr int whole_pieces(int G, int KPL) { return KPL == 8 ? 4 * G : (KPL - 1) * G; }
+
+// Where a row of W or H begins for a lane that knows its number: the number itself (WIDE), or the offset of its first float,
+// as long as byte offsets have 32 bits: the multiplication is then done once per nonzero, not in every lane and step,
+// and the load takes the matrix's address from scalar registers.  (us with a multiplication in every step and
+// masks on every piece of a ragged row, and so: uniform, 0.9 million nonzeros of 4000 rows, K = 32 / 100 / 200: 9.6 / 23.8 / 41 and 9.1 / 22.3 /
+// 38; 18 thousand, K = 100 / 200: 4.9 / 7.3 and 4.6 / 6.3; where the fabric bounds it the same.)
+template <bool WIDE>
+__device__ __forceinline__ vec4u row_piece_of(const float *m, uint32_t at, int off, int K)
+{
+    if constexpr (WIDE) return *reinterpret_cast<const vec4u *>(m + (size_t)at * K + off);
+    else return *reinterpret_cast<const vec4u *>(reinterpret_cast<const char *>(m) + ((at << 2) + ((uint32_t)off << 2)));
+}
+
 // RAGGED: K is not 4 * G * KPL (its pieces are masked; any K > 4 * G * (KPL - 1) up to 4 * G * KPL, K >= 4).
-template <int G, int KPL, bool RAGGED>
+template <int G, int KPL, bool RAGGED, bool WIDE>
 __global__ __launch_bounds__(kRowGatherBlock)
 void sddmm_gather_kernel(const KArgs a)
 {
@@ -124,6 +139,7 @@ void sddmm_gather_kernel(const KArgs a)
         }
         b.p = a.perm ? a.perm[pos] : pos;
         b.col = a.col_ind[b.p];
+        if constexpr (!WIDE) b.col = (int)((uint32_t)b.col * (uint32_t)K);
         b.v = a.sval ? a.sval[pos] : (a.val ? a.val[b.p] : 1.0f);
         return b;
     };
@@ -132,7 +148,7 @@ void sddmm_gather_kernel(const KArgs a)
 #pragma unroll
     for (int j = 0; j < KPL; ++j) w[0][j] = w[1][j] = vec4u{0.f, 0.f, 0.f, 0.f};
     auto mask_piece = [&](vec4u &v, int j) {
-        if constexpr (RAGGED) {
+        if (RAGGED && (j + 1) * G > whole_pieces(G, KPL)) {
             v.x = first[j] > 0 ? 0.f : v.x;
             v.y = first[j] > 1 ? 0.f : v.y;
             v.z = first[j] > 2 ? 0.f : v.z;
@@ -142,16 +158,16 @@ void sddmm_gather_kernel(const KArgs a)
     // requests the pieces of step I of a batch; changed: the lanes whose nonzero is in another row than the one before
     auto issue = [&]<int I>(std::integral_constant<int, I>, const Batch &b, uint64_t changed) {
         if (changed & (group_bits<G>() << I)) {
-            const float *wr = a.W + (size_t)group_bcast<G, I>(b.row) * K;
+            const uint32_t wr = (uint32_t)group_bcast<G, I>(WIDE ? b.row : b.row * K);
 #pragma unroll
-            for (int j = 0; j < KPL; ++j) w[I & 1][j] = *reinterpret_cast<const vec4u *>(wr + off[j]);
+            for (int j = 0; j < KPL; ++j) w[I & 1][j] = row_piece_of<WIDE>(a.W, wr, off[j], K);
         } else {
 #pragma unroll
             for (int j = 0; j < KPL; ++j) w[I & 1][j] = w[(I & 1) ^ 1][j];
         }
-        const float *hr = a.H + (size_t)group_bcast<G, I>(b.col) * K;
+        const uint32_t hr = (uint32_t)group_bcast<G, I>(b.col);
 #pragma unroll
-        for (int j = 0; j < KPL; ++j) h[I & 1][j] = *reinterpret_cast<const vec4u *>(hr + off[j]);
+        for (int j = 0; j < KPL; ++j) h[I & 1][j] = row_piece_of<WIDE>(a.H, hr, off[j], K);
     };
     // rows of a batch that differ from the row before: inside a group the lane before, for its first lane the
     // group's row at the end of the batch before
@@ -202,7 +218,7 @@ void sddmm_gather_kernel(const KArgs a)
 // another one or not (a copy of the step before would have to wait for that step's).  The sums are the same, bit for bit.
 // us per launch from a graph, the kernel above and this one: 18 thousand nonzeros, K = 16 / 32 / 64 / 128: 3.8 / 4.6 / 4.7 / 5.1
 // and 3.0 / 3.3 / 3.6 / 4.4; R-MAT, 1.86 million, K = 32 / 100 / 256: 43 / 86 / 257 and 30 / 77 / 230.  Where it is chosen: gather_shape.
-template <int G, int KPL, bool RAGGED>
+template <int G, int KPL, bool RAGGED, bool WIDE>
 __global__ __launch_bounds__(kRowGatherBlock)
 void sddmm_gather_once_kernel(const KArgs a)
 {
@@ -238,8 +254,9 @@ void sddmm_gather_once_kernel(const KArgs a)
         rows_of_range(a.row_ptr, a.n_rows, a.nnz, p0, 64, tab, lane);
         row = tab[pos - p0];
     }
+    const int h_at = WIDE ? col : (int)((uint32_t)col * (uint32_t)K), w_at = WIDE ? row : (int)((uint32_t)row * (uint32_t)K);
     auto mask_piece = [&](vec4u &x, int j) {
-        if constexpr (RAGGED) {
+        if (RAGGED && (j + 1) * G > whole_pieces(G, KPL)) {
             x.x = first[j] > 0 ? 0.f : x.x;
             x.y = first[j] > 1 ? 0.f : x.y;
             x.z = first[j] > 2 ? 0.f : x.z;
@@ -250,12 +267,12 @@ void sddmm_gather_once_kernel(const KArgs a)
     auto round = [&]<int BASE, int... I>(std::integer_sequence<int, BASE>, std::integer_sequence<int, I...>) {
         vec4u h[ROUND][KPL], w[ROUND][KPL];
         ((void)[&] {
-            const float *hr = a.H + (size_t)group_bcast<G, BASE + I>(col) * K;
+            const uint32_t hr = (uint32_t)group_bcast<G, BASE + I>(h_at);
 #pragma unroll
-            for (int j = 0; j < KPL; ++j) h[I][j] = *reinterpret_cast<const vec4u *>(hr + off[j]);
-            const float *wr = a.W + (size_t)group_bcast<G, BASE + I>(row) * K;
+            for (int j = 0; j < KPL; ++j) h[I][j] = row_piece_of<WIDE>(a.H, hr, off[j], K);
+            const uint32_t wr = (uint32_t)group_bcast<G, BASE + I>(w_at);
 #pragma unroll
-            for (int j = 0; j < KPL; ++j) w[I][j] = *reinterpret_cast<const vec4u *>(wr + off[j]);
+            for (int j = 0; j < KPL; ++j) w[I][j] = row_piece_of<WIDE>(a.W, wr, off[j], K);
         }(), ...);
         __builtin_amdgcn_sched_barrier(0);
         ((void)[&] {
@@ -373,18 +390,17 @@ GatherShape gather_shape(int64_t nnz, int64_t n_rows, const Variant &v)
     return {64 * per_wave * (kRowGatherBlock / 64), once};
 }
 
-KernelFn gather_kernel(const Variant &v, bool once)
+KernelFn gather_kernel(const Variant &v, bool once, bool wide)
 {
-#define SDDMM_CASE(g, kpl)                                                                 \
-    if (v.G == g && v.KPL == kpl) {                                                        \
-        if (once) return v.exact ? (KernelFn)sddmm_gather_once_kernel<g, kpl, false>       \
-                                 : (KernelFn)sddmm_gather_once_kernel<g, kpl, true>;       \
-        return v.exact ? (KernelFn)sddmm_gather_kernel<g, kpl, false>                      \
-                       : (KernelFn)sddmm_gather_kernel<g, kpl, true>;                      \
-    }
+#define SDDMM_FORM(g, kpl, ragged)                                                                                        \
+    (once ? (wide ? (KernelFn)sddmm_gather_once_kernel<g, kpl, ragged, true> : (KernelFn)sddmm_gather_once_kernel<g, kpl, ragged, false>) \
+          : (wide ? (KernelFn)sddmm_gather_kernel<g, kpl, ragged, true> : (KernelFn)sddmm_gather_kernel<g, kpl, ragged, false>))
+#define SDDMM_CASE(g, kpl) \
+    if (v.G == g && v.KPL == kpl) return v.exact ? SDDMM_FORM(g, kpl, false) : SDDMM_FORM(g, kpl, true);
     SDDMM_CASE(4, 1) SDDMM_CASE(8, 1) SDDMM_CASE(8, 2) SDDMM_CASE(8, 3) SDDMM_CASE(8, 4) SDDMM_CASE(16, 3) SDDMM_CASE(16, 4)
     SDDMM_CASE(32, 3) SDDMM_CASE(32, 4) SDDMM_CASE(64, 3) SDDMM_CASE(64, 4) SDDMM_CASE(64, 8)
 #undef SDDMM_CASE
+#undef SDDMM_FORM
     return nullptr;
 }
 

@@ -28,7 +28,7 @@ extern "C" int sddmm_csr_noalloc(int64_t n_rows, int64_t n_cols, int64_t nnz, co
     a.row_ptr = d_row_ptr; a.n_rows = (int32_t)n_rows;
     a.nnz = (int32_t)nnz; a.K = K; a.n_cols = (int32_t)n_cols; a.tile_x = (int32_t)n_cols;
     const GatherShape shape = gather_shape(nnz, n_rows, var);
-    const KernelFn fn = var.G ? gather_kernel(var, shape.once) : generic_kernel();
+    const KernelFn fn = var.G ? gather_kernel(var, shape.once, gather_wide(n_rows, n_cols, K)) : generic_kernel();
     a.chunk = shape.chunk;
     const int grid = (int)((nnz + a.chunk - 1) / a.chunk);
     const hipError_t e = launch(fn, dim3((unsigned)grid), dim3(kRowGatherBlock), 0, (hipStream_t)stream, a);

@@ -42,7 +42,7 @@ struct Launch {
     int32_t fn_kind = 0;  // 1 stream kernel (row gather), 2 stream kernel with an LDS tile, 3 tile kernel, 4 panel, 5 dense,
                           // 6 row blocks
     int32_t fn_g = 0, fn_kpl = 0, fn_exact = 0, fn_gather = 0, fn_nwaves = 0;
-    int32_t fn_once = 0;    // row gather: the kernel with one batch of 64 a wave
+    int32_t fn_once = 0, fn_wide = 0;  // row gather: the kernel with one batch of 64 a wave; W or H beyond 32-bit byte offsets
     int32_t fn_ragged = 0;  // tile kernel: the form for ranks that are no multiple of its width
     int32_t fn_nwm = 0;  // tile kernel: waves per workgroup that run the launch's matrix-core share (0: none)
     int32_t fused_slices = 0;  // sliced tile launch small enough that its K slices run inside one kernel launch

@@ -132,7 +132,7 @@ int resolve_functions(Launch &L)
     case 1:
     case 2: {
         const Variant v{L.fn_g, L.fn_kpl, L.fn_exact != 0};
-        L.fn = L.fn_kind == 2 ? stream_kernel(v) : v.G ? gather_kernel(v, L.fn_once != 0) : generic_kernel();
+        L.fn = L.fn_kind == 2 ? stream_kernel(v) : v.G ? gather_kernel(v, L.fn_once != 0, L.fn_wide != 0) : generic_kernel();
         if (!L.fn) return fail(SDDMM_ERR_ARG, "plan: no stream kernel for lanes %d x %d", v.G, v.KPL);
         if (L.lds > 0) HIP_TRY(hipFuncSetAttribute((const void *)L.fn, hipFuncAttributeMaxDynamicSharedMemorySize, L.lds));
         return SDDMM_OK;
@@ -291,6 +291,7 @@ int add_row_gather(Ctx &c, const std::vector<int32_t> &rows, bool all_rows)
     const GatherShape shape = gather_shape(n, (int64_t)rows.size(), var);
     a.chunk = shape.chunk;
     L.fn_once = shape.once;
+    L.fn_wide = gather_wide(c.n_rows, c.n_cols, c.K);
     a.K = c.K; a.n_cols = (int32_t)c.n_cols; a.tile_x = (int32_t)c.n_cols;
     L.grid = (int32_t)((n + a.chunk - 1) / a.chunk);
     L.block = kRowGatherBlock;

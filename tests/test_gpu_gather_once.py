@@ -51,3 +51,21 @@ def test_rule(n_rows, nnz, K):
                      torch.cuda.current_stream().cuda_stream)
     torch.cuda.synchronize()
     assert ((out[:nnz].cpu().double() - ref).abs() <= bound).all() and float(out[nnz]) == 7.0
+
+
+@pytest.mark.parametrize("repeat", [40, 12000])  # one batch a wave, several
+def test_h_beyond_32_bit_offsets(repeat):
+    n_rows, n_cols, K = 3, (1 << 22) + 3, 256  # 4.3 GB
+    cols = torch.tensor([n_cols - 1, 0, n_cols - 2, 1 << 21, 5, (1 << 22) - 1, 1 << 22], dtype=torch.int32, device="cuda").repeat(repeat)
+    nnz = cols.numel()
+    rp = torch.tensor([0, 5, 5, nnz], dtype=torch.int32, device="cuda")
+    g = torch.Generator(device="cuda").manual_seed(repeat)
+    W = torch.randn(n_rows, K, generator=g, device="cuda")
+    H = torch.empty(n_cols, K, device="cuda").normal_(generator=g)
+    out = torch.full((nnz + 1,), 7.0, device="cuda")
+    capi.csr_noalloc(n_rows, n_cols, nnz, rp.data_ptr(), cols.data_ptr(), 0, K, W.data_ptr(), H.data_ptr(), out.data_ptr(),
+                     torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    rows = torch.repeat_interleave(torch.arange(n_rows, device="cuda"), (rp[1:] - rp[:-1]).long())
+    terms = W[rows].double() * H[cols.long()].double()
+    assert bool(((out[:nnz].double() - terms.sum(1)).abs() <= K * 2.0 ** -24 * terms.abs().sum(1)).all()) and float(out[nnz]) == 7.0
