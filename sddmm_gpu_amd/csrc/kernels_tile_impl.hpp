@@ -692,18 +692,13 @@ void sddmm_tile_kernel(const TileArgs a)
                 pend_v = RESIDUAL ? v - (h.x + h.y) : (h.x + h.y) * v;
             } else if constexpr (SLICE == 1) {
                 pend_v = h.x + h.y;
-            } else if constexpr (FUSED) {
-                // (The roundings of every slice scaled and added.  With the sums of the sliced launches word counts, 1500 rows, K = 256,
-                // took 23.3 us, so 23.0, and the recommender at K = 512, whose short rows are such a launch, 2920 and 2862.
-                // A value that is no number scales the whole sum: the products could cancel as infinities.)
-                const float dot = h.x + h.y, sum = m.old + dot;
-                pend_v = sum;
-                if constexpr (RESIDUAL) pend_v = last_slice ? (v - dot) - m.old : sum;
-                else if constexpr (VMODE != 2) pend_v = last_slice ? (__builtin_isfinite(v) ? fmaf(dot, v, m.old * v) : sum * v) : sum;
             } else {
                 const Halves sum = add_to(m.old, h, (l & (XORDER ? G / 2 : 1)) != 0);
                 if constexpr (SLICE == 2) pend_v = sum.x + sum.y;
-                else pend_v = RESIDUAL ? (v - (h.x + h.y)) - m.old : VMODE == 2 ? sum.x + sum.y : fmaf(sum.x, v, sum.y * v);
+                else {
+                    pend_v = RESIDUAL ? (v - (h.x + h.y)) - m.old : VMODE == 2 ? sum.x + sum.y : fmaf(sum.x, v, sum.y * v);
+                    if constexpr (FUSED) pend_v = last_slice ? pend_v : sum.x + sum.y;
+                }
             }
             if constexpr (TO_OUT) pend_p = m.p;
             pend_o = m.o;
