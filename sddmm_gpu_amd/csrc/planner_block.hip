@@ -59,8 +59,7 @@ constexpr int64_t kUnitTiles = 4;   // tiles per unit of a row block that is sev
 // Where the line lies, in cells computed per nonzero.  Plans that serve the product as well (attention): 2.5.  us, row
 // blocks against tiles / walk and the softmax's own passes, softmax + product: windows of 128 on either side of 16,384
 // tokens, 1.1 cells, K = 32 / 64 / 128 39 / 53 / 75 against 102 / 135 / 227; with 1.9 cells (40 % left out) 24 / 35 / 52 against
-// 70 / 82 / 124; 2.5 24 / 34 / 51 against 60 / 71 / 101; of 400, 60,000 tokens, 2.9 cells 178 / 275 / 397 against 235 / 313 / 338; at
-// 300 tokens and 40 on either side 12 / 16 / 22 against 22 / 23 / 25.  The SDDMM alone: 1.6, from half a million nonzeros on
+// 70 / 82 / 124; 2.5 24 / 34 / 51 against 60 / 71 / 101; of 400, 60,000 tokens, 2.9 cells 178 / 275 / 397 against 235 / 313 / 338.  The SDDMM alone: 1.6, from half a million nonzeros on
 // (1.1 cells 15 / 21 / 35 against 24 / 40 / 77, 1.9 cells 12 / 17 / 24 against 12 / 17 / 27, 2.5 cells 12 / 17 / 24 against 11 / 14 / 24;
 // 400 thousand nonzeros, 1.6 cells 5.9 / 7.7 / 10.5 against 6.9 / 8.0 / 9.9, 200 thousand 5.6 / 7.4 / 10.1 against 4.8 / 5.6 / 8.3).
 int add_blocks(Ctx &c, const std::vector<int32_t> &rows, bool *taken)
@@ -128,6 +127,24 @@ int add_blocks(Ctx &c, const std::vector<int32_t> &rows, bool *taken)
         }
     });
     if (twice || (double)n_cells > most_cells) return SDDMM_OK;
+
+    // Few blocks: the one with the most tiles that a workgroup computes alone is what the launches take, and the general path's
+    // time grows with the nonzeros instead.  Both in us for softmax + product, from windows of 200 to 4000 tokens, K = 32 / 64 /
+    // 80 / 128: 559 tokens, 83 on either side, 24 full rows (18 tiles) 20 / 27 / 31 / 38 with blocks, 19 / 20 / 23 / 23 without; 1000, 40
+    // (32 tiles) 28 / 38 / 44 / 55 and 19 / 21 / 23 / 27; 334, 167 (11 tiles) 16 / 21 / 23 / 30 and 18 / 20 / 22 / 21; 2000, 100 (7 tiles, the full
+    // rows in parts) 20 / 24 / 27 / 32 and 36 / 40 / 46 / 46; 2000, 24 (4) 18 / 22 / 23 / 28 and 23 / 25 / 28 / 31.
+    if (product && n_blocks <= c.cus && c.opt.dense_blocks != 2) {
+        int64_t most = 0;
+        bool parts = false;
+        for (const Block &B : blocks) {
+            const int64_t n = (int64_t)B.cols.size() / R;
+            parts = parts || n > kBlockTiles;
+            most = std::max(most, n > kBlockTiles ? kUnitTiles : n);
+        }
+        const double K = c.K, with = 6.1 + 0.075 * K + (double)most * (0.4 + 0.0064 * K) + (parts ? 3.5 : 0.0);
+        const double without = 12.7 + 0.042 * K + 1e-6 * (double)c.nnz * (30.0 + 0.16 * K);
+        if (with > without) return SDDMM_OK;
+    }
 
     Launch L;
     L.kind = SDDMM_KERNEL_DENSE_BLOCK;

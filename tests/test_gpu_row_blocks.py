@@ -29,7 +29,7 @@ def plans(d, K, values=True, product=1, **kw):
     dev = torch.device(DEV)
     t = {k: d[k].to(dev) for k in ("row_ptr", "col_ind", "val", "W", "H")}
     out = []
-    for dense in (-1, 0):
+    for dense in (2, 0):  # (2: also where few blocks make the general path the faster one)
         plan = capi.Plan.from_device_csr(d["n_rows"], d["n_cols"], d["nnz"], t["row_ptr"].data_ptr(), t["col_ind"].data_ptr(), K,
                                          options=capi.PlanOptions.defaults(spmm_stream=product, ignore_env=1, dense_blocks=dense, **kw))
         if values:
@@ -190,3 +190,13 @@ def test_row_blocks_saved_and_loaded(tmp_path, n):
             torch.cuda.synchronize()
             got.append((o, Y))
         assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("n,half,every,K,blocks", [(559, 83, 24, 80, False), (1000, 40, 60, 32, False), (2000, 100, 100, 128, True), (334, 167, 38, 32, True)])
+def test_few_row_blocks_only_where_they_are_faster(n, half, every, K, blocks):
+    """Left to itself the planner takes the general path where one workgroup's tiles would be all that runs."""
+    d = window(n, n, half, every, K)
+    t = {k: d[k].to(torch.device(DEV)) for k in ("row_ptr", "col_ind")}
+    plan = capi.Plan.from_device_csr(n, n, d["nnz"], t["row_ptr"].data_ptr(), t["col_ind"].data_ptr(), K,
+                                     options=capi.PlanOptions.defaults(spmm_stream=1, ignore_env=1))
+    assert is_blocks(plan, d) == blocks
