@@ -388,12 +388,12 @@ int sddmm_execute_ws(const sddmm_plan *plan, const float *d_val, const float *d_
  * row-wise softmax of the results in place:
  *   out[p] = exp(s_p - m_r) / sum_{q in row r} exp(s_q - m_r),  s = val .* (W H^T) on S's pattern,
  * m_r the row's largest s.  One extra pass over out (the row totals must be known
- * before any entry can be normalised): every row of up to 16,376 entries is
+ * before any entry can be normalised): every row of up to 17,400 entries is
  * taken into registers whole -- by a lane, a group of lanes, a wave or a
  * workgroup, by its length -- so it is read once and written once; a longer row
- * is cut into pieces of up to 4096 entries whose (max, sum) records are merged by a
- * last kernel.  A plan on row blocks (SDDMM_KERNEL_DENSE_BLOCK on a locally dense
- * pattern) normalises the rows in the launch that computes them.  The layout of the work and those records are kept in fixed
+ * is cut into pieces of up to 16,384 entries whose (max, sum) records are merged by a
+ * second kernel.  A plan on row blocks (SDDMM_KERNEL_DENSE_BLOCK on a locally dense
+ * pattern) normalises the rows in the launch that computes them.  Those records are kept in fixed
  * device arrays of the library (6 MiB per GPU), so softmax calls that overlap
  * in time on one GPU (different streams or threads) race unless they bring a
  * workspace (sddmm_execute_ws); calls on one stream never do.

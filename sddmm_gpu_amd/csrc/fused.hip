@@ -25,21 +25,22 @@ namespace {
 // No staging: a row's loads are all in flight together, and 16 waves per compute unit hide their latency, which is
 // what bounds it until the entries do (the recommender pattern moves 0.8 GB at 3.3 TB/s).  Before this a kernel of its own laid chunks
 // of whole rows out, and rows that had been left over went through lists to a third one.  us, before and now: 18 thousand
-// entries 11.7 and 7.5; R-MAT, 1.9 million 34.7 and 18.1, 28 million 137 and 142; word counts, 0.7 million 18.4 and 14.3; window of 320 a
-// row, 5.2 million 24.7 and 18.2; 3 million rows of one entry 38 and 28; 20 thousand entries spread over 4 million rows 94 and
-// 26; a row of 30 million 331 and 102; recommender, 100 million 238 and 242.  (Maximum and sum by scans over the entries, whatever
-// the rows: 1072 there, bound by the vector ALU.)
+// entries 11.7 and 8.2; R-MAT, 1.9 million 34.7 and 18.5, 28 million 137 and 109, 189 million 541 and 583; word counts, 0.7 million 18.4 and
+// 16.0; window of 320 a row, 5.2 million 24.7 and 19.3; 3 million rows of one entry 38 and 28; 20 thousand entries spread over 4
+// million rows 94 and 22; a row of 30 million 331 and 98; recommender, 100 million 238 and 241.  (Maximum and sum by scans over the
+// entries, whatever the rows: 1072 there, bound by the vector ALU.)
 constexpr int kSmBlock = 256;
 constexpr int kSmWaves = kSmBlock / 64;
 constexpr int kSmLongQ = 17;                             // float4 per thread of the long-row function
 constexpr int kSmLongMax = kSmLongQ * 4 * kSmBlock - 8;  // (less what a misaligned start costs)
 constexpr int kSmByLane = 8, kSmBy8 = 96, kSmBy32 = 512, kSmByWave = 1024;  // row lengths up to which a lane / 8 lanes / 32 lanes / the wave work on a row
-constexpr int kSmRow = 16;                               // (a batch of 64 rows costs about what 1000 entries do; with 8 R-MAT, 1.9 million: 21)
-constexpr int kSmShareMax = 4096;                        // (recommender: 246, with 2048 295)
+constexpr int kSmRow = 4;                                // (with 16 R-MAT, 28 million: 155 instead of 131)
+constexpr int kSmShareMax = 8192;                        // (recommender, rows counting 4: 241, with 4096 258)
 constexpr int kSmLeft = (kSmShareMax - 1) / (kSmByWave + 1) + 1;  // rows of more than kSmByWave entries that start in a share, at most
-static_assert(kSmWaves * kSmShareMax <= kSmLongMax);     // (a piece of a huge row is worked on like a long row)
+constexpr int kSmPieceMax = 16384;                       // a unit of the largest share makes two pieces of a huge row, worked on like long rows
+static_assert(kSmPieceMax <= kSmLongMax);
 constexpr int64_t kSmScaleMax = (int64_t)1 << 32;        // (2^31 entries, and as much for the rows: see softmax_scale)
-constexpr int64_t kSmMaxUnits = kSmScaleMax / (kSmWaves * kSmShareMax);
+constexpr int64_t kSmMaxPieces = kSmScaleMax / kSmPieceMax;
 
 // The scale: row r starts at row_ptr[r] + row * r and the last one ends at `total`.
 struct SoftmaxScale {
@@ -47,6 +48,8 @@ struct SoftmaxScale {
     int row, share;
     __host__ __device__ int unit() const { return kSmWaves * share; }
     __host__ __device__ int64_t units() const { return (total + unit() - 1) / unit(); }
+    __host__ __device__ int piece() const { return unit() < kSmPieceMax ? unit() : kSmPieceMax; }
+    __host__ __device__ int64_t pieces() const { return (total + piece() - 1) / piece(); }
 };
 // Shares: as large as leaves 4096 of them, 64 to kSmShareMax.
 __host__ __device__ inline SoftmaxScale softmax_scale(int64_t nnz, int64_t n_rows)
@@ -59,12 +62,12 @@ __host__ __device__ inline SoftmaxScale softmax_scale(int64_t nnz, int64_t n_row
     return s;
 }
 
-// Per unit: (m, sum) of its piece of a huge row that began before it, [2u], and of one that starts in it, [2u + 1]; the rows
-// themselves plus one (0: none).  The kernels take both arrays as arguments: a caller's workspace (sddmm_execute_ws), or
+// Per unit, or half of one (see piece): (m, sum) of the piece of a huge row that began before it, [2i], and of one that starts
+// in it, [2i + 1]; the rows themselves plus one (0: none).  The kernels take both arrays as arguments: a caller's workspace (sddmm_execute_ws), or
 // these file-scope arrays, 4 + 2 MiB per device, held until the process ends -- softmax calls without a workspace
 // that overlap in time on one device share them and must not (calls on one stream never do).
-static __device__ __align__(256) float2 g_softmax_rec_store[2 * kSmMaxUnits];
-static __device__ __align__(256) int2 g_softmax_rows_store[kSmMaxUnits];
+static __device__ __align__(256) float2 g_softmax_rec_store[2 * kSmMaxPieces];
+static __device__ __align__(256) int2 g_softmax_rows_store[kSmMaxPieces];
 
 template <int GW>
 __device__ __forceinline__ float group_max(float v)
@@ -265,11 +268,12 @@ void sddmm_row_softmax_kernel(const int32_t *__restrict__ row_ptr, int64_t n_row
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n_rows = (int)n_rows_, nnz = row_ptr[n_rows];
     const SoftmaxScale scale = softmax_scale(nnz, n_rows);
-    const int64_t unit = scale.unit(), n_units = scale.units();
+    const int64_t unit = scale.unit(), n_units = scale.units(), piece = scale.piece();
     const bool vec_in = (reinterpret_cast<uintptr_t>(x) & 15u) == 0, vec_out = (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
     for (int64_t u = blockIdx.x; u < n_units; u += gridDim.x) {
         const int64_t k0 = u * unit, k1 = min(scale.total, k0 + unit);
         if (threadIdx.x == 0) n_left = 0;
+        if (threadIdx.x * piece < k1 - k0) rec_rows[k0 / piece + threadIdx.x] = make_int2(0, 0);
         __syncthreads();
         const int64_t s0 = k0 + wave * scale.share, s1 = min(k1, s0 + scale.share);
         if (s0 < s1) {
@@ -286,35 +290,37 @@ void sddmm_row_softmax_kernel(const int32_t *__restrict__ row_ptr, int64_t n_row
             }
         }
         __syncthreads();
-        int2 huge = make_int2(0, 0);
         const int n = n_left;
 #pragma unroll 1
         for (int w = -1; w < n; ++w) {  // (-1: the row that began before the unit, if it is a huge one)
             const int r = w < 0 ? first_row : left[w];
-            int64_t b = row_ptr[r], e = row_ptr[r + 1];
-            const int64_t at = b + (int64_t)scale.row * r;
-            float2 *piece = nullptr;
-            if (w < 0 && (at >= k0 || e - b <= kSmLongMax || at + (e - b) <= k0)) continue;
-            if (e - b > kSmLongMax) {  // what lies in this unit
-                piece = &rec[2 * u + (w < 0 ? 0 : 1)];
-                (w < 0 ? huge.x : huge.y) = r + 1;
-                e = min(e, b + (k1 - at));
-                b += max((int64_t)0, k0 - at);
+            const int64_t b = row_ptr[r], len = row_ptr[r + 1] - b, at = b + (int64_t)scale.row * r;
+            const bool huge = len > kSmLongMax;
+            if (w < 0 && (at >= k0 || !huge || at + len <= k0)) continue;
+            if (len <= 4 * 4 * kSmBlock - 8) {
+                softmax_long_row<4>(x, out, b, b + len, nnz, vec_in, vec_out, red, nullptr);
+                continue;
             }
-            if (e - b <= 4 * 4 * kSmBlock - 8) softmax_long_row<4>(x, out, b, e, nnz, vec_in, vec_out, red, piece);
-            else softmax_long_row<kSmLongQ>(x, out, b, e, nnz, vec_in, vec_out, red, piece);
+            // (of a huge row what lies in this unit, piece by piece)
+            const int64_t stop = huge ? min(len, k1 - at) : len;
+            for (int64_t p = huge ? max((int64_t)0, k0 - at) : 0; p < stop;) {
+                const int64_t i = (at + p) / piece, e = huge ? min(stop, (i + 1) * piece - at) : len;
+                const int which = at < i * piece ? 0 : 1;
+                if (huge && threadIdx.x == 0) (which ? rec_rows[i].y : rec_rows[i].x) = r + 1;
+                softmax_long_row<kSmLongQ>(x, out, b + p, b + e, nnz, vec_in, vec_out, red, huge ? &rec[2 * i + which] : nullptr);
+                p = e;
+            }
         }
-        if (threadIdx.x == 0) rec_rows[u] = huge;
         __syncthreads();  // (the next unit writes left, n_left and first_row)
     }
 }
 
 // (m, sum) of the huge row of len entries that starts at `at` on the scale from the records of its pieces: the second
-// one of the unit it starts in, the first ones of the others; every wave of the workgroup computes the same pair.
-__device__ __forceinline__ float2 merged_record(const float2 *__restrict__ rec, int64_t at, int64_t len, int unit)
+// one of the piece it starts in, the first ones of the others; every wave of the workgroup computes the same pair.
+__device__ __forceinline__ float2 merged_record(const float2 *__restrict__ rec, int64_t at, int64_t len, int piece)
 {
     const int lane = threadIdx.x & 63;
-    const int64_t ua = at / unit, ub = (at + len - 1) / unit;
+    const int64_t ua = at / piece, ub = (at + len - 1) / piece;
     float m = -INFINITY, s = 0.f;
     for (int64_t k = ua + lane; k <= ub; k += 64) {
         const float2 r = rec[2 * k + (k == ua ? 1 : 0)];
@@ -346,32 +352,31 @@ __device__ __forceinline__ void scale_range(float *out, int64_t b, int64_t e, fl
     }
 }
 
-// Second kernel: the pieces of huge rows are scaled to the whole row's maximum and sum.  A workgroup takes consecutive
-// ones, which mostly are of one row, and merges that row's records once.
+// Second kernel: the pieces of huge rows are scaled to the whole row's maximum and sum.  A workgroup takes four consecutive
+// pieces at a time, which mostly are of one row, and merges that row's records once; four and not an equal range, since
+// huge rows may lie together (R-MAT 2^22, 189 million: 583 us
+// in all, and 855 with a range for each of 256 workgroups).
 __global__ __launch_bounds__(kSmBlock)
 void sddmm_row_softmax_merge_kernel(const int32_t *__restrict__ row_ptr, int64_t n_rows, float *out, const float2 *__restrict__ rec,
                                     const int2 *__restrict__ rec_rows)
 {
     const SoftmaxScale scale = softmax_scale(row_ptr[n_rows], n_rows);
-    const int64_t unit = scale.unit(), n_units = scale.units(), per = (n_units + gridDim.x - 1) / gridDim.x;
-    const int64_t first = blockIdx.x * per, stop = min(n_units, first + per);
+    const int64_t size = scale.piece(), n_pieces = scale.pieces();
+    constexpr int kTogether = 4;
     int merged_row = -1;
     float2 all = make_float2(0.f, 1.f);
-    for (int64_t base = first; base < stop; base += kSmBlock) {
-        int2 mine = make_int2(0, 0);
-        if (base + threadIdx.x < stop) mine = rec_rows[base + threadIdx.x];
-        if (!__syncthreads_or(mine.x | mine.y)) continue;
-        for (int64_t u = base; u < min(stop, base + kSmBlock); ++u) {
+    for (int64_t base = (int64_t)blockIdx.x * kTogether; base < n_pieces; base += (int64_t)gridDim.x * kTogether) {
+        for (int64_t u = base; u < min(n_pieces, base + kTogether); ++u) {
             const int2 rows = rec_rows[u];
             for (int which = 0; which < 2; ++which) {
                 const int r = (which ? rows.y : rows.x) - 1;
                 if (r < 0) continue;
                 const int64_t rb = row_ptr[r], re = row_ptr[r + 1];
                 const int64_t at = rb + (int64_t)scale.row * r;
-                if (r != merged_row) all = merged_record(rec, at, re - rb, (int)unit);
+                if (r != merged_row) all = merged_record(rec, at, re - rb, (int)size);
                 merged_row = r;
                 const float2 piece = rec[2 * u + which];
-                scale_range(out, rb + max((int64_t)0, u * unit - at), min(re, rb + ((u + 1) * unit - at)), expf(piece.x - all.x) / all.y);
+                scale_range(out, rb + max((int64_t)0, u * size - at), min(re, rb + ((u + 1) * size - at)), expf(piece.x - all.x) / all.y);
             }
         }
     }
@@ -407,7 +412,7 @@ static int softmax_store(float2 **rec, int2 **rows)
 
 int64_t row_softmax_workspace_bytes(int64_t nnz, int64_t n_rows)
 {
-    return ((softmax_scale(nnz, n_rows).units() * 24 + 255) / 256) * 256;  // two float2 and one int2 per unit
+    return ((softmax_scale(nnz, n_rows).pieces() * 24 + 255) / 256) * 256;  // two float2 and one int2 per piece
 }
 
 int launch_row_softmax(int64_t n_rows, const int32_t *d_row_ptr, const float *d_x, float *d_out, void *stream, void *d_ws, int64_t nnz)
@@ -415,16 +420,16 @@ int launch_row_softmax(int64_t n_rows, const int32_t *d_row_ptr, const float *d_
     if (n_rows <= 0) return SDDMM_OK;
     float2 *rec = nullptr;
     int2 *rows = nullptr;
-    if (d_ws) {  // [2 * units] records, then [units] pairs of rows
+    if (d_ws) {  // [2 * pieces] records, then [pieces] pairs of rows
         rec = static_cast<float2 *>(d_ws);
-        rows = reinterpret_cast<int2 *>(rec + 2 * softmax_scale(nnz, n_rows).units());
+        rows = reinterpret_cast<int2 *>(rec + 2 * softmax_scale(nnz, n_rows).pieces());
     } else if (int rc = softmax_store(&rec, &rows)) {
         return rc;
     }
     // (the entry count lives on the device: the grids are sized for the machine, the kernels stride over it)
     const hipStream_t st = (hipStream_t)stream;
     hipError_t e = launch(sddmm_row_softmax_kernel, dim3(256 * 8), dim3(kSmBlock), 0, st, d_row_ptr, n_rows, d_x, d_out, rec, rows);
-    if (e == hipSuccess) e = launch(sddmm_row_softmax_merge_kernel, dim3(256), dim3(kSmBlock), 0, st, d_row_ptr, n_rows, d_out, rec, rows);
+    if (e == hipSuccess) e = launch(sddmm_row_softmax_merge_kernel, dim3(256 * 4), dim3(kSmBlock), 0, st, d_row_ptr, n_rows, d_out, rec, rows);
     if (e != hipSuccess) return fail(SDDMM_ERR_HIP, "sddmm_row_softmax: %s", hipGetErrorString(e));
     return SDDMM_OK;
 }
