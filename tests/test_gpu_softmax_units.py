@@ -51,3 +51,38 @@ def test_special_values_stay_in_their_row(oracle, at, value):
         softmax_ok(got[touched], oracle.row_softmax(rp, x)[touched])
     else:
         assert np.isnan(got[touched]).sum() >= 1
+
+
+# Pieces are 256 entries without filler rows and 1024 with them; a lane merges every 64th piece of a row.
+@pytest.mark.parametrize("filler,masked", [(0, [(0, 700)]), (0, [(16384, 18000)]), (0, [(0, 19999)]), (0, [(500, 20000)]),
+                                           (1200000, [(0, 5000)]), (1200000, [(0, 9000), (12000, 20000)])])
+def test_huge_row_with_pieces_all_masked(oracle, filler, masked):
+    """Pieces of a huge row in which every entry is minus infinity have weight 0 and leave the others theirs."""
+    lens = np.array([30, 20000, 700] + [300] * (filler // 300), dtype=np.int64)
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    x = np.random.default_rng(3).normal(0, 2, rp[-1]).astype(np.float32)
+    for b, e in masked:
+        x[rp[1] + b:rp[1] + e] = -np.inf
+    out = torch.empty(len(x), device="cuda")
+    xd, rpd = torch.from_numpy(x).cuda(), torch.from_numpy(rp).cuda()
+    capi.row_softmax(len(lens), rpd.data_ptr(), xd.data_ptr(), out.data_ptr())
+    torch.cuda.synchronize()
+    softmax_ok(out.cpu().numpy(), oracle.row_softmax(rp, x))
+
+
+@pytest.mark.parametrize("value", [float("nan"), -float("inf")])
+def test_huge_row_without_weights(oracle, value):
+    """A huge row of nothing but minus infinity, and one with a piece of nothing but NaN, are NaN throughout."""
+    lens = np.array([30, 20000, 700], dtype=np.int64)
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    x = np.random.default_rng(3).normal(0, 2, rp[-1]).astype(np.float32)
+    want = oracle.row_softmax(rp, x)
+    b, e = (0, 20000) if np.isinf(value) else (20 * 256 - 34, 22 * 256 - 34)  # (the row starts at 30 + 4 on the kernel's scale)
+    x[rp[1] + b:rp[1] + e] = value
+    out = torch.empty(len(x), device="cuda")
+    xd, rpd = torch.from_numpy(x).cuda(), torch.from_numpy(rp).cuda()
+    capi.row_softmax(len(lens), rpd.data_ptr(), xd.data_ptr(), out.data_ptr())
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert np.isnan(got[rp[1]:rp[2]]).all()
+    softmax_ok(np.delete(got, np.r_[rp[1]:rp[2]]), np.delete(want, np.r_[rp[1]:rp[2]]))
