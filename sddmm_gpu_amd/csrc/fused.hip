@@ -324,16 +324,16 @@ __device__ __forceinline__ float2 merged_record(const float2 *__restrict__ rec, 
     float m = -INFINITY, s = 0.f;
     for (int64_t k = ua + lane; k <= ub; k += 64) {
         const float2 r = rec[2 * k + (k == ua ? 1 : 0)];
-        if (r.y == 0.f) continue;  // (a piece of nothing but -inf: its terms vanish, and -inf - -inf would be a NaN)
         const float mn = fmaxf(m, r.x);
-        s = s * expf(m - mn) + r.y * expf(r.x - mn);  // (exp(-inf - finite) = 0 for the first record)
+        // (no record yet, or one of nothing but -inf: its term must vanish without producing inf - inf)
+        s = (s == 0.f ? 0.f : s * expf(m - mn)) + (r.y == 0.f ? 0.f : r.y * expf(r.x - mn));
         m = mn;
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         const float m2 = __shfl_xor(m, off), s2 = __shfl_xor(s, off);
         const float mn = fmaxf(m, m2);
-        // (a lane without records holds (-inf, 0): its term must vanish without producing inf - inf; one of NaNs alone (-inf, NaN))
+        // (a lane without records holds (-inf, 0), one with a record of NaNs alone (-inf, NaN))
         const float t1 = s == 0.f ? 0.f : s * expf(m - mn), t2 = s2 == 0.f ? 0.f : s2 * expf(m2 - mn);
         s = t1 + t2;
         m = mn;
