@@ -23,12 +23,13 @@ namespace {
 //        piece's own maximum m and leaves (m, sum) and the row in a record of the unit; a second kernel, which finds
 //        nothing to do on most matrices, merges the records of each huge row and scales its pieces.
 // No staging: a row's loads are all in flight together, and 16 waves per compute unit hide their latency, which is
-// what bounds it until the entries do (the recommender pattern moves 0.8 GB at 3.3 TB/s).  Before this a kernel of its own laid chunks
-// of whole rows out, and rows that had been left over went through lists to a third one.  us, before and now: 18 thousand
-// entries 11.7 and 8.2; R-MAT, 1.9 million 34.7 and 18.5, 28 million 137 and 109, 189 million 541 and 583; word counts, 0.7 million 18.4 and
-// 16.0; window of 320 a row, 5.2 million 24.7 and 19.3; 3 million rows of one entry 38 and 28; 20 thousand entries spread over 4
-// million rows 94 and 22; a row of 30 million 331 and 98; recommender, 100 million 238 and 241.  (Maximum and sum by scans over the
-// entries, whatever the rows: 1072 there, bound by the vector ALU.)
+// what bounds it until the entries do (the recommender pattern moves 0.8 GB at 3.5 TB/s).  Before this a kernel of its own
+// laid chunks of whole rows out, and rows that had been left over went through lists to a third one.  us, before and now: 18
+// thousand entries 11.8 and 8.9; R-MAT, 1.9 million 34 and 18, 28 million 134 and 111, 84 million 297 and 266, 189 million
+// 526 and 526; word counts, 0.7 million 18.5 and 16.5; window of 320 a row, 5.2 million 24 and 19; 3 million rows of one
+// entry 38 and 30; 20 thousand entries spread over 4 million rows 93 and 25; a row of 30 million 328 and 93; recommender,
+// 100 million 235 and 231.  (Maximum and sum by scans over the entries, whatever the rows: 1072 there, bound by the vector
+// ALU.)
 constexpr int kSmBlock = 256;
 constexpr int kSmWaves = kSmBlock / 64;
 constexpr int kSmLongQ = 17;                             // float4 per thread of the long-row function
@@ -355,8 +356,8 @@ __device__ __forceinline__ void scale_range(float *out, int64_t b, int64_t e, fl
 
 // Second kernel: the pieces of huge rows are scaled to the whole row's maximum and sum.  A workgroup takes four consecutive
 // pieces at a time, which mostly are of one row, and merges that row's records once; four and not an equal range, since
-// huge rows may lie together (R-MAT 2^22, 189 million: 583 us
-// in all, and 855 with a range for each of 256 workgroups).
+// huge rows may lie together (R-MAT 2^22, 189 million, the whole softmax: 583 us with 1024 workgroups, 855 with a range for
+// each of 256).
 __global__ __launch_bounds__(kSmBlock)
 void sddmm_row_softmax_merge_kernel(const int32_t *__restrict__ row_ptr, int64_t n_rows, float *out, const float2 *__restrict__ rec,
                                     const int2 *__restrict__ rec_rows)
@@ -427,10 +428,18 @@ int launch_row_softmax(int64_t n_rows, const int32_t *d_row_ptr, const float *d_
     } else if (int rc = softmax_store(&rec, &rows)) {
         return rc;
     }
-    // (the entry count lives on the device: the grids are sized for the machine, the kernels stride over it)
+    // The entry count lives on the device: the grids are sized by the rows, the kernels stride over the entries.  1024
+    // workgroups run at a time, and a unit of heavy rows takes long: the more workgroups the units are dealt to, the more
+    // evenly the machine is filled at the end, but a workgroup that finds nothing costs its launch.  us with 2048 / 4096 /
+    // 8192 workgroups: R-MAT 2^22, 189 million entries 574 / 544 / 536, 2^21, 84 million 297 / 282 / 282; recommender, 480
+    // thousand rows 239 / 231 / 231; 4096 rows, 18 thousand entries 8.8 / 8.9 / 11.1, 167 thousand 9.4 / 10.9.  With 1024 /
+    // 4096 for the merge: 574 / 564, 297 / 275, 4096 rows 8.8 / 10.8.  What the larger grids cost a matrix of a million
+    // rows or more with next to no entries: 4 million rows, 20 thousand entries 19.2 and 22.2.
+    const int main_groups = n_rows >= (int64_t)1 << 20 ? 8192 : n_rows >= (int64_t)1 << 18 ? 4096 : 2048;
+    const int merge_groups = n_rows >= (int64_t)1 << 20 ? 4096 : 1024;
     const hipStream_t st = (hipStream_t)stream;
-    hipError_t e = launch(sddmm_row_softmax_kernel, dim3(256 * 8), dim3(kSmBlock), 0, st, d_row_ptr, n_rows, d_x, d_out, rec, rows);
-    if (e == hipSuccess) e = launch(sddmm_row_softmax_merge_kernel, dim3(256 * 4), dim3(kSmBlock), 0, st, d_row_ptr, n_rows, d_out, rec, rows);
+    hipError_t e = launch(sddmm_row_softmax_kernel, dim3(main_groups), dim3(kSmBlock), 0, st, d_row_ptr, n_rows, d_x, d_out, rec, rows);
+    if (e == hipSuccess) e = launch(sddmm_row_softmax_merge_kernel, dim3(merge_groups), dim3(kSmBlock), 0, st, d_row_ptr, n_rows, d_out, rec, rows);
     if (e != hipSuccess) return fail(SDDMM_ERR_HIP, "sddmm_row_softmax: %s", hipGetErrorString(e));
     return SDDMM_OK;
 }

@@ -86,3 +86,19 @@ def test_huge_row_without_weights(oracle, value):
     got = out.cpu().numpy()
     assert np.isnan(got[rp[1]:rp[2]]).all()
     softmax_ok(np.delete(got, np.r_[rp[1]:rp[2]]), np.delete(want, np.r_[rp[1]:rp[2]]))
+
+
+# (the grids grow at 2^18 and at 2^20 rows; a row of 600,000 entries alone is more pieces than the smaller merge grid has workgroups)
+@pytest.mark.parametrize("rows", [2 ** 18 - 40, 2 ** 18, 2 ** 20 - 40, 2 ** 20])
+def test_many_rows(oracle, rows):
+    rng = np.random.default_rng(rows)
+    lens = rng.integers(0, 4, rows)
+    lens[[5, rows // 2, rows // 2 + 1, rows - 2]] = 600000, 17401, 3000, 40000
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    x = rng.normal(0, 4, rp[-1]).astype(np.float32)
+    xd, rpd = torch.from_numpy(x).cuda(), torch.from_numpy(rp).cuda()
+    out = torch.full((len(x) + 1,), float("nan"), device="cuda")
+    capi.row_softmax(rows, rpd.data_ptr(), xd.data_ptr(), out.data_ptr())
+    torch.cuda.synchronize()
+    softmax_ok(out[:-1].cpu().numpy(), oracle.row_softmax(rp, x))
+    assert bool(torch.isnan(out[-1]))
