@@ -263,9 +263,11 @@ typedef struct sddmm_plan_options {
     int32_t gather_sink;        /* 0/1 padding of that stream flagged and dropped   [SDDMM_GATHER_SINK]   */
     int32_t row_padded;         /* 0/1 ROW_GATHER plans use the padded gather kernel [SDDMM_ROW_PADDED]    */
     int32_t unpadded_tile;      /* 0/1 LDS_TILE plans use the unpadded stream kernel [SDDMM_UNPADDED_TILE] */
-    int32_t dense_blocks;       /* 0/1 dense core on the matrix cores, in bf16 parts that add up to the
-                                   fp32 operands (-1: by K, and all of a locally dense pattern; 2: of one however
-                                   small; 0: every product in fp32)                 [SDDMM_DENSE]      */
+    int32_t dense_blocks;       /* matrix cores, in bf16 parts that add up to the fp32 operands: 0 not at all
+                                   (every product in fp32); -1 for the dense core of a power-law matrix by K,
+                                   and for all of a locally dense pattern (its row blocks); 1 for the dense core
+                                   at any K, row blocks where there is none; 2 as 1, with row blocks also where
+                                   they are so few that the other kernels are faster     [SDDMM_DENSE]      */
     int32_t dense_permille;     /* least fill of a dense block, in 1/1000           [SDDMM_DENSE_PERMILLE] */
     int32_t dense_rb_group;     /* row blocks swept together by one die             [SDDMM_DENSE_RB_GROUP] */
     int32_t fuse_slices;        /* 0/1 the K slices of a launch run inside one kernel

@@ -783,7 +783,7 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
     // Plans that also serve the product with the dense factor keep the whole matrix on its column tiles below
     // 512: behind a dense core that product walks the CSR pattern (98 M nonzeros, K = 128: 2.98 ms against 1.46).
     // The threshold is flat: 3118 / 3113 / 3166 / 3284 us at K = 512 for 40 / 30 / 22 / 16 % filled.
-    const bool want_dense = (opt.dense_blocks > 0 && opt.dense_blocks != 2) || (opt.dense_blocks < 0 && K >= (opt.spmm_stream > 0 ? 512 : 384));
+    const bool want_dense = opt.dense_blocks > 0 || (opt.dense_blocks < 0 && K >= (opt.spmm_stream > 0 ? 512 : 384));
     if (kernel == SDDMM_KERNEL_HYBRID && want_dense && K % 32 == 0 && kt / 4 > 16 &&
         (int64_t)n_rows * (K / 4) <= (int64_t)UINT32_MAX && (int64_t)n_cols * (K / 4) <= (int64_t)UINT32_MAX) {
         const double threshold = (double)(opt.dense_permille > 0 ? opt.dense_permille : 300) / 1000.0;

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from sddmm_gpu_amd import capi
+from sddmm_gpu_amd import capi, synth
 from test_gpu_parity import _dict_of, check
 
 pytestmark = pytest.mark.gpu
@@ -200,3 +200,19 @@ def test_few_row_blocks_only_where_they_are_faster(n, half, every, K, blocks):
     plan = capi.Plan.from_device_csr(n, n, d["nnz"], t["row_ptr"].data_ptr(), t["col_ind"].data_ptr(), K,
                                      options=capi.PlanOptions.defaults(spmm_stream=1, ignore_env=1))
     assert is_blocks(plan, d) == blocks
+
+
+@pytest.mark.parametrize("dense", [-1, 0, 1, 2, 3])
+def test_what_dense_blocks_asks_for(dense):
+    """Every value but 0 leaves the dense core on (-1: from K = 384 on), and row blocks; 2 takes row blocks where they are few, too."""
+    def plan(d, K, **kw):
+        t = {k: d[k].to(torch.device(DEV)) for k in ("row_ptr", "col_ind")}
+        return capi.Plan.from_device_csr(d["n_rows"], d["n_cols"], d["nnz"], t["row_ptr"].data_ptr(), t["col_ind"].data_ptr(), K,
+                                         options=capi.PlanOptions.defaults(ignore_env=1, dense_blocks=dense, **kw))
+    ratings = synth.make(3, 0.03, K=4, device=DEV)
+    for K in (128, 512):
+        core = plan(ratings, K, dense_min_nnz=1000, split_min_nnz=0).info()["dense_nnz"]
+        assert (core > ratings["nnz"] // 10) == (dense > 0 or (dense < 0 and K == 512)) and core < ratings["nnz"]
+    many, few = window(2100, 2100, 300, 1000, 32), window(1000, 1000, 40, 60, 32)
+    assert is_blocks(plan(many, 32, spmm_stream=1), many) == (dense != 0)
+    assert is_blocks(plan(few, 32, spmm_stream=1), few) == (dense == 2)
