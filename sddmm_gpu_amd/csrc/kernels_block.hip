@@ -40,6 +40,12 @@ using namespace sddmm;
 namespace {
 
 constexpr int kRows = kBlockRows;     // 32
+// The product's X is multiplied by a power of two before it is cut into parts and its sums are divided by it: parts then hold
+// every bit of an X down to the smallest subnormal.  Softmax weights have all sizes below 1: one whose score lies 77 below
+// its row's maximum is less than 2^-110, from where on the unscaled parts lost bits, and a single one sent its unit to the
+// loop below that goes entry by entry.  At the other end a wave's sum of 2^84 or more now takes that loop (before 2^128).
+// us, 16,384 tokens, K = 64, scores of standard deviation 1 / 8 / 12 / 40: 23.7 / 316 / 457 / 457 unscaled, 23.9 / 23.5 / 23.5 / 23.5.
+constexpr float kXScale = 0x1p40f;
 constexpr int kXRow = 16 + 4;         // floats per row of half a tile of X in LDS: 16 rows' 16-byte reads fall into different banks
 
 // the product's LDS: the waves' tiles of X or their sums, then masks and columns of a unit's tiles
@@ -328,7 +334,7 @@ void sddmm_block_spmm_kernel(const BlockArgs a)
     };
     auto stage = [&](int s, int u) {  // (what a row does not have becomes 0 here: the entries need not have arrived before)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) xt[(xr0 + 4 * i) * kXRow + xc] = (info[u * kRows + xr0 + 4 * i].x >> (16 * s + xc)) & 1u ? x[i] : 0.f;
+        for (int i = 0; i < 8; ++i) xt[(xr0 + 4 * i) * kXRow + xc] = (info[u * kRows + xr0 + 4 * i].x >> (16 * s + xc)) & 1u ? x[i] * kXScale : 0.f;
     };
     // Operand element e of step s is column 16 s + 8 kh + e of the tile.
     auto request = [&](int q, int u) {
@@ -377,7 +383,7 @@ void sddmm_block_spmm_kernel(const BlockArgs a)
 #pragma unroll
     for (int n = 0; n < KT; ++n)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) bad |= !(fabsf(sum[n][v]) < INFINITY);
+        for (int v = 0; v < 16; ++v) bad |= !(fabsf(sum[n][v]) < 0x1p124f);  // (the sum of all waves' must not overflow either)
     float *record = a.part + (size_t)max(unit.w, 0) * (KT * 1024);
     auto put = [&](int n, int v, int lane_of, float y) {  // result register v of lane lane_of, elements 32 n on
         if (unit.w >= 0) {
@@ -431,7 +437,7 @@ void sddmm_block_spmm_kernel(const BlockArgs a)
             float y = lds[n * 1024 + v * 64 + lane];
 #pragma unroll
             for (int w = 1; w < 4; ++w) y += lds[(w * KT + n) * 1024 + v * 64 + lane];
-            put(n, v, lane, y);
+            put(n, v, lane, y * (1.0f / kXScale));
         }
 }
 

@@ -216,3 +216,34 @@ def test_what_dense_blocks_asks_for(dense):
     many, few = window(2100, 2100, 300, 1000, 32), window(1000, 1000, 40, 60, 32)
     assert is_blocks(plan(many, 32, spmm_stream=1), many) == (dense != 0)
     assert is_blocks(plan(few, 32, spmm_stream=1), few) == (dense == 2)
+
+
+@pytest.mark.parametrize("n,half,every,K", [(700, 40, 50, 64), (1500, 30, 400, 80)])
+def test_product_with_small_and_large_weights(oracle, n, half, every, K):
+    """X times a power of two gives Y times it, bit for bit, where nothing is subnormal: one path for weights of any size.
+    At the ends of the range the product is right."""
+    d = window(n, n, half, every, K)
+    t, (plan, _) = plans(d, K, values=False)
+    assert is_blocks(plan, d)
+    row, col, H = d["row_ind"].long(), d["col_ind"].long(), d["H"].double()
+
+    def product(x):
+        xd, Y = x.to(DEV), torch.full((n, K), float("nan"), device=DEV)
+        plan.spmm(xd.data_ptr(), t["H"].data_ptr(), Y.data_ptr())
+        torch.cuda.synchronize()
+        return Y.cpu()
+    g = torch.Generator().manual_seed(5)
+    x = (0.5 + 0.5 * torch.rand(d["nnz"], generator=g)) * (2 * torch.randint(0, 2, (d["nnz"],), generator=g) - 1)
+    Y = product(x)
+    for e in (-112, -60, 40, 70):
+        assert torch.equal(product(torch.ldexp(x, torch.tensor(e))), torch.ldexp(Y, torch.tensor(e))), e
+    # a few that vanish beside the others
+    mixed = torch.where(torch.rand(d["nnz"], generator=g) < 0.01, torch.ldexp(x, torch.tensor(-112)), x)
+    assert torch.equal(product(torch.ldexp(mixed, torch.tensor(30))), torch.ldexp(product(mixed), torch.tensor(30)))
+    deg = np.diff(d["row_ptr"].numpy())
+    for e in (-147, -125, 78, 83, 85, 88, 110, 118):
+        xe = torch.ldexp(x, torch.tensor(e))
+        mag = torch.zeros(n, K, dtype=torch.float64).index_add_(0, row, xe.double().abs()[:, None] * H.abs()[col])
+        ref = torch.zeros(n, K, dtype=torch.float64).index_add_(0, row, xe.double()[:, None] * H[col])
+        bound = 1e-5 * torch.from_numpy(np.sqrt(np.maximum(deg, 1)))[:, None] * mag + 2.0 ** -149 * torch.from_numpy(deg)[:, None]
+        assert bool(((product(xe).double() - ref).abs() <= bound).all()), e
