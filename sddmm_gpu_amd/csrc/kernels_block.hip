@@ -5,8 +5,8 @@
 // entry lies.  No list of nonzeros, no column per nonzero: 384 bytes per tile of up to 1024 nonzeros.
 //
 // Arithmetic: fp32 operands as three bf16 parts, eight products of parts, added up as in add_products (bf16_parts.hpp).
-// What parts cannot carry (infinities, NaNs, sums beyond the range, bits under bf16's smallest subnormal) is
-// found and computed once more in fp32.
+// What parts cannot carry is found and computed once more: with scaled operands where bits lie under bf16's smallest subnormal,
+// in fp32 where there are infinities, NaNs or sums beyond the range.
 //
 // A unit is a row block and a range of its tiles, dealt tile by tile to the four waves of a workgroup.  A row block of
 // long rows (tokens that look at all others) is several units.
@@ -40,12 +40,15 @@ using namespace sddmm;
 namespace {
 
 constexpr int kRows = kBlockRows;     // 32
-// The product's X is multiplied by a power of two before it is cut into parts and its sums are divided by it: parts then hold
-// every bit of an X down to the smallest subnormal.  Softmax weights have all sizes below 1: one whose score lies 77 below
-// its row's maximum is less than 2^-110, from where on the unscaled parts lost bits, and a single one sent its unit to the
-// loop below that goes entry by entry.  At the other end a wave's sum of 2^84 or more now takes that loop (before 2^128).
-// us, 16,384 tokens, K = 64, scores of standard deviation 1 / 8 / 12 / 40: 23.7 / 316 / 457 / 457 unscaled, 23.9 / 23.5 / 23.5 / 23.5.
-constexpr float kXScale = 0x1p40f;
+// A power of two that operands are multiplied by before they are cut into parts where they may be small, and that results are
+// divided by: parts then hold every bit of a value down to the smallest subnormal, of which they lose some from 2^-110 down.
+// The product's X always: softmax weights have all sizes below 1, and one whose score lies 77 below its row's maximum is
+// smaller than that.  W and H only where a unit meets such values: the unit is done once more, with both scaled.  At the other
+// end of the range sums overflow earlier, which is found as all overflow is: scaled dot products from 2^48 on, the product's
+// sums from 2^84, with H scaled from 2^44.  us, 16,384 tokens, K = 64, and when such units were computed in fp32, entry by
+// entry: product with scores of standard deviation 1 / 8 / 12 / 40 24.2 / 23.5 / 23.5 / 23.5, and 23.7 / 316 / 457 / 457; one
+// element of H (1.2e-36) softmax 30 and product 26, and 115 and 322; a whole column of H 38 and 38, and 221 and 451.
+constexpr float kScale = 0x1p40f;
 constexpr int kXRow = 16 + 4;         // floats per row of half a tile of X in LDS: 16 rows' 16-byte reads fall into different banks
 
 // the product's LDS: the waves' tiles of X or their sums, then masks and columns of a unit's tiles
@@ -105,11 +108,12 @@ void sddmm_block_kernel(const BlockArgs a)
         h[s % AHEAD][0] = hr[4 * s];
         h[s % AHEAD][1] = hr[4 * s + 1];
     };
-    if (t < unit.z) {
-        col = a.cols[t * kRows + m];
-        col_next = a.cols[min(t + NW, unit.z - 1) * kRows + m];
-    }
-    {
+    // What the wave's tiles from t on begin with.  SCALED: both operands are multiplied by a power of two before they are cut.
+    auto begin = [&]<bool SCALED>(std::bool_constant<SCALED>) {
+        if (t < unit.z) {
+            col = a.cols[t * kRows + m];
+            col_next = a.cols[min(t + NW, unit.z - 1) * kRows + m];
+        }
         const vec4f *w = W4 + ((uint32_t)block_rows[m] * K4 + 2 * kh);
         vec4f raw[KS][2];
 #pragma unroll
@@ -119,9 +123,12 @@ void sddmm_block_kernel(const BlockArgs a)
             for (int s = 0; s < AHEAD; ++s) request(col, s);
         }
         __builtin_amdgcn_sched_barrier(0);
+        constexpr float f = SCALED ? kScale : 1.0f;
 #pragma unroll
-        for (int s = 0; s < KS; ++s) split8(raw[s][0], raw[s][1], pa[s], lost);
-    }
+        for (int s = 0; s < KS; ++s) split8(raw[s][0] * f, raw[s][1] * f, pa[s], lost);
+    };
+    begin(std::false_type{});
+    bool scaled = false;  // (uniform) W or H has values below 2^-110: from there on both scaled, so that parts hold them
     // A softmax needs all of a row's scores at once; otherwise the tiles are taken a few at a time, for the LDS.
     const int round = SOFTMAX ? kBlockTiles : kRoundTiles;
     for (int t0 = unit.y; t0 < unit.z; t0 += round) {
@@ -129,26 +136,41 @@ void sddmm_block_kernel(const BlockArgs a)
         uint2 *kept_info = reinterpret_cast<uint2 *>(kept + (size_t)(SOFTMAX ? unit.z - unit.y : min(kRoundTiles, unit.z - unit.y)) * 1024);
         if (t0 > unit.y) __syncthreads();  // (the round before has been read)
         for (int i = threadIdx.x; i < nt * kRows; i += 64 * NW) kept_info[i] = a.info[t0 * kRows + i];
-        for (; t < t1; t += NW) {
-            // (behind the wave's last tile: the unit's last one again, never used)
-            const int col_after = a.cols[min(t + 2 * NW, unit.z - 1) * kRows + m];
-            floatx16 dot = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        const int first = t;
+        auto dots = [&]<bool SCALED>(std::bool_constant<SCALED>) {
+            constexpr float f = SCALED ? kScale : 1.0f;
+            for (; t < t1; t += NW) {
+                // (behind the wave's last tile: the unit's last one again, never used)
+                const int col_after = a.cols[min(t + 2 * NW, unit.z - 1) * kRows + m];
+                floatx16 dot = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int s = 0; s < KS; ++s) {
-                vec4w pb[3];
-                split8(h[s % AHEAD][0], h[s % AHEAD][1], pb, lost);
-                if (s + AHEAD < KS) request(col, s + AHEAD);
-                else request(col_next, s + AHEAD - KS);
-                __builtin_amdgcn_sched_barrier(0);
-                add_products(dot, pa[s], pb);
-                __builtin_amdgcn_sched_barrier(0);  // (more than one step's sums at a time do not fit the registers)
+                for (int s = 0; s < KS; ++s) {
+                    vec4w pb[3];
+                    split8(h[s % AHEAD][0] * f, h[s % AHEAD][1] * f, pb, lost);
+                    if (s + AHEAD < KS) request(col, s + AHEAD);
+                    else request(col_next, s + AHEAD - KS);
+                    __builtin_amdgcn_sched_barrier(0);
+                    add_products(dot, pa[s], pb);
+                    __builtin_amdgcn_sched_barrier(0);  // (more than one step's sums at a time do not fit the registers)
+                }
+#pragma unroll
+                for (int v = 0; v < 16; ++v) kept[(t - t0) * 1024 + v * 64 + lane] = SCALED ? dot[v] * (1.0f / kScale / kScale) : dot[v];
+                col = col_next;
+                col_next = col_after;
             }
-#pragma unroll
-            for (int v = 0; v < 16; ++v) kept[(t - t0) * 1024 + v * 64 + lane] = dot[v];
-            col = col_next;
-            col_next = col_after;
+        };
+        if (!scaled) {
+            dots(std::false_type{});
+            scaled = __syncthreads_or((lost & 0xffffu) != 0) != 0;
+            if (scaled) {
+                t = first;
+                begin(std::true_type{});
+            }
         }
-        const bool redo = __syncthreads_or((lost & 0xffffu) != 0) != 0;
+        if (scaled) {
+            dots(std::true_type{});
+            __syncthreads();
+        }
         // Each wave takes a quarter of the result registers, each half of it one row per register, all tiles.
         // the dot product of tile u's column in this lane once more, in fp32: where parts cannot carry it
         auto exact = [&](int u, int row) {
@@ -176,11 +198,11 @@ void sddmm_block_kernel(const BlockArgs a)
             }
 #pragma unroll
             for (int u = 0; u < T; ++u) odd = fmaf(score[u], 0.f, odd);
-            if (redo || !__all(odd == 0.f)) {
+            if (!__all(odd == 0.f)) {
 #pragma unroll 1
                 for (int u = 0; u < nt; ++u) {
                     float &place = kept[u * 1024 + v * 64 + lane];
-                    if ((kept_info[u * kRows + row].x & lane_bit) && (redo || !(fabsf(place) < INFINITY))) place = exact(u, row);
+                    if ((kept_info[u * kRows + row].x & lane_bit) && !(fabsf(place) < INFINITY)) place = exact(u, row);
                 }
 #pragma unroll
                 for (int u = 0; u < T; ++u) score[u] = kept[min(u, nt - 1) * 1024 + v * 64 + lane];
@@ -312,10 +334,6 @@ void sddmm_block_spmm_kernel(const BlockArgs a)
     }
     uint32_t lost = 0;
     floatx16 sum[KT];
-#pragma unroll
-    for (int n = 0; n < KT; ++n)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) sum[n][v] = 0.f;
     __syncthreads();
     // What a tile needs is requested while the one before is multiplied.
     // X comes half a tile at a time, H in portions: portion q is the elements 32 (q % KT) on of the columns' rows of step
@@ -334,7 +352,7 @@ void sddmm_block_spmm_kernel(const BlockArgs a)
     };
     auto stage = [&](int s, int u) {  // (what a row does not have becomes 0 here: the entries need not have arrived before)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) xt[(xr0 + 4 * i) * kXRow + xc] = (info[u * kRows + xr0 + 4 * i].x >> (16 * s + xc)) & 1u ? x[i] * kXScale : 0.f;
+        for (int i = 0; i < 8; ++i) xt[(xr0 + 4 * i) * kXRow + xc] = (info[u * kRows + xr0 + 4 * i].x >> (16 * s + xc)) & 1u ? x[i] * kScale : 0.f;
     };
     // Operand element e of step s is column 16 s + 8 kh + e of the tile.
     auto request = [&](int q, int u) {
@@ -346,44 +364,66 @@ void sddmm_block_spmm_kernel(const BlockArgs a)
         for (int e = 0; e < 8; ++e)  // (uniform base + 32-bit offset: no 64-bit addresses to compute and to keep)
             h[q % AHEAD][e] = 32 * n + m < K ? *reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.H) + (b[e] + 4 * m) + 128 * n) : 0.f;
     };
-    int u = wave;
-    if (u < nt) {
-        request(0, u);
-        fetch(0, u);
+    // The wave's sums over its tiles.  SCALED: H is multiplied by the power of two as well.
+    auto add_tiles = [&]<bool SCALED>(std::bool_constant<SCALED>) {
 #pragma unroll
-        for (int q = 1; q < AHEAD; ++q) request(q, u);
-    }
-    for (; u < nt; u += NW) {
-        const int next = min(u + NW, nt - 1);  // (behind the wave's last tile: the unit's last one, never used)
+        for (int n = 0; n < KT; ++n)
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            stage(s, u);
-            __builtin_amdgcn_wave_barrier();  // (written and read by this wave alone: its LDS operations complete in order)
-            vec4w pa[3];
-            const vec4f *xr = reinterpret_cast<const vec4f *>(xt + m * kXRow + 8 * kh);
-            split8(xr[0], xr[1], pa, lost);
-            __builtin_amdgcn_wave_barrier();
-            if (s == 0) fetch(1, u);
-            else fetch(0, next);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int v = 0; v < 16; ++v) sum[n][v] = 0.f;
+        int u = wave;
+        if (u < nt) {
+            request(0, u);
+            fetch(0, u);
 #pragma unroll
-            for (int n = 0; n < KT; ++n) {
-                vec4w pb[3];
-                const int q = s * KT + n;
-                const float *b = h[q % AHEAD];
-                split8(vec4f{b[0], b[1], b[2], b[3]}, vec4f{b[4], b[5], b[6], b[7]}, pb, lost);
-                if (q + AHEAD < 2 * KT) request(q + AHEAD, u);
-                else request(q + AHEAD - 2 * KT, next);
-                add_products(sum[n], pa, pb);
-                __builtin_amdgcn_sched_barrier(0);  // (more than one portion's sums at a time do not fit the registers)
+            for (int q = 1; q < AHEAD; ++q) request(q, u);
+        }
+        for (; u < nt; u += NW) {
+            const int next = min(u + NW, nt - 1);  // (behind the wave's last tile: the unit's last one, never used)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                stage(s, u);
+                __builtin_amdgcn_wave_barrier();  // (written and read by this wave alone: its LDS operations complete in order)
+                vec4w pa[3];
+                const vec4f *xr = reinterpret_cast<const vec4f *>(xt + m * kXRow + 8 * kh);
+                split8(xr[0], xr[1], pa, lost);
+                __builtin_amdgcn_wave_barrier();
+                if (s == 0) fetch(1, u);
+                else fetch(0, next);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int n = 0; n < KT; ++n) {
+                    vec4w pb[3];
+                    const int q = s * KT + n;
+                    const float *b = h[q % AHEAD];
+                    constexpr float f = SCALED ? kScale : 1.0f;
+                    split8(vec4f{b[0], b[1], b[2], b[3]} * f, vec4f{b[4], b[5], b[6], b[7]} * f, pb, lost);
+                    if (q + AHEAD < 2 * KT) request(q + AHEAD, u);
+                    else request(q + AHEAD - 2 * KT, next);
+                    add_products(sum[n], pa, pb);
+                    __builtin_amdgcn_sched_barrier(0);  // (more than one portion's sums at a time do not fit the registers)
+                }
             }
         }
+    };
+    auto beyond = [&]() {
+        bool bad = false;
+#pragma unroll
+        for (int n = 0; n < KT; ++n)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) bad |= !(fabsf(sum[n][v]) < 0x1p124f);  // (the sum of all waves' must not overflow either)
+        return bad;
+    };
+    add_tiles(std::false_type{});
+    float unscale = 1.0f / kScale;
+    bool redo = false;
+    if (__syncthreads_or(beyond() || (lost & 0xffffu) != 0)) {  // (the tiles of X have been read, too)
+        redo = true;
+        if (__syncthreads_or((lost & 0xffffu) != 0)) {  // H has values below 2^-110: once more, where parts hold them
+            add_tiles(std::true_type{});
+            unscale = 1.0f / kScale / kScale;
+            redo = __syncthreads_or(beyond()) != 0;
+        }
     }
-    bool bad = (lost & 0xffffu) != 0;
-#pragma unroll
-    for (int n = 0; n < KT; ++n)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) bad |= !(fabsf(sum[n][v]) < 0x1p124f);  // (the sum of all waves' must not overflow either)
     float *record = a.part + (size_t)max(unit.w, 0) * (KT * 1024);
     auto put = [&](int n, int v, int lane_of, float y) {  // result register v of lane lane_of, elements 32 n on
         if (unit.w >= 0) {
@@ -393,7 +433,7 @@ void sddmm_block_spmm_kernel(const BlockArgs a)
             if (k < K && !repeated_row(a.rows + unit.x * kRows, r)) a.Y[(size_t)a.rows[unit.x * kRows + r] * K + k] = y;
         }
     };
-    if (__syncthreads_or(bad)) {  // (the tiles of X have been read, too)
+    if (redo) {
         for (int r = wave; r < kRows; r += NW)
             for (int k = lane; k < K; k += 64) {
                 float y = 0.f;
@@ -437,7 +477,7 @@ void sddmm_block_spmm_kernel(const BlockArgs a)
             float y = lds[n * 1024 + v * 64 + lane];
 #pragma unroll
             for (int w = 1; w < 4; ++w) y += lds[(w * KT + n) * 1024 + v * 64 + lane];
-            put(n, v, lane, y * (1.0f / kXScale));
+            put(n, v, lane, y * unscale);
         }
 }
 

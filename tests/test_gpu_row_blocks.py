@@ -247,3 +247,41 @@ def test_product_with_small_and_large_weights(oracle, n, half, every, K):
         ref = torch.zeros(n, K, dtype=torch.float64).index_add_(0, row, xe.double()[:, None] * H[col])
         bound = 1e-5 * torch.from_numpy(np.sqrt(np.maximum(deg, 1)))[:, None] * mag + 2.0 ** -149 * torch.from_numpy(deg)[:, None]
         assert bool(((product(xe).double() - ref).abs() <= bound).all()), e
+
+
+@pytest.mark.parametrize("n,half,every,K", [(700, 40, 50, 64), (1500, 30, 400, 80), (700, 60, 60, 128)])
+def test_small_values_in_dense_factors(n, half, every, K):
+    """W, H times a power of two: the results times it, bit for bit, where nothing is subnormal; one small value among large
+    ones changes what it should."""
+    d = window(n, n, half, every, K)
+    t, (plan, _) = plans(d, K, values=False)
+    assert is_blocks(plan, d)
+    row, col = d["row_ind"].long(), d["col_ind"].long()
+    g = torch.Generator().manual_seed(6)
+    x = 0.5 + torch.rand(d["nnz"], generator=g)
+    W, H = (0.5 + torch.rand(n, K, generator=g) for _ in range(2))
+
+    def both(W, H, x):
+        out, Y = torch.full((d["nnz"],), float("nan"), device=DEV), torch.full((n, K), float("nan"), device=DEV)
+        W, H, x = W.to(DEV), H.to(DEV), x.to(DEV)
+        plan.execute(0, W.data_ptr(), H.data_ptr(), out.data_ptr())
+        plan.spmm(x.data_ptr(), H.data_ptr(), Y.data_ptr())
+        torch.cuda.synchronize()
+        return out.cpu(), Y.cpu()
+    s = lambda v, e: torch.ldexp(v, torch.tensor(e))
+    out, Y = both(W, H, x)
+    for ew, eh, ex in ((0, -112, 0), (-112, 0, 0), (-112, 80, 0), (30, -115, 20)):
+        o, y = both(s(W, ew), s(H, eh), s(x, ex))
+        assert torch.equal(o, s(out, ew + eh)) and (eh > 60 or torch.equal(y, s(Y, eh + ex))), (ew, eh)
+    # small values among others, and others so large that they leave the range once scaled
+    for what, e in (("H", 0), ("W", 0), ("H", 46), ("H", 100), ("W", 100)):
+        W2, H2 = s(W, e), H.clone()
+        (H2 if what == "H" else W2)[n // 2, 3:20] = s(H[n // 2, 3:20], -115)
+        if what == "H":
+            H2[:, K - 1] = s(H[:, K - 1], -140)
+        o, y = both(W2, H2, s(x, e))
+        size = (W2.double()[row] * H2.double()[col]).sum(1)
+        ysize = torch.zeros(n, K, dtype=torch.float64).index_add_(0, row, s(x, e).double()[:, None] * H2.double()[col])
+        # (one rounding per product and sum, in any order)
+        bound = (torch.from_numpy(np.diff(d["row_ptr"].numpy())) + 4)[:, None] * 2.0 ** -24 * ysize + 1e-42
+        assert bool(((o.double() - size).abs() <= (K + 4) * 2.0 ** -24 * size).all()) and bool(((y.double() - ysize).abs() <= bound).all()), (what, e)
