@@ -40,13 +40,13 @@ __device__ __forceinline__ int wave_max_scan(int v)
 }
 
 // tab[i] = the row of nonzero p0 + i for 0 <= i < n, tab in this wave's own LDS, n rounded up to 64, plus one entry;
-// nnz = row_ptr[n_rows] > p0.  Returns the row of p0.  tab[n] becomes a row other than that of nonzero p0 + n - 1 if a row ends there.
-// (Entries past the last nonzero hold n_rows.)  The row starts inside the range are marked, one coalesced read of
-// the row pointers for 64 rows, and a running maximum fills the rest; of the rows that start at one nonzero (empty
-// ones) the last counts.  Every read waits for the one before (0.34 us each), so the walk ends at the last
-// nonzero, and after as many steps as the search takes it is given up for that: each lane looks for the rows of its
-// own nonzeros among those left.  (20 thousand nonzeros, K = 16, us without / with both: 4 million empty rows behind
-// them 20700 / 8, spread over 4 million rows 59 / 15.)
+// nnz = row_ptr[n_rows] > p0.  Returns the row of p0.  tab[n] becomes a row other than that of nonzero p0 + n - 1 if a row
+// ends there. (Entries past the last nonzero hold n_rows.)  The row starts inside the range are marked, one coalesced read
+// of the row pointers for 64 rows, and a running maximum fills the rest; of the rows that start at one nonzero (empty ones)
+// the last counts.  Every read waits for the one before (0.34 us each), so the walk ends at the last nonzero, and after as
+// many steps as the search takes it is given up for that: each lane looks for the rows of its own nonzeros among those
+// left.  (20 thousand nonzeros, K = 16, us without / with both: 4 million empty rows behind them 20700 / 8, spread over 4
+// million rows 59 / 15.)
 __device__ __forceinline__ int rows_of_range(const int32_t *__restrict__ row_ptr, int n_rows, int nnz, int p0, int n, int *tab, int lane)
 {
     const int n_pad = (n + 63) & ~63;

@@ -64,9 +64,9 @@ __host__ __device__ inline SoftmaxScale softmax_scale(int64_t nnz, int64_t n_row
 }
 
 // Per unit, or half of one (see piece): (m, sum) of the piece of a huge row that began before it, [2i], and of one that starts
-// in it, [2i + 1]; the rows themselves plus one (0: none).  The kernels take both arrays as arguments: a caller's workspace (sddmm_execute_ws), or
-// these file-scope arrays, 4 + 2 MiB per device, held until the process ends -- softmax calls without a workspace
-// that overlap in time on one device share them and must not (calls on one stream never do).
+// in it, [2i + 1]; the rows themselves plus one (0: none).  The kernels take both arrays as arguments: a caller's workspace
+// (sddmm_execute_ws), or these file-scope arrays, 4 + 2 MiB per device, held until the process ends -- softmax calls
+// without a workspace that overlap in time on one device share them and must not (calls on one stream never do).
 static __device__ __align__(256) float2 g_softmax_rec_store[2 * kSmMaxPieces];
 static __device__ __align__(256) int2 g_softmax_rows_store[kSmMaxPieces];
 

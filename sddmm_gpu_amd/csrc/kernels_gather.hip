@@ -76,8 +76,8 @@ constexpr int whole_pieces(int G, int KPL) { return KPL == 8 ? 4 * G : (KPL - 1)
 // Where a row of W or H begins for a lane that knows its number: the number itself (WIDE), or the offset of its first float,
 // as long as byte offsets have 32 bits: the multiplication is then done once per nonzero, not in every lane and step,
 // and the load takes the matrix's address from scalar registers.  (us with a multiplication in every step and masks on every
-// piece of a ragged row, and so: uniform, 0.9 million nonzeros of 4000 rows, K = 32 / 100 / 200: 9.6 / 23.8 / 41 and 9.1 / 22.3 / 38;
-// 18 thousand, K = 100 / 200: 4.9 / 7.3 and 4.6 / 6.3; where the fabric bounds it the same.)
+// piece of a ragged row, and so: uniform, 0.9 million nonzeros of 4000 rows, K = 32 / 100 / 200: 9.6 / 23.8 / 41 and 9.1 /
+// 22.3 / 38; 18 thousand, K = 100 / 200: 4.9 / 7.3 and 4.6 / 6.3; where the fabric bounds it the same.)
 template <bool WIDE>
 __device__ __forceinline__ vec4u row_piece_of(const float *m, uint32_t at, int off, int K)
 {
@@ -375,15 +375,16 @@ Variant pick_gather_variant(int K)
 // One batch a wave (once), or several?  Reading every step's W row costs load path, the more the longer the rows: a row's
 // nonzeros are next to each other, and the kernel with several batches reads it once.  What it saves is waiting.
 // profiles/row_gather_batches.txt has both at up to 17 ranks on 40 patterns; us, several batches a wave and one:
-//   rows of up to 16 nonzeros: R-MAT, 0.44 million, K = 32 / 96 / 128 18 / 28 / 38 and 15 / 25 / 32, 2.1 million 48 / 95 / 163 and
-//       37 / 75 / 130.  Of up to 32 where nonzeros times pieces are many: 0.38 million of 24 a row, K = 96 / 128 / 256 18 / 24 / 56
-//       and 16 / 22 / 49, 3.9 million of 30, K = 32 / 96 72 / 218 and 69 / 199; but 0.24 million of 30, K = 100 / 128 / 256 11.3 / 12.0 /
-//       28.0 and 12.7 / 13.0 / 25.8, 0.9 million, K = 32 13.2 and 14.3, and up to K = 16 R-MAT, 28 million of 27, 344 and 381.
-//   K = 33 to 63, where a quarter to a half of the lanes' pieces are masked: several batches (R-MAT, 1.4 / 3.4 / 28 million, K = 40
-//       35 / 80 / 648 and 40 / 89 / 835; rows of uniform length would gain 3 to 13 %).  K = 64 gains from half a million on (R-MAT,
-//       2.1 / 28 million 74 / 1014 and 63 / 905), below it does not (0.2 million of 8 a row 10.2 and 10.6).
-//   longer rows: only up to K = 32 and 2^18 nonzeros (0.19 million of 323 a row, K = 16 / 32 / 64 4.5 / 4.7 / 5.5 and 3.8 / 4.5 / 5.8;
-//       0.8 million, K = 32 8.9 and 11.0).
+//   rows of up to 16 nonzeros: R-MAT, 0.44 million, K = 32 / 96 / 128 18 / 28 / 38 and 15 / 25 / 32, 2.1 million 48 / 95 /
+//       163 and 37 / 75 / 130.  Of up to 32 where nonzeros times pieces are many: 0.38 million of 24 a row, K = 96 / 128 /
+//       256 18 / 24 / 56 and 16 / 22 / 49, 3.9 million of 30, K = 32 / 96 72 / 218 and 69 / 199; but 0.24 million of 30, K =
+//       100 / 128 / 256 11.3 / 12.0 / 28.0 and 12.7 / 13.0 / 25.8, 0.9 million, K = 32 13.2 and 14.3, and up to K = 16
+//       R-MAT, 28 million of 27, 344 and 381.
+//   K = 33 to 63, where a quarter to a half of the lanes' pieces are masked: several batches (R-MAT, 1.4 / 3.4 / 28 million,
+//       K = 40 35 / 80 / 648 and 40 / 89 / 835; rows of uniform length would gain 3 to 13 %).  K = 64 gains from half a
+//       million on (R-MAT, 2.1 / 28 million 74 / 1014 and 63 / 905), below it does not (0.2 million of 8 a row 10.2 and 10.6).
+//   longer rows: only up to K = 32 and 2^18 nonzeros (0.19 million of 323 a row, K = 16 / 32 / 64 4.5 / 4.7 / 5.5 and 3.8 /
+//       4.5 / 5.8; 0.8 million, K = 32 8.9 and 11.0).
 // Batches a wave: up to 8, which is as many as share a search for the rows, but fewer where that would leave less than 4096
 // waves (16 per compute unit): 0.9 million nonzeros, K = 32 / 64 / 128 with 2048 waves 27 / 30 / 49, with 4096 19 / 23 / 44; from
 // 1.5 million on all take 8 (two million of 20,000 rows, K = 64: 35, and 38 with 7).

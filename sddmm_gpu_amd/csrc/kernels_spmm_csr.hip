@@ -19,8 +19,8 @@
 // a comparison of rows and two reads of LDS for each nonzero.  So an entry holds where its row of H begins, as a 32-bit offset
 // while H has them, and a mark where a row of S begins: one read, ahead of use, and four nonzeros of every group at a time
 // without a look at their rows where no mark is among them.  us, before and so: ratings of 5 million nonzeros in 5600
-// columns, K = 16 / 50 / 128 / 200 / 256: 45 / 73 / 107 / 243 / 266 and 37 / 69 / 103 / 186 / 227 (25 TB/s of H rows at K = 128); uniform, 4 million, K = 32
-// 40 and 35; R-MAT, 1.86 million, K = 100 83 and 81.
+// columns, K = 16 / 50 / 128 / 200 / 256: 45 / 73 / 107 / 243 / 266 and 37 / 69 / 103 / 186 / 227 (25 TB/s of H rows at K =
+// 128); uniform, 4 million, K = 32 40 and 35; R-MAT, 1.86 million, K = 100 83 and 81.
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include "internal.hpp"

@@ -613,8 +613,8 @@ void sddmm_tile_kernel(const TileArgs a)
             *dst = pend_v;
         };
         // c[I]: where the H row this lane works on in step I starts (LDS: byte address of
-        // this lane's first piece; gather form: float4 index of the row); cn: the same for the next batch, requested here after the last LDS
-        // read so that the latency hides behind the reduction
+        // this lane's first piece; gather form: float4 index of the row); cn: the same for the next batch, requested here
+        // after the last LDS read so that the latency hides behind the reduction
         auto compute = [&]<bool SHORT>(std::bool_constant<SHORT>, const float4 (&w_in)[KPL], const Meta &m, const int (&c)[G],
                                        int (&cn)[G], int next_col) {
             constexpr int STEPS = SHORT ? G / 2 : G;

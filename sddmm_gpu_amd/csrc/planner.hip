@@ -567,13 +567,14 @@ enum class Split { all_tiled, by_length, all_gathered, slabs };
 // elements does not stay in a die's 4 MB of L2: which slab width is cheapest, from the sampled rows.  Narrow slabs
 // have short runs (more padding, the W row once per run), wide ones miss the L2.  Picoseconds per padded position and
 // slice, measured with 2 / 4 / 8 / 16 / 32 MB of H slice per slab: uniform columns, w = 128: 28 / 30 / 43 / 55 / 62, w = 64:
-// 18 / 20 / 23 / 27 / 31; R-MAT, w = 128: 30 / 31 / 32 / 33 / 35 and 42 / 53 with 64 / 128 MB, w = 64: 16 to 20 up to 32 MB -- as if
-// its slabs were a twelfth as large, since few columns get most of the accesses.  So the size E counts by a power of the
-// share of the columns (in 1024 stretches) that gets 60 % of the nonzeros, and a position costs 26 + 40 E^2 / (E^2 + 70) at
-// w = 128, 17.5 + 16 E^2 / (E^2 + 110) at w = 64.  us against the best of the other three: uniform 95 M of 220,000 columns,
-// K = 128 6494 -> 3142; 20 M of 100,000, K = 64 563 -> 392, K = 256 2664 -> 1424; R-MAT 2^20, 78 M, K = 128 4094 -> 2990, 36 M, K = 512
-// 12960 -> 7154; 2^18, 13 M, K = 128 678 -> 467.  Slices of 32 gain nothing (2^20: 620 against 685), nor does a band whose
-// neighbouring rows use neighbouring columns anyway (200,000 rows, 20 of +-20,000 each: 300 against 342).
+// 18 / 20 / 23 / 27 / 31; R-MAT, w = 128: 30 / 31 / 32 / 33 / 35 and 42 / 53 with 64 / 128 MB, w = 64: 16 to 20 up to 32 MB
+// -- as if its slabs were a twelfth as large, since few columns get most of the accesses.  So the size E counts by a power
+// of the share of the columns (in 1024 stretches) that gets 60 % of the nonzeros, and a position costs 26 + 40 E^2 / (E^2 +
+// 70) at w = 128, 17.5 + 16 E^2 / (E^2 + 110) at w = 64.  us against the best of the other three: uniform 95 M of 220,000
+// columns, K = 128 6494 -> 3142; 20 M of 100,000, K = 64 563 -> 392, K = 256 2664 -> 1424; R-MAT 2^20, 78 M, K = 128 4094
+// -> 2990, 36 M, K = 512 12960 -> 7154; 2^18, 13 M, K = 128 678 -> 467.  Slices of 32 gain nothing (2^20: 620 against 685),
+// nor does a band whose neighbouring rows use neighbouring columns anyway (200,000 rows, 20 of +-20,000 each: 300 against
+// 342).
 struct SlabChoice { int64_t cols = 0; double us = 1e30; };
 static SlabChoice estimate_slabs(const Ctx &c, const std::vector<int32_t> &rows, int w)
 {

@@ -56,12 +56,14 @@ constexpr int64_t kUnitTiles = 4;   // tiles per unit of a row block that is sev
 // Lays S out for the row-block kernels if that pays; *taken: it does.  rows: the rows with nonzeros, ascending.  Rows of
 // more than twice the mean (tokens that look at all others) are put into blocks of their own, as they would fill the
 // others' with their columns.
-// Where the line lies, in cells computed per nonzero.  Plans that serve the product as well (attention): 2.5.  us, row
-// blocks against tiles / walk and the softmax's own passes, softmax + product: windows of 128 on either side of 16,384
-// tokens, 1.1 cells, K = 32 / 64 / 128 39 / 53 / 75 against 102 / 135 / 227; with 1.9 cells (40 % left out) 24 / 35 / 52 against
-// 70 / 82 / 124; 2.5 24 / 34 / 51 against 60 / 71 / 101; of 400, 60,000 tokens, 2.9 cells 178 / 275 / 397 against 235 / 313 / 338.  The SDDMM alone: 1.6, from half a million nonzeros on
-// (1.1 cells 15 / 21 / 35 against 24 / 40 / 77, 1.9 cells 12 / 17 / 24 against 12 / 17 / 27, 2.5 cells 12 / 17 / 24 against 11 / 14 / 24;
-// 400 thousand nonzeros, 1.6 cells 5.9 / 7.7 / 10.5 against 6.9 / 8.0 / 9.9, 200 thousand 5.6 / 7.4 / 10.1 against 4.8 / 5.6 / 8.3).
+// Where the line lies, in cells computed per nonzero; us, row blocks against tiles or walk and the softmax's own passes, at
+// K = 32 / 64 / 128.
+//   Plans that serve the product as well (attention), softmax + product: 2.5.  Windows of 128 on either side of 16,384 tokens,
+//       1.1 cells: 39 / 53 / 75 against 102 / 135 / 227; 1.9 cells (40 % left out): 24 / 35 / 52 against 70 / 82 / 124; 2.5
+//       cells: 24 / 34 / 51 against 60 / 71 / 101; of 400, 60,000 tokens, 2.9 cells: 178 / 275 / 397 against 235 / 313 / 338.
+//   The SDDMM alone: 1.6, from half a million nonzeros on.  1.1 cells: 15 / 21 / 35 against 24 / 40 / 77; 1.9: 12 / 17 / 24
+//       against 12 / 17 / 27; 2.5: 12 / 17 / 24 against 11 / 14 / 24; 400 thousand nonzeros, 1.6 cells: 5.9 / 7.7 / 10.5
+//       against 6.9 / 8.0 / 9.9, 200 thousand: 5.6 / 7.4 / 10.1 against 4.8 / 5.6 / 8.3.
 int add_blocks(Ctx &c, const std::vector<int32_t> &rows, bool *taken)
 {
     *taken = false;
@@ -128,11 +130,15 @@ int add_blocks(Ctx &c, const std::vector<int32_t> &rows, bool *taken)
     });
     if (twice || (double)n_cells > most_cells) return SDDMM_OK;
 
-    // Few blocks: the one with the most tiles that a workgroup computes alone is what the launches take, and the general path's
-    // time grows with the nonzeros instead.  Both in us for softmax + product, from windows of 200 to 4000 tokens, K = 32 / 64 /
-    // 80 / 128: 559 tokens, 83 on either side, 24 full rows (18 tiles) 20 / 27 / 31 / 38 with blocks, 19 / 20 / 23 / 23 without; 1000, 40
-    // (32 tiles) 28 / 38 / 44 / 55 and 19 / 21 / 23 / 27; 334, 167 (11 tiles) 16 / 21 / 23 / 30 and 18 / 20 / 22 / 21; 2000, 100 (7 tiles, the full
-    // rows in parts) 20 / 24 / 27 / 32 and 36 / 40 / 46 / 46; 2000, 24 (4) 18 / 22 / 23 / 28 and 23 / 25 / 28 / 31.
+    // Few blocks: the one with the most tiles that a workgroup computes alone is what the launches take, and the general
+    // path's time grows with the nonzeros instead.  Both in us for softmax + product, fitted to windows of 200 to 4000 tokens.
+    // Blocks and general path at K = 32 / 64 / 80 / 128: 559 tokens, 83 on either side, 24 full rows (18 tiles) 20 / 27 / 31 / 38
+    // and 19 / 20 / 23 / 23; 1000, 40 (32 tiles) 28 / 38 / 44 / 55 and 19 / 21 / 23 / 27; 334, 167 (11 tiles) 16 / 21 / 23
+    // / 30 and 18 / 20 / 22 / 21; 2000, 100 (7 tiles, the full rows in parts) 20 / 24 / 27 / 32 and 36 / 40 / 46 / 46;
+    // 2000, 24 (4) 18 / 22 / 23 / 28 and 23 / 25 / 28 / 31.  On 120 other patterns (windows without full rows, one-sided,
+    // thinned; dense blocks and triangles; profiles/row_blocks_few.txt) at four ranks what this takes is the faster one or
+    // within 5 % of it, but for 10 of 460 cases, at worst 19 % slower (1024 tokens in dense blocks of 64, K = 128: 21.3
+    // with blocks, 18.0 without).
     if (product && n_blocks <= c.cus && c.opt.dense_blocks != 2) {
         int64_t most = 0;
         bool parts = false;

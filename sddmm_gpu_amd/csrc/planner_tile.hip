@@ -240,8 +240,9 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         // and 58 / 55; uniform, 2.3 M, K = 64 37 / 37).  Both hold while H is about as large as a die's L2,
         // from where the walk then gathers; beyond, only really short runs, the shorter the longer the rows of H (ratings,
         // K = 384, 2 to 3.5 M nonzeros, H of 7 and 8 MB, runs of 10: 180 against 211 and 338 against 387 us; word counts of 6.9 M,
-        // K = 128, H of 27 MB, runs of 7 392 / 269; of 1.8 M, H of 13 to 39 MB, runs of 8, K = 128 58 / 58, K = 256 112 / 145, K = 384
-        // 166 / 251; uniform, K = 256, H of 17 and 31 MB, runs of 5 190 / 261 and 1515 / 1723, H of 21 MB, runs of 4 647 / 543).
+        // K = 128, H of 27 MB, runs of 7 392 / 269; of 1.8 M, H of 13 to 39 MB, runs of 8, K = 128 58 / 58, K = 256 112 /
+        // 145, K = 384 166 / 251; uniform, K = 256, H of 17 and 31 MB, runs of 5 190 / 261 and 1515 / 1723, H of 21 MB,
+        // runs of 4 647 / 543).
         const bool h_near = (int64_t)c.n_cols * c.K * 4 <= 6000000;
         if (want_spmm && rb == 0 && c.nnz == c.P->info.nnz &&
             (ragged || (h_near && (L.nnz < 12 * n_seg || product_walks(c.nnz, c.K, ks))) || L.nnz < (c.K <= 128 ? 8 : 5) * n_seg)) { want_spmm = false; sp_csr = true; }
@@ -717,12 +718,13 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
             // and is the faster one at any run length (windows of 400 to 600, 5 to 14 million nonzeros, items cut and
             // dealt out anew against the walk: K = 128 451 / 279, 283 / 236 and 423 / 287 us, K = 64 283 / 150, 175 / 126
             // and 155 / 68, K = 32 with runs of 41 220 / 84), but only so far as the caches go.  The walk has 2 to 3
-            // million nonzeros in flight (6144 waves of 512), so where rows touch few tiles it needs that share of H at a time.  Where
-            // the busiest workgroup has less than 3.5 times the mean, the longer the rows of H the smaller this may be (bands
-            // of 1.4 to 4.8 M, 2 to 2.5 times the mean: K = 64, H of 12, 48 and 53 MB 68 / 57, 108 / 81 and 133 / 150; K = 128, 16, 18
-            // and 20 MB 57 / 60, 55 / 64 and 99 / 117; K = 256, 37 and 41 MB 107 / 151 and 198 / 332; window of 313, 14 M, K = 128 and
-            // 256, a seventh of 21 and 41 MB 475 / 317 and 951 / 639; word counts of 24.5 M, K = 256, all of 110 MB 1946 / 2937; R-MAT of 4.3 M, 16 times the
-            // mean, K = 64 to 256, H of 34 to 134 MB 211 / 94, 369 / 227 and 777 / 618).
+            // million nonzeros in flight (6144 waves of 512), so where rows touch few tiles it needs that share of H at a
+            // time.  Where the busiest workgroup has less than 3.5 times the mean, the longer the rows of H the smaller
+            // this may be (bands of 1.4 to 4.8 M, 2 to 2.5 times the mean: K = 64, H of 12, 48 and 53 MB 68 / 57, 108 / 81
+            // and 133 / 150; K = 128, 16, 18 and 20 MB 57 / 60, 55 / 64 and 99 / 117; K = 256, 37 and 41 MB 107 / 151 and
+            // 198 / 332; window of 313, 14 M, K = 128 and 256, a seventh of 21 and 41 MB 475 / 317 and 951 / 639; word
+            // counts of 24.5 M, K = 256, all of 110 MB 1946 / 2937; R-MAT of 4.3 M, 16 times the mean, K = 64 to 256, H of
+            // 34 to 134 MB 211 / 94, 369 / 227 and 777 / 618).
             const bool local = 4 * n_seg <= (int64_t)rows.size() * T.n_tiles;
             const double h_part = local ? std::min(1.0, 2e6 / (double)L.nnz) : 1.0;
             if (want_spmm && uneven && c.nnz == c.P->info.nnz &&
