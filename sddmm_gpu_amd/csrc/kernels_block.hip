@@ -352,7 +352,10 @@ void sddmm_block_spmm_kernel(const BlockArgs a)
     };
     auto stage = [&](int s, int u) {  // (what a row does not have becomes 0 here: the entries need not have arrived before)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) xt[(xr0 + 4 * i) * kXRow + xc] = (info[u * kRows + xr0 + 4 * i].x >> (16 * s + xc)) & 1u ? x[i] * kScale : 0.f;
+        for (int i = 0; i < 8; ++i) {
+            const int has = __builtin_amdgcn_sbfe((int)info[u * kRows + xr0 + 4 * i].x, 16 * s + xc, 1);  // 0 or -1
+            xt[(xr0 + 4 * i) * kXRow + xc] = __int_as_float(__float_as_int(x[i]) & has) * kScale;
+        }
     };
     // Operand element e of step s is column 16 s + 8 kh + e of the tile.
     auto request = [&](int q, int u) {
