@@ -18,12 +18,14 @@
 //   sddmm_block_spmm_kernel: Y = X H.  The tile of X is put together from the nonzeros in LDS, the 32 columns' rows of H
 //     are the other operand; the waves' sums are added up in order through LDS.
 //
-// What bounds it is vector instructions and matrix instructions in turn, hardly overlapped, two waves per SIMD: per tile
-// 1024 clocks of matrix instructions, 1500 of cutting H into parts and adding, and about as many again for masks,
-// exponentials and stores.  Window of 128 on either side of 16,384 tokens, 32 full rows and columns, K = 64 (5.2 M nonzeros,
-// 5602 tiles), us: scores and softmax 22 + 8 for the long rows (tile kernel and three softmax kernels 41 + 34), product
-// 22 + 4 (walk over the pattern 66 + 5).  The relative error against 64 bits is smaller than that of those: scores 5.2e-8
-// (8.3e-8), product 6.6e-8 (11e-8), at K = 128 6.4e-8 (8.8e-8) and 6.6e-8 (15e-8).
+// What bounds it: vector instructions, 3640 clocks of them per tile for scores and softmax (cutting H into parts and adding
+// 1500, masks, exponentials, stores and the cutting of W the rest) and 3320 for the product, beside 1024 of matrix
+// instructions, 27 and 35 % of which lie under vector ones; that fills a SIMD for 59 and 53 % of the time its compute unit
+// has work, waits the rest: 2.5 units per compute unit, first loads, the barrier between tiles and rows
+// (profiles/row_blocks_attention_k64.txt).  Window of 128 on either side of 16,384 tokens, 32 full rows and columns, K = 64
+// (5.2 M nonzeros, 5602 tiles), us: scores and softmax 22 + 6 for the long rows (tile kernel and three softmax kernels 41 +
+// 34), product 22 + 4 (walk over the pattern 66 + 5).  The relative error against 64 bits is smaller than that of those:
+// scores 5.2e-8 (8.3e-8), product 6.6e-8 (11e-8), at K = 128 6.4e-8 (8.8e-8) and 6.6e-8 (15e-8).
 // Measured on the way, us of the two kernels: epilogue from the accumulators' layout, tiles' scores read back one at a time
 // 40; three waves per SIMD for all with 170 registers spilling 41 and 65 (a kernel that uses scratch memory starts late as
 // well); long rows' units of 12 tiles, in front, 30 (a second round of workgroups), of 4, behind, 23.

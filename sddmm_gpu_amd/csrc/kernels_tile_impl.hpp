@@ -307,10 +307,11 @@ __device__ __forceinline__ void matrix_core_waves(const TileArgs &a, int mw, int
 // products so far go to a.part, in stream order: one coalesced store per batch); 2 = a slice in between
 // (adds to what it reads back from a.part, coalesced); 4 = the last one, which alone reads positions and
 // values and touches out, with one scattered store per position.
-// (The slices before it are bound by the vector unit, two thirds busy, and by waits for W; the last one by its positions,
-// values and partial output lines.  Before, all of them read positions and values, columns in 32 bits, and scaled: a band of 64
-// in 4096 columns, 2^20 rows, K = 512, 4.02 -> 3.42 ms (1.46 -> 0.29 GB of stream data in each but the last); the remainder
-// of the recommender at K = 512, 1.39 -> 1.21.  Stream data four batches ahead, or with the non-temporal hint: the same.)
+// (All are bound by the load path, 81 to 83 % busy on a band of 64 in 4096 columns, 2^20 rows, K = 512, vector unit 64 % in
+// the slices before the last and 44 % in that, which has the positions, values and partial output lines.  Before, all of
+// them read positions and values, columns in 32 bits, and scaled: 4.02 -> 3.42 ms (16.5 -> 11.3 GB a step; 1.46 -> 0.29 GB of
+// stream data in each slice but the last); the remainder of the recommender at K = 512, 1.39 -> 1.21.  Stream data four
+// batches ahead, or with the non-temporal hint: the same.)
 // 3 = all a.n_slices K slices inside this one launch, one after the other (small matrices, where a
 // launch costs as much as its work): a wave meets the same positions in every slice, so the partial
 // results it left in a.part are its own, and a workgroup barrier between the slices is all the

@@ -8,7 +8,7 @@ A profile directory holds one sub-directory per rocprofv3 pass (the tool collect
 one counter set per run), each with the pass's ``*_counter_collection.csv`` and/or
 ``*_kernel_trace.csv`` and, as ``run.json``, the JSON line the profiled bench run
 printed (it carries ``config.executes``, the number of SDDMM steps the process
-issued).  Typical passes, each a run of its own on the GPU box::
+issued).  Typical passes, each a run of its own::
 
     rocprofv3 --pmc FETCH_SIZE --kernel-trace --output-format csv -d DIR/fetch -o p -- \\
         python3 bench.py --no-cpu --no-sweep --steps 3 --warmup 1 --spinup-ms 0 --copy-probe > DIR/fetch/run.json
@@ -150,7 +150,7 @@ def summarize(profile_dir):
 
 def as_text(s):
     lines = [f"rocprofv3 summary of {s['profile_dir']} (passes: {', '.join(s['passes'])}), made by python3 -m sddmm_gpu_amd.rocprof {s['profile_dir']}",
-             "each pass is a run of its own on the MI355X box, from the repository root, after cd /tmp && export TMPDIR=/tmp && cd back:"]
+             "each pass is a run of its own on one MI355X, from the repository root, after cd /tmp && export TMPDIR=/tmp && cd back:"]
     lines += ["  " + c for c in s["commands"]]
     lines.append("(the line each run prints is kept as run.json in its pass directory: it carries the number of steps the run issued)")
     lines.append("(bytes per step = counter in KiB x 1024 x scale factor, summed over the kernels of one sddmm_execute; the scale factor is")
