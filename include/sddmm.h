@@ -418,7 +418,11 @@ int sddmm_execute_ws(const sddmm_plan *plan, const float *d_val, const float *d_
  * nonzeros times K, H as above) and where a few workgroups would hold most of the work, the whole product
  * goes over the CSR pattern as sddmm_spmm_csr does it, with the parts of its cut rows
  * written down and added up in order; and a plan on row blocks multiplies its tiles
- * on the matrix cores.  No atomics: the same bits on every call.  The
+ * on the matrix cores (weights of any size at the same speed; where 32 rows meet values of
+ * H below 2^-110 they are done twice, where they meet infinities, NaNs or sums beyond
+ * 2^84, entry by entry in fp32, ten to twenty times slower; the same holds for its SDDMM and
+ * values of W or H, but only the results that are not finite are done again).
+ * No atomics: the same bits on every call.  The
  * partial rows (K floats per run; sddmm_plan_info.spmm_runs) live in the plan, so
  * calls on one plan must not overlap in time, or in d_workspace (NULL, or as for
  * sddmm_execute_ws): calls with a workspace each may.  Other plans (and H or Y not
