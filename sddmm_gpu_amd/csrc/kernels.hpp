@@ -119,6 +119,7 @@ TileVariant pick_tile_variant(int K, int want_g);
 // the kernel template); 1 and 2 are the same for every vmode
 // ragged: the form for ranks that are no multiple of the variant's width (see the kernel template)
 TileFn tile_kernel(const TileVariant &v, int vmode, bool gather, int slice, int nwaves, bool ragged);
+TileFn slab_gather_kernel(int k_slice, int vmode, int slice);  // its gather form on groups of 4 positions (kernels_slab.hip)
 int ragged_tile_width(int K);  // the width for such a rank (0: none)
 // The variant with a matrix-core share (TileArgs::mf_*): groups of 8 lanes on rows of 128 elements, all of K
 // in one launch, nw vector waves + nwm matrix-core waves per workgroup ((12, 4), (8, 8) or (8, 4)).

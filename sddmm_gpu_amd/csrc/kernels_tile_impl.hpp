@@ -782,6 +782,22 @@ TileFn fused_slices_kernel()
     else return nullptr;
 }
 
+// The gather form on groups of 8 lanes and more (on groups of 4: slab_gather_kernel).
+template <int G, int KPL, int VMODE>
+TileFn gather_tile_kernel(int slice)
+{
+    if constexpr (G > 4) {
+        if (slice == 0) return (TileFn)sddmm_tile_kernel<G, KPL, VMODE, 4, true, 0>;
+        if constexpr (VMODE == 2) {
+            if (slice == 1) return (TileFn)sddmm_tile_kernel<G, KPL, VMODE, 4, true, 1>;
+            if (slice == 2) return (TileFn)sddmm_tile_kernel<G, KPL, VMODE, 4, true, 2>;
+        }
+        if (slice == 3) return fused_slices_kernel<G, KPL, VMODE, 4, true>();
+        if (slice == 4) return (TileFn)sddmm_tile_kernel<G, KPL, VMODE, 4, true, 4>;
+    }
+    return nullptr;
+}
+
 // The ragged form exists for the widths the planner rounds other ranks up to: 32, 64 and 128 elements, and of the sliced
 // forms for slices of 128; null for everything else.
 template <int VMODE>

@@ -8,13 +8,13 @@ namespace sddmm {
 TileFn tile_kernel_part3(const TileVariant &v, int vmode, bool gather, int slice, int nwaves, bool ragged)
 {
     if (ragged) return ragged_tile_kernel<3>(v, gather, slice, nwaves);
-#define SDDMM_PICK_SLICE(g, kpl, vm, nw, ga)                                                                 \
-    (slice == 3 ? fused_slices_kernel<g, kpl, vm, nw, ga>()                                                 \
-     : slice == 4 ? (TileFn)sddmm_tile_kernel<g, kpl, vm, nw, ga, 4>                                        \
-                  : (TileFn)sddmm_tile_kernel<g, kpl, vm, nw, ga, 0>)
+#define SDDMM_PICK_SLICE(g, kpl, vm, nw)                                                                     \
+    (slice == 3 ? fused_slices_kernel<g, kpl, vm, nw, false>()                                              \
+     : slice == 4 ? (TileFn)sddmm_tile_kernel<g, kpl, vm, nw, false, 4>                                        \
+                  : (TileFn)sddmm_tile_kernel<g, kpl, vm, nw, false, 0>)
 #define SDDMM_PICK(g, kpl, vm)                                                                              \
-    (gather ? SDDMM_PICK_SLICE(g, kpl, vm, 4, true)                                                         \
-            : (nwaves == 12 ? SDDMM_PICK_SLICE(g, kpl, vm, 12, false) : SDDMM_PICK_SLICE(g, kpl, vm, 16, false)))
+    (gather ? gather_tile_kernel<g, kpl, vm>(slice)                                                         \
+            : (nwaves == 12 ? SDDMM_PICK_SLICE(g, kpl, vm, 12) : SDDMM_PICK_SLICE(g, kpl, vm, 16)))
 #define SDDMM_CASE(g, kpl)                                                                                  \
     if (v.G == g && v.KPL == kpl)                                                                           \
         return SDDMM_PICK(g, kpl, 3);

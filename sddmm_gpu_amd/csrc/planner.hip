@@ -572,7 +572,8 @@ enum class Split { all_tiled, by_length, all_gathered, slabs };
 // of the share of the columns (in 1024 stretches) that gets 60 % of the nonzeros, and a position costs 26 + 40 E^2 / (E^2 +
 // 70) at w = 128, 17.5 + 16 E^2 / (E^2 + 110) at w = 64.  us against the best of the other three: uniform 95 M of 220,000
 // columns, K = 128 6494 -> 3142; 20 M of 100,000, K = 64 563 -> 392, K = 256 2664 -> 1424; R-MAT 2^20, 78 M, K = 128 4094
-// -> 2990, 36 M, K = 512 12960 -> 7154; 2^18, 13 M, K = 128 678 -> 467.  Slices of 32 gain nothing (2^20: 620 against 685),
+// -> 2990, 36 M, K = 512 12960 -> 7154; 2^18, 13 M, K = 128 678 -> 467 (with four lanes to a position; with eight, see
+// kernels_slab.hip, 2 to 10 % less, at every width alike).  Slices of 32 gain nothing (2^20: 620 against 685),
 // nor does a band whose neighbouring rows use neighbouring columns anyway (200,000 rows, 20 of +-20,000 each: 300 against
 // 342).
 struct SlabChoice { int64_t cols = 0; double us = 1e30; };

@@ -473,20 +473,21 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         });
         np = np_new;
         if (flag_padding) {
-            // Gather form: in step I of a batch the 8 groups read the H rows of positions
-            // 64 b + 8 g + I.  A padding position there re-reads its own row's last column: one
+            // Gather form: in step I of a batch every 8 lanes (groups of 4: two groups; else every group) read the H
+            // row of their position I.  A padding position there re-reads its own row's last column: one
             // more cache line through the load path, which is what binds this kernel.  Point it
             // at the column another group reads in the same step instead (the same line, merged
             // by the load path), and flag its index so that the result is dropped.
             const int64_t nb64 = (np + 63) / 64;
+            const int at_a_time = std::max(G, 8);
             parallel_ranges(nb64, 1 << 8, [&](int64_t bb, int64_t be, int) {
                 for (int64_t b = bb; b < be; ++b) {
                     const int64_t base = b * 64, lim = std::min<int64_t>(np, base + 64);
-                    for (int I = 0; I < G; ++I) {
+                    for (int I = 0; I < at_a_time; ++I) {
                         int32_t common = scol[(size_t)base];  // (a group's first position is never padding)
-                        for (int64_t d = base + I; d < lim; d += G)
+                        for (int64_t d = base + I; d < lim; d += at_a_time)
                             if (perm[(size_t)d] >= 0) { common = scol[(size_t)d]; break; }
-                        for (int64_t d = base + I; d < lim; d += G)
+                        for (int64_t d = base + I; d < lim; d += at_a_time)
                             if (perm[(size_t)d] < 0) scol[(size_t)d] = common;
                     }
                 }
