@@ -258,7 +258,7 @@ typedef struct sddmm_plan_options {
                                    1 runs of neighbouring tiles to one die, 2 row ranges
                                    walked by groups of workgroups of one die (-1:
                                    2 where rows touch few tiles each, else 1)       [SDDMM_TILE_RUNS]     */
-    int32_t gather_lanes;       /* lanes per nonzero of the short-row launch        [SDDMM_GATHER_G]      */
+    int32_t gather_lanes;       /* positions per group of the short-row launch (rows are padded to it) [SDDMM_GATHER_G] */
     int32_t gather_padded;      /* 0/1 short rows through the padded gather kernel  [SDDMM_GATHER_PADDED] */
     int32_t gather_sink;        /* 0/1 padding of that stream flagged and dropped   [SDDMM_GATHER_SINK]   */
     int32_t row_padded;         /* 0/1 ROW_GATHER plans use the padded gather kernel [SDDMM_ROW_PADDED]    */

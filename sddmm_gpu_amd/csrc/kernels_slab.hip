@@ -16,14 +16,14 @@ namespace {
 // million of 100,000 columns, K = 64 / 128 419 / 713 and 375 / 703.  2048 positions a workgroup (chosen by the planner): 1024 /
 // 4096 / 8192 / 16384 on the first 4509 / 4419 / 4506 / 4763 where 2048 takes 4415; neighbouring workgroups bound to one die,
 // 4 to 1024 at a time: 4398 to 4453; four steps' pieces at a time instead of eight: the same.
-// VMODE, SLICE: as in the tile kernel (SLICE 0, 1, 2, 4).
+// VMODE, SLICE: as in the tile kernel.  (SLICE 3, all K slices inside one launch: a wave's partial results are its own.)
 template <int KPL, int VMODE, int SLICE>
 __global__ __launch_bounds__(256)
 void sddmm_slab_gather_kernel(const TileArgs a)
 {
     constexpr int L = 8, G = 4, NW = 4;
     constexpr int ROUND = KPL <= 2 ? 8 : 4;  // steps whose pieces of H are requested together
-    constexpr bool ACC = SLICE == 2 || SLICE == 4, PART = SLICE >= 1, TO_OUT = SLICE == 0 || SLICE == 4;
+    constexpr bool FUSED = SLICE == 3, ACC = SLICE == 2 || SLICE == 4, PART = SLICE >= 1, TO_OUT = SLICE == 0 || SLICE >= 3;
     constexpr bool RESIDUAL = VMODE >= 3, STREAM_VAL = VMODE == 0 || VMODE == 3, SORTED_VAL = VMODE == 1 || VMODE == 4;
     static_assert(TO_OUT || VMODE == 2);
     const int lane = threadIdx.x & 63, l = lane & (L - 1);
@@ -36,12 +36,17 @@ void sddmm_slab_gather_kernel(const TileArgs a)
     const int b0 = __builtin_amdgcn_readfirstlane(nb * wave / NW);
     const int b1 = __builtin_amdgcn_readfirstlane(nb * (wave + 1) / NW);
     if (b0 >= b1) return;
-    const float4 *__restrict__ W4 = reinterpret_cast<const float4 *>(a.W) + (a.k_off >> 2) + l;
-    const float4 *__restrict__ H4 = reinterpret_cast<const float4 *>(a.H) + (a.k_off >> 2) + l;
     const int32_t *perm = a.perm + lo, *scol = a.scol + lo, *grow = a.grow + lo / G;
     const float *sval = a.sval + lo;
     float *part = a.part + lo;
     const uint32_t last = (uint32_t)(total - 1 - lo);  // the stream's last position, counted from lo
+
+    const int n_slices = FUSED ? a.n_slices : 1;
+    for (int sl = 0; sl < n_slices; ++sl) {
+    const bool first_slice = sl == 0, last_slice = sl + 1 == n_slices;  // (used by the FUSED form only)
+    const float4 *__restrict__ W4 = reinterpret_cast<const float4 *>(a.W) + ((a.k_off >> 2) + sl * L * KPL + l);
+    const float4 *__restrict__ H4 = reinterpret_cast<const float4 *>(a.H) + ((a.k_off >> 2) + sl * L * KPL + l);
+    if (FUSED && sl > 0) __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // the partial results before are stored
 
     // Index data of one batch: lanes past the end of the stream repeat its last position, and their results are dropped
     // like those of padding; what is requested past a wave's range is dropped.
@@ -57,7 +62,11 @@ void sddmm_slab_gather_kernel(const TileArgs a)
         at += 64;
         return m;
     };
-    auto issue_old = [&](Meta &m) { m.old = ACC ? part[m.o] : 0.f; };
+    // (FUSED: the slot is read in every slice and ignored in the first: no load behind a branch)
+    auto issue_old = [&](Meta &m) {
+        m.old = ACC || FUSED ? part[m.o] : 0.f;
+        if constexpr (FUSED) m.old = first_slice ? 0.f : m.old;
+    };
     // both rows' pieces: lanes 0 to 3 of the eight hold the first group's row, lanes 4 to 7 the second one's
     auto issue_w = [&](float4 (&w)[2][KPL], uint32_t wrow) {
         const uint32_t other = (uint32_t)from_lane_xor<4>((int)wrow);
@@ -73,6 +82,7 @@ void sddmm_slab_gather_kernel(const TileArgs a)
         float *dst;
         if constexpr (!TO_OUT) dst = part + pend_o;
         else dst = (int32_t)pend_p < 0 ? a.sink + (((blockIdx.x & 255) << 6) + lane) : a.out + pend_p;
+        if constexpr (FUSED) dst = last_slice ? dst : part + pend_o;
         *dst = pend_v;
     };
     auto compute = [&](const float4 (&w)[2][KPL], const Meta &m) {
@@ -108,6 +118,7 @@ void sddmm_slab_gather_kernel(const TileArgs a)
             const Halves sum = add_to(m.old, d, (l & 1) != 0);
             if constexpr (SLICE == 2) pend_v = sum.x + sum.y;
             else pend_v = RESIDUAL ? (v - (d.x + d.y)) - m.old : VMODE == 2 ? sum.x + sum.y : fmaf(sum.x, v, sum.y * v);
+            if constexpr (FUSED) pend_v = last_slice ? pend_v : sum.x + sum.y;
         }
         if constexpr (TO_OUT) pend_p = m.p;
         pend_o = m.o;
@@ -135,12 +146,15 @@ void sddmm_slab_gather_kernel(const TileArgs a)
         m1 = m3;
     }
     flush();
+    }
 }
 
 template <int KPL, int VMODE>
 TileFn slab_gather(int slice)
 {
     if (slice == 0) return (TileFn)sddmm_slab_gather_kernel<KPL, VMODE, 0>;
+    if constexpr (KPL == 4)
+        if (slice == 3) return (TileFn)sddmm_slab_gather_kernel<KPL, VMODE, 3>;
     if (slice == 4) return (TileFn)sddmm_slab_gather_kernel<KPL, VMODE, 4>;
     if constexpr (VMODE == 2) {
         if (slice == 1) return (TileFn)sddmm_slab_gather_kernel<KPL, VMODE, 1>;

@@ -912,8 +912,11 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
             // (where the model above has its say it chooses the slabs; this is for plans whose caller set a threshold,
             // and for slices of less than 64 elements)
             const bool huge_h = slab_cols > 0 || (rl.empty() && D.n_dense == 0 && (int64_t)n_cols * K * 4 > ((int64_t)256 << 20));
-            int gg = opt.gather_lanes > 0 ? opt.gather_lanes : 8;
-            if (huge_h && opt.gather_lanes <= 0 && opt.gather_slab_cols != 0 && pick_tile_variant(kt, 4).G) gg = 4;
+            // Groups of 4 positions: less padding than groups of 8 (short rows of the recommender, 12 nonzeros on average: 5.9 M
+            // positions for 5.2 M nonzeros, and 7.0), and no slower a kernel.  us per product, 8 and 4: recommender, K = 32 / 64 /
+            // 128 / 256 / 512 382 / 560 / 811 / 1610 / 2870 and 377 / 554 / 803 / 1575 / 2750; 20 million nonzeros, K = 64 / 128 / 256
+            // / 512 119 / 174 / 364 / 634 and 115 / 170 / 350 / 596; 10 million, K = 128 / 512 103 / 359 and 95 / 342.
+            const int gg = opt.gather_lanes > 0 ? opt.gather_lanes : pick_tile_variant(kt, 4).G ? 4 : 8;
             const bool slabs = !ragged && huge_h && opt.gather_slab_cols != 0 && opt.gather_padded != 0 && pick_tile_variant(kt, gg).G != 0;
             const bool padded = !ragged && opt.gather_padded != 0 && pick_tile_variant(kt, gg).G != 0 && (!rl.empty() || D.n_dense > 0 || slabs);
             if (padded) {

@@ -818,7 +818,11 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         // over its own positions slice after slice (K=256, ms per step: bag-of-words 0.0328 -> 0.0309; recommender
         // shape at 1.1 M nonzeros 0.0381 -> 0.0345, at 5.3 M 0.1267 -> 0.1218).  Not for large streams, whose
         // workgroups share W rows in L2 by being on the same slice at the same time (99.8 M: 1.710 -> 1.742).
-        L.fused_slices = c.opt.fuse_slices >= 0 ? (c.opt.fuse_slices != 0) : (np <= ((int64_t)1 << 23));
+        // The gather form's waves share H rows in L2 by being on the same slice, so there the line is where its workgroups
+        // no longer run all at once (us, groups of 4, K = 512, one launch and one per slice: 0.1 / 0.25 / 0.5 / 1 million positions
+        // of ratings 14.7 / 28.5 / 55.0 / 101 and 21.3 / 33.3 / 57.4 / 96, of R-MAT 16.4 / 33.8 / 87 / 210 and 24.3 / 37.3 / 68 / 168;
+        // 5.9 million of the recommender's short rows, groups of 8: 893 and 769).
+        L.fused_slices = c.opt.fuse_slices >= 0 ? (c.opt.fuse_slices != 0) : np <= (gather ? (int64_t)5 << 16 : (int64_t)1 << 23);
     }
     if (gather) {
         float *d_sink = nullptr;

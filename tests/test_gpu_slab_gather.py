@@ -1,5 +1,6 @@
 """The padded gather on groups of 4 positions (eight lanes, two rows of W at a time): streams that end inside a batch, with one
-group or two in the last eight positions, padding flagged or repeated, one K slice or several, against 64-bit sums."""
+group or two in the last eight positions, padding flagged or repeated, one K slice or several (in one launch and one by one),
+against 64-bit sums."""
 import pytest
 import torch
 
@@ -8,10 +9,10 @@ from sddmm_gpu_amd import capi
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("K", [32, 64, 128, 384])
+@pytest.mark.parametrize("K,fuse", [(32, -1), (64, -1), (128, -1), (384, -1), (384, 0)])
 @pytest.mark.parametrize("n_rows,n_cols,nnz", [(1, 5, 1), (2, 9, 7), (3, 40, 64), (17, 50, 130), (301, 97, 5003), (40, 3000, 9001)])
 @pytest.mark.parametrize("sink,slab", [(1, 16), (0, 16), (1, 1 << 20)])
-def test_against_64_bits(n_rows, n_cols, nnz, K, sink, slab):
+def test_against_64_bits(n_rows, n_cols, nnz, K, fuse, sink, slab):
     g = torch.Generator().manual_seed(nnz + K)
     keys = torch.randperm(n_rows * n_cols, generator=g)[:nnz].sort().values
     rows, cols = keys // n_cols, keys % n_cols
@@ -24,8 +25,9 @@ def test_against_64_bits(n_rows, n_cols, nnz, K, sink, slab):
     rp, ci, dW, dH, dv = (t.cuda() for t in (row_ptr.int(), cols.int(), W, H, val))
     plan = capi.Plan.from_device_csr(n_rows, n_cols, nnz, rp.data_ptr(), ci.data_ptr(), K,
                                      options=capi.PlanOptions.defaults(kernel=capi.KERNEL_ROW_GATHER, row_padded=1, gather_lanes=4, gather_sink=sink,
-                                                                       k_slice=128 if K > 128 else 0, gather_slab_cols=slab, ignore_env=1))
+                                                                       k_slice=128 if K > 128 else 0, fuse_slices=fuse, gather_slab_cols=slab, ignore_env=1))
     assert plan.info()["padded_positions"] % 4 == 0 and plan.info()["padded_positions"] >= nnz
+    assert plan.info()["n_launches"] == (3 if fuse == 0 else 1)
     stream = torch.cuda.current_stream().cuda_stream
     out = torch.full((nnz + 1,), 7.0, device="cuda")
 
