@@ -362,7 +362,7 @@ namespace sddmm {
 
 // The smallest number of lanes whose pieces cover a row, at least 8 (128 contiguous bytes per gathered row) from
 // K = 17 on; K < 4 and K > 2048 are left to the generic kernel (G == 0).
-Variant pick_gather_variant(int K)
+static Variant pick_gather_variant(int K)
 {
     const int K4 = (K + 3) / 4;
     const int cand[][2] = {{4, 1}, {8, 1}, {8, 2}, {8, 3}, {8, 4}, {16, 3}, {16, 4}, {32, 3}, {32, 4}, {64, 3}, {64, 4}, {64, 8}};
@@ -380,23 +380,34 @@ Variant pick_gather_variant(int K)
 //       256 18 / 24 / 56 and 16 / 22 / 49, 3.9 million of 30, K = 32 / 96 72 / 218 and 69 / 199; but 0.24 million of 30, K =
 //       100 / 128 / 256 11.3 / 12.0 / 28.0 and 12.7 / 13.0 / 25.8, 0.9 million, K = 32 13.2 and 14.3, and up to K = 16
 //       R-MAT, 28 million of 27, 344 and 381.
-//   K = 33 to 63, where a quarter to a half of the lanes' pieces are masked: several batches (R-MAT, 1.4 / 3.4 / 28 million,
-//       K = 40 35 / 80 / 648 and 40 / 89 / 835; rows of uniform length would gain 3 to 13 %).  K = 64 gains from half a
-//       million on (R-MAT, 2.1 / 28 million 74 / 1014 and 63 / 905), below it does not (0.2 million of 8 a row 10.2 and 10.6).
+//   K = 33 to 64: one batch where sixteen lanes take a piece each (see below); with eight lanes and two pieces one batch was
+//       the slower form (R-MAT, 1.4 / 3.4 / 28 million, K = 40 35 / 80 / 648 and 40 / 89 / 835).
 //   longer rows: only up to K = 32 and 2^18 nonzeros (0.19 million of 323 a row, K = 16 / 32 / 64 4.5 / 4.7 / 5.5 and 3.8 /
 //       4.5 / 5.8; 0.8 million, K = 32 8.9 and 11.0).
 // Batches a wave: up to 8, which is as many as share a search for the rows, but fewer where that would leave less than 4096
 // waves (16 per compute unit): 0.9 million nonzeros, K = 32 / 64 / 128 with 2048 waves 27 / 30 / 49, with 4096 19 / 23 / 44; from
 // 1.5 million on all take 8 (two million of 20,000 rows, K = 64: 35, and 38 with 7).
-GatherShape gather_shape(int64_t nnz, int64_t n_rows, const Variant &v)
+//
+// With one batch a wave, from 2^18 nonzeros on, a row of up to 64 floats, or of 97 to 127, is read by as many lanes as it has
+// pieces, in one request a line (rows of such lengths begin anywhere in a line: eight lanes' 128 bytes lie in two lines each,
+// and the next piece's in the second of them again).  us, 8 lanes and 16 or 32: R-MAT, 0.55 million, K = 45 / 50 / 60 / 64 /
+// 100 / 120 20.8 / 20.4 / 21.5 / 17.5 / 26.7 / 28.4 and 16.7 / 16.6 / 17.2 / 15.9 / 25.7 / 26.7; 1.8 million 45 / 46 / 50 / 49 /
+// 76 / 81 and 43 / 43 / 46 / 42 / 71 / 78; 8.4 million 211 / 225 / 254 / 250 / 412 / 454 and 202 / 210 / 234 / 237 / 393 / 442.  Not
+// where a third of the lanes would idle in large matrices (K = 36, 1.8 / 8.4 million: 41 / 176 and 41 / 180), nor at K = 65 to
+// 96 (1.8 million, K = 72 / 90 57 / 65 and 66 / 69) and beyond 128 (K = 150 / 200 104 / 137 and 113 / 135), nor below (0.17
+// million, K = 50 / 100: 6.7 / 10.1 and 6.8 / 10.4), nor with several batches (R-MAT 2^15, 1.2 million, K = 100: 41 and 46).
+GatherShape gather_shape(int64_t nnz, int64_t n_rows, int K)
 {
-    const int pieces = v.G * v.KPL;
+    Variant v = pick_gather_variant(K);
+    const int pieces = v.G * v.KPL, used = (K + 3) / 4;
     const bool short_rows = nnz <= (pieces > 4 && nnz * pieces >= 8000000 ? 32 : 16) * n_rows;
-    const bool once = v.G != 0 && (nnz <= 1 << 16 || (short_rows ? pieces != 16 || (v.exact && nnz >= 1 << 19) : pieces <= 8 && nnz <= 1 << 18));
+    const bool line_wise = nnz >= 1 << 18 && ((pieces == 16 && (used >= 10 || nnz < 1 << 20)) || (pieces == 32 && !v.exact));
+    const bool once = v.G != 0 && (nnz <= 1 << 16 || (short_rows ? pieces != 16 || line_wise : pieces <= 8 && nnz <= 1 << 18));
+    if (once && line_wise) v = {pieces, 1, v.exact};
     const int64_t waves_wanted = 4096;
     const int per_wave = once ? 1 : nnz >= 1500000 ? kRowGatherBatchesPerWave
                                                    : (int)std::clamp<int64_t>(nnz / (64 * waves_wanted), 1, kRowGatherBatchesPerWave);
-    return {64 * per_wave * (kRowGatherBlock / 64), once};
+    return {v, 64 * per_wave * (kRowGatherBlock / 64), once};
 }
 
 KernelFn gather_kernel(const Variant &v, bool once, bool wide)
@@ -404,6 +415,11 @@ KernelFn gather_kernel(const Variant &v, bool once, bool wide)
 #define SDDMM_FORM(g, kpl, ragged)                                                                                        \
     (once ? (wide ? (KernelFn)sddmm_gather_once_kernel<g, kpl, ragged, true> : (KernelFn)sddmm_gather_once_kernel<g, kpl, ragged, false>) \
           : (wide ? (KernelFn)sddmm_gather_kernel<g, kpl, ragged, true> : (KernelFn)sddmm_gather_kernel<g, kpl, ragged, false>))
+    // (read line by line: one batch a wave only, and 32 lanes for ragged ranks only)
+#define SDDMM_LINE_WISE(g, ragged) (wide ? (KernelFn)sddmm_gather_once_kernel<g, 1, ragged, true> : (KernelFn)sddmm_gather_once_kernel<g, 1, ragged, false>)
+    if (v.KPL == 1 && v.G == 16) return !once ? nullptr : v.exact ? SDDMM_LINE_WISE(16, false) : SDDMM_LINE_WISE(16, true);
+    if (v.KPL == 1 && v.G == 32) return !once || v.exact ? nullptr : SDDMM_LINE_WISE(32, true);
+#undef SDDMM_LINE_WISE
 #define SDDMM_CASE(g, kpl) \
     if (v.G == g && v.KPL == kpl) return v.exact ? SDDMM_FORM(g, kpl, false) : SDDMM_FORM(g, kpl, true);
     SDDMM_CASE(4, 1) SDDMM_CASE(8, 1) SDDMM_CASE(8, 2) SDDMM_CASE(8, 3) SDDMM_CASE(8, 4) SDDMM_CASE(16, 3) SDDMM_CASE(16, 4)

@@ -21,14 +21,13 @@ extern "C" int sddmm_csr_noalloc(int64_t n_rows, int64_t n_cols, int64_t nnz, co
     if (!d_row_ptr || !d_col_ind || !d_W || !d_H || !d_out) return fail(SDDMM_ERR_ARG, "sddmm_csr_noalloc: NULL device pointer");
     if ((((uintptr_t)d_W | (uintptr_t)d_H) & 15u) && K % 4 == 0)
         return fail(SDDMM_ERR_ARG, "sddmm_csr_noalloc: W and H must be 16-byte aligned");
-    const Variant var = pick_gather_variant(K);
 
     KArgs a{};
     a.col_ind = d_col_ind; a.val = d_val; a.W = d_W; a.H = d_H; a.out = d_out;
     a.row_ptr = d_row_ptr; a.n_rows = (int32_t)n_rows;
     a.nnz = (int32_t)nnz; a.K = K; a.n_cols = (int32_t)n_cols; a.tile_x = (int32_t)n_cols;
-    const GatherShape shape = gather_shape(nnz, n_rows, var);
-    const KernelFn fn = var.G ? gather_kernel(var, shape.once, gather_wide(n_rows, n_cols, K)) : generic_kernel();
+    const GatherShape shape = gather_shape(nnz, n_rows, K);
+    const KernelFn fn = shape.v.G ? gather_kernel(shape.v, shape.once, gather_wide(n_rows, n_cols, K)) : generic_kernel();
     a.chunk = shape.chunk;
     const int grid = (int)((nnz + a.chunk - 1) / a.chunk);
     const hipError_t e = launch(fn, dim3((unsigned)grid), dim3(kRowGatherBlock), 0, (hipStream_t)stream, a);

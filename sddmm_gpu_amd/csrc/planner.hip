@@ -256,7 +256,8 @@ int add_row_gather(Ctx &c, const std::vector<int32_t> &rows, bool all_rows)
     const int64_t n = all_rows ? c.nnz : list_nnz(c, rows);
     L.nnz = n;
     if (n == 0) return SDDMM_OK;
-    const Variant var = pick_gather_variant(c.K);
+    const GatherShape shape = gather_shape(n, (int64_t)rows.size(), c.K);
+    const Variant var = shape.v;
     L.fn_kind = 1; L.fn_g = var.G; L.fn_kpl = var.KPL; L.fn_exact = var.exact;
     std::vector<int32_t> seg_end(rows.size()), perm;
     int64_t acc = 0;
@@ -288,7 +289,6 @@ int add_row_gather(Ctx &c, const std::vector<int32_t> &rows, bool all_rows)
     a.seg_row = d_seg_row; a.perm = d_perm; a.batch_seg = d_bseg; a.batch_mask = d_bmask;
     L.perm = d_perm;
     a.nnz = (int32_t)n;
-    const GatherShape shape = gather_shape(n, (int64_t)rows.size(), var);
     a.chunk = shape.chunk;
     L.fn_once = shape.once;
     L.fn_wide = gather_wide(c.n_rows, c.n_cols, c.K);
