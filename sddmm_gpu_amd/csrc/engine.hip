@@ -292,7 +292,7 @@ int sddmm_plan_spmm(const sddmm_plan *plan, const float *d_x, const float *d_H, 
     if (I.n_rows == 0) return SDDMM_OK;
     if (!d_Y || (I.nnz > 0 && (!d_x || !d_H))) return fail(SDDMM_ERR_ARG, "sddmm_plan_spmm: NULL device pointer");
     const Launch *Ls = spmm_launch(plan);
-    if (!Ls || (Ls->sp_on == 1 && ((((uintptr_t)d_H) | ((uintptr_t)d_Y)) & 15u))) {
+    if (!Ls || (Ls->sp_on == 1 && !Ls->fn_ragged && ((((uintptr_t)d_H) | ((uintptr_t)d_Y)) & 15u))) {
         // no tile stream for the product in this plan: the CSR form, gathering H rows
         if (!plan->d_row_ptr || (I.nnz > 0 && !plan->d_col)) return fail(SDDMM_ERR_ARG, "sddmm_plan_spmm: the plan holds no pattern");
         return sddmm_spmm_csr(I.n_rows, I.n_cols, I.nnz, plan->d_row_ptr, plan->d_col, d_x, I.K, d_H, d_Y, stream);
@@ -315,9 +315,10 @@ int sddmm_plan_spmm(const sddmm_plan *plan, const float *d_x, const float *d_H, 
     sa.x = d_x; sa.H = d_H; sa.Y = d_Y;
     sa.row_ptr = plan->d_row_ptr; sa.col_ind = plan->d_col;
     if (d_workspace) sa.part = reinterpret_cast<float *>(static_cast<char *>(d_workspace) + Ls->ws_sp_part);
-    for (int k_off = 0; k_off < I.K; k_off += Ls->k_slice) {
+    const int width = 4 * Ls->fn_g * Ls->fn_kpl;  // (k_slice is K where a wider kernel covers a ragged rank)
+    for (int k_off = 0; k_off < I.K; k_off += width) {
         sa.k_off = k_off;
-        launch_spmm_slice(sa, Ls->k_slice, Ls->sp_nwaves, Ls->sp_grid, Ls->k_slice * 4 * Ls->ta.tile_x, stream);
+        launch_spmm_slice(sa, width, Ls->sp_nwaves, Ls->sp_grid, width * 4 * Ls->ta.tile_x, stream);
     }
     HIP_TRY(hipGetLastError());
     return SDDMM_OK;

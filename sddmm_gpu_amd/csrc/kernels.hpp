@@ -151,7 +151,7 @@ struct SpmmArgs {
     int32_t tile_x, n_cols, K, k_off;
 };
 bool spmm_tile_supported(int k_slice);
-int spmm_tile_set_lds(int k_slice, int nwaves, int lds_bytes);  // 0 ok, 1 no such variant, 2 HIP error
+int spmm_tile_set_lds(int k_slice, int nwaves, bool ragged, int lds_bytes);  // 0 ok, 1 no such variant, 2 HIP error
 void launch_spmm_slice(const SpmmArgs &a, int k_slice, int nwaves, int grid, int lds_bytes, void *stream);
 
 // The product over a plain CSR pattern without atomics (K >= 4, kernels_spmm_csr.hip): d_part holds spmm_csr_records(nnz, K)

@@ -11,8 +11,15 @@
 // wave walk 8 runs side by side ("bundle"); the planner sorts an item's runs by length, so a
 // bundle's runs are about equally long.  Rows too short for the tiles gather their H rows from
 // global memory, one group of lanes per row.
+//
+// RAGGED: K is no multiple of the kernel's width, and K needs no alignment: tiles and partial rows have the full width, with
+// the tail of H rows filled up with zeros, the last piece of a row is read from its last four floats on (see RowPiece) and
+// only what is new in it goes to Y.  us per product, by the walk over the CSR pattern and so: ratings of 4.9 million nonzeros,
+// K = 50 / 100 / 250 / 300 68 / 102 / 240 / 395 and 54 / 88 / 183 / 273; 15.9 million, K = 50 / 100 / 250 / 300 175 / 286 / 984 /
+// 1672 and 122 / 258 / 553 / 804 (when it is chosen: ragged_product_tiles).
 #include <hip/hip_runtime.h>
 #include <utility>
+#include "csr_walk.hpp"
 #include "kernels.hpp"
 
 using namespace sddmm;
@@ -33,7 +40,7 @@ __device__ __forceinline__ int from_group_lane(int v, bool upper_group)
 }
 
 // KPL float4 per lane: a K slice of 32 * KPL elements on groups of 8 lanes
-template <int KPL, int NW>
+template <int KPL, int NW, bool RAGGED>
 __global__ __launch_bounds__(NW * 64)
 void sddmm_spmm_tile_kernel(const SpmmArgs a)
 {
@@ -68,7 +75,13 @@ void sddmm_spmm_tile_kernel(const SpmmArgs a)
             const int n4 = rows * K4;
             for (int i = threadIdx.x; i < n4; i += NW * 64) {
                 const int r = i / K4, q = i - r * K4;
-                lds_tile[i] = src[(size_t)r * row_k4 + q];
+                if constexpr (RAGGED) {
+                    const RowPiece pc = row_piece(q, a.K - a.k_off);
+                    const vec4u v = *reinterpret_cast<const vec4u *>(a.H + ((size_t)(tile_base + r) * a.K + a.k_off) + pc.off);
+                    lds_tile[i] = make_float4(pc.first > 0 ? 0.f : v.x, pc.first > 1 ? 0.f : v.y, pc.first > 2 ? 0.f : v.z, pc.first > 3 ? 0.f : v.w);
+                } else {
+                    lds_tile[i] = src[(size_t)r * row_k4 + q];
+                }
             }
             __syncthreads();
         }
@@ -147,9 +160,28 @@ void sddmm_spmm_tile_kernel(const SpmmArgs a)
     }
 }
 
+// A lane's piece of a row of Y.
+template <bool RAGGED>
+__device__ __forceinline__ void store_piece(const SpmmArgs &a, int row, int slot, const float4 &v)
+{
+    if constexpr (RAGGED) {
+        const RowPiece pc = row_piece(slot, a.K - a.k_off);
+        float *y = a.Y + ((size_t)row * a.K + a.k_off) + pc.off;
+        if (pc.first == 0) {
+            *reinterpret_cast<vec4u *>(y) = vec4u{v.x, v.y, v.z, v.w};
+        } else {
+            if (pc.first <= 1) y[1] = v.y;
+            if (pc.first <= 2) y[2] = v.z;
+            if (pc.first <= 3) y[3] = v.w;
+        }
+    } else {
+        reinterpret_cast<float4 *>(a.Y)[(size_t)row * (a.K >> 2) + (a.k_off >> 2) + slot] = v;
+    }
+}
+
 // Y[row, slice] = sum of the row's partial rows: one wave per listed row, group g takes the partial
 // rows g, g + 8, ... and the groups' sums are added across the wave.
-template <int KPL>
+template <int KPL, bool RAGGED>
 __device__ __forceinline__ void spmm_sum_rows(const SpmmArgs &a, int64_t block)
 {
     constexpr int G = 8, K4 = G * KPL;
@@ -178,16 +210,16 @@ __device__ __forceinline__ void spmm_sum_rows(const SpmmArgs &a, int64_t block)
         }
     }
     if (g == 0) {
-        float4 *y = reinterpret_cast<float4 *>(a.Y) + (size_t)a.sum_rows[w] * (a.K >> 2) + (a.k_off >> 2);
+        const int row = a.sum_rows[w];
 #pragma unroll
-        for (int j = 0; j < KPL; ++j) y[j * G + l] = acc[j];
+        for (int j = 0; j < KPL; ++j) store_piece<RAGGED>(a, row, j * G + l, acc[j]);
     }
 }
 
 // The rows outside the tiles (short ones, and rows without entries, which become 0): one group of 8
 // lanes per row, H rows gathered from global memory, four nonzeros in flight per step; the planner lists
 // the rows longest first, so that the eight rows of a wave are about equally long.
-template <int KPL>
+template <int KPL, bool RAGGED>
 __device__ __forceinline__ void spmm_gather_rows(const SpmmArgs &a, int64_t block)
 {
     constexpr int G = 8;
@@ -198,13 +230,26 @@ __device__ __forceinline__ void spmm_gather_rows(const SpmmArgs &a, int64_t bloc
     const int b = a.row_ptr[row], e = a.row_ptr[row + 1];
     const int row_k4 = a.K >> 2;
     const float4 *__restrict__ H4 = reinterpret_cast<const float4 *>(a.H) + (a.k_off >> 2) + l;
+    int off[RAGGED ? KPL : 1];
+    if constexpr (RAGGED) {
+#pragma unroll
+        for (int j = 0; j < KPL; ++j) off[j] = row_piece(j * G + l, a.K - a.k_off).off;
+    }
+    auto h_piece = [&](int c, int j) -> float4 {
+        if constexpr (RAGGED) {  // (what is not new in a piece is added up as well, and not stored)
+            const vec4u v = *reinterpret_cast<const vec4u *>(a.H + ((size_t)c * a.K + a.k_off) + off[j]);
+            return make_float4(v.x, v.y, v.z, v.w);
+        } else {
+            return H4[(size_t)c * row_k4 + j * G];
+        }
+    };
     float4 acc[KPL];
 #pragma unroll
     for (int j = 0; j < KPL; ++j) acc[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-    auto add = [&](const float4 *hr, float xs) {
+    auto add = [&](int c, float xs) {
 #pragma unroll
         for (int j = 0; j < KPL; ++j) {
-            const float4 h = hr[j * G];
+            const float4 h = h_piece(c, j);
             acc[j].x = fmaf(xs, h.x, acc[j].x); acc[j].y = fmaf(xs, h.y, acc[j].y);
             acc[j].z = fmaf(xs, h.z, acc[j].z); acc[j].w = fmaf(xs, h.w, acc[j].w);
         }
@@ -218,7 +263,7 @@ __device__ __forceinline__ void spmm_gather_rows(const SpmmArgs &a, int64_t bloc
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int j = 0; j < KPL; ++j) hh[i][j] = H4[(size_t)cc[i] * row_k4 + j * G];
+            for (int j = 0; j < KPL; ++j) hh[i][j] = h_piece(cc[i], j);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -227,23 +272,22 @@ __device__ __forceinline__ void spmm_gather_rows(const SpmmArgs &a, int64_t bloc
                 acc[j].z = fmaf(xx[i], hh[i][j].z, acc[j].z); acc[j].w = fmaf(xx[i], hh[i][j].w, acc[j].w);
             }
     }
-    for (; p < e; ++p) add(H4 + (size_t)a.col_ind[p] * row_k4, a.x[p]);
-    float4 *y = reinterpret_cast<float4 *>(a.Y) + (size_t)row * row_k4 + (a.k_off >> 2) + l;
+    for (; p < e; ++p) add(a.col_ind[p], a.x[p]);
 #pragma unroll
-    for (int j = 0; j < KPL; ++j) y[j * G] = acc[j];
+    for (int j = 0; j < KPL; ++j) store_piece<RAGGED>(a, row, j * G + l, acc[j]);
 }
 
 // Second kernel of a slice: the sums of the partial rows (a stream through memory) and the rows outside
 // the tiles (gathers from L2) side by side, sum_blocks and gather_blocks workgroups of each spread evenly
 // over the grid, so that the two kinds of traffic overlap.
-template <int KPL>
+template <int KPL, bool RAGGED>
 __global__ __launch_bounds__(256)
 void sddmm_spmm_rows_kernel(const SpmmArgs a, int64_t sum_blocks, int64_t gather_blocks)
 {
     const int64_t i = blockIdx.x, n = sum_blocks + gather_blocks;
     const int64_t sums_before = i * sum_blocks / n;  // (of the workgroups 0 .. i - 1)
-    if ((i + 1) * sum_blocks / n > sums_before) spmm_sum_rows<KPL>(a, sums_before);
-    else spmm_gather_rows<KPL>(a, i - sums_before);
+    if ((i + 1) * sum_blocks / n > sums_before) spmm_sum_rows<KPL, RAGGED>(a, sums_before);
+    else spmm_gather_rows<KPL, RAGGED>(a, i - sums_before);
 }
 
 }  // namespace
@@ -255,16 +299,18 @@ bool spmm_tile_supported(int k_slice)
     return k_slice == 32 || k_slice == 64 || k_slice == 128;
 }
 
-int spmm_tile_set_lds(int k_slice, int nwaves, int lds_bytes)
+using SpmmFn = void (*)(const SpmmArgs);
+
+int spmm_tile_set_lds(int k_slice, int nwaves, bool ragged, int lds_bytes)
 {
-    const void *fn = nullptr;
-#define SDDMM_SPMM_FN(kpl) (nwaves == 12 ? (const void *)sddmm_spmm_tile_kernel<kpl, 12> : (const void *)sddmm_spmm_tile_kernel<kpl, 16>)
+    SpmmFn fn = nullptr;
+#define SDDMM_SPMM_FN(kpl) (ragged ? (nwaves == 12 ? (SpmmFn)sddmm_spmm_tile_kernel<kpl, 12, true> : (SpmmFn)sddmm_spmm_tile_kernel<kpl, 16, true>) \
+                                   : (nwaves == 12 ? (SpmmFn)sddmm_spmm_tile_kernel<kpl, 12, false> : (SpmmFn)sddmm_spmm_tile_kernel<kpl, 16, false>))
     if (k_slice == 128) fn = SDDMM_SPMM_FN(4);
     else if (k_slice == 64) fn = SDDMM_SPMM_FN(2);
     else if (k_slice == 32) fn = SDDMM_SPMM_FN(1);
-#undef SDDMM_SPMM_FN
     if (!fn) return 1;
-    return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) == hipSuccess ? 0 : 2;
+    return hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) == hipSuccess ? 0 : 2;
 }
 
 // one K slice of the product: the tile kernel over the bundles, the sum of the partial rows, the gathered rows
@@ -273,19 +319,20 @@ void launch_spmm_slice(const SpmmArgs &a, int k_slice, int nwaves, int grid, int
     hipStream_t st = (hipStream_t)stream;
     const unsigned sum_grid = (unsigned)((a.n_sum_rows + 3) / 4);
     const unsigned rows_grid = (unsigned)((a.n_gather_rows + 31) / 32);
-#define SDDMM_SPMM_LAUNCH(kpl)                                                                                         \
-    do {                                                                                                               \
-        if (a.n_items > 0) {                                                                                           \
-            if (nwaves == 12) hipLaunchKernelGGL((sddmm_spmm_tile_kernel<kpl, 12>), dim3((unsigned)grid), dim3(12 * 64), (size_t)lds_bytes, st, a); \
-            else hipLaunchKernelGGL((sddmm_spmm_tile_kernel<kpl, 16>), dim3((unsigned)grid), dim3(16 * 64), (size_t)lds_bytes, st, a);              \
-        }                                                                                                              \
-        if (sum_grid + rows_grid > 0)                                                                                  \
-            hipLaunchKernelGGL((sddmm_spmm_rows_kernel<kpl>), dim3(sum_grid + rows_grid), dim3(256), 0, st, a, (int64_t)sum_grid, (int64_t)rows_grid); \
+    const bool ragged = a.K % k_slice != 0;
+#define SDDMM_SPMM_LAUNCH(kpl)                                                                                          \
+    do {                                                                                                                \
+        if (a.n_items > 0)                                                                                              \
+            hipLaunchKernelGGL(SDDMM_SPMM_FN(kpl), dim3((unsigned)grid), dim3(nwaves == 12 ? 12 * 64 : 16 * 64), (size_t)lds_bytes, st, a); \
+        if (sum_grid + rows_grid > 0)                                                                                   \
+            hipLaunchKernelGGL((ragged ? sddmm_spmm_rows_kernel<kpl, true> : sddmm_spmm_rows_kernel<kpl, false>), dim3(sum_grid + rows_grid), dim3(256), 0, st, \
+                               a, (int64_t)sum_grid, (int64_t)rows_grid);                                               \
     } while (0)
     if (k_slice == 128) SDDMM_SPMM_LAUNCH(4);
     else if (k_slice == 64) SDDMM_SPMM_LAUNCH(2);
     else if (k_slice == 32) SDDMM_SPMM_LAUNCH(1);
 #undef SDDMM_SPMM_LAUNCH
+#undef SDDMM_SPMM_FN
 }
 
 }  // namespace sddmm

@@ -164,6 +164,17 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
 // 2.8 where the tiles take slices of 64 (tiles against walk, ratings of 1.8, 2.4 and 3.6 M, K = 256: 108 / 101, 123 / 139 and
 // 167 / 190 us; of 2.6 and 3.8 M, K = 192: 148 / 131 and 180 / 184; K = 320, 1.8 and 2.6 M: 231 / 171 and 240 / 259).
 inline bool product_walks(int64_t nnz, int32_t K, int ks) { return nnz < 4000000 && nnz * K < (ks < 128 ? 700000000 : 450000000); }
+// And at a rank that is no multiple of the tiles' width ks, which they work on up to the next multiple?  From 4 million nonzeros
+// on they are the faster ones where little of that is padding (SDDMM + product, us, walk and tiles: ratings of 4.9 M, K = 20 / 30
+// / 36 / 50 / 75 / 120 68 / 77 / 95 / 102 / 160 / 179 and 73 / 75 / 90 / 92 / 143 / 153, K = 150 / 180 / 200 / 250 / 300 / 380 274 /
+// 285 / 313 / 368 / 577 / 624 and 282 / 290 / 293 / 305 / 441 / 457; 15.9 M, K = 50 / 120 / 150 / 200 / 300 257 / 506 / 780 / 964 / 2118
+// and 215 / 422 / 791 / 829 / 1250); below, where the walk has three slices or more (3.3 M, K = 200 / 220 / 250 / 280 / 340: 208 /
+// 218 / 240 / 387 / 402 and 248 / 250 / 253 / 365 / 370).
+inline bool ragged_product_tiles(int64_t nnz, int32_t K, int ks)
+{
+    const int padded = (K + ks - 1) / ks * ks;
+    return nnz < 4000000 ? K > 256 && !product_walks(nnz, K, ks) : K >= 28 && (K <= 128 || K * 100 >= padded * 72);
+}
 // planner_tile.hip: the rows' nonzeros in tile order (tiles of x columns), every (row, tile) run padded
 // ks: K elements per launch, a divisor of K or (ragged ranks) the width K is rounded up to
 int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t panel_rows, int want_g, int ks,

@@ -139,7 +139,7 @@ int resolve_functions(Launch &L)
     }
     case 3: {
         const TileVariant tv{L.fn_g, L.fn_kpl};
-        if (L.sp_on == 1 && spmm_tile_set_lds(L.k_slice, L.sp_nwaves, L.k_slice * 4 * L.ta.tile_x) != 0)
+        if (L.sp_on == 1 && spmm_tile_set_lds(4 * L.fn_g * L.fn_kpl, L.sp_nwaves, L.fn_ragged != 0, 16 * L.fn_g * L.fn_kpl * L.ta.tile_x) != 0)
             return fail(SDDMM_ERR_HIP, "plan: cannot set up the tile kernel of the product Y = X H");
         if (L.fn_nwm > 0) {  // (a launch with a matrix-core share covers all of K: one form per value mode)
             for (int vm = 0; vm < 5; ++vm) {
@@ -872,7 +872,7 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         // 213 + 338 / 188 + 500).  Below 4 million nonzeros the split is the model's: the fixed rules make one class of the rows
         // there, and the product mostly walks the CSR pattern (3 to 4 M, K = 256, windows: 196 + 174 by the fixed rules,
         // 113 + 169 by the model; uniform 522 + 517 and 332 + 515).
-        const bool tiled_product = opt.spmm_stream > 0 && nnz >= 4000000 && !ragged && spmm_tile_supported(kt);
+        const bool tiled_product = opt.spmm_stream > 0 && nnz >= 4000000 && (!ragged || ragged_product_tiles(nnz, K, kt)) && spmm_tile_supported(kt);
         const bool by_model = D.n_dense == 0 && opt.short_row_max < 0 && opt.stage_factor < 0 && opt.split_min_nnz < 0 && !tiled_product;
         int64_t slab_cols = 0;  // chosen by the model
         if (by_model) {

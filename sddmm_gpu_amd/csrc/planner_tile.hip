@@ -245,7 +245,7 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         // runs of 4 647 / 543).
         const bool h_near = (int64_t)c.n_cols * c.K * 4 <= 6000000;
         if (want_spmm && rb == 0 && c.nnz == c.P->info.nnz &&
-            (ragged || (h_near && (L.nnz < 12 * n_seg || product_walks(c.nnz, c.K, ks))) || L.nnz < (c.K <= 128 ? 8 : 5) * n_seg)) { want_spmm = false; sp_csr = true; }
+            ((ragged && !ragged_product_tiles(c.nnz, c.K, ks)) || (h_near && (L.nnz < 12 * n_seg || product_walks(c.nnz, c.K, ks))) || L.nnz < (c.K <= 128 ? 8 : 5) * n_seg)) { want_spmm = false; sp_csr = true; }
         // row-block boundaries of the 2-D assignment: equal shares of the rows' nonzeros
         std::vector<int32_t> cut;
         auto make_cuts = [&](int n_shares) {
