@@ -118,6 +118,7 @@ struct Ctx {
     // original positions: that is where outputs go and where values come from.
     const int32_t *orig = nullptr;
     sddmm_plan_options opt{};  // the caller's options with the environment overrides applied
+    int64_t sp_min_row = 0;    // the product on column tiles: rows of fewer nonzeros gather their H rows
     int32_t pos(int64_t p) const { return orig ? orig[p] : (int32_t)p; }
     float value(int64_t p) const { return vals[orig ? orig[p] : p]; }
 

@@ -866,14 +866,21 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         // By default the split that a model of the three kernels finds cheapest (see estimate_split): all rows tiled,
         // the long ones tiled and the short ones gathered, or all gathered.  A caller who sets one of the thresholds,
         // and the remainder of a dense core, get the fixed rules.
-        // So do plans that also serve the product with the dense factor on column tiles: that product wants long runs, and
-        // tiling the short rows as well, 10 % faster for the SDDMM alone, costs it more (ratings, SDDMM + product, us by
-        // length / all tiled: 15.7 M nonzeros, K = 64 93 + 132 / 82 + 229; 5.4 M, K = 128 64 + 103 / 67 + 145; 11.8 M, K = 192
-        // 213 + 338 / 188 + 500).  Below 4 million nonzeros the split is the model's: the fixed rules make one class of the rows
+        // Plans that also serve the product with the dense factor on column tiles, from 4 million nonzeros on, tile all rows
+        // for the SDDMM where the model finds that cheapest and K slices are of 64 at most, and the long ones (by the fixed rules)
+        // alone for the product, which wants long runs; otherwise the fixed rules hold for both.  SDDMM + product, us, long rows
+        // in both and so: ratings of 4.9 M, K = 32 / 50 / 64 / 192 24 + 50 / 38 + 55 / 34 + 54 / 105 + 160 and 21 + 49 / 33 + 55 / 31
+        // + 55 / 92 + 161, of 15.9 M 56 + 98 / 90 + 125 / 84 + 124 / 267 + 349 and 49 + 99 / 81 + 125 / 76 + 126 / 255 + 351; slices of
+        // 128, K = 100 / 128, 4.9 M: 59 + 91 / 56 + 93 and 64 + 91 / 65 + 94; all rows in both, 15.7 M, K = 64: 82 + 229.  Below 4 million nonzeros the split is the model's: the fixed rules make one class of the rows
         // there, and the product mostly walks the CSR pattern (3 to 4 M, K = 256, windows: 196 + 174 by the fixed rules,
         // 113 + 169 by the model; uniform 522 + 517 and 332 + 515).
         const bool tiled_product = opt.spmm_stream > 0 && nnz >= 4000000 && (!ragged || ragged_product_tiles(nnz, K, kt)) && spmm_tile_supported(kt);
-        const bool by_model = D.n_dense == 0 && opt.short_row_max < 0 && opt.stage_factor < 0 && opt.split_min_nnz < 0 && !tiled_product;
+        const bool model_fits = D.n_dense == 0 && opt.short_row_max < 0 && opt.stage_factor < 0 && opt.split_min_nnz < 0;
+        const bool by_model = model_fits && !tiled_product;
+        if (model_fits && tiled_product && kt <= 64 && estimate_split(c, ne, kt, x, g_long, short_max, 1e30) == Split::all_tiled) {
+            c.sp_min_row = short_max;
+            join(rl, rs, nl, nsh);
+        }
         int64_t slab_cols = 0;  // chosen by the model
         if (by_model) {
             SlabChoice slab;

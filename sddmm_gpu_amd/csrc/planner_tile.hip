@@ -209,7 +209,7 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
     bool sp_csr = false;
     struct SpmmHost {
         std::vector<WorkItem> items;
-        std::vector<int32_t> b_off, b_p0, b_len, row_part_ptr, part_slot;
+        std::vector<int32_t> b_off, b_p0, b_len, row_part_ptr, part_slot, rows;
         std::vector<uint16_t> cols;
         bool built = false;
     } sp;
@@ -244,8 +244,15 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         // 145, K = 384 166 / 251; uniform, K = 256, H of 17 and 31 MB, runs of 5 190 / 261 and 1515 / 1723, H of 21 MB,
         // runs of 4 647 / 543).
         const bool h_near = (int64_t)c.n_cols * c.K * 4 <= 6000000;
+        auto in_product = [&](int32_t row) { return c.row_ptr[row + 1] - c.row_ptr[row] >= c.sp_min_row; };
+        int64_t sp_nnz = L.nnz, sp_seg = n_seg;  // nonzeros and runs of the rows that would be tiled for it
+        if (want_spmm && rb == 0 && c.sp_min_row > 0) {
+            sp_nnz = sp_seg = 0;
+            for (int32_t r : rows) if (in_product(r)) sp_nnz += c.row_ptr[r + 1] - c.row_ptr[r];
+            for (int64_t s = 0; s < n_seg; ++s) sp_seg += in_product(T.active_row[s]);
+        }
         if (want_spmm && rb == 0 && c.nnz == c.P->info.nnz &&
-            ((ragged && !ragged_product_tiles(c.nnz, c.K, ks)) || (h_near && (L.nnz < 12 * n_seg || product_walks(c.nnz, c.K, ks))) || L.nnz < (c.K <= 128 ? 8 : 5) * n_seg)) { want_spmm = false; sp_csr = true; }
+            ((ragged && !ragged_product_tiles(c.nnz, c.K, ks)) || (h_near && (sp_nnz < 12 * sp_seg || product_walks(c.nnz, c.K, ks))) || sp_nnz < (c.K <= 128 ? 8 : 5) * sp_seg)) { want_spmm = false; sp_csr = true; }
         // row-block boundaries of the 2-D assignment: equal shares of the rows' nonzeros
         std::vector<int32_t> cut;
         auto make_cuts = [&](int n_shares) {
@@ -510,6 +517,7 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
                     auto &rv = runs[(size_t)k];
                     rv.reserve((size_t)(s1 - s0));
                     for (int64_t sg = s0; sg < s1; ++sg) {
+                        if (!in_product(T.active_row[(size_t)sg])) continue;
                         const int64_t b = seg_begin(j, sg);
                         rv.push_back({T.tiled_ind[(size_t)b], (int32_t)(T.active_end[(size_t)sg] - b), T.active_row[(size_t)sg],
                                       (int32_t)((int64_t)j * x)});
@@ -532,13 +540,14 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
                 sp.cols.assign((size_t)NBLK * 64, 0);
                 sp.b_off[(size_t)NB] = (int32_t)NBLK;
                 // the rows' partial rows: counted per row, then listed
+                std::copy_if(rows.begin(), rows.end(), std::back_inserter(sp.rows), in_product);
                 std::vector<int32_t> row_index((size_t)c.n_rows, -1);
-                for (size_t i = 0; i < rows.size(); ++i) row_index[(size_t)rows[i]] = (int32_t)i;
-                sp.row_part_ptr.assign(rows.size() + 1, 0);
+                for (size_t i = 0; i < sp.rows.size(); ++i) row_index[(size_t)sp.rows[i]] = (int32_t)i;
+                sp.row_part_ptr.assign(sp.rows.size() + 1, 0);
                 for (size_t k = 0; k < ni; ++k)
                     for (const Run &r : runs[k]) ++sp.row_part_ptr[(size_t)row_index[(size_t)r.row] + 1];
-                for (size_t i = 0; i < rows.size(); ++i) sp.row_part_ptr[i + 1] += sp.row_part_ptr[i];
-                sp.part_slot.assign((size_t)sp.row_part_ptr[rows.size()], 0);
+                for (size_t i = 0; i < sp.rows.size(); ++i) sp.row_part_ptr[i + 1] += sp.row_part_ptr[i];
+                sp.part_slot.assign((size_t)sp.row_part_ptr[sp.rows.size()], 0);
                 std::vector<int32_t> fill_at(sp.row_part_ptr.begin(), sp.row_part_ptr.end() - 1);
                 for (size_t k = 0; k < ni; ++k) {  // (in item order: a row's partial rows are listed in the order they are written)
                     const auto &rv = runs[k];
@@ -877,12 +886,12 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         WorkItem *d_it = nullptr;
         int32_t *d_off = nullptr, *d_p0 = nullptr, *d_len = nullptr, *d_rpp = nullptr, *d_slot = nullptr, *d_sum = nullptr, *d_gat = nullptr;
         uint16_t *d_cols = nullptr;
-        // the rows this launch does not hold (short ones, rows of other launches, rows without entries)
+        // the other rows (short ones, rows of other launches, rows without entries)
         std::vector<int32_t> others;
         {
             size_t k = 0;
             for (int64_t r = 0; r < c.n_rows; ++r) {
-                if (k < rows.size() && rows[k] == (int32_t)r) { ++k; continue; }
+                if (k < sp.rows.size() && sp.rows[k] == (int32_t)r) { ++k; continue; }
                 others.push_back((int32_t)r);
             }
             std::stable_sort(others.begin(), others.end(), [&](int32_t u, int32_t v) {
@@ -896,7 +905,7 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         if (int rc = c.up(&d_cols, sp.cols)) return rc;
         if (int rc = c.up(&d_rpp, sp.row_part_ptr)) return rc;
         if (int rc = c.up(&d_slot, sp.part_slot)) return rc;
-        if (int rc = c.up(&d_sum, rows)) return rc;
+        if (int rc = c.up(&d_sum, sp.rows)) return rc;
         if (int rc = c.up(&d_gat, others)) return rc;
         float *d_sp = nullptr;
         const size_t bytes = sp.b_p0.size() * (size_t)ks * 4;
@@ -904,7 +913,7 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         c.P->owned.push_back({d_sp, bytes, true});
         c.dev_bytes += (int64_t)bytes;
         sa.items = d_it; sa.n_items = (int32_t)sp.items.size(); sa.b_off = d_off; sa.b_p0 = d_p0; sa.b_len = d_len; sa.cols = d_cols;
-        sa.part = d_sp; sa.row_part_ptr = d_rpp; sa.part_slot = d_slot; sa.sum_rows = d_sum; sa.n_sum_rows = (int64_t)rows.size();
+        sa.part = d_sp; sa.row_part_ptr = d_rpp; sa.part_slot = d_slot; sa.sum_rows = d_sum; sa.n_sum_rows = (int64_t)sp.rows.size();
         sa.gather_rows = d_gat; sa.n_gather_rows = (int64_t)others.size();
         sa.tile_x = x; sa.n_cols = (int32_t)c.n_cols; sa.K = c.K;
         L.sp_on = 1; L.sp_part_bytes = (int64_t)bytes;

@@ -48,3 +48,29 @@ def test_against_64_bits(matrix, K):
     n = (rp[1:] - rp[:-1]).double()[:, None]  # a rounding per term of a row, however they are added up
     assert bool(((Y.double() - ref).abs() <= (n + 16) * 2.0 ** -24 * size).all())
     assert float(Y[-7:].abs().max()) == 0.0
+
+
+# all rows tiled for the SDDMM, the long ones alone for the product (K slices of up to 64), or the long ones alone for both
+@pytest.mark.parametrize("K", [32, 50, 64, 96, 128])
+def test_sddmm_and_product_of_one_plan(matrix, K):
+    n_rows, n_cols, nnz, rp, ci, rows = matrix
+    g = torch.Generator(device=DEV).manual_seed(K)
+    W, H = torch.randn(n_rows, K, generator=g, device=DEV), torch.randn(n_cols, K, generator=g, device=DEV)
+    out, Y = torch.full((nnz + 1,), 7.0, device=DEV), torch.full((n_rows * K + 1,), 7.0, device=DEV)
+    plan = capi.Plan.from_device_csr(n_rows, n_cols, nnz, rp.data_ptr(), ci.data_ptr(), K,
+                                     options=capi.PlanOptions.defaults(spmm_stream=1, ignore_env=1))
+    stream = torch.cuda.current_stream().cuda_stream
+    plan.execute(0, W.data_ptr(), H.data_ptr(), out.data_ptr(), stream)
+    plan.spmm(out.data_ptr(), H.data_ptr(), Y.data_ptr(), stream=stream)
+    torch.cuda.synchronize()
+    assert float(out[-1]) == 7.0 and float(Y[-1]) == 7.0
+    ref, size = torch.zeros(n_rows, K, dtype=torch.float64, device=DEV), torch.zeros(n_rows, K, dtype=torch.float64, device=DEV)
+    for b in range(0, nnz, 1 << 19):
+        r, h, o = rows[b:b + (1 << 19)], H[ci[b:b + (1 << 19)].long()].double(), out[b:min(nnz, b + (1 << 19))].double()
+        p = W[r].double() * h
+        assert bool(((o - p.sum(1)).abs() <= (K + 4) * 2.0 ** -24 * p.abs().sum(1)).all())
+        t = o[:, None] * h
+        ref.index_add_(0, r, t)
+        size.index_add_(0, r, t.abs())
+    n = (rp[1:] - rp[:-1]).double()[:, None]
+    assert bool(((Y[:-1].view(n_rows, K).double() - ref).abs() <= (n + 16) * 2.0 ** -24 * size).all())
