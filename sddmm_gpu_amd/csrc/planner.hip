@@ -674,6 +674,18 @@ static Split estimate_split(const Ctx &c, const std::vector<int32_t> &rows, int 
     return t_tile < t_gather ? Split::all_tiled : Split::all_gathered;
 }
 
+// Do most nonzeros lie in rows that hold a sixth of the columns or more?  The product with the dense factor then goes faster over
+// column tiles, where the runs of such rows are long, than over the CSR pattern, which is what is left to it beside a dense
+// core.  SDDMM + product, K = 512, us, with the core and without: ratings (nonzeros in rows of 31 % of the columns, on average)
+// of 4.9 / 15.9 / 31.5 million 665 / 2429 / 5646 and 567 / 1558 / 3524, 2.6 million: 355 and 368; word counts (9 and 5 %) of 5.3 /
+// 9.4 million 766 / 1782 and 926 / 2219.
+static bool long_rows(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_ptr)
+{
+    double squares = 0;
+    for (int64_t r = 0; r < n_rows; ++r) squares += (double)(row_ptr[r + 1] - row_ptr[r]) * (row_ptr[r + 1] - row_ptr[r]);
+    return squares * 6 >= (double)n_cols * (double)nnz;
+}
+
 // Has the caller left the choice of kernels and their layout to the planner?  (dense_blocks = 0 asks for fp32 throughout)
 static bool only_defaults(const sddmm_plan_options &o)
 {
@@ -783,9 +795,11 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
     // the remainder's shorter runs cost the tile kernel what the matrix cores save.  The search makes planning
     // 120-150 ms longer there, 600 calls' gain at K = 384 but 1300 at K = 256, so "choose" takes it from 384 on.
     // Plans that also serve the product with the dense factor keep the whole matrix on its column tiles below
-    // 512: behind a dense core that product walks the CSR pattern (98 M nonzeros, K = 128: 2.98 ms against 1.46).
+    // 512, and where rows are long also there: behind a dense core that product walks the CSR pattern (98 M nonzeros, K = 128:
+    // 2.98 ms against 1.46).
     // The threshold is flat: 3118 / 3113 / 3166 / 3284 us at K = 512 for 40 / 30 / 22 / 16 % filled.
-    const bool want_dense = opt.dense_blocks > 0 || (opt.dense_blocks < 0 && K >= (opt.spmm_stream > 0 ? 512 : 384));
+    bool want_dense = opt.dense_blocks > 0 || (opt.dense_blocks < 0 && K >= (opt.spmm_stream > 0 ? 512 : 384));
+    if (want_dense && opt.dense_blocks < 0 && opt.spmm_stream > 0 && nnz >= 4000000 && long_rows(n_rows, n_cols, nnz, row_ptr_all)) want_dense = false;
     if (kernel == SDDMM_KERNEL_HYBRID && want_dense && K % 32 == 0 && kt / 4 > 16 &&
         (int64_t)n_rows * (K / 4) <= (int64_t)UINT32_MAX && (int64_t)n_cols * (K / 4) <= (int64_t)UINT32_MAX) {
         const double threshold = (double)(opt.dense_permille > 0 ? opt.dense_permille : 300) / 1000.0;
