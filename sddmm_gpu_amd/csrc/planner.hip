@@ -628,10 +628,12 @@ static SlabChoice estimate_slabs(const Ctx &c, const std::vector<int32_t> &rows,
     }
     return best;
 }
-static Split estimate_split(const Ctx &c, const std::vector<int32_t> &rows, int w, int32_t x, int g, int64_t short_max, double slab_us)
+// us: of the split returned; gather_us: of all rows gathered (0: not estimated)
+struct SplitChoice { Split split; double us = 0, gather_us = 0; };
+static SplitChoice estimate_split(const Ctx &c, const std::vector<int32_t> &rows, int w, int32_t x, int g, int64_t short_max, double slab_us)
 {
     const size_t n = rows.size();
-    if (n == 0) return Split::all_gathered;
+    if (n == 0) return {Split::all_gathered};
     // a sample of whole rows, evenly spaced, of about a million nonzeros at most
     const size_t stride = std::max<size_t>({1, n / 4096, (size_t)((double)c.nnz / 1.0e6)});
     struct Class { double nnz = 0, runs = 0, pos = 0; } lng, shrt;
@@ -652,7 +654,7 @@ static Split estimate_split(const Ctx &c, const std::vector<int32_t> &rows, int 
             p = q;
         }
     }
-    if (sampled <= 0) return Split::by_length;
+    if (sampled <= 0) return {Split::by_length};
     const double f = (double)c.nnz / sampled;
     const double slices = (c.K + w - 1) / w, K = c.K;
     const double tiles = (double)((c.n_cols + x - 1) / x), h_slice = (double)c.n_cols * std::min<double>(w, K) * 4, h_all = (double)c.n_cols * K * 4;
@@ -669,9 +671,60 @@ static Split estimate_split(const Ctx &c, const std::vector<int32_t> &rows, int 
     const double t_tile = 1.12 * tile_us(lng.runs + shrt.runs, lng.pos + shrt.pos), t_gather = gather_us(lng.nnz + shrt.nnz);
     // (an H too large for the caches is gathered slab by slab, which takes all rows)
     const double t_both = lng.nnz > 0 && shrt.nnz > 0 && h_all <= 268.0e6 ? 3.0 + 1.12 * tile_us(lng.runs, lng.pos) + gather_us(shrt.nnz) : 1e30;
-    if (slab_us < std::min({t_both, t_tile, t_gather})) return Split::slabs;
-    if (t_both < t_tile && t_both < t_gather) return Split::by_length;
-    return t_tile < t_gather ? Split::all_tiled : Split::all_gathered;
+    if (slab_us < std::min({t_both, t_tile, t_gather})) return {Split::slabs, slab_us, t_gather};
+    if (t_both < t_tile && t_both < t_gather) return {Split::by_length, t_both, t_gather};
+    return {t_tile < t_gather ? Split::all_tiled : Split::all_gathered, std::min(t_tile, t_gather), t_gather};
+}
+
+// Microseconds of the tile kernel on all rows in K slices of w elements (32, 64 or 128), from the same sample, with what
+// estimate_split leaves out: that a launch takes as long as its busiest workgroup, whose items may be dealt out anew
+// (deal_evenly) where that gains enough, staging (a tile of x rows as 5.55 x positions of a workgroup), and runs, which cost
+// 1.8 to 3.4 positions each, more where the results of a row block do not stay in an L2 while its tiles add to them.
+// Fitted to 416 launches on 26 patterns at ten ranks (uniform, banded, R-MAT, word counts, ratings; 0.04 to 22 M
+// nonzeros): 19 % off (root mean square of the logarithm), estimate_split's own 29 %.
+static double tile_slices_us(const Ctx &c, const std::vector<int32_t> &rows, int w, double *run_length = nullptr)
+{
+    const int g = w >= 128 ? 8 : 4, i = w >= 128 ? 2 : w >= 64 ? 1 : 0;
+    constexpr double kPs[3] = {2.03, 4.05, 7.73}, kRun[3] = {3.38, 2.45, 1.81};
+    int64_t x = std::min<int64_t>(kLdsMaxBytes / (4 * w), c.n_cols), blocks = 1;
+    const int64_t least = (c.n_cols + x - 1) / x;
+    if (least <= c.cus) {  // (as add_tile has it)
+        int64_t n2 = least;
+        while (c.cus % n2) ++n2;
+        x = std::max<int64_t>(1, (c.n_cols + n2 - 1) / n2);
+        const int64_t nt = (c.n_cols + x - 1) / x, per_die = std::max(1, c.cus / 8);
+        blocks = c.cus / nt;
+        if (8.0 * nt * x * w * 4 <= 25.0 * c.nnz && nt == n2 && (n2 % per_die == 0 || per_die % n2 == 0)) blocks = 8 * std::max<int64_t>(1, per_die / n2);
+    }
+    const int64_t tiles = (c.n_cols + x - 1) / x;
+    const size_t n = rows.size(), stride = std::max<size_t>({1, n / 4096, (size_t)((double)c.nnz / 1.0e6)});
+    std::vector<double> items((size_t)(blocks * tiles), 0.0);
+    double sampled = 0, pos = 0, runs = 0;
+    for (size_t k = stride / 2; k < n; k += stride) {
+        const int32_t b = c.row_ptr[rows[k]], e = c.row_ptr[rows[k] + 1];
+        const int64_t block = std::min<int64_t>(blocks - 1, (int64_t)((double)b / c.nnz * blocks));
+        sampled += e - b;
+        for (int32_t p = b; p < e;) {
+            const int64_t tile = c.col_ind[p] / x;
+            int32_t q = p + 1;
+            while (q < e && c.col_ind[q] / x == tile) ++q;
+            const int len = q - p, r = len % g;
+            const double run = len - r + (r == 0 ? 0 : g == 8 && r <= 4 ? 4.5 : g);
+            items[(size_t)(block * tiles + tile)] += run;
+            pos += run;
+            runs += 1;
+            p = q;
+        }
+    }
+    if (sampled <= 0) return 1e30;
+    if (run_length) *run_length = sampled / runs;
+    const double f = c.nnz / sampled, slices = (c.K + w - 1) / w;
+    const double with_runs = 1.0 + kRun[i] * (c.nnz > 8400000 ? 2.34 : 1.0) * runs / pos;
+    const double turns = std::max(1.0, (double)(tiles * blocks) / c.cus), stage = 5.55 * x * turns;
+    const double mean = f * pos * with_runs / c.cus, most = std::max(mean, f * *std::max_element(items.begin(), items.end()) * with_runs) + stage;
+    const double dealt = 1.87 * mean + 2 * stage;
+    const double between = w == 128 && f * pos <= 8.4e6 ? 0 : 2.55;  // (small streams: all slices in one launch)
+    return 2.8 + (slices - 1) * between + slices * (0.6 + (dealt <= 0.7 * most ? dealt : most) * c.cus * 1e-6 * kPs[i]);
 }
 
 // Do most nonzeros lie in rows that hold a sixth of the columns or more?  The product with the dense factor then goes faster over
@@ -768,9 +821,9 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
     else if (K > 128 && K % 64 == 0) kt = 64;
     else if (pick_tile_variant(K, 0).G) kt = K;
     if (opt.k_slice > 0 && K % opt.k_slice == 0 && pick_tile_variant(opt.k_slice, 0).G) kt = opt.k_slice;
-    const bool ragged = kt == 0;  // no exact width: the tile kernel in a width K is rounded up to
+    bool ragged = kt == 0;  // no exact width: the tile kernel in a width K is rounded up to
     if (ragged) kt = ragged_tile_width(K);
-    const int32_t fit_t = kt ? kLdsMaxBytes / (kt * 4) : 0;  // H rows per LDS tile of the tile kernel
+    int32_t fit_t = kt ? kLdsMaxBytes / (kt * 4) : 0;  // H rows per LDS tile of the tile kernel
 
     // row-panel height of the tile kernel's stream: the panel's W slice (y rows of kt floats)
     // should stay L2-resident while the workgroups sweep the panel's column tiles
@@ -891,7 +944,7 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         const bool tiled_product = opt.spmm_stream > 0 && nnz >= 4000000 && (!ragged || ragged_product_tiles(nnz, K, kt)) && spmm_tile_supported(kt);
         const bool model_fits = D.n_dense == 0 && opt.short_row_max < 0 && opt.stage_factor < 0 && opt.split_min_nnz < 0;
         const bool by_model = model_fits && !tiled_product;
-        if (model_fits && tiled_product && kt <= 64 && estimate_split(c, ne, kt, x, g_long, short_max, 1e30) == Split::all_tiled) {
+        if (model_fits && tiled_product && kt <= 64 && estimate_split(c, ne, kt, x, g_long, short_max, 1e30).split == Split::all_tiled) {
             c.sp_min_row = short_max;
             join(rl, rs, nl, nsh);
         }
@@ -901,7 +954,41 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
             if (!ragged && opt.gather_lanes <= 0 && opt.gather_slab_cols < 0 && opt.gather_padded != 0 && opt.spmm_stream <= 0 &&
                 pick_tile_variant(kt, 4).G)
                 slab = estimate_slabs(c, ne, kt);
-            switch (estimate_split(c, ne, kt, x, g_long, short_max, slab.us)) {
+            SplitChoice choice = estimate_split(c, ne, kt, x, g_long, short_max, slab.us);
+            // A second look at three kinds of choice that it gets wrong by up to a factor of two, each with the margin at which
+            // 260 measured plans show gains and next to no losses (us before and so):
+            if (opt.k_slice <= 0 && opt.tile_lanes <= 0 && tile_x == 0 && (kt == 32 || kt == 64 || kt == 128) && nnz > 0) {
+                double run_length = 0;
+                const double tiled = tile_slices_us(c, ne, kt, &run_length);
+                // small matrices on tiles of which a few hold most (bands of 0.2 / 0.4 M, K = 96 / 50 15.5 / 17.9 and 7.8 / 9.5; R-MAT
+                // of 0.75 M, K = 96 40 and 23)
+                if (choice.split == Split::all_tiled && nnz < 1500000 && tiled > 1.2 * choice.gather_us) choice.split = Split::all_gathered;
+                // ranks whose rows of H lie across lines, gathered (K = 11, ratings of 4.9 / 16 M, word counts of 9.6 M 38 / 107 / 67 and
+                // 21 / 51 / 34)
+                else if (choice.split == Split::all_gathered && K % 32 != 0 && K != 16) {
+                    const double lines = nnz * ((4.0 * K - 4) / 128 + 1) * 128, h_all = (double)n_cols * K * 4;
+                    if (tiled < 0.62 * (4.5 + 1e-6 * lines / (h_all <= 4.2e6 ? 22.0 : h_all <= 64.0e6 ? 13.8 : 9.6))) choice.split = Split::all_tiled;
+                }
+                // runs of less than 4 in wide matrices: thinner slices have wider tiles (uniform, 4.7 M of 40,000 columns, K = 96 / 128 / 256 204 /
+                // 204 / 388 and 102 / 141 / 271; 17 M of 112,000, K = 96 654 and 412; word counts of 18 M, runs of 13, K = 128: 210 and 259)
+                else if (opt.spmm_stream <= 0 && run_length < 4) {
+                    const double now = choice.split == Split::all_tiled ? tiled : choice.us;
+                    int thin = 0;
+                    double thin_us = 0.8 * now;
+                    for (int w : {64, 32})
+                        if (w < kt && K % w == 0) {
+                            const double us = tile_slices_us(c, ne, w);
+                            if (us < thin_us) { thin = w; thin_us = us; }
+                        }
+                    if (thin) {
+                        choice.split = Split::all_tiled;
+                        kt = thin; ragged = false;
+                        fit_t = kLdsMaxBytes / (kt * 4);
+                        x = (int32_t)std::min<int64_t>(fit_t, std::max<int64_t>(n_cols, 1));
+                    }
+                }
+            }
+            switch (choice.split) {
             case Split::slabs: join(rs, rl, nsh, nl); slab_cols = slab.cols; break;
             case Split::all_tiled: join(rl, rs, nl, nsh); break;
             case Split::all_gathered: join(rs, rl, nsh, nl); break;

@@ -1,0 +1,47 @@
+"""Plans whose kernels the planner chooses by the busiest workgroup, by the lines a row of H lies in, or in thinner K slices than
+the widest: what is chosen, and the results with every source of the values, against 64-bit sums."""
+import pytest
+import torch
+
+from sddmm_gpu_amd import capi, synth
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("kind,sizes,K,kernel,k_slice", [
+    ("banded", (4000, 60, 400), 96, capi.KERNEL_ROW_GATHER, 96),         # a few tiles hold most
+    ("banded", (4000, 60, 400), 100, capi.KERNEL_ROW_GATHER, 100),
+    ("bag_of_words", (3000, 20000, 900), 11, capi.KERNEL_LDS_TILE, 11),  # 44-byte rows of H
+    ("uniform_random", (16598, 15299, 0.0091), 96, capi.KERNEL_LDS_TILE, 32),  # runs of one and two
+    ("uniform_random", (30281, 34347, 0.0063), 128, capi.KERNEL_LDS_TILE, 32),
+])
+def test_choice(kind, sizes, K, kernel, k_slice):
+    d = getattr(synth, kind)(*sizes, K=K, seed=3, device=DEV)
+    nnz = d["nnz"]
+    plan = capi.Plan.from_device_csr(d["n_rows"], d["n_cols"], nnz, d["row_ptr"].data_ptr(), d["col_ind"].data_ptr(), K,
+                                     options=capi.PlanOptions.defaults(ignore_env=1))
+    info = plan.info()
+    assert info["kernel"] == kernel and info["k_slice"] == k_slice, info
+    rows, cols, val = d["row_ind"].long(), d["col_ind"].long(), d["val"].double()
+    dot = torch.empty(nnz, dtype=torch.float64, device=DEV)
+    size = torch.empty_like(dot)
+    for b in range(0, nnz, 1 << 18):
+        p = d["W"][rows[b:b + (1 << 18)]].double() * d["H"][cols[b:b + (1 << 18)]].double()
+        dot[b:b + (1 << 18)] = p.sum(1)
+        size[b:b + (1 << 18)] = p.abs().sum(1)
+    W, H, out = d["W"].data_ptr(), d["H"].data_ptr(), torch.empty(nnz + 1, device=DEV)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def check(run, ref, scale):
+        out.fill_(7.0)
+        run()
+        torch.cuda.synchronize()
+        # a rounding per product and sum, a few per K slice, and the scaling
+        assert bool(((out[:nnz].double() - ref).abs() <= (K + 16) * 2.0 ** -24 * scale).all()) and float(out[nnz]) == 7.0
+
+    check(lambda: plan.execute(0, W, H, out.data_ptr(), stream), dot, size)
+    check(lambda: plan.execute(d["val"].data_ptr(), W, H, out.data_ptr(), stream), val * dot, val.abs() * size)
+    plan.set_values(d["val"].data_ptr(), stream)
+    check(lambda: plan.execute(0, W, H, out.data_ptr(), stream), val * dot, val.abs() * size)
+    check(lambda: plan.execute_epilogue(0, W, H, out.data_ptr(), capi.EPILOGUE_RESIDUAL, stream), val - dot, val.abs() + size)
