@@ -80,6 +80,7 @@ struct TileArgs {
     int32_t n_units;
     const WorkItem *items;     // non-null: workgroup b works on items b, b + grid, ... (each inside one tile)
     int32_t n_items;
+    int32_t in_turn;     // 1: the waves take an item's batches in turn, 0: a contiguous part each
     int32_t tile_x, n_cols;
     int32_t K;           // row length of W and H
     int32_t k_off;       // first K element covered by this launch (the kernel's own width is 4*G*KPL)

@@ -507,13 +507,16 @@ void sddmm_tile_kernel(const TileArgs a)
             for (; i < n4; i += kStride) lds_tile[i] = stage_piece(i);
             wg_sync();
         }
+        // A wave takes an equal, contiguous part of the item's batches or, where the plan asks for it, every NW-th of them.
+        const bool in_turn = !GATHER && a.in_turn;
+        const int turn = in_turn ? NW : 1;
         const int nb = (end - begin + 63) >> 6;
         // (the division runs on the vector unit; the results are uniform and go back to scalar
         // registers, so that the batch counter and the batch type bits are scalar work)
-        const int b0 = __builtin_amdgcn_readfirstlane((int)((int64_t)nb * wave / NW));
-        const int b1 = __builtin_amdgcn_readfirstlane((int)((int64_t)nb * (wave + 1) / NW));
+        const int b0 = in_turn ? wave : __builtin_amdgcn_readfirstlane((int)((int64_t)nb * wave / NW));
+        const int b1 = in_turn ? nb : __builtin_amdgcn_readfirstlane((int)((int64_t)nb * (wave + 1) / NW));
         if (b0 >= b1) continue;  // (no barrier below this point inside the tile)
-        const int bf = min(b1, (end - begin) >> 6);  // [b0, bf): this wave's batches of 64 whole positions
+        const int bf = min(b1, (end - begin) >> 6);  // of the batches below b1 those below bf have 64 whole positions
 
         // index data of one batch; positions past the item are clamped to its last
         // one (and repeat its work), so no load sits behind a branch
@@ -546,8 +549,8 @@ void sddmm_tile_kernel(const TileArgs a)
             else m.col = ld_meta<STREAM_HINT>(reinterpret_cast<const int *>(scol_b + o4));
             m.sv = STREAM_VAL ? ld_meta<STREAM_HINT>(reinterpret_cast<const float *>(sval_b + o4)) : 1.0f;
             m.o = o4;
-            o4 += 256;
-            og += 256 / G;
+            o4 += 256 * turn;
+            og += (256 / G) * turn;
             return m;
         };
         // an item's last, partial batch: positions past the end are clamped to the last one
@@ -738,28 +741,28 @@ void sddmm_tile_kernel(const TileArgs a)
             issue_w(wb, m1.wrow);
             __builtin_amdgcn_sched_barrier(0);  // keep the requests ahead of the arithmetic
             run(b0, wa, m0, ca, cb, m1.col);
-            for (int bi = b0 + 1; bi < bf; bi += 2) {
+            for (int bi = b0 + turn; bi < bf; bi += 2 * turn) {
                 flush();
-                const Meta n0 = issue_meta();  // batch bi + 2 (DEEP: bi + 4)
+                const Meta n0 = issue_meta();  // the wave's second next batch (DEEP: fourth)
                 if constexpr (!DEEP) m3 = n0;
                 issue_old(m2);
                 issue_w(wa, m2.wrow);
                 __builtin_amdgcn_sched_barrier(0);
                 run(bi, wb, m1, cb, ca, m2.col);
-                if (bi + 1 >= bf) break;
+                if (bi + turn >= bf) break;
                 flush();
-                const Meta n1 = issue_meta();  // batch bi + 3 (DEEP: bi + 5)
+                const Meta n1 = issue_meta();
                 issue_old(m3);
                 issue_w(wb, m3.wrow);
                 __builtin_amdgcn_sched_barrier(0);
-                run(bi + 1, wa, m2, ca, cb, m3.col);
+                run(bi + turn, wa, m2, ca, cb, m3.col);
                 m1 = m3;
                 if constexpr (DEEP) { m2 = m4; m3 = n0; m4 = n1; }
                 else m2 = n1;
             }
             flush();
         }
-        if (bf < b1) {
+        if (bf < b1 && (!in_turn || bf % NW == wave)) {
             // the item's last, partial batch: lanes past its end work on the last
             // position once more and store nothing
             Meta mt = issue_meta_tail(bf);

@@ -84,7 +84,7 @@ struct sddmm_plan {
 
 namespace sddmm {
 
-constexpr size_t kStreamSlack = 256;  // readable entries behind a tile stream's arrays
+constexpr size_t kStreamSlack = 5120;  // readable entries behind a tile stream's arrays: 16 waves' batches of 64, up to four ahead and one more
 
 // (the word mixer of the pattern hash and of the plan files' checksums)
 __host__ __device__ inline uint64_t mix64(uint64_t x)

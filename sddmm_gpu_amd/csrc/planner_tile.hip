@@ -193,7 +193,6 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
     int pl_groups = 0;     // groups of workgroups per die
     int pl_slots = 0;      // workgroups per group (a group works on one row range at a time)
     int64_t block_rows_max = 0;  // most rows in one row block / row range of the 2-D assignment
-    int64_t pl_sub = 0;    // batches per piece of an item
     // Short batches (see tile_variant_shorts): the last chunk of a (row, tile) run that holds at
     // most G/2 nonzeros is kept apart from the full chunks, and eight such chunks make a batch of
     // their own, which the kernel runs in half the steps.
@@ -309,9 +308,7 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
                     panel_local = true;
                     pl_groups = groups;
                     pl_slots = per_die / groups;
-                    // (banded 2^20, K=512, ms per step by batches per wave and piece: 4 -> 4.37, 8 -> 4.25,
-                    // 16 -> 4.24, 32 -> 4.27, 128 -> 4.44; whole tiles in runs of neighbours: 4.56)
-                    pl_sub = (int64_t)nwaves * 16;
+                    // (banded 2^20, K=512, ms per step then: 4.24; whole tiles in runs of neighbours: 4.56)
                 } else {
                     make_cuts(shares);
                 }
@@ -623,10 +620,12 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
                     }
             } else if (panel_local) {
                 // Range sh belongs to die sh % 8, group (sh / 8) % pl_groups.  Its items, in tile order, go to the
-                // group's workgroup that is free first (time counted in stream positions).  The waves of
-                // a workgroup split an item into equal contiguous parts, so an item is handed over in
-                // pieces of pl_sub batches: the rows a workgroup touches at one time then lie close
-                // together.  Pieces of one tile follow each other on the same workgroup (staged once).
+                // group's workgroup that is free first (time counted in stream positions).  The waves of a workgroup take
+                // an item's batches in turn, so that the rows it touches at one time lie close together.  (With a contiguous
+                // part each, items were handed over in pieces of 16 batches a wave, and every piece filled the waves' pipelines
+                // anew: bands of 2^20 rows, 64 of +-2048, K = 512 3390 and 3336 us; 300,000 rows, 40 of +-600, K = 512 654 and 619;
+                // 500,000, 30 of +-700, K = 64 141 and 130; 10^6, 45 of +-1200, K = 32 261 and 246.  Row blocks whose tiles
+                // all meet the same rows lose by it: recommender, K = 32 / 128 377 / 811 and 389 / 818.)
                 std::vector<std::vector<WorkItem>> seq((size_t)c.cus);
                 for (int sh = 0; sh < shares; ++sh) {
                     const int die = sh % 8, base = ((sh / 8) % pl_groups) * pl_slots;
@@ -636,12 +635,7 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
                         if (it.end <= it.begin) continue;
                         const int slot = (int)(std::min_element(free_at.begin(), free_at.end()) - free_at.begin());
                         auto &q = seq[(size_t)((base + slot) * 8 + die)];
-                        const int64_t nb = ((int64_t)it.end - it.begin + 63) / 64;
-                        for (int64_t k0 = 0; k0 < nb; k0 += pl_sub) {
-                            const int64_t k1 = std::min(nb, k0 + pl_sub);
-                            q.push_back({(int32_t)(it.begin + k0 * 64), (int32_t)std::min<int64_t>(it.end, it.begin + k1 * 64),
-                                         (int32_t)(it.batch_base + (shorts ? k0 : 0)), it.tile});
-                        }
+                        q.push_back(it);
                         free_at[(size_t)slot] += (int64_t)it.end - it.begin;
                     }
                 }
@@ -932,6 +926,7 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         c.P->info.spmm_runs += records;
     }
     L.grid = (int32_t)std::max<int64_t>(1, std::min<int64_t>((int64_t)c.cus, (np + 4095) / 4096));
+    a.in_turn = panel_local;  // (see there)
     if (grid2d) {
         WorkItem *d_items = nullptr;
         if (int rc = c.up(&d_items, items)) return rc;
