@@ -3,8 +3,8 @@
 // What bounds it is the host link (57 GB/s each way here).  The runtime's own copies of pageable memory reach 39
 // GB/s up and 18 down on one thread, which also takes the page faults of a fresh output array one after the other,
 // so the copies go through pinned pieces here: a few threads copy between the caller's memory and the pieces while
-// a copy kernel per piece moves the ones before over the link, on two streams so that one kernel's start hides
-// behind another's work.  27.4 MB up and 19.5 MB down: 2.20 -> 1.20 ms a call (0.83 ms of it the link).  The pieces, streams and
+// a copy kernel per piece moves the ones before over the link, on three streams so that one kernel's start hides
+// behind another's work.  27.4 MB up and 19.5 MB down: 2.20 -> 1.13 ms a call (0.83 ms of it the link).  The pieces, streams and
 // threads (HostPipe) are shared by all plans that have made such a call and go with the last of them; the device
 // arrays stay with their plan, until it is destroyed or sddmm_plan_release_host.
 #include <hip/hip_runtime.h>
@@ -24,9 +24,11 @@ namespace {
 
 typedef float vec4f __attribute__((ext_vector_type(4)));
 
-// n4 pieces of 16 bytes and `tail` floats, to or from pinned host memory (16-byte aligned).  32 workgroups with
-// four requests per thread keep more than the link's bandwidth times its latency in flight.
-constexpr int kCopyBlocks = 32;
+// n4 pieces of 16 bytes and `tail` floats, to or from pinned host memory (16-byte aligned).  16 workgroups with
+// four requests per thread, on three streams, keep more than the link's bandwidth times its latency in flight, and one
+// kernel's start and end hide behind two others (27.4 MB up, 19.5 MB down, us a call: 32 workgroups on one / two / four streams
+// 1416 / 1208 / 1203, 16 on two / three / four 1176 / 1131 / 1162, 8 on two / four 1167 / 1135, 64 on two 1295).
+constexpr int kCopyBlocks = 16;
 __global__ __launch_bounds__(256)
 void sddmm_host_copy_kernel(const vec4f *__restrict__ src, vec4f *__restrict__ dst, int n4, int tail)
 {
@@ -54,11 +56,12 @@ public:
     static constexpr size_t kPiece = (size_t)1 << 20;
     static constexpr int kThreads = 8;            // the caller and seven more
     static constexpr int kPieces = 2 * kThreads;  // a thread works on one of its pieces while the other is on its way
-    static constexpr int kStreams = 2;
+    static constexpr int kStreams = 3;
 
     hipStream_t stream[kStreams] = {};  // (a thread's pieces all travel on one of them)
     hipEvent_t fork = nullptr, join[kStreams] = {}, e0 = nullptr, e1 = nullptr;
     std::mutex busy;  // held by a call from its first piece to its last
+    int used = kStreams;  // streams of the call that holds it: one for less than 2 MB, whose events would cost more than they hide
 
     // the pipe of `device` (the current one), made if no plan holds it
     static std::shared_ptr<HostPipe> get(int device)
@@ -197,7 +200,7 @@ private:
             return e == hipSuccess;
         };
         if (id > 0 && !check(hipSetDevice(device))) return;
-        const hipStream_t st = stream[id % kStreams];
+        const hipStream_t st = stream[id % used];
         const Part *slot[2] = {};  // what travels through each of the two
         auto finish = [&](int k) {  // waits for the slot's copy; down: hands its bytes on
             const Part *p = slot[k];
@@ -266,17 +269,18 @@ int host_call(const sddmm_plan *plan, HostCall &c, const float *h_W, const float
     HostPipe &pipe = *c.pipe;
     // after whatever the caller has put on the default stream before
     HIP_TRY(hipEventRecord(pipe.fork, nullptr));
-    for (hipStream_t s : pipe.stream) HIP_TRY(hipStreamWaitEvent(s, pipe.fork, 0));
+    pipe.used = 4 * (I.n_rows * (int64_t)I.K + I.n_cols * (int64_t)I.K + I.nnz) < ((int64_t)2 << 20) ? 1 : HostPipe::kStreams;
+    for (int i = 0; i < pipe.used; ++i) HIP_TRY(hipStreamWaitEvent(pipe.stream[i], pipe.fork, 0));
     const HostPipe::Part in[2] = {{(const char *)h_W, (char *)c.W, (size_t)I.n_rows * I.K * 4}, {(const char *)h_H, (char *)c.H, (size_t)I.n_cols * I.K * 4}};
     HIP_TRY(pipe.move(in, 2, true));
-    for (int i = 1; i < HostPipe::kStreams; ++i) {
+    for (int i = 1; i < pipe.used; ++i) {
         HIP_TRY(hipEventRecord(pipe.join[i], pipe.stream[i]));
         HIP_TRY(hipStreamWaitEvent(pipe.stream[0], pipe.join[i], 0));
     }
     HIP_TRY(hipEventRecord(pipe.e0, pipe.stream[0]));
     if (int rc = sddmm_execute(plan, nullptr, c.W, c.H, c.out, pipe.stream[0])) return rc;
     HIP_TRY(hipEventRecord(pipe.e1, pipe.stream[0]));
-    for (int i = 1; i < HostPipe::kStreams; ++i) HIP_TRY(hipStreamWaitEvent(pipe.stream[i], pipe.e1, 0));
+    for (int i = 1; i < pipe.used; ++i) HIP_TRY(hipStreamWaitEvent(pipe.stream[i], pipe.e1, 0));
     const HostPipe::Part back[1] = {{(const char *)c.out, (char *)h_out, (size_t)I.nnz * 4}};
     HIP_TRY(pipe.move(back, 1, false));
     HIP_TRY(hipEventSynchronize(pipe.e1));  // (there is nothing to copy back from an empty matrix)
