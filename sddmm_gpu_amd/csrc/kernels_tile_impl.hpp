@@ -507,8 +507,9 @@ void sddmm_tile_kernel(const TileArgs a)
             for (; i < n4; i += kStride) lds_tile[i] = stage_piece(i);
             wg_sync();
         }
-        // A wave takes an equal, contiguous part of the item's batches or, where the plan asks for it, every NW-th of them.
-        const bool in_turn = !GATHER && a.in_turn;
+        // A wave takes an equal, contiguous part of the item's batches or, where the plan asks for it, every NW-th of them.  (Not
+        // in the largest form, all slices of a ragged rank in one launch, which the choice between both costs 4 %.)
+        const bool in_turn = !GATHER && !(RAGGED && FUSED) && a.in_turn;
         const int turn = in_turn ? NW : 1;
         const int nb = (end - begin + 63) >> 6;
         // (the division runs on the vector unit; the results are uniform and go back to scalar
