@@ -243,6 +243,9 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         // 145, K = 384 166 / 251; uniform, K = 256, H of 17 and 31 MB, runs of 5 190 / 261 and 1515 / 1723, H of 21 MB,
         // runs of 4 647 / 543).
         const bool h_near = (int64_t)c.n_cols * c.K * 4 <= 6000000;
+        // (small products of three slices and more walk up to twice that: beside each slice's two launches they have little to do.
+        // Ratings, K = 512, 0.48 and 1.05 million nonzeros, H of 6.2 and 8.1 MB, tiles and walk 134 / 170 and 57 / 98 us)
+        const bool small_walks = product_walks(c.nnz, c.K, ks) && (h_near || (c.K > 256 && (int64_t)c.n_cols * c.K * 4 <= 12000000));
         auto in_product = [&](int32_t row) { return c.row_ptr[row + 1] - c.row_ptr[row] >= c.sp_min_row; };
         int64_t sp_nnz = L.nnz, sp_seg = n_seg;  // nonzeros and runs of the rows that would be tiled for it
         if (want_spmm && rb == 0 && c.sp_min_row > 0) {
@@ -251,7 +254,7 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
             for (int64_t s = 0; s < n_seg; ++s) sp_seg += in_product(T.active_row[s]);
         }
         if (want_spmm && rb == 0 && c.nnz == c.P->info.nnz &&
-            ((ragged && !ragged_product_tiles(c.nnz, c.K, ks)) || (h_near && (sp_nnz < 12 * sp_seg || product_walks(c.nnz, c.K, ks))) || sp_nnz < (c.K <= 128 ? 8 : 5) * sp_seg)) { want_spmm = false; sp_csr = true; }
+            ((ragged && !ragged_product_tiles(c.nnz, c.K, ks)) || (h_near && sp_nnz < 12 * sp_seg) || small_walks || sp_nnz < (c.K <= 128 ? 8 : 5) * sp_seg)) { want_spmm = false; sp_csr = true; }
         // row-block boundaries of the 2-D assignment: equal shares of the rows' nonzeros
         std::vector<int32_t> cut;
         auto make_cuts = [&](int n_shares) {
