@@ -700,14 +700,16 @@ static double tile_slices_us(const Ctx &c, const std::vector<int32_t> &rows, int
     const size_t n = rows.size(), stride = std::max<size_t>({1, n / 4096, (size_t)((double)c.nnz / 1.0e6)});
     std::vector<double> items((size_t)(blocks * tiles), 0.0);
     double sampled = 0, pos = 0, runs = 0;
+    const int32_t width = (int32_t)x;
     for (size_t k = stride / 2; k < n; k += stride) {
         const int32_t b = c.row_ptr[rows[k]], e = c.row_ptr[rows[k] + 1];
         const int64_t block = std::min<int64_t>(blocks - 1, (int64_t)((double)b / c.nnz * blocks));
         sampled += e - b;
         for (int32_t p = b; p < e;) {
-            const int64_t tile = c.col_ind[p] / x;
+            const int32_t tile = c.col_ind[p] / width;
+            const int64_t end = ((int64_t)tile + 1) * width;
             int32_t q = p + 1;
-            while (q < e && c.col_ind[q] / x == tile) ++q;
+            while (q < e && c.col_ind[q] < end) ++q;
             const int len = q - p, r = len % g;
             const double run = len - r + (r == 0 ? 0 : g == 8 && r <= 4 ? 4.5 : g);
             items[(size_t)(block * tiles + tile)] += run;

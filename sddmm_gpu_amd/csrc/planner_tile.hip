@@ -544,16 +544,29 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
                 std::vector<int32_t> row_index((size_t)c.n_rows, -1);
                 for (size_t i = 0; i < sp.rows.size(); ++i) row_index[(size_t)sp.rows[i]] = (int32_t)i;
                 sp.row_part_ptr.assign(sp.rows.size() + 1, 0);
+                // (a row lies in one row block: the row blocks are independent of each other)
+                std::vector<std::vector<size_t>> of_block;
                 for (size_t k = 0; k < ni; ++k)
-                    for (const Run &r : runs[k]) ++sp.row_part_ptr[(size_t)row_index[(size_t)r.row] + 1];
+                    if (keys[k].first >= 0) {
+                        if (of_block.size() <= (size_t)keys[k].first) of_block.resize((size_t)keys[k].first + 1);
+                        of_block[(size_t)keys[k].first].push_back(k);
+                    }
+                parallel_ranges((int64_t)of_block.size(), 1, [&](int64_t bb, int64_t be, int) {
+                    for (int64_t b = bb; b < be; ++b)
+                        for (size_t k : of_block[(size_t)b])
+                            for (const Run &r : runs[k]) ++sp.row_part_ptr[(size_t)row_index[(size_t)r.row] + 1];
+                });
                 for (size_t i = 0; i < sp.rows.size(); ++i) sp.row_part_ptr[i + 1] += sp.row_part_ptr[i];
                 sp.part_slot.assign((size_t)sp.row_part_ptr[sp.rows.size()], 0);
                 std::vector<int32_t> fill_at(sp.row_part_ptr.begin(), sp.row_part_ptr.end() - 1);
-                for (size_t k = 0; k < ni; ++k) {  // (in item order: a row's partial rows are listed in the order they are written)
-                    const auto &rv = runs[k];
-                    for (size_t q = 0; q < rv.size(); ++q)
-                        sp.part_slot[(size_t)fill_at[(size_t)row_index[(size_t)rv[q].row]]++] = (int32_t)((n_bund[k] + (int64_t)q / 8) * 8 + (int64_t)q % 8);
-                }
+                parallel_ranges((int64_t)of_block.size(), 1, [&](int64_t bb, int64_t be, int) {
+                    for (int64_t b = bb; b < be; ++b)
+                        for (size_t k : of_block[(size_t)b]) {  // (in item order: a row's partial rows are listed in the order they are written)
+                            const auto &rv = runs[k];
+                            for (size_t q = 0; q < rv.size(); ++q)
+                                sp.part_slot[(size_t)fill_at[(size_t)row_index[(size_t)rv[q].row]]++] = (int32_t)((n_bund[k] + (int64_t)q / 8) * 8 + (int64_t)q % 8);
+                        }
+                });
                 parallel_ranges((int64_t)ni, 1, [&](int64_t ib, int64_t ie, int) {
                     for (int64_t k = ib; k < ie; ++k) {
                         const auto &rv = runs[(size_t)k];
