@@ -315,7 +315,7 @@ __device__ __forceinline__ void matrix_core_waves(const TileArgs &a, int mw, int
 // 3 = all a.n_slices K slices inside this one launch, one after the other (small matrices, where a
 // launch costs as much as its work): a wave meets the same positions in every slice, so the partial
 // results it left in a.part are its own, and a workgroup barrier between the slices is all the
-// ordering needed.
+// ordering needed.  5 = the same with a tile's batches in turn (see in_turn).
 // RAGGED: K is no multiple of the kernel's width (K <= 4 * G * KPL: one launch; else the last of several slices is cut
 // short), and K needs no alignment: H rows are staged with the tail filled up with zeros, W rows are read in pieces at
 // any 4-byte address, the one at the end of the row from its last four floats on with what it shares with the piece
@@ -328,7 +328,7 @@ template <int G, int KPL, int VMODE, int NW, bool GATHER, int SLICE, int NWM = 0
 __global__ __launch_bounds__((NW + NWM) * 64)
 void sddmm_tile_kernel(const TileArgs a)
 {
-    constexpr bool FUSED = SLICE == 3;
+    constexpr bool FUSED = SLICE == 3 || SLICE == 5;
     constexpr bool ACC = SLICE == 2 || SLICE == 4;
     constexpr bool PART = SLICE >= 1;
     constexpr bool TO_OUT = SLICE == 0 || SLICE >= 3;  // positions and values are needed
@@ -507,9 +507,10 @@ void sddmm_tile_kernel(const TileArgs a)
             for (; i < n4; i += kStride) lds_tile[i] = stage_piece(i);
             wg_sync();
         }
-        // A wave takes an equal, contiguous part of the item's batches or, where the plan asks for it, every NW-th of them.  (Not
-        // in the largest form, all slices of a ragged rank in one launch, which the choice between both costs 4 %.)
-        const bool in_turn = !GATHER && !(RAGGED && FUSED) && a.in_turn;
+        // A wave takes an equal, contiguous part of the item's batches or, where the plan asks for it, every NW-th of them.  (With
+        // all slices in one launch a kernel of its own: the choice between both inside it costs 1 % of word counts of 0.7 M
+        // nonzeros, K = 256, and 4 % at ragged ranks.)
+        const bool in_turn = FUSED ? SLICE == 5 : !GATHER && a.in_turn;
         const int turn = in_turn ? NW : 1;
         const int nb = (end - begin + 63) >> 6;
         // (the division runs on the vector unit; the results are uniform and go back to scalar
@@ -780,8 +781,10 @@ void sddmm_tile_kernel(const TileArgs a)
 // The all-slices-in-one-launch form exists for slices of 128 elements on groups of 8 lanes only (what the
 // planner uses for K > 128); null for the other variants.
 template <int G, int KPL, int VMODE, int NW, bool GATHER>
-TileFn fused_slices_kernel()
+TileFn fused_slices_kernel(int slice)
 {
+    if constexpr (G == 8 && KPL == 4 && !GATHER)
+        if (slice == 5) return (TileFn)sddmm_tile_kernel<G, KPL, VMODE, NW, GATHER, 5>;
     if constexpr (G == 8 && KPL == 4) return (TileFn)sddmm_tile_kernel<G, KPL, VMODE, NW, GATHER, 3>;
     else return nullptr;
 }
@@ -796,7 +799,7 @@ TileFn gather_tile_kernel(int slice)
             if (slice == 1) return (TileFn)sddmm_tile_kernel<G, KPL, VMODE, 4, true, 1>;
             if (slice == 2) return (TileFn)sddmm_tile_kernel<G, KPL, VMODE, 4, true, 2>;
         }
-        if (slice == 3) return fused_slices_kernel<G, KPL, VMODE, 4, true>();
+        if (slice == 3) return fused_slices_kernel<G, KPL, VMODE, 4, true>(slice);
         if (slice == 4) return (TileFn)sddmm_tile_kernel<G, KPL, VMODE, 4, true, 4>;
     }
     return nullptr;
@@ -817,6 +820,7 @@ TileFn ragged_tile_kernel(const TileVariant &v, bool gather, int slice, int nwav
             if (slice == 2) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 2, 0, true>;
         }
         if (slice == 3) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 3, 0, true>;
+        if (slice == 5) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 5, 0, true>;
         if (slice == 4) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 4, 0, true>;
     }
     return nullptr;

@@ -9,7 +9,7 @@ TileFn tile_kernel_part0(const TileVariant &v, int vmode, bool gather, int slice
 {
     if (ragged) return ragged_tile_kernel<0>(v, gather, slice, nwaves);
 #define SDDMM_PICK_SLICE(g, kpl, vm, nw)                                                                     \
-    (slice == 3 ? fused_slices_kernel<g, kpl, vm, nw, false>()                                              \
+    (slice == 3 || slice == 5 ? fused_slices_kernel<g, kpl, vm, nw, false>(slice)                               \
      : slice == 4 ? (TileFn)sddmm_tile_kernel<g, kpl, vm, nw, false, 4>                                        \
                   : (TileFn)sddmm_tile_kernel<g, kpl, vm, nw, false, 0>)
 #define SDDMM_PICK(g, kpl, vm)                                                                              \
