@@ -413,9 +413,10 @@ int sddmm_execute_ws(const sddmm_plan *plan, const float *d_val, const float *d_
  * from the column tile in LDS) over a run and writes one partial row; a second
  * kernel adds the partial rows of every row; the plan's other rows gather their
  * H rows as sddmm_spmm_csr does.  Where the runs are short (fewer than 8 entries, 5
- * from K = 129 on, 12 while H is about as large as a die's L2), at ranks without a tile
- * width of their own, on small matrices (fewer than 4 M nonzeros and 4.5e8 or 7e8
- * nonzeros times K, H as above) and where a few workgroups would hold most of the work, the whole product
+ * from K = 129 on, 12 while H is about as large as a die's L2), on small matrices (fewer than 4 M nonzeros
+ * and 4.5e8 or 7e8 nonzeros times K, H as above), at ranks without a tile width of their
+ * own below 4 M nonzeros (up to K = 256) or where more than a quarter of the rank rounded up
+ * would be padding, and where a few workgroups would hold most of the work, the whole product
  * goes over the CSR pattern as sddmm_spmm_csr does it, with the parts of its cut rows
  * written down and added up in order; and a plan on row blocks multiplies its tiles
  * on the matrix cores (weights of any size at the same speed; where 32 rows meet values of

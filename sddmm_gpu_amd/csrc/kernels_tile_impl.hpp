@@ -307,8 +307,8 @@ __device__ __forceinline__ void matrix_core_waves(const TileArgs &a, int mw, int
 // products so far go to a.part, in stream order: one coalesced store per batch); 2 = a slice in between
 // (adds to what it reads back from a.part, coalesced); 4 = the last one, which alone reads positions and
 // values and touches out, with one scattered store per position.
-// (All are bound by the load path, 81 to 83 % busy on a band of 64 in 4096 columns, 2^20 rows, K = 512, vector unit 64 % in
-// the slices before the last and 44 % in that, which has the positions, values and partial output lines.  Before, all of
+// (All are bound by the load path, 81 to 83 % busy on a band of 64 in 4096 columns, 2^20 rows, K = 512, vector unit 69 % in
+// the slices before the last and 45 % in that, which has the positions, values and partial output lines.  Before, all of
 // them read positions and values, columns in 32 bits, and scaled: 4.02 -> 3.42 ms (16.5 -> 11.3 GB a step; 1.46 -> 0.29 GB of
 // stream data in each slice but the last); the remainder of the recommender at K = 512, 1.39 -> 1.21.  Stream data four
 // batches ahead, or with the non-temporal hint: the same.)
@@ -345,8 +345,8 @@ void sddmm_tile_kernel(const TileArgs a)
     // The compact stream serves the thin K slices, where a batch is little arithmetic and the kernel moves
     // at the rate of its requests in flight: 16 waves x 2 batches x 448 bytes of index data per compute unit
     // are 14 KB, and at a microsecond of memory latency 256 compute units then fetch 3.6 TB/s -- what the
-    // K = 32 launch measured.  Its index data is therefore requested four batches ahead (the arrays' slack
-    // of 256 entries covers exactly the four batches past the end).
+    // K = 32 launch measured.  Its index data is therefore requested four batches ahead (the arrays'
+    // slack, kStreamSlack, covers the batches past the end).
     constexpr bool DEEP = COMPACT;
     constexpr bool COL16 = COMPACT || (!GATHER && PART);  // columns from a.scol16
     constexpr int ROW_SHIFT = __builtin_ctz(K4 * 16);     // log2 of an LDS row in bytes

@@ -1017,7 +1017,7 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
             // An H far larger than the caches (every die's 4 MB of L2, 32 MB together) and no tiled class:
             // every gathered H row would cross the fabric (R-MAT 2^22, K=64: 41.8 GB per step for 4.5 GB of
             // algorithmic bytes, 8.27 ms).  The padded gather then walks S in column slabs whose H rows
-            // come to 32 MB, with groups of 4 lanes (runs inside a slab are short): 26.3 GB, 4.96 ms.
+            // come to 32 MB, padded to groups of 4 positions (runs inside a slab are short): 26.3 GB, 4.42 ms.
             // Narrower slabs lose to the W rows re-read per (row, slab) run, wider ones to H misses.
             // (where the model above has its say it chooses the slabs; this is for plans whose caller set a threshold,
             // and for slices of less than 64 elements)
