@@ -970,10 +970,13 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
                 const double gathered = across ? 4.5 + 1e-6 * lines / (h_all <= 4.2e6 ? 22.0 : h_all <= 64.0e6 ? 13.8 : 9.6) : choice.gather_us;
                 if (choice.split == Split::all_tiled && nnz < 1500000 && tiled > (nnz < 500000 ? 1.0 : 1.2) * gathered) choice.split = Split::all_gathered;
                 // such ranks, gathered (K = 11, ratings of 4.9 / 16 M, word counts of 9.6 M 38 / 107 / 67 and 21 / 51 / 34)
-                else if (choice.split == Split::all_gathered && across && tiled < 0.62 * gathered) choice.split = Split::all_tiled;
-                // runs of less than 4 in wide matrices: thinner slices have wider tiles (uniform, 4.7 M of 40,000 columns, K = 96 / 128 / 256 204 /
-                // 204 / 388 and 102 / 141 / 271; 17 M of 112,000, K = 96 654 and 412; word counts of 18 M, runs of 13, K = 128: 210 and 259)
-                else if (opt.spmm_stream <= 0 && run_length < 4) {
+                else if (choice.split == Split::all_gathered && across && K <= kt && tiled < 0.62 * gathered) choice.split = Split::all_tiled;
+                // runs of less than 4 in wide matrices: thinner slices have wider tiles (uniform, 4.7 M of 40,000 columns, K = 256: 388 and
+                // 271; word counts of 18 M, runs of 13, K = 128: 210 and 259)
+                // (Neither gives K slices to a plan that has none: it would get partial results in a buffer of its own, and calls
+                // on it that overlap in time, which were right, would no longer be.  Uniform, 4.7 M of 40,000 columns, K = 96 / 128
+                // 204 / 204 and, in slices of 32, 102 / 141: a caller whose calls follow each other may ask for them, k_slice.)
+                else if (opt.spmm_stream <= 0 && K > kt && choice.split != Split::all_gathered && run_length < 4) {
                     const double now = choice.split == Split::all_tiled ? tiled : choice.us;
                     int thin = 0;
                     double thin_us = 0.8 * now;
