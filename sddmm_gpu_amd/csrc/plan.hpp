@@ -119,6 +119,7 @@ struct Ctx {
     const int32_t *orig = nullptr;
     sddmm_plan_options opt{};  // the caller's options with the environment overrides applied
     int64_t sp_min_row = 0;    // the product on column tiles: rows of fewer nonzeros gather their H rows
+    bool sp_walk = false;      // the product over the CSR pattern whatever the runs of the tile launch
     int32_t pos(int64_t p) const { return orig ? orig[p] : (int32_t)p; }
     float value(int64_t p) const { return vals[orig ? orig[p] : p]; }
 

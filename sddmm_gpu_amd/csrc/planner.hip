@@ -946,9 +946,26 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         const bool tiled_product = opt.spmm_stream > 0 && nnz >= 4000000 && (!ragged || ragged_product_tiles(nnz, K, kt)) && spmm_tile_supported(kt);
         const bool model_fits = D.n_dense == 0 && opt.short_row_max < 0 && opt.stage_factor < 0 && opt.split_min_nnz < 0;
         const bool by_model = model_fits && !tiled_product;
-        if (model_fits && tiled_product && kt <= 64 && estimate_split(c, ne, kt, x, g_long, short_max, 1e30).split == Split::all_tiled) {
-            c.sp_min_row = short_max;
-            join(rl, rs, nl, nsh);
+        // staging every H tile must be paid for by the nonzeros that use it
+        auto pays_for_staging = [&]() {
+            const int64_t n_tiles_all = (n_cols + x - 1) / x, stage_rows = std::max<int64_t>(n_tiles_all, c.cus) * x;
+            return nl >= (opt.stage_factor >= 0 ? opt.stage_factor : 8) * stage_rows;
+        };
+        // Where the long rows do not pay for it, or are a class too small, the product walks the CSR pattern: tiles that hold
+        // nothing, or little beside rows that one group of lanes gathers each, are no form for it.  All rows are then tiled for
+        // the SDDMM only where the second model below agrees (SDDMM + product, us, gathered and so: uniform, 5 M of 17,770
+        // columns, K = 32 / 64 47 + 43 / 74 + 75 and 30 + 45 / 59 + 76; 17 M of 112,000, K = 32, where it does not, 251 + 237 and
+        // 351 + 236), and not in K slices, which would keep partial results in a buffer that the gather does without.
+        if (model_fits && tiled_product && kt <= 64) {
+            const bool long_class = pays_for_staging() && nl * 50 >= nnz;
+            if (long_class || K <= kt) {
+                const SplitChoice choice = estimate_split(c, ne, kt, x, g_long, short_max, 1e30);
+                if (choice.split == Split::all_tiled && (long_class || tile_slices_us(c, ne, kt) < choice.gather_us)) {
+                    if (long_class) c.sp_min_row = short_max;
+                    else c.sp_walk = true;
+                    join(rl, rs, nl, nsh);
+                }
+            }
         }
         int64_t slab_cols = 0;  // chosen by the model
         if (by_model) {
@@ -1000,10 +1017,7 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
             case Split::by_length: break;
             }
         }
-        // staging every H tile must be paid for by the nonzeros that use it
-        const int64_t n_tiles_all = (n_cols + x - 1) / x;
-        const int64_t stage_rows = std::max<int64_t>(n_tiles_all, c.cus) * x;
-        if (!by_model && nl < (opt.stage_factor >= 0 ? opt.stage_factor : 8) * stage_rows) join(rs, rl, nsh, nl);
+        if (!by_model && !pays_for_staging()) join(rs, rl, nsh, nl);
         // a small problem is one launch: splitting it only adds launch latency
         if (!by_model && nl && nnz_part < (opt.split_min_nnz >= 0 ? opt.split_min_nnz : (int64_t)4 * 1000 * 1000)) join(rl, rs, nl, nsh);
         // a class too small to fill the machine joins the other

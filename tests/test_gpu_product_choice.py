@@ -1,0 +1,67 @@
+"""Plans that also serve the product with the dense factor, where their column tiles would hold little or nothing of it: the form
+that is chosen, SDDMM and product against 64-bit sums, the same bits on every call, and the plan saved and loaded."""
+import pytest
+import torch
+
+from sddmm_gpu_amd import capi, synth
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def even_rows(n_rows, n_cols, per_row, n_long=0, long_row=0):
+    """per_row nonzeros a row, one in each of as many stretches of the columns; the first n_long rows have long_row."""
+    g = torch.Generator(device=DEV).manual_seed(per_row)
+
+    def rows(n, per):
+        step = n_cols // per
+        return (torch.arange(per, device=DEV) * step + torch.randint(0, step, (n, per), generator=g, device=DEV)).reshape(-1)
+    cols = torch.cat([rows(n_long, long_row)] * (n_long > 0) + [rows(n_rows - n_long, per_row)]).int()
+    deg = torch.full((n_rows,), per_row, device=DEV)
+    deg[:n_long] = long_row
+    return dict(n_rows=n_rows, n_cols=n_cols, nnz=int(cols.numel()), row_ptr=torch.cat([deg.new_zeros(1), deg.cumsum(0)]).int(), col_ind=cols)
+
+
+def plan_of(d, K, **opts):
+    return capi.Plan.from_device_csr(d["n_rows"], d["n_cols"], d["nnz"], d["row_ptr"].data_ptr(), d["col_ind"].data_ptr(), K,
+                                     options=capi.PlanOptions.defaults(spmm_stream=1, ignore_env=1, **opts))
+
+
+def check(d, K, plan, path):
+    n_rows, nnz, ci, stream = d["n_rows"], d["nnz"], d["col_ind"].long(), torch.cuda.current_stream().cuda_stream
+    rows = torch.repeat_interleave(torch.arange(n_rows, device=DEV), (d["row_ptr"][1:] - d["row_ptr"][:-1]).long())
+    g = torch.Generator(device=DEV).manual_seed(K)
+    W, H = torch.randn(n_rows, K, generator=g, device=DEV), torch.randn(d["n_cols"], K, generator=g, device=DEV)
+
+    def run(p):
+        out, Y = torch.full((nnz + 1,), 7.0, device=DEV), torch.full((n_rows * K + 1,), 7.0, device=DEV)
+        p.execute(0, W.data_ptr(), H.data_ptr(), out.data_ptr(), stream)
+        p.spmm(out.data_ptr(), H.data_ptr(), Y.data_ptr(), stream=stream)
+        torch.cuda.synchronize()
+        return out, Y
+    out, Y = run(plan)
+    assert float(out[-1]) == 7.0 and float(Y[-1]) == 7.0
+    ref, size = torch.zeros(n_rows, K, dtype=torch.float64, device=DEV), torch.zeros(n_rows, K, dtype=torch.float64, device=DEV)
+    for b in range(0, nnz, 1 << 19):
+        r, h, o = rows[b:b + (1 << 19)], H[ci[b:b + (1 << 19)]].double(), out[b:min(nnz, b + (1 << 19))].double()
+        p = W[r].double() * h
+        assert bool(((o - p.sum(1)).abs() <= (K + 16) * 2.0 ** -24 * p.abs().sum(1)).all())
+        ref.index_add_(0, r, o[:, None] * h)
+        size.index_add_(0, r, (o[:, None] * h).abs())
+    n = (d["row_ptr"][1:] - d["row_ptr"][:-1]).double()[:, None]  # a rounding per term of a row, however they are added up
+    assert bool(((Y[:-1].view(n_rows, K).double() - ref).abs() <= (n + 16) * 2.0 ** -24 * size).all())
+    plan.save(path)
+    loaded = capi.Plan.load_device(path, n_rows, d["n_cols"], nnz, d["row_ptr"].data_ptr(), d["col_ind"].data_ptr(), K)
+    assert loaded.spmm_form() == plan.spmm_form()
+    for a, b in zip(run(loaded), (out, Y)):
+        assert torch.equal(a, b)
+
+
+# no row is long enough for the tiles, or a few are
+@pytest.mark.parametrize("n_long", [0, 40])
+@pytest.mark.parametrize("K", [32, 50, 64])
+def test_rows_too_short_for_the_tiles(tmp_path, K, n_long):
+    d = even_rows(120000, 5600, 34, n_long, 2000)
+    plan = plan_of(d, K)
+    assert plan.spmm_form() == capi.SPMM_WALK and plan.info()["class_nnz"] == [d["nnz"], 0, 0]
+    check(d, K, plan, tmp_path / "p.plan")
