@@ -940,12 +940,14 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         // alone for the product, which wants long runs; otherwise the fixed rules hold for both.  SDDMM + product, us, long rows
         // in both and so: ratings of 4.9 M, K = 32 / 50 / 64 / 192 24 + 50 / 38 + 55 / 34 + 54 / 105 + 160 and 21 + 49 / 33 + 55 / 31
         // + 55 / 92 + 161, of 15.9 M 56 + 98 / 90 + 125 / 84 + 124 / 267 + 349 and 49 + 99 / 81 + 125 / 76 + 126 / 255 + 351; slices of
-        // 128, K = 100 / 128, 4.9 M: 59 + 91 / 56 + 93 and 64 + 91 / 65 + 94; all rows in both, 15.7 M, K = 64: 82 + 229.  Below 4 million nonzeros the split is the model's: the fixed rules make one class of the rows
-        // there, and the product mostly walks the CSR pattern (3 to 4 M, K = 256, windows: 196 + 174 by the fixed rules,
-        // 113 + 169 by the model; uniform 522 + 517 and 332 + 515).
+        // 128, K = 128, 4.9 M: 56 + 93 and 65 + 94; all rows in both, 15.7 M, K = 64: 82 + 229.  Below 4 million nonzeros the split
+        // is the model's: the fixed rules make one class of the rows there, and the product mostly walks the CSR pattern (3 to 4 M,
+        // K = 256, windows: 196 + 174 by the fixed rules, 113 + 169 by the model; uniform 522 + 517 and 332 + 515).  So it is at
+        // ranks without a tile width of their own (K = 96 / 100 / 300, the SDDMM by the fixed rules and by the model: uniform of
+        // 4.7 and 6.5 M 192 / 245 / - and 227 / 263 / 703, and 161 / 173 / - and 175 / 186 / 457).
         const bool tiled_product = opt.spmm_stream > 0 && nnz >= 4000000 && (!ragged || ragged_product_tiles(nnz, K, kt)) && spmm_tile_supported(kt);
         const bool model_fits = D.n_dense == 0 && opt.short_row_max < 0 && opt.stage_factor < 0 && opt.split_min_nnz < 0;
-        const bool by_model = model_fits && !tiled_product;
+        const bool by_model = model_fits && (!tiled_product || ragged);
         // staging every H tile must be paid for by the nonzeros that use it
         auto pays_for_staging = [&]() {
             const int64_t n_tiles_all = (n_cols + x - 1) / x, stage_rows = std::max<int64_t>(n_tiles_all, c.cus) * x;
@@ -956,16 +958,15 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         // the SDDMM only where the second model below agrees (SDDMM + product, us, gathered and so: uniform, 5 M of 17,770
         // columns, K = 32 / 64 47 + 43 / 74 + 75 and 30 + 45 / 59 + 76; 17 M of 112,000, K = 32, where it does not, 251 + 237 and
         // 351 + 236), and not in K slices, which would keep partial results in a buffer that the gather does without.
-        if (model_fits && tiled_product && kt <= 64) {
-            const bool long_class = pays_for_staging() && nl * 50 >= nnz;
-            if (long_class || K <= kt) {
-                const SplitChoice choice = estimate_split(c, ne, kt, x, g_long, short_max, 1e30);
-                if (choice.split == Split::all_tiled && (long_class || tile_slices_us(c, ne, kt) < choice.gather_us)) {
-                    if (long_class) c.sp_min_row = short_max;
-                    else c.sp_walk = true;
-                    join(rl, rs, nl, nsh);
-                }
-            }
+        const bool long_class = tiled_product && pays_for_staging() && nl * 50 >= nnz;
+        auto tile_all = [&]() {
+            if (long_class) c.sp_min_row = short_max;
+            join(rl, rs, nl, nsh);
+        };
+        if (model_fits && tiled_product && !long_class && (ragged || K <= kt)) c.sp_walk = true;
+        if (model_fits && tiled_product && !ragged && kt <= 64 && (long_class || K <= kt)) {
+            const SplitChoice choice = estimate_split(c, ne, kt, x, g_long, short_max, 1e30);
+            if (choice.split == Split::all_tiled && (long_class || tile_slices_us(c, ne, kt) < choice.gather_us)) tile_all();
         }
         int64_t slab_cols = 0;  // chosen by the model
         if (by_model) {
@@ -1012,7 +1013,7 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
             }
             switch (choice.split) {
             case Split::slabs: join(rs, rl, nsh, nl); slab_cols = slab.cols; break;
-            case Split::all_tiled: join(rl, rs, nl, nsh); break;
+            case Split::all_tiled: tile_all(); break;
             case Split::all_gathered: join(rs, rl, nsh, nl); break;
             case Split::by_length: break;
             }

@@ -65,3 +65,14 @@ def test_rows_too_short_for_the_tiles(tmp_path, K, n_long):
     plan = plan_of(d, K)
     assert plan.spmm_form() == capi.SPMM_WALK and plan.info()["class_nnz"] == [d["nnz"], 0, 0]
     check(d, K, plan, tmp_path / "p.plan")
+
+
+# ranks without a tile width of their own: the SDDMM is planned as in a plan without the product, whose rows are too short for tiles
+@pytest.mark.parametrize("K", [96, 100])
+def test_sddmm_as_without_the_product(tmp_path, K):
+    d = synth.uniform_random(30000, 40000, 0.0039, K=4, device=DEV)
+    plan = plan_of(d, K)
+    alone = capi.Plan.from_device_csr(d["n_rows"], d["n_cols"], d["nnz"], d["row_ptr"].data_ptr(), d["col_ind"].data_ptr(), K,
+                                      options=capi.PlanOptions.defaults(ignore_env=1))
+    assert plan.spmm_form() == capi.SPMM_WALK and plan.info()["class_nnz"] == alone.info()["class_nnz"] == [d["nnz"], 0, 0]
+    check(d, K, plan, tmp_path / "p.plan")
