@@ -167,15 +167,33 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
 // 167 / 190 us; of 2.6 and 3.8 M, K = 192: 148 / 131 and 180 / 184; K = 320, 1.8 and 2.6 M: 231 / 171 and 240 / 259).
 inline bool product_walks(int64_t nnz, int32_t K, int ks) { return nnz < 4000000 && nnz * K < (ks < 128 ? 700000000 : 450000000); }
 // And at a rank that is no multiple of the tiles' width ks, which they work on up to the next multiple?  From 4 million nonzeros
-// on they are the faster ones where little of that is padding (SDDMM + product, us, walk and tiles: ratings of 4.9 M, K = 20 / 30
-// / 36 / 50 / 75 / 120 68 / 77 / 95 / 102 / 160 / 179 and 73 / 75 / 90 / 92 / 143 / 153, K = 150 / 180 / 200 / 250 / 300 / 380 274 /
-// 285 / 313 / 368 / 577 / 624 and 282 / 290 / 293 / 305 / 441 / 457; 15.9 M, K = 50 / 120 / 150 / 200 / 300 257 / 506 / 780 / 964 / 2118
-// and 215 / 422 / 791 / 829 / 1250); below, where the walk has three slices or more (3.3 M, K = 200 / 220 / 250 / 280 / 340: 208 /
-// 218 / 240 / 387 / 402 and 248 / 250 / 253 / 365 / 370).
+// on, where little of that is padding (SDDMM + product, us, walk and tiles: ratings of 4.9 M, K = 20 / 36 / 50 / 75 / 120 68 / 95
+// / 102 / 160 / 179 and 73 / 90 / 92 / 143 / 153, K = 150 / 180 / 200 / 250 / 300 / 380 274 / 285 / 313 / 368 / 577 / 624 and 282 /
+// 290 / 293 / 305 / 441 / 457; 15.9 M, K = 50 / 120 / 150 / 200 / 300 257 / 506 / 780 / 964 / 2118 and 215 / 422 / 791 / 829 / 1250);
+// below, where the walk has three slices or more (3.3 M, K = 200 / 220 / 250 / 280 / 340: 208 / 218 / 240 / 387 / 402 and 248 /
+// 250 / 253 / 365 / 370).  And not at a width of 32: the work is little and the longest run, which eight lanes walk alone, sets
+// the time (K = 28, product alone, ratings of 4.2 and 5.1 M 45 / 65 and 53 / 51, word counts of 5.9 and 7.4 M 57 / 72 and 69 / 75).
 inline bool ragged_product_tiles(int64_t nnz, int32_t K, int ks)
 {
     const int padded = (K + ks - 1) / ks * ks;
-    return nnz < 4000000 ? K > 256 && !product_walks(nnz, K, ks) : K >= 28 && (K <= 128 || K * 100 >= padded * 72);
+    return nnz < 4000000 ? K > 256 && !product_walks(nnz, K, ks) : K > 32 && (K <= 128 || K * 100 >= padded * 72);
+}
+// The runs it takes for that, in nonzeros per run on average: a run costs a partial row of the padded width, its nonzeros cost
+// the walk K elements each.  So the line is one of run length times the used share of the width.  Product alone, us, walk and
+// tiles at (that figure):
+//   width 64: word counts of 9.4 M, K = 36 / 50 / 60 101 / 119 (8.9), 120 / 121 (12.3), 131 / 124 (14.8); 8.9 M of 40,000 columns 109 /
+//       128 (13.4), 134 / 130 (18.7), 147 / 132 (22); uniform, 5.9 M, K = 44 / 50 74 / 69 (12.6), 79 / 69 (14.3)
+//   width 128: word counts of 5.3 M, K = 100 / 120 129 / 178 (7.6), 144 / 180 (9.1), 11 M, K = 100 / 120 227 / 275 (9.8), 254 / 277 (11.7),
+//       11.7 M, K = 72 / 100 203 / 203 (12.9), 258 / 205 (18); uniform, 11.7 M, K = 72 / 100 225 / 245 (8.5), 385 / 245 (11.9).  With
+//       an H of less than 2.5 MB, ratings of 4.9 and 6.3 M and word counts of 5.9 M, K = 72 101 / 92 (9.7), 123 / 103 (11.3), 112 / 103 (10.5)
+//   two slices: word counts of 11 M, K = 200 / 250 448 / 553 (9.8), 629 / 560 (12.2), 5.3 M 335 / 370 (9.5); ratings, 4.9 M, 193 / 181 (13.5)
+//   more: word counts of 9.4, 5.3 and 11 M, K = 300 905 / 1100 (6.3), 553 / 547 (7.6), 1028 / 835 (9.8); uniform, 11.7 M 1879 / 1152
+//       (7.1); below 4 M nonzeros, ratings of 3.4 M, K = 290 / 370 286 / 300 (7.5), 313 / 322 (9.5), of 2.4 M 204 / 194 (10.2)
+inline double ragged_product_run(int64_t nnz, int64_t n_cols, int32_t K, int ks)
+{
+    const double padded = (K + ks - 1) / ks * ks;
+    const double least = ks < 128 ? 13.5 : K <= 128 ? (4.0 * n_cols * K <= 2.5e6 ? 8.0 : 11.8) : K <= 256 ? 11.0 : nnz < 4000000 ? 10.0 : 7.0;
+    return least * padded / K;
 }
 // planner_tile.hip: the rows' nonzeros in tile order (tiles of x columns), every (row, tile) run padded
 // ks: K elements per launch, a divisor of K or (ragged ranks) the width K is rounded up to

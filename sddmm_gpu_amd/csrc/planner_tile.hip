@@ -255,7 +255,8 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         }
         // (sp_seg == 0: tiles that would hold nothing)
         if (want_spmm && rb == 0 && c.nnz == c.P->info.nnz &&
-            (c.sp_walk || sp_seg == 0 || (ragged && !ragged_product_tiles(c.nnz, c.K, ks)) || (h_near && sp_nnz < 12 * sp_seg) || small_walks || sp_nnz < (c.K <= 128 ? 8 : 5) * sp_seg)) { want_spmm = false; sp_csr = true; }
+            (c.sp_walk || sp_seg == 0 || (h_near && sp_nnz < 12 * sp_seg) || small_walks || sp_nnz < (c.K <= 128 ? 8 : 5) * sp_seg ||
+             (ragged && (!ragged_product_tiles(c.nnz, c.K, ks) || sp_nnz < ragged_product_run(c.nnz, c.n_cols, c.K, ks) * sp_seg)))) { want_spmm = false; sp_csr = true; }
         // row-block boundaries of the 2-D assignment: equal shares of the rows' nonzeros
         std::vector<int32_t> cut;
         auto make_cuts = [&](int n_shares) {

@@ -76,3 +76,20 @@ def test_sddmm_as_without_the_product(tmp_path, K):
                                       options=capi.PlanOptions.defaults(ignore_env=1))
     assert plan.spmm_form() == capi.SPMM_WALK and plan.info()["class_nnz"] == alone.info()["class_nnz"] == [d["nnz"], 0, 0]
     check(d, K, plan, tmp_path / "p.plan")
+
+
+# ranks without a tile width of their own: tiles where the runs, times the share of the width that is used, are long enough
+@pytest.mark.parametrize("kind,sizes,K,form", [
+    ("bag_of_words", (20000, 17000, 480), 28, capi.SPMM_WALK),
+    ("bag_of_words", (20000, 17000, 480), 36, capi.SPMM_WALK),
+    ("bag_of_words", (20000, 17000, 480), 60, capi.SPMM_TILES),
+    ("bag_of_words", (20000, 17000, 480), 100, capi.SPMM_WALK),
+    ("bag_of_words", (20000, 17000, 480), 300, capi.SPMM_WALK),
+    ("bag_of_words", (8000, 17000, 1500), 100, capi.SPMM_TILES),
+    ("uniform_random", (20000, 12000, 0.05), 300, capi.SPMM_TILES),
+])
+def test_form_by_the_length_of_runs(tmp_path, kind, sizes, K, form):
+    d = getattr(synth, kind)(*sizes, K=4, device=DEV)
+    plan = plan_of(d, K)
+    assert plan.spmm_form() == form
+    check(d, K, plan, tmp_path / "p.plan")
