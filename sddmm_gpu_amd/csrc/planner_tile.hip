@@ -760,6 +760,9 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
             build_spmm(keys);
         }
     }
+    // (ranks without a tile width of their own whose rows are dealt out to groups of workgroups, or whose stream has several
+    // panels: no runs to multiply, and the product walks the pattern with its cut rows kept)
+    if (want_spmm && ragged && !sp.built && c.nnz == c.P->info.nnz) { want_spmm = false; sp_csr = true; }
     unit_ptr.push_back((int32_t)np);
     const int64_t n_blocks = (int64_t)unit_tile.size();
     // The kernel requests index data two batches ahead without clamping: past the last

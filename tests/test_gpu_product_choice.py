@@ -93,3 +93,13 @@ def test_form_by_the_length_of_runs(tmp_path, kind, sizes, K, form):
     plan = plan_of(d, K)
     assert plan.spmm_form() == form
     check(d, K, plan, tmp_path / "p.plan")
+
+
+# ranks without a tile width of their own, rows dealt out to groups of workgroups or a stream of several panels: no runs for the
+# product, which walks the pattern and gives the same bits on every call
+@pytest.mark.parametrize("sizes,K,opts", [((100000, 64, 512), 100, {}), ((100000, 64, 512), 300, {}), ((20000, 300, 1000), 100, dict(tile_size_x=250, tile_size_y=5000))])
+def test_launches_without_runs(tmp_path, sizes, K, opts):
+    d = synth.banded(*sizes, K=4, device=DEV)
+    plan = plan_of(d, K, **opts)
+    assert plan.spmm_form() == capi.SPMM_WALK and plan.info()["n_row_panels"] > 1
+    check(d, K, plan, tmp_path / "p.plan")
