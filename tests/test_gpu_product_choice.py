@@ -103,3 +103,14 @@ def test_launches_without_runs(tmp_path, sizes, K, opts):
     plan = plan_of(d, K, **opts)
     assert plan.spmm_form() == capi.SPMM_WALK and plan.info()["n_row_panels"] > 1
     check(d, K, plan, tmp_path / "p.plan")
+
+
+# small matrices whose SDDMM alone would be gathered: beside a product it stays on tiles, for the product walks with its cut rows kept
+@pytest.mark.parametrize("kind,sizes,K", [("banded", (4000, 60, 400), 96), ("banded", (10000, 40, 300), 64), ("rmat", (15, 800000), 100)])
+def test_small_matrices_keep_the_walk(tmp_path, kind, sizes, K):
+    d = getattr(synth, kind)(*sizes, K=4, device=DEV)
+    alone = capi.Plan.from_device_csr(d["n_rows"], d["n_cols"], d["nnz"], d["row_ptr"].data_ptr(), d["col_ind"].data_ptr(), K,
+                                      options=capi.PlanOptions.defaults(ignore_env=1))
+    plan = plan_of(d, K)
+    assert alone.info()["kernel"] == capi.KERNEL_ROW_GATHER and plan.spmm_form() == capi.SPMM_WALK
+    check(d, K, plan, tmp_path / "p.plan")
