@@ -243,10 +243,11 @@ hipError_t launch_block_long_rows(const BlockArgs &a, const int32_t *row_ptr, vo
 hipError_t launch_block_spmm(const BlockArgs &a, int nwaves, void *stream);
 
 // lanes per nonzero and float4 slots per lane for a given K; G == 0: none
-// How the row gather over nnz nonzeros of n_rows rows is dealt out: its variant (any K from 4 to 2048), nonzeros per
-// workgroup, and whether a wave has one batch of 64 and the kernel made for that.
+// How the row gather over nnz nonzeros of a matrix of n_rows rows is dealt out, listed_rows of them with a nonzero if that is
+// known (else n_rows): its variant (any K from 4 to 2048), nonzeros per workgroup, and whether a wave has one batch of 64 and
+// the kernel made for that.
 struct GatherShape { Variant v; int chunk; bool once; };
-GatherShape gather_shape(int64_t nnz, int64_t n_rows, int K);
+GatherShape gather_shape(int64_t nnz, int64_t n_rows, int64_t listed_rows, int K);
 inline bool gather_wide(int64_t n_rows, int64_t n_cols, int K) { return std::max(n_rows, n_cols) * K >= (int64_t)1 << 30; }  // byte offsets of 32 bits do not do
 KernelFn gather_kernel(const Variant &v, bool once, bool wide);
 KernelFn generic_kernel();           // row gather, any K

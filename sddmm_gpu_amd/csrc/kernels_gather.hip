@@ -396,14 +396,17 @@ static Variant pick_gather_variant(int K)
 // where a third of the lanes would idle in large matrices (K = 36, 1.8 / 8.4 million: 41 / 176 and 41 / 180), nor at K = 65 to
 // 96 (1.8 million, K = 72 / 90 57 / 65 and 66 / 69) and beyond 128 (K = 150 / 200 104 / 137 and 113 / 135), nor below (0.17
 // million, K = 50 / 100: 6.7 / 10.1 and 6.8 / 10.4), nor with several batches (R-MAT 2^15, 1.2 million, K = 100: 41 and 46).
-GatherShape gather_shape(int64_t nnz, int64_t n_rows, int K)
+//
+// The form decides the order a dot product is added up in, and a plan and the call without one give the same bits: it goes by
+// n_rows, empty rows among them, which is what both know; listed_rows, the rows a plan has listed, decides the rest.
+GatherShape gather_shape(int64_t nnz, int64_t n_rows, int64_t listed_rows, int K)
 {
     Variant v = pick_gather_variant(K);
     const int pieces = v.G * v.KPL, used = (K + 3) / 4;
-    const bool short_rows = nnz <= (pieces > 4 && nnz * pieces >= 8000000 ? 32 : 16) * n_rows;
-    const bool line_wise = nnz >= 1 << 18 && ((pieces == 16 && (used >= 10 || nnz < 1 << 20)) || (pieces == 32 && !v.exact));
-    const bool once = v.G != 0 && (nnz <= 1 << 16 || (short_rows ? pieces != 16 || line_wise : pieces <= 8 && nnz <= 1 << 18));
-    if (once && line_wise) v = {pieces, 1, v.exact};
+    auto short_rows = [&](int64_t rows) { return nnz <= (pieces > 4 && nnz * pieces >= 8000000 ? 32 : 16) * rows; };
+    const bool line_wise = nnz >= 1 << 18 && short_rows(n_rows) && ((pieces == 16 && (used >= 10 || nnz < 1 << 20)) || (pieces == 32 && !v.exact));
+    const bool once = v.G != 0 && (line_wise || nnz <= 1 << 16 || (short_rows(listed_rows) ? pieces != 16 : pieces <= 8 && nnz <= 1 << 18));
+    if (line_wise) v = {pieces, 1, v.exact};
     const int64_t waves_wanted = 4096;
     const int per_wave = once ? 1 : nnz >= 1500000 ? kRowGatherBatchesPerWave
                                                    : (int)std::clamp<int64_t>(nnz / (64 * waves_wanted), 1, kRowGatherBatchesPerWave);

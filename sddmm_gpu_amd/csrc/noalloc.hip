@@ -26,7 +26,7 @@ extern "C" int sddmm_csr_noalloc(int64_t n_rows, int64_t n_cols, int64_t nnz, co
     a.col_ind = d_col_ind; a.val = d_val; a.W = d_W; a.H = d_H; a.out = d_out;
     a.row_ptr = d_row_ptr; a.n_rows = (int32_t)n_rows;
     a.nnz = (int32_t)nnz; a.K = K; a.n_cols = (int32_t)n_cols; a.tile_x = (int32_t)n_cols;
-    const GatherShape shape = gather_shape(nnz, n_rows, K);
+    const GatherShape shape = gather_shape(nnz, n_rows, n_rows, K);
     const KernelFn fn = shape.v.G ? gather_kernel(shape.v, shape.once, gather_wide(n_rows, n_cols, K)) : generic_kernel();
     a.chunk = shape.chunk;
     const int grid = (int)((nnz + a.chunk - 1) / a.chunk);

@@ -256,7 +256,7 @@ int add_row_gather(Ctx &c, const std::vector<int32_t> &rows, bool all_rows)
     const int64_t n = all_rows ? c.nnz : list_nnz(c, rows);
     L.nnz = n;
     if (n == 0) return SDDMM_OK;
-    const GatherShape shape = gather_shape(n, (int64_t)rows.size(), c.K);
+    const GatherShape shape = gather_shape(n, all_rows ? c.n_rows : (int64_t)rows.size(), (int64_t)rows.size(), c.K);
     const Variant var = shape.v;
     L.fn_kind = 1; L.fn_g = var.G; L.fn_kpl = var.KPL; L.fn_exact = var.exact;
     std::vector<int32_t> seg_end(rows.size()), perm;

@@ -94,3 +94,21 @@ def test_ranks_read_line_by_line(n_rows, nnz, K):
                      torch.cuda.current_stream().cuda_stream)
     torch.cuda.synchronize()
     assert ((out[:nnz].cpu().double() - ref).abs() <= bound).all() and float(out[nnz]) == 7.0
+
+
+# many empty rows: the plan lists the others, the call without a plan knows only how many there are of both
+@pytest.mark.parametrize("K", [33, 50, 64, 100])
+def test_same_bits_with_and_without_a_plan_beside_empty_rows(K):
+    used, n_rows, n_cols, nnz = 5000, 40000, 200, 2 ** 18
+    (rp, ci, val, W, H), ref, bound = _case(used, n_cols, nnz, K, K)
+    rp = torch.cat([rp, rp[-1:].repeat(n_rows - used)])
+    W = torch.cat([W, W.new_zeros(n_rows - used, K)])
+    outs = [torch.full((nnz + 1,), 7.0, device="cuda") for _ in range(2)]
+    stream = torch.cuda.current_stream().cuda_stream
+    capi.csr_noalloc(n_rows, n_cols, nnz, rp.data_ptr(), ci.data_ptr(), val.data_ptr(), K, W.data_ptr(), H.data_ptr(), outs[0].data_ptr(), stream)
+    plan = capi.Plan.from_device_csr(n_rows, n_cols, nnz, rp.data_ptr(), ci.data_ptr(), K,
+                                     options=capi.PlanOptions.defaults(kernel=capi.KERNEL_ROW_GATHER))
+    plan.execute(val.data_ptr(), W.data_ptr(), H.data_ptr(), outs[1].data_ptr(), stream)
+    torch.cuda.synchronize()
+    assert ((outs[0][:nnz].cpu().double() - ref).abs() <= bound).all()
+    assert torch.equal(outs[0], outs[1]) and float(outs[0][nnz]) == 7.0
