@@ -854,7 +854,9 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
     // 2.98 ms against 1.46).
     // The threshold is flat: 3118 / 3113 / 3166 / 3284 us at K = 512 for 40 / 30 / 22 / 16 % filled.
     bool want_dense = opt.dense_blocks > 0 || (opt.dense_blocks < 0 && K >= (opt.spmm_stream > 0 ? 512 : 384));
-    if (want_dense && opt.dense_blocks < 0 && opt.spmm_stream > 0 && nnz >= 4000000 && long_rows(n_rows, n_cols, nnz, row_ptr_all)) want_dense = false;
+    // (a caller who says how the core is to be found wants one)
+    const bool core_left_open = opt.dense_blocks < 0 && opt.dense_permille < 0 && opt.dense_min_nnz < 0 && opt.dense_rb_group < 0;
+    if (want_dense && core_left_open && opt.spmm_stream > 0 && nnz >= 4000000 && long_rows(n_rows, n_cols, nnz, row_ptr_all)) want_dense = false;
     if (kernel == SDDMM_KERNEL_HYBRID && want_dense && K % 32 == 0 && kt / 4 > 16 &&
         (int64_t)n_rows * (K / 4) <= (int64_t)UINT32_MAX && (int64_t)n_cols * (K / 4) <= (int64_t)UINT32_MAX) {
         const double threshold = (double)(opt.dense_permille > 0 ? opt.dense_permille : 300) / 1000.0;

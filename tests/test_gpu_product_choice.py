@@ -114,3 +114,11 @@ def test_small_matrices_keep_the_walk(tmp_path, kind, sizes, K):
     plan = plan_of(d, K)
     assert alone.info()["kernel"] == capi.KERNEL_ROW_GATHER and plan.spmm_form() == capi.SPMM_WALK
     check(d, K, plan, tmp_path / "p.plan")
+
+
+# where rows are long the product takes the column tiles, without a dense core, unless the caller has said how that is to be found
+@pytest.mark.parametrize("opts,core", [({}, False), (dict(dense_permille=250), True), (dict(dense_min_nnz=0), True), (dict(dense_blocks=1), True), (dict(dense_blocks=0), False)])
+def test_dense_core_that_was_asked_for(opts, core):
+    d = synth.recommender(44000, 5600, K=4, seed=5, device=DEV, max_deg=5000)
+    plan = plan_of(d, 512, **opts)
+    assert (plan.info()["dense_blocks"] > 0) == core and plan.spmm_form() == (capi.SPMM_CSR if core else capi.SPMM_TILES)
