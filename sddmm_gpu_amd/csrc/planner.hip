@@ -962,7 +962,7 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         // 351 + 236), and not in K slices, which would keep partial results in a buffer that the gather does without.
         const bool long_class = tiled_product && pays_for_staging() && nl * 50 >= nnz;
         auto tile_all = [&]() {
-            if (long_class) c.sp_min_row = short_max;
+            if (long_class && nsh * 2000 >= nnz) c.sp_min_row = short_max;  // (a handful of short rows are not worth gathering, as below)
             join(rl, rs, nl, nsh);
         };
         if (model_fits && tiled_product && !long_class && (ragged || K <= kt)) c.sp_walk = true;
