@@ -181,8 +181,10 @@ inline bool ragged_product_tiles(int64_t nnz, int32_t K, int ks)
 // The runs it takes for that, in nonzeros per run on average: a run costs a partial row of the padded width, its nonzeros cost
 // the walk K elements each.  So the line is one of run length times the used share of the width.  Product alone, us, walk and
 // tiles at (that figure):
-//   width 64: word counts of 9.4 M, K = 36 / 50 / 60 101 / 119 (8.9), 120 / 121 (12.3), 131 / 124 (14.8); 8.9 M of 40,000 columns 109 /
-//       128 (13.4), 134 / 130 (18.7), 147 / 132 (22); uniform, 5.9 M, K = 44 / 50 74 / 69 (12.6), 79 / 69 (14.3)
+//   width 64: word counts of 9.4 M, K = 50 / 60 120 / 121 (12.3), 131 / 124 (14.8); uniform, 5.9 M, K = 50 79 / 69 (14.3); up to
+//       K = 48, whose rows are few lines each to the walk, 8.9 M of 40,000 columns, K = 40 / 48 111 / 129 (15.0), 113 / 130 (18.0),
+//       uniform, 11.7 M, K = 40 127 / 94 (19.1); with an H of less than 2.5 MB, word counts of 7.4 M, K = 48 82 / 92 (14.4), of 11 M,
+//       K = 40 / 44 116 / 108 (15.4), 126 / 108 (16.9)
 //   width 128: word counts of 5.3 M, K = 100 / 120 129 / 178 (7.6), 144 / 180 (9.1), 11 M, K = 100 / 120 227 / 275 (9.8), 254 / 277 (11.7),
 //       11.7 M, K = 72 / 100 203 / 203 (12.9), 258 / 205 (18); uniform, 11.7 M, K = 72 / 100 225 / 245 (8.5), 385 / 245 (11.9).  With
 //       an H of less than 2.5 MB, ratings of 4.9 and 6.3 M and word counts of 5.9 M, K = 72 101 / 92 (9.7), 123 / 103 (11.3), 112 / 103 (10.5)
@@ -192,7 +194,8 @@ inline bool ragged_product_tiles(int64_t nnz, int32_t K, int ks)
 inline double ragged_product_run(int64_t nnz, int64_t n_cols, int32_t K, int ks)
 {
     const double padded = (K + ks - 1) / ks * ks;
-    const double least = ks < 128 ? 13.5 : K <= 128 ? (4.0 * n_cols * K <= 2.5e6 ? 8.0 : 11.8) : K <= 256 ? 11.0 : nnz < 4000000 ? 10.0 : 7.0;
+    const bool small_h = 4.0 * n_cols * K <= 2.5e6;
+    const double least = ks < 128 ? (K > 48 ? 13.5 : small_h ? 15.0 : 19.0) : K <= 128 ? (small_h ? 8.0 : 11.8) : K <= 256 ? 11.0 : nnz < 4000000 ? 10.0 : 7.0;
     return least * padded / K;
 }
 // planner_tile.hip: the rows' nonzeros in tile order (tiles of x columns), every (row, tile) run padded
