@@ -5,6 +5,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <unistd.h>
 #include "plan.hpp"
@@ -698,26 +699,40 @@ static double tile_slices_us(const Ctx &c, const std::vector<int32_t> &rows, int
     }
     const int64_t tiles = (c.n_cols + x - 1) / x;
     const size_t n = rows.size(), stride = std::max<size_t>({1, n / 4096, (size_t)((double)c.nnz / 1.0e6)});
-    std::vector<double> items((size_t)(blocks * tiles), 0.0);
-    double sampled = 0, pos = 0, runs = 0;
+    struct Part { std::vector<double> items; double sampled = 0, pos = 0, runs = 0; };
+    Part all;
+    all.items.assign((size_t)(blocks * tiles), 0.0);
+    std::mutex merge;
     const int32_t width = (int32_t)x;
-    for (size_t k = stride / 2; k < n; k += stride) {
-        const int32_t b = c.row_ptr[rows[k]], e = c.row_ptr[rows[k] + 1];
-        const int64_t block = std::min<int64_t>(blocks - 1, (int64_t)((double)b / c.nnz * blocks));
-        sampled += e - b;
-        for (int32_t p = b; p < e;) {
-            const int32_t tile = c.col_ind[p] / width;
-            const int64_t end = ((int64_t)tile + 1) * width;
-            int32_t q = p + 1;
-            while (q < e && c.col_ind[q] < end) ++q;
-            const int len = q - p, r = len % g;
-            const double run = len - r + (r == 0 ? 0 : g == 8 && r <= 4 ? 4.5 : g);
-            items[(size_t)(block * tiles + tile)] += run;
-            pos += run;
-            runs += 1;
-            p = q;
+    const int64_t rows_sampled = n > stride / 2 ? (int64_t)((n - stride / 2 + stride - 1) / stride) : 0;
+    // (65,000 nonzeros a thread at least; the sums are whole or half numbers, the same in any order)
+    const int64_t grain = std::max<int64_t>(1, rows_sampled * 65536 / std::max<int64_t>(1, (int64_t)((double)c.nnz / stride)));
+    parallel_ranges(rows_sampled, grain, [&](int64_t from, int64_t to, int) {
+        Part part;
+        part.items.assign(all.items.size(), 0.0);
+        for (int64_t k = from; k < to; ++k) {
+            const int32_t row = rows[stride / 2 + (size_t)k * stride], b = c.row_ptr[row], e = c.row_ptr[row + 1];
+            const int64_t block = std::min<int64_t>(blocks - 1, (int64_t)((double)b / c.nnz * blocks));
+            part.sampled += e - b;
+            for (int32_t p = b; p < e;) {
+                const int32_t tile = c.col_ind[p] / width;
+                const int64_t end = ((int64_t)tile + 1) * width;
+                int32_t q = p + 1;
+                while (q < e && c.col_ind[q] < end) ++q;
+                const int len = q - p, r = len % g;
+                const double run = len - r + (r == 0 ? 0 : g == 8 && r <= 4 ? 4.5 : g);
+                part.items[(size_t)(block * tiles + tile)] += run;
+                part.pos += run;
+                part.runs += 1;
+                p = q;
+            }
         }
-    }
+        std::lock_guard<std::mutex> one(merge);
+        for (size_t i = 0; i < part.items.size(); ++i) all.items[i] += part.items[i];
+        all.sampled += part.sampled; all.pos += part.pos; all.runs += part.runs;
+    });
+    const double sampled = all.sampled, pos = all.pos, runs = all.runs;
+    const std::vector<double> &items = all.items;
     if (sampled <= 0) return 1e30;
     if (run_length) *run_length = sampled / runs;
     const double f = c.nnz / sampled, slices = (c.K + w - 1) / w;
@@ -979,14 +994,16 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
             SplitChoice choice = estimate_split(c, ne, kt, x, g_long, short_max, slab.us);
             // A second look at three kinds of choice that it gets wrong by up to a factor of two, each with the margin at which
             // 260 measured plans show gains and next to no losses (us before and so):
-            if (opt.k_slice <= 0 && opt.tile_lanes <= 0 && tile_x == 0 && (kt == 32 || kt == 64 || kt == 128) && nnz > 0) {
+            // (rows of H of other ranks than 16 and multiples of 32 lie across lines: the row gather's time by lines)
+            const bool across = K % 32 != 0 && K != 16;
+            const bool open = (opt.spmm_stream <= 0 && choice.split == Split::all_tiled && nnz < 1500000) ||
+                              (choice.split == Split::all_gathered && across && K <= kt) || (opt.spmm_stream <= 0 && choice.split != Split::all_gathered && K > kt);
+            if (open && opt.k_slice <= 0 && opt.tile_lanes <= 0 && tile_x == 0 && (kt == 32 || kt == 64 || kt == 128) && nnz > 0) {
                 double run_length = 0;
                 const double tiled = tile_slices_us(c, ne, kt, &run_length);
                 // small matrices, and on tiles of which a few hold most (bands of 0.2 / 0.4 M, K = 96 / 50 15.5 / 17.9 and 7.8 / 9.5;
                 // R-MAT of 0.75 M, K = 96 40 and 23; ratings of 0.17 / 0.35 M, K = 96 / 32 8.0 / 6.6 and 6.1 / 5.3); not behind
                 // a product, which walks the pattern with its cut rows kept only beside a tile launch
-                // (rows of H of other ranks than 16 and multiples of 32 lie across lines: the row gather's time by lines)
-                const bool across = K % 32 != 0 && K != 16;
                 const double h_all = (double)n_cols * K * 4, lines = nnz * ((4.0 * K - 4) / 128 + 1) * 128;
                 const double gathered = across ? 4.5 + 1e-6 * lines / (h_all <= 4.2e6 ? 22.0 : h_all <= 64.0e6 ? 13.8 : 9.6) : choice.gather_us;
                 if (opt.spmm_stream <= 0 && choice.split == Split::all_tiled && nnz < 1500000 && tiled > (nnz < 500000 ? 1.0 : 1.2) * gathered) choice.split = Split::all_gathered;
