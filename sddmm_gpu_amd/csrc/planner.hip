@@ -844,7 +844,7 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
 
     // row-panel height of the tile kernel's stream: the panel's W slice (y rows of kt floats)
     // should stay L2-resident while the workgroups sweep the panel's column tiles
-    int32_t y_panel = tile_y > 0 ? tile_y : (kt ? (int32_t)std::max<int64_t>(256, (opt.panel_bytes > 0 ? opt.panel_bytes : (int64_t)(2 << 20)) / (kt * 4)) : 1);
+    auto y_panel = [&]() { return tile_y > 0 ? tile_y : (kt ? (int32_t)std::max<int64_t>(256, (opt.panel_bytes > 0 ? opt.panel_bytes : (int64_t)(2 << 20)) / (kt * 4)) : 1); };
 
     int kernel = want;
     if (kernel == SDDMM_KERNEL_AUTO) kernel = SDDMM_KERNEL_HYBRID;
@@ -1048,7 +1048,7 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         // banded 2^20, K = 512: 711 nonzeros took 0.065 ms of a 4.14 ms step)
         if (!rl.empty() && !rs.empty() && opt.short_row_max < 0 && nsh * 2000 < nnz_part) join(rl, rs, nl, nsh);
         if (!rl.empty())
-            if (int rc = add_tile(c, rl, x, y_panel, opt.tile_lanes, kt, &I, false, tile_x > 0)) return rc;
+            if (int rc = add_tile(c, rl, x, y_panel(), opt.tile_lanes, kt, &I, false, tile_x > 0)) return rc;
         if (!rs.empty()) {
             // short rows: the padded, pipelined kernel reading H from global memory when the
             // rows are short enough for padding to stay cheap; the plain row gather otherwise
@@ -1086,7 +1086,7 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         if (kt && opt.unpadded_tile <= 0) {
             int32_t x = tile_x > 0 ? std::min(tile_x, fit_t) : fit_t;
             x = (int32_t)std::min<int64_t>(x, std::max<int64_t>(n_cols, 1));
-            if (int rc = add_tile(c, ne, x, tile_y > 0 ? tile_y : y_panel, opt.tile_lanes, kt, &I, false, tile_x > 0)) return rc;
+            if (int rc = add_tile(c, ne, x, y_panel(), opt.tile_lanes, kt, &I, false, tile_x > 0)) return rc;
         } else {
             int32_t x = tile_x > 0 ? std::min(tile_x, fit_x) : fit_x;
             x = (int32_t)std::min<int64_t>(x, std::max<int64_t>(n_cols, 1));
