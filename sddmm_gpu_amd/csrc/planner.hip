@@ -997,7 +997,7 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
             // (rows of H of other ranks than 16 and multiples of 32 lie across lines: the row gather's time by lines)
             const bool across = K % 32 != 0 && K != 16;
             const bool open = (opt.spmm_stream <= 0 && choice.split == Split::all_tiled && nnz < 1500000) ||
-                              (choice.split == Split::all_gathered && across && K <= kt) || (opt.spmm_stream <= 0 && choice.split != Split::all_gathered && K > kt);
+                              (choice.split == Split::all_gathered && across && K <= kt) || (opt.spmm_stream <= 0 && choice.split != Split::all_gathered && K > kt && opt.fuse_slices <= 0);
             if (open && opt.k_slice <= 0 && opt.tile_lanes <= 0 && tile_x == 0 && (kt == 32 || kt == 64 || kt == 128) && nnz > 0) {
                 double run_length = 0;
                 const double tiled = tile_slices_us(c, ne, kt, &run_length);
@@ -1014,7 +1014,8 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
                 // (Neither gives K slices to a plan that has none: it would get partial results in a buffer of its own, and calls
                 // on it that overlap in time, which were right, would no longer be.  Uniform, 4.7 M of 40,000 columns, K = 96 / 128
                 // 204 / 204 and, in slices of 32, 102 / 141: a caller whose calls follow each other may ask for them, k_slice.)
-                else if (opt.spmm_stream <= 0 && K > kt && choice.split != Split::all_gathered && run_length < 4) {
+                // (And such slices have no form that runs them all in one launch, for a caller who asks for that.)
+                else if (opt.spmm_stream <= 0 && K > kt && choice.split != Split::all_gathered && opt.fuse_slices <= 0 && run_length < 4) {
                     const double now = choice.split == Split::all_tiled ? tiled : choice.us;
                     int thin = 0;
                     double thin_us = 0.8 * now;

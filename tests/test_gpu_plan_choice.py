@@ -83,3 +83,10 @@ def test_overlapping_calls(kind, sizes, K):
     torch.cuda.synchronize()
     for i, o in enumerate(outs):
         assert torch.equal(o, want[i % 2])
+
+
+def test_one_launch_that_was_asked_for():
+    d = synth.uniform_random(30281, 34347, 0.0063, K=4, seed=3, device=DEV)
+    plan = capi.Plan.from_device_csr(d["n_rows"], d["n_cols"], d["nnz"], d["row_ptr"].data_ptr(), d["col_ind"].data_ptr(), 256,
+                                     options=capi.PlanOptions.defaults(fuse_slices=1, ignore_env=1))
+    assert plan.info()["n_launches"] == 1 and plan.info()["k_slice"] == 128
