@@ -31,7 +31,7 @@ TileFn tile_kernel_part4(const TileVariant &v, int vmode, bool gather, int slice
 TileFn tile_kernel(const TileVariant &v, int vmode, bool gather, int slice, int nwaves, bool ragged)
 {
     if (gather && v.G == 4) return slab_gather_kernel(16 * v.KPL, slice == 1 || slice == 2 ? 2 : vmode, slice);
-    if (slice == 1 || slice == 2) return tile_kernel_part2(v, 2, gather, slice, nwaves, ragged);  // (no values read)
+    if (slice == 1 || slice == 2 || slice == 6 || slice == 7) return tile_kernel_part2(v, 2, gather, slice, nwaves, ragged);  // (no values read)
     switch (vmode) {
     case 0: return tile_kernel_part0(v, vmode, gather, slice, nwaves, ragged);
     case 1: return tile_kernel_part1(v, vmode, gather, slice, nwaves, ragged);

@@ -315,7 +315,7 @@ __device__ __forceinline__ void matrix_core_waves(const TileArgs &a, int mw, int
 // 3 = all a.n_slices K slices inside this one launch, one after the other (small matrices, where a
 // launch costs as much as its work): a wave meets the same positions in every slice, so the partial
 // results it left in a.part are its own, and a workgroup barrier between the slices is all the
-// ordering needed.  5 = the same with a tile's batches in turn (see in_turn).
+// ordering needed.  5 = the same with a tile's batches in turn (see in_turn); 6, 7, 8 = 1, 2, 4 so, of ragged ranks.
 // RAGGED: K is no multiple of the kernel's width (K <= 4 * G * KPL: one launch; else the last of several slices is cut
 // short), and K needs no alignment: H rows are staged with the tail filled up with zeros, W rows are read in pieces at
 // any 4-byte address, the one at the end of the row from its last four floats on with what it shares with the piece
@@ -328,10 +328,12 @@ template <int G, int KPL, int VMODE, int NW, bool GATHER, int SLICE, int NWM = 0
 __global__ __launch_bounds__((NW + NWM) * 64)
 void sddmm_tile_kernel(const TileArgs a)
 {
+    static_assert(SLICE <= 5 || RAGGED);
     constexpr bool FUSED = SLICE == 3 || SLICE == 5;
-    constexpr bool ACC = SLICE == 2 || SLICE == 4;
+    constexpr bool FIRST = SLICE == 1 || SLICE == 6, BETWEEN = SLICE == 2 || SLICE == 7, LAST = SLICE == 4 || SLICE == 8;
+    constexpr bool ACC = BETWEEN || LAST;
     constexpr bool PART = SLICE >= 1;
-    constexpr bool TO_OUT = SLICE == 0 || SLICE >= 3;  // positions and values are needed
+    constexpr bool TO_OUT = SLICE == 0 || FUSED || LAST;  // positions and values are needed
     static_assert(TO_OUT || VMODE == 2);
     static_assert(!RAGGED || (!GATHER && NWM == 0));
     extern __shared__ float4 lds_tile[];
@@ -508,9 +510,9 @@ void sddmm_tile_kernel(const TileArgs a)
             wg_sync();
         }
         // A wave takes an equal, contiguous part of the item's batches or, where the plan asks for it, every NW-th of them.  (With
-        // all slices in one launch a kernel of its own: the choice between both inside it costs 1 % of word counts of 0.7 M
-        // nonzeros, K = 256, and 4 % at ragged ranks.)
-        const bool in_turn = FUSED ? SLICE == 5 : !GATHER && a.in_turn;
+        // all slices in one launch, and in the slices of ragged ranks, a kernel of its own: the choice between both inside it costs
+        // 1 % of word counts of 0.7 M nonzeros, K = 256, and 2 to 4 % at ragged ranks, 9.4 / 11 M, K = 150: 168 / 174 and 165 / 168.)
+        const bool in_turn = FUSED || (RAGGED && PART) ? SLICE >= 5 : !GATHER && a.in_turn;
         const int turn = in_turn ? NW : 1;
         const int nb = (end - begin + 63) >> 6;
         // (the division runs on the vector unit; the results are uniform and go back to scalar
@@ -696,11 +698,11 @@ void sddmm_tile_kernel(const TileArgs a)
             // scaled and added; 3.93e-8 / 4.10e-8 so; with plain sums 4.20e-8 / 4.28e-8.)
             if constexpr (!PART) {
                 pend_v = RESIDUAL ? v - (h.x + h.y) : (h.x + h.y) * v;
-            } else if constexpr (SLICE == 1) {
+            } else if constexpr (FIRST) {
                 pend_v = h.x + h.y;
             } else {
                 const Halves sum = add_to(m.old, h, (l & (XORDER ? G / 2 : 1)) != 0);
-                if constexpr (SLICE == 2) pend_v = sum.x + sum.y;
+                if constexpr (BETWEEN) pend_v = sum.x + sum.y;
                 else {
                     pend_v = RESIDUAL ? (v - (h.x + h.y)) - m.old : VMODE == 2 ? sum.x + sum.y : fmaf(sum.x, v, sum.y * v);
                     if constexpr (FUSED) pend_v = last_slice ? pend_v : sum.x + sum.y;
@@ -818,10 +820,13 @@ TileFn ragged_tile_kernel(const TileVariant &v, bool gather, int slice, int nwav
         if constexpr (VMODE == 2) {
             if (slice == 1) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 1, 0, true>;
             if (slice == 2) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 2, 0, true>;
+            if (slice == 6) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 6, 0, true>;
+            if (slice == 7) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 7, 0, true>;
         }
         if (slice == 3) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 3, 0, true>;
         if (slice == 5) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 5, 0, true>;
         if (slice == 4) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 4, 0, true>;
+        if (slice == 8) return (TileFn)sddmm_tile_kernel<8, 4, VMODE, 12, false, 8, 0, true>;
     }
     return nullptr;
 }

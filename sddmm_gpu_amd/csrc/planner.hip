@@ -152,9 +152,10 @@ int resolve_functions(Launch &L)
             L.tfn = L.tfns[0][0];
             return SDDMM_OK;
         }
+        constexpr int kInTurn[5] = {0, 6, 7, 5, 8};  // (the slices of other ranks, and one launch over all of K, read in_turn)
         for (int vm = 0; vm < 5; ++vm)
             for (int ac = 0; ac < 5; ++ac) {
-                L.tfns[vm][ac] = tile_kernel(tv, vm, L.fn_gather != 0, ac == 3 && L.ta.in_turn ? 5 : ac, L.fn_nwaves, L.fn_ragged != 0);
+                L.tfns[vm][ac] = tile_kernel(tv, vm, L.fn_gather != 0, L.ta.in_turn && (ac == 3 || L.fn_ragged) ? kInTurn[ac] : ac, L.fn_nwaves, L.fn_ragged != 0);
                 if (!L.tfns[vm][ac] && ac == 3) { L.fused_slices = 0; continue; }  // (that form exists for some variants only)
                 if (!L.tfns[vm][ac] && ac > 0 && L.fn_ragged && L.k_slice >= L.ta.K) continue;  // (one launch: no sliced forms needed)
                 if (!L.tfns[vm][ac]) return fail(SDDMM_ERR_ARG, "plan: no tile kernel for lanes %d x %d", tv.G, tv.KPL);
