@@ -997,17 +997,18 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
             // 260 measured plans show gains and next to no losses (us before and so):
             // (rows of H of other ranks than 16 and multiples of 32 lie across lines: the row gather's time by lines)
             const bool across = K % 32 != 0 && K != 16;
-            const bool open = (opt.spmm_stream <= 0 && choice.split == Split::all_tiled && nnz < 1500000) ||
+            const bool open = (opt.spmm_stream <= 0 && choice.split == Split::all_tiled && nnz < 1500000 && K <= 512) ||
                               (choice.split == Split::all_gathered && across && K <= kt) || (opt.spmm_stream <= 0 && choice.split != Split::all_gathered && K > kt && opt.fuse_slices <= 0);
             if (open && opt.k_slice <= 0 && opt.tile_lanes <= 0 && tile_x == 0 && (kt == 32 || kt == 64 || kt == 128) && nnz > 0) {
                 double run_length = 0;
                 const double tiled = tile_slices_us(c, ne, kt, &run_length);
                 // small matrices, and on tiles of which a few hold most (bands of 0.2 / 0.4 M, K = 96 / 50 15.5 / 17.9 and 7.8 / 9.5;
-                // R-MAT of 0.75 M, K = 96 40 and 23; ratings of 0.17 / 0.35 M, K = 96 / 32 8.0 / 6.6 and 6.1 / 5.3); not behind
-                // a product, which walks the pattern with its cut rows kept only beside a tile launch
+                // R-MAT of 0.75 M, K = 96 40 and 23; ratings of 0.17 / 0.35 M, K = 96 / 32 8.0 / 6.6 and 6.1 / 5.3); not beyond
+                // the ranks they were measured at (band of 0.2 M, K = 896 / 2048: 50 / 109 and 75 / 197), and not behind a
+                // product, which walks the pattern with its cut rows kept only beside a tile launch
                 const double h_all = (double)n_cols * K * 4, lines = nnz * ((4.0 * K - 4) / 128 + 1) * 128;
                 const double gathered = across ? 4.5 + 1e-6 * lines / (h_all <= 4.2e6 ? 22.0 : h_all <= 64.0e6 ? 13.8 : 9.6) : choice.gather_us;
-                if (opt.spmm_stream <= 0 && choice.split == Split::all_tiled && nnz < 1500000 && tiled > (nnz < 500000 ? 1.0 : 1.2) * gathered) choice.split = Split::all_gathered;
+                if (opt.spmm_stream <= 0 && choice.split == Split::all_tiled && nnz < 1500000 && K <= 512 && tiled > (nnz < 500000 ? 1.0 : 1.2) * gathered) choice.split = Split::all_gathered;
                 // such ranks, gathered (K = 11, ratings of 4.9 / 16 M, word counts of 9.6 M 38 / 107 / 67 and 21 / 51 / 34)
                 else if (choice.split == Split::all_gathered && across && K <= kt && tiled < 0.62 * gathered) choice.split = Split::all_tiled;
                 // runs of less than 4 in wide matrices: thinner slices have wider tiles (uniform, 4.7 M of 40,000 columns, K = 256: 388 and

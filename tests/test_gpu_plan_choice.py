@@ -12,6 +12,7 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("kind,sizes,K,kernel,k_slice", [
     ("banded", (4000, 60, 400), 96, capi.KERNEL_ROW_GATHER, 96),         # a few tiles hold most
     ("banded", (4000, 60, 400), 100, capi.KERNEL_ROW_GATHER, 100),
+    ("banded", (4000, 60, 400), 1024, capi.KERNEL_LDS_TILE, 128),        # beyond the ranks that was measured at
     ("bag_of_words", (3000, 20000, 900), 11, capi.KERNEL_LDS_TILE, 11),  # 44-byte rows of H
     ("uniform_random", (16598, 15299, 0.0091), 96, capi.KERNEL_LDS_TILE, 96),  # runs of one and two: no slices of the planner's own up to K = 128
     ("uniform_random", (30281, 34347, 0.0063), 128, capi.KERNEL_LDS_TILE, 128),
