@@ -75,7 +75,7 @@ typedef struct sddmm_plan_info {
     int32_t K;
     int32_t tile_size_x;  /* columns of S (= rows of H) per LDS tile actually used */
     int32_t tile_size_y;  /* row-panel height actually used */
-    int32_t k_slice;      /* K elements of each H row resident in LDS at a time (== K: no slicing) */
+    int32_t k_slice;      /* K elements of each H row a launch works on at a time (== K: no slicing) */
     int32_t n_col_tiles, n_row_panels; /* (n_row_panels: row panels of the stream; with tile_runs = 2 the
                                           row ranges, one per group of workgroups) */
     int32_t kernel;       /* SDDMM_KERNEL_* actually chosen (HYBRID: more than one launch) */

@@ -1109,7 +1109,12 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         if (int rc = c.need_row_ptr()) return rc;
     if (!P->launches.empty() && I.grid == 0) { I.grid = P->launches[0].grid; I.block = P->launches[0].block; I.lds_bytes = P->launches[0].lds; }
     I.n_launches = 0;
-    for (const Launch &L : P->launches) I.n_launches += (L.k_slice > 0 && L.k_slice < K && !L.fused_slices) ? (K + L.k_slice - 1) / L.k_slice : 1;
+    for (const Launch &L : P->launches) {
+        I.n_launches += (L.k_slice > 0 && L.k_slice < K && !L.fused_slices) ? (K + L.k_slice - 1) / L.k_slice : 1;
+        // (the slices of a gathered class keep partial results in the plan as those of a tiled one do, and callers go by
+        // k_slice < K for what may overlap)
+        if (L.tfn && L.k_slice > 0) I.k_slice = std::min(I.k_slice, L.k_slice);
+    }
     I.device_bytes = c.dev_bytes;
     assign_workspace(P);
     I.plan_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();

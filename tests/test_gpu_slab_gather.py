@@ -45,3 +45,19 @@ def test_against_64_bits(n_rows, n_cols, nnz, K, fuse, sink, slab):
     plan.set_values(dv.data_ptr(), stream)
     check(lambda: plan.execute(0, *a, stream), v * dot, v * size)
     check(lambda: plan.execute_epilogue(0, *a, capi.EPILOGUE_RESIDUAL, stream), v - dot, v + size)
+
+
+# the K slices of a gathered class keep partial results in the plan like those of tiles: k_slice < K says so to its callers
+@pytest.mark.parametrize("opts,kernel,launches", [(dict(fuse_slices=0), capi.KERNEL_AUTO, 3), (dict(fuse_slices=1), capi.KERNEL_AUTO, 1),
+                                                  (dict(fuse_slices=0, row_padded=1), capi.KERNEL_ROW_GATHER, 3)])
+def test_slices_are_reported(opts, kernel, launches):
+    n, K = 200000, 384  # (factors of 307 MB: slabs)
+    g = torch.Generator().manual_seed(5)
+    cols = torch.randint(0, n // 2, (n, 2), generator=g)
+    cols[:, 1] += n // 2
+    rp, ci = torch.arange(0, 2 * n + 1, 2).int().cuda(), cols.reshape(-1).int().cuda()
+    plan = capi.Plan.from_device_csr(n, n, 2 * n, rp.data_ptr(), ci.data_ptr(), K,
+                                     options=capi.PlanOptions.defaults(kernel=kernel, short_row_max=1 << 20, ignore_env=1, **opts))
+    info = plan.info()
+    assert info["kernel"] == capi.KERNEL_ROW_GATHER and info["n_launches"] == launches and info["k_slice"] == 128, info
+    assert plan.workspace_bytes() >= 4 * info["padded_positions"] >= 8 * n
