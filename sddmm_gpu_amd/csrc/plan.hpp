@@ -179,23 +179,30 @@ inline bool ragged_product_tiles(int64_t nnz, int32_t K, int ks)
     return nnz < 4000000 ? K > 256 && !product_walks(nnz, K, ks) : K > 32 && (K <= 128 || K * 100 >= padded * 72);
 }
 // The runs it takes for that, in nonzeros per run on average: a run costs a partial row of the padded width, its nonzeros cost
-// the walk K elements each.  So the line is one of run length times the used share of the width.  Product alone, us, walk and
-// tiles at (that figure):
-//   width 64: word counts of 9.4 M, K = 50 / 60 120 / 121 (12.3), 131 / 124 (14.8); uniform, 5.9 M, K = 50 79 / 69 (14.3); up to
-//       K = 48, whose rows are few lines each to the walk, 8.9 M of 40,000 columns, K = 40 / 48 111 / 129 (15.0), 113 / 130 (18.0),
-//       uniform, 11.7 M, K = 40 127 / 94 (19.1); with an H of less than 2.5 MB, word counts of 7.4 M, K = 48 82 / 92 (14.4), of 11 M,
-//       K = 40 / 44 116 / 108 (15.4), 126 / 108 (16.9)
-//   width 128: word counts of 5.3 M, K = 100 / 120 129 / 178 (7.6), 144 / 180 (9.1), 11 M, K = 100 / 120 227 / 275 (9.8), 254 / 277 (11.7),
-//       11.7 M, K = 72 / 100 203 / 203 (12.9), 258 / 205 (18); uniform, 11.7 M, K = 72 / 100 225 / 245 (8.5), 385 / 245 (11.9).  With
-//       an H of less than 2.5 MB, ratings of 4.9 and 6.3 M and word counts of 5.9 M, K = 72 101 / 92 (9.7), 123 / 103 (11.3), 112 / 103 (10.5)
-//   two slices: word counts of 11 M, K = 200 / 250 448 / 553 (9.8), 629 / 560 (12.2), 5.3 M 335 / 370 (9.5); ratings, 4.9 M, 193 / 181 (13.5)
-//   more: word counts of 9.4, 5.3 and 11 M, K = 300 905 / 1100 (6.3), 553 / 547 (7.6), 1028 / 835 (9.8); uniform, 11.7 M 1879 / 1152
-//       (7.1); below 4 M nonzeros, ratings of 3.4 M, K = 290 / 370 286 / 300 (7.5), 313 / 322 (9.5), of 2.4 M 204 / 194 (10.2)
+// the walk K elements each.  So the line is one of run length times the used share of the width.  It is drawn on SDDMM + product
+// one after the other: a product alone finds its partial rows in the caches, behind an SDDMM it does not (ratings of 4.9 M, K = 187:
+// 184 / 172 alone and 302 / 336 together).  us, walk and tiles at (that figure):
+//   width 64: uniform, 5.4 / 9.0 M, K = 55 100 / 89 (14.9), 155 / 138 (17.0), 11.4 M 252 / 198 (13.7); up to K = 48, whose rows are few
+//       lines each to the walk, ratings of 5.1 M, K = 34 88 / 82 (18.1), and, product alone, with an H of more than 2.5 MB word counts of
+//       8.9 M, K = 40 / 48 111 / 129 (15.0), 113 / 130 (18.0), with a smaller one of 7.4 M, K = 48 82 / 92 (14.4)
+//   width 128: ratings of 4.5 / 5.6 / 7.3 M, K = 84 / 75 / 78 140 / 137 (10.7), 168 / 158 (10.6), 199 / 192 (12.5); of 8.2 / 11.8 / 12.3 M, K =
+//       69 / 75 / 90 216 / 234 (9.5), 307 / 325 (12.5), 323 / 343 (14.8), 8.7 M, K = 89 235 / 227 (15.6); an H of more than 4.5 MB, word
+//       counts of 6.1 / 4.4 M, K = 125 / 124 282 / 230 (11.9), 172 / 141 (13.2), 7.5 / 9.7 M, K = 110 / 92 360 / 359 (14.1), 388 / 408
+//   two slices: ratings of 4.9 M, K = 195 / 200 303 / 315 (14.4), 299 / 298 (15.1), 5.9 M, K = 208 362 / 341 (16.8); uniform, 4.4 M, K = 189
+//       222 / 257 (11.3); an H of more than 6 MB, word counts of 19 M, K = 238 2441 / 1634 (11.5), 5.5 M, K = 252 664 / 539 (12.8)
+//   more: word counts of 4.1 / 12.8 M, K = 337 / 518 737 / 775 (7.3), 4600 / 3341 (7.3); below 4 M nonzeros, ratings of 2.9 M, K = 286
+//       338 / 324 (10.1), 2.2 M, K = 352 / 357 259 / 265 (11.3), 275 / 266 (11.5), word counts of 3.0 M, K = 369 478 / 350 (10.9), and with
+//       four slices and an H of up to 11 MB ratings of 2.9 / 3.2 M, K = 418 / 488 384 / 434 (10.6), 473 / 512 (12.4), uniform, 3.8 M, K =
+//       496 428 / 472 (13.2), but H of 12.5 MB, 3.3 M, K = 450 630 / 409 (10.4)
 inline double ragged_product_run(int64_t nnz, int64_t n_cols, int32_t K, int ks)
 {
-    const double padded = (K + ks - 1) / ks * ks;
-    const bool small_h = 4.0 * n_cols * K <= 2.5e6;
-    const double least = ks < 128 ? (K > 48 ? 13.5 : small_h ? 15.0 : 19.0) : K <= 128 ? (small_h ? 8.0 : 11.8) : K <= 256 ? 11.0 : nnz < 4000000 ? 10.0 : 7.0;
+    const double padded = (K + ks - 1) / ks * ks, h = 4.0 * n_cols * K;
+    double least;
+    if (ks < 128) least = K > 48 ? 13.5 : h <= 2.5e6 ? 15.0 : 19.0;
+    else if (K <= 128) least = nnz < 7500000 ? (h <= 4.5e6 ? 10.5 : 11.8) : h <= 4.5e6 ? 15.0 : 14.0;
+    else if (K <= 256) least = h <= 6.0e6 ? 15.5 : 11.0;
+    else if (nnz < 4000000) least = K > 384 && h <= 11.0e6 ? 16.0 : 10.0;
+    else least = nnz < 6000000 ? 9.0 : 7.0;
     return least * padded / K;
 }
 // planner_tile.hip: the rows' nonzeros in tile order (tiles of x columns), every (row, tile) run padded

@@ -751,6 +751,13 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
             const double h_part = local ? std::min(1.0, 2e6 / (double)L.nnz) : 1.0;
             if (want_spmm && uneven && c.nnz == c.P->info.nnz &&
                 (busiest * c.cus * 2 >= total * 7 || h_part * c.n_cols * c.K * c.K * std::sqrt((double)c.K) <= 6.4e9)) { want_spmm = false; sp_csr = true; }
+            // At a rank without a tile width of its own, up to K = 64: few runs in an item are few bundles for a wave, which then
+            // waits for the longest of them.  Word counts, whose H of some MB makes many tiles for few rows, SDDMM + product, us, walk
+            // and tiles at runs per item (run length times used share): 4.7 M, K = 59 114 / 138 at 529 (20), 5.2 M, K = 62 122 / 138 at
+            // 668 (20), 7.5 M, K = 58 211 / 230 at 575 (15), 9.0 M, K = 53 192 / 194 at 771 (19); 7.3 M, K = 53 144 / 143 at 1163 (17), 8.7 M,
+            // K = 51 175 / 139 at 660 (26), 16.1 M, K = 55 371 / 289 at 755 (18); where rows touch few tiles, band of 5.5 M, K = 54, 197 / 151.
+            if (want_spmm && ragged && ks < 128 && !local && c.nnz == c.P->info.nnz && c.nnz < 10000000 && (int64_t)c.n_cols * c.K * 4 > 2500000 &&
+                sp_seg < 800 * (int64_t)item_keys.size() && sp_nnz * c.K < 24 * (int64_t)ks * sp_seg) { want_spmm = false; sp_csr = true; }
             if (want_spmm && !panel_local && item_keys.size() == items_whole) build_spmm(item_keys);
         } else if (want_spmm && rb == 0 && rows.size() <= (size_t)panel_rows) {
             // (equal position ranges for the SDDMM: the product takes one item per column tile)

@@ -87,9 +87,18 @@ def test_sddmm_as_without_the_product(tmp_path, K):
     ("bag_of_words", (20000, 17000, 480), 300, capi.SPMM_WALK),
     ("bag_of_words", (8000, 17000, 1500), 100, capi.SPMM_TILES),
     ("uniform_random", (20000, 12000, 0.05), 300, capi.SPMM_TILES),
+    # (and where SDDMM + product, one after the other, gain by the tiles)
+    ("bag_of_words", (3545, 33207, 1354), 59, capi.SPMM_WALK),  # few runs in an item
+    ("bag_of_words", (6074, 42148, 2706), 55, capi.SPMM_TILES),
+    ("recommender", (54211, 5638), 117, capi.SPMM_TILES),
+    ("recommender", (96122, 7724), 75, capi.SPMM_WALK),
+    ("recommender", (46295, 5912), 187, capi.SPMM_WALK),
+    ("uniform_random", (35484, 2456, 0.0524), 189, capi.SPMM_WALK),
+    ("recommender", (38596, 4965), 437, capi.SPMM_WALK),
+    ("uniform_random", (8615, 6969, 0.0569), 450, capi.SPMM_TILES),
 ])
 def test_form_by_the_length_of_runs(tmp_path, kind, sizes, K, form):
-    d = getattr(synth, kind)(*sizes, K=4, device=DEV)
+    d = getattr(synth, kind)(*sizes, K=4, device=DEV, **(dict(max_deg=int(0.9 * sizes[1])) if kind == "recommender" else {}))
     plan = plan_of(d, K)
     assert plan.spmm_form() == form
     check(d, K, plan, tmp_path / "p.plan")
