@@ -984,7 +984,15 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
         if (model_fits && tiled_product && !long_class && (ragged || K <= kt)) c.sp_walk = true;
         if (model_fits && tiled_product && !ragged && kt <= 64 && (long_class || K <= kt)) {
             const SplitChoice choice = estimate_split(c, ne, kt, x, g_long, short_max, 1e30);
-            if (choice.split == Split::all_tiled && (long_class || tile_slices_us(c, ne, kt) < choice.gather_us)) tile_all();
+            // Where many nonzeros lie in short rows their runs are short as well, and columns that are used unevenly are gathered
+            // faster than the model has it: only where it finds a clear gain (SDDMM + product, us, by length and all tiled at its
+            // ratio: R-MAT of 22 M, K = 32 507 / 747 (1.0), 23 M, K = 192 3307 / 3837 (0.9), 12.6 M, K = 320 3090 / 3488 (0.82), 4.8 M, K = 320
+            // 1125 / 1156 (0.67); uniform, 7.5 M, K = 32 190 / 148 (0.45), 23 M, K = 64 893 / 738 (0.51), 5.5 M, K = 32 94 / 83 (0.66))
+            auto gains = [&]() {
+                if (!long_class) return tile_slices_us(c, ne, kt) < choice.gather_us;
+                return nsh * 20 <= nnz * 3 || tile_slices_us(c, ne, kt) < 0.67 * (tile_slices_us(c, rl, kt) + choice.gather_us * (double)nsh / (double)nnz);
+            };
+            if (choice.split == Split::all_tiled && gains()) tile_all();
         }
         int64_t slab_cols = 0;  // chosen by the model
         if (by_model) {
