@@ -969,8 +969,12 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         if (L.grid != c.cus) return fail(SDDMM_ERR_ARG, "plan: matrix-core share on a launch of %d workgroups", L.grid);
     }
     L.k_slice = std::min(ks, c.K);
-    // (gather form: 2048 positions per workgroup, fewer where that would leave less than four workgroups per compute unit)
-    if (gather) L.grid = (int32_t)std::max<int64_t>({1, (np + 2047) / 2048, std::min<int64_t>(4 * (int64_t)c.cus, (np + 255) / 256)});
+    // (gather form: 2048 positions per workgroup, fewer where that would leave less than four workgroups per compute unit.  In column
+    // slabs 1024 up to 32 million positions: the workgroups in flight then lie in fewer slabs.  us, 2048 and 1024: uniform, 2.8 M
+    // nonzeros, K = 192 250 / 212, 18.7 M, K = 128 811 / 670, 5.9 M, K = 256 495 / 373, 9.4 M, K = 64 259 / 227; R-MAT of 3.7 M, K = 128
+    // 134 / 127, 6.6 M, K = 384 619 / 610, 19.6 M, K = 64 462 / 467, but 185 M 4415 / 4509)
+    const int64_t per_group = c.opt.gather_slab_cols > 0 && np < (int64_t)1 << 25 ? 1024 : 2048;
+    if (gather) L.grid = (int32_t)std::max<int64_t>({1, (np + per_group - 1) / per_group, std::min<int64_t>(4 * (int64_t)c.cus, (np + 255) / 256)});
     if (int rc = resolve_functions(L)) return rc;
     if (I) {
         I->tile_size_x = x; I->tile_size_y = grid2d ? (int32_t)std::min<int64_t>(block_rows_max, INT32_MAX) : panel_rows; I->n_col_tiles = n_tiles_all;

@@ -131,3 +131,13 @@ def test_dense_core_that_was_asked_for(opts, core):
     d = synth.recommender(44000, 5600, K=4, seed=5, device=DEV, max_deg=5000)
     plan = plan_of(d, 512, **opts)
     assert (plan.info()["dense_blocks"] > 0) == core and plan.spmm_form() == (capi.SPMM_CSR if core else capi.SPMM_TILES)
+
+
+# columns that are used unevenly: the short rows, most of the nonzeros, are gathered beside the tiled ones, and the product keeps the walk
+@pytest.mark.parametrize("scale,edges,K", [(17, 9369749, 32), (18, 14678406, 192)])
+def test_rows_stay_split(tmp_path, scale, edges, K):
+    d = synth.rmat(scale, edges, K=4, device=DEV)
+    plan = plan_of(d, K)
+    long_rows, _, short_rows = plan.info()["class_nnz"]
+    assert long_rows > 0 and short_rows > 0 and plan.spmm_form() == capi.SPMM_WALK
+    check(d, K, plan, tmp_path / "p.plan")
