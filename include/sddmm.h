@@ -415,8 +415,9 @@ int sddmm_execute_ws(const sddmm_plan *plan, const float *d_val, const float *d_
  * H rows as sddmm_spmm_csr does.  Where the runs are short (fewer than 8 entries, 5
  * from K = 129 on, 12 while H is about as large as a die's L2), on small matrices (fewer than 4 M nonzeros
  * and 4.5e8 or 7e8 nonzeros times K, H as above), at ranks without a tile width of their
- * own below 4 M nonzeros (up to K = 256) or where more than a quarter of the rank rounded up
- * would be padding, and where a few workgroups would hold most of the work, the whole product
+ * own up to K = 32, below 4 M nonzeros (up to K = 256), where more than 28 % of the rank rounded up
+ * would be padding (from K = 129 on) or the runs are short for the share that is not, where the
+ * rows long enough for the tiles are few, and where a few workgroups would hold most of the work, the whole product
  * goes over the CSR pattern as sddmm_spmm_csr does it, with the parts of its cut rows
  * written down and added up in order; and a plan on row blocks multiplies its tiles
  * on the matrix cores (weights of any size at the same speed; where 32 rows meet values of
@@ -426,8 +427,8 @@ int sddmm_execute_ws(const sddmm_plan *plan, const float *d_val, const float *d_
  * No atomics: the same bits on every call.  The
  * partial rows (K floats per run; sddmm_plan_info.spmm_runs) live in the plan, so
  * calls on one plan must not overlap in time, or in d_workspace (NULL, or as for
- * sddmm_execute_ws): calls with a workspace each may.  Other plans (and H or Y not
- * 16-byte aligned) take the sddmm_spmm_csr path on the plan's pattern.  d_x: nnz
+ * sddmm_execute_ws): calls with a workspace each may.  Other plans (and, at ranks with a tile width of their own, H or Y
+ * not 16-byte aligned) take the sddmm_spmm_csr path on the plan's pattern.  d_x: nnz
  * fp32 in sorted order, e.g. the output of sddmm_execute_softmax.            */
 int sddmm_execute_softmax(const sddmm_plan *plan, const float *d_val, const float *d_W, const float *d_H,
                           float *d_out, void *stream);
@@ -470,7 +471,7 @@ int sddmm_execute_profiled(const sddmm_plan *plan, const float *d_val, const flo
  * the quantity the reference prints at sddmm.cu:109-114.  The device copies of W,
  * H and the result stay with the plan after its first call (counted in
  * sddmm_plan_info.device_bytes), and with the first such call on a device 16 MiB
- * of pinned host memory, two streams and up to seven threads, which all plans
+ * of pinned host memory, three streams and up to seven threads, which all plans
  * share; sddmm_plan_release_host gives the plan's arrays and its share in the
  * rest back (the next call makes them anew), as sddmm_plan_destroy does.  Calls
  * from several threads take turns.  The kernels of a call are an sddmm_execute of

@@ -13,9 +13,10 @@ namespace {
 // that do not): on R-MAT 2^22, K = 64, 43 % of 60 GB of rows cross the fabric.
 // us per product, with four lanes and so: R-MAT 2^22, 185 million nonzeros, K = 64 4896 and 4541; 2^20, K = 64 (28 million) 645 and
 // 590, K = 128 (70 million) 2800 and 2741, K = 512 (33 million) 6457 and 6280; 2^18, 12 million, K = 128 466 and 446; uniform, 20
-// million of 100,000 columns, K = 64 / 128 419 / 713 and 375 / 703.  2048 positions a workgroup (chosen by the planner): 1024 /
-// 4096 / 8192 / 16384 on the first 4509 / 4419 / 4506 / 4763 where 2048 takes 4415; neighbouring workgroups bound to one die,
-// 4 to 1024 at a time: 4398 to 4453; four steps' pieces at a time instead of eight: the same.
+// million of 100,000 columns, K = 64 / 128 419 / 713 and 375 / 703 (all with 2048 positions a workgroup, which the planner chooses
+// from 32 million on; below it takes 1024, see there): 1024 / 4096 / 8192 / 16384 on the first 4509 / 4419 / 4506 / 4763 where 2048
+// takes 4415; neighbouring workgroups bound to one die, 4 to 1024 at a time: 4398 to 4453; four steps' pieces at a time instead of
+// eight: the same.
 // VMODE, SLICE: as in the tile kernel.  (SLICE 3, all K slices inside one launch: a wave's partial results are its own.)
 template <int KPL, int VMODE, int SLICE>
 __global__ __launch_bounds__(256)
