@@ -61,7 +61,9 @@ public:
     hipStream_t stream[kStreams] = {};  // (a thread's pieces all travel on one of them)
     hipEvent_t fork = nullptr, join[kStreams] = {}, e0 = nullptr, e1 = nullptr;
     std::mutex busy;  // held by a call from its first piece to its last
-    int used = kStreams;  // streams of the call that holds it: one for less than 2 MB, whose events would cost more than they hide
+    // Streams of the call that holds it: small calls wait for more events than the streams hide.  us a call, one / two / three: 0.9 MB
+    // 112 / 123 / 134, 1.3 MB 126 / 134 / 139, 2.4 MB 186 / 175 / 180, 3.5 MB 225 / 204 / 208, 5.2 MB 290 / 254 / 247, 14.7 MB 581 / 487 / 472.
+    int used = kStreams;
 
     // the pipe of `device` (the current one), made if no plan holds it
     static std::shared_ptr<HostPipe> get(int device)
@@ -269,7 +271,8 @@ int host_call(const sddmm_plan *plan, HostCall &c, const float *h_W, const float
     HostPipe &pipe = *c.pipe;
     // after whatever the caller has put on the default stream before
     HIP_TRY(hipEventRecord(pipe.fork, nullptr));
-    pipe.used = 4 * (I.n_rows * (int64_t)I.K + I.n_cols * (int64_t)I.K + I.nnz) < ((int64_t)2 << 20) ? 1 : HostPipe::kStreams;
+    const int64_t bytes = 4 * (I.n_rows * (int64_t)I.K + I.n_cols * (int64_t)I.K + I.nnz);
+    pipe.used = bytes < ((int64_t)2 << 20) ? 1 : bytes < ((int64_t)4 << 20) ? 2 : HostPipe::kStreams;
     for (int i = 0; i < pipe.used; ++i) HIP_TRY(hipStreamWaitEvent(pipe.stream[i], pipe.fork, 0));
     const HostPipe::Part in[2] = {{(const char *)h_W, (char *)c.W, (size_t)I.n_rows * I.K * 4}, {(const char *)h_H, (char *)c.H, (size_t)I.n_cols * I.K * 4}};
     HIP_TRY(pipe.move(in, 2, true));

@@ -28,7 +28,7 @@ def expected(plan, W, H, nnz):
     return out.cpu().numpy()
 
 
-@pytest.mark.parametrize("n_rows,n_cols,nnz,K", [(1, 1, 1, 1), (3, 5, 7, 5), (257, 256, 65536, 32), (5000, 3001, 1_500_001, 64),
+@pytest.mark.parametrize("n_rows,n_cols,nnz,K", [(1, 1, 1, 1), (3, 5, 7, 5), (257, 256, 65536, 32), (4001, 1999, 300_001, 64), (5000, 3001, 1_500_001, 64),
                                                  (40001, 999, 3_000_003, 50)])
 def test_transfers_of_all_sizes(n_rows, n_cols, nnz, K):
     plan, W, H = make(n_rows, n_cols, nnz, K, nnz)
