@@ -26,7 +26,7 @@ namespace {
 // what bounds it until the entries do (the recommender pattern moves 0.8 GB at 3.5 TB/s).  Before this a kernel of its own
 // laid chunks of whole rows out, and rows that had been left over went through lists to a third one.  us, before and now: 18
 // thousand entries 11.8 and 8.9; R-MAT, 1.9 million 34 and 18, 28 million 134 and 111, 84 million 297 and 266, 189 million
-// 526 and 526; word counts, 0.7 million 18.5 and 16.5; window of 320 a row, 5.2 million 24 and 19; 3 million rows of one
+// 526 and 526; window of 320 a row, 5.2 million 24 and 19; 3 million rows of one
 // entry 38 and 30; 20 thousand entries spread over 4 million rows 93 and 25; a row of 30 million 328 and 93; recommender,
 // 100 million 235 and 231.  (Maximum and sum by scans over the entries, whatever the rows: 1072 there, bound by the vector
 // ALU.)
@@ -52,14 +52,20 @@ struct SoftmaxScale {
     __host__ __device__ int piece() const { return unit() < kSmPieceMax ? unit() : kSmPieceMax; }
     __host__ __device__ int64_t pieces() const { return (total + piece() - 1) / piece(); }
 };
-// Shares: as large as leaves 4096 of them, 64 to kSmShareMax.
+// Shares: from 2^21 on the scale as large as leaves 4096 of them, up to kSmShareMax; below as small as makes no more than
+// 4096, which is what runs at a time, not below 64: what a share costs whatever it holds, a search and the row pointers, is
+// most of the time there, and a second turn of workgroups pays for it again.  us of the kernel alone with 4096 shares at
+// least and at most: rows of 14, 0.23 million entries 9.8 and 6.0; of 900, 0.9 million 11.4 and 7.4; of 40, 1.2 million 10.0
+// and 7.9; R-MAT, 0.24 / 0.69 / 1.3 million 10.7 / 14.5 / 15.0 and 9.2 / 10.4 / 14.3, but 1.86 million (2.4 on the scale) 15.5
+// and 18.2.
 __host__ __device__ inline SoftmaxScale softmax_scale(int64_t nnz, int64_t n_rows)
 {
     SoftmaxScale s;
     s.row = n_rows <= (int64_t)1 << 27 ? kSmRow : 1;
     s.total = nnz + s.row * n_rows;
-    s.share = kSmShareMax;
-    while (s.share > 64 && s.total < (int64_t)4096 * s.share) s.share /= 2;
+    s.share = 64;
+    while (s.share < 512 && s.total > (int64_t)4096 * s.share) s.share *= 2;
+    while (s.share < kSmShareMax && s.total >= (int64_t)4096 * 2 * s.share) s.share *= 2;
     return s;
 }
 
@@ -199,13 +205,14 @@ __device__ __forceinline__ void softmax_long_row(const float *x, float *out, int
     // (the next row writes its maxima after this row's second barrier and its sums after its own first: no barrier needed here)
 }
 
-// 64 rows by a wave: the lane's one has len entries from rb on (0: none, or not to be done here; at most kSmByWave).
-__device__ __forceinline__ void softmax_row_batch(const float *x, float *out, int rb, int len, int lane)
+// 64 rows by a wave: the lane's one has len entries from rb on (0: none, or not to be done here; at most kSmByWave), and
+// rows of up to by_lane entries have a lane each.
+__device__ __forceinline__ void softmax_row_batch(const float *x, float *out, int rb, int len, int lane, int by_lane)
 {
     // a lane per row
-    if (__ballot(len >= 1 && len <= kSmByLane)) softmax_row_by_group<1, kSmByLane>(x + rb, out + rb, len, len <= kSmByLane);
+    if (__ballot(len >= 1 && len <= by_lane)) softmax_row_by_group<1, kSmByLane>(x + rb, out + rb, len, len <= by_lane);
     // groups of 8 lanes: eight rows at a time
-    uint64_t todo = __ballot(len > kSmByLane && len <= kSmBy8);
+    uint64_t todo = __ballot(len > by_lane && len <= kSmBy8);
     while (todo) {
         int src = -1;  // the lane that holds the row of this lane's group
 #pragma unroll
@@ -264,40 +271,48 @@ void sddmm_row_softmax_kernel(const int32_t *__restrict__ row_ptr, int64_t n_row
                               int2 *__restrict__ rec_rows)
 {
     __shared__ float red[2 * kSmWaves];
-    __shared__ int left[kSmWaves * kSmLeft];  // rows that the waves leave to the workgroup
-    __shared__ int n_left, first_row;   // first_row: the row at the unit's beginning
+    // rows that the waves leave to the workgroup: row, first entry, length (read once more from the row pointers, and the row
+    // that began before the unit looked up there by all, they cost units without any such row 3 us)
+    __shared__ int3 left[kSmWaves * kSmLeft + 1];
+    __shared__ int n_left;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n_rows = (int)n_rows_, nnz = row_ptr[n_rows];
     const SoftmaxScale scale = softmax_scale(nnz, n_rows);
     const int64_t unit = scale.unit(), n_units = scale.units(), piece = scale.piece();
+    // (a share of 64 starts sixteen rows at most: two passes of groups of 8, and another kind of pass before them is one more
+    // chain of loads and sums.  18 thousand entries in 4096 rows, R-MAT: 6.4 us and 5.9; where sixteen rows or fewer are at
+    // hand in larger shares, 3.5 million: 20.9 and 22.5)
+    const int by_lane = scale.share == 64 ? 0 : kSmByLane;
     const bool vec_in = (reinterpret_cast<uintptr_t>(x) & 15u) == 0, vec_out = (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
     for (int64_t u = blockIdx.x; u < n_units; u += gridDim.x) {
         const int64_t k0 = u * unit, k1 = min(scale.total, k0 + unit);
+        if (u != blockIdx.x) __syncthreads();  // (left has been read)
         if (threadIdx.x == 0) n_left = 0;
         if (threadIdx.x * piece < k1 - k0) rec_rows[k0 / piece + threadIdx.x] = make_int2(0, 0);
         __syncthreads();
         const int64_t s0 = k0 + wave * scale.share, s1 = min(k1, s0 + scale.share);
         if (s0 < s1) {
             const int r0 = softmax_row_at(row_ptr, n_rows, scale.row, s0, lane);
-            if (threadIdx.x == 0) first_row = r0;
             for (int64_t w0 = r0;; w0 += 64) {
                 const int64_t r = w0 + lane;
                 const int rb = row_ptr[min(r, (int64_t)n_rows)], re = row_ptr[min(r + 1, (int64_t)n_rows)];
                 const int64_t at = rb + scale.row * r;
                 const int len = at >= s0 && at < s1 ? re - rb : 0;  // (r0 may begin before the share)
-                if (len > kSmByWave) left[atomicAdd(&n_left, 1)] = (int)r;
-                softmax_row_batch(x, out, rb, len > kSmByWave ? 0 : len, lane);
+                // (and the row that began before the unit, if it is a huge one that goes on in it)
+                const bool goes_on = wave == 0 && at < k0 && re - rb > kSmLongMax && at + (re - rb) > k0;
+                if (len > kSmByWave || goes_on) left[atomicAdd(&n_left, 1)] = make_int3((int)r, rb, re - rb);
+                softmax_row_batch(x, out, rb, len > kSmByWave ? 0 : len, lane, by_lane);
                 if (__ballot(r >= n_rows || at >= s1)) break;
             }
         }
         __syncthreads();
         const int n = n_left;
 #pragma unroll 1
-        for (int w = -1; w < n; ++w) {  // (-1: the row that began before the unit, if it is a huge one)
-            const int r = w < 0 ? first_row : left[w];
-            const int64_t b = row_ptr[r], len = row_ptr[r + 1] - b, at = b + (int64_t)scale.row * r;
+        for (int w = 0; w < n; ++w) {
+            const int3 l = left[w];
+            const int r = l.x;
+            const int64_t b = l.y, len = l.z, at = b + (int64_t)scale.row * r;
             const bool huge = len > kSmLongMax;
-            if (w < 0 && (at >= k0 || !huge || at + len <= k0)) continue;
             if (len <= 4 * 4 * kSmBlock - 8) {
                 softmax_long_row<4>(x, out, b, b + len, nnz, vec_in, vec_out, red, nullptr);
                 continue;
@@ -312,7 +327,6 @@ void sddmm_row_softmax_kernel(const int32_t *__restrict__ row_ptr, int64_t n_row
                 p = e;
             }
         }
-        __syncthreads();  // (the next unit writes left, n_left and first_row)
     }
 }
 

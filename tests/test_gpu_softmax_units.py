@@ -53,7 +53,7 @@ def test_special_values_stay_in_their_row(oracle, at, value):
         assert np.isnan(got[touched]).sum() >= 1
 
 
-# Pieces are 256 entries without filler rows and 1024 with them; a lane merges every 64th piece of a row.
+# Pieces are 256 entries without filler rows and 2048 with them; a lane merges every 64th piece of a row.
 @pytest.mark.parametrize("filler,masked", [(0, [(0, 700)]), (0, [(16384, 18000)]), (0, [(0, 19999)]), (0, [(500, 20000)]),
                                            (1200000, [(0, 5000)]), (1200000, [(0, 9000), (12000, 20000)])])
 def test_huge_row_with_pieces_all_masked(oracle, filler, masked):
