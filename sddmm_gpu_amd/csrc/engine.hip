@@ -235,7 +235,7 @@ int sddmm_execute_softmax(const sddmm_plan *plan, const float *d_val, const floa
         HIP_TRY(issue_launch(plan, L, d_val, d_W, d_H, d_out, (hipStream_t)stream, SDDMM_EPILOGUE_SCALE, nullptr, in_launch));
     if (in_launch) return SDDMM_OK;
     if (!plan->d_row_ptr) return fail(SDDMM_ERR_ARG, "sddmm_execute_softmax: the plan holds no row pointers");
-    return launch_row_softmax(plan->info.n_rows, plan->d_row_ptr, d_out, d_out, stream, nullptr, 0);
+    return launch_row_softmax(plan->info.n_rows, plan->d_row_ptr, d_out, d_out, stream, nullptr, 0, plan->launches[0].longest_row);
 }
 
 int sddmm_plan_workspace_bytes(const sddmm_plan *plan, int64_t *bytes)
@@ -265,7 +265,7 @@ int sddmm_execute_ws(const sddmm_plan *plan, const float *d_val, const float *d_
     for (const Launch &L : plan->launches) HIP_TRY(issue_launch(plan, L, d_val, d_W, d_H, d_out, (hipStream_t)stream, epilogue, ws, in_launch));
     if (!softmax || in_launch) return SDDMM_OK;
     if (!plan->d_row_ptr) return fail(SDDMM_ERR_ARG, "sddmm_execute_ws: the plan holds no row pointers");
-    return launch_row_softmax(plan->info.n_rows, plan->d_row_ptr, d_out, d_out, stream, ws + plan->ws_softmax, plan->info.nnz);
+    return launch_row_softmax(plan->info.n_rows, plan->d_row_ptr, d_out, d_out, stream, ws + plan->ws_softmax, plan->info.nnz, plan->launches[0].longest_row);
 }
 
 static const Launch *spmm_launch(const sddmm_plan *plan)

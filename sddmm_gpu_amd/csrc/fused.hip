@@ -431,7 +431,7 @@ int64_t row_softmax_workspace_bytes(int64_t nnz, int64_t n_rows)
     return ((softmax_scale(nnz, n_rows).pieces() * 24 + 255) / 256) * 256;  // two float2 and one int2 per piece
 }
 
-int launch_row_softmax(int64_t n_rows, const int32_t *d_row_ptr, const float *d_x, float *d_out, void *stream, void *d_ws, int64_t nnz)
+int launch_row_softmax(int64_t n_rows, const int32_t *d_row_ptr, const float *d_x, float *d_out, void *stream, void *d_ws, int64_t nnz, int64_t longest_row)
 {
     if (n_rows <= 0) return SDDMM_OK;
     float2 *rec = nullptr;
@@ -453,7 +453,7 @@ int launch_row_softmax(int64_t n_rows, const int32_t *d_row_ptr, const float *d_
     const int merge_groups = n_rows >= (int64_t)1 << 20 ? 4096 : 1024;
     const hipStream_t st = (hipStream_t)stream;
     hipError_t e = launch(sddmm_row_softmax_kernel, dim3(main_groups), dim3(kSmBlock), 0, st, d_row_ptr, n_rows, d_x, d_out, rec, rows);
-    if (e == hipSuccess) e = launch(sddmm_row_softmax_merge_kernel, dim3(merge_groups), dim3(kSmBlock), 0, st, d_row_ptr, n_rows, d_out, rec, rows);
+    if (e == hipSuccess && longest_row > kSmLongMax) e = launch(sddmm_row_softmax_merge_kernel, dim3(merge_groups), dim3(kSmBlock), 0, st, d_row_ptr, n_rows, d_out, rec, rows);
     if (e != hipSuccess) return fail(SDDMM_ERR_HIP, "sddmm_row_softmax: %s", hipGetErrorString(e));
     return SDDMM_OK;
 }
@@ -466,7 +466,7 @@ int sddmm_row_softmax(int64_t n_rows, const int32_t *d_row_ptr, const float *d_x
 {
     if (n_rows < 0 || (n_rows > 0 && (!d_row_ptr || !d_x || !d_out))) return fail(SDDMM_ERR_ARG, "sddmm_row_softmax: bad arguments");
     if (n_rows >= INT32_MAX) return fail(SDDMM_ERR_RANGE, "sddmm_row_softmax: more than 2^31 - 2 rows");
-    return launch_row_softmax(n_rows, d_row_ptr, d_x, d_out, stream, nullptr, 0);
+    return launch_row_softmax(n_rows, d_row_ptr, d_x, d_out, stream, nullptr, 0, INT64_MAX);
 }
 
 }  // extern "C"

@@ -91,8 +91,9 @@ void parallel_dynamic(int64_t n, int64_t chunk, const std::function<void(int64_t
 
 // out[p] = softmax over the entries of p's row of x (out may be x), on `stream` (a hipStream_t).  d_ws: device memory of
 // row_softmax_workspace_bytes(nnz, n_rows) bytes for the pass's records, nnz the number of entries (d_row_ptr[n_rows]); null: the
-// library's own per-device arrays, which calls that overlap in time would share.
-int launch_row_softmax(int64_t n_rows, const int32_t *d_row_ptr, const float *d_x, float *d_out, void *stream, void *d_ws, int64_t nnz);
+// library's own per-device arrays, which calls that overlap in time would share.  longest_row: no row has more entries
+// (the second kernel, which merges the pieces of huge rows, is left out where there are none).
+int launch_row_softmax(int64_t n_rows, const int32_t *d_row_ptr, const float *d_x, float *d_out, void *stream, void *d_ws, int64_t nnz, int64_t longest_row);
 int64_t row_softmax_workspace_bytes(int64_t nnz, int64_t n_rows);
 
 bool check_sorted(const sddmm_coo &S);

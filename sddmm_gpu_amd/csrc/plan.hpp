@@ -38,6 +38,7 @@ struct Launch {
     int32_t grid = 0, block = 0, lds = 0, k_slice = 0;
     int32_t tile_g = 0, gather_g = 8;
     int64_t nnz = 0, rows = 0, positions = 0;
+    int64_t longest_row = 0;  // most nonzeros in a row of S (the same for all launches of a plan)
     // what the function pointers above were looked up with (they are looked up again when a saved plan is loaded)
     int32_t fn_kind = 0;  // 1 stream kernel (row gather), 2 stream kernel with an LDS tile, 3 tile kernel, 4 panel, 5 dense,
                           // 6 row blocks

@@ -1115,6 +1115,11 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
     c.row_ptr = row_ptr_all;
     if (nnz > 0)
         if (int rc = c.need_row_ptr()) return rc;
+    std::vector<int32_t> longest((size_t)hw_threads() + 1, 0);
+    parallel_ranges(n_rows, 1 << 15, [&](int64_t b, int64_t e, int t) {
+        for (int64_t r = b; r < e; ++r) longest[(size_t)t] = std::max(longest[(size_t)t], row_ptr_all[r + 1] - row_ptr_all[r]);
+    });
+    for (Launch &L : P->launches) L.longest_row = *std::max_element(longest.begin(), longest.end());
     if (!P->launches.empty() && I.grid == 0) { I.grid = P->launches[0].grid; I.block = P->launches[0].block; I.lds_bytes = P->launches[0].lds; }
     I.n_launches = 0;
     for (const Launch &L : P->launches) {
