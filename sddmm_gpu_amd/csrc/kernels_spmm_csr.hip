@@ -36,12 +36,15 @@ constexpr int kSpmmUnroll = 4;  // H pieces requested together
 constexpr uint32_t kRowChange = 0x80000000u;
 
 // Zeroes the rows of Y that the product adds to or leaves out: empty rows, and rows cut between workgroups (of 2^shift nonzeros).
+// A wave looks at 64 rows, or fewer as in the kernel below: a small matrix of long rows of H has 16 to 64 nonzeros to a workgroup,
+// so nearly all of its rows are cut.  us with 64 rows a wave and so: 1024 rows, K = 256 6.0 and 2.3; 4096,
+// K = 384 10.0 and 3.3; 32,768, K = 192 7.2 and 5.6.
 __global__ __launch_bounds__(256)
-void sddmm_spmm_zero_rows_kernel(const int32_t *__restrict__ row_ptr, float *Y, int64_t n_rows, int K, int shift)
+void sddmm_spmm_zero_rows_kernel(const int32_t *__restrict__ row_ptr, float *Y, int64_t n_rows, int K, int shift, int rows_per_wave)
 {
     __shared__ int list[4][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t r = lane < rows_per_wave ? ((int64_t)blockIdx.x * 4 + wave) * rows_per_wave + lane : n_rows;
     bool zero = false;
     if (r < n_rows) {
         const int s = row_ptr[r], e = row_ptr[r + 1];
@@ -372,6 +375,14 @@ hipError_t launch_csr(const CsrShape &c, int64_t n_rows, int64_t n_cols, int64_t
     return hipErrorInvalidValue;
 }
 
+// Rows that a wave of the kernels beside the product looks at.
+int rows_per_wave(int64_t n_rows, int K)
+{
+    int per_wave = 64;
+    while (per_wave > 1 && n_rows < (int64_t)1024 * per_wave && per_wave / 2 * ((K + 3) / 4) >= 64) per_wave /= 2;
+    return per_wave;
+}
+
 }  // namespace
 
 namespace sddmm {
@@ -384,8 +395,7 @@ int launch_spmm_csr_records(int64_t n_rows, int64_t n_cols, int64_t nnz, const i
     const CsrShape c = csr_shape(nnz, K);
     hipStream_t st = (hipStream_t)stream;
     if (int rc = checked(launch_csr<true>(c, n_rows, n_cols, nnz, d_row_ptr, d_col_ind, d_x, K, d_H, d_Y, d_part, st))) return rc;
-    int per_wave = 64;
-    while (per_wave > 1 && n_rows < (int64_t)1024 * per_wave && per_wave / 2 * ((K + 3) / 4) >= 64) per_wave /= 2;
+    const int per_wave = rows_per_wave(n_rows, K);
     return checked(launch(sddmm_spmm_cut_rows_kernel, dim3((unsigned)((n_rows + 4 * per_wave - 1) / (4 * per_wave))), dim3(256), 0, st, d_row_ptr,
                           d_part, d_Y, n_rows, (int)K, c.wg_shift, per_wave));
 }
@@ -405,8 +415,9 @@ extern "C" int sddmm_spmm_csr(int64_t n_rows, int64_t n_cols, int64_t nnz, const
         return checked(launch(sddmm_spmm_generic_kernel, dim3(grid), dim3(256), 0, st, d_row_ptr, d_col_ind, d_x, d_H, d_Y, n_rows, (int)K));
     }
     const CsrShape c = csr_shape(nnz, K);
-    if (int rc = checked(launch(sddmm_spmm_zero_rows_kernel, dim3((unsigned)((n_rows + 255) / 256)), dim3(256), 0, st, d_row_ptr, d_Y, n_rows,
-                                (int)K, c.wg_shift)))
+    const int per_wave = rows_per_wave(n_rows, K);
+    if (int rc = checked(launch(sddmm_spmm_zero_rows_kernel, dim3((unsigned)((n_rows + 4 * per_wave - 1) / (4 * per_wave))), dim3(256), 0, st, d_row_ptr,
+                                d_Y, n_rows, (int)K, c.wg_shift, per_wave)))
         return rc;
     if (nnz == 0) return SDDMM_OK;
     return checked(launch_csr<false>(c, n_rows, n_cols, nnz, d_row_ptr, d_col_ind, d_x, K, d_H, d_Y, nullptr, st));
