@@ -338,11 +338,43 @@ struct CsrShape {
     int G, shift, wg_shift, slices, slice_pieces;
     int64_t workgroups;
 };
-CsrShape csr_shape(int64_t nnz, int K)
+// Pieces of four floats in a slice of a row, at most.  The slices of H follow each other over the whole matrix (the grid's
+// second dimension), so a slice that fits a die's 4 MB of L2 is gathered from there, and the columns and values read once
+// more per slice, 8 bytes a nonzero, cost less than that gives.  Where rows lie on lines of 128 bytes (K a multiple of 32):
+// the widest slices of 32, 16 or 8 pieces that divide a row and fit, at least 16 below 1.5 million nonzeros; whole rows where H
+// fits as a whole, and at narrow ranks where there is too little to gain.  us, whole rows (two slices beyond K = 256) and so:
+// band of 11.6 million in +-600 columns, K = 64 / 128 / 512 290 / 708 / 3067 and 193 / 385 / 1503; uniform, 3 million of 17,000
+// columns, K = 128 / 256 128 / 337 and 85 / 156; word counts of 10 million, K = 96 / 256 267 / 973 and 213 / 558; ratings of
+// 4.9 / 16.8 million, K = 256 225 / 1076 and 186 / 642; R-MAT of 1.8 / 7.5 million, K = 256 250 / 1236 and 165 / 785; window of
+// 16,384 tokens, 5.2 million, K = 256 282 and 197.  Uniform over 400,000 columns, whose slices fit nowhere, loses 2 to 4 %
+// (K = 64 / 256, 4.7 million: 191 / 737 and 199 / 757).  Rows across lines of 128 bytes gain nothing up to K = 256 (a slice
+// touches one line more); beyond, slices of 32 or 16 pieces fill their lanes better than two of up to 64 (K = 300: ratings of 4.9
+// million 393 and 312, uniform of 3 million 579 and 440).  And few nonzeros: a group has 4 of them, so a workgroup of whole
+// rows has 16, and nearly every row of S is cut and added atomically; slices have more to a workgroup (14 thousand, K = 256 15.9
+// and 9.4).
+int slice_pieces_most(int64_t nnz, int64_t n_cols, int K)
+{
+    constexpr int64_t kL2 = 4200000;
+    const int pieces = (K + 3) / 4;
+    const int64_t h = 16 * (int64_t)pieces * n_cols;
+    if (nnz <= 65536) return K >= 160 ? 16 : 64;
+    const int wide = K <= 256 ? 64 : 32;
+    if (nnz < 300000 || h <= kL2) return wide;
+    if (K % 32 != 0) return K > 256 && nnz >= 1500000 ? 16 : wide;
+    if (K < 192 && (nnz < (K < 96 ? 4000000 : K < 128 ? 2000000 : 1500000) || h <= (K < 96 ? 20000000 : K < 128 ? 6000000 : kL2))) return wide;
+    int narrow = 0;  // the narrowest that divides a row
+    for (int p : {32, 16, 8}) {
+        if (p >= pieces || pieces % p != 0 || (p == 8 && nnz < 1500000)) continue;
+        narrow = p;
+        if (16 * (int64_t)p * n_cols <= kL2) break;
+    }
+    return narrow ? narrow : wide;
+}
+CsrShape csr_shape(int64_t nnz, int64_t n_cols, int K)
 {
     CsrShape c;
-    const int pieces = (K + 3) / 4;
-    c.slices = (pieces + 63) / 64;
+    const int pieces = (K + 3) / 4, most = slice_pieces_most(nnz, n_cols, K);
+    c.slices = (pieces + most - 1) / most;
     c.slice_pieces = (pieces + c.slices - 1) / c.slices;
     c.G = 4;
     while (c.G < c.slice_pieces) c.G *= 2;
@@ -387,12 +419,12 @@ int rows_per_wave(int64_t n_rows, int K)
 
 namespace sddmm {
 
-int64_t spmm_csr_records(int64_t nnz, int K) { return K < 4 ? 0 : 2 * csr_shape(nnz, K).workgroups; }
+int64_t spmm_csr_records(int64_t nnz, int64_t n_cols, int K) { return K < 4 ? 0 : 2 * csr_shape(nnz, n_cols, K).workgroups; }
 
 int launch_spmm_csr_records(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *d_row_ptr, const int32_t *d_col_ind, const float *d_x, int32_t K,
                             const float *d_H, float *d_Y, float *d_part, void *stream)
 {
-    const CsrShape c = csr_shape(nnz, K);
+    const CsrShape c = csr_shape(nnz, n_cols, K);
     hipStream_t st = (hipStream_t)stream;
     if (int rc = checked(launch_csr<true>(c, n_rows, n_cols, nnz, d_row_ptr, d_col_ind, d_x, K, d_H, d_Y, d_part, st))) return rc;
     const int per_wave = rows_per_wave(n_rows, K);
@@ -414,7 +446,7 @@ extern "C" int sddmm_spmm_csr(int64_t n_rows, int64_t n_cols, int64_t nnz, const
         const unsigned grid = (unsigned)std::min<int64_t>((n_rows + 3) / 4, 256 * 64);
         return checked(launch(sddmm_spmm_generic_kernel, dim3(grid), dim3(256), 0, st, d_row_ptr, d_col_ind, d_x, d_H, d_Y, n_rows, (int)K));
     }
-    const CsrShape c = csr_shape(nnz, K);
+    const CsrShape c = csr_shape(nnz, n_cols, K);
     const int per_wave = rows_per_wave(n_rows, K);
     if (int rc = checked(launch(sddmm_spmm_zero_rows_kernel, dim3((unsigned)((n_rows + 4 * per_wave - 1) / (4 * per_wave))), dim3(256), 0, st, d_row_ptr,
                                 d_Y, n_rows, (int)K, c.wg_shift, per_wave)))
