@@ -24,7 +24,7 @@
 // has work, waits the rest: 2.5 units per compute unit, first loads, the barrier between tiles and rows
 // (profiles/row_blocks_attention_k64.txt).  Window of 128 on either side of 16,384 tokens, 32 full rows and columns, K = 64
 // (5.2 M nonzeros, 5602 tiles), us: scores and softmax 22 + 6 for the long rows (tile kernel and three softmax kernels 41 +
-// 34), product 22 + 4 (walk over the pattern 66 + 5).  The relative error against 64 bits is smaller than that of those:
+// 34), product 19 + 4 (walk over the pattern 66 + 5).  The relative error against 64 bits is smaller than that of those:
 // scores 5.2e-8 (8.3e-8), product 6.6e-8 (11e-8), at K = 128 6.4e-8 (8.8e-8) and 6.6e-8 (15e-8).
 // Measured on the way, us of the two kernels: epilogue from the accumulators' layout, tiles' scores read back one at a time
 // 40; three waves per SIMD for all with 170 registers spilling 41 and 65 (a kernel that uses scratch memory starts late as
@@ -317,7 +317,7 @@ void sddmm_block_long_rows_kernel(const BlockArgs a, const int32_t *__restrict__
 
 // KT: K / 32 rounded up
 template <int KT, int NW>
-__global__ __launch_bounds__(64 * NW, 2)
+__global__ __launch_bounds__(64 * NW, KT == 2 && NW == 4 ? 3 : 2)
 void sddmm_block_spmm_kernel(const BlockArgs a)
 {
     extern __shared__ float lds[];  // the waves' tiles of X, afterwards their sums; behind them the unit's masks and columns
@@ -340,7 +340,10 @@ void sddmm_block_spmm_kernel(const BlockArgs a)
     // What a tile needs is requested while the one before is multiplied.
     // X comes half a tile at a time, H in portions: portion q is the elements 32 (q % KT) on of the columns' rows of step
     // q / KT, and portion q + AHEAD is requested when portion q has been multiplied.
-    constexpr int AHEAD = KT == 3 ? 3 : KT == 1 ? 2 : 4;
+    // (K = 33 to 64 in workgroups of four waves: two portions ahead instead of four leave 168 registers of 185, and a SIMD holds three
+    // waves instead of two; 16,384 tokens, K = 64, window of 128 on either side, us of this kernel 22.0 and 18.7, scores, softmax
+    // and product of 32,359 tokens, 73 on either side, 67.5 and 62.7; level below 10,000 tokens)
+    constexpr int AHEAD = KT == 3 ? 3 : KT == 1 || (KT == 2 && NW == 4) ? 2 : 4;
     float x[8], h[AHEAD][8];
     const int xc = lane & 15, xr0 = lane >> 4;  // this lane's column in half a tile, its first row
     auto fetch = [&](int s, int u) {  // half a tile: columns 16 s on, rows xr0 + 4 i
