@@ -28,15 +28,27 @@ namespace {
 
 typedef float vec4f __attribute__((ext_vector_type(4)));
 
-// The value that lane I of this lane's group of 8 holds, by two row broadcasts of the data-parallel
-// primitives (one per half of a 16-lane row) and a select: vector-ALU work with no trip through the LDS
-// pipe, which the H reads keep busy and whose latency would sit in front of every round.
+// The value that lane I of this lane's group of 8 holds, by two row broadcasts of the data-parallel primitives, the second
+// for the upper half of a 16-lane row only: vector-ALU work with no trip through the LDS pipe, which the H reads keep busy
+// and whose latency would sit in front of every round.
 template <int I>
-__device__ __forceinline__ int from_group_lane(int v, bool upper_group)
+__device__ __forceinline__ int from_group_lane(int v)
 {
-    const int lo = __builtin_amdgcn_update_dpp(0, v, 0x150 + I, 0xf, 0xf, false);      // row_newbcast:I
-    const int up = __builtin_amdgcn_update_dpp(0, v, 0x150 + I + 8, 0xf, 0xf, false);  // row_newbcast:I+8
-    return upper_group ? up : lo;
+    const int lo = __builtin_amdgcn_update_dpp(0, v, 0x150 + I, 0xf, 0xf, false);   // row_newbcast:I
+    return __builtin_amdgcn_update_dpp(lo, v, 0x150 + I + 8, 0xf, 0xc, false);      // row_newbcast:I+8
+}
+// base + what lane 0, 1, ... 7 of this lane's group holds in v: the broadcasts as operands of the additions, which the
+// compiler does not find.  (The s_nop covers the two wait states between a vector write of v and its use as such an operand.)
+__device__ __forceinline__ void add_of_group(int v, int base, int (&sum)[8])
+{
+#define SDDMM_ADD_OF(i, j)                                                       \
+    "v_add_u32_dpp %" #i ", %8, %9 row_newbcast:" #i " row_mask:0xf bank_mask:0x3\n\t" \
+    "v_add_u32_dpp %" #i ", %8, %9 row_newbcast:" #j " row_mask:0xf bank_mask:0xc\n\t"
+    asm("s_nop 1\n\t" SDDMM_ADD_OF(0, 8) SDDMM_ADD_OF(1, 9) SDDMM_ADD_OF(2, 10) SDDMM_ADD_OF(3, 11) SDDMM_ADD_OF(4, 12) SDDMM_ADD_OF(5, 13)
+        SDDMM_ADD_OF(6, 14) SDDMM_ADD_OF(7, 15)
+        : "=&v"(sum[0]), "=&v"(sum[1]), "=&v"(sum[2]), "=&v"(sum[3]), "=&v"(sum[4]), "=&v"(sum[5]), "=&v"(sum[6]), "=&v"(sum[7])
+        : "v"(v), "v"(base));
+#undef SDDMM_ADD_OF
 }
 
 // KPL float4 per lane: a K slice of 32 * KPL elements on groups of 8 lanes
@@ -56,8 +68,8 @@ void sddmm_spmm_tile_kernel(const SpmmArgs a)
     int piece[KPL];  // float4 index inside a row of this lane's j-th piece
 #pragma unroll
     for (int j = 0; j < KPL; ++j) piece[j] = (j ^ rot) * G + l;
-    // (its address is the row's + lane_e + 128 j for even j, + lane_o + 128 j for odd j: two adds per row)
-    const int lane_e = lds_base + (l + rot * G) * 16, lane_o = lds_base + (l - rot * G) * 16;
+    // (its address is the row's + lane_e + 128 j for even j, that + odd for odd j)
+    const int lane_e = lds_base + (l + rot * G) * 16, odd = -2 * rot * G * 16;
     const int row_k4 = a.K >> 2;
     const float4 *__restrict__ H4 = reinterpret_cast<const float4 *>(a.H) + (a.k_off >> 2);
     float4 *__restrict__ part4 = reinterpret_cast<float4 *>(a.part);
@@ -85,77 +97,109 @@ void sddmm_spmm_tile_kernel(const SpmmArgs a)
             }
             __syncthreads();
         }
-        // A wave takes the bundles wave, wave + NW, ... of the item.  While bundle b is walked, the headers of bundle
-        // b + 2 NW and the first three rounds of bundle b + NW are requested; inside a bundle round r + 3 is requested
-        // while round r is computed.  A round is 8 steps: lane l of a group fetches the column and the value of the
-        // group's step 8 r + l, and the group's lanes take them from each other (from_group_lane).
+        // A wave takes the bundles wave, wave + NW, ... of the item, round by round; a round is 8 steps: lane l of a group
+        // fetches the column and the value of the group's step 8 r + l, and the group's lanes take them from each other
+        // (from_group_lane).  Three rounds are in flight, whatever the bundles' ends, and the header of the bundle behind the
+        // one that they come from.  The rounds' registers go round by name, four in turn: a copy of what is in flight from one
+        // name to another waits for it, and with three names that were shifted every round and every bundle waited for its
+        // latest loads.  Nor are steps behind a bundle's longest run done, but for one where that is odd.  us of residual and
+        // product together, with those waits, steps and a select per broadcast, and so: ratings of 4.9 million nonzeros, K = 50
+        // 91.7 and 84.9; 15 million, K = 32 157.7 and 136.6; 98 million, K = 128 2249 and 2079; 17 million, K = 200 874 and 830.
+        // (More loads in flight while a tile is staged give nothing.)
         if (wi.begin + wave >= wi.end) continue;
-        struct Hdr { int p0, len, off, n8; };
-        auto header = [&](int b) -> Hdr {
+        struct Header { int p0, len, off, end; };
+        auto header = [&](int b) -> Header {
             const int bc = min(b, wi.end - 1);  // (beyond the item: the last bundle again, never used)
-            Hdr h;
-            h.p0 = a.b_p0[bc * 8 + g]; h.len = a.b_len[bc * 8 + g];
-            h.off = a.b_off[bc]; h.n8 = a.b_off[bc + 1] - h.off;
-            return h;
+            return {a.b_p0[bc * 8 + g], a.b_len[bc * 8 + g], a.b_off[bc], a.b_off[bc + 1]};
         };
-        struct Round { uint32_t c; float x; };
-        auto fetch = [&](const Hdr &h, int r) -> Round {
-            const int rc = min(r, h.n8 - 1);
-            Round q;
-            q.c = a.cols[((size_t)(h.off + rc) * 8 + g) * 8 + l];
-            const int s = 8 * rc + l;
-            const float xv = a.x[h.p0 + min(s, max(h.len, 1) - 1)];
-            q.x = s < h.len ? xv : 0.f;
+        struct Round {
+            uint32_t c;  // column of step l
+            float x;     // its value, or that of the group's last step
+            int rem;     // the group's steps from the lane's one on
+            int bundle, steps, before;  // (uniform) bundle, its steps from here on, those of the rounds before
+            bool last;
+        };
+        int bundle = wi.begin + wave, r = 0, off, n8, longest;  // what is fetched next: round r of the bundle's n8
+        int first, last, lim;  // of the lane's step in the bundle's round 0, of the group's last one; the group's steps from the former on
+        auto enter = [&](const Header &h) {
+            off = __builtin_amdgcn_readfirstlane(h.off);
+            n8 = __builtin_amdgcn_readfirstlane(h.end) - off;
+            longest = __builtin_amdgcn_readfirstlane(h.len);  // (the bundle's first run)
+            first = h.p0 + l;
+            last = h.p0 + (max(h.len, 1) - 1);
+            lim = h.len - l;
+        };
+        enter(header(bundle));
+        Header ahead = header(bundle + NW);
+        auto fetch = [&]() -> Round {
+            if (r == n8) {
+                bundle += NW;
+                r = 0;
+                enter(ahead);
+                ahead = header(bundle + NW);
+            }
+            const uint16_t *cols = a.cols + (size_t)(off + r) * 64;
+            const Round q = {cols[lane], a.x[min(first + 8 * r, last)], lim - 8 * r, bundle, longest - 8 * r, 8 * r, r + 1 == n8};
+            ++r;
             return q;
         };
-        Hdr h0 = header(wi.begin + wave), h1 = header(wi.begin + wave + NW);
-        Round q0 = fetch(h0, 0), q1 = fetch(h0, 1), q2 = fetch(h0, 2);
-        for (int b = wi.begin + wave; b < wi.end; b += NW) {
-            const Hdr h2 = header(b + 2 * NW);
-            Round n0 = fetch(h1, 0), n1 = fetch(h1, 1), n2 = fetch(h1, 2);
-            const int n8 = __builtin_amdgcn_readfirstlane(h0.n8);
-            float4 acc[KPL];
+        float4 acc[KPL];
 #pragma unroll
-            for (int j = 0; j < KPL; ++j) acc[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-            auto rd = [&](vec4f (&h)[KPL], int off) {
-                const int addr_e = off + lane_e, addr_o = off + lane_o;
+        for (int j = 0; j < KPL; ++j) acc[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+        auto rd = [&](vec4f (&h)[KPL], int addr_e) {
+            const int addr_o = addr_e + odd;
 #pragma unroll
-                for (int j = 0; j < KPL; ++j) h[j] = *(lds_f4_ptr)(uintptr_t)(uint32_t)(((j & 1) ? addr_o : addr_e) + j * 128);
-            };
-            for (int r = 0; r < n8; ++r) {
-                const Round q3 = fetch(h0, r + 3);
-                // the columns (as row offsets in the tile) and the values of the round's eight steps, taken from the
-                // group's lanes
-                int row_off[8];
-                float xs[8];
-                const int my_off = (int)q0.c * (K4 * 16), my_x = __float_as_int(q0.x);
-                const bool upper = (lane & 8) != 0;
-                [&]<int... I>(std::integer_sequence<int, I...>) {
-                    ((row_off[I] = from_group_lane<I>(my_off, upper), xs[I] = __int_as_float(from_group_lane<I>(my_x, upper))), ...);
-                }(std::make_integer_sequence<int, 8>{});
-                // the H pieces of step i + 1 are requested before the arithmetic of step i
-                vec4f hb[2][KPL];
-                rd(hb[0], row_off[0]);
+            for (int j = 0; j < KPL; ++j) h[j] = *(lds_f4_ptr)(uintptr_t)(uint32_t)(((j & 1) ? addr_o : addr_e) + j * 128);
+        };
+        auto compute = [&](const Round &q) {
+            // where this lane's pieces of the H rows of the round's eight steps begin, and the values, taken from the
+            // group's lanes
+            int at[8];
+            float xs[8];
+            add_of_group((int)q.c * (K4 * 16), lane_e, at);
+            const int my_x = __float_as_int(q.rem > 0 ? q.x : 0.f);
+            [&]<int... I>(std::integer_sequence<int, I...>) {
+                ((xs[I] = __int_as_float(from_group_lane<I>(my_x))), ...);
+            }(std::make_integer_sequence<int, 8>{});
+            // the H pieces of step i + 1 are requested before the arithmetic of step i
+            vec4f hb[2][KPL];
+            rd(hb[0], at[0]);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    if (i + 1 < 8) rd(hb[(i + 1) & 1], row_off[i + 1]);
-                    __builtin_amdgcn_sched_barrier(0);
+            for (int i = 0; i < 8; ++i) {
+                if (i > 0 && i % 2 == 0 && i >= q.steps) break;
+                if (i + 1 < 8) rd(hb[(i + 1) & 1], at[i + 1]);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int j = 0; j < KPL; ++j) {
-                        const vec4f h = hb[i & 1][j];
-                        acc[j].x = fmaf(xs[i], h.x, acc[j].x); acc[j].y = fmaf(xs[i], h.y, acc[j].y);
-                        acc[j].z = fmaf(xs[i], h.z, acc[j].z); acc[j].w = fmaf(xs[i], h.w, acc[j].w);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
+                for (int j = 0; j < KPL; ++j) {
+                    const vec4f h = hb[i & 1][j];
+                    acc[j].x = fmaf(xs[i], h.x, acc[j].x); acc[j].y = fmaf(xs[i], h.y, acc[j].y);
+                    acc[j].z = fmaf(xs[i], h.z, acc[j].z); acc[j].w = fmaf(xs[i], h.w, acc[j].w);
                 }
-                q0 = q1; q1 = q2; q2 = q3;
+                __builtin_amdgcn_sched_barrier(0);
             }
-            if (h0.len > 0) {
-                float4 *dst = part4 + ((size_t)b * 8 + g) * K4;
+            if (q.last) {
+                float4 *dst = part4 + ((size_t)q.bundle * 8 + g) * K4;
 #pragma unroll
-                for (int j = 0; j < KPL; ++j) dst[piece[j]] = acc[j];
+                for (int j = 0; j < KPL; ++j) {
+                    if (q.rem + q.before + l > 0) dst[piece[j]] = acc[j];
+                    acc[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+                }
             }
-            h0 = h1; h1 = h2; q0 = n0; q1 = n1; q2 = n2;
+        };
+        Round q0 = fetch(), q1 = fetch(), q2 = fetch();
+        for (;;) {
+            const Round q3 = fetch();
+            if (q0.bundle >= wi.end) break;
+            compute(q0);
+            q0 = fetch();
+            if (q1.bundle >= wi.end) break;
+            compute(q1);
+            q1 = fetch();
+            if (q2.bundle >= wi.end) break;
+            compute(q2);
+            q2 = fetch();
+            if (q3.bundle >= wi.end) break;
+            compute(q3);
         }
     }
 }
