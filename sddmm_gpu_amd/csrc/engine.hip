@@ -153,7 +153,7 @@ static hipError_t issue_launch(const sddmm_plan *plan, const Launch &L, const fl
         if (!softmax) return launch(L.bfns[0], dim3((unsigned)L.grid), dim3((unsigned)L.block), std::min<size_t>((size_t)L.lds, (size_t)kRoundTiles * kBlockTileBytes), stream, ba);
         if (ws && ba.long_records) ba.long_records = reinterpret_cast<float2 *>(ws + L.ws_part);
         if (hipError_t e = launch(L.bfns[1], dim3((unsigned)L.grid), dim3((unsigned)(64 * L.softmax_waves)), (size_t)L.lds, stream, ba)) return e;
-        return launch_block_long_rows(ba, plan->d_row_ptr, stream);
+        return launch_block_long_rows(ba, stream);
     } else if (L.tfn) {
         TileArgs ta = L.ta;
         ta.val = val;

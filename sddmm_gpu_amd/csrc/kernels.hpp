@@ -220,8 +220,8 @@ struct BlockArgs {
     const int32_t *rows;      // [n_blocks][32] the blocks' rows (a short block repeats its last row, with empty masks)
     const int32_t *cols;      // [n_tiles][32] the tiles' columns, ascending (a short tile repeats its last one, with no bit set)
     const uint2 *info;        // [n_tiles][32] per row: which of the tile's columns it has; sorted position of the first one
-    // the rows of blocks that are several units, in pieces of kLongPiece entries: row, its first piece, its pieces, the number
-    // of this one among them; records of the pieces for the softmax (null where every row is one piece)
+    // the rows of blocks that are several units, in pieces of kLongPiece entries: first entry, entries, the row's
+    // first piece, its pieces; records of the pieces for the softmax (null where every row is one piece)
     const int4 *long_pieces;
     float2 *long_records;
     const int4 *sums;         // [n_sums] blocks that are several units: row block, first record, records
@@ -239,7 +239,7 @@ using BlockFn = void (*)(const BlockArgs);
 bool block_supported(int K);
 BlockFn block_kernel(int K, bool softmax, int nwaves);  // nwaves: waves per workgroup, 4 or 8
 hipError_t block_spmm_set_lds(int K, int nwaves);
-hipError_t launch_block_long_rows(const BlockArgs &a, const int32_t *row_ptr, void *stream);  // the softmax of a.long_pieces, in place in a.out
+hipError_t launch_block_long_rows(const BlockArgs &a, void *stream);  // the softmax of a.long_pieces, in place in a.out
 hipError_t launch_block_spmm(const BlockArgs &a, int nwaves, void *stream);
 
 // lanes per nonzero and float4 slots per lane for a given K; G == 0: none

@@ -23,7 +23,7 @@
 // instructions, 27 and 35 % of which lie under vector ones; that fills a SIMD for 59 and 53 % of the time its compute unit
 // has work, waits the rest: 2.5 units per compute unit, first loads, the barrier between tiles and rows
 // (profiles/row_blocks_attention_k64.txt).  Window of 128 on either side of 16,384 tokens, 32 full rows and columns, K = 64
-// (5.2 M nonzeros, 5602 tiles), us: scores and softmax 22 + 6 for the long rows (tile kernel and three softmax kernels 41 +
+// (5.2 M nonzeros, 5602 tiles), us: scores and softmax 22 + 5.5 for the long rows (tile kernel and three softmax kernels 41 +
 // 34), product 19 + 4 (walk over the pattern 66 + 5).  The relative error against 64 bits is smaller than that of those:
 // scores 5.2e-8 (8.3e-8), product 6.6e-8 (11e-8), at K = 128 6.4e-8 (8.8e-8) and 6.6e-8 (15e-8).
 // Measured on the way, us of the two kernels: epilogue from the accumulators' layout, tiles' scores read back one at a time
@@ -254,19 +254,21 @@ void sddmm_block_kernel(const BlockArgs a)
 
 // The softmax of the rows whose blocks are several units, in place, in pieces of up to 16,384 entries, each held in the
 // registers of a workgroup.  A row of one piece is done at once; of a longer one the first pass (RECORD) leaves the
-// pieces' (max, sum), the second joins them and writes.
+// pieces' (max, sum), the second joins them and writes.  A few workgroups, bound by their chain of loads, so a piece says where
+// its entries lie (looked up in the row pointers, and with the sum kernel below asking for its row only after its sums: scores,
+// softmax and product of 16,384 tokens, K = 64, 48.6 us, now 47.9; 32,359 tokens 63.4 and 62.8).
 constexpr int kLongThreads = 1024, kLongEach = kLongPiece / kLongThreads;
 
 template <bool RECORD>
 __global__ __launch_bounds__(kLongThreads)
-void sddmm_block_long_rows_kernel(const BlockArgs a, const int32_t *__restrict__ row_ptr)
+void sddmm_block_long_rows_kernel(const BlockArgs a)
 {
     __shared__ float red[2][kLongThreads / 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int4 piece = a.long_pieces[blockIdx.x];  // row, its first piece, its pieces, this one's number among them
-    if (!RECORD && piece.z == 1) return;
-    const int rb = row_ptr[piece.x] + piece.w * kLongPiece, len = min(kLongPiece, row_ptr[piece.x + 1] - rb);
-    float *o = a.out + rb;
+    const int4 piece = a.long_pieces[blockIdx.x];  // first entry, entries, the row's first piece, its pieces
+    if (!RECORD && piece.w == 1) return;
+    const int len = piece.y;
+    float *o = a.out + piece.x;
     float v[kLongEach];
 #pragma unroll
     for (int i = 0; i < kLongEach; ++i) {
@@ -285,7 +287,7 @@ void sddmm_block_long_rows_kernel(const BlockArgs a, const int32_t *__restrict__
 #pragma unroll
         for (int i = 0; i < kLongEach; ++i) {
             const float e = v[i] == -INFINITY ? 0.f : exp_nonpositive(v[i] - all);  // (a piece's maximum may be that)
-            v[i] = piece.z == 1 && all == -INFINITY ? NAN : e;                      // (a row's: no weights)
+            v[i] = piece.w == 1 && all == -INFINITY ? NAN : e;                      // (a row's: no weights)
             s += e;
         }
 #pragma unroll
@@ -294,14 +296,14 @@ void sddmm_block_long_rows_kernel(const BlockArgs a, const int32_t *__restrict__
         __syncthreads();
         s = 0.f;
         for (int w = 0; w < kLongThreads / 64; ++w) s += red[1][w];
-        if (piece.z > 1) {
-            if (threadIdx.x == 0) a.long_records[piece.y + piece.w] = make_float2(all, s);
+        if (piece.w > 1) {
+            if (threadIdx.x == 0) a.long_records[blockIdx.x] = make_float2(all, s);
             return;
         }
     } else {
-        for (int k = 0; k < piece.z; ++k) all = fmaxf(all, a.long_records[piece.y + k].x);
-        for (int k = 0; k < piece.z; ++k) {
-            const float2 r = a.long_records[piece.y + k];
+        for (int k = 0; k < piece.w; ++k) all = fmaxf(all, a.long_records[piece.z + k].x);
+        for (int k = 0; k < piece.w; ++k) {
+            const float2 r = a.long_records[piece.z + k];
             s += r.y == 0.f ? 0.f : r.y * exp_nonpositive(r.x - all);
         }
 #pragma unroll
@@ -501,6 +503,10 @@ void sddmm_block_sum_kernel(const BlockArgs a, int results, int sum_groups)
         const int4 block = a.sums[blockIdx.x / parts];  // row block, first record, records
         const int e = (blockIdx.x % parts) * 64 + lane;
         const float *rec = a.part + (size_t)block.y * results + e;
+        const int k = 32 * (e >> 10) + (e & 31), r = result_row((e >> 6) & 15, (e >> 5) & 1);
+        const int32_t *rows = a.rows + block.x * kRows;
+        const int row = rows[r], row_before = rows[max(r, 1) - 1];  // (on their way beside the records)
+        __builtin_amdgcn_sched_barrier(0);
         const int k1 = block.z * (wave + 1) / 4;
         float y = 0.f;
         for (int k0 = block.z * wave / 4; k0 < k1; k0 += 16) {  // (sixteen records in flight)
@@ -512,9 +518,8 @@ void sddmm_block_sum_kernel(const BlockArgs a, int results, int sum_groups)
         }
         quarter[wave][lane] = y;
         __syncthreads();
-        const int k = 32 * (e >> 10) + (e & 31), r = result_row((e >> 6) & 15, (e >> 5) & 1);
-        if (wave == 0 && k < K && !repeated_row(a.rows + block.x * kRows, r))
-            a.Y[(size_t)a.rows[block.x * kRows + r] * K + k] = (quarter[0][lane] + quarter[1][lane]) + (quarter[2][lane] + quarter[3][lane]);
+        if (wave == 0 && k < K && !(r > 0 && row == row_before))
+            a.Y[(size_t)row * K + k] = (quarter[0][lane] + quarter[1][lane]) + (quarter[2][lane] + quarter[3][lane]);
         return;
     }
     const int64_t n = (int64_t)a.n_empty * K, stride = (int64_t)(gridDim.x - sum_groups) * 256;
@@ -566,12 +571,12 @@ hipError_t block_spmm_set_lds(int K, int nwaves)
     return hipFuncSetAttribute((const void *)block_spmm_of(K, nwaves), hipFuncAttributeMaxDynamicSharedMemorySize, (int)spmm_lds_bytes((K + 31) / 32, nwaves));
 }
 
-hipError_t launch_block_long_rows(const BlockArgs &a, const int32_t *row_ptr, void *stream)
+hipError_t launch_block_long_rows(const BlockArgs &a, void *stream)
 {
     if (a.n_long_pieces <= 0) return hipSuccess;
     const dim3 grid((unsigned)a.n_long_pieces), block(kLongThreads);
-    hipError_t e = launch(sddmm_block_long_rows_kernel<true>, grid, block, 0, (hipStream_t)stream, a, row_ptr);
-    if (e == hipSuccess && a.long_records) e = launch(sddmm_block_long_rows_kernel<false>, grid, block, 0, (hipStream_t)stream, a, row_ptr);
+    hipError_t e = launch(sddmm_block_long_rows_kernel<true>, grid, block, 0, (hipStream_t)stream, a);
+    if (e == hipSuccess && a.long_records) e = launch(sddmm_block_long_rows_kernel<false>, grid, block, 0, (hipStream_t)stream, a);
     return e;
 }
 

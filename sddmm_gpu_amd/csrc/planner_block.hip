@@ -187,7 +187,8 @@ int add_blocks(Ctx &c, const std::vector<int32_t> &rows, bool *taken)
         for (int i = 0; i < R; ++i)
             if (const int32_t r = block_rows[(size_t)(b * R + i)]; r >= 0) {
                 const int n = (int)((len(r) + kLongPiece - 1) / kLongPiece), first = (int)long_pieces.size();
-                for (int k = 0; k < n; ++k) long_pieces.push_back(make_int4(r, first, n, k));
+                for (int k = 0; k < n; ++k)
+                    long_pieces.push_back(make_int4(c.row_ptr[r] + k * kLongPiece, (int)std::min<int64_t>(kLongPiece, len(r) - (int64_t)k * kLongPiece), first, n));
                 in_pieces = in_pieces || n > 1;
             }
     }
