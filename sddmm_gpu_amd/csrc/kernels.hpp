@@ -36,6 +36,9 @@ struct KArgs {
     // Plan-free form (batch_seg and batch_mask are null then): the rows are found from the row pointers.
     const int32_t *row_ptr;    // [n_rows+1]
     int32_t n_rows;
+    // Row gather: W and H begin at the first element of a slice of K elements of rows that are ld long.
+    int32_t ld;
+    int32_t add, part;         // add: out holds the dot product of the slices before; part: slices follow (out = dot)
 };
 
 constexpr int kRowGatherBlock = 256;   // 4 waves
@@ -251,6 +254,9 @@ GatherShape gather_shape(int64_t nnz, int64_t n_rows, int64_t listed_rows, int K
 inline bool gather_wide(int64_t n_rows, int64_t n_cols, int K) { return std::max(n_rows, n_cols) * K >= (int64_t)1 << 30; }  // byte offsets of 32 bits do not do
 KernelFn gather_kernel(const Variant &v, bool once, bool wide);
 KernelFn generic_kernel();           // row gather, any K
+int gather_slice(int64_t nnz, int64_t n_cols, int K);  // elements of a row per launch over all of a matrix
+// the row gather over a.nnz nonzeros on `stream`: fn over whole rows in workgroups of a.chunk, or slice by slice
+hipError_t launch_row_gather(KArgs a, KernelFn fn, int64_t listed_rows, int64_t n_rows, bool wide, int slice, void *stream);
 Variant pick_stream_variant(int K);  // unpadded LDS tile (K % 4 == 0)
 KernelFn stream_kernel(const Variant &v);
 

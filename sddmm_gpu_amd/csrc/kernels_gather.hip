@@ -18,6 +18,7 @@
 #include <utility>
 #include "kernels.hpp"
 #include "csr_walk.hpp"
+#include "launch.hpp"
 
 using namespace sddmm;
 
@@ -79,10 +80,17 @@ constexpr int whole_pieces(int G, int KPL) { return KPL == 8 ? 4 * G : (KPL - 1)
 // piece of a ragged row, and so: uniform, 0.9 million nonzeros of 4000 rows, K = 32 / 100 / 200: 9.6 / 23.8 / 41 and 9.1 /
 // 22.3 / 38; 18 thousand, K = 100 / 200: 4.9 / 7.3 and 4.6 / 6.3; where the fabric bounds it the same.)
 template <bool WIDE>
-__device__ __forceinline__ vec4u row_piece_of(const float *m, uint32_t at, int off, int K)
+__device__ __forceinline__ vec4u row_piece_of(const float *m, uint32_t at, int off, int ld)
 {
-    if constexpr (WIDE) return *reinterpret_cast<const vec4u *>(m + (size_t)at * K + off);
+    if constexpr (WIDE) return *reinterpret_cast<const vec4u *>(m + (size_t)at * ld + off);
     else return *reinterpret_cast<const vec4u *>(reinterpret_cast<const char *>(m) + ((at << 2) + ((uint32_t)off << 2)));
+}
+
+// The dot product of sorted position p, complete or a slice's share of it.
+__device__ __forceinline__ void finish(const KArgs &a, int p, float v, float dot)
+{
+    if (a.add) dot += a.out[p];
+    a.out[p] = a.part ? dot : a.residual ? v - dot : dot * v;
 }
 
 // RAGGED: K is not 4 * G * KPL (its pieces are masked; any K > 4 * G * (KPL - 1) up to 4 * G * KPL, K >= 4).
@@ -95,7 +103,7 @@ void sddmm_gather_kernel(const KArgs a)
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l = lane & (G - 1);
-    const int K = a.K;
+    const int K = a.K, ld = a.ld;
     const uint64_t le = (lane == 63) ? ~0ull : ((2ull << lane) - 1ull);
 
     int off[KPL];
@@ -139,7 +147,7 @@ void sddmm_gather_kernel(const KArgs a)
         }
         b.p = a.perm ? a.perm[pos] : pos;
         b.col = a.col_ind[b.p];
-        if constexpr (!WIDE) b.col = (int)((uint32_t)b.col * (uint32_t)K);
+        if constexpr (!WIDE) b.col = (int)((uint32_t)b.col * (uint32_t)ld);
         b.v = a.sval ? a.sval[pos] : (a.val ? a.val[b.p] : 1.0f);
         return b;
     };
@@ -158,16 +166,16 @@ void sddmm_gather_kernel(const KArgs a)
     // requests the pieces of step I of a batch; changed: the lanes whose nonzero is in another row than the one before
     auto issue = [&]<int I>(std::integral_constant<int, I>, const Batch &b, uint64_t changed) {
         if (changed & (group_bits<G>() << I)) {
-            const uint32_t wr = (uint32_t)group_bcast<G, I>(WIDE ? b.row : b.row * K);
+            const uint32_t wr = (uint32_t)group_bcast<G, I>(WIDE ? b.row : b.row * ld);
 #pragma unroll
-            for (int j = 0; j < KPL; ++j) w[I & 1][j] = row_piece_of<WIDE>(a.W, wr, off[j], K);
+            for (int j = 0; j < KPL; ++j) w[I & 1][j] = row_piece_of<WIDE>(a.W, wr, off[j], ld);
         } else {
 #pragma unroll
             for (int j = 0; j < KPL; ++j) w[I & 1][j] = w[(I & 1) ^ 1][j];
         }
         const uint32_t hr = (uint32_t)group_bcast<G, I>(b.col);
 #pragma unroll
-        for (int j = 0; j < KPL; ++j) h[I & 1][j] = row_piece_of<WIDE>(a.H, hr, off[j], K);
+        for (int j = 0; j < KPL; ++j) h[I & 1][j] = row_piece_of<WIDE>(a.H, hr, off[j], ld);
     };
     // rows of a batch that differ from the row before: inside a group the lane before, for its first lane the
     // group's row at the end of the batch before
@@ -206,7 +214,7 @@ void sddmm_gather_kernel(const KArgs a)
             }(), ...);
         }(std::make_integer_sequence<int, G>{});
         transpose_reduce_step<G>(acc, l);
-        if (begin + (bi << 6) + lane < end) a.out[cur.p] = a.residual ? cur.v - acc[0] : acc[0] * cur.v;
+        if (begin + (bi << 6) + lane < end) finish(a, cur.p, cur.v, acc[0]);
         cur = nxt;
         nxt = after;
         changed = changed_next;
@@ -229,7 +237,7 @@ void sddmm_gather_once_kernel(const KArgs a)
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l = lane & (G - 1);
-    const int K = a.K;
+    const int K = a.K, ld = a.ld;
     const int batch = blockIdx.x * (kRowGatherBlock / 64) + wave;
     const int p0 = batch << 6;
     if (p0 >= a.nnz) return;
@@ -255,7 +263,7 @@ void sddmm_gather_once_kernel(const KArgs a)
         rows_of_range(a.row_ptr, a.n_rows, a.nnz, p0, 64, tab, lane);
         row = tab[pos - p0];
     }
-    const int h_at = WIDE ? col : (int)((uint32_t)col * (uint32_t)K), w_at = WIDE ? row : (int)((uint32_t)row * (uint32_t)K);
+    const int h_at = WIDE ? col : (int)((uint32_t)col * (uint32_t)ld), w_at = WIDE ? row : (int)((uint32_t)row * (uint32_t)ld);
     auto mask_piece = [&](vec4u &x, int j) {
         if (RAGGED && (j + 1) * G > whole_pieces(G, KPL)) {
             x.x = first[j] > 0 ? 0.f : x.x;
@@ -270,10 +278,10 @@ void sddmm_gather_once_kernel(const KArgs a)
         ((void)[&] {
             const uint32_t hr = (uint32_t)group_bcast<G, BASE + I>(h_at);
 #pragma unroll
-            for (int j = 0; j < KPL; ++j) h[I][j] = row_piece_of<WIDE>(a.H, hr, off[j], K);
+            for (int j = 0; j < KPL; ++j) h[I][j] = row_piece_of<WIDE>(a.H, hr, off[j], ld);
             const uint32_t wr = (uint32_t)group_bcast<G, BASE + I>(w_at);
 #pragma unroll
-            for (int j = 0; j < KPL; ++j) w[I][j] = row_piece_of<WIDE>(a.W, wr, off[j], K);
+            for (int j = 0; j < KPL; ++j) w[I][j] = row_piece_of<WIDE>(a.W, wr, off[j], ld);
         }(), ...);
         __builtin_amdgcn_sched_barrier(0);
         ((void)[&] {
@@ -293,7 +301,7 @@ void sddmm_gather_once_kernel(const KArgs a)
         (round(std::integer_sequence<int, R * ROUND>{}, std::make_integer_sequence<int, ROUND>{}), ...);
     }(std::make_integer_sequence<int, G / ROUND>{});
     transpose_reduce_step<G>(acc, l);
-    if (p0 + lane < a.nnz) a.out[p] = a.residual ? v - acc[0] : acc[0] * v;
+    if (p0 + lane < a.nnz) finish(a, p, v, acc[0]);
 }
 
 // Any K >= 1 (used below 4 and beyond 2048): 8 lanes per nonzero striding over the row one float at a time,
@@ -430,6 +438,48 @@ KernelFn gather_kernel(const Variant &v, bool once, bool wide)
 #undef SDDMM_CASE
 #undef SDDMM_FORM
     return nullptr;
+}
+
+// Elements of a row that one launch takes: K, or 64 in turn where the rows of H do not fit a die's 4 MB of L2 and slices of them
+// are found there more often.  The dot products so far wait in out, and columns and rows are read once more for every slice,
+// which it takes long rows and enough nonzeros to pay.  us at K = 256 / 512, whole rows and slices: R-MAT 2^17, 2.6 / 6.1 million
+// nonzeros, K = 256 320 / 801 and 259 / 616, 1.5 million, K = 512 459 and 369; 2^18, 6.5 million, K = 256 886 and 681, 4.1 million, K =
+// 512 1236 and 931; uniform, 3.1 million of 57,000 columns 430 / 812 and 384 / 735; word counts, 3 million of 40,000 240 / 556 and
+// 193 / 380; band of 3 million 429 / 814 and 420 / 808; K = 448, R-MAT 2^17, 5.7 million 1072 and 825.  Not
+//   below (R-MAT 2^15, 1.4 million, K = 256 103 and 121; 2^18, 1.1 million, K = 512 359 and 377; 1.6 million, K = 448 343 and 367),
+//   where few columns take most nonzeros and their rows fit (R-MAT 2^14, 3.0 million, K = 256 162 and 191; ratings of 6.2 million,
+//       5600 columns 284 and 300; uniform over 17,000 columns would gain: 3.2 million, K = 256 368 and 219),
+//   where most columns are used once (R-MAT 2^20, 1.6 million, K = 512 647 and 687; 3.3 million, K = 448 808 and 820),
+//   at other ranks (K = 384, whose lanes hold three pieces instead of four, R-MAT 2^15, 2.5 million 281 and 257, but band of 3 million
+//       594 and 653; K = 128, R-MAT 2^15, 4.4 million 121 and 133, uniform, 6 million 295 and 214).
+// Slices of 128 are faster on half of these, but at K = 512 their error against 64 bits is larger (9.9e-8 whole, 10.0e-8; of 64
+// 9.4e-8; K = 256 9.5e-8, 9.5e-8 and 8.6e-8).
+int gather_slice(int64_t nnz, int64_t n_cols, int K)
+{
+    const int64_t least = K == 256 ? 2500000 : K == 512 ? 1400000 : K == 448 ? 3000000 : INT64_MAX;
+    return nnz >= std::max(least, 4 * n_cols) && n_cols >= (K == 256 ? 24000 : 11000) ? 64 : K;
+}
+
+// One launch over whole rows, fn of shape's form, or one per slice.
+hipError_t launch_row_gather(KArgs a, KernelFn fn, int64_t listed_rows, int64_t n_rows, bool wide, int slice, void *stream)
+{
+    const hipStream_t st = (hipStream_t)stream;
+    auto run = [&](KernelFn f) { return launch(f, dim3((unsigned)((a.nnz + (int64_t)a.chunk - 1) / a.chunk)), dim3(kRowGatherBlock), 0, st, a); };
+    const int K = a.K;
+    a.ld = K;
+    // (values that lie where the results go would be overwritten by the first slice's)
+    const uintptr_t v = (uintptr_t)(a.sval ? a.sval : a.val), o = (uintptr_t)a.out, bytes = (uintptr_t)a.nnz * 4;
+    if (slice >= K || (v && v < o + bytes && o < v + bytes)) return run(fn);
+    const float *W = a.W, *H = a.H;
+    for (int k = 0; k < K; k += slice) {
+        a.K = std::min(slice, K - k);
+        a.W = W + k; a.H = H + k;
+        a.add = k > 0; a.part = k + slice < K;
+        const GatherShape s = gather_shape(a.nnz, n_rows, listed_rows, a.K);
+        a.chunk = s.chunk;
+        if (hipError_t e = run(gather_kernel(s.v, s.once, wide))) return e;
+    }
+    return hipSuccess;
 }
 
 KernelFn generic_kernel() { return (KernelFn)sddmm_generic_kernel; }

@@ -1,9 +1,8 @@
-// Plan-free SDDMM over a device CSR that allocates no memory and keeps none: one launch of the row-gather
-// kernel, which finds the rows of its nonzeros from the row pointers.
+// Plan-free SDDMM over a device CSR that allocates no memory and keeps none: the row-gather kernel in one
+// launch, or one per slice of K (gather_slice), finding the rows of its nonzeros from the row pointers.
 #include <hip/hip_runtime.h>
 #include "internal.hpp"
 #include "kernels.hpp"
-#include "launch.hpp"
 
 using namespace sddmm;
 
@@ -29,8 +28,7 @@ extern "C" int sddmm_csr_noalloc(int64_t n_rows, int64_t n_cols, int64_t nnz, co
     const GatherShape shape = gather_shape(nnz, n_rows, n_rows, K);
     const KernelFn fn = shape.v.G ? gather_kernel(shape.v, shape.once, gather_wide(n_rows, n_cols, K)) : generic_kernel();
     a.chunk = shape.chunk;
-    const int grid = (int)((nnz + a.chunk - 1) / a.chunk);
-    const hipError_t e = launch(fn, dim3((unsigned)grid), dim3(kRowGatherBlock), 0, (hipStream_t)stream, a);
+    const hipError_t e = launch_row_gather(a, fn, n_rows, n_rows, gather_wide(n_rows, n_cols, K), gather_slice(nnz, n_cols, K), stream);
     if (e != hipSuccess) return fail(SDDMM_ERR_HIP, "sddmm_csr_noalloc: launch failed: %s", hipGetErrorString(e));
     return SDDMM_OK;
 }

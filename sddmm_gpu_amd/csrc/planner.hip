@@ -297,7 +297,7 @@ int add_row_gather(Ctx &c, const std::vector<int32_t> &rows, bool all_rows)
     a.K = c.K; a.n_cols = (int32_t)c.n_cols; a.tile_x = (int32_t)c.n_cols;
     L.grid = (int32_t)((n + a.chunk - 1) / a.chunk);
     L.block = kRowGatherBlock;
-    L.k_slice = c.K;
+    L.k_slice = all_rows ? gather_slice(n, c.n_cols, c.K) : c.K;  // (as in the call without a plan)
     if (int rc = resolve_functions(L)) return rc;
     c.P->info.lanes_per_nnz = var.G ? var.G : 8;
     L.gather_g = var.G ? var.G : 8; L.positions = n;
