@@ -86,15 +86,23 @@ __device__ __forceinline__ vec4u row_piece_of(const float *m, uint32_t at, int o
     else return *reinterpret_cast<const vec4u *>(reinterpret_cast<const char *>(m) + ((at << 2) + ((uint32_t)off << 2)));
 }
 
-// The dot product of sorted position p, complete or a slice's share of it.
+// The dot product of sorted position p, complete or (SLICE) a slice's share of it.
+template <bool SLICE>
 __device__ __forceinline__ void finish(const KArgs &a, int p, float v, float dot)
 {
-    if (a.add) dot += a.out[p];
-    a.out[p] = a.part ? dot : a.residual ? v - dot : dot * v;
+    if constexpr (SLICE) {
+        if (a.add) dot += a.out[p];
+        if (a.part) {
+            a.out[p] = dot;
+            return;
+        }
+    }
+    a.out[p] = a.residual ? v - dot : dot * v;
 }
 
 // RAGGED: K is not 4 * G * KPL (its pieces are masked; any K > 4 * G * (KPL - 1) up to 4 * G * KPL, K >= 4).
-template <int G, int KPL, bool RAGGED, bool WIDE>
+// SLICE: K elements of rows that are ld long (forms of their own: what that takes costs small calls 0.2 us of 3.8, K = 21).
+template <int G, int KPL, bool RAGGED, bool WIDE, bool SLICE = false>
 __global__ __launch_bounds__(kRowGatherBlock)
 void sddmm_gather_kernel(const KArgs a)
 {
@@ -103,7 +111,7 @@ void sddmm_gather_kernel(const KArgs a)
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l = lane & (G - 1);
-    const int K = a.K, ld = a.ld;
+    const int K = a.K, ld = SLICE ? a.ld : K;
     const uint64_t le = (lane == 63) ? ~0ull : ((2ull << lane) - 1ull);
 
     int off[KPL];
@@ -214,7 +222,7 @@ void sddmm_gather_kernel(const KArgs a)
             }(), ...);
         }(std::make_integer_sequence<int, G>{});
         transpose_reduce_step<G>(acc, l);
-        if (begin + (bi << 6) + lane < end) finish(a, cur.p, cur.v, acc[0]);
+        if (begin + (bi << 6) + lane < end) finish<SLICE>(a, cur.p, cur.v, acc[0]);
         cur = nxt;
         nxt = after;
         changed = changed_next;
@@ -227,7 +235,7 @@ void sddmm_gather_kernel(const KArgs a)
 // us per launch from a graph, the kernel above and this one: 18 thousand nonzeros, K = 16 / 32 / 64 / 128: 3.8 / 4.6 / 4.7 / 5.1
 // and 3.0 / 3.3 / 3.6 / 4.4; R-MAT, 1.86 million, K = 32 / 100 / 256: 43 / 86 / 257 and 30 / 77 / 230.  Where it is chosen:
 // gather_shape.
-template <int G, int KPL, bool RAGGED, bool WIDE>
+template <int G, int KPL, bool RAGGED, bool WIDE, bool SLICE = false>
 __global__ __launch_bounds__(kRowGatherBlock)
 void sddmm_gather_once_kernel(const KArgs a)
 {
@@ -237,7 +245,7 @@ void sddmm_gather_once_kernel(const KArgs a)
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l = lane & (G - 1);
-    const int K = a.K, ld = a.ld;
+    const int K = a.K, ld = SLICE ? a.ld : K;
     const int batch = blockIdx.x * (kRowGatherBlock / 64) + wave;
     const int p0 = batch << 6;
     if (p0 >= a.nnz) return;
@@ -301,7 +309,7 @@ void sddmm_gather_once_kernel(const KArgs a)
         (round(std::integer_sequence<int, R * ROUND>{}, std::make_integer_sequence<int, ROUND>{}), ...);
     }(std::make_integer_sequence<int, G / ROUND>{});
     transpose_reduce_step<G>(acc, l);
-    if (p0 + lane < a.nnz) finish(a, p, v, acc[0]);
+    if (p0 + lane < a.nnz) finish<SLICE>(a, p, v, acc[0]);
 }
 
 // Any K >= 1 (used below 4 and beyond 2048): 8 lanes per nonzero striding over the row one float at a time,
@@ -460,6 +468,15 @@ int gather_slice(int64_t nnz, int64_t n_cols, int K)
     return nnz >= std::max(least, 4 * n_cols) && n_cols >= (K == 256 ? 24000 : 11000) ? 64 : K;
 }
 
+// the kernel for slices of 64 elements
+static KernelFn gather_slice_kernel(const Variant &v, bool once, bool wide)
+{
+    if (v.G == 16 && v.KPL == 1 && once) return wide ? (KernelFn)sddmm_gather_once_kernel<16, 1, false, true, true> : (KernelFn)sddmm_gather_once_kernel<16, 1, false, false, true>;
+    if (v.G == 8 && v.KPL == 2 && once) return wide ? (KernelFn)sddmm_gather_once_kernel<8, 2, false, true, true> : (KernelFn)sddmm_gather_once_kernel<8, 2, false, false, true>;
+    if (v.G == 8 && v.KPL == 2) return wide ? (KernelFn)sddmm_gather_kernel<8, 2, false, true, true> : (KernelFn)sddmm_gather_kernel<8, 2, false, false, true>;
+    return nullptr;
+}
+
 // One launch over whole rows, fn of shape's form, or one per slice.
 hipError_t launch_row_gather(KArgs a, KernelFn fn, int64_t listed_rows, int64_t n_rows, bool wide, int slice, void *stream)
 {
@@ -471,13 +488,13 @@ hipError_t launch_row_gather(KArgs a, KernelFn fn, int64_t listed_rows, int64_t 
     const uintptr_t v = (uintptr_t)(a.sval ? a.sval : a.val), o = (uintptr_t)a.out, bytes = (uintptr_t)a.nnz * 4;
     if (slice >= K || (v && v < o + bytes && o < v + bytes)) return run(fn);
     const float *W = a.W, *H = a.H;
+    a.K = slice;
+    const GatherShape s = gather_shape(a.nnz, n_rows, listed_rows, slice);
+    a.chunk = s.chunk;
     for (int k = 0; k < K; k += slice) {
-        a.K = std::min(slice, K - k);
         a.W = W + k; a.H = H + k;
         a.add = k > 0; a.part = k + slice < K;
-        const GatherShape s = gather_shape(a.nnz, n_rows, listed_rows, a.K);
-        a.chunk = s.chunk;
-        if (hipError_t e = run(gather_kernel(s.v, s.once, wide))) return e;
+        if (hipError_t e = run(gather_slice_kernel(s.v, s.once, wide))) return e;
     }
     return hipSuccess;
 }
