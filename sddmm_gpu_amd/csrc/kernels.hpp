@@ -255,8 +255,14 @@ inline bool gather_wide(int64_t n_rows, int64_t n_cols, int K) { return std::max
 KernelFn gather_kernel(const Variant &v, bool once, bool wide);
 KernelFn generic_kernel();           // row gather, any K
 int gather_slice(int64_t nnz, int64_t n_cols, int K);  // elements of a row per launch over all of a matrix
-// the row gather over a.nnz nonzeros on `stream`: fn over whole rows in workgroups of a.chunk, or slice by slice
-hipError_t launch_row_gather(KArgs a, KernelFn fn, int64_t listed_rows, int64_t n_rows, bool wide, int slice, void *stream);
+// Do values lie where the results go?  The first slice's dot products would overwrite them: rows are taken whole then.
+inline bool values_in_results(const KArgs &a)
+{
+    const uintptr_t v = (uintptr_t)(a.sval ? a.sval : a.val), o = (uintptr_t)a.out, bytes = (uintptr_t)a.nnz * 4;
+    return v && v < o + bytes && o < v + bytes;
+}
+// the row gather over a.nnz nonzeros of a matrix of n_rows rows, listed_rows of them with a nonzero, on `stream`, slice by slice
+hipError_t launch_gather_slices(KArgs a, int64_t listed_rows, int64_t n_rows, bool wide, int slice, void *stream);
 Variant pick_stream_variant(int K);  // unpadded LDS tile (K % 4 == 0)
 KernelFn stream_kernel(const Variant &v);
 

@@ -477,24 +477,20 @@ static KernelFn gather_slice_kernel(const Variant &v, bool once, bool wide)
     return nullptr;
 }
 
-// One launch over whole rows, fn of shape's form, or one per slice.
-hipError_t launch_row_gather(KArgs a, KernelFn fn, int64_t listed_rows, int64_t n_rows, bool wide, int slice, void *stream)
+hipError_t launch_gather_slices(KArgs a, int64_t listed_rows, int64_t n_rows, bool wide, int slice, void *stream)
 {
-    const hipStream_t st = (hipStream_t)stream;
-    auto run = [&](KernelFn f) { return launch(f, dim3((unsigned)((a.nnz + (int64_t)a.chunk - 1) / a.chunk)), dim3(kRowGatherBlock), 0, st, a); };
     const int K = a.K;
-    a.ld = K;
-    // (values that lie where the results go would be overwritten by the first slice's)
-    const uintptr_t v = (uintptr_t)(a.sval ? a.sval : a.val), o = (uintptr_t)a.out, bytes = (uintptr_t)a.nnz * 4;
-    if (slice >= K || (v && v < o + bytes && o < v + bytes)) return run(fn);
     const float *W = a.W, *H = a.H;
-    a.K = slice;
     const GatherShape s = gather_shape(a.nnz, n_rows, listed_rows, slice);
+    const KernelFn fn = gather_slice_kernel(s.v, s.once, wide);
+    a.ld = K;
+    a.K = slice;
     a.chunk = s.chunk;
-    for (int k = 0; k < K; k += slice) {
+    const dim3 grid((unsigned)((a.nnz + (int64_t)a.chunk - 1) / a.chunk));
+    for (int k = 0; k < K; k += slice) {  // (slices divide K)
         a.W = W + k; a.H = H + k;
         a.add = k > 0; a.part = k + slice < K;
-        if (hipError_t e = run(gather_slice_kernel(s.v, s.once, wide))) return e;
+        if (hipError_t e = launch(fn, grid, dim3(kRowGatherBlock), 0, (hipStream_t)stream, a)) return e;
     }
     return hipSuccess;
 }

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include "internal.hpp"
 #include "kernels.hpp"
+#include "launch.hpp"
 
 using namespace sddmm;
 
@@ -25,10 +26,18 @@ extern "C" int sddmm_csr_noalloc(int64_t n_rows, int64_t n_cols, int64_t nnz, co
     a.col_ind = d_col_ind; a.val = d_val; a.W = d_W; a.H = d_H; a.out = d_out;
     a.row_ptr = d_row_ptr; a.n_rows = (int32_t)n_rows;
     a.nnz = (int32_t)nnz; a.K = K; a.n_cols = (int32_t)n_cols; a.tile_x = (int32_t)n_cols;
-    const GatherShape shape = gather_shape(nnz, n_rows, n_rows, K);
-    const KernelFn fn = shape.v.G ? gather_kernel(shape.v, shape.once, gather_wide(n_rows, n_cols, K)) : generic_kernel();
-    a.chunk = shape.chunk;
-    const hipError_t e = launch_row_gather(a, fn, n_rows, n_rows, gather_wide(n_rows, n_cols, K), gather_slice(nnz, n_cols, K), stream);
+    const bool wide = gather_wide(n_rows, n_cols, K);
+    const int slice = gather_slice(nnz, n_cols, K);
+    hipError_t e;
+    if (slice < K && !values_in_results(a)) {
+        e = launch_gather_slices(a, n_rows, n_rows, wide, slice, stream);
+    } else {
+        const GatherShape shape = gather_shape(nnz, n_rows, n_rows, K);
+        const KernelFn fn = shape.v.G ? gather_kernel(shape.v, shape.once, wide) : generic_kernel();
+        a.chunk = shape.chunk;
+        const int grid = (int)((nnz + a.chunk - 1) / a.chunk);
+        e = launch(fn, dim3((unsigned)grid), dim3(kRowGatherBlock), 0, (hipStream_t)stream, a);
+    }
     if (e != hipSuccess) return fail(SDDMM_ERR_HIP, "sddmm_csr_noalloc: launch failed: %s", hipGetErrorString(e));
     return SDDMM_OK;
 }
