@@ -57,15 +57,17 @@ struct SoftmaxScale {
 // most of the time there, and a second turn of workgroups pays for it again.  us of the kernel alone with 4096 shares at
 // least and at most: rows of 14, 0.23 million entries 9.8 and 6.0; of 900, 0.9 million 11.4 and 7.4; of 40, 1.2 million 10.0
 // and 7.9; R-MAT, 0.24 / 0.69 / 1.3 million 10.7 / 14.5 / 15.0 and 9.2 / 10.4 / 14.3, but 1.86 million (2.4 on the scale) 15.5
-// and 18.2.
+// and 18.2.  (By counting zeros: in two loops that double the share it cost the workgroups of a large grid that find no unit
+// more than launching them.  4 million empty rows, softmax and merge, with loops 23.4 us, so 19.2; two million rows of one 26.1 and 24.4.)
 __host__ __device__ inline SoftmaxScale softmax_scale(int64_t nnz, int64_t n_rows)
 {
     SoftmaxScale s;
     s.row = n_rows <= (int64_t)1 << 27 ? kSmRow : 1;
     s.total = nnz + s.row * n_rows;
-    s.share = 64;
-    while (s.share < 512 && s.total > (int64_t)4096 * s.share) s.share *= 2;
-    while (s.share < kSmShareMax && s.total >= (int64_t)4096 * 2 * s.share) s.share *= 2;
+    const uint64_t t = s.total > 2 ? s.total : 2;
+    // (log2 of a 4096th of the scale, rounded up and down)
+    const int up = 64 - __builtin_clzll(t - 1) - 12, down = 63 - __builtin_clzll(t) - 12;
+    s.share = 1 << (down < 10 ? (up < 6 ? 6 : up < 9 ? up : 9) : down < 13 ? down : 13);
     return s;
 }
 
@@ -205,14 +207,16 @@ __device__ __forceinline__ void softmax_long_row(const float *x, float *out, int
     // (the next row writes its maxima after this row's second barrier and its sums after its own first: no barrier needed here)
 }
 
-// 64 rows by a wave: the lane's one has len entries from rb on (0: none, or not to be done here; at most kSmByWave), and
-// rows of up to by_lane entries have a lane each.
-__device__ __forceinline__ void softmax_row_batch(const float *x, float *out, int rb, int len, int lane, int by_lane)
+// 64 rows by a wave: the lane's one has len entries from rb on (0: none, or not to be done here; at most kSmByWave).
+// few: rows of up to kSmByLane entries go with the next longer ones where that saves a pass.
+__device__ __forceinline__ void softmax_row_batch(const float *x, float *out, int rb, int len, int lane, bool few)
 {
+    const uint64_t by_lane = __ballot(len >= 1 && len <= kSmByLane);
+    uint64_t todo = __ballot(len > kSmByLane && len <= kSmBy8);
     // a lane per row
-    if (__ballot(len >= 1 && len <= by_lane)) softmax_row_by_group<1, kSmByLane>(x + rb, out + rb, len, len <= by_lane);
+    if (few && (__builtin_popcountll(todo) + 7) / 8 >= (__builtin_popcountll(by_lane | todo) + 7) / 8) todo |= by_lane;
+    else if (by_lane) softmax_row_by_group<1, kSmByLane>(x + rb, out + rb, len, len <= kSmByLane);
     // groups of 8 lanes: eight rows at a time
-    uint64_t todo = __ballot(len > by_lane && len <= kSmBy8);
     while (todo) {
         int src = -1;  // the lane that holds the row of this lane's group
 #pragma unroll
@@ -272,17 +276,19 @@ void sddmm_row_softmax_kernel(const int32_t *__restrict__ row_ptr, int64_t n_row
 {
     __shared__ float red[2 * kSmWaves];
     // rows that the waves leave to the workgroup: row, first entry, length (read once more from the row pointers, and the row
-    // that began before the unit looked up there by all, they cost units without any such row 3 us)
+    // that began before the unit looked up there by all waves, they cost units without any such row 3 us)
     __shared__ int3 left[kSmWaves * kSmLeft + 1];
     __shared__ int n_left;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n_rows = (int)n_rows_, nnz = row_ptr[n_rows];
     const SoftmaxScale scale = softmax_scale(nnz, n_rows);
     const int64_t unit = scale.unit(), n_units = scale.units(), piece = scale.piece();
-    // (a share of 64 starts sixteen rows at most: two passes of groups of 8, and another kind of pass before them is one more
-    // chain of loads and sums.  18 thousand entries in 4096 rows, R-MAT: 6.4 us and 5.9; where sixteen rows or fewer are at
-    // hand in larger shares, 3.5 million: 20.9 and 22.5)
-    const int by_lane = scale.share == 64 ? 0 : kSmByLane;
+    // (A share of 64 starts sixteen rows at most, two passes of groups of 8: a pass of lanes before them is one more chain of loads and
+    // sums where it saves none of theirs, and one less where it does.  us of softmax and merge, a lane per short row never, always
+    // and by that rule: R-MAT of 1024 rows, 25 / 36 thousand entries 7.9 / 7.9, 8.4 / 8.4 and 8.0 / 7.9; 4096 rows, 29 / 117 thousand 7.9 /
+    // 8.7, 8.3 / 9.1 and 8.0 / 8.6 (18 thousand 7.8, 7.5 and 7.7); 20 thousand rows of one 8.3, 6.4 and 6.6.  In larger shares always:
+    // 3.5 million, R-MAT, 20.9, never 22.5.)
+    const bool few = scale.share == 64;
     const bool vec_in = (reinterpret_cast<uintptr_t>(x) & 15u) == 0, vec_out = (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
     for (int64_t u = blockIdx.x; u < n_units; u += gridDim.x) {
         const int64_t k0 = u * unit, k1 = min(scale.total, k0 + unit);
@@ -293,16 +299,19 @@ void sddmm_row_softmax_kernel(const int32_t *__restrict__ row_ptr, int64_t n_row
         const int64_t s0 = k0 + wave * scale.share, s1 = min(k1, s0 + scale.share);
         if (s0 < s1) {
             const int r0 = softmax_row_at(row_ptr, n_rows, scale.row, s0, lane);
-            for (int64_t w0 = r0;; w0 += 64) {
-                const int64_t r = w0 + lane;
-                const int rb = row_ptr[min(r, (int64_t)n_rows)], re = row_ptr[min(r + 1, (int64_t)n_rows)];
-                const int64_t at = rb + scale.row * r;
+            if (wave == 0) {  // (the row that began before the unit, if it is a huge one that goes on in it)
+                const int rb = row_ptr[r0], re = row_ptr[r0 + 1];
+                const int64_t at = rb + (int64_t)scale.row * r0;
+                if (re - rb > kSmLongMax && at < k0 && at + (re - rb) > k0 && lane == 0) left[atomicAdd(&n_left, 1)] = make_int3(r0, rb, re - rb);
+            }
+            for (uint32_t w0 = r0;; w0 += 64) {
+                const uint32_t r = w0 + lane;
+                const int rb = row_ptr[min(r, (uint32_t)n_rows)], re = row_ptr[min(r + 1, (uint32_t)n_rows)];
+                const int64_t at = rb + (int64_t)scale.row * r;
                 const int len = at >= s0 && at < s1 ? re - rb : 0;  // (r0 may begin before the share)
-                // (and the row that began before the unit, if it is a huge one that goes on in it)
-                const bool goes_on = wave == 0 && at < k0 && re - rb > kSmLongMax && at + (re - rb) > k0;
-                if (len > kSmByWave || goes_on) left[atomicAdd(&n_left, 1)] = make_int3((int)r, rb, re - rb);
-                softmax_row_batch(x, out, rb, len > kSmByWave ? 0 : len, lane, by_lane);
-                if (__ballot(r >= n_rows || at >= s1)) break;
+                if (len > kSmByWave) left[atomicAdd(&n_left, 1)] = make_int3((int)r, rb, re - rb);
+                softmax_row_batch(x, out, rb, len > kSmByWave ? 0 : len, lane, few);
+                if (__ballot(r >= (uint32_t)n_rows || at >= s1)) break;
             }
         }
         __syncthreads();

@@ -53,6 +53,22 @@ def test_special_values_stay_in_their_row(oracle, at, value):
         assert np.isnan(got[touched]).sum() >= 1
 
 
+# Short rows alone and among longer ones in shares of 64, both sides of the scale's lines between shares (entries + 4 rows = 2^18,
+# 2^19, 2^20, 2^22), and the smallest matrices.
+@pytest.mark.parametrize("lens", [[0], [1], [1, 0, 0, 2], [1] * 3000, [8] * 3000, [8, 8, 8, 8, 8, 20, 20, 20] * 200, [8, 8, 8, 8, 8, 8, 20, 20, 20] * 200,
+                                  [1, 9, 1, 1, 1, 1, 1, 1, 1, 1, 1] * 200, [3, 0, 96, 0, 1, 97, 7, 513, 8, 9] * 40, [5] * 29126 + [6], [5] * 29126 + [7],
+                                  [28] * 16384, [28] * 16384 + [0], [28] * 32768, [28] * 32768 + [1], [60] * 65535 + [59], [60] * 65536])
+def test_short_rows_and_lines_between_shares(oracle, lens):
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    x = np.random.default_rng(len(lens)).normal(0, 4, rp[-1]).astype(np.float32)
+    xd, rpd = torch.from_numpy(x).cuda(), torch.from_numpy(rp).cuda()
+    out = torch.full((len(x) + 1,), float("nan"), device="cuda")
+    capi.row_softmax(len(lens), rpd.data_ptr(), xd.data_ptr() if len(x) else out.data_ptr(), out.data_ptr())
+    torch.cuda.synchronize()
+    softmax_ok(out[:-1].cpu().numpy(), oracle.row_softmax(rp, x))
+    assert bool(torch.isnan(out[-1]))
+
+
 # Pieces are 256 entries without filler rows and 2048 with them; a lane merges every 64th piece of a row.
 @pytest.mark.parametrize("filler,masked", [(0, [(0, 700)]), (0, [(16384, 18000)]), (0, [(0, 19999)]), (0, [(500, 20000)]),
                                            (1200000, [(0, 5000)]), (1200000, [(0, 9000), (12000, 20000)])])
