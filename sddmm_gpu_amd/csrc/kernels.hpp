@@ -158,9 +158,9 @@ bool spmm_tile_supported(int k_slice);
 int spmm_tile_set_lds(int k_slice, int nwaves, bool ragged, int lds_bytes);  // 0 ok, 1 no such variant, 2 HIP error
 void launch_spmm_slice(const SpmmArgs &a, int k_slice, int nwaves, int grid, int lds_bytes, void *stream);
 
-// The product over a plain CSR pattern without atomics (K >= 4, kernels_spmm_csr.hip): d_part holds spmm_csr_records(nnz, n_cols, K)
+// The product over a plain CSR pattern without atomics (K >= 4, kernels_spmm_csr.hip): d_part holds spmm_csr_records(nnz, n_rows, n_cols, K)
 // rows of K floats.  Returns an SDDMM_* code.
-int64_t spmm_csr_records(int64_t nnz, int64_t n_cols, int K);
+int64_t spmm_csr_records(int64_t nnz, int64_t n_rows, int64_t n_cols, int K);
 int launch_spmm_csr_records(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *d_row_ptr, const int32_t *d_col_ind, const float *d_x, int32_t K,
                             const float *d_H, float *d_Y, float *d_part, void *stream);
 

@@ -33,20 +33,23 @@ namespace {
 
 constexpr int kSpmmMost = 512;  // nonzeros of a wave at most
 constexpr int kSpmmUnroll = 4;  // H pieces requested together
+constexpr int kMostSlices = 65535;  // (a grid's second dimension)
 constexpr uint32_t kRowChange = 0x80000000u;
 
 // Zeroes the rows of Y that the product adds to or leaves out: empty rows, and rows cut between workgroups (of 2^shift nonzeros).
-// A wave looks at 64 rows, or fewer as in the kernel below: a small matrix of long rows of H has 16 to 64 nonzeros to a workgroup,
-// so nearly all of its rows are cut.  us with 64 rows a wave and so: 1024 rows, K = 256 6.0 and 2.3; 4096,
-// K = 384 10.0 and 3.3; 32,768, K = 192 7.2 and 5.6.
+// A wave looks at 64 rows, or (2^rows_log2) at fewer as in the kernel below: a small matrix of long rows of H has 16 to 64 nonzeros
+// to a workgroup, so nearly all of its rows are cut.  us with 64 rows a wave and so: 1024 rows, K = 256 6.0 and 2.3;
+// 4096, K = 384 10.0 and 3.3; 32,768, K = 192 7.2 and 5.6; with the product, 18 thousand nonzeros of 4096 rows, R-MAT, K = 16 / 32 / 64 /
+// 100 7.0 / 7.2 / 8.5 / 9.6 and 6.8 / 6.9 / 7.8 / 8.2.  (Where few rows are cut there is nothing to gain: uniform, 0.2 million of 20,000
+// rows, K = 16 / 32 / 64 7.9 / 8.1 / 10.2 and 8.0 / 8.3 / 10.4.)
 __global__ __launch_bounds__(256)
-void sddmm_spmm_zero_rows_kernel(const int32_t *__restrict__ row_ptr, float *Y, int64_t n_rows, int K, int shift, int rows_per_wave)
+void sddmm_spmm_zero_rows_kernel(const int32_t *__restrict__ row_ptr, float *Y, uint32_t n_rows, int K, int shift, int rows_log2)
 {
     __shared__ int list[4][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t r = lane < rows_per_wave ? ((int64_t)blockIdx.x * 4 + wave) * rows_per_wave + lane : n_rows;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t r = ((blockIdx.x * 4 + wave) << rows_log2) + lane;
     bool zero = false;
-    if (r < n_rows) {
+    if (r < n_rows && lane >> rows_log2 == 0) {
         const int s = row_ptr[r], e = row_ptr[r + 1];
         zero = s >= e || (s >> shift) != ((e - 1) >> shift);
     }
@@ -341,39 +344,51 @@ struct CsrShape {
 // Pieces of four floats in a slice of a row, at most.  The slices of H follow each other over the whole matrix (the grid's
 // second dimension), so a slice that fits a die's 4 MB of L2 is gathered from there, and the columns and values read once
 // more per slice, 8 bytes a nonzero, cost less than that gives.  Where rows lie on lines of 128 bytes (K a multiple of 32):
-// the widest slices of 32, 16 or 8 pieces that divide a row and fit, at least 16 below 1.5 million nonzeros; whole rows where H
-// fits as a whole, and at narrow ranks where there is too little to gain.  us, whole rows (two slices beyond K = 256) and so:
-// band of 11.6 million in +-600 columns, K = 64 / 128 / 512 290 / 708 / 3067 and 193 / 385 / 1503; uniform, 3 million of 17,000
+// the widest slices of 32, 16 or 8 pieces that divide a row and fit, at least 16 below 1.5 million nonzeros, or the narrowest where
+// none fits; whole rows where H fits as a whole, and at narrow ranks where there is too little to gain.  us, whole rows (two
+// slices beyond K = 256) and so: band of 11.6 million in +-600 columns, K = 64 / 128 / 512 290 / 708 / 3067 and 193 / 385 / 1503; uniform, 3 million of 17,000
 // columns, K = 128 / 256 128 / 337 and 85 / 156; word counts of 10 million, K = 96 / 256 267 / 973 and 213 / 558; ratings of
 // 4.9 / 16.8 million, K = 256 225 / 1076 and 186 / 642; R-MAT of 1.8 / 7.5 million, K = 256 250 / 1236 and 165 / 785; window of
-// 16,384 tokens, 5.2 million, K = 256 282 and 197.  Uniform over 400,000 columns, whose slices fit nowhere, loses 2 to 4 %
-// (K = 64 / 256, 4.7 million: 191 / 737 and 199 / 757).  Rows across lines of 128 bytes gain nothing up to K = 256 (a slice
+// 16,384 tokens, 5.2 million, K = 256 282 and 197.  Rows across lines of 128 bytes gain nothing up to K = 256 (a slice
 // touches one line more); beyond, slices of 32 or 16 pieces fill their lanes better than two of up to 64 (K = 300: ratings of 4.9
-// million 393 and 312, uniform of 3 million 579 and 440).  And few nonzeros: a group has 4 of them, so a workgroup of whole
-// rows has 16, and nearly every row of S is cut and added atomically; slices have more to a workgroup (14 thousand, K = 256 15.9
-// and 9.4).
-int slice_pieces_most(int64_t nnz, int64_t n_cols, int K)
+// million 393 and 312, uniform of 3 million 579 and 440).
+//   Beyond K = 512, where the rows of S are looked up once more per slice as well: band of 2.4 million, K = 1024 / 2048 1246 / 2468 and
+// 818 / 2151, ratings of 5 million 937 / 1845 and 745 / 1469, R-MAT 2^18, 2.9 million, K = 1024 2001 and 1469.
+//   Where not even slices of 8 pieces fit, it depends on how evenly the columns are used, which the call does not know: R-MAT of
+// 2^18 to 2^20 vertices gains at five uses a column or more (2.9 / 4.9 million, K = 256 465 / 1074 and 301 / 810), uniform over
+// 400,000 columns at 8 and 12 uses a column loses 3 to 8 % (4.7 million, K = 64 / 256 / 1024 174 / 673 / 2665 and 181 / 704 / 2833).  At
+// less than four uses (few_uses) slices of 8 pieces lose below K = 256 (R-MAT 2^20, 1.6 million, K = 128 / 192 216 / 304 and 231 /
+// 323, with 16 pieces 212 / 305; K = 96, 3.0 million of 1.5 million columns, 175 and 192), slices of 16 at K = 300 (uniform, 2
+// million of a million columns 1116 and 1175) and below 1 to 1.5 million nonzeros (1.3 million of 400,000 columns, K = 256 248 and 265; R-MAT 2^17,
+// 0.39 million, K = 512 129 and 141), and gain otherwise (R-MAT 2^20, 1.6 million, K = 256 / 512 488 / 1017 and 439 / 880).
+//   Few nonzeros: a group has 4 of them, so a workgroup of whole rows has 16, and nearly every row of S is cut and added
+// atomically; slices have more to a workgroup (14 thousand, K = 256 15.9 and 9.4).  Not where rows of S have next to no nonzeros
+// (16 to 64 thousand in 65,536 rows, R-MAT, K = 160 / 200 17.8-22.4 / 19.6-24.6 and 22.3-25.1 / 25.0-27.7), from fewer rows on where slices
+// of 16 pieces are not whole lines (uniform, 40 thousand in 30,000 rows, K = 200 16.1 and 19.0).
+int slice_pieces_most(int64_t nnz, int64_t n_rows, int64_t n_cols, int K)
 {
     constexpr int64_t kL2 = 4200000;
     const int pieces = (K + 3) / 4;
     const int64_t h = 16 * (int64_t)pieces * n_cols;
-    if (nnz <= 65536) return K >= 160 ? 16 : 64;
-    const int wide = K <= 256 ? 64 : 32;
-    if (nnz < 300000 || h <= kL2) return wide;
-    if (K % 32 != 0) return K > 256 && nnz >= 1500000 ? 16 : wide;
+    if (nnz <= 65536) return K >= 160 && n_rows <= (K % 64 == 0 ? 40000 : nnz * 2 / 3) && pieces <= 16 * kMostSlices ? 16 : 64;
+    const int wide = K <= 256 || pieces > 32 * kMostSlices ? 64 : 32;
+    if (nnz < 300000 || h <= kL2 || pieces > 8 * kMostSlices) return wide;
+    const bool few_uses = nnz < 4 * n_cols;
+    if (K % 32 != 0) return K > 256 && nnz >= 1500000 && !few_uses ? 16 : wide;
     if (K < 192 && (nnz < (K < 96 ? 4000000 : K < 128 ? 2000000 : 1500000) || h <= (K < 96 ? 20000000 : K < 128 ? 6000000 : kL2))) return wide;
+    if (few_uses && nnz < (K <= 256 ? 1500000 : 1000000)) return wide;
     int narrow = 0;  // the narrowest that divides a row
     for (int p : {32, 16, 8}) {
-        if (p >= pieces || pieces % p != 0 || (p == 8 && nnz < 1500000)) continue;
+        if (p >= pieces || pieces % p != 0 || (p == 8 && (nnz < 1500000 || (few_uses && K < 256)))) continue;
         narrow = p;
         if (16 * (int64_t)p * n_cols <= kL2) break;
     }
     return narrow ? narrow : wide;
 }
-CsrShape csr_shape(int64_t nnz, int64_t n_cols, int K)
+CsrShape csr_shape(int64_t nnz, int64_t n_rows, int64_t n_cols, int K)
 {
     CsrShape c;
-    const int pieces = (K + 3) / 4, most = slice_pieces_most(nnz, n_cols, K);
+    const int pieces = (K + 3) / 4, most = slice_pieces_most(nnz, n_rows, n_cols, K);
     c.slices = (pieces + most - 1) / most;
     c.slice_pieces = (pieces + c.slices - 1) / c.slices;
     c.G = 4;
@@ -419,12 +434,12 @@ int rows_per_wave(int64_t n_rows, int K)
 
 namespace sddmm {
 
-int64_t spmm_csr_records(int64_t nnz, int64_t n_cols, int K) { return K < 4 ? 0 : 2 * csr_shape(nnz, n_cols, K).workgroups; }
+int64_t spmm_csr_records(int64_t nnz, int64_t n_rows, int64_t n_cols, int K) { return K < 4 ? 0 : 2 * csr_shape(nnz, n_rows, n_cols, K).workgroups; }
 
 int launch_spmm_csr_records(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *d_row_ptr, const int32_t *d_col_ind, const float *d_x, int32_t K,
                             const float *d_H, float *d_Y, float *d_part, void *stream)
 {
-    const CsrShape c = csr_shape(nnz, n_cols, K);
+    const CsrShape c = csr_shape(nnz, n_rows, n_cols, K);
     hipStream_t st = (hipStream_t)stream;
     if (int rc = checked(launch_csr<true>(c, n_rows, n_cols, nnz, d_row_ptr, d_col_ind, d_x, K, d_H, d_Y, d_part, st))) return rc;
     const int per_wave = rows_per_wave(n_rows, K);
@@ -446,10 +461,10 @@ extern "C" int sddmm_spmm_csr(int64_t n_rows, int64_t n_cols, int64_t nnz, const
         const unsigned grid = (unsigned)std::min<int64_t>((n_rows + 3) / 4, 256 * 64);
         return checked(launch(sddmm_spmm_generic_kernel, dim3(grid), dim3(256), 0, st, d_row_ptr, d_col_ind, d_x, d_H, d_Y, n_rows, (int)K));
     }
-    const CsrShape c = csr_shape(nnz, n_cols, K);
+    const CsrShape c = csr_shape(nnz, n_rows, n_cols, K);
     const int per_wave = rows_per_wave(n_rows, K);
     if (int rc = checked(launch(sddmm_spmm_zero_rows_kernel, dim3((unsigned)((n_rows + 4 * per_wave - 1) / (4 * per_wave))), dim3(256), 0, st, d_row_ptr,
-                                d_Y, n_rows, (int)K, c.wg_shift, per_wave)))
+                                d_Y, (uint32_t)n_rows, (int)K, c.wg_shift, __builtin_ctz(per_wave))))
         return rc;
     if (nnz == 0) return SDDMM_OK;
     return checked(launch_csr<false>(c, n_rows, n_cols, nnz, d_row_ptr, d_col_ind, d_x, K, d_H, d_Y, nullptr, st));

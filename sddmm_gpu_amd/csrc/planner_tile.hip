@@ -943,7 +943,7 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         c.P->info.spmm_runs += (int64_t)sp.part_slot.size();
     }
     if (sp_csr) {
-        const int64_t records = spmm_csr_records(c.nnz, c.n_cols, c.K);
+        const int64_t records = spmm_csr_records(c.nnz, c.n_rows, c.n_cols, c.K);
         float *d_sp = nullptr;
         const size_t bytes = (size_t)records * c.K * 4;
         HIP_TRY(hipMalloc((void **)&d_sp, bytes));

@@ -59,3 +59,36 @@ def test_any_rank_on_awkward_patterns(oracle, kind, K):
     ref, mag = oracle.spmm_csr(rp, ci, val, H, with_abs=True)
     bound = 1e-5 * np.sqrt(np.maximum(np.diff(rp), 1))[:, None] * mag
     assert np.all(np.abs(Y.cpu().numpy().astype(np.float64) - ref) <= bound)
+
+
+# The slices of H's rows that the product takes in turn (slice_pieces_most in kernels_spmm_csr.hip): 8 pieces from 1.5 million nonzeros
+# on, two slices at K = 64 from 4 million and 20 MB of H on, 16 pieces at ranks beyond 256 across lines and where columns are used
+# less than four times, whole rows on the other side of those lines and where rows have next to no nonzeros.  Rows: lengths that differ,
+# every seventh empty.
+@pytest.mark.parametrize("n_rows,n_cols,nnz,K", [
+    (30000, 40000, 1500000, 192), (30000, 40000, 1499999, 192), (30000, 40000, 2000001, 96), (60000, 100000, 4000000, 64), (60000, 100000, 3999999, 64),
+    (20000, 20000, 1500001, 300), (20000, 20000, 1499999, 300), (20000, 400000, 1599999, 192), (20000, 400000, 1600000, 192), (20000, 400000, 1599999, 301),
+    (20000, 100000, 399999, 256), (20000, 100000, 400001, 256), (40000, 3000, 65536, 192), (40001, 3000, 65536, 192), (43690, 3000, 65536, 200),
+    (43692, 3000, 65536, 200), (3000, 3000, 65537, 192)])
+def test_product_in_slices_against_64_bits(n_rows, n_cols, nnz, K):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(nnz + K)
+    lens = torch.rand(n_rows, generator=g, device="cuda") ** 2
+    lens[torch.arange(n_rows, device="cuda") % 7 == 3] = 0
+    rows = torch.searchsorted(torch.cumsum(lens, 0) / lens.sum(), torch.rand(nnz, generator=g, device="cuda")).clamp_(max=n_rows - 1).sort().values
+    rp = torch.zeros(n_rows + 1, dtype=torch.int64, device="cuda")
+    rp[1:] = torch.cumsum(torch.bincount(rows, minlength=n_rows), 0)
+    ci = torch.randint(0, n_cols, (nnz,), generator=g, device="cuda")  # (any order, pairs may repeat: the product allows it)
+    x, H = torch.randn(nnz, generator=g, device="cuda"), torch.randn(n_cols, K, generator=g, device="cuda")
+    rp32, ci32 = rp.int(), ci.int()
+    Y = torch.full((n_rows, K), float("nan"), device="cuda")
+    capi.spmm_csr(n_rows, n_cols, nnz, rp32.data_ptr(), ci32.data_ptr(), x.data_ptr(), K, H.data_ptr(), Y.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    for k in range(0, K, 64):
+        want = torch.zeros(n_rows, min(64, K - k), dtype=torch.float64, device="cuda")
+        mag = torch.zeros_like(want)
+        for i in range(0, nnz, 1 << 19):
+            part = x[i:i + (1 << 19), None].double() * H[ci[i:i + (1 << 19)], k:k + 64].double()
+            want.index_add_(0, rows[i:i + (1 << 19)], part)
+            mag.index_add_(0, rows[i:i + (1 << 19)], part.abs())
+        bound = 1e-5 * torch.diff(rp).clamp(min=1).double().sqrt()[:, None] * mag
+        assert bool(((Y[:, k:k + 64].double() - want).abs() <= bound).all())
