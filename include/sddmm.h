@@ -493,8 +493,8 @@ int sddmm_plan_release_host(const sddmm_plan *plan);
  * pay.  Same result as
  * sddmm_plan_create_device(..., SDDMM_KERNEL_ROW_GATHER) + sddmm_execute, bit
  * for bit: the row-gather kernel in one launch, at K = 256, 448 and 512 on large
- * matrices one per 64 elements of K with the sums so far in d_out (unless d_val lies
- * there: those may differ in the last bits), every wave finding the rows of its
+ * matrices one per 64 elements of K with the sums so far in d_out (where d_val lies
+ * there, one that keeps them to itself), every wave finding the rows of its
  * nonzeros from the row pointers.  All pointers are device pointers; d_val may be
  * NULL (out[p] = dot).  The pattern is not validated (that would need a copy
  * to the host): d_row_ptr must be monotone with d_row_ptr[0] = 0 and

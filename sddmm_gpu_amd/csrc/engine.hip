@@ -192,7 +192,7 @@ static hipError_t issue_launch(const sddmm_plan *plan, const Launch &L, const fl
         a.sval = d_val ? nullptr : L.sval;
         a.W = d_W; a.H = d_H; a.out = d_out;
         a.residual = residual;
-        if (L.fn_kind == 1 && L.k_slice < I.K && !values_in_results(a)) return launch_gather_slices(a, L.rows, I.n_rows, L.fn_wide != 0, L.k_slice, stream);
+        if (L.fn_kind == 1 && L.k_slice < I.K) return launch_gather_slices(a, L.rows, I.n_rows, L.fn_wide != 0, L.k_slice, stream);
         return launch(L.fn, dim3((unsigned)L.grid), dim3((unsigned)L.block), (size_t)L.lds, stream, a);
     }
 }

@@ -36,7 +36,7 @@ struct KArgs {
     // Plan-free form (batch_seg and batch_mask are null then): the rows are found from the row pointers.
     const int32_t *row_ptr;    // [n_rows+1]
     int32_t n_rows;
-    // Row gather: W and H begin at the first element of a slice of K elements of rows that are ld long.
+    // Row gather in slices: W and H begin at the first element of a slice of K elements of rows that are ld long.
     int32_t ld;
     int32_t add, part;         // add: out holds the dot product of the slices before; part: slices follow (out = dot)
 };
@@ -255,14 +255,10 @@ inline bool gather_wide(int64_t n_rows, int64_t n_cols, int K) { return std::max
 KernelFn gather_kernel(const Variant &v, bool once, bool wide);
 KernelFn generic_kernel();           // row gather, any K
 int gather_slice(int64_t nnz, int64_t n_cols, int K);  // elements of a row per launch over all of a matrix
-// Do values lie where the results go?  The first slice's dot products would overwrite them: rows are taken whole then.
-inline bool values_in_results(const KArgs &a)
-{
-    const uintptr_t v = (uintptr_t)(a.sval ? a.sval : a.val), o = (uintptr_t)a.out, bytes = (uintptr_t)a.nnz * 4;
-    return v && v < o + bytes && o < v + bytes;
-}
-// the row gather over a.nnz nonzeros of a matrix of n_rows rows, listed_rows of them with a nonzero, on `stream`, slice by slice
+// the row gather over a.nnz nonzeros of a matrix of n_rows rows, listed_rows of them with a nonzero, on `stream`: slice by slice, a
+// launch each, or one launch that takes all slices where values lie where the results go; and which of the two it is
 hipError_t launch_gather_slices(KArgs a, int64_t listed_rows, int64_t n_rows, bool wide, int slice, void *stream);
+int gather_slice_launches(const KArgs &a, int slice);
 Variant pick_stream_variant(int K);  // unpadded LDS tile (K % 4 == 0)
 KernelFn stream_kernel(const Variant &v);
 

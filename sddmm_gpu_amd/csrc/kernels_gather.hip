@@ -86,11 +86,16 @@ __device__ __forceinline__ vec4u row_piece_of(const float *m, uint32_t at, int o
     else return *reinterpret_cast<const vec4u *>(reinterpret_cast<const char *>(m) + ((at << 2) + ((uint32_t)off << 2)));
 }
 
-// The dot product of sorted position p, complete or (SLICE) a slice's share of it.
-template <bool SLICE>
+// What a launch takes of the rows: all K elements at once; K elements of rows that are ld long, the dot products so far in out; all
+// of those slices one after the other, the dot products so far in the kernel (values lie where the results go then, see
+// launch_gather_slices).  Every dot product is added up in the same order in the last two.
+enum class Take { Rows, Slice, Slices };
+
+// The dot product of sorted position p, complete or a slice's share of it.
+template <Take TAKE>
 __device__ __forceinline__ void finish(const KArgs &a, int p, float v, float dot)
 {
-    if constexpr (SLICE) {
+    if constexpr (TAKE == Take::Slice) {
         if (a.add) dot += a.out[p];
         if (a.part) {
             a.out[p] = dot;
@@ -101,17 +106,19 @@ __device__ __forceinline__ void finish(const KArgs &a, int p, float v, float dot
 }
 
 // RAGGED: K is not 4 * G * KPL (its pieces are masked; any K > 4 * G * (KPL - 1) up to 4 * G * KPL, K >= 4).
-// SLICE: K elements of rows that are ld long (forms of their own: what that takes costs small calls 0.2 us of 3.8, K = 21).
-template <int G, int KPL, bool RAGGED, bool WIDE, bool SLICE = false>
+// (Slices are forms of their own: what they take costs small calls 0.2 us of 3.8, K = 21.)
+template <int G, int KPL, bool RAGGED, bool WIDE, Take TAKE = Take::Rows>
 __global__ __launch_bounds__(kRowGatherBlock)
 void sddmm_gather_kernel(const KArgs a)
 {
     constexpr int NW = kRowGatherBlock / 64;
     __shared__ int row_tab[NW][64 * kRowGatherBatchesPerWave + 1];  // (plan-free form)
+    __shared__ float so_far[TAKE == Take::Slices ? NW : 1][TAKE == Take::Slices ? 64 * kRowGatherBatchesPerWave : 1];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l = lane & (G - 1);
-    const int K = a.K, ld = SLICE ? a.ld : K;
+    const int K = a.K, ld = TAKE == Take::Rows ? K : a.ld;
+    const float *W = a.W, *H = a.H;  // (their first elements that are taken)
     const uint64_t le = (lane == 63) ? ~0ull : ((2ull << lane) - 1ull);
 
     int off[KPL];
@@ -176,14 +183,14 @@ void sddmm_gather_kernel(const KArgs a)
         if (changed & (group_bits<G>() << I)) {
             const uint32_t wr = (uint32_t)group_bcast<G, I>(WIDE ? b.row : b.row * ld);
 #pragma unroll
-            for (int j = 0; j < KPL; ++j) w[I & 1][j] = row_piece_of<WIDE>(a.W, wr, off[j], ld);
+            for (int j = 0; j < KPL; ++j) w[I & 1][j] = row_piece_of<WIDE>(W, wr, off[j], ld);
         } else {
 #pragma unroll
             for (int j = 0; j < KPL; ++j) w[I & 1][j] = w[(I & 1) ^ 1][j];
         }
         const uint32_t hr = (uint32_t)group_bcast<G, I>(b.col);
 #pragma unroll
-        for (int j = 0; j < KPL; ++j) h[I & 1][j] = row_piece_of<WIDE>(a.H, hr, off[j], ld);
+        for (int j = 0; j < KPL; ++j) h[I & 1][j] = row_piece_of<WIDE>(H, hr, off[j], ld);
     };
     // rows of a batch that differ from the row before: inside a group the lane before, for its first lane the
     // group's row at the end of the batch before
@@ -193,39 +200,50 @@ void sddmm_gather_kernel(const KArgs a)
         return __ballot(b.row != before);
     };
 
-    Batch cur = load_batch(b0);
-    Batch nxt = load_batch(b0 + 1);
-    uint64_t changed = row_changes(cur, -1);
-    issue(std::integral_constant<int, 0>{}, cur, changed);
-    for (int bi = b0; bi < b1; ++bi) {
-        float acc[G];
-        const Batch after = load_batch(bi + 2);
-        const uint64_t changed_next = row_changes(nxt, group_bcast<G, G - 1>(cur.row));
-        [&]<int... I>(std::integer_sequence<int, I...>) {
-            ((void)[&] {
-                if constexpr (I + 1 < G) issue(std::integral_constant<int, I + 1>{}, cur, changed);
-                __builtin_amdgcn_sched_barrier(0);
-                float s = 0.f;
+    for (int k = 0;; k += K, W += K, H += K) {  // (once, but for Slices)
+        Batch cur = load_batch(b0);
+        Batch nxt = load_batch(b0 + 1);
+        uint64_t changed = row_changes(cur, -1);
+        issue(std::integral_constant<int, 0>{}, cur, changed);
+        for (int bi = b0; bi < b1; ++bi) {
+            float acc[G];
+            const Batch after = load_batch(bi + 2);
+            const uint64_t changed_next = row_changes(nxt, group_bcast<G, G - 1>(cur.row));
+            [&]<int... I>(std::integer_sequence<int, I...>) {
+                ((void)[&] {
+                    if constexpr (I + 1 < G) issue(std::integral_constant<int, I + 1>{}, cur, changed);
+                    __builtin_amdgcn_sched_barrier(0);
+                    float s = 0.f;
 #pragma unroll
-                for (int j = 0; j < KPL; ++j) {
-                    vec4u hv = h[I & 1][j], wv = w[I & 1][j];
-                    mask_piece(hv, j);
-                    mask_piece(wv, j);
-                    s = fmaf(wv.x, hv.x, s); s = fmaf(wv.y, hv.y, s);
-                    s = fmaf(wv.z, hv.z, s); s = fmaf(wv.w, hv.w, s);
-                }
-                asm volatile("" : "+v"(s));  // (computed here: left alone the compiler sinks it behind the branches of the later steps)
-                acc[I] = s;
-                // (the last step's: the next batch's first, requested before the reduction)
-                if constexpr (I + 1 == G) issue(std::integral_constant<int, 0>{}, nxt, changed_next);
-                __builtin_amdgcn_sched_barrier(0);
-            }(), ...);
-        }(std::make_integer_sequence<int, G>{});
-        transpose_reduce_step<G>(acc, l);
-        if (begin + (bi << 6) + lane < end) finish<SLICE>(a, cur.p, cur.v, acc[0]);
-        cur = nxt;
-        nxt = after;
-        changed = changed_next;
+                    for (int j = 0; j < KPL; ++j) {
+                        vec4u hv = h[I & 1][j], wv = w[I & 1][j];
+                        mask_piece(hv, j);
+                        mask_piece(wv, j);
+                        s = fmaf(wv.x, hv.x, s); s = fmaf(wv.y, hv.y, s);
+                        s = fmaf(wv.z, hv.z, s); s = fmaf(wv.w, hv.w, s);
+                    }
+                    asm volatile("" : "+v"(s));  // (computed here: left alone the compiler sinks it behind the branches of the later steps)
+                    acc[I] = s;
+                    // (the last step's: the next batch's first, requested before the reduction)
+                    if constexpr (I + 1 == G) issue(std::integral_constant<int, 0>{}, nxt, changed_next);
+                    __builtin_amdgcn_sched_barrier(0);
+                }(), ...);
+            }(std::make_integer_sequence<int, G>{});
+            transpose_reduce_step<G>(acc, l);
+            float dot = acc[0];
+            bool done = begin + (bi << 6) + lane < end;
+            if constexpr (TAKE == Take::Slices) {
+                float &sum = so_far[wave][((bi - b0) << 6) + lane];
+                if (k > 0) dot += sum;
+                sum = dot;
+                done = done && k + K == ld;
+            }
+            if (done) finish<TAKE>(a, cur.p, cur.v, dot);
+            cur = nxt;
+            nxt = after;
+            changed = changed_next;
+        }
+        if (TAKE != Take::Slices || k + K == ld) break;
     }
 }
 
@@ -235,7 +253,7 @@ void sddmm_gather_kernel(const KArgs a)
 // us per launch from a graph, the kernel above and this one: 18 thousand nonzeros, K = 16 / 32 / 64 / 128: 3.8 / 4.6 / 4.7 / 5.1
 // and 3.0 / 3.3 / 3.6 / 4.4; R-MAT, 1.86 million, K = 32 / 100 / 256: 43 / 86 / 257 and 30 / 77 / 230.  Where it is chosen:
 // gather_shape.
-template <int G, int KPL, bool RAGGED, bool WIDE, bool SLICE = false>
+template <int G, int KPL, bool RAGGED, bool WIDE, Take TAKE = Take::Rows>
 __global__ __launch_bounds__(kRowGatherBlock)
 void sddmm_gather_once_kernel(const KArgs a)
 {
@@ -245,7 +263,8 @@ void sddmm_gather_once_kernel(const KArgs a)
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l = lane & (G - 1);
-    const int K = a.K, ld = SLICE ? a.ld : K;
+    const int K = a.K, ld = TAKE == Take::Rows ? K : a.ld;
+    const float *W = a.W, *H = a.H;  // (their first elements that are taken)
     const int batch = blockIdx.x * (kRowGatherBlock / 64) + wave;
     const int p0 = batch << 6;
     if (p0 >= a.nnz) return;
@@ -286,10 +305,10 @@ void sddmm_gather_once_kernel(const KArgs a)
         ((void)[&] {
             const uint32_t hr = (uint32_t)group_bcast<G, BASE + I>(h_at);
 #pragma unroll
-            for (int j = 0; j < KPL; ++j) h[I][j] = row_piece_of<WIDE>(a.H, hr, off[j], ld);
+            for (int j = 0; j < KPL; ++j) h[I][j] = row_piece_of<WIDE>(H, hr, off[j], ld);
             const uint32_t wr = (uint32_t)group_bcast<G, BASE + I>(w_at);
 #pragma unroll
-            for (int j = 0; j < KPL; ++j) w[I][j] = row_piece_of<WIDE>(a.W, wr, off[j], ld);
+            for (int j = 0; j < KPL; ++j) w[I][j] = row_piece_of<WIDE>(W, wr, off[j], ld);
         }(), ...);
         __builtin_amdgcn_sched_barrier(0);
         ((void)[&] {
@@ -305,11 +324,16 @@ void sddmm_gather_once_kernel(const KArgs a)
             acc[BASE + I] = s;
         }(), ...);
     };
-    [&]<int... R>(std::integer_sequence<int, R...>) {
-        (round(std::integer_sequence<int, R * ROUND>{}, std::make_integer_sequence<int, ROUND>{}), ...);
-    }(std::make_integer_sequence<int, G / ROUND>{});
-    transpose_reduce_step<G>(acc, l);
-    if (p0 + lane < a.nnz) finish<SLICE>(a, p, v, acc[0]);
+    float dot = 0.f;
+    for (int k = 0;; k += K, W += K, H += K) {  // (once, but for Slices)
+        [&]<int... R>(std::integer_sequence<int, R...>) {
+            (round(std::integer_sequence<int, R * ROUND>{}, std::make_integer_sequence<int, ROUND>{}), ...);
+        }(std::make_integer_sequence<int, G / ROUND>{});
+        transpose_reduce_step<G>(acc, l);
+        dot = TAKE == Take::Slices && k > 0 ? acc[0] + dot : acc[0];
+        if (TAKE != Take::Slices || k + K == ld) break;
+    }
+    if (p0 + lane < a.nnz) finish<TAKE>(a, p, v, dot);
 }
 
 // Any K >= 1 (used below 4 and beyond 2048): 8 lanes per nonzero striding over the row one float at a time,
@@ -468,28 +492,40 @@ int gather_slice(int64_t nnz, int64_t n_cols, int K)
     return nnz >= std::max(least, 4 * n_cols) && n_cols >= (K == 256 ? 24000 : 11000) ? 64 : K;
 }
 
-// the kernel for slices of 64 elements
-static KernelFn gather_slice_kernel(const Variant &v, bool once, bool wide)
+// Do values lie where the results go?  The first slice's dot products would overwrite them.
+static bool values_in_results(const KArgs &a)
 {
-    if (v.G == 16 && v.KPL == 1 && once) return wide ? (KernelFn)sddmm_gather_once_kernel<16, 1, false, true, true> : (KernelFn)sddmm_gather_once_kernel<16, 1, false, false, true>;
-    if (v.G == 8 && v.KPL == 2 && once) return wide ? (KernelFn)sddmm_gather_once_kernel<8, 2, false, true, true> : (KernelFn)sddmm_gather_once_kernel<8, 2, false, false, true>;
-    if (v.G == 8 && v.KPL == 2) return wide ? (KernelFn)sddmm_gather_kernel<8, 2, false, true, true> : (KernelFn)sddmm_gather_kernel<8, 2, false, false, true>;
+    const uintptr_t v = (uintptr_t)(a.sval ? a.sval : a.val), o = (uintptr_t)a.out, bytes = (uintptr_t)a.nnz * 4;
+    return v && v < o + bytes && o < v + bytes;
+}
+
+int gather_slice_launches(const KArgs &a, int slice) { return values_in_results(a) ? 1 : a.K / slice; }
+
+// The kernel for slices of 64 elements.  gather_shape gives sixteen lanes of one piece with one batch a wave there, or eight of two with
+// several (slices begin far above the sizes where eight have one).
+template <Take TAKE>
+static KernelFn gather_slice_kernel(const GatherShape &s, bool wide)
+{
+    if (s.v.G == 16 && s.v.KPL == 1 && s.once) return wide ? (KernelFn)sddmm_gather_once_kernel<16, 1, false, true, TAKE> : (KernelFn)sddmm_gather_once_kernel<16, 1, false, false, TAKE>;
+    if (s.v.G == 8 && s.v.KPL == 2 && !s.once) return wide ? (KernelFn)sddmm_gather_kernel<8, 2, false, true, TAKE> : (KernelFn)sddmm_gather_kernel<8, 2, false, false, TAKE>;
     return nullptr;
 }
 
+// Values where the results go: one launch that takes the slices in turn keeps the sums so far in registers or LDS, so the results have
+// the same bits; its waves are at about the same slice, which brings part of what separate launches gain.  us, whole rows, slices in a
+// launch each and in one: R-MAT 2^17, 5.8 million, K = 256 / 512 767 / 1785, 600 / 1237 and 680 / 1537; ratings of 7.8 million, K = 256 / 448
+// 630 / 1337, 450 / 871 and 542 / 1108; band of 3 million, K = 448 717, 714 and 717.
 hipError_t launch_gather_slices(KArgs a, int64_t listed_rows, int64_t n_rows, bool wide, int slice, void *stream)
 {
-    const int K = a.K;
-    const float *W = a.W, *H = a.H;
     const GatherShape s = gather_shape(a.nnz, n_rows, listed_rows, slice);
-    const KernelFn fn = gather_slice_kernel(s.v, s.once, wide);
-    a.ld = K;
-    a.K = slice;
+    const int launches = gather_slice_launches(a, slice);
+    const KernelFn fn = launches == 1 ? gather_slice_kernel<Take::Slices>(s, wide) : gather_slice_kernel<Take::Slice>(s, wide);
+    a.ld = a.K;
+    a.K = slice;  // (divides it)
     a.chunk = s.chunk;
     const dim3 grid((unsigned)((a.nnz + (int64_t)a.chunk - 1) / a.chunk));
-    for (int k = 0; k < K; k += slice) {  // (slices divide K)
-        a.W = W + k; a.H = H + k;
-        a.add = k > 0; a.part = k + slice < K;
+    for (int i = 0; i < launches; ++i, a.W += slice, a.H += slice) {
+        a.add = i > 0; a.part = i + 1 < launches;
         if (hipError_t e = launch(fn, grid, dim3(kRowGatherBlock), 0, (hipStream_t)stream, a)) return e;
     }
     return hipSuccess;

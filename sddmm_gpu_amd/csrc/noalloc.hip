@@ -29,7 +29,7 @@ extern "C" int sddmm_csr_noalloc(int64_t n_rows, int64_t n_cols, int64_t nnz, co
     const bool wide = gather_wide(n_rows, n_cols, K);
     const int slice = gather_slice(nnz, n_cols, K);
     hipError_t e;
-    if (slice < K && !values_in_results(a)) {
+    if (slice < K) {
         e = launch_gather_slices(a, n_rows, n_rows, wide, slice, stream);
     } else {
         const GatherShape shape = gather_shape(nnz, n_rows, n_rows, K);

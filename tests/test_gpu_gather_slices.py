@@ -1,5 +1,5 @@
 """Row gather in slices of K (gather_slice in kernels_gather.hip): without and with a plan, from where the rule takes over,
-against 64 bits; every value mode; values that lie where the results go (whole rows then)."""
+against 64 bits; every value mode; values that lie where the results go (all slices in one launch then), bit for bit the same."""
 import pytest
 import torch
 
@@ -25,11 +25,13 @@ def make(n_rows, n_cols, nnz, K, seed):
 
 
 # On both sides of each line: nonzeros, columns, rank.  Slices: launches of a plan that gathers all rows.  40,000 and 300,000
-# rows: kernels with several batches a wave and with one.
+# rows: kernels with several batches a wave and with one; W or H beyond 4 GB: rows found
+# with 64-bit offsets.
 @pytest.mark.parametrize("n_rows,n_cols,nnz,K,slices", [
     (40000, 24000, 2500000, 256, 4), (300000, 25001, 2500003, 256, 4), (40000, 23999, 2500000, 256, 1), (40000, 24000, 2499999, 256, 1),
     (40000, 11000, 3000000, 448, 7), (40000, 11000, 2999999, 448, 1), (150000, 11000, 1400001, 512, 8), (40000, 11000, 1399999, 512, 1),
-    (9000, 350001, 1400003, 512, 1), (9000, 350000, 1400001, 512, 8), (40000, 24000, 3000000, 384, 1)])
+    (9000, 350001, 1400003, 512, 1), (9000, 350000, 1400001, 512, 8), (40000, 24000, 3000000, 384, 1),
+    (2101248, 11000, 1500001, 512, 8), (100000, 2101248, 8405000, 512, 8)])
 def test_slices_against_64_bits(n_rows, n_cols, nnz, K, slices):
     rp, ci, val, W, H, dot = make(n_rows, n_cols, nnz, K, K + slices)
     st = torch.cuda.current_stream().cuda_stream
@@ -48,6 +50,7 @@ def test_slices_against_64_bits(n_rows, n_cols, nnz, K, slices):
     close(out, val.double() * dot)
     plan.execute(p(val), p(W), p(H), p(out2), st)
     assert torch.equal(out, out2)
+    scaled = out.clone()
     noalloc(0, out)
     close(out, dot)
     plan.execute_epilogue(p(val), p(W), p(H), p(out2), capi.EPILOGUE_RESIDUAL, st)
@@ -55,7 +58,10 @@ def test_slices_against_64_bits(n_rows, n_cols, nnz, K, slices):
     for run in (lambda v: noalloc(p(v), v), lambda v: plan.execute(p(v), p(W), p(H), p(v), st)):
         v = val.clone()
         run(v)
-        close(v, val.double() * dot)
+        assert torch.equal(v, scaled)
+    v = val.clone()
+    plan.execute_epilogue(p(v), p(W), p(H), p(v), capi.EPILOGUE_RESIDUAL, st)
+    assert torch.equal(v, out2)
     plan.close()
 
 
