@@ -75,12 +75,13 @@ typedef struct sddmm_plan_info {
     int32_t K;
     int32_t tile_size_x;  /* columns of S (= rows of H) per LDS tile actually used */
     int32_t tile_size_y;  /* row-panel height actually used */
-    int32_t k_slice;      /* K elements of each H row a launch works on at a time (== K: no slicing) */
+    int32_t k_slice;      /* K elements of each H row a launch works on at a time (== K: no slices with partial
+                             results in the plan; a row gather may take slices all the same, with those in d_out) */
     int32_t n_col_tiles, n_row_panels; /* (n_row_panels: row panels of the stream; with tile_runs = 2 the
                                           row ranges, one per group of workgroups) */
     int32_t kernel;       /* SDDMM_KERNEL_* actually chosen (HYBRID: more than one launch) */
-    int32_t n_launches;   /* kernel launches per sddmm_execute */
-    int32_t lanes_per_nnz;
+    int32_t n_launches;   /* kernel launches per sddmm_execute (a row gather in slices: one where d_val lies in d_out) */
+    int32_t lanes_per_nnz; /* of the kernel that is launched */
     int32_t lds_bytes;    /* LDS per workgroup of the main kernel */
     int32_t grid, block;  /* launch shape of the main kernel */
     int64_t n_blocks;     /* (row panel, column tile) work items with at least one nonzero */
@@ -455,7 +456,7 @@ typedef struct sddmm_launch_profile {
     int32_t kernel;            /* SDDMM_KERNEL_ROW_GATHER / LDS_TILE / PANEL */
     int32_t lanes_per_nnz;
     int32_t k_slice;           /* K elements per kernel launch */
-    int32_t n_kernel_launches; /* K / k_slice */
+    int32_t n_kernel_launches; /* K / k_slice, or 1 where one launch takes all slices */
     int64_t nnz, rows;         /* nonzeros and rows this entry covers */
     int64_t stream_positions;  /* positions walked, padding included */
     float ms;

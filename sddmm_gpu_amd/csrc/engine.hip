@@ -120,6 +120,16 @@ static int check_execute_args(const sddmm_plan *plan, const float *d_W, const fl
     return SDDMM_OK;
 }
 
+// A row gather's or an unpadded tile's arguments: what it reads values from and writes to.
+static KArgs gather_args(const sddmm_plan *plan, const Launch &L, const float *d_val, float *d_out)
+{
+    KArgs a = L.ka;
+    a.val = d_val ? d_val : plan->d_val;
+    a.sval = d_val ? nullptr : L.sval;
+    a.out = d_out;
+    return a;
+}
+
 // Issues the kernels of one launch-list entry (one per K slice) on `stream`.
 // ws: the caller's workspace (null: the plan's own scratch memory); softmax: of the rows as well (see softmax_in_launch)
 static hipError_t issue_launch(const sddmm_plan *plan, const Launch &L, const float *d_val, const float *d_W,
@@ -186,11 +196,9 @@ static hipError_t issue_launch(const sddmm_plan *plan, const Launch &L, const fl
         }
         return hipSuccess;
     } else {
-        KArgs a = L.ka;
+        KArgs a = gather_args(plan, L, d_val, d_out);
         a.col_ind = plan->d_col;
-        a.val = val;
-        a.sval = d_val ? nullptr : L.sval;
-        a.W = d_W; a.H = d_H; a.out = d_out;
+        a.W = d_W; a.H = d_H;
         a.residual = residual;
         if (L.fn_kind == 1 && L.k_slice < I.K) return launch_gather_slices(a, L.rows, I.n_rows, L.fn_wide != 0, L.k_slice, stream);
         return launch(L.fn, dim3((unsigned)L.grid), dim3((unsigned)L.block), (size_t)L.lds, stream, a);
@@ -382,7 +390,9 @@ int sddmm_execute_profiled(const sddmm_plan *plan, const float *d_val, const flo
         prof[i].kernel = L.kind;
         prof[i].lanes_per_nnz = L.dfn || L.bfns[0] ? 0 : L.kind == SDDMM_KERNEL_PANEL ? 8 : (L.tfn ? L.tile_g : L.gather_g);
         prof[i].k_slice = L.k_slice;
-        prof[i].n_kernel_launches = (L.k_slice > 0 && L.k_slice < plan->info.K && !L.fused_slices) ? (plan->info.K + L.k_slice - 1) / L.k_slice : 1;
+        const bool slices = L.k_slice > 0 && L.k_slice < plan->info.K && !L.fused_slices;
+        prof[i].n_kernel_launches = !slices ? 1 : L.fn_kind == 1 ? gather_slice_launches(gather_args(plan, L, d_val, d_out), L.k_slice)
+                                                                 : (plan->info.K + L.k_slice - 1) / L.k_slice;
         prof[i].nnz = L.nnz;
         prof[i].rows = L.rows;
         prof[i].stream_positions = L.positions;

@@ -295,12 +295,13 @@ int add_row_gather(Ctx &c, const std::vector<int32_t> &rows, bool all_rows)
     L.fn_once = shape.once;
     L.fn_wide = gather_wide(c.n_rows, c.n_cols, c.K);
     a.K = c.K; a.n_cols = (int32_t)c.n_cols; a.tile_x = (int32_t)c.n_cols;
-    L.grid = (int32_t)((n + a.chunk - 1) / a.chunk);
-    L.block = kRowGatherBlock;
     L.k_slice = all_rows ? gather_slice(n, c.n_cols, c.K) : c.K;  // (as in the call without a plan)
+    const GatherShape launched = L.k_slice < c.K ? gather_shape(n, c.n_rows, (int64_t)rows.size(), L.k_slice) : shape;
+    L.grid = (int32_t)((n + launched.chunk - 1) / launched.chunk);
+    L.block = kRowGatherBlock;
     if (int rc = resolve_functions(L)) return rc;
-    c.P->info.lanes_per_nnz = var.G ? var.G : 8;
-    L.gather_g = var.G ? var.G : 8; L.positions = n;
+    L.gather_g = launched.v.G ? launched.v.G : 8; L.positions = n;
+    c.P->info.lanes_per_nnz = L.gather_g;
     c.P->launches.push_back(L);
     return SDDMM_OK;
 }

@@ -62,6 +62,10 @@ def test_slices_against_64_bits(n_rows, n_cols, nnz, K, slices):
     v = val.clone()
     plan.execute_epilogue(p(v), p(W), p(H), p(v), capi.EPILOGUE_RESIDUAL, st)
     assert torch.equal(v, out2)
+    for v, d_out, launches in ((val, out, slices), (v, v, 1)):
+        prof = plan.execute_profiled(p(v), p(W), p(H), p(d_out), st)
+        lanes = 8 if nnz > 32 * n_rows else 16  # (those of the kernel on slices)
+        assert [q["n_kernel_launches"] for q in prof] == [launches] and (slices == 1 or prof[0]["lanes_per_nnz"] == plan.info()["lanes_per_nnz"] == lanes)
     plan.close()
 
 
