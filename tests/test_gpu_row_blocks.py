@@ -285,3 +285,35 @@ def test_small_values_in_dense_factors(n, half, every, K):
         # (one rounding per product and sum, in any order)
         bound = (torch.from_numpy(np.diff(d["row_ptr"].numpy())) + 4)[:, None] * 2.0 ** -24 * ysize + 1e-42
         assert bool(((o.double() - size).abs() <= (K + 4) * 2.0 ** -24 * size).all()) and bool(((y.double() - ysize).abs() <= bound).all()), (what, e)
+
+
+# Full rows of one piece of 16,384 entries, of two with one entry in the last, of three: their softmax joins the pieces' records.
+@pytest.mark.parametrize("m", [16384, 16385, 32769, 40000])
+def test_full_rows_in_pieces(oracle, tmp_path, m):
+    n, K = 608, 64
+    rng = np.random.default_rng(m)
+    full = np.arange(0, n, 19)  # (32 rows: a block)
+    r, c = np.repeat(np.arange(n), 49), (np.arange(n)[:, None] + np.arange(49)).reshape(-1)
+    keep = ~np.isin(r, full)
+    key = np.unique(np.concatenate([r[keep].astype(np.int64) * m + c[keep], (full[:, None].astype(np.int64) * m + np.arange(m)).reshape(-1)]))
+    d = _dict_of(n, m, key // m, key % m, K, rng)
+    t, (plan, general) = plans(d, K)
+    assert is_blocks(plan, d), plan.info()
+    W, H = t["W"].data_ptr(), t["H"].data_ptr()
+    scores = torch.empty(d["nnz"], device=DEV)
+    plan.execute(0, W, H, scores.data_ptr())
+    want = oracle.row_softmax(d["row_ptr"].numpy(), scores.cpu().numpy())
+    path = tmp_path / "blocks.plan"
+    plan.save(path)
+    loaded = capi.Plan.load_device(path, n, m, d["nnz"], t["row_ptr"].data_ptr(), t["col_ind"].data_ptr(), K, keep=t)
+    first = None
+    for p in (plan, loaded):
+        nbytes = p.workspace_bytes()
+        ws = torch.full((nbytes // 4 + 1,), float("nan"), device=DEV)
+        for run in (lambda o: p.execute_softmax(0, W, H, o), lambda o: p.execute_ws(0, W, H, o, ws.data_ptr(), nbytes, capi.FORM_SOFTMAX)):
+            out = torch.full((d["nnz"],), float("nan"), device=DEV)
+            run(out.data_ptr())
+            torch.cuda.synchronize()
+            first = out if first is None else first
+            assert torch.equal(out, first)
+    assert np.allclose(first.cpu().numpy(), want, rtol=1e-5, atol=1e-30)

@@ -118,3 +118,37 @@ def test_many_rows(oracle, rows):
     torch.cuda.synchronize()
     softmax_ok(out[:-1].cpu().numpy(), oracle.row_softmax(rp, x))
     assert bool(torch.isnan(out[-1]))
+
+
+# A plan knows its longest row and leaves the kernel that joins the pieces of huge rows out where there are none: the longest row that
+# is none, the shortest that is one, one of several pieces.
+@pytest.mark.parametrize("longest", [17400, 17401, 40000])
+@pytest.mark.parametrize("kernel", [capi.KERNEL_ROW_GATHER, capi.KERNEL_LDS_TILE, capi.KERNEL_HYBRID])
+def test_longest_row_of_a_plan(oracle, tmp_path, kernel, longest):
+    rng = np.random.default_rng(longest)
+    n_cols, K = 40000, 32
+    lens = np.concatenate([rng.integers(0, 200, 150), [longest, 0, 1100], rng.integers(0, 200, 150)])
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    ci = np.concatenate([np.sort(rng.choice(n_cols, c, replace=False)) for c in lens]).astype(np.int32)
+    n, nnz = len(lens), len(ci)
+    rpd, cid = torch.from_numpy(rp).cuda(), torch.from_numpy(ci).cuda()
+    g = torch.Generator(device="cuda")
+    g.manual_seed(longest)
+    W, H, val = (torch.randn(*s, generator=g, device="cuda") for s in ((n, K), (n_cols, K), (nnz,)))
+    plan = capi.Plan.from_device_csr(n, n_cols, nnz, rpd.data_ptr(), cid.data_ptr(), K, options=capi.PlanOptions.defaults(kernel=kernel, dense_blocks=0, ignore_env=1))
+    plan.set_values(val.data_ptr())
+    scores = torch.empty(nnz, device="cuda")
+    plan.execute(0, W.data_ptr(), H.data_ptr(), scores.data_ptr())
+    path = tmp_path / "softmax.plan"
+    plan.save(path)
+    loaded = capi.Plan.load_device(path, n, n_cols, nnz, rpd.data_ptr(), cid.data_ptr(), K, keep=(rpd, cid))
+    want = oracle.row_softmax(rp, scores.cpu().numpy())
+    for p in (plan, loaded):
+        nbytes = p.workspace_bytes()
+        ws = torch.full((nbytes // 4 + 1,), float("nan"), device="cuda")
+        for run in (lambda o: p.execute_softmax(0, W.data_ptr(), H.data_ptr(), o),
+                    lambda o: p.execute_ws(0, W.data_ptr(), H.data_ptr(), o, ws.data_ptr(), nbytes, capi.FORM_SOFTMAX)):
+            out = torch.full((nnz,), float("nan"), device="cuda")
+            run(out.data_ptr())
+            torch.cuda.synchronize()
+            softmax_ok(out.cpu().numpy(), want)
