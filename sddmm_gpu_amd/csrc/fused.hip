@@ -25,9 +25,9 @@ namespace {
 // No staging: a row's loads are all in flight together, and 16 waves per compute unit hide their latency, which is
 // what bounds it until the entries do (the recommender pattern moves 0.8 GB at 3.5 TB/s).  Before this a kernel of its own
 // laid chunks of whole rows out, and rows that had been left over went through lists to a third one.  us, before and now: 18
-// thousand entries 11.8 and 8.9; R-MAT, 1.9 million 34 and 18, 28 million 134 and 111, 84 million 297 and 266, 189 million
+// thousand entries 11.8 and 7.7; R-MAT, 1.9 million 34 and 18, 28 million 134 and 111, 84 million 297 and 266, 189 million
 // 526 and 526; window of 320 a row, 5.2 million 24 and 19; 3 million rows of one
-// entry 38 and 30; 20 thousand entries spread over 4 million rows 93 and 25; a row of 30 million 328 and 93; recommender,
+// entry 38 and 30; 20 thousand entries spread over 4 million rows 93 and 23; a row of 30 million 328 and 93; recommender,
 // 100 million 235 and 231.  (Maximum and sum by scans over the entries, whatever the rows: 1072 there, bound by the vector
 // ALU.)
 constexpr int kSmBlock = 256;

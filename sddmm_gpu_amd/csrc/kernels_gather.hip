@@ -482,10 +482,15 @@ KernelFn gather_kernel(const Variant &v, bool once, bool wide)
 //   where few columns take most nonzeros and their rows fit (R-MAT 2^14, 3.0 million, K = 256 162 and 191; ratings of 6.2 million,
 //       5600 columns 284 and 300; uniform over 17,000 columns would gain: 3.2 million, K = 256 368 and 219),
 //   where most columns are used once (R-MAT 2^20, 1.6 million, K = 512 647 and 687; 3.3 million, K = 448 808 and 820),
-//   at other ranks (K = 384, whose lanes hold three pieces instead of four, R-MAT 2^15, 2.5 million 281 and 257, but band of 3 million
-//       594 and 653; K = 128, R-MAT 2^15, 4.4 million 121 and 133, uniform, 6 million 295 and 214).
-// Slices of 128 are faster on half of these, but at K = 512 their error against 64 bits is larger (9.9e-8 whole, 10.0e-8; of 64
-// 9.4e-8; K = 256 9.5e-8, 9.5e-8 and 8.6e-8).
+//   beyond K = 512, where the sums of slices have the larger error against 64 bits (R-MAT 2^17, K = 576 / 1024 9.2e-8 / 10.3e-8 whole,
+//       9.3e-8 / 10.6e-8 in slices, but K = 256 / 512 9.5e-8 / 9.9e-8 and 8.3e-8 / 9.2e-8); they would gain as at 512 (5.8 million, K = 640 /
+//       1024 1693 / 3498 and 1262 / 2409),
+//   at other ranks: at K = 192, 320 and 384 the lanes hold three pieces of whole rows instead of four, at 448 nearly four, so that
+//       slices gain less and lose more (K = 192 / 320 / 384, R-MAT 2^17, 2.6 million 167 / 319 / 405 and 178 / 310 / 398, band of 3 million 299 /
+//       494 / 598 and 327 / 498 / 656; large ones would gain, 5.8 million 386 / 740 / 951 and 330 / 609 / 751); K = 128, R-MAT 2^15, 1.0
+//       million 40 and 48, band 182 and 195, R-MAT 2^17, 5.8 million 283 and 232; ranks that 64 does not divide have a last slice across lines.
+// Slices of 128 are faster on half of these, but at K = 512 their error is larger (9.9e-8 whole, 10.0e-8; of 64 9.4e-8; K = 256 9.5e-8,
+// 9.5e-8 and 8.6e-8).
 int gather_slice(int64_t nnz, int64_t n_cols, int K)
 {
     const int64_t least = K == 256 ? 2500000 : K == 512 ? 1400000 : K == 448 ? 3000000 : INT64_MAX;

@@ -165,7 +165,8 @@ int make_plan(int64_t n_rows, int64_t n_cols, int64_t nnz, const int32_t *row_pt
 // the CSR pattern whatever the runs (see add_tile)?  From 4 million nonzeros on the rows are split by length, and tiles that
 // hold long rows only are the faster ones; so they are when the walk, at 17 TB/s, has more than 1.8 GB of H rows to read,
 // 2.8 where the tiles take slices of 64 (tiles against walk, ratings of 1.8, 2.4 and 3.6 M, K = 256: 108 / 101, 123 / 139 and
-// 167 / 190 us; of 2.6 and 3.8 M, K = 192: 148 / 131 and 180 / 184; K = 320, 1.8 and 2.6 M: 231 / 171 and 240 / 259).
+// 167 / 190 us; of 2.6 and 3.8 M, K = 192: 148 / 131 and 180 / 184; K = 320, 1.8 and 2.6 M: 231 / 171 and 240 / 259).  The walk's times from
+// K = 192 on are those before it took slices of H; with them it is faster up to more nonzeros (ratings of 1.2 M, K = 384 120 / 82).
 inline bool product_walks(int64_t nnz, int32_t K, int ks) { return nnz < 4000000 && nnz * K < (ks < 128 ? 700000000 : 450000000); }
 // And at a rank that is no multiple of the tiles' width ks, which they work on up to the next multiple?  From 4 million nonzeros
 // on, where little of that is padding (SDDMM + product, us, walk and tiles: ratings of 4.9 M, K = 20 / 36 / 50 / 75 / 120 68 / 95
@@ -195,6 +196,8 @@ inline bool ragged_product_tiles(int64_t nnz, int32_t K, int ks)
 //       338 / 324 (10.1), 2.2 M, K = 352 / 357 259 / 265 (11.3), 275 / 266 (11.5), word counts of 3.0 M, K = 369 478 / 350 (10.9), and with
 //       four slices and an H of up to 11 MB ratings of 2.9 / 3.2 M, K = 418 / 488 384 / 434 (10.6), 473 / 512 (12.4), uniform, 3.8 M, K =
 //       496 428 / 472 (13.2), but H of 12.5 MB, 3.3 M, K = 450 630 / 409 (10.4)
+// (The tiles have become 2 to 20 % faster since; of 302 pairs the slower form is taken by more than 5 % in 44, a walk in 39 of them:
+// profiles/product_pairs_ragged.txt.)
 inline double ragged_product_run(int64_t nnz, int64_t n_cols, int32_t K, int ks)
 {
     const double padded = (K + ks - 1) / ks * ks, h = 4.0 * n_cols * K;

@@ -241,7 +241,10 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
         // K = 384, 2 to 3.5 M nonzeros, H of 7 and 8 MB, runs of 10: 180 against 211 and 338 against 387 us; word counts of 6.9 M,
         // K = 128, H of 27 MB, runs of 7 392 / 269; of 1.8 M, H of 13 to 39 MB, runs of 8, K = 128 58 / 58, K = 256 112 /
         // 145, K = 384 166 / 251; uniform, K = 256, H of 17 and 31 MB, runs of 5 190 / 261 and 1515 / 1723, H of 21 MB,
-        // runs of 4 647 / 543).
+        // runs of 4 647 / 543).  (Drawn before the walk took slices of H and the tiles' rounds got shorter.  As both are now,
+        // profiles/spmm_tiles_or_walk.txt, 89 of 488 pairs are on tiles where the walk is more than 5 % faster, most of them from K = 192 on
+        // with an H beyond 15 MB, word counts and bands above all: 4.6 million, K = 256, H of 25 MB, runs of 7.5 468 / 230; and 18 walk where
+        // tiles are, uniform below 4 million at K = 32 and 64: 3.7 million, K = 64 34 / 47.)
         const bool h_near = (int64_t)c.n_cols * c.K * 4 <= 6000000;
         // (small products of three slices and more walk up to twice that: beside each slice's two launches they have little to do.
         // Ratings, K = 512, 0.48 and 1.05 million nonzeros, H of 6.2 and 8.1 MB, tiles and walk 134 / 170 and 57 / 98 us)
@@ -746,7 +749,8 @@ int add_tile(Ctx &c, const std::vector<int32_t> &rows_in, int32_t x, int32_t pan
             // and 133 / 150; K = 128, 16, 18 and 20 MB 57 / 60, 55 / 64 and 99 / 117; K = 256, 37 and 41 MB 107 / 151 and
             // 198 / 332; window of 313, 14 M, K = 128 and 256, a seventh of 21 and 41 MB 475 / 317 and 951 / 639; word
             // counts of 24.5 M, K = 256, all of 110 MB 1946 / 2937; R-MAT of 4.3 M, 16 times the mean, K = 64 to 256, H of
-            // 34 to 134 MB 211 / 94, 369 / 227 and 777 / 618).
+            // 34 to 134 MB 211 / 94, 369 / 227 and 777 / 618).  (That is the walk before it took slices of H: now windows of 5.6 and 8.9 million,
+            // K = 256, 1.8 to 2.6 times the mean, H of 33 and 37 MB, are on tiles for 378 and 698 where it takes 259 and 391.)
             const bool local = 4 * n_seg <= (int64_t)rows.size() * T.n_tiles;
             const double h_part = local ? std::min(1.0, 2e6 / (double)L.nnz) : 1.0;
             if (want_spmm && uneven && c.nnz == c.P->info.nnz &&
