@@ -92,3 +92,16 @@ def test_product_in_slices_against_64_bits(n_rows, n_cols, nnz, K):
             mag.index_add_(0, rows[i:i + (1 << 19)], part.abs())
         bound = 1e-5 * torch.diff(rp).clamp(min=1).double().sqrt()[:, None] * mag
         assert bool(((Y[:, k:k + 64].double() - want).abs() <= bound).all())
+
+
+def test_product_of_more_slices_than_a_grid_has():
+    """Rows of 16 MB: in slices of 16 pieces more than a grid's second dimension holds."""
+    K = 4 * 16 * 65535 + 4
+    rp = torch.tensor([0, 2, 3], dtype=torch.int32, device="cuda")
+    ci = torch.tensor([0, 1, 1], dtype=torch.int32, device="cuda")
+    x, H = torch.randn(3, device="cuda"), torch.randn(2, K, device="cuda")
+    Y = torch.full((2, K), float("nan"), device="cuda")
+    capi.spmm_csr(2, 2, 3, rp.data_ptr(), ci.data_ptr(), x.data_ptr(), K, H.data_ptr(), Y.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    want = torch.stack([x[0].double() * H[0].double() + x[1].double() * H[1].double(), x[2].double() * H[1].double()])
+    mag = torch.stack([(x[0] * H[0]).abs() + (x[1] * H[1]).abs(), (x[2] * H[1]).abs()])
+    assert bool(((Y.double() - want).abs() <= 1e-6 * mag.double() + 1e-30).all())
