@@ -37,19 +37,19 @@ constexpr int kMostSlices = 65535;  // (a grid's second dimension)
 constexpr uint32_t kRowChange = 0x80000000u;
 
 // Zeroes the rows of Y that the product adds to or leaves out: empty rows, and rows cut between workgroups (of 2^shift nonzeros).
-// A wave looks at 64 rows, or (2^rows_log2) at fewer as in the kernel below: a small matrix of long rows of H has 16 to 64 nonzeros
+// A wave looks at 64 rows, or fewer as in the kernel below: a small matrix of long rows of H has 16 to 64 nonzeros
 // to a workgroup, so nearly all of its rows are cut.  us with 64 rows a wave and so: 1024 rows, K = 256 6.0 and 2.3;
 // 4096, K = 384 10.0 and 3.3; 32,768, K = 192 7.2 and 5.6; with the product, 18 thousand nonzeros of 4096 rows, R-MAT, K = 16 / 32 / 64 /
 // 100 7.0 / 7.2 / 8.5 / 9.6 and 6.8 / 6.9 / 7.8 / 8.2.  (Where few rows are cut there is nothing to gain: uniform, 0.2 million of 20,000
 // rows, K = 16 / 32 / 64 7.9 / 8.1 / 10.2 and 8.0 / 8.3 / 10.4.)
 __global__ __launch_bounds__(256)
-void sddmm_spmm_zero_rows_kernel(const int32_t *__restrict__ row_ptr, float *Y, uint32_t n_rows, int K, int shift, int rows_log2)
+void sddmm_spmm_zero_rows_kernel(const int32_t *__restrict__ row_ptr, float *Y, int64_t n_rows, int K, int shift, int rows_per_wave)
 {
     __shared__ int list[4][64];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t r = ((blockIdx.x * 4 + wave) << rows_log2) + lane;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t r = lane < rows_per_wave ? ((int64_t)blockIdx.x * 4 + wave) * rows_per_wave + lane : n_rows;
     bool zero = false;
-    if (r < n_rows && lane >> rows_log2 == 0) {
+    if (r < n_rows) {
         const int s = row_ptr[r], e = row_ptr[r + 1];
         zero = s >= e || (s >> shift) != ((e - 1) >> shift);
     }
@@ -464,7 +464,7 @@ extern "C" int sddmm_spmm_csr(int64_t n_rows, int64_t n_cols, int64_t nnz, const
     const CsrShape c = csr_shape(nnz, n_rows, n_cols, K);
     const int per_wave = rows_per_wave(n_rows, K);
     if (int rc = checked(launch(sddmm_spmm_zero_rows_kernel, dim3((unsigned)((n_rows + 4 * per_wave - 1) / (4 * per_wave))), dim3(256), 0, st, d_row_ptr,
-                                d_Y, (uint32_t)n_rows, (int)K, c.wg_shift, __builtin_ctz(per_wave))))
+                                d_Y, n_rows, (int)K, c.wg_shift, per_wave)))
         return rc;
     if (nnz == 0) return SDDMM_OK;
     return checked(launch_csr<false>(c, n_rows, n_cols, nnz, d_row_ptr, d_col_ind, d_x, K, d_H, d_Y, nullptr, st));
